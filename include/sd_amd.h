@@ -456,6 +456,14 @@ int sd_linear_two_inputs(const void* W, const void* x, const void* x2, int64_t l
  * sd_qkv_rope_wide pass N = (Hq + 2*Hkv) * D and SD_EPI_STORE.              */
 size_t sd_linear_wide_workspace_bytes(int M, int N, int K, int epilogue);
 
+/* The same linear layers over any number of rows, made for the hundreds of a
+ * prompt pass (bf16 tiles; K % 64 == 0, K >= 128; no workspace): both operands
+ * pass through LDS by direct loads.  A row has the bits that sd_linear_wide
+ * gives it.                                                                  */
+int sd_linear_prompt(const void* W, const void* x, int64_t ldx, const void* bias,
+                     const void* residual, void* out, int64_t ldo, int M, int N,
+                     int K, int epilogue, sd_stream_t stream);
+
 /* Rotary positions that differ from the cache position (the multimodal rotary
  * embedding of Qwen2-VL: transformers/models/qwen2_vl/modeling_qwen2_vl.py,
  * apply_multimodal_rotary_pos_emb and get_rope_index).  Frequency index i of a

@@ -649,3 +649,27 @@ def test_wide_qkv_rope_append_matches_narrow_ops(Hq, Hkv, D, H, rope):
     for a, b in zip(*caches):
         torch.testing.assert_close(a, b, rtol=2e-2, atol=2e-2)
     assert caches[1][1].abs().sum() > 0 and caches[1][2].abs().sum() > 0
+
+
+@pytest.mark.parametrize("M", [257, 384, 400, 513])
+@pytest.mark.parametrize("N,K", [(16, 128), (130, 192), (1000, 704), (768, 4096), (16400, 320), (17000, 256)])
+def test_prompt_linear_has_the_bits_of_the_wide_kernels(M, N, K):
+    """Row counts, outputs and K at the edges of the blocks (128 and 256 rows and outputs, 64 columns a stage, K one
+    to several splits, an odd number of stages), every epilogue: equal to sd_linear_wide over blocks of 256 rows,
+    whose sums the kernel repeats (same MFMA order, splits added in index order)."""
+    ops = _ops()
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=gen, device="cuda").to(torch.bfloat16)
+    W2 = (torch.randn(2 * N, K, generator=gen, device="cuda") * K ** -0.5).to(torch.bfloat16)
+    bias = torch.randn(2 * N, generator=gen, device="cuda").to(torch.bfloat16)
+    res = torch.randn(M, N, generator=gen, device="cuda").to(torch.bfloat16)
+    for epi in range(6):
+        gated = epi == ops.EPI_SILU_MUL
+        Wt = ops._tiled(W2 if gated else W2[:N].contiguous(), epi)
+        for b in (None, bias if gated else bias[:N].contiguous()):
+            r = res if epi == ops.EPI_RESIDUAL else None
+            got = ops.linear_prompt(Wt, x, b, r, epi)
+            few = torch.cat([ops.linear_wide(Wt, x[i:i + 256].contiguous(), b,
+                                             None if r is None else r[i:i + 256].contiguous(), epi)
+                             for i in range(0, M, 256)])
+            assert torch.equal(got, few), (epi, b is not None)

@@ -1,0 +1,320 @@
+// Linear layers over more than 256 token rows (prompt passes) on the tiled bf16 weights of the other linear
+// kernels.
+//
+// sd_linear_wide's kernels stream the weights past at most 256 rows held in LDS; a prompt of 1024 rows read
+// every weight four times, split K over workgroups whenever a matrix had fewer than 128 groups (partial sums of
+// S x rows x N floats written and read back) and left most of the matrix pipe idle (640 TFLOP/s on the split
+// matrices of an 8B model without their second launch, 880 on gate/up).  With hundreds of rows the op is bound
+// by the matrix pipe and by what feeds it.  Here both operands of a block pass through LDS by direct loads
+// (16 bytes a lane, no registers), 64 columns a stage, two stages; four waves, each with its own TN x TM tiles
+// of 16 x 16 in registers, so a fragment read from LDS feeds TM (or TN) MFMAs:
+//   8 x 8 tiles a wave (256 x 256 a block): 64 B of LDS reads a clock against 128, one wave a SIMD, every
+//     accumulator register there is;
+//   4 x 4 (128 x 128): two blocks a CU, and room for a second set of sums.
+// The second set is for matrices whose K the narrower kernels split: a row's bits must not depend on how many
+// rows share its pass, so the sums of a split are chained in one accumulator, and the splits' sums are added in
+// index order from zero, as wide_epilogue_kernel adds them; in registers, without a second launch.
+//
+// A stage of a row is 128 bytes (8 pieces of 16); piece c of row r lies at slot c ^ (r & 7), which spreads the
+// 16-row fragment reads over the banks; the source address carries the permutation, so a wave's direct load
+// still covers whole 128-byte lines.  Loads past the matrix or past the last row are clamped or answered with
+// zeros by the buffer's bounds; what they feed is never stored.
+#include <type_traits>
+
+#include "sd_common.h"
+#include "sd_wide_epi.h"
+
+namespace {
+
+struct PromptArgs {
+  const bf16_t* W;
+  const bf16_t* x;
+  int64_t ldx;
+  int M, KS, n_tiles, ks_per_split;
+  int n_blocks, m_blocks;  // grid = n_blocks * m_blocks
+  WideEpiArgs epi;
+};
+
+typedef __attribute__((address_space(3))) void lds_void;
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, unsigned bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00027000);
+}
+
+// Workgroups go round the 8 XCDs in launch order.  Each XCD takes a contiguous run of the work list, in which eight
+// row blocks of one weight block are next to each other: the 32 or 64 blocks that an XCD runs at once then read
+// about as many different weight blocks as row blocks, the least bytes for its L2 (all row blocks of a weight block
+// next to each other: 963 TFLOP/s at 4096 rows of 14336, where 2048 rows reached 1197).
+constexpr int kRowGroup = 8;
+__device__ __forceinline__ int xcd_order(int id, int n) {
+  const int q = n >> 3, r = n & 7, x = id & 7, i = id >> 3;
+  return x * q + min(x, r) + i;
+}
+
+// Barrier of the workgroup behind this wave's LDS reads and all but the newest LEFT of its direct loads
+// (__syncthreads() would wait for every load in flight in some places and for none in others: it does not count
+// direct loads as LDS writes).
+template <int LEFT>
+__device__ __forceinline__ void meet() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LEFT) : "memory");
+}
+
+template <int TN, int TM, int STAGES, bool SPLIT, int EPI>
+__global__ __launch_bounds__(256, SPLIT ? 2 : 1) void prompt_gemm_kernel(PromptArgs a) {
+  constexpr int BN = 2 * TN, BM = 2 * TM * 16;         // weight tiles and token rows of the block
+  constexpr int kABytes = BN * 2 * 1024, kBBytes = BM * 128;
+  constexpr int kAPieces = BN * 2 / 4, kBPieces = BM / 8 / 4;  // 1 KiB direct loads per wave and stage
+  __shared__ __attribute__((aligned(1024))) char s0[kABytes + kBBytes];
+  __shared__ __attribute__((aligned(1024))) char s1[kABytes + kBBytes];
+  __shared__ __attribute__((aligned(1024))) char s2[STAGES == 4 ? kABytes + kBBytes : 1024];
+  __shared__ __attribute__((aligned(1024))) char s3[STAGES == 4 ? kABytes + kBBytes : 1024];
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int work = xcd_order(blockIdx.x, gridDim.x);
+  const int grp = work / (a.n_blocks * kRowGroup), in_grp = work - grp * a.n_blocks * kRowGroup;
+  const int grp_rows = min(kRowGroup, a.m_blocks - grp * kRowGroup);
+  const int nb = in_grp / grp_rows, mb = grp * kRowGroup + in_grp - nb * grp_rows;
+  const int tile0 = nb * BN, row0 = mb * BM;
+  const int n_it = a.KS >> 1;
+
+  // this wave's direct loads: weights, piece p = (tile p >> 1, k-step p & 1) of the block's tiles
+  const char* wbase = reinterpret_cast<const char*>(a.W) + (size_t)tile0 * a.KS * 1024;
+  const int live_tiles = min(BN, a.n_tiles - tile0);
+  const auto wr = buffer_of(wbase, (unsigned)min((size_t)live_tiles * a.KS * 1024, (size_t)0xffffffffu));
+  const int w_step = a.KS * 1024;
+  // rows, piece p = rows 8p .. 8p + 7 of the block
+  const char* xbase = reinterpret_cast<const char*>(a.x) + (size_t)row0 * a.ldx * 2;
+  const int live_rows = min(BM, a.M - row0);
+  const auto xr = buffer_of(xbase, (unsigned)((size_t)(live_rows - 1) * a.ldx * 2 + (size_t)a.KS * 64));
+  const unsigned x_lane = (unsigned)(lane >> 3) * (unsigned)a.ldx * 2 + (((lane & 7) ^ (lane >> 3)) << 4);
+  const unsigned x_step = 8u * (unsigned)a.ldx * 2;
+  constexpr int kPieces = kAPieces + kBPieces;
+  auto stage_piece = [&](char* s, int it, int i) __attribute__((always_inline)) {
+    if (i < kAPieces) {
+      const int p = wave + 4 * i;
+      // (the tile is part of the lane offset: that is what the bounds check sees)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void*)(s + p * 1024), 16, lane * 16 + (p >> 1) * w_step,
+                                               (2 * it + (p & 1)) * 1024, 0, 0);
+    } else {
+      const int p = wave + 4 * (i - kAPieces);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void*)(s + kABytes + p * 1024), 16, x_lane + p * x_step,
+                                               it * 128, 0, 0);
+    }
+  };
+
+  const int wn = wave & 1, wm = wave >> 1;
+  const int xc = lane & 15, xq = lane >> 4;
+  const int a_off = wn * TN * 2048 + lane * 16;
+  const int b_row = kABytes + (wm * TM * 16 + xc) * 128;
+  const int b_sw[2] = {((xq ^ (xc & 7)) << 4), (((xq + 4) ^ (xc & 7)) << 4)};
+  bf16x8 fa[2][TN], fb[2][TM];
+  constexpr int kReads = TN + TM, kMfma = TN * TM;
+  static_assert(kReads <= kMfma * 3 / 4, "at most one LDS read an MFMA");
+  auto read_piece = [&](const char* s, int ks, int i) __attribute__((always_inline)) {
+    if (i < TN)
+      fa[ks][i] = *reinterpret_cast<const bf16x8*>(s + a_off + i * 2048 + ks * 1024);
+    else
+      fb[ks][i - TN] = *reinterpret_cast<const bf16x8*>(s + b_row + (i - TN) * 2048 + b_sw[ks]);
+  };
+  f32x4 acc[TN][TM], tot[SPLIT ? TN : 1][SPLIT ? TM : 1];
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < TN; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+      acc[i][j] = zero;
+      if (SPLIT) tot[i][j] = zero;
+    }
+  // Left to itself the compiler moves accumulators between registers around its MFMAs (two moves per MFMA in the
+  // largest shape: 876 TFLOP/s where 1050 are reached in place, 8192 x 2 x 1024 outputs of 4096), so the instruction
+  // is written out with its accumulator tied in place.  The wait states that the compiler would insert between it
+  // and other accesses of the accumulators are then placed by hand (settle).
+  auto settle = [&]() __attribute__((always_inline)) {
+    asm volatile("s_nop 15\n\ts_nop 15");
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j) {
+        if constexpr (SPLIT) asm volatile("" : "+v"(acc[i][j]));
+        else asm volatile("" : "+a"(acc[i][j]));
+      }
+    asm volatile("s_nop 15");
+  };
+  auto mfma = [&](int ks, int i, int j) __attribute__((always_inline)) {
+    if constexpr (SPLIT)
+      asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc[i][j]) : "v"(fa[ks][i]), "v"(fb[ks][j]));
+    else
+      asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(fa[ks][i]), "v"(fb[ks][j]));
+  };
+  // The MFMAs of one k-step with the next one's LDS reads (`from`) and the direct loads of a later stage between them
+  auto phase = [&](auto k_step, const char* from, auto loads, char* to, int it) __attribute__((always_inline)) {
+    constexpr int ks = decltype(k_step)::value;
+    constexpr bool kLoads = decltype(loads)::value;
+#pragma unroll
+    for (int n = 0; n < kMfma; ++n) {
+      mfma(ks, n / TM, n % TM);
+      // (the reads in the first three quarters: the last one has its latency behind it at the phase's end)
+      constexpr int kOver = kMfma * 3 / 4;
+      if (n < kOver && (n + 1) * kReads / kOver > n * kReads / kOver) read_piece(from, ks ^ 1, n * kReads / kOver);
+      if (kLoads && (n + 1) * kPieces / kMfma > n * kPieces / kMfma) stage_piece(to, it, n * kPieces / kMfma);
+    }
+  };
+  const int its_per_split = SPLIT ? a.ks_per_split >> 1 : 0;
+  int next_split = its_per_split;
+  // One stage of 64 columns: `cur` holds it (its first k-step's fragments are in registers already), `nxt` the
+  // stage behind it; cur's place is then loaded with the stage STAGES further on.
+  auto step = [&](char* cur, char* nxt, int it) __attribute__((always_inline)) {
+    phase(std::integral_constant<int, 0>{}, cur, std::false_type{}, nullptr, 0);
+    // every wave has read `cur` and its own part of `nxt` has landed
+    meet<(STAGES - 2) * kPieces>();
+    phase(std::integral_constant<int, 1>{}, nxt, std::true_type{}, cur, min(it + STAGES, n_it - 1));
+    if (SPLIT && it + 1 == next_split && it + 1 < n_it) {
+      settle();
+#pragma unroll
+      for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int j = 0; j < TM; ++j) {
+          tot[i][j] += acc[i][j];
+          acc[i][j] = zero;
+        }
+      next_split += its_per_split;
+      settle();
+    }
+  };
+  auto fill = [&](char* s, int it) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) stage_piece(s, min(it, n_it - 1), i);
+  };
+  fill(s0, 0);
+  fill(s1, 1);
+  if constexpr (STAGES == 4) {
+    fill(s2, 2);
+    fill(s3, 3);
+  }
+  meet<(STAGES - 1) * kPieces>();
+#pragma unroll
+  for (int i = 0; i < kReads; ++i) read_piece(s0, 0, i);
+  settle();
+  int it = 0;
+  if constexpr (STAGES == 4) {
+    for (; it + 3 < n_it; it += 4) {
+      step(s0, s1, it);
+      step(s1, s2, it + 1);
+      step(s2, s3, it + 2);
+      step(s3, s0, it + 3);
+    }
+    if (it < n_it) step(s0, s1, it);
+    if (it + 1 < n_it) step(s1, s2, it + 1);
+    if (it + 2 < n_it) step(s2, s3, it + 2);
+  } else {
+    for (; it + 1 < n_it; it += 2) {
+      step(s0, s1, it);
+      step(s1, s0, it + 1);
+    }
+    if (it < n_it) step(s0, s1, it);
+  }
+  meet<0>();  // no direct load outlives the workgroup's use of LDS
+  settle();
+
+  if (SPLIT) {
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j) acc[i][j] = tot[i][j] + acc[i][j];
+  }
+  // acc[i][j][reg] = (tile row 4 * xq + reg of tile i, token 16 j + xc).  Through LDS, 16 token rows at a time
+  // and each wave for itself, so that the lanes of a store hold neighbouring outputs of a row (and the epilogue
+  // is there once per token tile, not once per pair of tiles).
+  constexpr bool PAIRED = EPI == SD_EPI_SILU_MUL || EPI == EPI_QKV_ROPE;
+  constexpr int kLd = TN * 16 + 4;                        // floats; 16 rows start on different banks
+  constexpr int kUnits = PAIRED ? TN * 2 : TN * 4;        // of a row; 64 lanes take 64 / kUnits rows at once
+  float* img = reinterpret_cast<float*>(wave < 2 ? s0 : s1) + (wave & 1) * 16 * kLd;
+  const int u = lane % kUnits, ui = PAIRED ? u >> 1 : u >> 2, r0 = PAIRED ? (u & 1) * 4 : (u & 3) * 4;
+  const int tile = tile0 + wn * TN + ui;
+#pragma unroll
+  for (int j = 0; j < TM; ++j) {
+#pragma unroll
+    for (int i = 0; i < TN; ++i) *reinterpret_cast<f32x4*>(img + xc * kLd + i * 16 + 4 * xq) = acc[i][j];
+#pragma unroll 1
+    for (int r = lane / kUnits; r < 16; r += 64 / kUnits) {
+      const int m = row0 + (wm * TM + j) * 16 + r;
+      const float* src = img + r * kLd + ui * 16 + r0;
+      const f32x4 lo = *reinterpret_cast<const f32x4*>(src);
+      f32x4 hi = zero;
+      if (PAIRED) hi = *reinterpret_cast<const f32x4*>(src + 8);
+      if (tile < a.n_tiles && m < a.M) emit_unit<EPI>(a.epi, m, tile, r0, lo, hi);
+    }
+  }
+}
+
+template <int TN, int TM, int STAGES, bool SPLIT, int EPI>
+int launch_prompt(PromptArgs a, hipStream_t st) {
+  a.n_blocks = (a.n_tiles + 2 * TN - 1) / (2 * TN);
+  a.m_blocks = (a.M + 32 * TM - 1) / (32 * TM);
+  hipLaunchKernelGGL((prompt_gemm_kernel<TN, TM, STAGES, SPLIT, EPI>), dim3(a.n_blocks * a.m_blocks), dim3(256), 0, st, a);
+  SD_CHECK_LAUNCH("sd_prompt_linear");
+  return SD_OK;
+}
+
+template <int EPI>
+int prompt_shape(const PromptArgs& a, int S, hipStream_t st) {
+  const long big = (long)((a.n_tiles + 15) / 16) * ((a.M + 255) / 256);
+  const long small = (long)((a.n_tiles + 7) / 8) * ((a.M + 127) / 128);
+  if (S == 1 && big >= 128) return launch_prompt<8, 8, 2, false, EPI>(a, st);
+  if (small <= 256) return launch_prompt<4, 4, 4, true, EPI>(a, st);
+  return launch_prompt<4, 4, 2, true, EPI>(a, st);
+}
+
+}  // namespace
+
+bool sd_prompt_linear_fits_(int M, int n_tiles, int K, int64_t ldx) {
+  // 256 rows are one pass of the wide kernels.  Few blocks of a long K leave most CUs idle for a long time: 48 blocks
+  // of K 8192 59 us against 50 in two passes of the wide kernels (300 rows, 2048 outputs), 96 blocks of K 14336 as
+  // long as those, 48 blocks of K 2048 23 us against 36.
+  const long blocks = (long)((n_tiles + 7) / 8) * ((M + 127) / 128);
+  return M > 256 && K % 64 == 0 && K >= 128 && (blocks > 64 || K <= 4096) && 512 * ldx < 0x7fffffff;
+}
+
+// epi: an SD_EPI_* number or EPI_QKV_ROPE, with what that epilogue reads in `e`.
+int sd_prompt_linear_(const void* W, const void* x, int64_t ldx, int M, int K, int n_tiles, int epi,
+                      const WideEpiArgs& epi_args, sd_stream_t stream) {
+  int S, ksp, g;
+  WideEpiArgs e = epi_args;
+  e.M = M;
+  e.NR = n_tiles * 16;
+  e.S = 1;
+  plan_split(n_tiles, K, S, ksp, g);
+  PromptArgs a{(const bf16_t*)W, (const bf16_t*)x, ldx, M, K / 32, n_tiles, ksp, 0, 0, e};
+  hipStream_t st = (hipStream_t)stream;
+  switch (epi) {
+    case SD_EPI_F32: return prompt_shape<SD_EPI_F32>(a, S, st);
+    case SD_EPI_STORE: return prompt_shape<SD_EPI_STORE>(a, S, st);
+    case SD_EPI_RESIDUAL: return prompt_shape<SD_EPI_RESIDUAL>(a, S, st);
+    case SD_EPI_SILU_MUL: return prompt_shape<SD_EPI_SILU_MUL>(a, S, st);
+    case SD_EPI_RELU: return prompt_shape<SD_EPI_RELU>(a, S, st);
+    case SD_EPI_GELU_TANH: return prompt_shape<SD_EPI_GELU_TANH>(a, S, st);
+    case EPI_QKV_ROPE: return prompt_shape<EPI_QKV_ROPE>(a, S, st);
+  }
+  sd_set_error("sd_prompt_linear: unknown epilogue %d", epi);
+  return SD_ERR_INVALID;
+}
+
+extern "C" int sd_linear_prompt(const void* W, const void* x, int64_t ldx, const void* bias, const void* residual,
+                                void* out, int64_t ldo, int M, int N, int K, int epilogue, sd_stream_t stream) {
+  SD_REQUIRE(W && x && out, SD_ERR_INVALID, "sd_linear_prompt: null pointer");
+  SD_REQUIRE(epilogue >= SD_EPI_STORE && epilogue <= SD_EPI_GELU_TANH && (epilogue != SD_EPI_RESIDUAL || residual),
+             SD_ERR_INVALID, "sd_linear_prompt: unknown epilogue %d, or a residual missing", epilogue);
+  SD_REQUIRE(M >= 0 && N >= 1 && ldo >= N && ldx >= K && ldx % 8 == 0 && 512 * ldx < 0x7fffffff && sd_aligned16(W) &&
+                 sd_aligned16(x), SD_ERR_INVALID, "sd_linear_prompt: rows must be 16-byte aligned (M=%d N=%d K=%d ldx=%lld)",
+             M, N, K, (long long)ldx);
+  SD_REQUIRE(K % 64 == 0 && K >= 128, SD_ERR_UNSUPPORTED, "sd_linear_prompt: K must be a multiple of 64, at least 128 (K=%d)", K);
+  if (M == 0) return SD_OK;
+  WideEpiArgs e{};
+  e.N = N;
+  e.bias = (const bf16_t*)bias;
+  e.residual = (const bf16_t*)residual;
+  e.out = out;
+  e.ldo = ldo;
+  return sd_prompt_linear_(W, x, ldx, M, K, tiles_of(N, epilogue), epilogue, e, stream);
+}

@@ -15,6 +15,7 @@
 #include <vector>
 
 #include "sd_common.h"
+#include "sd_wide_epi.h"
 
 namespace {
 
@@ -1286,6 +1287,9 @@ int seq_linear(const void* w_rm, const void* w_tiled, int w_f32, const float* x,
   if (!w_tiled) return sd_matmul_rows(x, x2, ldx, w_rm, w_f32, bias, y, ldy, M, N, K, stream);
   SD_REQUIRE(!bias, SD_ERR_INVALID, "seq_linear: a tiled matrix takes no f32 bias");
   if (M <= 16) return sd_linear(w_tiled, nullptr, x_b, ldxb, nullptr, nullptr, y, ldy, M, N, K, SD_EPI_F32, stream);
+  if (sd_aligned16(w_tiled) && sd_aligned16(x_b) && ldxb % 8 == 0 && ldxb >= K &&
+      sd_prompt_linear_fits_(M, tiles_of(N, SD_EPI_F32), K, ldxb))
+    return sd_linear_prompt(w_tiled, x_b, ldxb, nullptr, nullptr, y, ldy, M, N, K, SD_EPI_F32, stream);
   for (int r0 = 0; r0 < M; r0 += kWideRows) {
     const int mm = M - r0 < kWideRows ? M - r0 : kWideRows;
     const int rc = sd_linear_wide(w_tiled, nullptr, (const bf16_t*)x_b + (size_t)r0 * ldxb, ldxb, nullptr, nullptr,

@@ -1000,6 +1000,8 @@ extern "C" int sd_row_scales_fp8(const void*, int64_t, int, int, float*, sd_stre
   set_error("sd_row_scales_fp8: not available in the CPU build");
   return SD_ERR_UNSUPPORTED;
 }
+extern "C" int sd_linear_prompt(const void*, const void*, int64_t, const void*, const void*, void*, int64_t, int, int,
+                                int, int, sd_stream_t) { UNSUPPORTED("sd_linear_prompt"); }
 extern "C" int sd_linear_wide_a8(const void*, const float*, const float*, const void*, int64_t, const void*,
                                  const void*, void*, int64_t, int, int, int, int, void*, size_t, sd_stream_t) {
   set_error("sd_linear_wide_a8: not available in the CPU build");

@@ -611,6 +611,23 @@ def linear_wide(W, x, bias=None, residual=None, epilogue=EPI_STORE, out=None,
     return out
 
 
+def linear_prompt(W, x, bias=None, residual=None, epilogue=EPI_STORE, out=None) -> torch.Tensor:
+    """linear() for the many rows of a prompt pass (sd_linear_prompt: bf16 weights, K a multiple of 64 from 128 up);
+    a row has the bits linear_wide gives it."""
+    _need(x, torch.bfloat16, "x")
+    Wt = _tiled(W, epilogue)
+    if Wt.scale is not None:
+        raise _lib.SdError("linear_prompt takes bf16 weights")
+    M, K = x.shape
+    if K != Wt.K:
+        raise _lib.SdError(f"linear_prompt: rows of {K} columns for a matrix of {Wt.K}")
+    if out is None:
+        out = torch.empty(M, Wt.N, dtype=torch.float32 if epilogue == EPI_F32 else torch.bfloat16, device=x.device)
+    _lib.check(_lib.load().sd_linear_prompt(_p(Wt.data), _p(x), x.stride(0), _p(bias), _p(residual), _p(out),
+                                            out.stride(0), M, Wt.N, K, epilogue, _stream()), "sd_linear_prompt")
+    return out
+
+
 def _rope_positions(rope_pos, rope_delta, mrope_section, rows):
     """ctypes sd_rope_positions (or None): rope_pos int32 [3, rows], rope_delta int32 [B],
     mrope_section = (temporal, height, width) frequency counts."""

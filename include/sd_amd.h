@@ -464,6 +464,20 @@ int sd_linear_prompt(const void* W, const void* x, int64_t ldx, const void* bias
                      const void* residual, void* out, int64_t ldo, int M, int N,
                      int K, int epilogue, sd_stream_t stream);
 
+/* Attention of a prompt pass over the paged cache (which holds the pass's keys
+ * and values already).  items [n_items][4] i32 (device, 16-byte aligned), one
+ * per run of consecutive tokens of a sequence: {first row, tokens, row of
+ * block_tables, position of the first token}, 1 <= tokens <=
+ * SD_PROMPT_BLOCK_ROWS / (Hq/Hkv); a row sees the keys up to its own position.
+ * max_ctx: host bound on position + 1.  split_tokens (128 or 256) as for
+ * sd_paged_attention, whose bits a row gets however a prompt is cut into items. */
+#define SD_PROMPT_BLOCK_ROWS 128
+int sd_prompt_attention(const void* q, int64_t ldq, const void* k_cache,
+                        const void* v_cache, const int32_t* block_tables,
+                        int max_blocks_per_seq, const int32_t* items, int n_items,
+                        void* out, int64_t ldo, int Hq, int Hkv, int D, float scale,
+                        int max_ctx, int split_tokens, sd_stream_t stream);
+
 /* Rotary positions that differ from the cache position (the multimodal rotary
  * embedding of Qwen2-VL: transformers/models/qwen2_vl/modeling_qwen2_vl.py,
  * apply_multimodal_rotary_pos_emb and get_rope_index).  Frequency index i of a
@@ -857,10 +871,33 @@ typedef struct {
   int32_t* argmax_idx;
 } sd_forward_args;
 
+/* A prompt pass: any number of token rows of any sequences (sd_model_forward's
+ * rows are B x q_len of at most 256), e.g. several prompts of different lengths
+ * one behind the other.  The linear layers have the bits of sd_model_forward's
+ * wide family; the attention is sd_prompt_attention.  A row's results do not
+ * depend on what shares its pass or on how a prompt is cut into passes.       */
+typedef struct {
+  int rows, n_items, n_out;
+  const int32_t* token_ids; /* [rows]                                         */
+  const int32_t* row_seq;   /* [rows] row of kv->block_tables                  */
+  const int32_t* row_pos;   /* [rows] position in its sequence                 */
+  const int32_t* items;     /* [n_items][4], as for sd_prompt_attention        */
+  const int32_t* out_rows;  /* [n_out] rows whose logits are wanted (<= 256)   */
+  float* logits;            /* [n_out, vocab (or lm_vocab)] f32                */
+  const void* input_embeds; /* [rows, hidden] bf16 instead of token_ids, or NULL */
+  const int32_t* rope_pos;  /* [3][rows] (models with mrope sections), or NULL */
+  int wide_a8;              /* as in sd_forward_args                           */
+  int max_ctx, split_tokens; /* as for sd_prompt_attention                     */
+} sd_prompt_args;
+
+
 size_t sd_model_workspace_bytes(const sd_model* m, int max_rows, int max_ctx,
                                 int split_tokens);
 /* One forward pass of B*q_len token rows: embeds, runs every layer (appending
  * K/V to the cache), final norm and LM head.  Enqueues kernels only.        */
+size_t sd_model_prompt_workspace_bytes(const sd_model* m, int max_rows);
+int sd_model_prompt(sd_model* m, const sd_kv_cache* kv, const sd_prompt_args* args,
+                    void* workspace, size_t workspace_bytes, sd_stream_t stream);
 int sd_model_forward(sd_model* m, const sd_kv_cache* kv,
                      const sd_forward_args* a, void* workspace,
                      size_t workspace_bytes, sd_stream_t stream);

@@ -1,0 +1,77 @@
+"""Prompt passes: packed rows of several prompts through sd_model_prompt and its attention, against the passes of
+sd_model_forward, whose bits they must have."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("Hq,Hkv,D", [(4, 1, 128), (14, 2, 64), (7, 1, 128), (4, 4, 64), (64, 1, 128)])
+@pytest.mark.parametrize("split", [128, 256])
+def test_prompt_attention_has_the_bits_of_paged_attention(Hq, Hkv, D, split):
+    """Runs that start and end at the edges of pages (16), tiles (32), chains and splits; group sizes that do and do not
+    divide a workgroup's 128 rows; wide score ranges (a running maximum that moves)."""
+    from vllm_omni_draft_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(Hq + D + split)
+    G = Hq // Hkv
+    runs = [(0, 1), (0, 33), (15, 17), (31, 130), (255, 2), (300, 257), (1023, 70)]   # first position, tokens
+    ctx = 1100
+    pages = (ctx + 15) // 16
+    kc = torch.randn(len(runs) * pages, Hkv, 16 * D, generator=g, device="cuda").to(torch.bfloat16)
+    vc = torch.randn(len(runs) * pages, Hkv, 16 * D, generator=g, device="cuda").to(torch.bfloat16)
+    bt = torch.randperm(len(runs) * pages, generator=g, device="cuda").to(torch.int32).view(len(runs), pages)
+    rows = sum(n for _, n in runs)
+    q = (torch.randn(rows, Hq * D, generator=g, device="cuda") * 3).to(torch.bfloat16)
+    block = ops.PROMPT_BLOCK_ROWS // G
+    items, ref, row = [], [], 0
+    for s, (p0, n) in enumerate(runs):
+        items += [(row + i, min(block, n - i), s, p0 + i) for i in range(0, n, block)]
+        lens = torch.tensor([p0], dtype=torch.int32, device="cuda")
+        ref.append(ops.paged_attention_blocked(q[row:row + n].contiguous(), kc, vc, bt[s:s + 1].contiguous(), lens, 0, 1, n,
+                                               max(1, min(n, 64 // G)), Hq, Hkv, D, D ** -0.5, max_ctx=pages * 16,
+                                               split_tokens=split))
+        row += n
+    got = ops.prompt_attention(q, kc, vc, bt, torch.tensor(items[::-1], dtype=torch.int32, device="cuda"), Hq, Hkv, D,
+                               D ** -0.5, max(p + n for p, n in runs), split)
+    ref = torch.cat(ref).view(rows, Hq * D)
+    assert torch.isfinite(got.float()).all() and torch.equal(got, ref)
+
+
+@pytest.mark.parametrize("kw", [{}, {"fp8": True}, {"arch": "opt"}, {"qkv_bias": True, "n_kv_heads": 1, "n_heads": 7, "head_dim": 64}])
+def test_packed_prompts_have_the_bits_of_forward_passes(kw):
+    """Several prompts in one pass of more than 256 rows against forward passes of each alone: logits and caches."""
+    from vllm_omni_draft_amd import config, weights
+    from vllm_omni_draft_amd.engine import _KvView
+    from vllm_omni_draft_amd.kv_cache import PagedKVCache
+    from vllm_omni_draft_amd.model_runner import DecoderModel
+    fp8 = kw.pop("fp8", False)
+    cfg = config.create_model_config(None, **{**dict(n_layers=2, hidden=256, n_heads=4, n_kv_heads=2, head_dim=64, ffn=512,
+                                                     vocab=512, max_pos=1024), **kw})
+    model = DecoderModel(weights.random_init(cfg, seed=3, fp8=fp8), 600, wide=True)
+    lens = [300, 1, 17, 129]
+    g = torch.Generator().manual_seed(5)
+    prompts = [torch.randint(0, cfg.vocab, (n,), generator=g).tolist() for n in lens]
+
+    def cache():
+        kv = PagedKVCache(cfg, PagedKVCache.pages_for(cfg, len(lens), 600), len(lens), 600)
+        for b, n in enumerate(lens):
+            kv.ensure_capacity(b, n)
+        return kv
+
+    one, two = cache(), cache()
+    got = torch.empty(len(lens), cfg.vocab, device="cuda")
+    # the first prompt in two pieces, the second piece behind the others
+    model.prompt(one, [(0, prompts[0][:280], 0, False)])
+    model.prompt(one, [(1, prompts[1], 0, True), (2, prompts[2], 0, True), (3, prompts[3], 0, True),
+                       (0, prompts[0][280:], 280, True)], got)
+    zero = torch.zeros(1, dtype=torch.int32, device="cuda")
+    for i, b in enumerate((1, 2, 3, 0)):
+        t = torch.tensor(prompts[b], dtype=torch.int32, device="cuda")
+        for c in range(0, lens[b], 200):
+            n = min(200, lens[b] - c)
+            out = torch.empty(n, cfg.vocab, device="cuda")
+            model.forward(_KvView(two, b), t, 0, c, zero, c, 1, n, out, wide=True)
+        assert torch.equal(got[i], out[-1]), b
+    assert torch.equal(one.k, two.k) and torch.equal(one.v, two.v)
+    with pytest.raises(Exception):
+        model.prompt(one, [(1, prompts[0], 0, True)], got)      # no pages for it

@@ -63,6 +63,12 @@ class ForwardArgs(C.Structure):
                 ("wide_a8", i32), ("argmax_val", vp), ("argmax_idx", vp)]
 
 
+class PromptArgs(C.Structure):
+    _fields_ = [("rows", i32), ("n_items", i32), ("n_out", i32), ("token_ids", vp), ("row_seq", vp), ("row_pos", vp),
+                ("items", vp), ("out_rows", vp), ("logits", vp), ("input_embeds", vp), ("rope_pos", vp), ("wide_a8", i32),
+                ("max_ctx", i32), ("split_tokens", i32)]
+
+
 class UniformRegion(C.Structure):
     _fields_ = [("offset", i64), ("n", i32), ("stride_j", i64), ("stride_b", i64)]
 
@@ -204,6 +210,9 @@ SIGNATURES = {
     "sd_model_create": (vp, [C.POINTER(ModelDesc)]),
     "sd_model_destroy": (None, [vp]),
     "sd_model_workspace_bytes": (C.c_size_t, [vp, i32, i32, i32]),
+    "sd_model_prompt_workspace_bytes": (C.c_size_t, [vp, i32]),
+    "sd_model_prompt": (i32, [vp, C.POINTER(KvCacheDesc), C.POINTER(PromptArgs), vp, C.c_size_t, vp]),
+    "sd_prompt_attention": (i32, [vp, i64, vp, vp, vp, i32, vp, i32, vp, i64, i32, i32, i32, C.c_float, i32, i32, vp]),
     "sd_model_forward": (i32, [vp, C.POINTER(KvCacheDesc), C.POINTER(ForwardArgs), vp,
                                C.c_size_t, vp]),
     "sd_store_proposal": (i32, [vp, vp, i32, i32, i32, vp]),

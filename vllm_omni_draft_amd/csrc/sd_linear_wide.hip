@@ -1098,6 +1098,39 @@ static int qkv_rope_wide_entry(const void* W, const float* w_scale, const float*
                      (hipStream_t)stream, x_scales);
 }
 
+// The rows of a prompt pass (any number; see sd_wide_epi.h): in one launch where sd_prompt.hip's kernels fit, else in
+// blocks of 256 rows, with the same bits.
+#if !defined(SD_WIDE_F32_ONLY)
+int sd_linear_rows_(const void* W, const float* w_scale, float* x_scales, const void* x, int64_t ldx, int M, int K,
+                    int n_tiles, int epi, const WideEpiArgs& all, void* workspace, size_t ws_bytes, sd_stream_t stream) {
+  hipStream_t st = (hipStream_t)stream;
+  const bool aligned = sd_aligned16(W) && sd_aligned16(x) && ldx % 8 == 0 && ldx >= K;
+  if (!w_scale && aligned && sd_prompt_linear_fits_(M, n_tiles, K, ldx))
+    return sd_prompt_linear_(W, x, ldx, M, K, n_tiles, epi, all, stream);
+  const size_t out_el = epi == SD_EPI_F32 ? 4 : 2;
+  for (int r0 = 0; r0 < M; r0 += 256) {
+    const int mm = min(256, M - r0);
+    WideEpiArgs e = all;
+    e.w_scale = w_scale;
+    e.out = (char*)all.out + (size_t)r0 * all.ldo * out_el;
+    if (e.residual) e.residual += (size_t)r0 * all.ldo;
+    if (epi == EPI_QKV_ROPE) {
+      e.rope.seq_lens += r0;
+      e.rope.row_seq += r0;
+      if (e.rope.mp.pos) e.rope.mp.pos += r0;
+    }
+    const bf16_t* xb = (const bf16_t*)x + (size_t)r0 * ldx;
+    if (x_scales) {
+      const int rc = sd_row_scales_fp8(xb, ldx, mm, K, x_scales, stream);
+      if (rc != SD_OK) return rc;
+    }
+    const int rc = wide_common(W, xb, ldx, mm, K, n_tiles, epi, e, workspace, ws_bytes, st, x_scales);
+    if (rc != SD_OK) return rc;
+  }
+  return SD_OK;
+}
+#endif
+
 extern "C" int sd_qkv_rope_wide(const void* W, const float* w_scale, const void* x, int64_t ldx,
                                 const void* bias,
                                 void* q_out, int64_t ldq, const float* rope_cs, int max_pos,

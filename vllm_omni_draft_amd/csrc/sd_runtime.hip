@@ -7,6 +7,7 @@
 #include <vector>
 
 #include "sd_common.h"
+#include "sd_wide_epi.h"
 #include <rccl/rccl.h>
 
 struct sd_model {
@@ -445,6 +446,136 @@ extern "C" int sd_model_forward(sd_model* m, const sd_kv_cache* kv, const sd_for
     SD_REQUIRE(a->logits, SD_ERR_INVALID,
                "sd_model_forward: this pass's shape needs `logits` for the slice maxima");
     SD_TRY(sd_argmax_partial(a->logits, lm_vocab, a->argmax_val, a->argmax_idx, rows, lm_vocab, stream));
+  }
+  return SD_OK;
+}
+
+// ------------------------------------------------------------------ prompt passes
+namespace {
+
+struct PromptWs {
+  size_t h, xn, q, attn, act, out_h, wide_ws, wide_ws_bytes, x_scales, total;
+};
+
+PromptWs plan_prompt(const sd_model_desc& d, int rows) {
+  PromptWs w;
+  const size_t R = (size_t)rows, QD = (size_t)d.n_heads * d.head_dim;
+  const int H = d.hidden, F = d.ffn, V = d.lm_vocab > 0 ? d.lm_vocab : d.vocab;
+  const int b = rows < 256 ? rows : 256;
+  const int up_epi = d.arch == SD_ARCH_LLAMA ? SD_EPI_SILU_MUL : SD_EPI_RELU;
+  size_t off = 0;
+  w.h = off;    off += align256(R * H * 2);
+  w.xn = off;   off += align256(R * H * 2);
+  w.q = off;    off += align256(R * QD * 2);
+  w.attn = off; off += align256(R * QD * 2);
+  w.act = off;  off += align256(R * F * 2);
+  w.out_h = off; off += align256((size_t)256 * H * 2);
+  const size_t need[5] = {
+      sd_linear_wide_workspace_bytes(b, (d.n_heads + 2 * d.n_kv_heads) * d.head_dim, H, SD_EPI_STORE),
+      sd_linear_wide_workspace_bytes(b, H, (int)QD, SD_EPI_RESIDUAL),
+      sd_linear_wide_workspace_bytes(b, F, H, up_epi),
+      sd_linear_wide_workspace_bytes(b, H, F, SD_EPI_RESIDUAL),
+      sd_linear_wide_workspace_bytes(b, V, H, SD_EPI_F32)};
+  w.wide_ws_bytes = 256;
+  for (size_t n : need) w.wide_ws_bytes = n > w.wide_ws_bytes ? n : w.wide_ws_bytes;
+  w.wide_ws = off; off += align256(w.wide_ws_bytes);
+  w.x_scales = off; off += align256((size_t)2 * 256 * sizeof(float));
+  w.total = off;
+  return w;
+}
+
+__global__ __launch_bounds__(256) void gather_rows_kernel(const u32x4* __restrict__ in, const int32_t* __restrict__ rows,
+                                                          u32x4* __restrict__ out, int n16, int n_rows) {
+  const int row = rows[blockIdx.x];
+  if (row < 0 || row >= n_rows) return;
+  for (int i = threadIdx.x; i < n16; i += 256) out[(size_t)blockIdx.x * n16 + i] = in[(size_t)row * n16 + i];
+}
+
+}  // namespace
+
+extern "C" size_t sd_model_prompt_workspace_bytes(const sd_model* m, int max_rows) {
+  return !m || max_rows < 1 ? 0 : plan_prompt(m->d, max_rows).total;
+}
+
+extern "C" int sd_model_prompt(sd_model* m, const sd_kv_cache* kv, const sd_prompt_args* a, void* workspace,
+                               size_t workspace_bytes, sd_stream_t stream) {
+  SD_REQUIRE(m && kv && a && workspace, SD_ERR_INVALID, "sd_model_prompt: null argument");
+  const sd_model_desc& d = m->d;
+  const int rows = a->rows, H = d.hidden, D = d.head_dim, Hq = d.n_heads, Hkv = d.n_kv_heads, F = d.ffn, QD = Hq * D;
+  const bool llama = d.arch == SD_ARCH_LLAMA;
+  SD_REQUIRE(rows >= 1 && rows <= (1 << 20) && a->n_items >= 1 && a->n_out >= 0 && a->n_out <= 256 && a->n_out <= rows,
+             SD_ERR_INVALID,
+             "sd_model_prompt: %d rows in %d items, %d wanted", rows, a->n_items, a->n_out);
+  SD_REQUIRE((a->token_ids || a->input_embeds) && a->row_seq && a->row_pos && a->items && kv->k_cache && kv->v_cache &&
+                 kv->block_tables && (a->n_out == 0 || (a->out_rows && a->logits)),
+             SD_ERR_INVALID, "sd_model_prompt: null buffer");
+  SD_REQUIRE(!d.allreduce, SD_ERR_UNSUPPORTED, "sd_model_prompt: tensor-parallel models take sd_model_forward");
+  const bool mrope = d.mrope_section_t || d.mrope_section_h;
+  SD_REQUIRE(mrope || !a->rope_pos, SD_ERR_INVALID, "sd_model_prompt: rotary positions given to a model without sections");
+  SD_REQUIRE(llama || !a->input_embeds, SD_ERR_UNSUPPORTED, "sd_model_prompt: input_embeds need a rotary model");
+  const PromptWs w = plan_prompt(d, rows);
+  SD_REQUIRE(workspace_bytes >= w.total, SD_ERR_WORKSPACE, "sd_model_prompt: workspace %zu < %zu bytes", workspace_bytes,
+             w.total);
+  SD_REQUIRE(sd_aligned16(workspace), SD_ERR_INVALID, "sd_model_prompt: workspace unaligned");
+  char* base = (char*)workspace;
+  void *h = base + w.h, *xn = base + w.xn, *q = base + w.q, *attn = base + w.attn, *act = base + w.act;
+  float* xsc = reinterpret_cast<float*>(base + w.x_scales);
+  if (a->input_embeds) {
+    const hipError_t e = hipMemcpyAsync(h, a->input_embeds, (size_t)rows * H * 2, hipMemcpyDeviceToDevice, (hipStream_t)stream);
+    SD_REQUIRE(e == hipSuccess, SD_ERR_HIP, "sd_model_prompt: copying input_embeds: %s", hipGetErrorString(e));
+  } else {
+    SD_TRY(sd_embed(a->token_ids, 1, 0, d.embed, d.embed_tiled, d.pos_table, d.pos_bias, a->row_pos, 0, h, rows, 1, H,
+                    d.vocab, stream));
+  }
+  const sd_rope_positions rp{a->rope_pos, nullptr, d.mrope_section_t, d.mrope_section_h};
+  auto norm = [&](const void* in, const void* g, const void* b, void* out, int n) {
+    return llama ? sd_rmsnorm(in, H, g, out, H, n, H, d.norm_eps, stream)
+                 : sd_layernorm(in, H, g, b, out, H, n, H, d.norm_eps, stream);
+  };
+  auto linear = [&](const void* W, const float* s, bool a8, const void* x, int K, const void* bias, const void* res, void* out,
+                    int64_t ldo, int M, int N, int epi) {
+    WideEpiArgs e{};
+    e.N = N;
+    e.bias = (const bf16_t*)bias;
+    e.residual = (const bf16_t*)res;
+    e.out = out;
+    e.ldo = ldo;
+    return sd_linear_rows_(W, s, a8 ? xsc : nullptr, x, K, M, K, tiles_of(N, epi), epi, e, base + w.wide_ws, w.wide_ws_bytes,
+                           stream);
+  };
+  for (int li = 0; li < d.n_layers; ++li) {
+    const sd_layer_weights& l = m->layers[li];
+    void* kc = (char*)kv->k_cache + (size_t)li * kv->layer_stride_bytes;
+    void* vc = (char*)kv->v_cache + (size_t)li * kv->layer_stride_bytes;
+    const bool a8 = a->wide_a8 && llama && l.qkv_s && l.o_s && l.up_s && l.down_s && H % 128 == 0 && F % 128 == 0 &&
+                    QD % 128 == 0;
+    SD_TRY(norm(h, l.attn_norm_w, l.attn_norm_b, xn, rows));
+    WideEpiArgs e{};
+    e.N = QD + 2 * Hkv * D;
+    e.bias = (const bf16_t*)l.qkv_b;
+    e.out = q;
+    e.ldo = QD;
+    e.rope = WideRope{llama ? d.rope_cs : nullptr, d.max_pos, (bf16_t*)kc, (bf16_t*)vc, kv->block_tables,
+                      kv->max_blocks_per_seq, a->row_pos, 0, 1, Hq, Hkv, D,
+                      sd_make_rope_pos(mrope && a->rope_pos ? &rp : nullptr, rows), a->row_seq};
+    SD_TRY(sd_linear_rows_(l.qkv_w, l.qkv_s, a8 ? xsc : nullptr, xn, H, rows, H, e.N / 16, EPI_QKV_ROPE, e, base + w.wide_ws,
+                           w.wide_ws_bytes, stream));
+    SD_TRY(sd_prompt_attention(q, QD, kc, vc, kv->block_tables, kv->max_blocks_per_seq, a->items, a->n_items, attn, QD, Hq,
+                               Hkv, D, d.attn_scale, a->max_ctx, a->split_tokens, stream));
+    SD_TRY(linear(l.o_w, l.o_s, a8, attn, QD, l.o_b, h, h, H, rows, H, SD_EPI_RESIDUAL));
+    SD_TRY(norm(h, l.mlp_norm_w, l.mlp_norm_b, xn, rows));
+    SD_TRY(linear(l.up_w, l.up_s, a8, xn, H, l.up_b, nullptr, act, F, rows, F, llama ? SD_EPI_SILU_MUL : SD_EPI_RELU));
+    SD_TRY(linear(l.down_w, l.down_s, a8, act, F, l.down_b, h, h, H, rows, H, SD_EPI_RESIDUAL));
+  }
+  if (a->n_out) {
+    void* oh = base + w.out_h;
+    hipLaunchKernelGGL(gather_rows_kernel, dim3(a->n_out), dim3(256), 0, (hipStream_t)stream, (const u32x4*)h, a->out_rows,
+                       (u32x4*)oh, H / 8, rows);
+    SD_CHECK_LAUNCH("sd_model_prompt(gather)");
+    SD_TRY(norm(oh, d.final_norm_w, d.final_norm_b, xn, a->n_out));
+    const int V = d.lm_vocab > 0 ? d.lm_vocab : d.vocab;
+    SD_TRY(linear(d.lm_head, d.lm_head_s, a->wide_a8 && llama && d.lm_head_s && H % 128 == 0, xn, H, nullptr, nullptr,
+                  a->logits, V, a->n_out, V, SD_EPI_F32));
   }
   return SD_OK;
 }

@@ -3,7 +3,7 @@
 #pragma once
 #include "sd_common.h"
 
-namespace {
+namespace sd_wide {
 
 constexpr int EPI_QKV_ROPE = 100;
 
@@ -226,10 +226,17 @@ __device__ __forceinline__ void emit_unit(const WideEpiArgs& a, int m, int tile,
   }
 }
 
-}  // namespace
+}  // namespace sd_wide
+using namespace sd_wide;
 
 // sd_prompt.hip: the shapes its kernels are the better choice for (every other call goes through sd_linear_wide's in
 // blocks of 256 rows; same bits), and the call.  epi: an SD_EPI_* number or EPI_QKV_ROPE with what that reads in `e`.
 bool sd_prompt_linear_fits_(int M, int n_tiles, int K, int64_t ldx);
 int sd_prompt_linear_(const void* W, const void* x, int64_t ldx, int M, int K, int n_tiles, int epi,
                       const WideEpiArgs& e, sd_stream_t stream);
+
+// sd_linear_wide.hip: a linear layer over the rows of a prompt pass.  `e` holds what the epilogue reads (bias,
+// residual, out, ldo, N; for EPI_QKV_ROPE the rope with one block-table row and position per row); w_scale: fp8
+// weights; x_scales (2 x 256 floats): activations quantised per row as well.  workspace: of 256 rows.
+int sd_linear_rows_(const void* W, const float* w_scale, float* x_scales, const void* x, int64_t ldx, int M, int K,
+                    int n_tiles, int epi, const WideEpiArgs& e, void* workspace, size_t ws_bytes, sd_stream_t stream);

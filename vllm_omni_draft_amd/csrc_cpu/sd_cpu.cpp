@@ -1002,6 +1002,14 @@ extern "C" int sd_row_scales_fp8(const void*, int64_t, int, int, float*, sd_stre
 }
 extern "C" int sd_linear_prompt(const void*, const void*, int64_t, const void*, const void*, void*, int64_t, int, int,
                                 int, int, sd_stream_t) { UNSUPPORTED("sd_linear_prompt"); }
+extern "C" int sd_prompt_attention(const void*, int64_t, const void*, const void*, const int32_t*, int, const int32_t*, int,
+                                   void*, int64_t, int, int, int, float, int, int, sd_stream_t) {
+  UNSUPPORTED("sd_prompt_attention");
+}
+extern "C" size_t sd_model_prompt_workspace_bytes(const sd_model*, int) { return 0; }
+extern "C" int sd_model_prompt(sd_model*, const sd_kv_cache*, const sd_prompt_args*, void*, size_t, sd_stream_t) {
+  UNSUPPORTED("sd_model_prompt");
+}
 extern "C" int sd_linear_wide_a8(const void*, const float*, const float*, const void*, int64_t, const void*,
                                  const void*, void*, int64_t, int, int, int, int, void*, size_t, sd_stream_t) {
   set_error("sd_linear_wide_a8: not available in the CPU build");

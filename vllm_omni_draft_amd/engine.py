@@ -728,45 +728,61 @@ class SpecEngine:
 
     def _prefill_range(self, slot: int, prompt: Sequence[int], c_from: int, c_to: int, final: bool,
                        rope_positions=None, input_embeds=None, decoded_from: Optional[int] = None) -> None:
-        """Passes over prompt tokens c_from..c_to-1 of the sequence in `slot` (both models, chunks
-        of prefill_rows tokens on the wide family).  final: c_to is the prompt's end; its last
-        token gets a pass of its own whose logits (target) land in t_out[0].
+        """Passes over prompt tokens c_from..c_to-1 of the sequence in `slot` (both models: prompt passes,
+        or forward passes of prefill_rows tokens on the wide family where a model has none).  final: c_to
+        is the prompt's end; its last token's logits (target) land in t_out[0].
         decoded_from: tokens from this position on were first computed by decode passes (the
         sequence is being rebuilt from its own output): a model whose decode passes run on the
-        narrow family recomputes them in narrow passes of at most a decode pass's rows.  A narrow
+        narrow family recomputes them in narrow passes of at most a decode pass's rows.  A
         row's bits depend on nothing else in its pass, so the cache entries equal those the
         decode passes wrote, whatever the grouping was then."""
         n = len(prompt)
-        self.prompt_buf[c_from:c_to].copy_(torch.tensor(list(prompt[c_from:c_to]), dtype=torch.int32))
         self._ctx = self._ctx_bucket(n + self._slack)
-        zl = self.zero_lens[slot:slot + 1]
-        body_end = c_to - 1 if final else c_to
         for model, kv in ((self.target, self.t_kv), (self.draft, self.d_kv)):
             if model is None:
                 continue
-            # only the last token's logits are needed, so the prompt ends with a 1-token pass
-            chunk = model.prefill_rows
-            wide = chunk > MAX_ROWS or self.wide
-            narrow_from = n if decoded_from is None or model.wide else max(int(decoded_from), 0)
-            narrow_rows = min(MAX_ROWS, 64 // (model.cfg.n_heads // model.cfg.n_kv_heads))
-            wide_end = min(body_end, narrow_from)
-            passes = [(c0, min(c0 + chunk, wide_end), wide) for c0 in range(c_from, wide_end, chunk)]
-            passes += [(c0, min(c0 + narrow_rows, body_end), False)
-                       for c0 in range(max(c_from, wide_end), body_end, narrow_rows)]
-            if final:
-                passes.append((body_end, c_to, wide and narrow_from >= n))
-            for c0, c1, family_wide in passes:
-                if c1 <= c0:
-                    continue
-                want = final and c1 == n and model is self.target
-                view = _KvView(kv, slot)
-                mm = {}
-                if rope_positions is not None and model.cfg.mrope_section:
-                    mm["rope_pos"] = rope_positions[:, c0:c1].contiguous()
-                if input_embeds is not None and model is self.target:
-                    mm["input_embeds"] = input_embeds[c0:c1].contiguous()
-                model.forward(view, self.prompt_buf, 0, c0, zl, c0, 1, c1 - c0,
-                              self.t_out[:c1 - c0] if want else None, self._ctx, wide=family_wide, **mm)
+            narrow_from = n if decoded_from is None or model.wide else min(max(int(decoded_from), 0), n)
+            logits = self.t_out if model is self.target else None
+            embeds = input_embeds if model is self.target else None
+            positions = rope_positions if model.cfg.mrope_section else None
+            c_done = c_from
+            if model.packs_prompts and c_from < min(c_to, narrow_from):
+                c_done = min(c_to, narrow_from)
+                want = final and c_done == n and model is self.target
+                model.prompt(kv, [(slot, prompt[c_from:c_done], c_from, want)], logits if want else None,
+                             None if embeds is None else embeds[c_from:c_done].contiguous(),
+                             None if positions is None else positions[:, c_from:c_done])
+            if c_done < c_to:
+                self._forward_range(model, kv, slot, prompt, c_done, c_to, final, positions, embeds, narrow_from)
+
+    def _forward_range(self, model, kv, slot, prompt, c_from, c_to, final, rope_positions, input_embeds,
+                       narrow_from: int) -> None:
+        """_prefill_range by forward passes, the wide family up to narrow_from, the narrow one from there on."""
+        n = len(prompt)
+        self.prompt_buf[c_from:c_to].copy_(torch.tensor(list(prompt[c_from:c_to]), dtype=torch.int32))
+        zl = self.zero_lens[slot:slot + 1]
+        body_end = c_to - 1 if final else c_to
+        # only the last token's logits are needed, so the prompt ends with a 1-token pass
+        chunk = model.prefill_rows
+        wide = chunk > MAX_ROWS or self.wide
+        narrow_rows = min(MAX_ROWS, 64 // (model.cfg.n_heads // model.cfg.n_kv_heads))
+        wide_end = min(body_end, narrow_from)
+        passes = [(c0, min(c0 + chunk, wide_end), wide) for c0 in range(c_from, wide_end, chunk)]
+        passes += [(c0, min(c0 + narrow_rows, body_end), False)
+                   for c0 in range(max(c_from, wide_end), body_end, narrow_rows)]
+        if final:
+            passes.append((body_end, c_to, wide and narrow_from >= n))
+        for c0, c1, family_wide in passes:
+            if c1 <= c0:
+                continue
+            want = final and c1 == n and model is self.target
+            mm = {}
+            if rope_positions is not None:
+                mm["rope_pos"] = rope_positions[:, c0:c1].contiguous()
+            if input_embeds is not None:
+                mm["input_embeds"] = input_embeds[c0:c1].contiguous()
+            model.forward(_KvView(kv, slot), self.prompt_buf, 0, c0, zl, c0, 1, c1 - c0,
+                          self.t_out[:c1 - c0] if want else None, self._ctx, wide=family_wide, **mm)
 
     def _add_request(self, slot: int, prompt: Sequence[int], input_embeds=None,
                      rope_positions=None, seed: Optional[int] = None, start: int = 0,
@@ -834,9 +850,9 @@ class SpecEngine:
                      biases: Optional[Sequence[Optional[dict]]] = None) -> List[int]:
         """Prefills several text prompts in the same passes and returns their first tokens (one
         synchronisation for all of them).  The prompts take the next free slots in order.
-        Every pass carries a chunk of each prompt (prefill_rows // len(prompts) tokens per
-        sequence, wide kernel family); rows past the end of a shorter prompt are padding whose
-        cache entries are overwritten before anything reads them.  A row's bits do not depend
+        The prompts' rows go one behind the other through prompt passes (a model without them: forward
+        passes that carry a chunk of each prompt, rows past the end of a shorter one being padding whose
+        cache entries are overwritten before anything reads them).  A row's bits do not depend
         on what shares its pass, so the streams equal those of add_request called once per
         prompt."""
         with _rt.stream_ctx(self.stream):
@@ -893,38 +909,22 @@ class SpecEngine:
             if self.logprobs_top is not None:
                 self.last_logprobs = lp
             return out
-        if self._prompt_rows is None or self._prompt_rows.shape[0] < Bp:
-            self._prompt_rows = torch.zeros(self.cfg.max_batch, max(self.cfg.max_seq_len, 8),
-                                            dtype=torch.int32, device=self.device)
-        stride = self._prompt_rows.shape[1]
-        host = torch.zeros(Bp, n_max, dtype=torch.int32)
-        for i, p in enumerate(prompts):
-            host[i, :lens[i]] = torch.tensor(p, dtype=torch.int32)
-        self._prompt_rows[:Bp, :n_max].copy_(host)
         last = torch.tensor([p[-1] for p in prompts], dtype=torch.int32).to(self.device)
         lens_dev = torch.tensor(lens, dtype=torch.int32).to(self.device)
-        for i in range(Bp):
-            # padding rows write up to n_max - 2 in every sequence's cache
-            self.t_kv.ensure_capacity(slot0 + i, n_max + self._slack)
-            if self.d_kv is not None:
-                self.d_kv.ensure_capacity(slot0 + i, n_max + self._slack)
+        models = [(m, kv) for m, kv in ((self.target, self.t_kv), (self.draft, self.d_kv)) if m is not None]
+        for m, kv in models:
+            for i in range(Bp):
+                # (padding rows of forward passes write up to n_max - 2 in every sequence's cache)
+                kv.ensure_capacity(slot0 + i, (lens[i] if m.packs_prompts else n_max) + self._slack)
         self.rope_delta[slot0:slot0 + Bp] = 0
         self._ctx = self._ctx_bucket(n_max + self._slack)
-        zl = self.zero_lens[slot0:slot0 + Bp]
-        toks = self._prompt_rows.view(-1)
-        for model, kv in ((self.target, self.t_kv), (self.draft, self.d_kv)):
-            if model is None:
-                continue
-            view = _KvView(kv, slot0)
-            # all but each prompt's last token, in chunks: no logits wanted
-            chunk = max(1, model.prefill_rows // Bp)
-            wide = model.prefill_rows > MAX_ROWS or self.wide    # the family add_request uses
-            for c0 in range(0, n_max - 1, chunk):
-                model.forward(view, toks, stride, c0, zl, c0, Bp, min(chunk, n_max - 1 - c0), None,
-                              self._ctx, wide=wide)
-            # every prompt's last token at its own position
-            model.forward(view, last, 1, 0, lens_dev, -1, Bp, 1,
-                          self.t_out[:Bp] if model is self.target else None, self._ctx, wide=wide)
+        for model, kv in models:
+            if model.packs_prompts:   # the prompts' rows one behind the other
+                target = model is self.target
+                model.prompt(kv, [(slot0 + i, p, 0, target) for i, p in enumerate(prompts)],
+                             self.t_out[:Bp] if target else None)
+            else:
+                self._forward_prompts(model, kv, slot0, prompts, last, lens_dev)
         self._apply_bias(Bp, 1, slot0=slot0)
         if self.sampling:
             self._target_full_rows(Bp)
@@ -954,6 +954,29 @@ class SpecEngine:
         if self.logprobs_top is not None:
             self._logprob_rows([[i] for i in range(Bp)], [[t] for t in firsts])
         return firsts
+
+    def _forward_prompts(self, model, kv, slot0: int, prompts, last, lens_dev) -> None:
+        """Several prompts by forward passes that carry a chunk of each (padding past a shorter prompt's end)."""
+        Bp, n_max = len(prompts), max(len(p) for p in prompts)
+        if self._prompt_rows is None or self._prompt_rows.shape[0] < Bp:
+            self._prompt_rows = torch.zeros(self.cfg.max_batch, max(self.cfg.max_seq_len, 8),
+                                            dtype=torch.int32, device=self.device)
+        stride = self._prompt_rows.shape[1]
+        host = torch.zeros(Bp, n_max, dtype=torch.int32)
+        for i, p in enumerate(prompts):
+            host[i, :len(p)] = torch.tensor(p, dtype=torch.int32)
+        self._prompt_rows[:Bp, :n_max].copy_(host)
+        view = _KvView(kv, slot0)
+        zl = self.zero_lens[slot0:slot0 + Bp]
+        # all but each prompt's last token, in chunks: no logits wanted
+        chunk = max(1, model.prefill_rows // Bp)
+        wide = model.prefill_rows > MAX_ROWS or self.wide    # the family add_request uses
+        for c0 in range(0, n_max - 1, chunk):
+            model.forward(view, self._prompt_rows.view(-1), stride, c0, zl, c0, Bp, min(chunk, n_max - 1 - c0), None,
+                          self._ctx, wide=wide)
+        # every prompt's last token at its own position
+        model.forward(view, last, 1, 0, lens_dev, -1, Bp, 1,
+                      self.t_out[:Bp] if model is self.target else None, self._ctx, wide=wide)
 
     # ------------------------------------------------------------------ log-probabilities
     def _logprob_rows(self, rows: List[List[int]], toks: List[List[int]]) -> None:

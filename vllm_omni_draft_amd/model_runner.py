@@ -8,16 +8,18 @@ from __future__ import annotations
 import ctypes as C
 from typing import Optional
 
+import numpy as np
 import torch
 
 from . import _lib, ops
 from .config import ModelConfig
-from .kv_cache import PagedKVCache
+from .kv_cache import PAGE, PagedKVCache
 from .weights import ModelWeights
 
 MAX_ROWS = 16        # token rows one forward pass may carry (B * q_len), narrow kernel family
 MAX_ROWS_WIDE = 256  # the same for the wide family (batched draft passes / verify)
 PREFILL_ROWS = 256   # prompt tokens of one sequence per prefill pass (wide family)
+PROMPT_ROWS = 4096   # token rows per prompt pass (DecoderModel.prompt)
 
 
 def _ptr(t):
@@ -46,6 +48,11 @@ class DecoderModel:
         # tokens per pass): every engine prefills the same way, so streams stay comparable.
         self.prefill_rows = PREFILL_ROWS if (wide or wide_prefill) else min(
             MAX_ROWS, 64 // (cfg.n_heads // cfg.n_kv_heads))
+        # Prompts go through prompt() on the GPU build; tensor-parallel models, whose all-reduce buffers are sized for
+        # the rows of a forward pass, keep to forward() in chunks of prefill_rows.
+        self.packs_prompts = (ops.on_gpu() and tp_group is None and bool(wide or wide_prefill)
+                              and ops.prompt_attention_fits(max_ctx, split_tokens))
+        self._prompt_ws: Optional[torch.Tensor] = None
         if max_ctx > cfg.max_pos:
             raise ValueError(f"max_ctx {max_ctx} exceeds the model's max_pos {cfg.max_pos}")
         self.max_ctx = max_ctx
@@ -198,6 +205,77 @@ class DecoderModel:
                                           ws.data_ptr(), ws.numel(),
                                           ops._stream())
         _lib.check(rc, "sd_model_forward")
+
+
+    def prompt(self, kv: PagedKVCache, runs, logits: Optional[torch.Tensor] = None,
+               input_embeds: Optional[torch.Tensor] = None, rope_pos: Optional[torch.Tensor] = None) -> None:
+        """Enqueues prompt tokens on the current stream: runs = [(cache slot, tokens, position of the first, whether
+        the last one's logits are wanted)], their rows one behind the other in passes of at most PROMPT_ROWS.  The
+        cache must hold pages for every position.  logits (f32 [wanted, head rows]) receives the wanted rows in the
+        order of the runs.  input_embeds [rows, hidden] bf16 and rope_pos [3, rows] int32 as for forward().  A row has
+        the bits that a forward() of the wide family gives it."""
+        if not self.packs_prompts:
+            raise _lib.SdError("this model's prompts go through forward()")
+        runs = [(int(slot), np.asarray(toks, dtype=np.int32), int(pos), bool(want)) for slot, toks, pos, want in runs]
+        total = sum(len(t) for _, t, _, _ in runs)
+        wanted = sum(w for _, _, _, w in runs)
+        if any(len(t) < 1 or pos < 0 or pos + len(t) > self.max_ctx or not 0 <= slot < kv.block_tables.shape[0]
+               for slot, t, pos, _ in runs):
+            raise ValueError(f"a run needs a cache slot and tokens at positions 0..{self.max_ctx - 1}")
+        if any(len(kv.pages_of(slot)) * PAGE < pos + len(t) for slot, t, pos, _ in runs):
+            raise _lib.SdError("the cache has no pages for some of the tokens")
+        if wanted and (logits is None or logits.dtype != torch.float32 or not logits.is_contiguous()
+                       or logits.numel() < wanted * self.cfg.head_rows):
+            raise _lib.SdError("wanted rows need contiguous float32 logits [wanted, head rows]")
+        if input_embeds is not None and (input_embeds.dtype != torch.bfloat16 or not input_embeds.is_contiguous()
+                                         or tuple(input_embeds.shape) != (total, self.cfg.hidden)):
+            raise _lib.SdError("input_embeds must be a contiguous bfloat16 [rows, hidden] tensor")
+        if rope_pos is not None and (rope_pos.dtype != torch.int32 or tuple(rope_pos.shape) != (3, total)
+                                     or not self.cfg.mrope_section):
+            raise _lib.SdError("rope_pos: int32 [3, rows], for a model with mrope_section")
+        block = ops.PROMPT_BLOCK_ROWS // (self.cfg.n_heads // self.cfg.n_kv_heads)
+        done = out_at = at = 0        # rows of earlier passes, wanted rows of earlier passes, tokens of runs[0] done
+        runs = list(runs)
+        while runs:
+            toks, seq, pos, items, out_rows, rows = [], [], [], [], [], 0
+            while runs and rows < PROMPT_ROWS and len(out_rows) < MAX_ROWS_WIDE:
+                slot, t, p0, want = runs[0]
+                n = min(len(t) - at, PROMPT_ROWS - rows)
+                toks.append(t[at:at + n])
+                seq.append(np.full(n, slot, np.int32))
+                pos.append(np.arange(p0 + at, p0 + at + n, dtype=np.int32))
+                items += [(rows + i, min(block, n - i), slot, p0 + at + i) for i in range(0, n, block)]
+                rows += n
+                at += n
+                if at == len(t):
+                    if want:
+                        out_rows.append(rows - 1)
+                    runs.pop(0)
+                    at = 0
+            items.sort(key=lambda i: -i[3])    # the longest first: they take longest
+            host = np.concatenate([np.asarray(items, np.int32).reshape(-1), *toks, *seq, *pos,
+                                   np.asarray(out_rows, np.int32)])
+            dev = torch.from_numpy(host).to(kv.block_tables.device)
+            need = int(_lib.load().sd_model_prompt_workspace_bytes(self._handle, rows))
+            if self._prompt_ws is None or self._prompt_ws.numel() < need:
+                self._prompt_ws = torch.empty(need, dtype=torch.uint8, device=dev.device)
+            o, rp = 4 * len(items), None if rope_pos is None else rope_pos[:, done:done + rows].contiguous()
+            kvd = _lib.KvCacheDesc(k_cache=kv.k.data_ptr(), v_cache=kv.v.data_ptr(),
+                                   layer_stride_bytes=kv.layer_stride_bytes, block_tables=kv.block_tables.data_ptr(),
+                                   max_blocks_per_seq=kv.max_blocks_per_seq)
+            args = _lib.PromptArgs(
+                rows=rows, n_items=len(items), n_out=len(out_rows), token_ids=dev[o:].data_ptr(),
+                row_seq=dev[o + rows:].data_ptr(), row_pos=dev[o + 2 * rows:].data_ptr(), items=dev.data_ptr(),
+                out_rows=dev[o + 3 * rows:].data_ptr() if out_rows else None,
+                logits=logits.data_ptr() + 4 * out_at * self.cfg.head_rows if out_rows else None,
+                input_embeds=None if input_embeds is None else input_embeds[done:].data_ptr(), rope_pos=_ptr(rp),
+                wide_a8=int(self.fp8_activations), max_ctx=max(i[3] + i[1] for i in items),
+                split_tokens=self.split_tokens)
+            _lib.check(_lib.load().sd_model_prompt(self._handle, C.byref(kvd), C.byref(args),
+                                                   self._prompt_ws.data_ptr(), self._prompt_ws.numel(), ops._stream()),
+                       "sd_model_prompt")
+            done += rows
+            out_at += len(out_rows)
 
 
 # ---------------------------------------------------------------------------------------------

@@ -611,6 +611,26 @@ def linear_wide(W, x, bias=None, residual=None, epilogue=EPI_STORE, out=None,
     return out
 
 
+PROMPT_BLOCK_ROWS = 128   # query rows of one KV head in a workgroup of sd_prompt_attention
+
+
+def prompt_attention_fits(max_ctx: int, split_tokens: int) -> bool:
+    """Whether sd_prompt_attention takes this split size and context (its table of the splits' maxima lies in LDS)."""
+    return split_tokens in (128, 256) and -(-max_ctx // split_tokens) * PROMPT_BLOCK_ROWS * 4 <= 88 * 1024
+
+
+def prompt_attention(q, k_cache, v_cache, block_tables, items, Hq, Hkv, D, scale, max_ctx, split_tokens) -> torch.Tensor:
+    """Attention of prompt rows q [rows, Hq * D] (sd_prompt_attention); items: int32 [n, 4] device tensor of {first row,
+    tokens, row of block_tables, first position}."""
+    _need(q, torch.bfloat16, "q")
+    _need(items, torch.int32, "items")
+    out = torch.zeros_like(q)
+    _lib.check(_lib.load().sd_prompt_attention(_p(q), q.stride(0), _p(k_cache), _p(v_cache), _p(block_tables),
+                                               block_tables.shape[1], _p(items), items.shape[0], _p(out), out.stride(0),
+                                               Hq, Hkv, D, scale, max_ctx, split_tokens, _stream()), "sd_prompt_attention")
+    return out
+
+
 def linear_prompt(W, x, bias=None, residual=None, epilogue=EPI_STORE, out=None) -> torch.Tensor:
     """linear() for the many rows of a prompt pass (sd_linear_prompt: bf16 weights, K a multiple of 64 from 128 up);
     a row has the bits linear_wide gives it."""

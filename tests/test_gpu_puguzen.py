@@ -575,3 +575,21 @@ def test_sampling_through_the_worker_is_seeded_per_request():
     alone, among = run(0), run(3)
     assert len(alone) == 10 and alone == among
     assert len(set(alone)) > 2
+
+
+@pytest.mark.parametrize("wdt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K", [(17, 33, 4), (64, 64, 32), (65, 130, 100), (200, 1000, 644), (2049, 2060, 72)])
+def test_matmul_rows_on_the_matrix_instruction_has_the_bits_of_few_rows(M, N, K, wdt):
+    """More than 16 rows (blocks of 64 and of 128, remainders of both and of the 32 columns of a stage) against the same
+    rows 16 at a time, which run on the vector pipe: sums over k in ascending order by fused multiply-adds either way."""
+    from vllm_omni_draft_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    x = torch.randn(M, K, generator=g, device="cuda")
+    x2 = torch.randn(M, K, generator=g, device="cuda")
+    w = torch.randn(N, K, generator=g, device="cuda").to(wdt)
+    b = torch.randn(N, generator=g, device="cuda")
+    for bias, up in ((None, None), (b, x2)):
+        got = ops.matmul_rows(x, w, bias, up)
+        few = torch.cat([ops.matmul_rows(x[i:i + 16].contiguous(), w, bias, None if up is None else up[i:i + 16].contiguous())
+                         for i in range(0, M, 16)])
+        assert torch.equal(got, few)

@@ -721,6 +721,132 @@ __global__ __launch_bounds__(256) void matmul_skinny_kernel(
   if (Yb) Yb[n] = (bf16_t)o;
 }
 
+// The same product for more rows, on the f32 matrix instruction: v_mfma_f32_32x32x2_f32 is two fused multiply-adds in
+// ascending k for every element, so the sums are matmul_rows_kernel's to the bit (tests compare them).  Four waves, NT x
+// MT tiles of 32 x 32 each; 32 columns of K a stage, through registers into two LDS buffers.  A row's 32 values lie
+// as 16 of even k, then 16 of odd k: the lanes of an instruction's first k read the former, those of its second the
+// latter, four instructions' worth in one 16-byte read.  Bound by the matrix pipe (64 FLOP a clock and SIMD): 777 x
+// 13312 x 1024 ran at 20 TFLOP/s on the vector pipe, whose inner loop read as many LDS words as it multiplied.
+constexpr int kMmK = 32, kMmLd = kMmK + 4;
+template <typename T, int NT, int MT>
+__global__ __launch_bounds__(256, 2) void matmul_mfma_kernel(
+    const float* __restrict__ X, const float* __restrict__ X2, int64_t ldx, const T* __restrict__ Wt,
+    const float* __restrict__ bias, float* __restrict__ Y, int64_t ldy, int M, int N, int K, int round,
+    int64_t bx, int64_t bw, int64_t by, bf16_t* __restrict__ Yb) {
+  constexpr int BN = 64 * NT, BM = 64 * MT;
+  constexpr int kWPieces = BN * (kMmK / 4) / 256, kXPieces = BM * (kMmK / 4) / 256;  // four values each
+  __shared__ __attribute__((aligned(16))) float lds[2][(BN + BM) * kMmLd];
+  X += (size_t)blockIdx.z * bx;
+  Wt += (size_t)blockIdx.z * bw;
+  Y += (size_t)blockIdx.z * by;
+  if (Yb) Yb += (size_t)blockIdx.z * by;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int r = lane & 31, h = lane >> 5, wn = wave & 1, wm = wave >> 1;
+  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+  f32x4 wv[kWPieces], xv[kXPieces], gv[kXPieces];
+  // (unguarded loads on clamped addresses; what lies past K is zeroed at the LDS store)
+  auto load = [&](int k0) {
+#pragma unroll
+    for (int i = 0; i < kWPieces; ++i) {
+      const int p = tid + i * 256, n = min(n0 + p / (kMmK / 4), N - 1), k = min(k0 + (p % (kMmK / 4)) * 4, K - 4);
+      if constexpr (sizeof(T) == 2) {
+        const bf16x4 v = *reinterpret_cast<const bf16x4*>(Wt + (size_t)n * K + k);
+        wv[i] = f32x4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
+      } else {
+        wv[i] = *reinterpret_cast<const f32x4*>(Wt + (size_t)n * K + k);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kXPieces; ++i) {
+      const int p = tid + i * 256, m = min(m0 + p / (kMmK / 4), M - 1), k = min(k0 + (p % (kMmK / 4)) * 4, K - 4);
+      xv[i] = *reinterpret_cast<const f32x4*>(X + (size_t)m * ldx + k);
+      if (X2) gv[i] = *reinterpret_cast<const f32x4*>(X2 + (size_t)m * ldx + k);
+    }
+  };
+  auto put = [&](float* dst, int p, f32x4 v, bool live) {
+    typedef float f32x2_t __attribute__((ext_vector_type(2)));
+    float* row = dst + (p / (kMmK / 4)) * kMmLd + (p % (kMmK / 4)) * 2;
+    *reinterpret_cast<f32x2_t*>(row) = live ? f32x2_t{v[0], v[2]} : f32x2_t{0.f, 0.f};
+    *reinterpret_cast<f32x2_t*>(row + 16) = live ? f32x2_t{v[1], v[3]} : f32x2_t{0.f, 0.f};
+  };
+  auto store = [&](float* buf, int k0) {
+#pragma unroll
+    for (int i = 0; i < kWPieces; ++i) {
+      const int p = tid + i * 256;
+      put(buf, p, wv[i], k0 + (p % (kMmK / 4)) * 4 < K);
+    }
+#pragma unroll
+    for (int i = 0; i < kXPieces; ++i) {
+      const int p = tid + i * 256;
+      f32x4 v = xv[i];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if (X2) v[e] = fmaxf(v[e], 0.f) * gv[i][e];
+        v[e] = maybe_round(v[e], round);
+      }
+      put(buf + BN * kMmLd, p, v, k0 + (p % (kMmK / 4)) * 4 < K);
+    }
+  };
+  f32x16 acc[NT][MT];
+#pragma unroll
+  for (int i = 0; i < NT; ++i)
+#pragma unroll
+    for (int j = 0; j < MT; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+  const int n_it = (K + kMmK - 1) / kMmK;
+  load(0);
+  store(lds[0], 0);
+  __syncthreads();
+  for (int it = 0; it < n_it; ++it) {
+    if (it + 1 < n_it) load((it + 1) * kMmK);
+    const float* wb = lds[it & 1] + (wn * NT * 32 + r) * kMmLd + h * 16;
+    const float* xb = lds[it & 1] + (BN + wm * MT * 32 + r) * kMmLd + h * 16;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      f32x4 a[NT], b[MT];
+#pragma unroll
+      for (int i = 0; i < NT; ++i) a[i] = *reinterpret_cast<const f32x4*>(wb + i * 32 * kMmLd + g * 4);
+#pragma unroll
+      for (int j = 0; j < MT; ++j) b[j] = *reinterpret_cast<const f32x4*>(xb + j * 32 * kMmLd + g * 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+          for (int j = 0; j < MT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][e], b[j][e], acc[i][j], 0, 0, 0);
+    }
+    if (it + 1 < n_it) store(lds[(it + 1) & 1], (it + 1) * kMmK);
+    __syncthreads();
+  }
+  // acc[i][j][e]: column n0 + (wn NT + i) 32 + (e & 3) + 8 (e >> 2) + 4 h of row m0 + (wm MT + j) 32 + r
+#pragma unroll
+  for (int j = 0; j < MT; ++j) {
+    const int m = m0 + (wm * MT + j) * 32 + r;
+    if (m >= M) continue;
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int n = n0 + (wn * NT + i) * 32 + 8 * q + 4 * h;
+        f32x4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = acc[i][j][4 * q + e] + (bias && n + e < N ? bias[n + e] : 0.f);
+        if (n + 3 < N && (ldy & 3) == 0) {
+          *reinterpret_cast<f32x4*>(Y + (size_t)m * ldy + n) = o;
+          if (Yb) *reinterpret_cast<bf16x4*>(Yb + (size_t)m * ldy + n) = bf16x4{(bf16_t)o[0], (bf16_t)o[1], (bf16_t)o[2], (bf16_t)o[3]};
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (n + e < N) {
+              Y[(size_t)m * ldy + n + e] = o[e];
+              if (Yb) Yb[(size_t)m * ldy + n + e] = (bf16_t)o[e];
+            }
+        }
+      }
+  }
+}
+
 template <typename T>
 int launch_matmul(const float* X, const float* X2, int64_t ldx, const void* Wt, const float* bias, float* Y,
                   int64_t ldy, int M, int N, int K, int round, hipStream_t st, int batch = 1, int64_t bx = 0,
@@ -738,6 +864,17 @@ int launch_matmul(const float* X, const float* X2, int64_t ldx, const void* Wt, 
     dim3 grid((N + 127) / 128, (M + 15) / 16, batch);
     matmul_rows_kernel<T, 16, 128, 2, 4><<<grid, 256, 0, st>>>(X, X2, ldx, (const T*)Wt, bias, Y, ldy, M, N, K, round,
                                                                bx, bw, by, Yb);
+  } else if (K % 4 == 0 && ldx % 4 == 0 && (bx | bw | by) % 4 == 0 && sd_aligned16(X) && (!X2 || sd_aligned16(X2)) &&
+             sd_aligned16(Wt) && sd_aligned16(Y) && (!Yb || ((uintptr_t)Yb & 7) == 0)) {
+    // 16-byte loads; blocks of 128 x 128 once they fill the chip
+    const long blocks = (long)((N + 127) / 128) * ((M + 127) / 128) * batch;
+    if (blocks >= 256) {
+      dim3 grid((N + 127) / 128, (M + 127) / 128, batch);
+      matmul_mfma_kernel<T, 2, 2><<<grid, 256, 0, st>>>(X, X2, ldx, (const T*)Wt, bias, Y, ldy, M, N, K, round, bx, bw, by, Yb);
+    } else {
+      dim3 grid((N + 63) / 64, (M + 63) / 64, batch);
+      matmul_mfma_kernel<T, 1, 1><<<grid, 256, 0, st>>>(X, X2, ldx, (const T*)Wt, bias, Y, ldy, M, N, K, round, bx, bw, by, Yb);
+    }
   } else {
     dim3 grid((N + 63) / 64, (M + 63) / 64, batch);
     matmul_rows_kernel<T, 64, 64, 4, 4><<<grid, 256, 0, st>>>(X, X2, ldx, (const T*)Wt, bias, Y, ldy, M, N, K, round,

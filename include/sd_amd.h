@@ -1614,6 +1614,12 @@ size_t sd_decay_chunks_scratch_bytes(int n_rows, int n_entries, int H, int dk, i
 int sd_decay_chunks(const float* q, const float* k, const float* v, int64_t ld, const float* decay, float q_scale,
                     float* state, const int32_t* entries, int n_entries, int n_rows, float* out, int H, int dk, int dv,
                     void* scratch, size_t scratch_bytes, sd_stream_t stream);
+/* The same for the recurrence of sd_decay_scan_rows (decay_per_row: decay [rows, H]) and for one fixed decay per
+ * head (decay [H]); scratch as above.                                                        */
+int sd_head_decay_chunks(const float* q, const float* k, int64_t ldqk, const float* v, int64_t ldv,
+                         const float* decay, int decay_per_row, const float* k_scale, const void* skip, int w_f32,
+                         float* state, const int32_t* entries, int n_entries, int n_rows, float* out, int H, int Gq,
+                         int dk, int dv, void* scratch, size_t scratch_bytes, sd_stream_t stream);
 /* x[r, c] *= s                                                                             */
 int sd_scale_rows(float* x, int64_t ld, float s, int n_rows, int n_cols, sd_stream_t stream);
 

@@ -593,3 +593,44 @@ def test_matmul_rows_on_the_matrix_instruction_has_the_bits_of_few_rows(M, N, K,
         few = torch.cat([ops.matmul_rows(x[i:i + 16].contiguous(), w, bias, None if up is None else up[i:i + 16].contiguous())
                          for i in range(0, M, 16)])
         assert torch.equal(got, few)
+
+
+@pytest.mark.parametrize("H,Gq,dk,dv", [(4, 4, 128, 128), (6, 2, 33, 70), (3, 1, 20, 64)])
+@pytest.mark.parametrize("per_row", [False, True])
+@pytest.mark.parametrize("lens", [[300], [1, 130, 16, 64, 65]])
+def test_head_decay_in_chunks_against_the_recurrence(H, Gq, dk, dv, per_row, lens):
+    """Portions in chunks (lengths at the edges of blocks of 16 and chunks of 64, shared q / k groups, odd sizes) against
+    the recurrence in float64, and no further from it than the token-by-token scan is by more than its own error."""
+    from vllm_omni_draft_amd import ops
+    g = torch.Generator().manual_seed(H + dk + sum(lens))
+    n = sum(lens)
+    rn = lambda *shape: torch.randn(*shape, generator=g)
+    q, k, v = rn(n, Gq * dk) * dk ** -0.5, rn(n, Gq * dk), rn(n, H * dv)
+    decay = torch.sigmoid(rn(n, H) + 3) if per_row else torch.tensor([1 - 2.0 ** (-3 - i) for i in range(H)])
+    scale, skip = (torch.rand(n, H, generator=g), rn(H)) if per_row else (None, None)
+    S0 = rn(len(lens), H, dk, dv)
+    pos = [0 if i % 2 else 7 for i in range(len(lens))]
+    ents, row, want = [], 0, []
+    S_want = S0.double().clone()
+    for i, m in enumerate(lens):
+        ents.append([i, row, m, pos[i]])
+        S = S_want[i] if pos[i] else torch.zeros_like(S_want[i])
+        for t in range(row, row + m):
+            kk = k[t].double().view(Gq, dk).repeat_interleave(H // Gq, 0)
+            qq = q[t].double().view(Gq, dk).repeat_interleave(H // Gq, 0)
+            vv = v[t].double().view(H, dv)
+            d = (decay[t] if per_row else decay).double()
+            if scale is not None:
+                kk = kk * scale[t].double()[:, None]
+            S = d[:, None, None] * S + kk[:, :, None] * vv[:, None, :]
+            o = torch.einsum("hkv,hk->hv", S, qq)
+            want.append((o if skip is None else o + skip.double()[:, None] * vv).reshape(-1))
+        S_want[i] = S
+        row += m
+    want = torch.stack(want)
+    dev = lambda t: None if t is None else t.cuda().contiguous()
+    e = torch.tensor(ents, dtype=torch.int32).cuda()
+    S1 = dev(S0)
+    got = ops.head_decay_chunks(dev(q), dev(k), dev(v), dev(decay), S1, e, dev(scale), dev(skip))
+    off = lambda a, b: ((a.double().cpu() - b).norm() / b.norm()).item()
+    assert off(got, want) < 1e-6 and off(S1, S_want) < 1e-6

@@ -1249,6 +1249,7 @@ SeqWs plan_seq(const sd_seq_model& m, int rows, int n_out, int max_ctx) {
     const size_t n = sd_linear_wide_workspace_bytes(M, N, K, SD_EPI_F32);
     wide = n > wide ? n : wide;
   };
+  const int plan_ents = rows < kPlanEntries ? rows : kPlanEntries;   // (enough for any number of portions up to it)
   for (const sd_seq_layer& l : m.layers) {
     if (l.block == SD_BLOCK_STREAMS) {
       const StCols c = st_cols(l);
@@ -1261,8 +1262,7 @@ SeqWs plan_seq(const sd_seq_model& m, int rows, int n_out, int max_ctx) {
       need(l.w_o_tiled, wr, W, K1);
       need(l.out_stacked ? l.w_o_tiled : l.w_o2_tiled, wr, W, K2);
       up(attn, sd_multimap_softmax_attention_scratch_bytes(rows, l.heads, 1, l.vdim, l.window, l.keep_first, 0, max_ctx));
-      const int ents = rows < kPlanEntries ? rows : kPlanEntries;   // (enough for any number of portions up to it)
-      up(mem, sd_decay_chunks_scratch_bytes(rows + ents, ents, l.s_heads, l.s_state, l.s_vdim));
+      up(mem, sd_decay_chunks_scratch_bytes(rows + plan_ents, plan_ents, l.s_heads, l.s_state, l.s_vdim));
       if (l.ff > 0) {
         up(proj, (size_t)2 * l.ff);
         up(ff, (size_t)l.ff);
@@ -1288,8 +1288,7 @@ SeqWs plan_seq(const sd_seq_model& m, int rows, int n_out, int max_ctx) {
       if (l.kind == SD_MIX_MLSTM) {
         up(hv, (size_t)l.heads * (l.vdim + 1));
         up(sh, (size_t)l.heads);
-        const int ents = rows < kPlanEntries ? rows : kPlanEntries;   // (enough for any number of portions up to it)
-        up(mem, sd_mlstm_scratch_bytes(rows + ents, ents, l.heads, l.dim, l.vdim));
+        up(mem, sd_mlstm_scratch_bytes(rows + plan_ents, plan_ents, l.heads, l.dim, l.vdim));
       } else {
         up(pq, (size_t)l.heads * l.dim);
         up(attn, sd_multimap_softmax_attention_scratch_bytes(rows, l.heads, 1, l.vdim, l.window, 0, 0, max_ctx));
@@ -1347,6 +1346,7 @@ SeqWs plan_seq(const sd_seq_model& m, int rows, int n_out, int max_ctx) {
         up(conv, (size_t)c.conv_ch);
         up(sh, (size_t)l.s_heads);
         need(l.w_o2_tiled, wr, W, c.inner);
+        if (l.w_in_tiled) up(mem, sd_decay_chunks_scratch_bytes(rows + plan_ents, plan_ents, l.s_heads, l.s_state, l.s_vdim));
       }
       if (l.n_experts > 0) {
         up(ne, (size_t)l.n_experts);
@@ -1364,6 +1364,8 @@ SeqWs plan_seq(const sd_seq_model& m, int rows, int n_out, int max_ctx) {
     need(l.w_in_tiled, wr, (int)t, W);
     need(l.w_o_tiled, wr, W, l.heads * l.vdim);
     need(l.w_down_tiled, wr, W, l.ff);
+    if (l.kind != SD_MIX_WINDOW_POOL && l.w_in_tiled)
+      up(mem, sd_decay_chunks_scratch_bytes(rows + plan_ents, plan_ents, l.heads, l.dim, l.vdim));
     if (l.kind == SD_MIX_WINDOW_POOL) {
       const size_t n = sd_window_pool_attention_scratch_bytes(rows, l.heads, l.vdim, l.window, l.pool, max_ctx);
       attn = n > attn ? n : attn;
@@ -1635,8 +1637,14 @@ int postnorm_layer(const sd_seq_model& m, const sd_seq_layer& l, const sd_seq_ba
     SQ_TRY(sd_causal_conv_rows(proj + c.xbc, ld, l.conv_w, l.conv_b, f32, l.conv_state, b.row_pos, b.row_slot,
                                b.entries, b.n_entries, conv, c.conv_ch, R, c.conv_ch, l.s_taps, 1, stream));
     SQ_TRY(sd_ssd_steps(proj + c.dt, ld, l.dt_bias, l.a_log, f32, step, decay, R, Hs, stream));
-    SQ_TRY(sd_decay_scan_rows(conv + inner + Gs * N, conv + inner, c.conv_ch, conv, c.conv_ch, decay, step, l.skip_d,
-                              f32, l.state, b.entries, b.n_entries, o, Hs, Gs, N, P, stream));
+    // (long portions of models whose linear layers sum few and many rows in different orders anyway; the scan keeps a
+    // row's bits however a prompt is cut)
+    if (l.w_in_tiled && w.mem_bytes > 0 && sd_decay_chunks_scratch_bytes(R, b.n_entries, Hs, N, P) > 0)
+      SQ_TRY(sd_head_decay_chunks(conv + inner + Gs * N, conv + inner, c.conv_ch, conv, c.conv_ch, decay, 1, step, l.skip_d,
+                                  f32, l.state, b.entries, b.n_entries, R, o, Hs, Gs, N, P, base + w.mem, w.mem_bytes, stream));
+    else
+      SQ_TRY(sd_decay_scan_rows(conv + inner + Gs * N, conv + inner, c.conv_ch, conv, c.conv_ch, decay, step, l.skip_d,
+                                f32, l.state, b.entries, b.n_entries, o, Hs, Gs, N, P, stream));
     SQ_TRY(sd_rmsnorm_parts(o, inner, proj + c.z, ld, l.s_norm_w, f32, eps, y, inner, l.w_o2_tiled ? yb : nullptr,
                             inner, R, inner, l.s_norm_groups, rnd, stream));
     SQ_TRY(seq_linear(l.w_o2, l.w_o2_tiled, f32, y, nullptr, inner, yb, inner, nullptr, mix2, W, R, W, inner, wide_ws,
@@ -2144,8 +2152,16 @@ extern "C" int sd_seq_model_forward(sd_seq_model* m, const sd_seq_batch* b, void
         SQ_TRY(sd_matmul_rows(proj + c.a1, nullptr, ld, l.w_a2, f32, l.b_a2, z, (int64_t)H * dk, R, H * dk, l.rank, stream));
         SQ_TRY(sd_sigmoid_power(z, (int64_t)H * dk, l.tau, dec, R, H * dk, stream));
       }
-      SQ_TRY(sd_decay_scan(proj + c.q, proj + c.k, proj + c.v, ld, pc ? dec : l.head_decay, pc, l.state,
-                           b->entries, b->n_entries, o, H, dk, dv, stream));
+      // (chunks: as in postnorm_layer)
+      if (!l.w_in_tiled || sd_decay_chunks_scratch_bytes(R, b->n_entries, H, dk, dv) == 0)
+        SQ_TRY(sd_decay_scan(proj + c.q, proj + c.k, proj + c.v, ld, pc ? dec : l.head_decay, pc, l.state,
+                             b->entries, b->n_entries, o, H, dk, dv, stream));
+      else if (pc)
+        SQ_TRY(sd_decay_chunks(proj + c.q, proj + c.k, proj + c.v, ld, dec, 1.f, l.state, b->entries, b->n_entries, R, o, H,
+                               dk, dv, base + w.mem, w.mem_bytes, stream));
+      else
+        SQ_TRY(sd_head_decay_chunks(proj + c.q, proj + c.k, ld, proj + c.v, ld, l.head_decay, 0, nullptr, nullptr, 1, l.state,
+                                    b->entries, b->n_entries, R, o, H, H, dk, dv, base + w.mem, w.mem_bytes, stream));
       SQ_TRY(sd_head_post(o, proj + c.g, ld, l.head_norm_w, f32, 1, d.norm_eps, 0, y, y_b, R, H, dv, rnd, stream));
     }
     SQ_TRY(seq_linear(l.w_o, l.w_o_tiled, f32, y, nullptr, (int64_t)H * dv, yb, (int64_t)H * dv, nullptr, mix, W, R,

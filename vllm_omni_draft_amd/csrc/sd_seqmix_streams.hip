@@ -518,8 +518,12 @@ struct ChunkArgs {
   const float* q;
   const float* k;
   const float* v;
-  int64_t ld;
-  const float* decay;      // [rows, H*dk]
+  int64_t ld, ldv;         // row strides of q and k, and of v
+  const float* decay;      // [rows, H*dk]; one number per head: at row * ld_decay + head
+  int64_t ld_decay;
+  const float* k_scale;    // [rows, H] or null: factors of k
+  const void* skip;        // [H] or null: o_t += skip v_t
+  int skip_f32, hpg;       // heads per group of q and k
   float q_scale;
   float* state;            // [slots, H, dk, dv]
   const int32_t* entries;
@@ -558,8 +562,19 @@ struct BlockRows {
       v[u] = ld_pack<V>(src + (size_t)(t < rows ? t : rows - 1) * ld + (c < cols ? c : cols - V));
     }
   }
-  // times f; what lies outside is `pad`
-  __device__ __forceinline__ void store(float* dst, int ldd, int rows, int cols, float f, float pad) {
+  // one number per row in place of its columns
+  __device__ __forceinline__ void load_scalars(const float* src, int64_t ld, int rows) {
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      const int t = (threadIdx.x + kChunkThreads * u) / (COLS / V);
+      const float x = src[(size_t)(t < rows ? t : rows - 1) * ld];
+#pragma unroll
+      for (int e = 0; e < V; ++e) v[u].v[e] = x;
+    }
+  }
+  // times f and, element by element, m; what lies outside is `pad`
+  __device__ __forceinline__ void store(float* dst, int ldd, int rows, int cols, float f, float pad,
+                                        const BlockRows* m = nullptr) {
 #pragma unroll
     for (int u = 0; u < N; ++u) {
       const int idx = threadIdx.x + kChunkThreads * u, t = idx / (COLS / V), c = idx % (COLS / V) * V;
@@ -567,6 +582,10 @@ struct BlockRows {
       Pack<V> p;
 #pragma unroll
       for (int e = 0; e < V; ++e) p.v[e] = t < rows && c < cols ? v[u].v[e] * f : pad;
+      if (m) {
+#pragma unroll
+        for (int e = 0; e < V; ++e) p.v[e] *= m->v[u].v[e];
+      }
       st_pack<V>(dst + t * ldd + c, p);
     }
   }
@@ -577,7 +596,7 @@ constexpr size_t decay_chunk_lds() {
   return sizeof(float) * (4 * (size_t)kBlock * (DKP + 4) + (size_t)DKP * kTokLd + DKP +
                           (size_t)kBlock * (kBlockCols + 4) + (size_t)kBlock * kTokLd);
 }
-template <int DKP, int V, int MODE>   // keys of up to DKP channels
+template <int DKP, int V, int MODE, bool SCALAR>   // keys of up to DKP channels; SCALAR: one decay for a head's channels
 __global__ __launch_bounds__(kChunkThreads, DKP <= 128 ? 4 : 2) void decay_chunk_kernel(ChunkArgs g) {
   extern __shared__ float lds[];
   constexpr int LDK = DKP + 4, LDV = kBlockCols + 4, KT = DKP / 16;
@@ -605,15 +624,22 @@ __global__ __launch_bounds__(kChunkThreads, DKP <= 128 ? 4 : 2) void decay_chunk
   const int nt = MODE == kWhole ? left : (left < g.chunk ? left : g.chunk);
   const size_t at = ((size_t)blockIdx.x * H + h) * dk;            // the chunk's place in ct, and (times dv) in cs
   float* slot_state = g.state + ((size_t)slot * H + h) * dk * dv + c0;
-  BlockRows<DKP, V> rq, rk, rd;
+  BlockRows<DKP, V> rq, rk, rd, rs;
   BlockRows<kBlockCols, V> rv;
+  const size_t qk_at = (size_t)(h / g.hpg) * dk;
+  const float skip = !SCALAR || !g.skip ? 0.f : (g.skip_f32 ? ((const float*)g.skip)[h] : (float)((const bf16_t*)g.skip)[h]);
   auto fetch = [&](int t0) {
     const size_t row = (size_t)(row0 + t0);
     const int n = nt - t0 < kBlock ? nt - t0 : kBlock;
-    if constexpr (MODE != kSums) rq.load(g.q + row * g.ld + (size_t)h * dk, g.ld, n, dk);
-    rk.load(g.k + row * g.ld + (size_t)h * dk, g.ld, n, dk);
-    rd.load(g.decay + row * H * dk + (size_t)h * dk, (int64_t)H * dk, n, dk);
-    rv.load(g.v + row * g.ld + (size_t)h * dv + c0, g.ld, n, cols);
+    if constexpr (MODE != kSums) rq.load(g.q + row * g.ld + qk_at, g.ld, n, dk);
+    rk.load(g.k + row * g.ld + qk_at, g.ld, n, dk);
+    if constexpr (SCALAR) {
+      rd.load_scalars(g.decay + row * g.ld_decay + h, g.ld_decay, n);
+      if (g.k_scale) rs.load_scalars(g.k_scale + row * H + h, H, n);
+    } else {
+      rd.load(g.decay + row * H * dk + (size_t)h * dk, (int64_t)H * dk, n, dk);
+    }
+    rv.load(g.v + row * g.ldv + (size_t)h * dv + c0, g.ldv, n, cols);
   };
   fetch(0);
   const int c = 16 * wave + col;       // this wave's columns of the state; rows 16 * kt + 4 * quad + i
@@ -637,7 +663,7 @@ __global__ __launch_bounds__(kChunkThreads, DKP <= 128 ? 4 : 2) void decay_chunk
     const int n = nt - t0 < kBlock ? nt - t0 : kBlock;
     __syncthreads();
     if constexpr (MODE != kSums) rq.store(qs, LDK, n, dk, g.q_scale, 0.f);
-    rk.store(ks, LDK, n, dk, 1.f, 0.f);
+    rk.store(ks, LDK, n, dk, 1.f, 0.f, SCALAR && g.k_scale ? &rs : nullptr);
     rd.store(ds, LDK, n, dk, 1.f, 1.f);
     rv.store(vs, LDV, n, cols, 1.f, 0.f);
     __syncthreads();
@@ -743,6 +769,7 @@ __global__ __launch_bounds__(kChunkThreads, DKP <= 128 ? 4 : 2) void decay_chunk
         acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], vv[i], acc, 0, 0, 0);
       }
       o += o2;
+      if constexpr (SCALAR) o += skip * vv;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int t = 4 * quad + i;
@@ -805,14 +832,14 @@ __global__ __launch_bounds__(256) void chunk_carry_kernel(ChunkArgs g) {
   *st = val;
 }
 
-template <int DKP, int V>
+template <int DKP, int V, bool SCALAR>
 hipError_t launch_decay_chunks(const ChunkArgs& c, size_t nc, hipStream_t st) {
   static std::once_flag once;
   static hipError_t err = hipSuccess;
   std::call_once(once, [] {
-    const void* fns[3] = {reinterpret_cast<const void*>(decay_chunk_kernel<DKP, V, kSums>),
-                          reinterpret_cast<const void*>(decay_chunk_kernel<DKP, V, kReads>),
-                          reinterpret_cast<const void*>(decay_chunk_kernel<DKP, V, kWhole>)};
+    const void* fns[3] = {reinterpret_cast<const void*>(decay_chunk_kernel<DKP, V, kSums, SCALAR>),
+                          reinterpret_cast<const void*>(decay_chunk_kernel<DKP, V, kReads, SCALAR>),
+                          reinterpret_cast<const void*>(decay_chunk_kernel<DKP, V, kWhole, SCALAR>)};
     for (const void* f : fns)
       if (err == hipSuccess) err = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
   });
@@ -820,11 +847,11 @@ hipError_t launch_decay_chunks(const ChunkArgs& c, size_t nc, hipStream_t st) {
   constexpr size_t lds = decay_chunk_lds<DKP>();
   const unsigned z = (c.dv + kBlockCols - 1) / kBlockCols;
   if (nc == 0) {
-    decay_chunk_kernel<DKP, V, kWhole><<<dim3(c.n_entries, c.H, z), kChunkThreads, lds, st>>>(c);
+    decay_chunk_kernel<DKP, V, kWhole, SCALAR><<<dim3(c.n_entries, c.H, z), kChunkThreads, lds, st>>>(c);
   } else {
-    decay_chunk_kernel<DKP, V, kSums><<<dim3((unsigned)nc, c.H, z), kChunkThreads, lds, st>>>(c);
+    decay_chunk_kernel<DKP, V, kSums, SCALAR><<<dim3((unsigned)nc, c.H, z), kChunkThreads, lds, st>>>(c);
     chunk_carry_kernel<<<dim3((c.dk * c.dv + 255) / 256, c.H, c.n_entries), 256, 0, st>>>(c);
-    decay_chunk_kernel<DKP, V, kReads><<<dim3((unsigned)nc, c.H, z), kChunkThreads, lds, st>>>(c);
+    decay_chunk_kernel<DKP, V, kReads, SCALAR><<<dim3((unsigned)nc, c.H, z), kChunkThreads, lds, st>>>(c);
   }
   return hipGetLastError();
 }
@@ -969,29 +996,28 @@ extern "C" size_t sd_decay_chunks_scratch_bytes(int n_rows, int n_entries, int H
   return sizeof(float) * ((size_t)n_rows / kChunkMin + n_entries) * H * ((size_t)dk * dv + dk);
 }
 
-extern "C" int sd_decay_chunks(const float* q, const float* k, const float* v, int64_t ld, const float* decay,
-                               float q_scale, float* state, const int32_t* entries, int n_entries, int n_rows, float* out,
-                               int H, int dk, int dv, void* scratch, size_t scratch_bytes, sd_stream_t stream) {
-  SD_REQUIRE(q && k && v && decay && state && entries && out && n_entries >= 1 && n_rows >= n_entries && H >= 1 && dv >= 1,
-             SD_ERR_INVALID, "sd_decay_chunks: bad argument");
-  SD_REQUIRE(dk >= 1 && dk <= 256, SD_ERR_UNSUPPORTED, "sd_decay_chunks: key size %d outside 1..256", dk);
-  const size_t need = sd_decay_chunks_scratch_bytes(n_rows, n_entries, H, dk, dv);
+namespace {
+int decay_chunks(ChunkArgs c, bool scalar, int n_rows, void* scratch, size_t scratch_bytes, sd_stream_t stream) {
+  const int H = c.H, dk = c.dk, dv = c.dv;
+  const size_t need = sd_decay_chunks_scratch_bytes(n_rows, c.n_entries, H, dk, dv);
   const bool cut = need > 0 && scratch && scratch_bytes >= need && sd_aligned16(scratch);
-  ChunkArgs c{q, k, v, ld, decay, q_scale, state, entries, out, nullptr, nullptr, n_entries, H, dk, dv, kChunkMin};
   size_t nc = 0;
+  c.chunk = kChunkMin;
   if (cut) {
     // (longer chunks, and so less carried state, where they still fill the chip)
     const long long wgs = (long long)(n_rows / kChunkMax) * H * ((dv + kBlockCols - 1) / kBlockCols);
     c.chunk = wgs >= 256 ? kChunkMax : kChunkMin;
-    nc = (size_t)n_rows / c.chunk + n_entries;
+    nc = (size_t)n_rows / c.chunk + c.n_entries;
     c.cs = (float*)scratch;
     c.ct = c.cs + nc * H * dk * dv;
   }
-  const bool quad = ld % 4 == 0 && dk % 4 == 0 && dv % 4 == 0 && sd_aligned16(q) && sd_aligned16(k) && sd_aligned16(v) &&
-                    sd_aligned16(decay);
+  const bool quad = c.ld % 4 == 0 && c.ldv % 4 == 0 && dk % 4 == 0 && dv % 4 == 0 && sd_aligned16(c.q) && sd_aligned16(c.k) &&
+                    sd_aligned16(c.v) && (scalar || sd_aligned16(c.decay));
   hipStream_t st = (hipStream_t)stream;
   hipError_t err;
-#define SD_GO(D) err = quad ? launch_decay_chunks<D, 4>(c, nc, st) : launch_decay_chunks<D, 1>(c, nc, st)
+#define SD_GO(D)                                                                                                        \
+  err = scalar ? (quad ? launch_decay_chunks<D, 4, true>(c, nc, st) : launch_decay_chunks<D, 1, true>(c, nc, st))       \
+               : (quad ? launch_decay_chunks<D, 4, false>(c, nc, st) : launch_decay_chunks<D, 1, false>(c, nc, st))
   if (dk <= 32) SD_GO(32);
   else if (dk <= 64) SD_GO(64);
   else if (dk <= 128) SD_GO(128);
@@ -999,4 +1025,31 @@ extern "C" int sd_decay_chunks(const float* q, const float* k, const float* v, i
 #undef SD_GO
   SD_REQUIRE(err == hipSuccess, SD_ERR_HIP, "sd_decay_chunks: launch failed: %s", hipGetErrorString(err));
   return SD_OK;
+}
+}  // namespace
+
+extern "C" int sd_decay_chunks(const float* q, const float* k, const float* v, int64_t ld, const float* decay,
+                               float q_scale, float* state, const int32_t* entries, int n_entries, int n_rows, float* out,
+                               int H, int dk, int dv, void* scratch, size_t scratch_bytes, sd_stream_t stream) {
+  SD_REQUIRE(q && k && v && decay && state && entries && out && n_entries >= 1 && n_rows >= n_entries && H >= 1 && dv >= 1,
+             SD_ERR_INVALID, "sd_decay_chunks: bad argument");
+  SD_REQUIRE(dk >= 1 && dk <= 256, SD_ERR_UNSUPPORTED, "sd_decay_chunks: key size %d outside 1..256", dk);
+  ChunkArgs c{q, k, v, ld, ld, decay, 0, nullptr, nullptr, 0, 1, q_scale, state, entries, out, nullptr, nullptr, n_entries,
+              H, dk, dv, kChunkMin};
+  return decay_chunks(c, false, n_rows, scratch, scratch_bytes, stream);
+}
+
+// One decay per head (of every row: decay_per_row, else of the head): all channels of a block then share their running
+// products, the rest is the same.
+extern "C" int sd_head_decay_chunks(const float* q, const float* k, int64_t ldqk, const float* v, int64_t ldv,
+                                    const float* decay, int decay_per_row, const float* k_scale, const void* skip, int w_f32,
+                                    float* state, const int32_t* entries, int n_entries, int n_rows, float* out, int H,
+                                    int Gq, int dk, int dv, void* scratch, size_t scratch_bytes, sd_stream_t stream) {
+  SD_REQUIRE(q && k && v && decay && state && entries && out && n_entries >= 1 && n_rows >= n_entries && H >= 1 && Gq >= 1 &&
+                 H % Gq == 0 && dv >= 1,
+             SD_ERR_INVALID, "sd_head_decay_chunks: bad argument");
+  SD_REQUIRE(dk >= 1 && dk <= 256, SD_ERR_UNSUPPORTED, "sd_head_decay_chunks: key size %d outside 1..256", dk);
+  ChunkArgs c{q, k, v, ldqk, ldv, decay, decay_per_row ? H : 0, k_scale, skip, w_f32, H / Gq, 1.f, state, entries, out,
+              nullptr, nullptr, n_entries, H, dk, dv, kChunkMin};
+  return decay_chunks(c, true, n_rows, scratch, scratch_bytes, stream);
 }

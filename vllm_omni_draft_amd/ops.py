@@ -1833,6 +1833,23 @@ def decay_chunks(q, k, v, decay, state, entries, q_scale=1.0, cut=True, scratch=
     return out
 
 
+def head_decay_chunks(q, k, v, decay, state, entries, k_scale=None, skip=None) -> torch.Tensor:
+    """The recurrence with one decay per head over portions, in chunks: q, k f32 [rows, Gq*dk], v [rows, H*dv], decay f32
+    [H] or [rows, H], k_scale f32 [rows, H], skip [H]; state f32 [slots, H, dk, dv] moves on -> f32 [rows, H*dv]."""
+    for t, nm in ((q, "q"), (k, "k"), (v, "v"), (decay, "decay"), (state, "state")):
+        _f32(t, nm)
+    H, dk, dv = state.shape[1:]
+    n, lib = q.shape[0], _lib.load()
+    scratch = decay_chunks_scratch(n, entries.shape[0], H, dk, dv, q.device)
+    out = torch.empty(n, H * dv, dtype=torch.float32, device=q.device)
+    _lib.check(lib.sd_head_decay_chunks(_p(q), _p(k), q.shape[1], _p(v), v.shape[1], _p(decay), int(decay.dim() == 2),
+                                        _p(k_scale), _p(skip), 1 if skip is None else _wkind(skip, "skip"), _p(state),
+                                        _p(entries), entries.shape[0], n, _p(out), H, q.shape[1] // dk, dk, dv,
+                                        _p(scratch), scratch.numel() if scratch is not None else 0, _stream()),
+               "sd_head_decay_chunks")
+    return out
+
+
 def matmul_rows_batched(x, w) -> torch.Tensor:
     """x f32 [M, B, K], w [B, N, K] -> f32 [M, B, N]: product b uses w[b]."""
     _f32(x, "x")

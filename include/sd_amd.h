@@ -1236,6 +1236,14 @@ int sd_window_softmax_attention(const float* q, int64_t ldq, const void* k_cache
                                 int window, int keep_first, float scale, float* out,
                                 void* out_bf16, void* scratch, size_t scratch_bytes,
                                 sd_stream_t stream);
+/* The same attention for the many rows of a prompt over a bf16 cache: entries as for the recurrences (a row's
+ * position follows from its entry).  Heads of 128 / 128 channels, or latent rows (v_cache NULL) of 576 with 512 value
+ * channels; pages of 16; H/G <= 64; 16-byte aligned rows.  f32 queries and weights enter the bf16 matrix instruction
+ * in three parts, which together are all of their bits.                                      */
+int sd_rows_softmax_attention(const float* q, int64_t ldq, const void* k_cache, const void* v_cache,
+                              const int32_t* block_tables, int max_blocks, int page, int n_rows, int H, int G,
+                              int dk, int dv, int window, int keep_first, float scale, const int32_t* entries,
+                              int n_entries, float* out, void* out_bf16, int64_t ldo, sd_stream_t stream);
 /* y[z][M, N] = x[z][M, K] w[z][N, K]^T for z < batch: x + z*bx (row stride ldx), w + z*bw,
  * y + z*by (row stride ldy); y_bf16 (or NULL) laid out as y.                                */
 int sd_matmul_rows_batched(const float* x, int64_t ldx, int64_t bx, const void* w, int w_f32,

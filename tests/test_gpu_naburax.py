@@ -676,3 +676,48 @@ def test_greedy_generation_through_worker_and_scheduler():
                 assert (top[0] - top[1]) / logits.std() < 1e-4
                 break
             logits = N.forward(cfg, t64, [tok], seq)[-1]
+
+
+@pytest.mark.parametrize("H,G,dk,dv", [(4, 1, 128, 128), (6, 2, 128, 128), (16, 1, 576, 512), (5, 1, 576, 512)])
+@pytest.mark.parametrize("window,keep", [(5000, 0), (100, 0), (70, 3), (33, 70), (1, 1)])
+def test_rows_softmax_attention_against_float64(H, G, dk, dv, window, keep):
+    """Portions that start anywhere, lengths at the edges of a workgroup's tokens and of stages of 64 keys, kept tokens
+    before and inside the window, rows of caches whose pages lie anywhere and hold NaN behind the portion: against
+    float64, with the bound of the kernel on the vector pipe (sums of f32 products)."""
+    from vllm_omni_draft_amd import ops
+    latent = dv == 512
+    g = torch.Generator(device="cuda").manual_seed(H + window)
+    runs = [(0, 1), (0, 65), (130, 64), (63, 2), (15, 17)]
+    lens = [p + n for p, n in runs]
+    pages = (max(lens) + 15) // 16
+    perm = torch.randperm(len(runs) * pages, generator=g, device="cuda").to(torch.int32)
+    bt = perm.view(len(runs), pages)
+    kc = torch.randn(len(runs) * pages, G, 16, dk, generator=g, device="cuda").to(torch.bfloat16)
+    vc = None if latent else torch.randn(len(runs) * pages, G, 16, dv, generator=g, device="cuda").to(torch.bfloat16)
+    rows = sum(n for _, n in runs)
+    q = torch.randn(rows, H * dk, generator=g, device="cuda") * 2
+    ents, row, want = [], 0, []
+    for s, (p0, n) in enumerate(runs):
+        ents.append([s, row, n, p0])
+        m = p0 + n
+        for c in (kc,) if latent else (kc, vc):
+            c[bt[s, m // 16:].long()[1:] if m % 16 else bt[s, m // 16:].long()] = float("nan")
+            if m % 16:
+                c[bt[s, m // 16].long(), :, m % 16:] = float("nan")
+        k = kc[bt[s].long()].transpose(1, 2).reshape(-1, G, dk)[:m].double()
+        v = k[..., :dv] if latent else vc[bt[s].long()].transpose(1, 2).reshape(-1, G, dv)[:m].double()
+        qq = q[row:row + n].double().view(n, H, dk)
+        i = torch.arange(p0, m, device="cuda")[:, None]
+        j = torch.arange(m, device="cuda")[None, :]
+        seen = (j <= i) & ((i - j < window) | (j < keep))
+        for t in range(0, n, 64):
+            o = []
+            for h in range(H):
+                sc = qq[t:t + 64, h] @ k[:, h // (H // G)].T * dk ** -0.5
+                sc = sc.masked_fill(~seen[t:t + 64], float("-inf"))
+                o.append(torch.softmax(sc, -1) @ v[:, h // (H // G)])
+            want.append(torch.cat(o, 1))
+        row += n
+    got = ops.rows_softmax_attention(q, kc, vc, bt.contiguous(), i32(ents), H, G, dk, dv, window, keep, dk ** -0.5)
+    off = ((got.double() - torch.cat(want)).norm() / torch.cat(want).norm()).item()
+    assert off < 3e-6, off

@@ -43,6 +43,9 @@ int sd_tiled_window_attention_(const float* q, int64_t ldq, const void* k_cache,
                                int64_t ldg, const int32_t* entries, int n_entries, float* out, void* out_bf16,
                                int64_t ldo, sd_stream_t stream);
 
+// Softmax attention of a prompt's rows on the matrix cores (sd_seqmix_attn.hip); v_cache nullptr: latent rows.
+bool sd_rows_softmax_attention_fits_(int H, int G, int dk, int dv, int page, bool latent);
+
 #define SD_REQUIRE(cond, code, ...)            \
   do {                                         \
     if (!(cond)) {                             \

@@ -1568,6 +1568,16 @@ extern "C" size_t sd_seq_model_workspace_bytes(const sd_seq_model* m, int max_ro
     if (rc__ != SD_OK) return rc__; \
   } while (0)
 
+// Attention on the matrix cores for a pass with more than a few prompt rows (as for the chunked recurrences: of models
+// whose linear layers sum few and many rows in different orders anyway; a row's bits do not depend on the cut else).
+// 64 rows of one portion: 16 heads over 4 of 128 channels 14.8 -> 13.3 us from nothing, 362 -> 143 behind 4000 tokens;
+// 16 latent heads 63 -> 18 and 1305 -> 482; portions of 9 rows gain as much.
+constexpr int kPromptRows = 64;
+bool rows_attention(const sd_seq_layer& l, const sd_seq_batch& b, int H, int G, int dk, int dv, bool latent) {
+  return l.w_in_tiled && sd_aligned16(l.k_cache) && (!l.v_cache || sd_aligned16(l.v_cache)) && b.n_rows - b.n_entries >= kPromptRows && l.window >= 1 &&
+         sd_rows_softmax_attention_fits_(H, G, dk, dv, b.page, latent);
+}
+
 namespace {
 // One layer normed on its sublayers' outputs: x += norm1(mixer(x)); x += norm2(experts(x)).
 // x [R, W] f32 and its bf16 copy hb are current on entry and on return.
@@ -1608,7 +1618,12 @@ int postnorm_layer(const sd_seq_model& m, const sd_seq_layer& l, const sd_seq_ba
     if (dr > 0)
       SQ_TRY(sd_rope_copy_rows(pq, (int64_t)H * dh, dh, dk, qe, (int64_t)H * de, de, rk, b.row_pos, R, H, dr,
                                l.rot_dims, 1, l.inv_freq, l.rot_mag, stream));
-    SQ_TRY(sd_window_softmax_attention(qe, (int64_t)H * de, l.k_cache, nullptr, f32, b.row_pos, b.row_slot,
+    if (rows_attention(l, b, H, 1, de, rk, true))
+      SQ_TRY(sd_rows_softmax_attention(qe, (int64_t)H * de, l.k_cache, nullptr, b.block_tables, b.max_blocks, b.page, R, H, 1,
+                                       de, rk, l.window, 0, l.score_scale, b.entries, b.n_entries, o, nullptr,
+                                       (int64_t)H * rk, stream));
+    else
+      SQ_TRY(sd_window_softmax_attention(qe, (int64_t)H * de, l.k_cache, nullptr, f32, b.row_pos, b.row_slot,
                                        b.block_tables, b.max_blocks, b.page, R, H, 1, de, rk, l.window, 0,
                                        l.score_scale, o, nullptr, base + w.attn, w.attn_bytes, stream));
     // a head's value expansion applied to its weighted latent
@@ -1623,7 +1638,12 @@ int postnorm_layer(const sd_seq_model& m, const sd_seq_layer& l, const sd_seq_ba
     SQ_TRY(sd_qk_norm_append(proj + c.q, H * dk, l.q_norm_w, proj + c.k, G, dk, l.k_norm_w, proj + c.v, dv, ld, f32, eps,
                              l.k_cache, l.v_cache, b.row_pos, b.row_slot, b.block_tables, b.max_blocks, b.page, R,
                              stream));
-    SQ_TRY(sd_window_softmax_attention(proj + c.q, ld, l.k_cache, l.v_cache, f32, b.row_pos, b.row_slot,
+    if (ld % 4 == 0 && c.q % 4 == 0 && rows_attention(l, b, H, G, dk, dv, false))
+      SQ_TRY(sd_rows_softmax_attention(proj + c.q, ld, l.k_cache, l.v_cache, b.block_tables, b.max_blocks, b.page, R, H, G, dk,
+                                       dv, l.window, l.keep_first, l.score_scale, b.entries, b.n_entries, o,
+                                       l.w_o_tiled ? yb : nullptr, (int64_t)H * dv, stream));
+    else
+      SQ_TRY(sd_window_softmax_attention(proj + c.q, ld, l.k_cache, l.v_cache, f32, b.row_pos, b.row_slot,
                                        b.block_tables, b.max_blocks, b.page, R, H, G, dk, dv, l.window, l.keep_first,
                                        l.score_scale, o, l.w_o_tiled ? yb : nullptr, base + w.attn, w.attn_bytes,
                                        stream));

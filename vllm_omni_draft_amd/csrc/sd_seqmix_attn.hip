@@ -1,0 +1,316 @@
+// Softmax attention of layer-list models for the many rows of a prompt, over bf16 caches of plain rows (page, kv head,
+// token): grouped heads, and latent rows whose first channels are the values.
+//
+// The queries and the weights of these models are f32 and stay so: each enters the bf16 matrix instruction as the sum
+// of three bf16 parts (8 + 8 + 8 bits: all of an f32's), keys and values are the cache's bf16 values, so products are
+// exact and sums f32, as on the vector pipe, at a third of the matrix rate.  The kernel before took one workgroup a row
+// and read every key and value from L2 for it on the vector pipe (18 TFLOP/s of f32 work).
+//
+// A workgroup takes one kv head and 64 query rows (64 / (H/G) tokens x the heads of the group) of one portion, a wave
+// 16 of them; 64 keys (four pages) a stage pass through LDS by direct loads, two stages, one barrier a stage.  A page of
+// a head is contiguous, so a wave brings one page; 16-byte piece c of row r of a page lies at c ^ (r & 7) within its
+// 128 bytes, which spreads the fragment reads over the banks.  S^T = K Q^T has a query's scores in one accumulator
+// column, as they are the right operand of O^T = V^T P^T; V^T comes out of the row-major tile by the transposing LDS
+// read (a group of 16 lanes reads 4 keys x 16 channels, a lane receives 4 keys of one channel).
+// Bound by the matrix pipe and the exponentials between its parts (one wave a SIMD for latent rows, whose queries and
+// sums fill the registers): 1024 rows of 16 latent heads (576 / 512 channels) 972 -> 133 us, 1024 rows of 16 heads over 4
+// of 128 channels 344 -> 42 us.
+// A non-finite value at a position of the portion itself can reach rows of up to 63 positions before it.
+#include <math.h>
+
+#include "sd_common.h"
+
+namespace {
+
+struct RowsAttnArgs {
+  const float* q;
+  int64_t ldq;
+  const bf16_t* kc;
+  const bf16_t* vc;
+  const int32_t* block_tables;
+  const int32_t* entries;
+  float* out;
+  bf16_t* out_b;
+  int64_t ldo;
+  float scale;
+  int max_blocks, n_entries, H, G, window, keep_first;
+};
+
+typedef __attribute__((address_space(3))) void lds_void;
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+constexpr int kPage = 16, kKeys = 64, kRowsPerBlock = 64;
+
+// Two f32 values as three pairs of bf16 whose sums they are: 8 bits of the significand each, cut off (the differences
+// are exact), the first value in the low halves.
+__device__ __forceinline__ void three_parts(float x, float y, unsigned& a, unsigned& b, unsigned& c) {
+  auto upper = [](float v) { return __uint_as_float(__float_as_uint(v) & 0xffff0000u); };
+  auto pack = [](float u, float v) { return __builtin_amdgcn_perm(__float_as_uint(v), __float_as_uint(u), 0x07060302u); };
+  const float xr = x - upper(x), yr = y - upper(y);
+  a = pack(x, y);
+  b = pack(xr, yr);
+  c = pack(xr - upper(xr), yr - upper(yr));
+}
+
+// e^x for x <= 0 (-inf: 0), to about one unit in the last place: the product with log2 e in two parts, no branch.
+__device__ __forceinline__ float exp_neg(float x) {
+  x = fmaxf(x, -200.f);   // (e^-200 is 0 in f32)
+  const float hi = x * 1.44269502f;
+  const float lo = fmaf(x, 1.92596300e-8f, fmaf(x, 1.44269502f, -hi));
+  const float y = __builtin_amdgcn_exp2f(hi);
+  return fmaf(y, lo * 0.693147181f, y);
+}
+
+// KS: key channels / 32 (even); VT: value channels / 16 (a multiple of 4); LATENT: values are the keys' first channels
+template <int KS, int VT, bool LATENT>
+__global__ __launch_bounds__(256, KS > 4 ? 1 : 2) void rows_attn_kernel(RowsAttnArgs g) {
+  constexpr int DK = 32 * KS, DV = 16 * VT;
+  constexpr int kKeyPage = kPage * DK * 2, kValPage = LATENT ? 0 : kPage * DV * 2;   // bytes of a page of one head
+  constexpr int kStage = 4 * (kKeyPage + kValPage);
+  __shared__ __attribute__((aligned(1024))) char s0[kStage];
+  __shared__ __attribute__((aligned(1024))) char s1[kStage];
+  const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, quad = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kvh = blockIdx.y, qh = g.H / g.G, per = kRowsPerBlock / qh;
+  // the portion and the first token of this group of tokens; the last ones, which see most, first
+  int e = 0, first = gridDim.x - 1 - blockIdx.x;
+  for (; e < g.n_entries; ++e) {
+    const int n = (g.entries[4 * e + 2] + per - 1) / per;
+    if (first < n) break;
+    first -= n;
+  }
+  if (e == g.n_entries) return;
+  first *= per;
+  const int slot = g.entries[4 * e], row0 = g.entries[4 * e + 1], pos0 = g.entries[4 * e + 3] + first;
+  const int n_tok = min(per, g.entries[4 * e + 2] - first), m_rows = n_tok * qh;
+  const int32_t* tbl = g.block_tables + (size_t)slot * g.max_blocks;
+  const int last = pos0 + n_tok - 1;                         // the workgroup's last position
+  int base0 = max(pos0 - g.window + 1, 0) & ~(kPage - 1);    // the window's first page
+  const int n_kept = min(g.keep_first, base0);               // kept tokens before it, in stages of their own
+  const int kept_stages = (n_kept + kKeys - 1) / kKeys, stages = kept_stages + (last - base0) / kKeys + 1;
+  auto stage_base = [&](int s) { return s < kept_stages ? s * kKeys : base0 + (s - kept_stages) * kKeys; };
+
+  const int m = min(16 * wave + col, m_rows - 1), t = m / qh, h = kvh * qh + m - t * qh;   // this lane's query
+  const bool mine = 16 * wave + col < m_rows;
+  const int p = pos0 + t;
+  const bool works = 16 * wave < m_rows;
+  const int wave_last = works ? pos0 + (min(16 * wave + 16, m_rows) - 1) / qh : -1;
+  // The query times the scale.  Its parts are kept where the registers allow; wide rows (kKept false) keep the f32
+  // values and take them apart at every use, which the vector pipe does beside the matrix pipe.
+  constexpr bool kKept = KS <= 4;
+  f32x4 qf[kKept ? 1 : KS][2];
+  bf16x8 qp[kKept ? KS : 1][3];
+  auto parts = [&](const f32x4 (&x)[2], bf16x8 (&y)[3]) __attribute__((always_inline)) {
+    u32x4 a, b, c;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      unsigned pa, pb, pc;
+      three_parts(x[i >> 1][2 * (i & 1)], x[i >> 1][2 * (i & 1) + 1], pa, pb, pc);
+      a[i] = pa;
+      b[i] = pb;
+      c[i] = pc;
+    }
+    y[0] = __builtin_bit_cast(bf16x8, a);
+    y[1] = __builtin_bit_cast(bf16x8, b);
+    y[2] = __builtin_bit_cast(bf16x8, c);
+  };
+  {
+    const float* qr = g.q + (size_t)(row0 + first + t) * g.ldq + (size_t)h * DK + 8 * quad;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const f32x4 x[2] = {*reinterpret_cast<const f32x4*>(qr + 32 * s) * g.scale,
+                          *reinterpret_cast<const f32x4*>(qr + 32 * s + 4) * g.scale};
+      if constexpr (kKept) parts(x, qp[s]);
+      else {
+        qf[s][0] = x[0];
+        qf[s][1] = x[1];
+      }
+    }
+  }
+  // wave w brings page w of the stage (behind the stage's last key: that key's page), its number asked for a stage ahead
+  auto stage_last = [&](int s) { return s < kept_stages ? n_kept - 1 : last; };
+  auto page_of = [&](int st) {
+    st = min(st, stages - 1);
+    return tbl[min(stage_base(st) + wave * kPage, stage_last(st)) / kPage];
+  };
+  int page = page_of(0);
+  auto load = [&](char* s, int st) __attribute__((always_inline)) {
+    const int blk = __builtin_amdgcn_readfirstlane(page);
+    page = page_of(st + 1);
+    const size_t row = ((size_t)blk * g.G + kvh) * kPage;
+    const auto kr = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(g.kc + row * DK), 0, kKeyPage, 0x00027000);
+#pragma unroll
+    for (int i = 0; i < kKeyPage / 1024; ++i) {
+      const int r = (i * 8 + (lane >> 3)) / (DK / 64);       // the row of the page that this lane's 128 bytes belong to
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(kr, (lds_void*)(s + wave * kKeyPage + i * 1024), 16,
+                                               i * 1024 + (lane >> 3) * 128 + (((lane & 7) ^ (r & 7)) << 4), 0, 0, 0);
+    }
+    if constexpr (!LATENT) {
+      const auto vr = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(g.vc + row * DV), 0, kValPage, 0x00027000);
+#pragma unroll
+      for (int i = 0; i < kValPage / 1024; ++i) {
+        const int r = (i * 8 + (lane >> 3)) / (DV / 64);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(vr, (lds_void*)(s + 4 * kKeyPage + wave * kValPage + i * 1024), 16,
+                                                 i * 1024 + (lane >> 3) * 128 + (((lane & 7) ^ (r & 7)) << 4), 0, 0, 0);
+      }
+    }
+  };
+  f32x4 o[VT];
+#pragma unroll
+  for (int v = 0; v < VT; ++v) o[v] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.f;                      // (a query's sum is spread over its four lanes)
+  const int k_off = col * DK * 2;
+  const int k_sw[2] = {(quad ^ (col & 7)) << 4, ((quad + 4) ^ (col & 7)) << 4};
+  constexpr int kVRow = (LATENT ? DK : DV) * 2;
+  const int v_key = 4 * quad + (col >> 2);                   // of the 16 keys of a half; channels 4 (col & 3) on
+  const int v_off = (LATENT ? 0 : 4 * kKeyPage) + v_key * kVRow + (col & 1) * 8;
+  int v_sw[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v_sw[i] = ((2 * i + ((col & 3) >> 1)) ^ (v_key & 7)) << 4;
+
+  auto attend = [&](const char* s, int st) __attribute__((always_inline)) {
+    const int base = stage_base(st);
+    // (a stage of kept tokens holds no key of the window; in the window's stages kept tokens are seen too)
+    const int key_end = st < kept_stages ? n_kept : 0x7fffffff;
+    if (!works || base > wave_last) return;
+    f32x4 sc[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) sc[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // (the four tiles of 16 keys side by side: four chains of sums)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      bf16x8 a[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) a[u] = *reinterpret_cast<const bf16x8*>(s + u * kKeyPage + k_off + (ks >> 1) * 128 + k_sw[ks & 1]);
+      bf16x8 y[3];
+      if constexpr (kKept) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) y[c] = qp[ks][c];
+      } else {
+        f32x4 x[2] = {qf[ks][0], qf[ks][1]};
+        asm volatile("" : "+v"(x[0]), "+v"(x[1]));   // (or the parts would be formed ahead of the loop and kept)
+        parts(x, y);
+      }
+#pragma unroll
+      for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) sc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], y[c], sc[u], 0, 0, 0);
+    }
+    float mx = m_run;
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int j = base + 16 * u + 4 * quad + i, d = p - j;
+        // (bitwise: a chain of && would become branches)
+        const bool seen = (d >= 0) & ((d < g.window) | (j < g.keep_first)) & (j < key_end);
+        sc[u][i] = seen ? sc[u][i] : -INFINITY;
+        mx = fmaxf(mx, sc[u][i]);
+      }
+    mx = fmaxf(mx, __shfl_xor(mx, 16, SD_WAVE));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, SD_WAVE));
+    const float ref = mx == -INFINITY ? 0.f : mx;            // (no key seen yet)
+    const float corr = exp_neg(m_run - ref);   // (nothing summed yet: 0)
+    m_run = mx;
+    float sum = 0.f;
+    bf16x8 pw[2][3];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        sc[u][i] = exp_neg(sc[u][i] - ref);
+        sum += sc[u][i];
+      }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const f32x4 x[2] = {sc[2 * u], sc[2 * u + 1]};
+      parts(x, pw[u]);
+    }
+    l_run = fmaf(l_run, corr, sum);
+    if (__any(corr != 1.f)) {
+#pragma unroll
+      for (int v = 0; v < VT; ++v) o[v] *= corr;
+    }
+    // (two tiles of 16 channels side by side)
+#pragma unroll
+    for (int v = 0; v < VT; v += 2)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        bf16x8 a[2];
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+          const char* at = s + 32 * u * kVRow + v_off + (v >> 2) * 128 + v_sw[(v + w) & 3];
+          const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(at));
+          const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(at + 16 * kVRow));
+          a[w] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        }
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+          for (int w = 0; w < 2; ++w) o[v + w] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[w], pw[u][c], o[v + w], 0, 0, 0);
+      }
+  };
+  // stage st is in `cur` once this wave's loads have landed and every wave is here; then nobody reads `nxt` any more
+  auto step = [&](char* cur, char* nxt, int st) __attribute__((always_inline)) {
+    // Rows behind the stage's last key hold what a page's earlier owner left, or nothing: a weight of 0 does not clear a
+    // NaN, so they are cleared here, by the wave that brought them.
+    const int left = stage_last(st) + 1 - stage_base(st) - wave * kPage;
+    if (left < kPage) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      char* rows = cur + (LATENT ? wave * kKeyPage : 4 * kKeyPage + wave * kValPage);
+      for (int at = max(left, 0) * kVRow + lane * 16; at < kPage * kVRow; at += 64 * 16) *reinterpret_cast<u32x4*>(rows + at) = u32x4{0, 0, 0, 0};
+    }
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (st + 1 < stages) load(nxt, st + 1);
+    attend(cur, st);
+  };
+  load(s0, 0);
+  int st = 0;
+  for (; st + 1 < stages; st += 2) {
+    step(s0, s1, st);
+    step(s1, s0, st + 1);
+  }
+  if (st < stages) step(s0, s1, st);
+  l_run += __shfl_xor(l_run, 16, SD_WAVE);
+  l_run += __shfl_xor(l_run, 32, SD_WAVE);
+  if (!mine) return;
+  const float inv = 1.f / l_run;
+  const size_t at = (size_t)(row0 + first + t) * g.ldo + (size_t)h * DV + 4 * quad;
+#pragma unroll
+  for (int v = 0; v < VT; ++v) {
+    const f32x4 y = o[v] * inv;
+    if (g.out) *reinterpret_cast<f32x4*>(g.out + at + 16 * v) = y;
+    if (g.out_b)
+      *reinterpret_cast<bf16x4*>(g.out_b + at + 16 * v) = bf16x4{(bf16_t)y[0], (bf16_t)y[1], (bf16_t)y[2], (bf16_t)y[3]};
+  }
+}
+
+}  // namespace
+
+// Whether sd_rows_softmax_attention takes these sizes (v_cache nullptr: latent rows).
+bool sd_rows_softmax_attention_fits_(int H, int G, int dk, int dv, int page, bool latent) {
+  if (page != kPage || H % G || H / G > kRowsPerBlock) return false;
+  return latent ? dk == 576 && dv == 512 : dk == 128 && dv == 128;
+}
+
+extern "C" int sd_rows_softmax_attention(const float* q, int64_t ldq, const void* k_cache, const void* v_cache,
+                                         const int32_t* block_tables, int max_blocks, int page, int n_rows, int H, int G,
+                                         int dk, int dv, int window, int keep_first, float scale, const int32_t* entries,
+                                         int n_entries, float* out, void* out_b, int64_t ldo, sd_stream_t stream) {
+  SD_REQUIRE(q && k_cache && block_tables && entries && (out || out_b) && max_blocks >= 1 && n_rows >= 1 && n_entries >= 1 &&
+                 n_rows >= n_entries && H >= 1 && G >= 1 && window >= 1 && keep_first >= 0,
+             SD_ERR_INVALID, "sd_rows_softmax_attention: bad argument");
+  SD_REQUIRE(sd_rows_softmax_attention_fits_(H, G, dk, dv, page, !v_cache), SD_ERR_UNSUPPORTED,
+             "sd_rows_softmax_attention: %d heads over %d of %d / %d channels, pages of %d", H, G, dk, dv, page);
+  RowsAttnArgs g{q, ldq, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, entries, out, (bf16_t*)out_b, ldo,
+                 scale, max_blocks, n_entries, H, G, window, keep_first};
+  SD_REQUIRE(ldq % 4 == 0 && ldo % 4 == 0 && ldq >= (int64_t)H * dk && ldo >= (int64_t)H * dv && sd_aligned16(q) &&
+                 sd_aligned16(k_cache) && (!v_cache || sd_aligned16(v_cache)) && (!out || sd_aligned16(out)) &&
+                 (!out_b || (reinterpret_cast<uintptr_t>(out_b) & 7) == 0),
+             SD_ERR_INVALID, "sd_rows_softmax_attention: rows must be 16-byte aligned");
+  const dim3 grid(n_rows / (kRowsPerBlock / (H / G)) + n_entries, G);
+  if (v_cache) hipLaunchKernelGGL((rows_attn_kernel<4, 8, false>), grid, dim3(256), 0, (hipStream_t)stream, g);
+  else hipLaunchKernelGGL((rows_attn_kernel<18, 32, true>), grid, dim3(256), 0, (hipStream_t)stream, g);
+  SD_CHECK_LAUNCH("sd_rows_softmax_attention");
+  return SD_OK;
+}

@@ -1284,6 +1284,20 @@ def window_softmax_attention(q, k_cache, v_cache, row_pos, row_slot, block_table
     return out
 
 
+def rows_softmax_attention(q, k_cache, v_cache, block_tables, entries, H, G, dk, dv, window, keep_first,
+                           scale) -> torch.Tensor:
+    """window_softmax_attention for a prompt's rows over a bf16 cache, on the matrix cores; entries int32 [n, 4] {slot,
+    first row, rows, first position}."""
+    _f32(q, "q")
+    _need(k_cache, torch.bfloat16, "k_cache")
+    out = torch.empty(q.shape[0], H * dv, dtype=torch.float32, device=q.device)
+    _lib.check(_lib.load().sd_rows_softmax_attention(
+        _p(q), q.shape[1], _p(k_cache), _p(v_cache), _p(block_tables), block_tables.shape[1], PAGE, q.shape[0], H, G, dk, dv,
+        int(window), int(keep_first), float(scale), _p(entries), entries.shape[0], _p(out), None, H * dv, _stream()),
+        "sd_rows_softmax_attention")
+    return out
+
+
 def masked_softmax_attention(q, k_cache, v_cache, row_pos, row_slot, block_tables, H, G, dk, dv, scale, window=0,
                              keep_first=0, chunk=0, softcap=0.0, sinks=None, split=True) -> torch.Tensor:
     """window_softmax_attention with the further masks of sd_masked_softmax_attention: window 0

@@ -1244,6 +1244,12 @@ int sd_rows_softmax_attention(const float* q, int64_t ldq, const void* k_cache, 
                               const int32_t* block_tables, int max_blocks, int page, int n_rows, int H, int G,
                               int dk, int dv, int window, int keep_first, float scale, const int32_t* entries,
                               int n_entries, float* out, void* out_bf16, int64_t ldo, sd_stream_t stream);
+/* sd_window_pool_attention for the many rows of a prompt over a bf16 cache (heads of 128 / 128 channels, pages of 16),
+ * entries as above.                                                                          */
+int sd_rows_pool_attention(const float* q, int64_t ldq, const void* k_cache, const void* v_cache, float* pk_cache,
+                           float* pv_cache, const int32_t* block_tables, int max_blocks, int page, int n_rows, int H,
+                           int G, int dk, int dv, int window, int pool, float scale, const float* head_bias,
+                           const int32_t* entries, int n_entries, float* out, sd_stream_t stream);
 /* y[z][M, N] = x[z][M, K] w[z][N, K]^T for z < batch: x + z*bx (row stride ldx), w + z*bw,
  * y + z*by (row stride ldy); y_bf16 (or NULL) laid out as y.                                */
 int sd_matmul_rows_batched(const float* x, int64_t ldx, int64_t bx, const void* w, int w_f32,

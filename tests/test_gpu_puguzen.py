@@ -311,6 +311,38 @@ def test_window_pool_attention_many_keys(dtype):
             assert rel(small[a].view(H, dv)[h], ref) < 5e-6 and rel(big[i].view(H, dv)[h], ref) < 5e-6, (i, h)
 
 
+@pytest.mark.parametrize("H,G,window,pool", [(4, 1, 100, 16), (6, 2, 33, 5), (2, 2, 1, 1), (3, 1, 17, 32), (64, 1, 300, 16),
+                                             (4, 2, 5000, 3)])
+def test_rows_pool_attention_against_float64(H, G, window, pool):
+    """The same attention on the matrix cores: portions at the edges of a workgroup's tokens, of stages of 64 keys and of
+    32 blocks, blocks across pages and several a page, page slots without a token NaN; the vector kernel's bound."""
+    from vllm_omni_draft_amd import ops
+    g = torch.Generator().manual_seed(H + window)
+    n, d = 420, 128
+    k, v = (torch.randn(n, G * d, generator=g).to(torch.bfloat16).float() for _ in range(2))
+    q, bias = torch.randn(n, H * d, generator=g), torch.randn(H, generator=g) - 3
+    bed = _AttnBed(G, d, d, pool, n, torch.bfloat16)
+    for c in (bed.k, bed.v, bed.pk, bed.pv):
+        c.fill_(float("nan"))
+    out, at = [], 0
+    for c in (64, 1, 65, 17, 128, 145):
+        pos = list(range(at, at + c))
+        bed.append(k[at:at + c], v[at:at + c], pos)
+        out.append(ops.rows_pool_attention(dev(q[at:at + c]), bed.k, bed.v, bed.pk, bed.pv, bed.tables,
+                                           i32([[0, 0, c, at]]), H, G, d, d, window, pool, d ** -0.5, dev(bias)))
+        at += c
+    out = torch.cat(out).cpu().double().view(n, H, d)
+    K, V, Q = (dev(t).double() for t in (k.view(n, G, d), v.view(n, G, d), q.view(n, H, d)))
+    nb = n // pool
+    i, j, b = (torch.arange(m, device=DEV) for m in (n, n, nb))
+    seen = torch.cat([(j[None] <= i[:, None]) & (i[:, None] - j[None] < window),
+                      b[None] * pool + pool - 1 <= i[:, None] - window], 1)
+    Ka, Va = (torch.cat([t, t[:nb * pool].view(nb, pool, G, d).mean(1)]) for t in (K, V))
+    for h in range(H):
+        w = torch.sigmoid(Q[:, h] @ Ka[:, h // (H // G)].T * d ** -0.5 + bias[h].double()) * seen
+        assert rel(out[:, h], (w @ Va[:, h // (H // G)]).cpu()) < 5e-6, h
+
+
 @pytest.mark.parametrize("window,pool", [(9, 4), (7, 5), (16, 16), (17, 3), (1, 1), (5, 32)])
 @pytest.mark.parametrize("decode", [False, True])
 def test_window_pool_attention_sees_exactly_its_keys(window, pool, decode):

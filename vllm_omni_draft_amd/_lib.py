@@ -321,6 +321,8 @@ SIGNATURES = {
     "sd_decay_chunks_scratch_bytes": (C.c_size_t, [i32, i32, i32, i32, i32]),
     "sd_rows_softmax_attention": (i32, [vp, i64, vp, vp, vp, i32, i32, i32, i32, i32, i32, i32, i32, i32, C.c_float, vp, i32,
                                         vp, vp, i64, vp]),
+    "sd_rows_pool_attention": (i32, [vp, i64, vp, vp, vp, vp, vp, i32, i32, i32, i32, i32, i32, i32, i32, i32, C.c_float,
+                                     vp, vp, i32, vp, vp]),
     "sd_head_decay_chunks": (i32, [vp, vp, i64, vp, i64, vp, i32, vp, vp, i32, vp, vp, i32, i32, vp, i32, i32, i32, i32, vp,
                                    C.c_size_t, vp]),
     "sd_decay_chunks": (i32, [vp, vp, vp, i64, vp, C.c_float, vp, vp, i32, i32, vp, i32, i32, i32, vp, C.c_size_t, vp]),

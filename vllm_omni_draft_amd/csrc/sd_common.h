@@ -45,6 +45,10 @@ int sd_tiled_window_attention_(const float* q, int64_t ldq, const void* k_cache,
 
 // Softmax attention of a prompt's rows on the matrix cores (sd_seqmix_attn.hip); v_cache nullptr: latent rows.
 bool sd_rows_softmax_attention_fits_(int H, int G, int dk, int dv, int page, bool latent);
+int sd_rows_pool_attention_(const float* q, int64_t ldq, const void* k_cache, const void* v_cache, const float* pk, const float* pv,
+                            const int32_t* block_tables, int max_blocks, int n_rows, int H, int G, int window, int pool, int pslots,
+                            float scale, const float* head_bias, const int32_t* entries, int n_entries, float* out,
+                            sd_stream_t stream);
 
 #define SD_REQUIRE(cond, code, ...)            \
   do {                                         \

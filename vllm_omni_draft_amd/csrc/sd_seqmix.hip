@@ -372,30 +372,63 @@ __global__ void head_post_kernel(const float* __restrict__ o, const float* __res
 // In-page slot of pooled block b, whose last token lies in logical page lp.
 __device__ __forceinline__ int pooled_slot(int b, int lp, int page, int pool) { return b - (lp * page) / pool; }
 
-// Mean key / value of every block of `pool` tokens that a new row completes, from the rows the
-// cache holds.  One wave per (row, kv head).
+// Mean key / value of block b of a sequence, from the rows the cache holds; a thread a column.  Chains of dependent
+// reads, so kBatch tokens are asked for at once.
 template <typename T>
-__global__ void pool_blocks_kernel(const T* __restrict__ k_cache, const T* __restrict__ v_cache,
-                                   float* __restrict__ pk_cache, float* __restrict__ pv_cache,
-                                   const int32_t* __restrict__ row_pos, const int32_t* __restrict__ row_slot,
-                                   const int32_t* __restrict__ block_tables, int max_blocks, int page,
-                                   int pslots, int G, int dk, int dv, int pool) {
-  const int r = blockIdx.x, g = blockIdx.y, lane = threadIdx.x;
-  const int pos = row_pos[r];
-  if (pos % pool != pool - 1) return;
-  const int b = pos / pool;
-  const int32_t* tbl = block_tables + (size_t)row_slot[r] * max_blocks;
-  const int lp = pos / page;
+__device__ __forceinline__ void pool_block(const T* k_cache, const T* v_cache, float* pk_cache, float* pv_cache,
+                                           const int32_t* tbl, int b, int g, int page, int pslots, int G, int dk, int dv,
+                                           int pool) {
+  constexpr int kBatch = 8;
+  const int last = b * pool + pool - 1, lp = last / page;
   const size_t dst = ((size_t)tbl[lp] * G + g) * pslots + pooled_slot(b, lp, page, pool);
-  for (int c = lane; c < dk + dv; c += 64) {
+  for (int c = threadIdx.x; c < dk + dv; c += blockDim.x) {
     const bool is_k = c < dk;
     const int cc = is_k ? c : c - dk;
     const int d = is_k ? dk : dv;
     const T* cache = is_k ? k_cache : v_cache;
     float sum = 0.f;
-    for (int j = b * pool; j <= pos; ++j)
-      sum += ld_f(cache + (((size_t)tbl[j / page] * G + g) * page + j % page) * d + cc);
+    for (int j0 = b * pool; j0 <= last; j0 += kBatch) {
+      float v[kBatch];
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) {
+        const int j = j0 + u < last ? j0 + u : last;
+        v[u] = ld_f(cache + (((size_t)tbl[j / page] * G + g) * page + j % page) * d + cc);
+      }
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u)
+        if (j0 + u <= last) sum += v[u];
+    }
     (is_k ? pk_cache : pv_cache)[dst * d + cc] = sum / (float)pool;
+  }
+}
+
+// Every block that a new row completes: one workgroup per (row, kv head).
+template <typename T>
+__global__ __launch_bounds__(256) void pool_blocks_kernel(
+    const T* __restrict__ k_cache, const T* __restrict__ v_cache, float* __restrict__ pk_cache, float* __restrict__ pv_cache,
+    const int32_t* __restrict__ row_pos, const int32_t* __restrict__ row_slot, const int32_t* __restrict__ block_tables,
+    int max_blocks, int page, int pslots, int G, int dk, int dv, int pool) {
+  const int pos = row_pos[blockIdx.x];
+  if (pos % pool != pool - 1) return;
+  pool_block(k_cache, v_cache, pk_cache, pv_cache, block_tables + (size_t)row_slot[blockIdx.x] * max_blocks, pos / pool,
+             blockIdx.y, page, pslots, G, dk, dv, pool);
+}
+
+// The same by portions: one workgroup per (completed block, kv head).  With rows in the grid every 16th workgroup works
+// (16 tokens a block), and all of those are on one XCD: 2048 rows of 4 heads 43 us, by portions 7.
+__global__ __launch_bounds__(256) void pool_spans_kernel(
+    const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache, float* __restrict__ pk_cache,
+    float* __restrict__ pv_cache, const int32_t* __restrict__ entries, int n_entries, const int32_t* __restrict__ block_tables,
+    int max_blocks, int page, int pslots, int G, int dk, int dv, int pool) {
+  int i = blockIdx.x;
+  for (int e = 0; e < n_entries; ++e) {
+    const int p0 = entries[4 * e + 3], b0 = p0 / pool, n = (p0 + entries[4 * e + 2]) / pool - b0;
+    if (i < n) {
+      pool_block(k_cache, v_cache, pk_cache, pv_cache, block_tables + (size_t)entries[4 * e] * max_blocks, b0 + i, blockIdx.y,
+                 page, pslots, G, dk, dv, pool);
+      return;
+    }
+    i -= n;
   }
 }
 
@@ -1039,10 +1072,10 @@ extern "C" int sd_window_pool_attention(const float* q, int64_t ldq, const void*
              dk, dv, lds);
   float* dst = split ? (float*)scratch : out;
   if (cache_f32)
-    pool_blocks_kernel<float><<<gp, 64, 0, st>>>((const float*)k_cache, (const float*)v_cache, pk_cache, pv_cache,
+    pool_blocks_kernel<float><<<gp, 256, 0, st>>>((const float*)k_cache, (const float*)v_cache, pk_cache, pv_cache,
                                                  row_pos, row_slot, block_tables, max_blocks, page, pslots, G, dk, dv, pool);
   else
-    pool_blocks_kernel<bf16_t><<<gp, 64, 0, st>>>((const bf16_t*)k_cache, (const bf16_t*)v_cache, pk_cache, pv_cache,
+    pool_blocks_kernel<bf16_t><<<gp, 256, 0, st>>>((const bf16_t*)k_cache, (const bf16_t*)v_cache, pk_cache, pv_cache,
                                                   row_pos, row_slot, block_tables, max_blocks, page, pslots, G, dk, dv, pool);
   SD_CHECK_LAUNCH("sd_window_pool_attention (pool)");
 #define SD_ATTN_NH(T, N)                                                                                          \
@@ -1067,6 +1100,28 @@ extern "C" int sd_window_pool_attention(const float* q, int64_t ldq, const void*
     SD_CHECK_LAUNCH("sd_window_pool_attention (sum)");
   }
   return SD_OK;
+}
+
+extern "C" int sd_rows_pool_attention(const float* q, int64_t ldq, const void* k_cache, const void* v_cache, float* pk_cache,
+                                      float* pv_cache, const int32_t* block_tables, int max_blocks, int page, int n_rows,
+                                      int H, int G, int dk, int dv, int window, int pool, float scale,
+                                      const float* head_bias, const int32_t* entries, int n_entries, float* out,
+                                      sd_stream_t stream) {
+  SD_REQUIRE(q && k_cache && v_cache && pk_cache && pv_cache && block_tables && entries && out, SD_ERR_INVALID,
+             "sd_rows_pool_attention: null argument");
+  SD_REQUIRE(n_entries >= 1 && n_rows >= n_entries && H >= 1 && G >= 1 && window >= 1 && pool >= 1 && max_blocks >= 1 &&
+                 ldq >= (int64_t)H * dk,
+             SD_ERR_INVALID, "sd_rows_pool_attention: bad shape");
+  SD_REQUIRE(sd_rows_softmax_attention_fits_(H, G, dk, dv, page, false), SD_ERR_UNSUPPORTED,
+             "sd_rows_pool_attention: %d heads over %d of %d / %d channels, pages of %d", H, G, dk, dv, page);
+  const int pslots = sd_pooled_slots_per_page(page, pool);
+  // (n rows complete at most n / pool + 1 blocks)
+  pool_spans_kernel<<<dim3(n_rows / pool + n_entries, G), 256, 0, (hipStream_t)stream>>>(
+      (const bf16_t*)k_cache, (const bf16_t*)v_cache, pk_cache, pv_cache, entries, n_entries, block_tables, max_blocks, page,
+      pslots, G, dk, dv, pool);
+  SD_CHECK_LAUNCH("sd_rows_pool_attention (pool)");
+  return sd_rows_pool_attention_(q, ldq, k_cache, v_cache, pk_cache, pv_cache, block_tables, max_blocks, n_rows, H, G, window,
+                                 pool, pslots, scale, head_bias, entries, n_entries, out, stream);
 }
 
 extern "C" int sd_gated_residual(float* x, const float* z1, const float* z2, int64_t ldz, const float* c1,
@@ -1571,7 +1626,9 @@ extern "C" size_t sd_seq_model_workspace_bytes(const sd_seq_model* m, int max_ro
 // Attention on the matrix cores for a pass with more than a few prompt rows (as for the chunked recurrences: of models
 // whose linear layers sum few and many rows in different orders anyway; a row's bits do not depend on the cut else).
 // 64 rows of one portion: 16 heads over 4 of 128 channels 14.8 -> 13.3 us from nothing, 362 -> 143 behind 4000 tokens;
-// 16 latent heads 63 -> 18 and 1305 -> 482; portions of 9 rows gain as much.
+// 16 latent heads 63 -> 18 and 1305 -> 482; portions of 9 rows gain as much.  With a window of 1024 and pooled blocks (16
+// heads over 4): 21.7 -> 17.6 from nothing, 132 -> 65 behind 4000 tokens, 816 -> 78 for a prompt of 2048; with a window of
+// 128 no slower from nothing (16.9, 17.4) and 57 -> 48 behind 4000.
 constexpr int kPromptRows = 64;
 bool rows_attention(const sd_seq_layer& l, const sd_seq_batch& b, int H, int G, int dk, int dv, bool latent) {
   return l.w_in_tiled && sd_aligned16(l.k_cache) && (!l.v_cache || sd_aligned16(l.v_cache)) && b.n_rows - b.n_entries >= kPromptRows && l.window >= 1 &&
@@ -2156,7 +2213,13 @@ extern "C" int sd_seq_model_forward(sd_seq_model* m, const sd_seq_batch* b, void
       SQ_TRY(sd_head_prep(proj + c.q, proj + c.k, proj + c.v, ld, b->row_pos, b->row_slot, R, H, G, dk, dv,
                           l.rot_dims, l.rot_layout, l.inv_freq, l.qk_unit_norm, d.norm_eps, l.q_scale, l.k_scale,
                           l.k_cache, l.v_cache, f32, b->block_tables, b->max_blocks, b->page, stream));
-      SQ_TRY(sd_window_pool_attention(proj + c.q, ld, l.k_cache, l.v_cache, f32, l.pk_cache, l.pv_cache,
+      if (ld % 4 == 0 && c.q % 4 == 0 && sd_aligned16(l.pk_cache) && sd_aligned16(l.pv_cache) &&
+          rows_attention(l, *b, H, G, dk, dv, false))
+        SQ_TRY(sd_rows_pool_attention(proj + c.q, ld, l.k_cache, l.v_cache, l.pk_cache, l.pv_cache, b->block_tables,
+                                      b->max_blocks, b->page, R, H, G, dk, dv, l.window, l.pool, l.score_scale,
+                                      l.head_bias, b->entries, b->n_entries, o, stream));
+      else
+        SQ_TRY(sd_window_pool_attention(proj + c.q, ld, l.k_cache, l.v_cache, f32, l.pk_cache, l.pv_cache,
                                       b->row_pos, b->row_slot, b->block_tables, b->max_blocks, b->page, R, H, G,
                                       dk, dv, l.window, l.pool, l.score_scale, l.head_bias, o, base + w.attn,
                                       w.attn_bytes, stream));

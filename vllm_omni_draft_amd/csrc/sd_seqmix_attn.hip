@@ -15,6 +15,7 @@
 // Bound by the matrix pipe and the exponentials between its parts (one wave a SIMD for latent rows, whose queries and
 // sums fill the registers): 1024 rows of 16 latent heads (576 / 512 channels) 972 -> 133 us, 1024 rows of 16 heads over 4
 // of 128 channels 344 -> 42 us.
+// 2048 rows of 16 heads over 4 with a window of 1024 and pooled blocks 789 -> 73 us.
 // A non-finite value at a position of the portion itself can reach rows of up to 63 positions before it.
 #include <math.h>
 
@@ -34,12 +35,16 @@ struct RowsAttnArgs {
   int64_t ldo;
   float scale;
   int max_blocks, n_entries, H, G, window, keep_first;
+  // pooled keys and values of whole blocks of `pool` tokens behind the window (f32), `pslots` a page
+  const float *pk, *pv, *head_bias;
+  int pool, pslots;
 };
 
 typedef __attribute__((address_space(3))) void lds_void;
+typedef __attribute__((address_space(1))) const void global_void;
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-constexpr int kPage = 16, kKeys = 64, kRowsPerBlock = 64;
+constexpr int kPage = 16, kKeys = 64, kRowsPerBlock = 64, kPooled = 32;
 
 // Two f32 values as three pairs of bf16 whose sums they are: 8 bits of the significand each, cut off (the differences
 // are exact), the first value in the low halves.
@@ -61,8 +66,21 @@ __device__ __forceinline__ float exp_neg(float x) {
   return fmaf(y, lo * 0.693147181f, y);
 }
 
-// KS: key channels / 32 (even); VT: value channels / 16 (a multiple of 4); LATENT: values are the keys' first channels
-template <int KS, int VT, bool LATENT>
+// 1 / (1 + e^-x), to about two units in the last place (below e^-87: 0 or next to it)
+__device__ __forceinline__ float sigmoid_of(float x) {
+  x = -fmaxf(x, -87.f);
+  const float hi = x * 1.44269502f;
+  const float lo = fmaf(x, 1.92596300e-8f, fmaf(x, 1.44269502f, -hi));
+  const float y = __builtin_amdgcn_exp2f(hi);
+  const float d = 1.f + fmaf(y, lo * 0.693147181f, y), r = __builtin_amdgcn_rcpf(d);
+  return fmaf(fmaf(-d, r, 1.f), r, r);
+}
+
+// KS: key channels / 32 (even); VT: value channels / 16 (a multiple of 4); LATENT: values are the keys' first channels;
+// POOLED: weights are sigmoids of the scores plus a bias, and the blocks behind the window take part as their means.
+// The means are f32: stages of 32 of them take the f32 matrix instruction, whose fragments of 4 channels are the 8
+// channels of a lane in turn; the scores' accumulators are its right operand as they are.
+template <int KS, int VT, bool LATENT, bool POOLED>
 __global__ __launch_bounds__(256, KS > 4 ? 1 : 2) void rows_attn_kernel(RowsAttnArgs g) {
   constexpr int DK = 32 * KS, DV = 16 * VT;
   constexpr int kKeyPage = kPage * DK * 2, kValPage = LATENT ? 0 : kPage * DV * 2;   // bytes of a page of one head
@@ -86,8 +104,11 @@ __global__ __launch_bounds__(256, KS > 4 ? 1 : 2) void rows_attn_kernel(RowsAttn
   const int32_t* tbl = g.block_tables + (size_t)slot * g.max_blocks;
   const int last = pos0 + n_tok - 1;                         // the workgroup's last position
   int base0 = max(pos0 - g.window + 1, 0) & ~(kPage - 1);    // the window's first page
-  const int n_kept = min(g.keep_first, base0);               // kept tokens before it, in stages of their own
-  const int kept_stages = (n_kept + kKeys - 1) / kKeys, stages = kept_stages + (last - base0) / kKeys + 1;
+  // what is seen before it, in stages of their own: kept tokens, or pooled blocks
+  auto blocks_of = [&](int pos) { return max(pos - g.window + 1, 0) / g.pool; };
+  const int n_kept = POOLED ? blocks_of(last) : min(g.keep_first, base0);
+  constexpr int kKept0 = POOLED ? kPooled : kKeys;
+  const int kept_stages = (n_kept + kKept0 - 1) / kKept0, stages = kept_stages + (last - base0) / kKeys + 1;
   auto stage_base = [&](int s) { return s < kept_stages ? s * kKeys : base0 + (s - kept_stages) * kKeys; };
 
   const int m = min(16 * wave + col, m_rows - 1), t = m / qh, h = kvh * qh + m - t * qh;   // this lane's query
@@ -130,11 +151,24 @@ __global__ __launch_bounds__(256, KS > 4 ? 1 : 2) void rows_attn_kernel(RowsAttn
   // wave w brings page w of the stage (behind the stage's last key: that key's page), its number asked for a stage ahead
   auto stage_last = [&](int s) { return s < kept_stages ? n_kept - 1 : last; };
   auto page_of = [&](int st) {
-    st = min(st, stages - 1);
+    st = max(min(st, stages - 1), POOLED ? kept_stages : 0);
     return tbl[min(stage_base(st) + wave * kPage, stage_last(st)) / kPage];
   };
   int page = page_of(0);
   auto load = [&](char* s, int st) __attribute__((always_inline)) {
+    if (POOLED && st < kept_stages) {   // wave w: means 8w on of the stage (behind the last one: that one)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = 2 * i + (lane >> 5), idx = min(st * kPooled + wave * 8 + r, n_kept - 1);
+        const int lp = (idx * g.pool + g.pool - 1) / kPage;   // the page whose slots hold block idx
+        const size_t at = (((size_t)tbl[lp] * g.G + kvh) * g.pslots + idx - lp * kPage / g.pool) * 512 + (((lane & 31) ^ r) << 4);
+        static_assert(!POOLED || (DK == 128 && DV == 128), "rows of 512 bytes");
+        __builtin_amdgcn_global_load_lds((global_void*)((const char*)g.pk + at), (lds_void*)(s + wave * 4096 + i * 1024), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((global_void*)((const char*)g.pv + at), (lds_void*)(s + kPooled * 512 + wave * 4096 + i * 1024),
+                                         16, 0, 0);
+      }
+      return;
+    }
     const int blk = __builtin_amdgcn_readfirstlane(page);
     page = page_of(st + 1);
     const size_t row = ((size_t)blk * g.G + kvh) * kPage;
@@ -168,6 +202,50 @@ __global__ __launch_bounds__(256, KS > 4 ? 1 : 2) void rows_attn_kernel(RowsAttn
 #pragma unroll
   for (int i = 0; i < 4; ++i) v_sw[i] = ((2 * i + ((col & 3) >> 1)) ^ (v_key & 7)) << 4;
 
+  const float bias = POOLED && g.head_bias ? g.head_bias[h] : 0.f;
+  const int my_blocks = POOLED ? blocks_of(p) : 0, wave_blocks = POOLED ? blocks_of(wave_last) : 0;
+  auto attend_pooled = [&](const char* s, int st) __attribute__((always_inline)) {
+    if (!works || st * kPooled >= wave_blocks) return;
+    int cl = col, qd = quad;
+    asm volatile("" : "+v"(cl), "+v"(qd));   // (or every address would be formed ahead of the loop and kept)
+    f32x4 sc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      f32x4 a[2][2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          a[u][i] = *reinterpret_cast<const f32x4*>(s + (16 * u + cl) * 512 + (((8 * ks + 2 * qd + i) ^ (cl & 7)) << 4));
+      bf16x8 y[3] = {qp[kKept ? ks : 0][0], qp[kKept ? ks : 0][1], qp[kKept ? ks : 0][2]};
+      asm volatile("" : "+v"(y[0]), "+v"(y[1]), "+v"(y[2]));   // (formed here, not ahead of the loop and kept)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {   // (the three parts make up the query's f32 value again)
+        const float x = ((float)y[2][j] + (float)y[1][j]) + (float)y[0][j];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) sc[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u][j >> 2][j & 3], x, sc[u], 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = 16 * u + 4 * qd + i;
+        const float wt = sigmoid_of(sc[u][i] + bias);
+        sc[u][i] = st * kPooled + r < my_blocks ? wt : 0.f;
+      }
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = 16 * u + 4 * qd + i;
+        const char* at = s + (kPooled + r) * 512 + (cl & 3) * 4;
+#pragma unroll
+        for (int v = 0; v < VT; ++v)
+          o[v] = __builtin_amdgcn_mfma_f32_16x16x4f32(*reinterpret_cast<const float*>(at + (((4 * v + (cl >> 2)) ^ (r & 7)) << 4)),
+                                                      sc[u][i], o[v], 0, 0, 0);
+      }
+  };
   auto attend = [&](const char* s, int st) __attribute__((always_inline)) {
     const int base = stage_base(st);
     // (a stage of kept tokens holds no key of the window; in the window's stages kept tokens are seen too)
@@ -196,40 +274,51 @@ __global__ __launch_bounds__(256, KS > 4 ? 1 : 2) void rows_attn_kernel(RowsAttn
 #pragma unroll
         for (int u = 0; u < 4; ++u) sc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], y[c], sc[u], 0, 0, 0);
     }
-    float mx = m_run;
+    if constexpr (POOLED) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+      for (int u = 0; u < 4; ++u)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int j = base + 16 * u + 4 * quad + i, d = p - j;
-        // (bitwise: a chain of && would become branches)
-        const bool seen = (d >= 0) & ((d < g.window) | (j < g.keep_first)) & (j < key_end);
-        sc[u][i] = seen ? sc[u][i] : -INFINITY;
-        mx = fmaxf(mx, sc[u][i]);
+        for (int i = 0; i < 4; ++i) {
+          const int d = p - (base + 16 * u + 4 * quad + i);
+          const float wt = sigmoid_of(sc[u][i] + bias);
+          sc[u][i] = ((d >= 0) & (d < g.window)) ? wt : 0.f;
+        }
+    } else {
+      float mx = m_run;
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int j = base + 16 * u + 4 * quad + i, d = p - j;
+          // (bitwise: a chain of && would become branches)
+          const bool seen = (d >= 0) & ((d < g.window) | (j < g.keep_first)) & (j < key_end);
+          sc[u][i] = seen ? sc[u][i] : -INFINITY;
+          mx = fmaxf(mx, sc[u][i]);
+        }
+      mx = fmaxf(mx, __shfl_xor(mx, 16, SD_WAVE));
+      mx = fmaxf(mx, __shfl_xor(mx, 32, SD_WAVE));
+      const float ref = mx == -INFINITY ? 0.f : mx;            // (no key seen yet)
+      const float corr = exp_neg(m_run - ref);   // (nothing summed yet: 0)
+      m_run = mx;
+      float sum = 0.f;
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          sc[u][i] = exp_neg(sc[u][i] - ref);
+          sum += sc[u][i];
+        }
+      l_run = fmaf(l_run, corr, sum);
+      if (__any(corr != 1.f)) {
+#pragma unroll
+        for (int v = 0; v < VT; ++v) o[v] *= corr;
       }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, SD_WAVE));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, SD_WAVE));
-    const float ref = mx == -INFINITY ? 0.f : mx;            // (no key seen yet)
-    const float corr = exp_neg(m_run - ref);   // (nothing summed yet: 0)
-    m_run = mx;
-    float sum = 0.f;
+    }
     bf16x8 pw[2][3];
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        sc[u][i] = exp_neg(sc[u][i] - ref);
-        sum += sc[u][i];
-      }
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const f32x4 x[2] = {sc[2 * u], sc[2 * u + 1]};
       parts(x, pw[u]);
-    }
-    l_run = fmaf(l_run, corr, sum);
-    if (__any(corr != 1.f)) {
-#pragma unroll
-      for (int v = 0; v < VT; ++v) o[v] *= corr;
     }
     // (two tiles of 16 channels side by side)
 #pragma unroll
@@ -254,7 +343,8 @@ __global__ __launch_bounds__(256, KS > 4 ? 1 : 2) void rows_attn_kernel(RowsAttn
   auto step = [&](char* cur, char* nxt, int st) __attribute__((always_inline)) {
     // Rows behind the stage's last key hold what a page's earlier owner left, or nothing: a weight of 0 does not clear a
     // NaN, so they are cleared here, by the wave that brought them.
-    const int left = stage_last(st) + 1 - stage_base(st) - wave * kPage;
+    const bool means = POOLED && st < kept_stages;
+    const int left = means ? kPage : stage_last(st) + 1 - stage_base(st) - wave * kPage;
     if (left < kPage) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       char* rows = cur + (LATENT ? wave * kKeyPage : 4 * kKeyPage + wave * kValPage);
@@ -262,7 +352,8 @@ __global__ __launch_bounds__(256, KS > 4 ? 1 : 2) void rows_attn_kernel(RowsAttn
     }
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if (st + 1 < stages) load(nxt, st + 1);
-    attend(cur, st);
+    if (means) attend_pooled(cur, st);
+    else attend(cur, st);
   };
   load(s0, 0);
   int st = 0;
@@ -271,10 +362,13 @@ __global__ __launch_bounds__(256, KS > 4 ? 1 : 2) void rows_attn_kernel(RowsAttn
     step(s1, s0, st + 1);
   }
   if (st < stages) step(s0, s1, st);
-  l_run += __shfl_xor(l_run, 16, SD_WAVE);
-  l_run += __shfl_xor(l_run, 32, SD_WAVE);
+  float inv = 1.f;
+  if constexpr (!POOLED) {
+    l_run += __shfl_xor(l_run, 16, SD_WAVE);
+    l_run += __shfl_xor(l_run, 32, SD_WAVE);
+    inv = 1.f / l_run;
+  }
   if (!mine) return;
-  const float inv = 1.f / l_run;
   const size_t at = (size_t)(row0 + first + t) * g.ldo + (size_t)h * DV + 4 * quad;
 #pragma unroll
   for (int v = 0; v < VT; ++v) {
@@ -303,14 +397,30 @@ extern "C" int sd_rows_softmax_attention(const float* q, int64_t ldq, const void
   SD_REQUIRE(sd_rows_softmax_attention_fits_(H, G, dk, dv, page, !v_cache), SD_ERR_UNSUPPORTED,
              "sd_rows_softmax_attention: %d heads over %d of %d / %d channels, pages of %d", H, G, dk, dv, page);
   RowsAttnArgs g{q, ldq, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, entries, out, (bf16_t*)out_b, ldo,
-                 scale, max_blocks, n_entries, H, G, window, keep_first};
+                 scale, max_blocks, n_entries, H, G, window, keep_first, nullptr, nullptr, nullptr, 1, 0};
   SD_REQUIRE(ldq % 4 == 0 && ldo % 4 == 0 && ldq >= (int64_t)H * dk && ldo >= (int64_t)H * dv && sd_aligned16(q) &&
                  sd_aligned16(k_cache) && (!v_cache || sd_aligned16(v_cache)) && (!out || sd_aligned16(out)) &&
                  (!out_b || (reinterpret_cast<uintptr_t>(out_b) & 7) == 0),
              SD_ERR_INVALID, "sd_rows_softmax_attention: rows must be 16-byte aligned");
   const dim3 grid(n_rows / (kRowsPerBlock / (H / G)) + n_entries, G);
-  if (v_cache) hipLaunchKernelGGL((rows_attn_kernel<4, 8, false>), grid, dim3(256), 0, (hipStream_t)stream, g);
-  else hipLaunchKernelGGL((rows_attn_kernel<18, 32, true>), grid, dim3(256), 0, (hipStream_t)stream, g);
+  if (v_cache) hipLaunchKernelGGL((rows_attn_kernel<4, 8, false, false>), grid, dim3(256), 0, (hipStream_t)stream, g);
+  else hipLaunchKernelGGL((rows_attn_kernel<18, 32, true, false>), grid, dim3(256), 0, (hipStream_t)stream, g);
   SD_CHECK_LAUNCH("sd_rows_softmax_attention");
+  return SD_OK;
+}
+
+// Window and pooled blocks with sigmoid weights (the means of the rows' own blocks are in the cache already).
+int sd_rows_pool_attention_(const float* q, int64_t ldq, const void* k_cache, const void* v_cache, const float* pk, const float* pv,
+                            const int32_t* block_tables, int max_blocks, int n_rows, int H, int G, int window, int pool, int pslots,
+                            float scale, const float* head_bias, const int32_t* entries, int n_entries, float* out,
+                            sd_stream_t stream) {
+  RowsAttnArgs g{q, ldq, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, entries, out, nullptr, (int64_t)H * 128,
+                 scale, max_blocks, n_entries, H, G, window, 0, pk, pv, head_bias, pool, pslots};
+  SD_REQUIRE(ldq % 4 == 0 && sd_aligned16(q) && sd_aligned16(k_cache) && sd_aligned16(v_cache) && sd_aligned16(pk) &&
+                 sd_aligned16(pv) && sd_aligned16(out),
+             SD_ERR_INVALID, "sd_rows_pool_attention: rows must be 16-byte aligned");
+  hipLaunchKernelGGL((rows_attn_kernel<4, 8, false, true>), dim3(n_rows / (kRowsPerBlock / (H / G)) + n_entries, G), dim3(256), 0,
+                     (hipStream_t)stream, g);
+  SD_CHECK_LAUNCH("sd_rows_pool_attention");
   return SD_OK;
 }

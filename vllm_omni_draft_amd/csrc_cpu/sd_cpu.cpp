@@ -1681,6 +1681,9 @@ extern "C" int sd_low_rank_decay(const float*, int64_t, const void*, const float
   UNSUPPORTED("sd_low_rank_decay");
 }
 extern "C" size_t sd_decay_chunks_scratch_bytes(int, int, int, int, int) { return 0; }
+extern "C" int sd_rows_pool_attention(const float*, int64_t, const void*, const void*, float*, float*,
+                                      const int32_t*, int, int, int, int, int, int, int, int, int, float, const float*,
+                                      const int32_t*, int, float*, sd_stream_t) { UNSUPPORTED("sd_rows_pool_attention"); }
 extern "C" int sd_rows_softmax_attention(const float*, int64_t, const void*, const void*, const int32_t*, int, int, int, int, int,
                                          int, int, int, int, float, const int32_t*, int, float*, void*, int64_t,
                                          sd_stream_t) { UNSUPPORTED("sd_rows_softmax_attention"); }

@@ -1189,6 +1189,19 @@ def window_pool_attention(q, k_cache, v_cache, pk_cache, pv_cache, row_pos, row_
     return out
 
 
+def rows_pool_attention(q, k_cache, v_cache, pk_cache, pv_cache, block_tables, entries, H, G, dk, dv,
+                        window, pool, scale, head_bias=None) -> torch.Tensor:
+    """window_pool_attention for a prompt's rows over a bf16 cache, on the matrix cores; entries int32 [n, 4] {slot, first
+    row, rows, first position}."""
+    _f32(q, "q")
+    _need(k_cache, torch.bfloat16, "k_cache")
+    out = torch.empty(q.shape[0], H * dv, dtype=torch.float32, device=q.device)
+    _lib.check(_lib.load().sd_rows_pool_attention(
+        _p(q), q.shape[1], _p(k_cache), _p(v_cache), _p(pk_cache), _p(pv_cache), _p(block_tables), block_tables.shape[1],
+        PAGE, q.shape[0], H, G, dk, dv, int(window), int(pool), float(scale), _p(head_bias), _p(entries), entries.shape[0], _p(out), _stream()), "sd_rows_pool_attention")
+    return out
+
+
 def gated_residual(x, z1, a, z2=None, b=None, c1=None, c2=None) -> None:
     """x += sigmoid(z1 + c1) * a (+ sigmoid(z2 + c2) * b), in place; x, z, a, b f32 [rows, W],
     the bias rows c1, c2 f32 [W]."""
@@ -1939,7 +1952,7 @@ def moe_route_rows(x, w_router, top, score="sigmoid", renorm=False):
 
 def moe_experts(x, sel_e, sel_w, w_gate_up, w_down, scale_input=True, act="silu") -> torch.Tensor:
     """x f32 [rows, W]; w_gate_up [E, 2F, W], w_down [E, W, F]; returns f32 [rows, top, W]: every
-    chosen expert's result.  act "relu2": experts of two matrices, w_gate_up is [E, F, W]."""
+    chosen expert's result.  act "relu2": experts of two matrices, w_gate_up is [E, F, W]. """
     _f32(x, "x")
     n, W = x.shape
     top, E, F = sel_e.shape[1], w_gate_up.shape[0], w_down.shape[2]

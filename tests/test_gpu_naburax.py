@@ -721,3 +721,22 @@ def test_rows_softmax_attention_against_float64(H, G, dk, dv, window, keep):
     got = ops.rows_softmax_attention(q, kc, vc, bt.contiguous(), i32(ents), H, G, dk, dv, window, keep, dk ** -0.5)
     off = ((got.double() - torch.cat(want)).norm() / torch.cat(want).norm()).item()
     assert off < 3e-6, off
+
+
+@pytest.mark.parametrize("E,F,W,n", [(4, 96, 160, 100), (3, 64, 128, 63), (2, 160, 96, 300), (5, 320, 64, 200)])
+@pytest.mark.parametrize("act,scale_input", [("silu", True), ("silu", False), ("relu2", False)])
+def test_moe_experts_of_many_rows_have_the_bits_of_few(E, F, W, n, act, scale_input):
+    """Groups at the edges of the tiles of 64 rows, an expert that nobody chose and one that most did, columns and k that
+    end inside a tile: the products through LDS against those of the kernel that converts f32 rows itself, bit for bit."""
+    from vllm_omni_draft_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(E * n)
+    x = torch.randn(n, W, generator=g, device="cuda")
+    mats = 1 if act == "relu2" else 2
+    gu = (torch.randn(E, mats * F, W, generator=g, device="cuda") * 0.1).to(torch.bfloat16)
+    dn = (torch.randn(E, W, F, generator=g, device="cuda") * 0.1).to(torch.bfloat16)
+    sel_w = torch.rand(n, 2, generator=g, device="cuda")
+    for full in (n, 64, 65, 1):   # rows whose first choice is expert 0; the last expert is never chosen
+        sel = torch.randint(1, max(E - 1, 2), (n, 2), generator=g, device="cuda", dtype=torch.int32)
+        sel[:full, 0] = 0
+        a = ops.moe_experts(x, sel, sel_w, gu, dn, scale_input, act, bf16_copy=True)
+        assert torch.equal(a, ops.moe_experts(x, sel, sel_w, gu, dn, scale_input, act)), full

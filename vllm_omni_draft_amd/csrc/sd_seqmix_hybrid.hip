@@ -1088,6 +1088,7 @@ __device__ __forceinline__ float expert_act(float a, float u, int kind, float li
 }
 
 constexpr int kMoeBM = 32;   // assignment rows per tile of the grouped products
+constexpr int kMoeLdsBM = 64;   // the same of the kernel through LDS
 constexpr int kMoeDirect = 16;  // at most this many assignments: each is its own tile, nothing is grouped
 // cnt[e] = assignments of expert e.  One workgroup per expert.
 __global__ void moe_count_kernel(const int32_t* __restrict__ sel_e, int n, int32_t* __restrict__ cnt) {
@@ -1428,6 +1429,144 @@ __global__ __launch_bounds__(256) void moe_down_mfma_kernel(
       if (n0 < N) out[(size_t)a * N + n0] = sc * acc[mt][0][i];
       if (n1 < N) out[(size_t)a * N + n1] = sc * acc[mt][1][i];
     }
+}
+
+// ---- the same two products with bf16 rows: both operands through LDS.
+// A workgroup takes BM assignments of one expert and 128 of its weight rows (gated: 64 of the gate and the 64 of the up
+// matrix that belong to them), a wave half of either; K goes by in steps of 64, three stages of direct loads, one barrier
+// a step.  Weights are row-major: 64 k of a row are 128 bytes, whose 16-byte piece c lies at c ^ (row & 7), which spreads
+// the fragment reads over the banks.  Columns beyond the matrix, rows beyond the group and k beyond K are out of the
+// buffer's bounds and arrive as zeros.  A sum runs over k ascending with the same instruction as above, so the bits are
+// the same.
+// The workgroups of one column block and expert are issued close together and land on one XCD (where the column blocks
+// are a multiple of 8), so an expert's weights come from memory about once.
+struct MoeArgs {
+  const bf16_t* x;
+  int64_t ldx;
+  unsigned x_bytes, w_bytes;   // of all rows, of one expert
+  const int32_t *perm, *tiles, *n_tiles;
+  const float* sel_w;
+  const bf16_t* w;
+  bf16_t* act;
+  float* out;
+  int top, E, N, K, scale_input, act_kind;
+  float limit;
+};
+
+typedef __attribute__((address_space(3))) void lds_void;
+constexpr int kMoeStages = 3, kMoeStep = 128, kMoeCols = 128;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, unsigned bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00027000);
+}
+// 16 bytes a lane from byte `at` of a buffer to 1024 bytes of LDS, in order of the lanes
+__device__ __forceinline__ void load_lds(__amdgpu_buffer_rsrc_t b, char* lds, unsigned at) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(b, (lds_void*)lds, 16, at, 0, 0, 0);
+}
+constexpr unsigned kOutside = 0x80000000u;   // (buffers are smaller: reads of zero)
+
+template <int LEFT>
+__device__ __forceinline__ void meet() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LEFT) : "memory");
+}
+
+enum { kGated = 0, kSquare = 1, kDown = 2 };
+
+template <int BM, int EPI>
+__global__ __launch_bounds__(256, 2) void moe_rows_kernel(MoeArgs g) {
+  if ((int)blockIdx.y >= g.n_tiles[0]) return;
+  const int e = g.tiles[3 * blockIdx.y], p0 = g.tiles[3 * blockIdx.y + 1], rows = g.tiles[3 * blockIdx.y + 2];
+  if ((unsigned)e >= (unsigned)g.E) return;
+  constexpr int kStage = (kMoeCols + BM) * kMoeStep, MT = BM / 32;
+  constexpr int kXLoads = BM / 32, kLoads = kMoeCols / 32 + kXLoads;   // of a wave and stage; 8 rows each
+  __shared__ __attribute__((aligned(1024))) char s0[kStage];
+  __shared__ __attribute__((aligned(1024))) char s1[kStage];
+  __shared__ __attribute__((aligned(1024))) char s2[kStage];
+  const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, kq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wn = wave & 1, wm = wave >> 1;
+  constexpr int kNew = EPI == kGated ? kMoeCols / 2 : kMoeCols;   // output columns of a workgroup
+  const int n0 = blockIdx.x * kNew;
+  const int n_mats = EPI == kGated ? 2 : 1;
+  const auto wr = buffer_of(g.w + (size_t)e * n_mats * g.N * g.K, g.w_bytes);
+  const auto xr = buffer_of(g.x, g.x_bytes);
+  const int piece = ((lane & 7) ^ (lane >> 3)) << 4, k_bytes = 2 * g.K;
+  unsigned w_at[kMoeCols / 32], x_at[kXLoads];
+#pragma unroll
+  for (int i = 0; i < kMoeCols / 32; ++i) {
+    const int r = (wave * (kMoeCols / 32) + i) * 8 + (lane >> 3), n = n0 + (EPI == kGated ? r & 63 : r);
+    w_at[i] = n < g.N ? (unsigned)((EPI == kGated && r >= 64 ? g.N : 0) + n) * k_bytes + piece : kOutside;
+  }
+#pragma unroll
+  for (int i = 0; i < kXLoads; ++i) {
+    const int r = (wave * kXLoads + i) * 8 + (lane >> 3);
+    x_at[i] = r < rows ? (unsigned)(g.perm[p0 + r] / g.top * g.ldx * 2) + piece : kOutside;
+  }
+  const int n_steps = (g.K + 63) / 64;
+  auto load = [&](char* s, int it) __attribute__((always_inline)) {
+    const unsigned k = it * kMoeStep;
+    const bool in = (int)k + piece < k_bytes;
+#pragma unroll
+    for (int i = 0; i < kMoeCols / 32; ++i)
+      load_lds(wr, s + (wave * (kMoeCols / 32) + i) * 1024, in ? w_at[i] + k : kOutside);
+#pragma unroll
+    for (int i = 0; i < kXLoads; ++i)
+      load_lds(xr, s + kMoeCols * kMoeStep + (wave * kXLoads + i) * 1024, in ? x_at[i] + k : kOutside);
+  };
+  f32x4 acc[4][MT];
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[t][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // tile t of this wave's weight rows: gate, gate, up, up
+  auto w_row = [&](int t) { return EPI == kGated ? (t >> 1) * 64 + 32 * wn + 16 * (t & 1) : 64 * wn + 16 * t; };
+  auto step = [&](const char* cur, char* nxt, int it) __attribute__((always_inline)) {
+    meet<(kMoeStages - 2) * kLoads>();
+    load(nxt, it + kMoeStages - 1);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      const int at = lr * kMoeStep + (((4 * ks + kq) ^ (lr & 7)) << 4);
+      bf16x8 a[4], b[MT];
+#pragma unroll
+      for (int t = 0; t < 4; ++t) a[t] = *reinterpret_cast<const bf16x8*>(cur + w_row(t) * kMoeStep + at);
+#pragma unroll
+      for (int m = 0; m < MT; ++m) b[m] = *reinterpret_cast<const bf16x8*>(cur + (kMoeCols + wm * (BM / 2) + 16 * m) * kMoeStep + at);
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[t][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t], b[m], acc[t][m], 0, 0, 0);
+    }
+  };
+  load(s0, 0);
+  load(s1, 1);
+  int it = 0;
+  for (; it + 2 < n_steps; it += 3) {
+    step(s0, s2, it);
+    step(s1, s0, it + 1);
+    step(s2, s1, it + 2);
+  }
+  if (it < n_steps) step(s0, s2, it);
+  if (it + 1 < n_steps) step(s1, s0, it + 1);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no direct load outlives the workgroup's use of LDS
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    const int r = wm * (BM / 2) + 16 * m + lr;
+    if (r >= rows) continue;
+    const int a = g.perm[p0 + r];
+    const float sc = (EPI == kDown) == (g.scale_input != 0) ? 1.f : g.sel_w[a];
+#pragma unroll
+    for (int t = 0; t < (EPI == kGated ? 2 : 4); ++t) {
+      const int n = n0 + (EPI == kGated ? 32 * wn + 16 * t : 64 * wn + 16 * t) + 4 * kq;
+      if (n >= g.N) continue;
+      if constexpr (EPI == kDown) {
+        *reinterpret_cast<f32x4*>(g.out + (size_t)a * g.N + n) = sc * acc[t][m];
+      } else {
+        bf16x4 y;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          y[i] = (bf16_t)expert_act(sc * acc[t][m][i], sc * acc[EPI == kGated ? t + 2 : t][m][i], g.act_kind, g.limit);
+        *reinterpret_cast<bf16x4*>(g.act + (size_t)a * g.N + n) = y;
+      }
+    }
+  }
 }
 
 // ---- a few assignments (decoding): each is a matrix-vector product.  A workgroup holds the
@@ -2256,12 +2395,18 @@ extern "C" int sd_moe_experts_clamped(const float* x, const void* x_bf16, int64_
   int32_t* perm = (int32_t*)(base + p.perm);
   int32_t* tiles = (int32_t*)(base + p.tiles);
   float* act = (float*)(base + p.act);
-  const int n = n_rows * top;
   const bool mfma = !w_f32 && W % 32 == 0 && F % 32 == 0 && sd_aligned16(w_gate_up) && sd_aligned16(w_down) &&
                     ldx % 8 == 0 && sd_aligned16(x) && (!x_bf16 || sd_aligned16(x_bf16));
-  // (tiles of 128 rows for experts with many rows, the template's MT = 8 with chunks of 128 columns,
-  // measured slower than tiles of 32: 95-156 against 153-183 TFLOP/s at 1024-2048 rows)
-  const int bm = kMoeBM;
+  // With the rows as bf16 already: both operands through LDS.  Two gated matrices and the last of 16 experts 2048 x 2048,
+  // against the kernel that converts f32 rows (the call, 2 experts a row): 64 rows 121 -> 106 us, 512 202 -> 127, 1024
+  // 325 -> 162, 2048 532 -> 231 (446 TFLOP/s); 64 experts 768 wide 155 -> 135 already at 2 rows an expert.  Tiles of 32
+  // rows are no quicker anywhere and 198, 320 us at 1024, 2048 rows.
+  const size_t x_bytes = (size_t)n_rows * ldx * 2, act_bytes = (size_t)n_rows * top * F * 2,
+               gu_bytes = (size_t)F * W * (act_kind == 1 ? 2 : 4), down_bytes = (size_t)F * W * 2;
+  const int n = n_rows * top;
+  const bool lds_rows = mfma && x_bf16 && n > kMoeDirect && sd_aligned16(out) && x_bytes < kOutside &&
+                        act_bytes < kOutside && gu_bytes < kOutside && down_bytes < kOutside;
+  const int bm = lds_rows ? kMoeLdsBM : kMoeBM;
   int tiles_y = n;
   if (n <= kMoeDirect) {   // a few assignments: each runs as a tile of its own, straight from the router's choice
     perm = const_cast<int32_t*>(sel_expert);
@@ -2292,6 +2437,18 @@ extern "C" int sd_moe_experts_clamped(const float* x, const void* x_bf16, int64_
     SD_CHECK_LAUNCH("sd_moe_experts (gate, up)");
     moe_gemv_down_kernel<<<dim3((W + 15) / 16, n), 256, sizeof(float) * F, st>>>(
         act_b, sel_expert, sel_weight, (const bf16_t*)w_down, out, E, W, F, scale_input);
+  } else if (lds_rows) {
+    bf16_t* act_b = (bf16_t*)act;
+    MoeArgs g{(const bf16_t*)x_bf16, ldx, (unsigned)x_bytes, (unsigned)gu_bytes, perm, tiles, n_tiles, sel_weight,
+              (const bf16_t*)w_gate_up, act_b, nullptr, top, E, F, W, scale_input, act_kind, limit};
+    if (act_kind != 1)
+      moe_rows_kernel<kMoeLdsBM, kGated><<<dim3((F + kMoeCols / 2 - 1) / (kMoeCols / 2), tiles_y), 256, 0, st>>>(g);
+    else
+      moe_rows_kernel<kMoeLdsBM, kSquare><<<dim3((F + kMoeCols - 1) / kMoeCols, tiles_y), 256, 0, st>>>(g);
+    SD_CHECK_LAUNCH("sd_moe_experts (gate, up)");
+    MoeArgs d{act_b, F, (unsigned)act_bytes, (unsigned)down_bytes, perm, tiles, n_tiles, sel_weight, (const bf16_t*)w_down,
+              nullptr, out, 1, E, W, F, scale_input, act_kind, limit};
+    moe_rows_kernel<kMoeLdsBM, kDown><<<dim3((W + kMoeCols - 1) / kMoeCols, tiles_y), 256, 0, st>>>(d);
   } else if (mfma) {
     // (act holds n * F floats: its first half serves as the bf16 activations)
     bf16_t* act_b = (bf16_t*)act;

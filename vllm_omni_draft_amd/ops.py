@@ -1950,9 +1950,10 @@ def moe_route_rows(x, w_router, top, score="sigmoid", renorm=False):
     return sel_e, sel_w, logits
 
 
-def moe_experts(x, sel_e, sel_w, w_gate_up, w_down, scale_input=True, act="silu") -> torch.Tensor:
+def moe_experts(x, sel_e, sel_w, w_gate_up, w_down, scale_input=True, act="silu", bf16_copy=False) -> torch.Tensor:
     """x f32 [rows, W]; w_gate_up [E, 2F, W], w_down [E, W, F]; returns f32 [rows, top, W]: every
-    chosen expert's result.  act "relu2": experts of two matrices, w_gate_up is [E, F, W]. """
+    chosen expert's result.  act "relu2": experts of two matrices, w_gate_up is [E, F, W].  bf16_copy: give the
+    rows as bf16 too, as a layer does (groups of many rows take them)."""
     _f32(x, "x")
     n, W = x.shape
     top, E, F = sel_e.shape[1], w_gate_up.shape[0], w_down.shape[2]
@@ -1960,7 +1961,8 @@ def moe_experts(x, sel_e, sel_w, w_gate_up, w_down, scale_input=True, act="silu"
     nb = int(lib.sd_moe_experts_scratch_bytes(n, top, E, F, W))
     scratch = torch.empty(nb, dtype=torch.uint8, device=x.device)
     out = torch.empty(n, top, W, dtype=torch.float32, device=x.device)
-    _lib.check(lib.sd_moe_experts(_p(x), None, W, _p(sel_e), _p(sel_w), _p(w_gate_up), _p(w_down), _wkind(w_down, "w_down"),
+    xb = x.to(torch.bfloat16) if bf16_copy else None
+    _lib.check(lib.sd_moe_experts(_p(x), _p(xb), W, _p(sel_e), _p(sel_w), _p(w_gate_up), _p(w_down), _wkind(w_down, "w_down"),
                                   _p(out), n, top, E, F, W, int(scale_input), {"silu": 0, "relu2": 1}[act], _p(scratch),
                                   nb, _stream()),
                "sd_moe_experts")

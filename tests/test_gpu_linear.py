@@ -673,3 +673,22 @@ def test_prompt_linear_has_the_bits_of_the_wide_kernels(M, N, K):
                                              None if r is None else r[i:i + 256].contiguous(), epi)
                              for i in range(0, M, 256)])
             assert torch.equal(got, few), (epi, b is not None)
+
+
+@pytest.mark.parametrize("N,K,epi", [(19000, 128, "F32"), (18008, 192, "F32"), (16400, 640, "F32"), (8200, 256, "SILU_MUL"),
+                                     (1000, 4096, "RESIDUAL"), (272, 2112, "STORE"), (3072, 2048, "STORE")])
+def test_wide_rows_have_their_bits_at_every_row_count(N, K, epi):
+    """Row counts at the edges of the kernels' blocks of rows and of the rules between kernels, matrices that end inside a
+    block of weights and whose splits of K are of different lengths: every row has the bits that it has among 17."""
+    from vllm_omni_draft_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(N + K)
+    kind = getattr(ops, "EPI_" + epi)
+    W = ops._tiled((torch.randn(2 * N if epi == "SILU_MUL" else N, K, generator=g, device="cuda") * 0.05).bfloat16(), kind)
+    x = torch.randn(256, K, generator=g, device="cuda").bfloat16()
+    res = torch.randn(256, N, generator=g, device="cuda").bfloat16() if epi == "RESIDUAL" else None
+
+    def run(lo, hi):
+        return ops.linear_wide(W, x[lo:hi], None, None if res is None else res[lo:hi], kind)
+    want = torch.cat([run(r, min(r + 17, 256)) for r in range(0, 256, 17)])
+    for m in (32, 33, 64, 65, 96, 128, 129, 192, 193, 255, 256):
+        assert torch.equal(run(0, m), want[:m]), m

@@ -1003,6 +1003,12 @@ int wide_common(const void* W, const void* x, int64_t ldx, int M, int K, int n_t
   e.NR = n_tiles * 16;
   a.epi = e;
   const int mt = (M + 15) / 16;
+#ifndef SD_WIDE_F32_ONLY
+  if (!e.w_scale && sd_rows_linear_fits_(M, n_tiles, K, ldx, S, ksp, epi)) {  // (the same bits)
+    const int rc = sd_rows_linear_(W, x, ldx, M, K, n_tiles, S, ksp, epi, e, (float*)workspace, st);
+    return rc != SD_OK || S == 1 ? rc : epilogue_by_kind(e, epi, st);
+  }
+#endif
   if (S == 1) return gemm_by_rows<true>(a, mt, epi, S, st);
   const int rc = gemm_by_rows<false>(a, mt, epi, S, st);
   if (rc != SD_OK) return rc;

@@ -31,11 +31,13 @@ struct PromptArgs {
   const bf16_t* x;
   int64_t ldx;
   int M, KS, n_tiles, ks_per_split;
-  int n_blocks, m_blocks;  // grid = n_blocks * m_blocks
+  int n_blocks, m_blocks;  // grid = n_blocks * m_blocks (* splits: EPI_PARTIAL)
+  float* part;             // EPI_PARTIAL: [splits][M][n_tiles * 16]
   WideEpiArgs epi;
 };
 
 typedef __attribute__((address_space(3))) void lds_void;
+constexpr int EPI_PARTIAL = -1;  // the sums of one split of K, for wide_epilogue_kernel
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, unsigned bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00027000);
@@ -66,17 +68,20 @@ __global__ __launch_bounds__(256, SPLIT ? 2 : 1) void prompt_gemm_kernel(PromptA
   constexpr int kAPieces = BN * 2 / 4, kBPieces = BM / 8 / 4;  // 1 KiB direct loads per wave and stage
   __shared__ __attribute__((aligned(1024))) char s0[kABytes + kBBytes];
   __shared__ __attribute__((aligned(1024))) char s1[kABytes + kBBytes];
-  __shared__ __attribute__((aligned(1024))) char s2[STAGES == 4 ? kABytes + kBBytes : 1024];
+  __shared__ __attribute__((aligned(1024))) char s2[STAGES >= 3 ? kABytes + kBBytes : 1024];
   __shared__ __attribute__((aligned(1024))) char s3[STAGES == 4 ? kABytes + kBBytes : 1024];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int work = xcd_order(blockIdx.x, gridDim.x);
+  const int blocks = EPI == EPI_PARTIAL ? a.n_blocks * a.m_blocks : (int)gridDim.x;
+  const int split = EPI == EPI_PARTIAL ? (int)blockIdx.x / blocks : 0;
+  const int work = xcd_order(blockIdx.x - split * blocks, blocks);
   const int grp = work / (a.n_blocks * kRowGroup), in_grp = work - grp * a.n_blocks * kRowGroup;
   const int grp_rows = min(kRowGroup, a.m_blocks - grp * kRowGroup);
   const int nb = in_grp / grp_rows, mb = grp * kRowGroup + in_grp - nb * grp_rows;
   const int tile0 = nb * BN, row0 = mb * BM;
-  const int n_it = a.KS >> 1;
+  const int k0 = split * a.ks_per_split;               // first k-step (EPI_PARTIAL)
+  const int n_it = EPI == EPI_PARTIAL ? min(a.ks_per_split, a.KS - k0) >> 1 : a.KS >> 1;
 
   // this wave's direct loads: weights, piece p = (tile p >> 1, k-step p & 1) of the block's tiles
   const char* wbase = reinterpret_cast<const char*>(a.W) + (size_t)tile0 * a.KS * 1024;
@@ -95,11 +100,11 @@ __global__ __launch_bounds__(256, SPLIT ? 2 : 1) void prompt_gemm_kernel(PromptA
       const int p = wave + 4 * i;
       // (the tile is part of the lane offset: that is what the bounds check sees)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_void*)(s + p * 1024), 16, lane * 16 + (p >> 1) * w_step,
-                                               (2 * it + (p & 1)) * 1024, 0, 0);
+                                               (k0 + 2 * it + (p & 1)) * 1024, 0, 0);
     } else {
       const int p = wave + 4 * (i - kAPieces);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void*)(s + kABytes + p * 1024), 16, x_lane + p * x_step,
-                                               it * 128, 0, 0);
+                                               k0 * 64 + it * 128, 0, 0);
     }
   };
 
@@ -110,7 +115,8 @@ __global__ __launch_bounds__(256, SPLIT ? 2 : 1) void prompt_gemm_kernel(PromptA
   const int b_sw[2] = {((xq ^ (xc & 7)) << 4), (((xq + 4) ^ (xc & 7)) << 4)};
   bf16x8 fa[2][TN], fb[2][TM];
   constexpr int kReads = TN + TM, kMfma = TN * TM;
-  static_assert(kReads <= kMfma * 3 / 4, "at most one LDS read an MFMA");
+  constexpr int kOver = kMfma * 3 / 4 > kReads ? kMfma * 3 / 4 : kReads;
+  static_assert(kReads <= kMfma && kPieces <= kMfma, "at most one LDS read and one direct load an MFMA");
   auto read_piece = [&](const char* s, int ks, int i) __attribute__((always_inline)) {
     if (i < TN)
       fa[ks][i] = *reinterpret_cast<const bf16x8*>(s + a_off + i * 2048 + ks * 1024);
@@ -155,7 +161,6 @@ __global__ __launch_bounds__(256, SPLIT ? 2 : 1) void prompt_gemm_kernel(PromptA
     for (int n = 0; n < kMfma; ++n) {
       mfma(ks, n / TM, n % TM);
       // (the reads in the first three quarters: the last one has its latency behind it at the phase's end)
-      constexpr int kOver = kMfma * 3 / 4;
       if (n < kOver && (n + 1) * kReads / kOver > n * kReads / kOver) read_piece(from, ks ^ 1, n * kReads / kOver);
       if (kLoads && (n + 1) * kPieces / kMfma > n * kPieces / kMfma) stage_piece(to, it, n * kPieces / kMfma);
     }
@@ -188,10 +193,8 @@ __global__ __launch_bounds__(256, SPLIT ? 2 : 1) void prompt_gemm_kernel(PromptA
   };
   fill(s0, 0);
   fill(s1, 1);
-  if constexpr (STAGES == 4) {
-    fill(s2, 2);
-    fill(s3, 3);
-  }
+  if constexpr (STAGES >= 3) fill(s2, 2);
+  if constexpr (STAGES == 4) fill(s3, 3);
   meet<(STAGES - 1) * kPieces>();
 #pragma unroll
   for (int i = 0; i < kReads; ++i) read_piece(s0, 0, i);
@@ -207,6 +210,14 @@ __global__ __launch_bounds__(256, SPLIT ? 2 : 1) void prompt_gemm_kernel(PromptA
     if (it < n_it) step(s0, s1, it);
     if (it + 1 < n_it) step(s1, s2, it + 1);
     if (it + 2 < n_it) step(s2, s3, it + 2);
+  } else if constexpr (STAGES == 3) {
+    for (; it + 2 < n_it; it += 3) {
+      step(s0, s1, it);
+      step(s1, s2, it + 1);
+      step(s2, s0, it + 2);
+    }
+    if (it < n_it) step(s0, s1, it);
+    if (it + 1 < n_it) step(s1, s2, it + 1);
   } else {
     for (; it + 1 < n_it; it += 2) {
       step(s0, s1, it);
@@ -236,14 +247,19 @@ __global__ __launch_bounds__(256, SPLIT ? 2 : 1) void prompt_gemm_kernel(PromptA
   for (int j = 0; j < TM; ++j) {
 #pragma unroll
     for (int i = 0; i < TN; ++i) *reinterpret_cast<f32x4*>(img + xc * kLd + i * 16 + 4 * xq) = acc[i][j];
+    asm volatile("" ::: "memory");  // (other lanes read them: the stores of a lane without a unit stay here)
 #pragma unroll 1
-    for (int r = lane / kUnits; r < 16; r += 64 / kUnits) {
+    for (int r = lane < 64 / kUnits * kUnits ? lane / kUnits : 16; r < 16; r += 64 / kUnits) {
       const int m = row0 + (wm * TM + j) * 16 + r;
       const float* src = img + r * kLd + ui * 16 + r0;
       const f32x4 lo = *reinterpret_cast<const f32x4*>(src);
       f32x4 hi = zero;
       if (PAIRED) hi = *reinterpret_cast<const f32x4*>(src + 8);
-      if (tile < a.n_tiles && m < a.M) emit_unit<EPI>(a.epi, m, tile, r0, lo, hi);
+      if (tile < a.n_tiles && m < a.M) {
+        if constexpr (EPI == EPI_PARTIAL)
+          *reinterpret_cast<f32x4*>(a.part + ((size_t)split * a.M + m) * a.n_tiles * 16 + tile * 16 + r0) = lo;
+        else emit_unit<EPI>(a.epi, m, tile, r0, lo, hi);
+      }
     }
   }
 }
@@ -255,6 +271,36 @@ int launch_prompt(PromptArgs a, hipStream_t st) {
   hipLaunchKernelGGL((prompt_gemm_kernel<TN, TM, STAGES, SPLIT, EPI>), dim3(a.n_blocks * a.m_blocks), dim3(256), 0, st, a);
   SD_CHECK_LAUNCH("sd_prompt_linear");
   return SD_OK;
+}
+
+// ---- passes of at most 256 rows: one block holds all of them, so every weight is read once; four waves, three stages.
+// The MFMAs need the accumulators in place here too; 192 rows x 10 weight tiles a block are 120 of them a lane.
+template <int TN, int EPI>
+int launch_few(PromptArgs a, int S, hipStream_t st) {
+  a.n_blocks = (a.n_tiles + 2 * TN - 1) / (2 * TN);
+  a.m_blocks = 1;
+  const dim3 grid(a.n_blocks * S);
+  if (a.M <= 64) hipLaunchKernelGGL((prompt_gemm_kernel<TN, 2, 3, false, EPI>), grid, dim3(256), 0, st, a);
+  else if (a.M <= 128) hipLaunchKernelGGL((prompt_gemm_kernel<TN, 4, 3, false, EPI>), grid, dim3(256), 0, st, a);
+  else if (a.M <= 192) hipLaunchKernelGGL((prompt_gemm_kernel<TN, 6, 3, false, EPI>), grid, dim3(256), 0, st, a);
+  else hipLaunchKernelGGL((prompt_gemm_kernel<TN, 8, 3, false, EPI>), grid, dim3(256), 0, st, a);
+  SD_CHECK_LAUNCH("sd_rows_linear");
+  return SD_OK;
+}
+
+// Tiles a wave of a matrix whose K is whole: the fewest rounds of 256 blocks x tiles a block, larger blocks where that is
+// the same.
+int few_cost(int n_tiles, int tn) { return ((n_tiles + 2 * tn - 1) / (2 * tn) + 255) / 256 * tn; }
+int few_tiles(int n_tiles) {
+  const int c2 = few_cost(n_tiles, 2), c4 = few_cost(n_tiles, 4), c5 = few_cost(n_tiles, 5);
+  return c5 <= c4 && c5 <= c2 ? 5 : c4 <= c2 ? 4 : 2;
+}
+
+template <int EPI>
+int few_shape(const PromptArgs& a, hipStream_t st) {
+  const int tn = few_tiles(a.n_tiles);
+  if (tn == 5) return launch_few<5, EPI>(a, 1, st);
+  return tn == 4 ? launch_few<4, EPI>(a, 1, st) : launch_few<2, EPI>(a, 1, st);
 }
 
 template <int EPI>
@@ -276,6 +322,30 @@ bool sd_prompt_linear_fits_(int M, int n_tiles, int K, int64_t ldx) {
   return M > 256 && K % 64 == 0 && K >= 128 && (blocks > 64 || K <= 4096) && 512 * ldx < 0x7fffffff;
 }
 
+// At most 256 rows: the products themselves (splits of K: the partial sums, for the caller's epilogue kernel).  Against
+// the wide kernels, whose weights go through registers, with the epilogue's launch, weights from memory (us):
+//   whole K, one round of blocks (gate and up of 8192 x 2048, 14336 x 4096, 18944 x 3584): 24 rows 20.7 -> 17.4, 44.3 ->
+//   46.2, 56.1 -> 53.1, so not below 33; 128 rows 27.9 -> 20.2, 55.8 -> 55.5, 72.8 -> 60.2; 256 rows 42 -> 27, 76 -> 68,
+//   127 -> 81 (the wide kernels leave CUs without a group, and spill at 256 rows);
+//   more rounds (heads of 128256 x 2048, 152064 x 3584): 128 rows 110 -> 122, 228 -> 249; 256 rows 180 -> 154, 331 -> 317;
+//   splits of 512 columns or more: 64 rows even, 96 rows 23.4 -> 20.1 (6144 x 4096) and never slower, 256 rows 62 -> 50
+//   (3584 x 18944); of 256 columns: 96 rows 15.0 -> 15.3, 128 rows even, 256 rows 22.9 -> 20.2 (3072 x 2048); of 128
+//   columns (2 stages) 5% slower up to 192 rows.
+bool sd_rows_linear_fits_(int M, int n_tiles, int K, int64_t ldx, int S, int ks_per_split, int epi) {
+  if (M > 256 || K % 64 != 0 || K < 128 || 512 * ldx >= 0x7fffffff) return false;
+  if (S > 1) return M > 64 && (ks_per_split >= 16 || (M > 128 && ks_per_split >= 8));
+  const int tn = few_tiles(n_tiles);
+  return M > 32 && (epi == SD_EPI_SILU_MUL || epi == SD_EPI_F32) && (M > 192 || few_cost(n_tiles, tn) == tn);
+}
+
+int sd_rows_linear_(const void* W, const void* x, int64_t ldx, int M, int K, int n_tiles, int S, int ks_per_split, int epi,
+                    const WideEpiArgs& epi_args, float* part, sd_stream_t stream) {
+  PromptArgs a{(const bf16_t*)W, (const bf16_t*)x, ldx, M, K / 32, n_tiles, ks_per_split, 0, 0, part, epi_args};
+  hipStream_t st = (hipStream_t)stream;
+  if (S > 1) return launch_few<4, EPI_PARTIAL>(a, S, st);
+  return epi == SD_EPI_F32 ? few_shape<SD_EPI_F32>(a, st) : few_shape<SD_EPI_SILU_MUL>(a, st);
+}
+
 // epi: an SD_EPI_* number or EPI_QKV_ROPE, with what that epilogue reads in `e`.
 int sd_prompt_linear_(const void* W, const void* x, int64_t ldx, int M, int K, int n_tiles, int epi,
                       const WideEpiArgs& epi_args, sd_stream_t stream) {
@@ -285,7 +355,7 @@ int sd_prompt_linear_(const void* W, const void* x, int64_t ldx, int M, int K, i
   e.NR = n_tiles * 16;
   e.S = 1;
   plan_split(n_tiles, K, S, ksp, g);
-  PromptArgs a{(const bf16_t*)W, (const bf16_t*)x, ldx, M, K / 32, n_tiles, ksp, 0, 0, e};
+  PromptArgs a{(const bf16_t*)W, (const bf16_t*)x, ldx, M, K / 32, n_tiles, ksp, 0, 0, nullptr, e};
   hipStream_t st = (hipStream_t)stream;
   switch (epi) {
     case SD_EPI_F32: return prompt_shape<SD_EPI_F32>(a, S, st);

@@ -231,6 +231,9 @@ using namespace sd_wide;
 
 // sd_prompt.hip: the shapes its kernels are the better choice for (every other call goes through sd_linear_wide's in
 // blocks of 256 rows; same bits), and the call.  epi: an SD_EPI_* number or EPI_QKV_ROPE with what that reads in `e`.
+bool sd_rows_linear_fits_(int M, int n_tiles, int K, int64_t ldx, int S, int ks_per_split, int epi);
+int sd_rows_linear_(const void* W, const void* x, int64_t ldx, int M, int K, int n_tiles, int S, int ks_per_split, int epi,
+                    const sd_wide::WideEpiArgs& epi_args, float* part, sd_stream_t stream);
 bool sd_prompt_linear_fits_(int M, int n_tiles, int K, int64_t ldx);
 int sd_prompt_linear_(const void* W, const void* x, int64_t ldx, int M, int K, int n_tiles, int epi,
                       const WideEpiArgs& e, sd_stream_t stream);

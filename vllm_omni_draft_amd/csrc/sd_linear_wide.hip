@@ -12,6 +12,9 @@
 // (waves without a second tile still pay for it); 4-wave workgroups of 8 tiles, two per CU,
 // with 64-column chunks (the x staging latency of a chunk is then longer than the chunk).
 //
+// bf16 passes of more than 32 rows over many of the matrices run on sd_prompt.hip's kernel instead, with the same bits
+// (sd_rows_linear_fits_ says which, and by how much it is faster).
+//
 // wide_gemm4_kernel (further down) serves the many-row passes of some matrices with another
 // chunk structure on four waves; same tiles, same sums, same bits.
 //

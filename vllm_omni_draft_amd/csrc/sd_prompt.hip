@@ -1,5 +1,5 @@
-// Linear layers over more than 256 token rows (prompt passes) on the tiled bf16 weights of the other linear
-// kernels.
+// Linear layers over more than 256 token rows (prompt passes), and over 33..256 where that is faster than sd_linear_wide's
+// kernels, on the tiled bf16 weights of the other linear kernels.
 //
 // sd_linear_wide's kernels stream the weights past at most 256 rows held in LDS; a prompt of 1024 rows read
 // every weight four times, split K over workgroups whenever a matrix had fewer than 128 groups (partial sums of

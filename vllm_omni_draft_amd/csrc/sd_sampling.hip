@@ -1020,8 +1020,7 @@ __device__ int pick_from_parts(const float* __restrict__ p, const float* __restr
   __shared__ int s_i[kPartThreads / 64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // the masses before every slice, summed in order, and the slice that holds u's share: a lane a slice (one thread for
-  // all: 64 reads, two walks; 13.0 and 10.6 us for 8 rows of
-  // 128256 in the two launches that pick, now 7.4 and 5.1)
+  // all: 64 reads, two walks; 13.0 and 10.6 us for 8 rows of 128256 in the two launches that pick, now 7.4 and 5.1)
   static_assert(kRowParts == 64, "a slice a lane");
   if (wave == 0) {
     const double m = sc.mass[(size_t)r * kRowParts + lane];

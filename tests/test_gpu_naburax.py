@@ -740,3 +740,37 @@ def test_moe_experts_of_many_rows_have_the_bits_of_few(E, F, W, n, act, scale_in
         sel[:full, 0] = 0
         a = ops.moe_experts(x, sel, sel_w, gu, dn, scale_input, act, bf16_copy=True)
         assert torch.equal(a, ops.moe_experts(x, sel, sel_w, gu, dn, scale_input, act)), full
+
+
+def same_where_finite(got, want, tol=1e-5):
+    """The same entries are finite in both, and those agree."""
+    assert torch.equal(torch.isfinite(got), torch.isfinite(want))
+    ok = torch.isfinite(want)
+    assert (got - want)[ok].abs().max() <= tol * want[ok].abs().max()
+
+
+@pytest.mark.parametrize("H,G,dk,dv,window,keep", [(4, 2, 128, 128, 5000, 0), (6, 1, 128, 128, 40, 3), (3, 1, 576, 512, 5000, 0)])
+def test_rows_softmax_attention_of_scores_that_are_no_numbers(H, G, dk, dv, window, keep):
+    """Queries and keys with infinities and NaN (keys before the portion, so that every row or none sees them): the rows
+    that come out finite are those of the kernel on the vector pipe, an infinite score of the right sign is a weight of 0
+    (queries of few bits too, whose lower parts are 0), and nothing not a number is left out of a sum."""
+    from vllm_omni_draft_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(dk + window)
+    p0, n = 100, 70
+    pages = (p0 + n + 15) // 16
+    bt = torch.randperm(pages, generator=g, device="cuda").to(torch.int32).view(1, pages)
+    kc = torch.randn(pages, G, 16, dk, generator=g, device="cuda").to(torch.bfloat16)
+    vc = None if dv == 512 else torch.randn(pages, G, 16, dv, generator=g, device="cuda").to(torch.bfloat16)
+    q = torch.randn(n, H * dk, generator=g, device="cuda")
+    q[::2] = q[::2].to(torch.bfloat16).float()
+    q[5, 3], q[9, dk + 7], q[12, 1] = float("nan"), float("inf"), float("-inf")
+    at = lambda p: (bt[0, p // 16].long(), 0, p % 16)
+    if vc is not None:      # (a latent row's channels are values too)
+        kc[at(70)][4] = float("-inf")
+        if window > p0:
+            kc[at(20)][9] = float("inf")
+    pos, slot = i32(range(p0, p0 + n)), i32([0] * n)
+    want = ops.window_softmax_attention(q, kc, vc, pos, slot, bt, H, G, dk, dv, window, keep, 0.0625)
+    got = ops.rows_softmax_attention(q, kc, vc, bt, i32([[0, 0, n, p0]]), H, G, dk, dv, window, keep, 0.0625)
+    assert not torch.isfinite(want).all()
+    same_where_finite(got, want)

@@ -666,3 +666,28 @@ def test_head_decay_in_chunks_against_the_recurrence(H, Gq, dk, dv, per_row, len
     got = ops.head_decay_chunks(dev(q), dev(k), dev(v), dev(decay), S1, e, dev(scale), dev(skip))
     off = lambda a, b: ((a.double().cpu() - b).norm() / b.norm()).item()
     assert off(got, want) < 1e-6 and off(S1, S_want) < 1e-6
+
+
+@pytest.mark.parametrize("H,G,window,pool", [(4, 2, 60, 16), (6, 1, 33, 5)])
+def test_rows_pool_attention_of_scores_that_are_no_numbers(H, G, window, pool):
+    """Queries, keys and a head's bias with infinities and NaN (keys before the portion): finite where the kernel on the
+    vector pipe is, a score of plus infinity weighs 1 and one of minus infinity 0, a NaN stays one."""
+    from vllm_omni_draft_amd import ops
+    g = torch.Generator().manual_seed(H + window)
+    p0, n, d = 96, 70, 128
+    k, v = (torch.randn(p0 + n, G * d, generator=g).to(torch.bfloat16).float() for _ in range(2))
+    q, bias = torch.randn(n, H * d, generator=g), torch.randn(H, generator=g)
+    q[::2] = q[::2].to(torch.bfloat16).float()
+    q[5, 3], q[9, d + 7], q[12, 1] = float("nan"), float("inf"), float("-inf")
+    k[90, 4], k[93, 9] = float("inf"), float("-inf")
+    bias[0] = float("inf")
+    bed = _AttnBed(G, d, d, pool, p0 + n, torch.bfloat16)
+    bed.append(k[:p0], v[:p0], list(range(p0)))
+    bed.attend(torch.zeros(p0, H * d), list(range(p0)), H, window, 1.0, None)   # (fills the pooled blocks)
+    bed.append(k[p0:], v[p0:], list(range(p0, p0 + n)))
+    want = bed.attend(q, list(range(p0, p0 + n)), H, window, 0.0625, bias)
+    got = ops.rows_pool_attention(dev(q), bed.k, bed.v, bed.pk, bed.pv, bed.tables, i32([[0, 0, n, p0]]), H, G, d, d, window,
+                                  pool, 0.0625, dev(bias))
+    bad = ~torch.isfinite(want)
+    assert bad.any() and not bad.all() and torch.equal(~torch.isfinite(got), bad)
+    assert (got - want)[~bad].abs().max() <= 1e-5 * want[~bad].abs().max()

@@ -18,6 +18,7 @@
 // 2048 rows of 16 heads over 4 with a window of 1024 and pooled blocks 789 -> 73 us.
 // A non-finite value at a position of the portion itself can reach rows of up to 63 positions before it.
 #include <math.h>
+#include <type_traits>
 
 #include "sd_common.h"
 
@@ -47,28 +48,31 @@ typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 constexpr int kPage = 16, kKeys = 64, kRowsPerBlock = 64, kPooled = 32;
 
 // Two f32 values as three pairs of bf16 whose sums they are: 8 bits of the significand each, cut off (the differences
-// are exact), the first value in the low halves.
+// are exact), the first value in the low halves.  INF: the values may be infinite, and are their first part then.
+template <bool INF = false>
 __device__ __forceinline__ void three_parts(float x, float y, unsigned& a, unsigned& b, unsigned& c) {
   auto upper = [](float v) { return __uint_as_float(__float_as_uint(v) & 0xffff0000u); };
   auto pack = [](float u, float v) { return __builtin_amdgcn_perm(__float_as_uint(v), __float_as_uint(u), 0x07060302u); };
-  const float xr = x - upper(x), yr = y - upper(y);
+  auto rest = [&](float v) { return INF && fabsf(v) == INFINITY ? 0.f : v - upper(v); };
+  const float xr = rest(x), yr = rest(y);
   a = pack(x, y);
   b = pack(xr, yr);
   c = pack(xr - upper(xr), yr - upper(yr));
 }
 
 // e^x for x <= 0 (-inf: 0), to about one unit in the last place: the product with log2 e in two parts, no branch.
+// (The limits here and below let a NaN through, as fmaxf would not: one instruction either way.)
 __device__ __forceinline__ float exp_neg(float x) {
-  x = fmaxf(x, -200.f);   // (e^-200 is 0 in f32)
+  x = __builtin_elementwise_maximum(x, -200.f);   // (e^-200 is 0 in f32)
   const float hi = x * 1.44269502f;
   const float lo = fmaf(x, 1.92596300e-8f, fmaf(x, 1.44269502f, -hi));
   const float y = __builtin_amdgcn_exp2f(hi);
   return fmaf(y, lo * 0.693147181f, y);
 }
 
-// 1 / (1 + e^-x), to about two units in the last place (below e^-87: 0 or next to it)
+// 1 / (1 + e^-x), to about two units in the last place (below e^-87: 0 or next to it; +inf: 1)
 __device__ __forceinline__ float sigmoid_of(float x) {
-  x = -fmaxf(x, -87.f);
+  x = -__builtin_elementwise_minimum(__builtin_elementwise_maximum(x, -87.f), 87.f);
   const float hi = x * 1.44269502f;
   const float lo = fmaf(x, 1.92596300e-8f, fmaf(x, 1.44269502f, -hi));
   const float y = __builtin_amdgcn_exp2f(hi);
@@ -121,12 +125,12 @@ __global__ __launch_bounds__(256, KS > 4 ? 1 : 2) void rows_attn_kernel(RowsAttn
   constexpr bool kKept = KS <= 4;
   f32x4 qf[kKept ? 1 : KS][2];
   bf16x8 qp[kKept ? KS : 1][3];
-  auto parts = [&](const f32x4 (&x)[2], bf16x8 (&y)[3]) __attribute__((always_inline)) {
+  auto parts = [&](const f32x4 (&x)[2], bf16x8 (&y)[3], auto inf) __attribute__((always_inline)) {
     u32x4 a, b, c;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       unsigned pa, pb, pc;
-      three_parts(x[i >> 1][2 * (i & 1)], x[i >> 1][2 * (i & 1) + 1], pa, pb, pc);
+      three_parts<decltype(inf)::value>(x[i >> 1][2 * (i & 1)], x[i >> 1][2 * (i & 1) + 1], pa, pb, pc);
       a[i] = pa;
       b[i] = pb;
       c[i] = pc;
@@ -135,17 +139,15 @@ __global__ __launch_bounds__(256, KS > 4 ? 1 : 2) void rows_attn_kernel(RowsAttn
     y[1] = __builtin_bit_cast(bf16x8, b);
     y[2] = __builtin_bit_cast(bf16x8, c);
   };
-  {
-    const float* qr = g.q + (size_t)(row0 + first + t) * g.ldq + (size_t)h * DK + 8 * quad;
+  const float* qr = g.q + (size_t)(row0 + first + t) * g.ldq + (size_t)h * DK;
 #pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      const f32x4 x[2] = {*reinterpret_cast<const f32x4*>(qr + 32 * s) * g.scale,
-                          *reinterpret_cast<const f32x4*>(qr + 32 * s + 4) * g.scale};
-      if constexpr (kKept) parts(x, qp[s]);
-      else {
-        qf[s][0] = x[0];
-        qf[s][1] = x[1];
-      }
+  for (int s = 0; s < KS; ++s) {
+    const f32x4 x[2] = {*reinterpret_cast<const f32x4*>(qr + 32 * s + 8 * quad) * g.scale,
+                        *reinterpret_cast<const f32x4*>(qr + 32 * s + 8 * quad + 4) * g.scale};
+    if constexpr (kKept) parts(x, qp[s], std::true_type{});
+    else {
+      qf[s][0] = x[0];
+      qf[s][1] = x[1];
     }
   }
   // wave w brings page w of the stage (behind the stage's last key: that key's page), its number asked for a stage ahead
@@ -246,6 +248,24 @@ __global__ __launch_bounds__(256, KS > 4 ? 1 : 2) void rows_attn_kernel(RowsAttn
                                                       sc[u][i], o[v], 0, 0, 0);
       }
   };
+  // The scores again, term by term: a part of a query that is 0 makes a NaN of an infinite key, where the query's product
+  // with it is infinite and its weight a number.
+  auto plain_scores = [&](const char* s, f32x4 (&sc)[4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) sc[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int c = 0; c < DK; ++c) {
+      const float x = qr[c] * g.scale;
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int r = 4 * quad + i;
+          const char* at = s + u * kKeyPage + r * DK * 2 + (c >> 6) * 128 + ((((c >> 3) & 7) ^ (r & 7)) << 4) + (c & 7) * 2;
+          sc[u][i] = fmaf(x, (float)*reinterpret_cast<const bf16_t*>(at), sc[u][i]);
+        }
+    }
+  };
   auto attend = [&](const char* s, int st) __attribute__((always_inline)) {
     const int base = stage_base(st);
     // (a stage of kept tokens holds no key of the window; in the window's stages kept tokens are seen too)
@@ -267,47 +287,74 @@ __global__ __launch_bounds__(256, KS > 4 ? 1 : 2) void rows_attn_kernel(RowsAttn
       } else {
         f32x4 x[2] = {qf[ks][0], qf[ks][1]};
         asm volatile("" : "+v"(x[0]), "+v"(x[1]));   // (or the parts would be formed ahead of the loop and kept)
-        parts(x, y);
+        parts(x, y, std::false_type{});
       }
 #pragma unroll
       for (int c = 0; c < 3; ++c)
 #pragma unroll
         for (int u = 0; u < 4; ++u) sc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], y[c], sc[u], 0, 0, 0);
     }
-    if constexpr (POOLED) {
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int d = p - (base + 16 * u + 4 * quad + i);
-          const float wt = sigmoid_of(sc[u][i] + bias);
-          sc[u][i] = ((d >= 0) & (d < g.window)) ? wt : 0.f;
-        }
-    } else {
-      float mx = m_run;
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int j = base + 16 * u + 4 * quad + i, d = p - j;
-          // (bitwise: a chain of && would become branches)
-          const bool seen = (d >= 0) & ((d < g.window) | (j < g.keep_first)) & (j < key_end);
-          sc[u][i] = seen ? sc[u][i] : -INFINITY;
-          mx = fmaxf(mx, sc[u][i]);
-        }
-      mx = fmaxf(mx, __shfl_xor(mx, 16, SD_WAVE));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, SD_WAVE));
-      const float ref = mx == -INFINITY ? 0.f : mx;            // (no key seen yet)
-      const float corr = exp_neg(m_run - ref);   // (nothing summed yet: 0)
-      m_run = mx;
+    // The weights of a stage's scores in their place: the new maximum, the factor of what has been summed, the sum of the
+    // weights (a query's is spread over its four lanes; pooled: only whether it is a number matters)
+    auto weigh = [&](f32x4 (&x)[4], float& mx, float& corr) __attribute__((always_inline)) {
       float sum = 0.f;
+      mx = m_run;
+      if constexpr (POOLED) {
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
+        for (int u = 0; u < 4; ++u)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          sc[u][i] = exp_neg(sc[u][i] - ref);
-          sum += sc[u][i];
-        }
+          for (int i = 0; i < 4; ++i) {
+            const int d = p - (base + 16 * u + 4 * quad + i);
+            const float wt = sigmoid_of(x[u][i] + bias);
+            x[u][i] = ((d >= 0) & (d < g.window)) ? wt : 0.f;
+            sum += x[u][i];
+          }
+      } else {
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int j = base + 16 * u + 4 * quad + i, d = p - j;
+            // (bitwise: a chain of && would become branches)
+            const bool seen = (d >= 0) & ((d < g.window) | (j < g.keep_first)) & (j < key_end);
+            x[u][i] = seen ? x[u][i] : -INFINITY;
+            mx = fmaxf(mx, x[u][i]);
+          }
+        mx = fmaxf(mx, __shfl_xor(mx, 16, SD_WAVE));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, SD_WAVE));
+        const float ref = mx == -INFINITY ? 0.f : mx;            // (no key seen yet)
+        corr = exp_neg(m_run - ref);   // (nothing summed yet: 0)
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            x[u][i] = exp_neg(x[u][i] - ref);
+            sum += x[u][i];
+          }
+      }
+      return sum;
+    };
+    float mx, corr = 1.f, sum = weigh(sc, mx, corr);
+    if constexpr (!LATENT) {   // (an infinite channel of a latent row is an infinite value too)
+      if (__any(sum != sum)) {   // of such queries only
+        f32x4 again[4];
+        float mx2, corr2 = 1.f;
+        plain_scores(s, again);
+        const float sum2 = weigh(again, mx2, corr2);
+        int redo = sum != sum;
+        redo |= __shfl_xor(redo, 16, SD_WAVE);
+        redo |= __shfl_xor(redo, 32, SD_WAVE);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) sc[u][i] = redo ? again[u][i] : sc[u][i];
+        mx = redo ? mx2 : mx;
+        corr = redo ? corr2 : corr;
+        sum = redo ? sum2 : sum;
+      }
+    }
+    if constexpr (!POOLED) {
+      m_run = mx;
       l_run = fmaf(l_run, corr, sum);
       if (__any(corr != 1.f)) {
 #pragma unroll
@@ -318,7 +365,7 @@ __global__ __launch_bounds__(256, KS > 4 ? 1 : 2) void rows_attn_kernel(RowsAttn
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       const f32x4 x[2] = {sc[2 * u], sc[2 * u + 1]};
-      parts(x, pw[u]);
+      parts(x, pw[u], std::false_type{});
     }
     // (two tiles of 16 channels side by side)
 #pragma unroll

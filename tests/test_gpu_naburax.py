@@ -774,3 +774,40 @@ def test_rows_softmax_attention_of_scores_that_are_no_numbers(H, G, dk, dv, wind
     got = ops.rows_softmax_attention(q, kc, vc, bt, i32([[0, 0, n, p0]]), H, G, dk, dv, window, keep, 0.0625)
     assert not torch.isfinite(want).all()
     same_where_finite(got, want)
+
+
+@pytest.mark.parametrize("H,G,dk,dv", [(4, 2, 128, 128), (16, 1, 128, 128), (3, 1, 576, 512)])
+@pytest.mark.parametrize("window,keep", [(5000, 0), (40, 0), (70, 33), (1, 1)])
+def test_rows_softmax_attention_of_values_that_are_no_numbers(H, G, dk, dv, window, keep):
+    """Infinite and NaN keys and values before, inside and at the end of a portion: they reach the rows that see their
+    token, in the channels that they are in, and no other row or channel: as on the vector pipe, which reads the keys that a
+    row sees and no others."""
+    from vllm_omni_draft_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(dk + window + H)
+    p0, n = 37, 150
+    pages = (p0 + n + 15) // 16
+    bt = torch.randperm(pages, generator=g, device="cuda").to(torch.int32).view(1, pages)
+    kc = torch.randn(pages, G, 16, dk, generator=g, device="cuda").to(torch.bfloat16)
+    vc = None if dv == 512 else torch.randn(pages, G, 16, dv, generator=g, device="cuda").to(torch.bfloat16)
+    q = torch.randn(n, H * dk, generator=g, device="cuda")
+    pos, slot, ents = i32(range(p0, p0 + n)), i32([0] * n), i32([[0, 0, n, p0]])
+    run = lambda: (ops.window_softmax_attention(q, kc, vc, pos, slot, bt, H, G, dk, dv, window, keep, dk ** -0.5),
+                   ops.rows_softmax_attention(q, kc, vc, bt, ents, H, G, dk, dv, window, keep, dk ** -0.5))
+    clean = run()[1]
+    inf, nan = float("inf"), float("nan")
+    for p, c, x in ((p0 + 99, 7, inf), (p0 + 100, 120, -inf), (p0 + 130, slice(None), nan), (p0 + n - 1, 0, nan), (36, 5, nan), (2, 9, inf)):
+        if p < p0 and window > p0:
+            continue              # (every row would see it)
+        if vc is not None:
+            vc[bt[0, p // 16].long(), 0, p % 16, c] = x
+        else:
+            kc[bt[0, p // 16].long(), 0, p % 16, slice(None)] = nan
+        want, got = run()
+        if window > 1 or p >= p0 or p < keep:
+            assert not torch.isfinite(want).all()
+        same_where_finite(got, want)
+        touched = ~torch.isfinite(want)
+        assert torch.equal(got[~touched], clean[~touched])       # (and the rest has its bits)
+    kc[bt[0, (p0 + 60) // 16].long(), 0, (p0 + 60) % 16] = nan
+    want, got = run()
+    same_where_finite(got, want)

@@ -691,3 +691,31 @@ def test_rows_pool_attention_of_scores_that_are_no_numbers(H, G, window, pool):
     bad = ~torch.isfinite(want)
     assert bad.any() and not bad.all() and torch.equal(~torch.isfinite(got), bad)
     assert (got - want)[~bad].abs().max() <= 1e-5 * want[~bad].abs().max()
+
+
+@pytest.mark.parametrize("H,G,window,pool", [(4, 2, 60, 16), (16, 1, 33, 5), (2, 2, 1, 1), (3, 1, 17, 32)])
+def test_rows_pool_attention_of_values_that_are_no_numbers(H, G, window, pool):
+    """Infinite and NaN values before and inside a portion, and so in the means of blocks: they reach the rows that see
+    the token or a block with it, in their channels, and nothing else, as on the vector pipe."""
+    from vllm_omni_draft_amd import ops
+    g = torch.Generator().manual_seed(H + window)
+    p0, n, d = 37, 190, 128
+    k, v = (torch.randn(p0 + n, G * d, generator=g).to(torch.bfloat16).float() for _ in range(2))
+    q, bias = torch.randn(n, H * d, generator=g), torch.randn(H, generator=g)
+
+    def run():
+        bed = _AttnBed(G, d, d, pool, p0 + n, torch.bfloat16)
+        bed.append(k[:p0], v[:p0], list(range(p0)))
+        bed.attend(torch.zeros(p0, H * d), list(range(p0)), H, window, 1.0, None)   # (fills the pooled blocks)
+        bed.append(k[p0:], v[p0:], list(range(p0, p0 + n)))
+        got = ops.rows_pool_attention(dev(q), bed.k, bed.v, bed.pk, bed.pv, bed.tables, i32([[0, 0, n, p0]]), H, G, d, d, window,
+                                      pool, d ** -0.5, dev(bias))
+        return bed.attend(q, list(range(p0, p0 + n)), H, window, d ** -0.5, bias), got
+    clean = run()[1]
+    for p, c, x in ((p0 + 160, 7, float("inf")), (p0 + 161, slice(0, d), float("nan")), (p0 + n - 1, 3, float("nan")),
+                    (p0 + 70, 5, float("-inf")), (p0 - 1, 20, float("nan"))):
+        v[p, c] = x
+        want, got = run()
+        bad = ~torch.isfinite(want)
+        assert bad.any() and not bad.all() and torch.equal(~torch.isfinite(got), bad)
+        assert (got - want)[~bad].abs().max() <= 1e-5 * want[~bad].abs().max() and torch.equal(got[~bad], clean[~bad])

@@ -16,7 +16,8 @@
 // sums fill the registers): 1024 rows of 16 latent heads (576 / 512 channels) 972 -> 133 us, 1024 rows of 16 heads over 4
 // of 128 channels 344 -> 42 us.
 // 2048 rows of 16 heads over 4 with a window of 1024 and pooled blocks 789 -> 73 us.
-// A non-finite value at a position of the portion itself can reach rows of up to 63 positions before it.
+// A weight of 0 does not clear a value that is no number: in the stages that not all rows of a workgroup see whole, such
+// values become 0 as they arrive, and the rows that see them get them added (add_odd).
 #include <math.h>
 #include <type_traits>
 
@@ -91,6 +92,7 @@ __global__ __launch_bounds__(256, KS > 4 ? 1 : 2) void rows_attn_kernel(RowsAttn
   constexpr int kStage = 4 * (kKeyPage + kValPage);
   __shared__ __attribute__((aligned(1024))) char s0[kStage];
   __shared__ __attribute__((aligned(1024))) char s1[kStage];
+  __shared__ unsigned odd[2][4];   // of a stage and a wave's part of it: the rows that held values that are no numbers
   const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, quad = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kvh = blockIdx.y, qh = g.H / g.G, per = kRowsPerBlock / qh;
@@ -386,21 +388,88 @@ __global__ __launch_bounds__(256, KS > 4 ? 1 : 2) void rows_attn_kernel(RowsAttn
           for (int w = 0; w < 2; ++w) o[v + w] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[w], pw[u][c], o[v + w], 0, 0, 0);
       }
   };
+  // whether some row of the workgroup does not see all of stage st
+  auto mixed = [&](int st) {
+    if (st < kept_stages) return POOLED && (st + 1) * kPooled > blocks_of(pos0);
+    return stage_base(st) + kKeys - 1 > pos0 || stage_base(st) <= last - g.window;
+  };
+  // This wave's rows of a stage's values, once they are in LDS: what is no number becomes 0.  Returns the rows.
+  auto clear_odd = [&](char* rows, auto element, int row_bytes, int bytes) __attribute__((always_inline)) {
+    constexpr bool kWide = sizeof(element) == 4;
+    unsigned found = 0;
+    for (int at = lane * 16; at < bytes; at += 64 * 16) {
+      const u32x4 d = *reinterpret_cast<const u32x4*>(rows + at);
+      unsigned bad[4], any = 0;   // the top bit of each element whose exponent is all ones
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        bad[i] = kWide ? ((d[i] & 0x7f800000u) + 0x00800000u) & 0x80000000u : ((d[i] & 0x7f807f80u) + 0x00800080u) & 0x80008000u;
+        any |= bad[i];
+      }
+      if (any) {
+        u32x4 z = d;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if (bad[i] & 0x80000000u) z[i] &= kWide ? 0u : 0x0000ffffu;
+          if (bad[i] & 0x00008000u) z[i] &= 0xffff0000u;
+        }
+        *reinterpret_cast<u32x4*>(rows + at) = z;
+        found |= 1u << at / row_bytes;
+      }
+    }
+    if (__any(found != 0)) {
+#pragma unroll
+      for (int x = 1; x < 64; x <<= 1) found |= __shfl_xor(found, x, SD_WAVE);
+    }
+    return found;
+  };
+  // ... and reaches the queries that see its row: of latent rows, whose scores are no numbers then, as a whole.
+  auto add_odd = [&](int st, bool means) __attribute__((always_inline)) {
+#pragma unroll 1
+    for (int w = 0; w < 4; ++w)
+#pragma unroll 1
+      for (unsigned rows = odd[st & 1][w]; rows; rows &= rows - 1) {
+        const int j = means ? st * kPooled + 8 * w + __builtin_ctz(rows) : stage_base(st) + kPage * w + __builtin_ctz(rows);
+        const int d = p - j;
+        const bool seen = means ? j < my_blocks : (d >= 0) & ((d < g.window) | (j < g.keep_first));
+        if constexpr (LATENT) {
+          l_run = seen ? NAN : l_run;
+        } else {
+          const int jj = means ? min(j, n_kept - 1) : j, lp = means ? (jj * g.pool + g.pool - 1) / kPage : jj / kPage;
+          const size_t head = (size_t)tbl[lp] * g.G + kvh;
+          const float* pv = g.pv + (head * g.pslots + jj - lp * kPage / g.pool) * DV + 4 * quad;
+          const bf16_t* vc = g.vc + (head * kPage + (jj & (kPage - 1))) * DV + 4 * quad;
+#pragma unroll
+          for (int v = 0; v < VT; ++v)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const float x = means ? pv[16 * v + i] : (float)vc[16 * v + i];
+              if (seen & !(fabsf(x) < INFINITY)) o[v][i] += x;
+            }
+        }
+      }
+  };
   // stage st is in `cur` once this wave's loads have landed and every wave is here; then nobody reads `nxt` any more
   auto step = [&](char* cur, char* nxt, int st) __attribute__((always_inline)) {
-    // Rows behind the stage's last key hold what a page's earlier owner left, or nothing: a weight of 0 does not clear a
-    // NaN, so they are cleared here, by the wave that brought them.
-    const bool means = POOLED && st < kept_stages;
+    // Rows behind the stage's last key hold what a page's earlier owner left, or nothing: they are cleared here, by the
+    // wave that brought them.
+    const bool means = POOLED && st < kept_stages, some = mixed(st);
     const int left = means ? kPage : stage_last(st) + 1 - stage_base(st) - wave * kPage;
-    if (left < kPage) {
+    if (left < kPage || some) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       char* rows = cur + (LATENT ? wave * kKeyPage : 4 * kKeyPage + wave * kValPage);
-      for (int at = max(left, 0) * kVRow + lane * 16; at < kPage * kVRow; at += 64 * 16) *reinterpret_cast<u32x4*>(rows + at) = u32x4{0, 0, 0, 0};
+      if (left < kPage)
+        for (int at = max(left, 0) * kVRow + lane * 16; at < kPage * kVRow; at += 64 * 16) *reinterpret_cast<u32x4*>(rows + at) = u32x4{0, 0, 0, 0};
+      if (some) {
+        const unsigned found = means ? clear_odd(cur + kPooled * 512 + wave * 4096, float(), 512, 4096)
+                                     : clear_odd(rows, bf16_t(), kVRow, kPage * kVRow);
+        if (lane == 0) odd[st & 1][wave] = found;
+      }
     }
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if (st + 1 < stages) load(nxt, st + 1);
     if (means) attend_pooled(cur, st);
     else attend(cur, st);
+    if (some && (odd[st & 1][0] | odd[st & 1][1] | odd[st & 1][2] | odd[st & 1][3])) add_odd(st, means);
   };
   load(s0, 0);
   int st = 0;

@@ -505,7 +505,8 @@ __global__ __launch_bounds__(1024) void decay_step_kernel(StepArgs a, QkvArgs g,
 // the decays behind s, and S the state at the block's start:
 //   o_t = (q_t P_t) S + sum_{s <= t} (sum_c q_t[c] k_s[c] d_{s+1}[c] .. d_t[c]) v_s
 //   S  <- diag(P_last) S + (k_s R_s)^T v_s
-// Every factor is a product of decays, at most one: nothing is divided, however strong the decay.  The
+// Every factor is a product of decays, at most one: nothing is divided, however strong the decay; products carry what
+// their roundings left (see Product), so that the results are as near to 64 bits as those of the scan token by token.  The
 // inner sums of a block are formed channel by channel with running products.  A wave owns 16 value
 // columns; its part of S lives in accumulators, whose layout is that of the right operand of q S as it is
 // (the key channels of an MFMA step in the order the accumulators hold them).
@@ -529,7 +530,7 @@ struct ChunkArgs {
   const int32_t* entries;
   float* out;              // [rows, H*dv]
   float* cs;               // [chunks, H, dk, dv]: own sums, then the state at the chunk's start
-  float* ct;               // [chunks, H, dk]: product of the chunk's decays
+  float* ct;               // [chunks, H, 2, dk]: product of the chunk's decays, and what its rounding left
   int n_entries, H, dk, dv, chunk;
 };
 constexpr int kBlock = 16;       // tokens of a block
@@ -591,9 +592,27 @@ struct BlockRows {
   }
 };
 
+// A product and what its roundings left (hi + lo is the product to about 46 bits): a state of a slow decay is multiplied
+// by products of the same decays over and over, and the error of one rounded product would add up with every block.
+struct Product {
+  float hi = 1.f, lo = 0.f;
+  __device__ __forceinline__ void times(float d) {
+    const float h = hi * d;
+    lo = fmaf(lo, d, fmaf(hi, d, -h));
+    hi = h;
+  }
+  __device__ __forceinline__ void times(const Product& p) {
+    const float h = hi * p.hi;
+    lo = fmaf(lo, p.hi, fmaf(hi, p.lo, fmaf(hi, p.hi, -h)));
+    hi = h;
+  }
+  // x times it, plus y
+  __device__ __forceinline__ float of(float x, float y = 0.f) const { return fmaf(x, hi, fmaf(x, lo, y)); }
+};
+
 template <int DKP>
 constexpr size_t decay_chunk_lds() {
-  return sizeof(float) * (4 * (size_t)kBlock * (DKP + 4) + (size_t)DKP * kTokLd + DKP +
+  return sizeof(float) * (4 * (size_t)kBlock * (DKP + 4) + (size_t)DKP * kTokLd + 2 * DKP +
                           (size_t)kBlock * (kBlockCols + 4) + (size_t)kBlock * kTokLd);
 }
 template <int DKP, int V, int MODE, bool SCALAR>   // keys of up to DKP channels; SCALAR: one decay for a head's channels
@@ -605,8 +624,8 @@ __global__ __launch_bounds__(kChunkThreads, DKP <= 128 ? 4 : 2) void decay_chunk
   float* ds = ks + kBlock * LDK;       // [16][LDK] decays
   float* qp = ds + kBlock * LDK;       // [16][LDK] q_t P_t
   float* kr = qp + kBlock * LDK;       // [DKP][kTokLd] k_s R_s, transposed
-  float* tot = kr + DKP * kTokLd;      // [DKP] P_last
-  float* vs = tot + DKP;               // [16][LDV]
+  float* tot = kr + DKP * kTokLd;      // [2][DKP] P_last
+  float* vs = tot + 2 * DKP;           // [16][LDV]
   float* as = vs + kBlock * LDV;       // [16][kTokLd] the block's inner sums
   const int tid = threadIdx.x, lane = tid & 63, col = lane & 15, quad = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -658,7 +677,7 @@ __global__ __launch_bounds__(kChunkThreads, DKP <= 128 ? 4 : 2) void decay_chunk
         S[kt][i] = k < dk && c < cols ? s : 0.f;
       }
   }
-  float run = 1.f;                     // kSums: product of the chunk's decays, thread < DKP a channel
+  Product run;                         // kSums: product of the chunk's decays, thread < DKP a channel
   for (int t0 = 0; t0 < nt; t0 += kBlock) {
     const int n = nt - t0 < kBlock ? nt - t0 : kBlock;
     __syncthreads();
@@ -670,7 +689,8 @@ __global__ __launch_bounds__(kChunkThreads, DKP <= 128 ? 4 : 2) void decay_chunk
     if (t0 + kBlock < nt) fetch(t0 + kBlock);
     // products of decays, a thread per channel: forward, and (other threads) backward
     if (tid < DKP) {
-      float d[kBlock], p = 1.f;
+      float d[kBlock];
+      Product p;
 #pragma unroll
       for (int t = 0; t < kBlock; ++t) d[t] = ds[t * LDK + tid];
       if constexpr (MODE != kSums) {
@@ -679,18 +699,20 @@ __global__ __launch_bounds__(kChunkThreads, DKP <= 128 ? 4 : 2) void decay_chunk
         for (int t = 0; t < kBlock; ++t) q[t] = qs[t * LDK + tid];
 #pragma unroll
         for (int t = 0; t < kBlock; ++t) {
-          p *= d[t];
-          qp[t * LDK + tid] = q[t] * p;
+          p.times(d[t]);
+          qp[t * LDK + tid] = p.of(q[t]);
         }
       } else {
 #pragma unroll
-        for (int t = 0; t < kBlock; ++t) p *= d[t];
+        for (int t = 0; t < kBlock; ++t) p.times(d[t]);
       }
-      tot[tid] = p;
-      run *= p;
+      tot[tid] = p.hi;
+      tot[DKP + tid] = p.lo;
+      if constexpr (MODE == kSums) run.times(p);
     } else if (tid < 2 * DKP) {
       const int ch = tid - DKP;
-      float d[kBlock], w[kBlock], p = 1.f;
+      float d[kBlock], w[kBlock];
+      Product p;
 #pragma unroll
       for (int t = 0; t < kBlock; ++t) {
         d[t] = ds[t * LDK + ch];
@@ -698,8 +720,8 @@ __global__ __launch_bounds__(kChunkThreads, DKP <= 128 ? 4 : 2) void decay_chunk
       }
 #pragma unroll
       for (int t = kBlock - 1; t >= 0; --t) {
-        w[t] *= p;
-        p *= d[t];
+        w[t] = p.of(w[t]);
+        p.times(d[t]);
       }
 #pragma unroll
       for (int t = 0; t < kBlock; t += 4)
@@ -752,23 +774,19 @@ __global__ __launch_bounds__(kChunkThreads, DKP <= 128 ? 4 : 2) void decay_chunk
 #pragma unroll
     for (int i = 0; i < 4; ++i) vv[i] = vs[(4 * quad + i) * LDV + c];
     if constexpr (MODE != kSums) {
-      f32x4 o = {0.f, 0.f, 0.f, 0.f}, o2 = {0.f, 0.f, 0.f, 0.f};
+      f32x4 part[4];   // (four short chains of sums)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) part[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int kt = 0; kt < KT; ++kt) {
         const f32x4 a = *reinterpret_cast<const f32x4*>(qp + col * LDK + 16 * kt + 4 * quad);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          f32x4& acc = i & 1 ? o2 : o;
-          acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], S[kt][i], acc, 0, 0, 0);
-        }
+        for (int i = 0; i < 4; ++i) part[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], S[kt][i], part[i], 0, 0, 0);
       }
       const f32x4 a = *reinterpret_cast<const f32x4*>(as + col * kTokLd + 4 * quad);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        f32x4& acc = i & 1 ? o2 : o;
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], vv[i], acc, 0, 0, 0);
-      }
-      o += o2;
+      for (int i = 0; i < 4; ++i) part[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], vv[i], part[i], 0, 0, 0);
+      f32x4 o = (part[0] + part[1]) + (part[2] + part[3]);
       if constexpr (SCALAR) o += skip * vv;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -777,13 +795,21 @@ __global__ __launch_bounds__(kChunkThreads, DKP <= 128 ? 4 : 2) void decay_chunk
       }
     }
     if (MODE != kReads || t0 + kBlock < nt) {
-#pragma unroll
-      for (int kt = 0; kt < KT; ++kt) S[kt] *= *reinterpret_cast<const f32x4*>(tot + 16 * kt + 4 * quad);
+      // (the block's own sum first: one rounding of the state a block)
 #pragma unroll
       for (int kt = 0; kt < KT; ++kt) {
         const f32x4 a = *reinterpret_cast<const f32x4*>(kr + (16 * kt + col) * kTokLd + 4 * quad);
+        const f32x4 hi = *reinterpret_cast<const f32x4*>(tot + 16 * kt + 4 * quad);
+        const f32x4 lo = *reinterpret_cast<const f32x4*>(tot + DKP + 16 * kt + 4 * quad);
+        f32x4 own = {0.f, 0.f, 0.f, 0.f}, own2 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) S[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], vv[i], S[kt], 0, 0, 0);
+        for (int i = 0; i < 2; ++i) {
+          own = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], vv[i], own, 0, 0, 0);
+          own2 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i + 2], vv[i + 2], own2, 0, 0, 0);
+        }
+        own += own2;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) S[kt][i] = Product{hi[i], lo[i]}.of(S[kt][i], own[i]);
       }
     }
   }
@@ -796,7 +822,10 @@ __global__ __launch_bounds__(kChunkThreads, DKP <= 128 ? 4 : 2) void decay_chunk
         const int k = 16 * kt + 4 * quad + i;
         if (k < dk && c < cols) dst[(size_t)k * dv + c] = S[kt][i];
       }
-    if (MODE == kSums && blockIdx.z == 0 && tid < dk) g.ct[at + tid] = run;
+    if (MODE == kSums && blockIdx.z == 0 && tid < dk) {
+      g.ct[2 * at + tid] = run.hi;
+      g.ct[2 * at + dk + tid] = run.lo;
+    }
   }
 }
 
@@ -810,23 +839,24 @@ __global__ __launch_bounds__(256) void chunk_carry_kernel(ChunkArgs g) {
   const int nc = (len + g.chunk - 1) / g.chunk;
   float* st = g.state + ((size_t)slot * H + h) * dk * dv + x;
   float* own = g.cs + ((size_t)first * H + h) * dk * dv + x;
-  const float* ct = g.ct + ((size_t)first * H + h) * dk + x / dv;
-  const size_t step = (size_t)H * dk * dv, step_t = (size_t)H * dk;
+  const float* ct = g.ct + ((size_t)first * H + h) * 2 * dk + x / dv;
+  const size_t step = (size_t)H * dk * dv, step_t = (size_t)H * 2 * dk;
   float val = g.entries[4 * e + 3] > 0 ? *st : 0.f;
   constexpr int U = 8;
   for (int i = 0; i < nc; i += U) {
-    float v[U], d[U];
+    float v[U];
+    Product d[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int c = i + u < nc ? i + u : nc - 1;
       v[u] = own[c * step];
-      d[u] = ct[c * step_t];
+      d[u] = Product{ct[c * step_t], ct[c * step_t + dk]};
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (i + u >= nc) break;
       own[(i + u) * step] = val;
-      val = fmaf(d[u], val, v[u]);
+      val = d[u].of(val, v[u]);
     }
   }
   *st = val;
@@ -993,7 +1023,7 @@ extern "C" int sd_low_rank_decay(const float* a1, int64_t ld, const void* a2, co
 extern "C" size_t sd_decay_chunks_scratch_bytes(int n_rows, int n_entries, int H, int dk, int dv) {
   // (rows that fill no more than a chunk beyond one per portion run in one go)
   if (n_rows < 1 || n_entries < 1 || n_rows - n_entries < kChunkMin || H < 1 || dk < 1 || dv < 1) return 0;
-  return sizeof(float) * ((size_t)n_rows / kChunkMin + n_entries) * H * ((size_t)dk * dv + dk);
+  return sizeof(float) * ((size_t)n_rows / kChunkMin + n_entries) * H * ((size_t)dk * dv + 2 * dk);
 }
 
 namespace {

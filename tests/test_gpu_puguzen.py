@@ -753,3 +753,35 @@ def test_chunked_recurrences_are_as_near_to_64_bits_as_the_scan(kind, H, Gq, dk,
     off = lambda a, b: ((a.double() - b).norm() / b.norm()).item()
     assert off(got, want) <= 1.1 * off(scan, want) and off(S2[0], S) <= 1.1 * off(S1[0], S), \
         (off(got, want), off(scan, want), off(S2[0], S), off(S1[0], S))
+
+
+@pytest.mark.parametrize("kind,H,Gq,dk,dv", [("head", 2, 2, 128, 128), ("row", 6, 2, 33, 70), ("channel", 2, 2, 64, 130)])
+@pytest.mark.parametrize("n", [200, 40])
+def test_chunked_recurrences_of_values_that_are_no_numbers(kind, H, Gq, dk, dv, n):
+    """Infinite and NaN values, keys and queries inside blocks of 16 tokens and chunks (and of a portion in one go, 40):
+    what the scan token by token leaves finite is finite and the same."""
+    from vllm_omni_draft_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(H + n + dk)
+    rn = lambda *shape: torch.randn(*shape, generator=g, device=DEV)
+    q, k, v = rn(n, Gq * dk) * dk ** -0.5, rn(n, Gq * dk), rn(n, H * dv)
+    decay = {"head": lambda: torch.tensor([0.9, 0.5], device=DEV), "row": lambda: torch.sigmoid(rn(n, H) + 1),
+             "channel": lambda: torch.sigmoid(rn(n, H * dk) + 1)}[kind]()
+    scale, skip = (torch.rand(n, H, generator=g, device=DEV), rn(H)) if kind == "row" else (None, None)
+    ents, S0 = i32([[0, 0, n, 5]]), rn(1, H, dk, dv)
+
+    def run():
+        S1, S2 = S0.clone(), S0.clone()
+        if kind == "row":
+            a = ops.decay_scan_rows(q, k, v, decay, scale, skip, S1, ents, H, Gq, dk, dv)
+        else:
+            a = ops.decay_scan(q, k, v, decay, S1, ents, H, dk, dv)
+        b = ops.decay_chunks(q, k, v, decay, S2, ents) if kind == "channel" else ops.head_decay_chunks(q, k, v, decay, S2, ents, scale, skip)
+        for want, got in ((a, b), (S1, S2)):
+            ok = torch.isfinite(want)
+            assert torch.equal(torch.isfinite(got), ok)
+            assert (got - want)[ok].abs().max() <= 2e-5 * want[ok].abs().max()
+        return a
+    inf, nan = float("inf"), float("nan")
+    for x, t, c, y in ((v, n - 3, 4, inf), (v, n - 20, 70 if H * dv > 140 else 1, nan), (q, 7, 3, nan), (v, 21, dv + 2, -inf), (k, n - 30, 5, nan)):
+        x[t, c] = y
+        assert not torch.isfinite(run()).all()

@@ -766,7 +766,8 @@ __global__ __launch_bounds__(kChunkThreads, DKP <= 128 ? 4 : 2) void decay_chunk
       }
       a[0] += __shfl_xor(a[0], 32, SD_WAVE);
       const int idx = (int)(__brev((unsigned)lane) >> 27);       // the value that this lane is left with
-      if (lane < 32) as[(idx & 15) * kTokLd + wave + 8 * (idx >> 4)] = a[0];
+      const int t = idx & 15, from = wave + 8 * (idx >> 4);
+      if (lane < 32) as[t * kTokLd + from] = t >= from ? a[0] : 0.f;   // (a key that is no number is not 0 times 0)
     }
     __syncthreads();
     if (!works) continue;
@@ -774,6 +775,14 @@ __global__ __launch_bounds__(kChunkThreads, DKP <= 128 ? 4 : 2) void decay_chunk
 #pragma unroll
     for (int i = 0; i < 4; ++i) vv[i] = vs[(4 * quad + i) * LDV + c];
     if constexpr (MODE != kSums) {
+      // A value that is no number stays out of the product with the inner sums, whose zeros would hand it to the tokens
+      // before its own; the tokens behind it get it below.
+      auto odd = [](float x) { return !(fabsf(x) < INFINITY); };
+      const bool some = __any(odd(vv[0]) | odd(vv[1]) | odd(vv[2]) | odd(vv[3]));
+      if (some) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) vv[i] = odd(vv[i]) ? 0.f : vv[i];
+      }
       f32x4 part[4];   // (four short chains of sums)
 #pragma unroll
       for (int i = 0; i < 4; ++i) part[i] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -787,7 +796,18 @@ __global__ __launch_bounds__(kChunkThreads, DKP <= 128 ? 4 : 2) void decay_chunk
 #pragma unroll
       for (int i = 0; i < 4; ++i) part[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], vv[i], part[i], 0, 0, 0);
       f32x4 o = (part[0] + part[1]) + (part[2] + part[3]);
-      if constexpr (SCALAR) o += skip * vv;
+      if (some) {
+#pragma unroll 1
+        for (int from = 0; from < kBlock; ++from) {
+          const float x = vs[from * LDV + c];
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (odd(x) & (4 * quad + i >= from)) o[i] = fmaf(as[(4 * quad + i) * kTokLd + from], x, o[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) vv[i] = vs[(4 * quad + i) * LDV + c];
+      }
+      if (SCALAR && g.skip) o += skip * vv;
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int t = 4 * quad + i;

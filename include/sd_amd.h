@@ -1622,8 +1622,9 @@ int sd_low_rank_decay(const float* a1, int64_t ld, const void* a2, const float* 
                       float* out, int n_rows, int n_cols, sd_stream_t stream);
 /* The recurrence of sd_decay_scan with decays per key channel ([rows, H*dk]) and q multiplied by q_scale, in
  * blocks of 16 tokens on the f32 matrix instruction.  With scratch of sd_decay_chunks_scratch_bytes bytes (0: few
- * rows) long portions run in chunks side by side: the chunks' own sums, a pass over the chunks, then the tokens'
- * results; otherwise a portion runs in one go.                                              */
+ * rows) portions of more than 64 rows run in chunks side by side: the chunks' own sums, a pass over the chunks, then the
+ * tokens' results; other portions, and all without scratch, run in one go.  How a portion runs, its chunks included,
+ * depends on its own rows alone. */
 size_t sd_decay_chunks_scratch_bytes(int n_rows, int n_entries, int H, int dk, int dv);
 int sd_decay_chunks(const float* q, const float* k, const float* v, int64_t ld, const float* decay, float q_scale,
                     float* state, const int32_t* entries, int n_entries, int n_rows, float* out, int H, int dk, int dv,
@@ -1851,6 +1852,8 @@ typedef struct {
   float* layer_out;        /* NULL, or [n_layers, n_rows, width]: the residual after each layer */
   const int32_t* prev_tokens; /* [n_rows] the token before each row in its sequence, -1: none
                                  (models with a bigram table; NULL otherwise) */
+  int shortest, longest;   /* rows of the shortest and the longest portion, 0: not known.  Spares launches; portions
+                              outside of them may be left out. */
 } sd_seq_batch;
 
 typedef struct sd_seq_model sd_seq_model;

@@ -811,3 +811,15 @@ def test_rows_softmax_attention_of_values_that_are_no_numbers(H, G, dk, dv, wind
     kc[bt[0, (p0 + 60) // 16].long(), 0, (p0 + 60) % 16] = nan
     want, got = run()
     same_where_finite(got, want)
+
+
+def test_a_portions_bits_do_not_depend_on_what_shares_its_pass():
+    """The state-space recurrence on either side of the line between the scan and chunks (64 rows): the same bits alone
+    and beside a long prompt and seventy decoded tokens."""
+    from tests.test_gpu_puguzen import beside_others
+    cfg = model_cfg([parallel(s_heads=16, s_vdim=32, state=64, window=20) for _ in range(3)], width=128)
+    st, toks, alone, beside = beside_others(build, cfg, [400, 64, 20, 65])
+    for t, a, b in zip(toks, alone, beside):
+        assert torch.equal(a, b), len(t)
+        want = oracle_logits(cfg, st, t)
+        assert sorted(rel(b[r], want[r]) for r in range(len(t)))[len(t) // 2] < 2e-2   # (see test_bfloat16_serving_stays_close)

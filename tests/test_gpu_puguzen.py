@@ -785,3 +785,33 @@ def test_chunked_recurrences_of_values_that_are_no_numbers(kind, H, Gq, dk, dv, 
     for x, t, c, y in ((v, n - 3, 4, inf), (v, n - 20, 70 if H * dv > 140 else 1, nan), (q, 7, 3, nan), (v, 21, dv + 2, -inf), (k, n - 30, 5, nan)):
         x[t, c] = y
         assert not torch.isfinite(run()).all()
+
+
+def beside_others(build, cfg, lens, layers=None, **kw):
+    """Logits of every token of prompts of these lengths, each alone in a pass (of more than 16 rows), and all in one pass
+    with a longer prompt and seventy decoded tokens of other requests between them."""
+    st, eng = build(cfg, torch.bfloat16, seed=3, max_seqs=80, max_tokens=8192, **kw)
+    toks = [prompt(cfg, n, i) for i, n in enumerate(lens)]
+    alone = []
+    for i, t in enumerate(toks):
+        alone.append(eng.step([("a", t, list(range(len(t))))]).cpu())
+        eng.finish("a")
+    eng.step([(f"s{i}", prompt(cfg, 3, 50 + i), []) for i in range(70)])
+    singles = [(f"s{i}", prompt(cfg, 1, 90 + i), []) for i in range(70)]
+    ents = singles[:30] + [("long", prompt(cfg, 333, 7), [])]
+    for i, t in enumerate(toks):
+        ents += [(f"p{i}", t, list(range(len(t))))] + singles[30 + 10 * i:40 + 10 * i]
+    ents += singles[30 + 10 * len(toks):]
+    got = eng.step(ents).cpu()
+    return st, toks, alone, torch.split(got, lens)
+
+
+def test_a_portions_bits_do_not_depend_on_what_shares_its_pass():
+    """Portions on either side of the line between the scan and chunks (64 rows), in a pass of more portions than scratch
+    was once planned for: the same bits as alone."""
+    cfg = model_cfg([layer("retention", heads=3, dim=24, vdim=40), layer("gla", heads=2, dim=32, vdim=16), layer("attention", window=20)],
+                    width=128)
+    st, toks, alone, beside = beside_others(build, cfg, [100, 64, 20, 65])
+    for t, a, b in zip(toks, alone, beside):
+        assert torch.equal(a, b), len(t)
+        assert rel(b, oracle_logits(cfg, st, t)) < 0.03

@@ -151,7 +151,7 @@ class SeqModelDesc(C.Structure):
 class SeqBatch(C.Structure):
     _fields_ = [("n_rows", i32), ("n_entries", i32), ("tokens", vp), ("row_pos", vp), ("row_slot", vp),
                 ("entries", vp), ("block_tables", vp), ("max_blocks", i32), ("page", i32), ("n_out", i32),
-                ("out_rows", vp), ("logits", vp), ("layer_out", vp), ("prev_tokens", vp)]
+                ("out_rows", vp), ("logits", vp), ("layer_out", vp), ("prev_tokens", vp), ("shortest", i32), ("longest", i32)]
 
 
 # name -> (restype, argtypes); every symbol include/sd_amd.h declares.

@@ -1,6 +1,7 @@
 // Shared device helpers for the gfx950 speculative-decoding kernels.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <limits.h>
 #include <stdint.h>
 #include <stdio.h>
 #include "../../include/sd_amd.h"
@@ -33,6 +34,48 @@ sd_pf_range sd_linear_pf_range(const void* W, int N, int K, int epi, int fp8, in
                                size_t max_bytes);
 // Applies to the next attention launch of this host thread (then forgotten); n <= 2.
 void sd_attn_prefetch_next(const sd_pf_range* r, int n);
+
+// Layer-list models whose matrices are tiled: a portion of a pass with more rows than this runs on kernels for many
+// rows, which sum in another order than those for few.  A portion's own rows decide, so that what shares its pass does
+// not change its bits (linear layers, which have one rule for passes of up to 16 rows and one for others, aside).
+constexpr int kLongPortion = 64;
+// Whether row r belongs to a long portion (all lanes of a wave ask for the same row).
+__device__ __forceinline__ bool sd_in_long_portion(const int32_t* entries, int n_entries, int r) {
+  bool yes = false;
+  for (int e = threadIdx.x & 63; e < n_entries; e += 64) {
+    const int first = entries[4 * e + 1], rows = entries[4 * e + 2];
+    yes |= (rows > kLongPortion) & (r >= first) & (r < first + rows);
+  }
+  return __any(yes);
+}
+
+// sd_decay_scan and sd_decay_scan_rows for the portions of at most max_rows rows.
+int sd_decay_scan_(const float* q, const float* k, const float* v, int64_t ld, const float* decay, int per_channel,
+                   float* state, const int32_t* entries, int n_entries, int max_rows, float* out, int H, int dk, int dv,
+                   sd_stream_t stream);
+int sd_decay_scan_rows_(const float* q, const float* k, int64_t ldqk, const float* v, int64_t ldv, const float* decay,
+                        const float* k_scale, const void* skip, int w_f32, float* state, const int32_t* entries,
+                        int n_entries, int max_rows, float* out, int H, int Gq, int dk, int dv, sd_stream_t stream);
+// sd_decay_chunks / sd_head_decay_chunks with the long portions (chunks), the others (whole), or both.
+struct sd_chunked_decay {
+  const float *q, *k;
+  int64_t ldqk;
+  const float* v;
+  int64_t ldv;
+  const float* decay;
+  int per;              // 0: decay [H], 1: [rows, H], 2: [rows, H*dk]
+  const float* k_scale;
+  const void* skip;
+  int w_f32;
+  float q_scale;
+  float* state;
+  const int32_t* entries;
+  int n_entries, n_rows;
+  float* out;
+  int H, Gq, dk, dv;
+};
+int sd_decay_chunks_(const sd_chunked_decay* a, bool chunks, bool whole, void* scratch, size_t scratch_bytes,
+                     sd_stream_t stream);
 
 // sd_gated_softmax_attention's tiled form (sd_seqmix_joint.hip); SD_ERR_UNSUPPORTED: sizes it does
 // not take.

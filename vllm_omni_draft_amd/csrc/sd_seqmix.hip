@@ -236,7 +236,8 @@ template <bool PER_CHANNEL>
 __global__ __launch_bounds__(256) void decay_scan_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v, int64_t ld,
     const float* __restrict__ decay, float* __restrict__ state, const int32_t* __restrict__ entries,
-    float* __restrict__ out, int H, int dk, int dv, int CT, int NS, int CH) {
+    float* __restrict__ out, int H, int dk, int dv, int CT, int NS, int CH, int max_rows) {
+  if (entries[4 * blockIdx.z + 2] > max_rows) return;
   extern __shared__ float lds[];
   const int dkp = NS * kStrip;
   float* qs = lds;                  // [CH][dkp]
@@ -989,6 +990,12 @@ extern "C" int sd_sigmoid_power(const float* z, int64_t ldz, float tau, float* o
 extern "C" int sd_decay_scan(const float* q, const float* k, const float* v, int64_t ld, const float* decay,
                              int per_channel, float* state, const int32_t* entries, int n_entries,
                              float* out, int H, int dk, int dv, sd_stream_t stream) {
+  return sd_decay_scan_(q, k, v, ld, decay, per_channel, state, entries, n_entries, INT_MAX, out, H, dk, dv, stream);
+}
+
+int sd_decay_scan_(const float* q, const float* k, const float* v, int64_t ld, const float* decay, int per_channel,
+                   float* state, const int32_t* entries, int n_entries, int max_rows, float* out, int H, int dk, int dv,
+                   sd_stream_t stream) {
   SD_REQUIRE(q && k && v && decay && state && entries && out && n_entries >= 1 && H >= 1 && dv >= 1,
              SD_ERR_INVALID, "sd_decay_scan: bad argument");
   SD_REQUIRE(dk >= 1 && dk <= 256, SD_ERR_UNSUPPORTED, "sd_decay_scan: key size %d outside 1..256", dk);
@@ -1006,9 +1013,11 @@ extern "C" int sd_decay_scan(const float* q, const float* k, const float* v, int
   const size_t lds = sizeof(float) * ((size_t)(per_channel ? 3 : 2) * CH * dkp + (size_t)CH * CT + (size_t)CH * NS * CT);
   dim3 grid(tiles, H, n_entries);
   if (per_channel)
-    decay_scan_kernel<true><<<grid, CT * NS, lds, st>>>(q, k, v, ld, decay, state, entries, out, H, dk, dv, CT, NS, CH);
+    decay_scan_kernel<true><<<grid, CT * NS, lds, st>>>(q, k, v, ld, decay, state, entries, out, H, dk, dv, CT, NS, CH,
+                                                        max_rows);
   else
-    decay_scan_kernel<false><<<grid, CT * NS, lds, st>>>(q, k, v, ld, decay, state, entries, out, H, dk, dv, CT, NS, CH);
+    decay_scan_kernel<false><<<grid, CT * NS, lds, st>>>(q, k, v, ld, decay, state, entries, out, H, dk, dv, CT, NS, CH,
+                                                         max_rows);
   SD_CHECK_LAUNCH("sd_decay_scan");
   return SD_OK;
 }
@@ -1305,6 +1314,7 @@ SeqWs plan_seq(const sd_seq_model& m, int rows, int n_out, int max_ctx) {
     wide = n > wide ? n : wide;
   };
   const int plan_ents = rows < kPlanEntries ? rows : kPlanEntries;   // (enough for any number of portions up to it)
+  const int long_ents = rows > kLongPortion ? rows / (kLongPortion + 1) : 1;   // (as many portions as have chunks)
   for (const sd_seq_layer& l : m.layers) {
     if (l.block == SD_BLOCK_STREAMS) {
       const StCols c = st_cols(l);
@@ -1317,7 +1327,7 @@ SeqWs plan_seq(const sd_seq_model& m, int rows, int n_out, int max_ctx) {
       need(l.w_o_tiled, wr, W, K1);
       need(l.out_stacked ? l.w_o_tiled : l.w_o2_tiled, wr, W, K2);
       up(attn, sd_multimap_softmax_attention_scratch_bytes(rows, l.heads, 1, l.vdim, l.window, l.keep_first, 0, max_ctx));
-      up(mem, sd_decay_chunks_scratch_bytes(rows + plan_ents, plan_ents, l.s_heads, l.s_state, l.s_vdim));
+      up(mem, sd_decay_chunks_scratch_bytes(rows, long_ents, l.s_heads, l.s_state, l.s_vdim));
       if (l.ff > 0) {
         up(proj, (size_t)2 * l.ff);
         up(ff, (size_t)l.ff);
@@ -1401,7 +1411,7 @@ SeqWs plan_seq(const sd_seq_model& m, int rows, int n_out, int max_ctx) {
         up(conv, (size_t)c.conv_ch);
         up(sh, (size_t)l.s_heads);
         need(l.w_o2_tiled, wr, W, c.inner);
-        if (l.w_in_tiled) up(mem, sd_decay_chunks_scratch_bytes(rows + plan_ents, plan_ents, l.s_heads, l.s_state, l.s_vdim));
+        if (l.w_in_tiled) up(mem, sd_decay_chunks_scratch_bytes(rows, long_ents, l.s_heads, l.s_state, l.s_vdim));
       }
       if (l.n_experts > 0) {
         up(ne, (size_t)l.n_experts);
@@ -1420,7 +1430,7 @@ SeqWs plan_seq(const sd_seq_model& m, int rows, int n_out, int max_ctx) {
     need(l.w_o_tiled, wr, W, l.heads * l.vdim);
     need(l.w_down_tiled, wr, W, l.ff);
     if (l.kind != SD_MIX_WINDOW_POOL && l.w_in_tiled)
-      up(mem, sd_decay_chunks_scratch_bytes(rows + plan_ents, plan_ents, l.heads, l.dim, l.vdim));
+      up(mem, sd_decay_chunks_scratch_bytes(rows, long_ents, l.heads, l.dim, l.vdim));
     if (l.kind == SD_MIX_WINDOW_POOL) {
       const size_t n = sd_window_pool_attention_scratch_bytes(rows, l.heads, l.vdim, l.window, l.pool, max_ctx);
       attn = n > attn ? n : attn;
@@ -1623,6 +1633,17 @@ extern "C" size_t sd_seq_model_workspace_bytes(const sd_seq_model* m, int max_ro
     if (rc__ != SD_OK) return rc__; \
   } while (0)
 
+// Whether a pass has portions of at most kLongPortion rows (few), and longer ones (many).
+struct Portions {
+  bool few, many;
+};
+Portions portions(const sd_seq_batch& b) {
+  const int most = b.n_rows - b.n_entries + 1;
+  const int longest = b.longest > 0 && b.longest < most ? b.longest : most;
+  const int shortest = b.n_entries == 1 ? b.n_rows : (b.shortest > 0 ? b.shortest : 1);
+  return {shortest <= kLongPortion, longest > kLongPortion};
+}
+
 // Attention on the matrix cores for a pass with more than a few prompt rows (as for the chunked recurrences: of models
 // whose linear layers sum few and many rows in different orders anyway; a row's bits do not depend on the cut else).
 // 64 rows of one portion: 16 heads over 4 of 128 channels 14.8 -> 13.3 us from nothing, 362 -> 143 behind 4000 tokens;
@@ -1714,14 +1735,19 @@ int postnorm_layer(const sd_seq_model& m, const sd_seq_layer& l, const sd_seq_ba
     SQ_TRY(sd_causal_conv_rows(proj + c.xbc, ld, l.conv_w, l.conv_b, f32, l.conv_state, b.row_pos, b.row_slot,
                                b.entries, b.n_entries, conv, c.conv_ch, R, c.conv_ch, l.s_taps, 1, stream));
     SQ_TRY(sd_ssd_steps(proj + c.dt, ld, l.dt_bias, l.a_log, f32, step, decay, R, Hs, stream));
-    // (long portions of models whose linear layers sum few and many rows in different orders anyway; the scan keeps a
-    // row's bits however a prompt is cut)
-    if (l.w_in_tiled && w.mem_bytes > 0 && sd_decay_chunks_scratch_bytes(R, b.n_entries, Hs, N, P) > 0)
-      SQ_TRY(sd_head_decay_chunks(conv + inner + Gs * N, conv + inner, c.conv_ch, conv, c.conv_ch, decay, 1, step, l.skip_d,
-                                  f32, l.state, b.entries, b.n_entries, R, o, Hs, Gs, N, P, base + w.mem, w.mem_bytes, stream));
-    else
-      SQ_TRY(sd_decay_scan_rows(conv + inner + Gs * N, conv + inner, c.conv_ch, conv, c.conv_ch, decay, step, l.skip_d,
-                                f32, l.state, b.entries, b.n_entries, o, Hs, Gs, N, P, stream));
+    // (long portions in chunks, of models whose linear layers sum few and many rows in different orders anyway; the scan
+    // keeps a row's bits however a prompt is cut)
+    const Portions has = portions(b);
+    const bool chunks = l.w_in_tiled && has.many;
+    if (chunks) {
+      const sd_chunked_decay a{conv + inner + Gs * N, conv + inner, c.conv_ch, conv, c.conv_ch, decay, 1, step, l.skip_d, f32,
+                               1.f, l.state, b.entries, b.n_entries, R, o, Hs, Gs, N, P};
+      SQ_TRY(sd_decay_chunks_(&a, true, false, base + w.mem, w.mem_bytes, stream));
+    }
+    if (has.few || !chunks)
+      SQ_TRY(sd_decay_scan_rows_(conv + inner + Gs * N, conv + inner, c.conv_ch, conv, c.conv_ch, decay, step, l.skip_d,
+                                 f32, l.state, b.entries, b.n_entries, chunks ? kLongPortion : INT_MAX, o, Hs, Gs, N, P,
+                                 stream));
     SQ_TRY(sd_rmsnorm_parts(o, inner, proj + c.z, ld, l.s_norm_w, f32, eps, y, inner, l.w_o2_tiled ? yb : nullptr,
                             inner, R, inner, l.s_norm_groups, rnd, stream));
     SQ_TRY(seq_linear(l.w_o2, l.w_o2_tiled, f32, y, nullptr, inner, yb, inner, nullptr, mix2, W, R, W, inner, wide_ws,
@@ -2019,8 +2045,10 @@ int streams_layer(const sd_seq_model& m, const sd_seq_layer& l, const sd_seq_lay
     float* dec = (float*)(base + w.dec);
     float* o2 = (float*)(base + w.o2);
     SQ_TRY(sd_low_rank_decay(proj + c.a1, ld, l.w_a2, l.b_a2, f32, l.rank, l.tau, dec, R, Hs * N, stream));
-    SQ_TRY(sd_decay_chunks(proj + c.rq, proj + c.rk, proj + c.rv, ld, dec, l.q_scale, l.state, b.entries, b.n_entries, R,
-                           o2, Hs, N, P, base + w.mem, w.mem_bytes, stream));
+    const Portions has = portions(b);
+    const sd_chunked_decay a{proj + c.rq, proj + c.rk, ld, proj + c.rv, ld, dec, 2, nullptr, nullptr, 1, l.q_scale, l.state,
+                             b.entries, b.n_entries, R, o2, Hs, Hs, N, P};
+    SQ_TRY(sd_decay_chunks_(&a, has.many, has.few, base + w.mem, w.mem_bytes, stream));
     SQ_TRY(sd_head_post(o2, proj + c.rg, ld, l.s_norm_w, f32, 1, eps, 0, y2, tiled ? y2b : nullptr, R, Hs, P, rnd, stream));
   }
   // both output matrices: one launch for a few rows where they are stacked
@@ -2236,15 +2264,16 @@ extern "C" int sd_seq_model_forward(sd_seq_model* m, const sd_seq_batch* b, void
         SQ_TRY(sd_sigmoid_power(z, (int64_t)H * dk, l.tau, dec, R, H * dk, stream));
       }
       // (chunks: as in postnorm_layer)
-      if (!l.w_in_tiled || sd_decay_chunks_scratch_bytes(R, b->n_entries, H, dk, dv) == 0)
-        SQ_TRY(sd_decay_scan(proj + c.q, proj + c.k, proj + c.v, ld, pc ? dec : l.head_decay, pc, l.state,
-                             b->entries, b->n_entries, o, H, dk, dv, stream));
-      else if (pc)
-        SQ_TRY(sd_decay_chunks(proj + c.q, proj + c.k, proj + c.v, ld, dec, 1.f, l.state, b->entries, b->n_entries, R, o, H,
-                               dk, dv, base + w.mem, w.mem_bytes, stream));
-      else
-        SQ_TRY(sd_head_decay_chunks(proj + c.q, proj + c.k, ld, proj + c.v, ld, l.head_decay, 0, nullptr, nullptr, 1, l.state,
-                                    b->entries, b->n_entries, R, o, H, H, dk, dv, base + w.mem, w.mem_bytes, stream));
+      const Portions has = portions(*b);
+      const bool chunks = l.w_in_tiled && has.many;
+      if (chunks) {
+        const sd_chunked_decay a{proj + c.q, proj + c.k, ld, proj + c.v, ld, pc ? dec : l.head_decay, pc ? 2 : 0, nullptr,
+                                 nullptr, 1, 1.f, l.state, b->entries, b->n_entries, R, o, H, H, dk, dv};
+        SQ_TRY(sd_decay_chunks_(&a, true, false, base + w.mem, w.mem_bytes, stream));
+      }
+      if (has.few || !chunks)
+        SQ_TRY(sd_decay_scan_(proj + c.q, proj + c.k, proj + c.v, ld, pc ? dec : l.head_decay, pc, l.state, b->entries,
+                              b->n_entries, chunks ? kLongPortion : INT_MAX, o, H, dk, dv, stream));
       SQ_TRY(sd_head_post(o, proj + c.g, ld, l.head_norm_w, f32, 1, d.norm_eps, 0, y, y_b, R, H, dv, rnd, stream));
     }
     SQ_TRY(seq_linear(l.w_o, l.w_o_tiled, f32, y, nullptr, (int64_t)H * dv, yb, (int64_t)H * dv, nullptr, mix, W, R,

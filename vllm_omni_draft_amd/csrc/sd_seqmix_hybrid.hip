@@ -844,7 +844,8 @@ __global__ __launch_bounds__(256) void decay_scan_rows_kernel(
     const float* __restrict__ q, const float* __restrict__ k, int64_t ldqk, const float* __restrict__ v, int64_t ldv,
     const float* __restrict__ decay, const float* __restrict__ k_scale, const T* __restrict__ skip,
     float* __restrict__ state, const int32_t* __restrict__ entries,
-    float* __restrict__ out, int H, int hpg, int dk, int dv, int CT, int NS, int CH) {
+    float* __restrict__ out, int H, int hpg, int dk, int dv, int CT, int NS, int CH, int max_rows) {
+  if (entries[4 * blockIdx.z + 2] > max_rows) return;
   extern __shared__ float lds[];
   const int dkp = NS * kStrip;
   float* qs = lds;                  // [CH][dkp]
@@ -2328,6 +2329,13 @@ extern "C" int sd_decay_scan_rows(const float* q, const float* k, int64_t ldqk, 
                                   const float* decay, const float* k_scale, const void* skip, int w_f32, float* state,
                                   const int32_t* entries, int n_entries, float* out, int H, int Gq, int dk, int dv,
                                   sd_stream_t stream) {
+  return sd_decay_scan_rows_(q, k, ldqk, v, ldv, decay, k_scale, skip, w_f32, state, entries, n_entries, INT_MAX, out, H,
+                             Gq, dk, dv, stream);
+}
+
+int sd_decay_scan_rows_(const float* q, const float* k, int64_t ldqk, const float* v, int64_t ldv, const float* decay,
+                        const float* k_scale, const void* skip, int w_f32, float* state, const int32_t* entries,
+                        int n_entries, int max_rows, float* out, int H, int Gq, int dk, int dv, sd_stream_t stream) {
   SD_REQUIRE(q && k && v && decay && state && entries && out && n_entries >= 1 && H >= 1 && Gq >= 1 && H % Gq == 0 &&
                  dv >= 1,
              SD_ERR_INVALID, "sd_decay_scan_rows: bad argument");
@@ -2349,10 +2357,10 @@ extern "C" int sd_decay_scan_rows(const float* q, const float* k, int64_t ldqk, 
   const int hpg = H / Gq;
   if (w_f32)
     decay_scan_rows_kernel<float><<<grid, CT * NS, lds, st>>>(q, k, ldqk, v, ldv, decay, k_scale, (const float*)skip,
-                                                              state, entries, out, H, hpg, dk, dv, CT, NS, CH);
+                                                              state, entries, out, H, hpg, dk, dv, CT, NS, CH, max_rows);
   else
     decay_scan_rows_kernel<bf16_t><<<grid, CT * NS, lds, st>>>(q, k, ldqk, v, ldv, decay, k_scale, (const bf16_t*)skip,
-                                                               state, entries, out, H, hpg, dk, dv, CT, NS, CH);
+                                                               state, entries, out, H, hpg, dk, dv, CT, NS, CH, max_rows);
   SD_CHECK_LAUNCH("sd_decay_scan_rows");
   return SD_OK;
 }

@@ -531,24 +531,37 @@ struct ChunkArgs {
   float* out;              // [rows, H*dv]
   float* cs;               // [chunks, H, dk, dv]: own sums, then the state at the chunk's start
   float* ct;               // [chunks, H, 2, dk]: product of the chunk's decays, and what its rounding left
-  int n_entries, H, dk, dv, chunk;
+  int n_entries, H, dk, dv;
+  int whole_rows;          // kWhole: portions of more rows are left alone
 };
 constexpr int kBlock = 16;       // tokens of a block
 constexpr int kBlockCols = 128;  // value columns per workgroup
 constexpr int kTokLd = kBlock + 4;
 constexpr int kChunkThreads = 512;
 
-// The portion and the first row (inside it) of the n-th group of `per` rows over all portions.
-__device__ __forceinline__ bool nth_group(const int32_t* entries, int n_entries, int per, int n, int* e, int* first) {
+// Tokens of a chunk of a portion: more, and so less carried state, where the portion alone still fills the chip; and how
+// many chunks it has.  (Of the portion's own rows: what shares its pass must not change its sums.)
+constexpr int kChunkMin = kLongPortion, kChunkMax = 2 * kLongPortion;
+__host__ __device__ inline int chunk_of(int rows, int H, int dv) {
+  return (long long)(rows / kChunkMax) * H * ((dv + kBlockCols - 1) / kBlockCols) >= 256 ? kChunkMax : kChunkMin;
+}
+__host__ __device__ inline int chunks_of(int rows, int H, int dv) {
+  const int c = chunk_of(rows, H, dv);
+  return rows <= kLongPortion ? 0 : (rows + c - 1) / c;
+}
+
+// The portion and the first row (inside it) of the n-th chunk over all portions.
+__device__ __forceinline__ bool nth_chunk(const ChunkArgs& g, int n, int* e, int* first) {
   int i = 0;
-  for (; i < n_entries; ++i) {
-    const int len = entries[4 * i + 2], groups = len / per + (len % per != 0);
-    if (n < groups) break;
-    n -= groups;
+  for (; i < g.n_entries; ++i) {
+    const int chunks = chunks_of(g.entries[4 * i + 2], g.H, g.dv);
+    if (n < chunks) break;
+    n -= chunks;
   }
+  if (i == g.n_entries) return false;
   *e = i;
-  *first = n * per;
-  return i < n_entries;
+  *first = n * chunk_of(g.entries[4 * i + 2], g.H, g.dv);
+  return true;
 }
 
 // Up to 16 rows of up to COLS columns on their way from memory to LDS, V columns a piece.
@@ -635,12 +648,13 @@ __global__ __launch_bounds__(kChunkThreads, DKP <= 128 ? 4 : 2) void decay_chunk
   if constexpr (MODE == kWhole) {
     e = blockIdx.x;
     first = 0;
+    if (g.entries[4 * e + 2] > g.whole_rows) return;
   } else {
-    if (!nth_group(g.entries, g.n_entries, g.chunk, blockIdx.x, &e, &first)) return;
+    if (!nth_chunk(g, blockIdx.x, &e, &first)) return;
   }
   const int slot = g.entries[4 * e], row0 = g.entries[4 * e + 1] + first, left = g.entries[4 * e + 2] - first;
   const bool kept = g.entries[4 * e + 3] > 0;
-  const int nt = MODE == kWhole ? left : (left < g.chunk ? left : g.chunk);
+  const int nt = MODE == kWhole ? left : min(left, chunk_of(g.entries[4 * e + 2], H, dv));
   const size_t at = ((size_t)blockIdx.x * H + h) * dk;            // the chunk's place in ct, and (times dv) in cs
   float* slot_state = g.state + ((size_t)slot * H + h) * dk * dv + c0;
   BlockRows<DKP, V> rq, rk, rd, rs;
@@ -855,8 +869,9 @@ __global__ __launch_bounds__(256) void chunk_carry_kernel(ChunkArgs g) {
   if (x >= dk * dv) return;
   const int slot = g.entries[4 * e], len = g.entries[4 * e + 2];
   int first = 0;
-  for (int i = 0; i < e; ++i) first += (g.entries[4 * i + 2] + g.chunk - 1) / g.chunk;
-  const int nc = (len + g.chunk - 1) / g.chunk;
+  const int nc = chunks_of(len, H, dv);
+  if (nc == 0) return;
+  for (int i = 0; i < e; ++i) first += chunks_of(g.entries[4 * i + 2], H, dv);
   float* st = g.state + ((size_t)slot * H + h) * dk * dv + x;
   float* own = g.cs + ((size_t)first * H + h) * dk * dv + x;
   const float* ct = g.ct + ((size_t)first * H + h) * 2 * dk + x / dv;
@@ -882,8 +897,9 @@ __global__ __launch_bounds__(256) void chunk_carry_kernel(ChunkArgs g) {
   *st = val;
 }
 
+// nc chunks at most (0: none), and with `whole` the portions of at most c.whole_rows rows
 template <int DKP, int V, bool SCALAR>
-hipError_t launch_decay_chunks(const ChunkArgs& c, size_t nc, hipStream_t st) {
+hipError_t launch_decay_chunks(const ChunkArgs& c, size_t nc, bool whole, hipStream_t st) {
   static std::once_flag once;
   static hipError_t err = hipSuccess;
   std::call_once(once, [] {
@@ -896,16 +912,14 @@ hipError_t launch_decay_chunks(const ChunkArgs& c, size_t nc, hipStream_t st) {
   if (err != hipSuccess) return err;
   constexpr size_t lds = decay_chunk_lds<DKP>();
   const unsigned z = (c.dv + kBlockCols - 1) / kBlockCols;
-  if (nc == 0) {
-    decay_chunk_kernel<DKP, V, kWhole, SCALAR><<<dim3(c.n_entries, c.H, z), kChunkThreads, lds, st>>>(c);
-  } else {
+  if (whole) decay_chunk_kernel<DKP, V, kWhole, SCALAR><<<dim3(c.n_entries, c.H, z), kChunkThreads, lds, st>>>(c);
+  if (nc > 0) {
     decay_chunk_kernel<DKP, V, kSums, SCALAR><<<dim3((unsigned)nc, c.H, z), kChunkThreads, lds, st>>>(c);
     chunk_carry_kernel<<<dim3((c.dk * c.dv + 255) / 256, c.H, c.n_entries), 256, 0, st>>>(c);
     decay_chunk_kernel<DKP, V, kReads, SCALAR><<<dim3((unsigned)nc, c.H, z), kChunkThreads, lds, st>>>(c);
   }
   return hipGetLastError();
 }
-constexpr int kChunkMin = 64, kChunkMax = 128;
 
 int check_step(const sd_decay_step* s, const int32_t* row_pos, const int32_t* row_slot, int n_rows) {
   SD_REQUIRE(s && s->q && s->k && s->v && s->a1 && s->a2 && s->a2_bias && s->state && s->gate && s->norm_w &&
@@ -1041,33 +1055,43 @@ extern "C" int sd_low_rank_decay(const float* a1, int64_t ld, const void* a2, co
 }
 
 extern "C" size_t sd_decay_chunks_scratch_bytes(int n_rows, int n_entries, int H, int dk, int dv) {
-  // (rows that fill no more than a chunk beyond one per portion run in one go)
-  if (n_rows < 1 || n_entries < 1 || n_rows - n_entries < kChunkMin || H < 1 || dk < 1 || dv < 1) return 0;
-  return sizeof(float) * ((size_t)n_rows / kChunkMin + n_entries) * H * ((size_t)dk * dv + 2 * dk);
+  // (no portion is longer than n_rows - n_entries + 1, and those of up to kLongPortion rows have no chunks)
+  if (n_rows < 1 || n_entries < 1 || n_rows - n_entries < kLongPortion || H < 1 || dk < 1 || dv < 1) return 0;
+  const int most = n_rows / (kLongPortion + 1);
+  return sizeof(float) * ((size_t)n_rows / kChunkMin + (n_entries < most ? n_entries : most)) * H * ((size_t)dk * dv + 2 * dk);
 }
 
-namespace {
-int decay_chunks(ChunkArgs c, bool scalar, int n_rows, void* scratch, size_t scratch_bytes, sd_stream_t stream) {
+int sd_decay_chunks_(const sd_chunked_decay* a, bool chunks, bool whole, void* scratch, size_t scratch_bytes,
+                     sd_stream_t stream) {
+  SD_REQUIRE(a->q && a->k && a->v && a->decay && a->state && a->entries && a->out && a->n_entries >= 1 &&
+                 a->n_rows >= a->n_entries && a->H >= 1 && a->Gq >= 1 && a->H % a->Gq == 0 && a->dv >= 1,
+             SD_ERR_INVALID, "sd_decay_chunks: bad argument");
+  SD_REQUIRE(a->dk >= 1 && a->dk <= 256, SD_ERR_UNSUPPORTED, "sd_decay_chunks: key size %d outside 1..256", a->dk);
+  ChunkArgs c{a->q, a->k, a->v, a->ldqk, a->ldv, a->decay, a->per == 1 ? a->H : 0, a->k_scale, a->skip, a->w_f32, a->H / a->Gq,
+              a->q_scale, a->state, a->entries, a->out, nullptr, nullptr, a->n_entries, a->H, a->dk, a->dv, INT_MAX};
+  const bool scalar = a->per != 2;   // (one decay per head: all channels of a block share their running products)
   const int H = c.H, dk = c.dk, dv = c.dv;
-  const size_t need = sd_decay_chunks_scratch_bytes(n_rows, c.n_entries, H, dk, dv);
-  const bool cut = need > 0 && scratch && scratch_bytes >= need && sd_aligned16(scratch);
+  const size_t need = sd_decay_chunks_scratch_bytes(a->n_rows, c.n_entries, H, dk, dv);
   size_t nc = 0;
-  c.chunk = kChunkMin;
-  if (cut) {
-    // (longer chunks, and so less carried state, where they still fill the chip)
-    const long long wgs = (long long)(n_rows / kChunkMax) * H * ((dv + kBlockCols - 1) / kBlockCols);
-    c.chunk = wgs >= 256 ? kChunkMax : kChunkMin;
-    nc = (size_t)n_rows / c.chunk + c.n_entries;
-    c.cs = (float*)scratch;
-    c.ct = c.cs + nc * H * dk * dv;
+  if (chunks && need > 0) {
+    if (scratch && scratch_bytes >= need && sd_aligned16(scratch)) {
+      const size_t room = need / (sizeof(float) * H * ((size_t)dk * dv + 2 * dk));
+      nc = c.n_entries == 1 ? chunks_of(a->n_rows, H, dv) : room;
+      c.cs = (float*)scratch;
+      c.ct = c.cs + room * H * dk * dv;
+      c.whole_rows = kLongPortion;
+      whole = whole && c.n_entries > 1;
+    } else {
+      SD_REQUIRE(whole, SD_ERR_WORKSPACE, "sd_decay_chunks: scratch %zu < %zu bytes", scratch_bytes, need);
+    }
   }
   const bool quad = c.ld % 4 == 0 && c.ldv % 4 == 0 && dk % 4 == 0 && dv % 4 == 0 && sd_aligned16(c.q) && sd_aligned16(c.k) &&
                     sd_aligned16(c.v) && (scalar || sd_aligned16(c.decay));
   hipStream_t st = (hipStream_t)stream;
   hipError_t err;
 #define SD_GO(D)                                                                                                        \
-  err = scalar ? (quad ? launch_decay_chunks<D, 4, true>(c, nc, st) : launch_decay_chunks<D, 1, true>(c, nc, st))       \
-               : (quad ? launch_decay_chunks<D, 4, false>(c, nc, st) : launch_decay_chunks<D, 1, false>(c, nc, st))
+  err = scalar ? (quad ? launch_decay_chunks<D, 4, true>(c, nc, whole, st) : launch_decay_chunks<D, 1, true>(c, nc, whole, st)) \
+               : (quad ? launch_decay_chunks<D, 4, false>(c, nc, whole, st) : launch_decay_chunks<D, 1, false>(c, nc, whole, st))
   if (dk <= 32) SD_GO(32);
   else if (dk <= 64) SD_GO(64);
   else if (dk <= 128) SD_GO(128);
@@ -1076,30 +1100,21 @@ int decay_chunks(ChunkArgs c, bool scalar, int n_rows, void* scratch, size_t scr
   SD_REQUIRE(err == hipSuccess, SD_ERR_HIP, "sd_decay_chunks: launch failed: %s", hipGetErrorString(err));
   return SD_OK;
 }
-}  // namespace
 
+// (a portion beyond kLongPortion rows runs in one go without scratch)
 extern "C" int sd_decay_chunks(const float* q, const float* k, const float* v, int64_t ld, const float* decay,
                                float q_scale, float* state, const int32_t* entries, int n_entries, int n_rows, float* out,
                                int H, int dk, int dv, void* scratch, size_t scratch_bytes, sd_stream_t stream) {
-  SD_REQUIRE(q && k && v && decay && state && entries && out && n_entries >= 1 && n_rows >= n_entries && H >= 1 && dv >= 1,
-             SD_ERR_INVALID, "sd_decay_chunks: bad argument");
-  SD_REQUIRE(dk >= 1 && dk <= 256, SD_ERR_UNSUPPORTED, "sd_decay_chunks: key size %d outside 1..256", dk);
-  ChunkArgs c{q, k, v, ld, ld, decay, 0, nullptr, nullptr, 0, 1, q_scale, state, entries, out, nullptr, nullptr, n_entries,
-              H, dk, dv, kChunkMin};
-  return decay_chunks(c, false, n_rows, scratch, scratch_bytes, stream);
+  const sd_chunked_decay a{q, k, ld, v, ld, decay, 2, nullptr, nullptr, 0, q_scale, state, entries, n_entries, n_rows, out, H,
+                           H, dk, dv};
+  return sd_decay_chunks_(&a, true, true, scratch, scratch_bytes, stream);
 }
 
-// One decay per head (of every row: decay_per_row, else of the head): all channels of a block then share their running
-// products, the rest is the same.
 extern "C" int sd_head_decay_chunks(const float* q, const float* k, int64_t ldqk, const float* v, int64_t ldv,
                                     const float* decay, int decay_per_row, const float* k_scale, const void* skip, int w_f32,
                                     float* state, const int32_t* entries, int n_entries, int n_rows, float* out, int H,
                                     int Gq, int dk, int dv, void* scratch, size_t scratch_bytes, sd_stream_t stream) {
-  SD_REQUIRE(q && k && v && decay && state && entries && out && n_entries >= 1 && n_rows >= n_entries && H >= 1 && Gq >= 1 &&
-                 H % Gq == 0 && dv >= 1,
-             SD_ERR_INVALID, "sd_head_decay_chunks: bad argument");
-  SD_REQUIRE(dk >= 1 && dk <= 256, SD_ERR_UNSUPPORTED, "sd_head_decay_chunks: key size %d outside 1..256", dk);
-  ChunkArgs c{q, k, v, ldqk, ldv, decay, decay_per_row ? H : 0, k_scale, skip, w_f32, H / Gq, 1.f, state, entries, out,
-              nullptr, nullptr, n_entries, H, dk, dv, kChunkMin};
-  return decay_chunks(c, true, n_rows, scratch, scratch_bytes, stream);
+  const sd_chunked_decay a{q, k, ldqk, v, ldv, decay, decay_per_row ? 1 : 0, k_scale, skip, w_f32, 1.f, state, entries,
+                           n_entries, n_rows, out, H, Gq, dk, dv};
+  return sd_decay_chunks_(&a, true, true, scratch, scratch_bytes, stream);
 }

@@ -459,12 +459,13 @@ class SeqModel:
         self.workspace = torch.empty(int(n), dtype=torch.uint8, device=self.weights.embed.device)
 
     def forward(self, n_rows: int, n_entries: int, tokens, row_pos, row_slot, entries, n_out: int,
-                out_rows, logits, layer_out=None, prev_tokens=None) -> None:
+                out_rows, logits, layer_out=None, prev_tokens=None, portion_rows=(0, 0)) -> None:
         """int32 device tensors tokens / row_pos / row_slot [n_rows], entries [n_entries, 4]
         {slot, first row, rows, first position}, out_rows [n_out]; logits f32 [n_out, vocab];
         layer_out (optional) f32 [n_layers, n_rows, width] receives the residual after each layer;
         prev_tokens int32 [n_rows] (models with a bigram table): the token before each row in its
-        sequence, -1 for a sequence's first."""
+        sequence, -1 for a sequence's first; portion_rows: rows of the shortest and the longest entry, where
+        known."""
         if self.cfg.bigram is not None:
             if prev_tokens is None or prev_tokens.dtype != torch.int32 or not prev_tokens.is_contiguous() \
                     or not prev_tokens.is_cuda or prev_tokens.numel() < n_rows:
@@ -490,7 +491,7 @@ class SeqModel:
                               max_blocks=c.max_blocks_per_seq, page=c.page, n_out=n_out,
                               out_rows=_ptr(out_rows) if n_out else None,
                               logits=_ptr(logits) if n_out else None, layer_out=_ptr(layer_out),
-                              prev_tokens=_ptr(prev_tokens))
+                              prev_tokens=_ptr(prev_tokens), shortest=portion_rows[0], longest=portion_rows[1])
         rc = _lib.load().sd_seq_model_forward(self._handle, C.byref(batch), self.workspace.data_ptr(),
                                               self.workspace.numel(), ops._stream())
         _lib.check(rc, "sd_seq_model_forward")

@@ -238,7 +238,7 @@ class SeqEngine:
             dst = logits[out_dst[0]:out_dst[0] + O]
         else:
             dst = torch.empty(O, V, dtype=torch.float32, device=self.device)
-        self.model.forward(R, E, a, b, c, e, O, o if O else None, dst, trace, p)
+        self.model.forward(R, E, a, b, c, e, O, o if O else None, dst, trace, p, (min(ents[2::4]), max(ents[2::4])))
         if O and not contiguous_out:
             logits[torch.tensor(out_dst, device=self.device)] = dst
         self.passes += 1

@@ -823,3 +823,29 @@ def test_a_portions_bits_do_not_depend_on_what_shares_its_pass():
         assert torch.equal(a, b), len(t)
         want = oracle_logits(cfg, st, t)
         assert sorted(rel(b[r], want[r]) for r in range(len(t)))[len(t) // 2] < 2e-2   # (see test_bfloat16_serving_stays_close)
+
+
+def test_attention_of_a_portion_does_not_depend_on_what_shares_its_pass():
+    """The same with heads whose long portions attend on the matrix cores (grouped heads of 128 channels with kept tokens,
+    latent rows of 512 + 64), short portions and decoded tokens beside them on the vector pipe; and a prompt in one pass
+    and cut against the plain model."""
+    from tests.test_gpu_puguzen import beside_others
+    attn = dict(heads=4, kv_heads=2, dim=128, vdim=128, scale=128 ** -0.5)
+    lat = dict(heads=2, dim=32, rot_dim=64, vdim=32, q_rank=32, kv_rank=512, scale=0.1)
+    cfg = model_cfg([latent(window=60, **lat), parallel(window=50, keep_first=3, s_heads=4, s_vdim=32, state=32, **attn)], width=128)
+    mid = lambda x, y: sorted(rel(x[r], y[r]) for r in range(len(y)))[len(y) // 2]   # (see test_bfloat16_serving_stays_close)
+    st, toks, alone, beside = beside_others(build, cfg, [150, 64, 20, 65])
+    for t, a, b in zip(toks, alone, beside):
+        assert torch.equal(a, b), len(t)
+        assert mid(b, oracle_logits(cfg, st, t)) < 2e-2
+    cfg = model_cfg([latent(window=1000, **lat), parallel(window=200, keep_first=3, s_heads=4, s_vdim=32, state=32, **attn)], width=128)
+    st, eng = build(cfg, torch.bfloat16)
+    t = prompt(cfg, 400, 1)
+    want = oracle_logits(cfg, st, t)
+    for cuts in ([400], [100, 300], [70, 1, 200, 17, 112]):
+        at, got = 0, []
+        for c in cuts:
+            got.append(eng.step([("c", t[at:at + c], list(range(c)))]))
+            at += c
+        eng.finish("c")
+        assert mid(torch.cat(got), want) < 2e-2, cuts

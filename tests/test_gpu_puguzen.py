@@ -815,3 +815,25 @@ def test_a_portions_bits_do_not_depend_on_what_shares_its_pass():
     for t, a, b in zip(toks, alone, beside):
         assert torch.equal(a, b), len(t)
         assert rel(b, oracle_logits(cfg, st, t)) < 0.03
+
+
+def test_attention_of_a_portion_does_not_depend_on_what_shares_its_pass():
+    """The same with heads whose long portions attend on the matrix cores, decoded tokens and short portions beside them on
+    the vector pipe; and a prompt in one pass, cut, and beside others against the plain model."""
+    cfg = model_cfg([layer("attention", heads=4, kv_heads=2, dim=128, vdim=128, window=40, pool=16, scale=128 ** -0.5),
+                     layer("retention", heads=2, dim=128, vdim=128), layer("attention", heads=2, kv_heads=2, dim=128, vdim=128, window=300,
+                                                                           pool=5, scale=128 ** -0.5)], width=128)
+    st, toks, alone, beside = beside_others(build, cfg, [150, 64, 20, 65])
+    for t, a, b in zip(toks, alone, beside):
+        assert torch.equal(a, b), len(t)
+        assert rel(b, oracle_logits(cfg, st, t)) < 0.03
+    _, eng = build(cfg, torch.bfloat16, seed=3)
+    t = prompt(cfg, 400, 1)
+    want = oracle_logits(cfg, st, t)
+    for cuts in ([400], [100, 300], [70, 1, 200, 17, 112]):
+        at, got = 0, []
+        for c in cuts:
+            got.append(eng.step([("c", t[at:at + c], list(range(c)))]))
+            at += c
+        eng.finish("c")
+        assert rel(torch.cat(got), want) < 0.03, cuts

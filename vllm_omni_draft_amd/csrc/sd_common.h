@@ -77,6 +77,25 @@ struct sd_chunked_decay {
 int sd_decay_chunks_(const sd_chunked_decay* a, bool chunks, bool whole, void* scratch, size_t scratch_bytes,
                      sd_stream_t stream);
 
+// sd_window_softmax_attention and sd_window_pool_attention without the rows of long portions (skip_long; the pooled
+// blocks are in the cache already then), whose attention is sd_rows_softmax_attention's and sd_rows_pool_attention's:
+// here with the long portions alone (long_only; all portions' blocks are pooled).
+int sd_window_softmax_attention_(const float* q, int64_t ldq, const void* k_cache, const void* v_cache, int cache_f32,
+                                 const int32_t* row_pos, const int32_t* row_slot, const int32_t* block_tables,
+                                 int max_blocks, int page, int n_rows, int H, int G, int dk, int dv, int window,
+                                 int keep_first, float scale, const int32_t* entries, int n_entries, bool skip_long,
+                                 float* out, void* out_bf16, void* scratch, size_t scratch_bytes, sd_stream_t stream);
+int sd_window_pool_attention_(const float* q, int64_t ldq, const void* k_cache, const void* v_cache, int cache_f32,
+                              float* pk_cache, float* pv_cache, const int32_t* row_pos, const int32_t* row_slot,
+                              const int32_t* block_tables, int max_blocks, int page, int n_rows, int H, int G, int dk,
+                              int dv, int window, int pool, float scale, const float* head_bias, const int32_t* entries,
+                              int n_entries, bool skip_long, float* out, void* scratch, size_t scratch_bytes,
+                              sd_stream_t stream);
+int sd_rows_softmax_attention_(const float* q, int64_t ldq, const void* k_cache, const void* v_cache,
+                               const int32_t* block_tables, int max_blocks, int page, int n_rows, int H, int G, int dk,
+                               int dv, int window, int keep_first, float scale, const int32_t* entries, int n_entries,
+                               bool long_only, float* out, void* out_bf16, int64_t ldo, sd_stream_t stream);
+
 // sd_gated_softmax_attention's tiled form (sd_seqmix_joint.hip); SD_ERR_UNSUPPORTED: sizes it does
 // not take.
 int sd_tiled_window_attention_(const float* q, int64_t ldq, const void* k_cache, const void* v_cache,
@@ -90,8 +109,8 @@ int sd_tiled_window_attention_(const float* q, int64_t ldq, const void* k_cache,
 bool sd_rows_softmax_attention_fits_(int H, int G, int dk, int dv, int page, bool latent);
 int sd_rows_pool_attention_(const float* q, int64_t ldq, const void* k_cache, const void* v_cache, const float* pk, const float* pv,
                             const int32_t* block_tables, int max_blocks, int n_rows, int H, int G, int window, int pool, int pslots,
-                            float scale, const float* head_bias, const int32_t* entries, int n_entries, float* out,
-                            sd_stream_t stream);
+                            float scale, const float* head_bias, const int32_t* entries, int n_entries, bool long_only,
+                            float* out, sd_stream_t stream);
 
 #define SD_REQUIRE(cond, code, ...)            \
   do {                                         \

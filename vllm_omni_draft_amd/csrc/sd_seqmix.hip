@@ -514,7 +514,9 @@ __global__ __launch_bounds__(256) void window_pool_attn_kernel(
     const int32_t* __restrict__ row_pos, const int32_t* __restrict__ row_slot,
     const int32_t* __restrict__ block_tables, int max_blocks, int page, int pslots, int H, int G, int dk,
     int dv, int window, int pool, float scale, const float* __restrict__ head_bias,
-    float* __restrict__ out, int n_hgroups, int n_splits, size_t split_stride) {
+    float* __restrict__ out, int n_hgroups, int n_splits, size_t split_stride, const int32_t* __restrict__ skip,
+    int n_skip) {
+  if (skip && sd_in_long_portion(skip, n_skip, blockIdx.x)) return;   // (entries whose long portions have another kernel)
   extern __shared__ float lds[];
   unsigned long long* vat = reinterpret_cast<unsigned long long*>(lds);  // [kAttnTile] cache row of the value
   float* wt = reinterpret_cast<float*>(vat + kAttnTile);                 // [NH][kAttnTile]
@@ -633,12 +635,12 @@ void launch_attn_nc(dim3 grid, size_t lds, hipStream_t st, int nc, const float* 
                     const void* vc, const float* pk, const float* pv, const int32_t* row_pos,
                     const int32_t* row_slot, const int32_t* bt, int max_blocks, int page, int pslots, int H, int G,
                     int dk, int dv, int window, int pool, float scale, const float* head_bias, float* out,
-                    int n_hgroups, int n_splits, size_t split_stride) {
+                    int n_hgroups, int n_splits, size_t split_stride, const int32_t* skip, int n_skip) {
 #define SD_ATTN_GO(NC)                                                                                           \
   window_pool_attn_kernel<T, NH, NC><<<grid, 256, lds, st>>>(q, ldq, (const T*)kc, (const T*)vc, pk, pv, row_pos, \
                                                              row_slot, bt, max_blocks, page, pslots, H, G, dk, dv, \
                                                              window, pool, scale, head_bias, out, n_hgroups,       \
-                                                             n_splits, split_stride)
+                                                             n_splits, split_stride, skip, n_skip)
   if (nc == 1) SD_ATTN_GO(1);
   else if (nc == 2) SD_ATTN_GO(2);
   else SD_ATTN_GO(4);
@@ -1056,6 +1058,17 @@ extern "C" int sd_window_pool_attention(const float* q, int64_t ldq, const void*
                                         int H, int G, int dk, int dv, int window, int pool, float scale,
                                         const float* head_bias, float* out, void* scratch, size_t scratch_bytes,
                                         sd_stream_t stream) {
+  return sd_window_pool_attention_(q, ldq, k_cache, v_cache, cache_f32, pk_cache, pv_cache, row_pos, row_slot, block_tables,
+                                   max_blocks, page, n_rows, H, G, dk, dv, window, pool, scale, head_bias, nullptr, 0, false,
+                                   out, scratch, scratch_bytes, stream);
+}
+
+int sd_window_pool_attention_(const float* q, int64_t ldq, const void* k_cache, const void* v_cache, int cache_f32,
+                              float* pk_cache, float* pv_cache, const int32_t* row_pos, const int32_t* row_slot,
+                              const int32_t* block_tables, int max_blocks, int page, int n_rows, int H, int G, int dk,
+                              int dv, int window, int pool, float scale, const float* head_bias, const int32_t* entries,
+                              int n_entries, bool skip_long, float* out, void* scratch, size_t scratch_bytes,
+                              sd_stream_t stream) {
   SD_REQUIRE(q && k_cache && v_cache && pk_cache && pv_cache && row_pos && row_slot && block_tables && out,
              SD_ERR_INVALID, "sd_window_pool_attention: null argument");
   SD_REQUIRE(n_rows >= 1 && H >= 1 && G >= 1 && H % G == 0 && dk >= 1 && window >= 1 && pool >= 1 && page >= 1,
@@ -1071,7 +1084,8 @@ extern "C" int sd_window_pool_attention(const float* q, int64_t ldq, const void*
   const int nc = dv <= 64 ? 1 : (dv <= 128 ? 2 : 4);
   // Few rows: the keys of a row are cut into tiles that run as workgroups of their own.
   const size_t need = sd_window_pool_attention_scratch_bytes(n_rows, H, dv, window, pool, max_blocks * page);
-  const bool split = need > 0 && scratch && scratch_bytes >= need;
+  // (a pass with a long portion has more rows than are ever split)
+  const bool split = !skip_long && need > 0 && scratch && scratch_bytes >= need;
   const int n_splits = split ? (int)(need / ((size_t)n_rows * H * dv * sizeof(float))) : 1;
   const size_t split_stride = (size_t)n_rows * H * dv;
   dim3 ga(n_rows, G, n_hgroups * n_splits);
@@ -1080,17 +1094,19 @@ extern "C" int sd_window_pool_attention(const float* q, int64_t ldq, const void*
   SD_REQUIRE(lds <= 64 * 1024, SD_ERR_UNSUPPORTED, "sd_window_pool_attention: dim %d / vdim %d need %zu bytes of LDS",
              dk, dv, lds);
   float* dst = split ? (float*)scratch : out;
-  if (cache_f32)
-    pool_blocks_kernel<float><<<gp, 256, 0, st>>>((const float*)k_cache, (const float*)v_cache, pk_cache, pv_cache,
-                                                 row_pos, row_slot, block_tables, max_blocks, page, pslots, G, dk, dv, pool);
-  else
-    pool_blocks_kernel<bf16_t><<<gp, 256, 0, st>>>((const bf16_t*)k_cache, (const bf16_t*)v_cache, pk_cache, pv_cache,
-                                                  row_pos, row_slot, block_tables, max_blocks, page, pslots, G, dk, dv, pool);
+  if (!skip_long) {
+    if (cache_f32)
+      pool_blocks_kernel<float><<<gp, 256, 0, st>>>((const float*)k_cache, (const float*)v_cache, pk_cache, pv_cache, row_pos,
+                                                    row_slot, block_tables, max_blocks, page, pslots, G, dk, dv, pool);
+    else
+      pool_blocks_kernel<bf16_t><<<gp, 256, 0, st>>>((const bf16_t*)k_cache, (const bf16_t*)v_cache, pk_cache, pv_cache, row_pos,
+                                                     row_slot, block_tables, max_blocks, page, pslots, G, dk, dv, pool);
+  }
   SD_CHECK_LAUNCH("sd_window_pool_attention (pool)");
 #define SD_ATTN_NH(T, N)                                                                                          \
   launch_attn_nc<T, N>(ga, lds, st, nc, q, ldq, k_cache, v_cache, pk_cache, pv_cache, row_pos, row_slot, block_tables, \
                        max_blocks, page, pslots, H, G, dk, dv, window, pool, scale, head_bias, dst, n_hgroups,     \
-                       n_splits, split_stride)
+                       n_splits, split_stride, skip_long ? entries : nullptr, n_entries)
 #define SD_ATTN_T(T)                  \
   do {                                \
     if (NH == 1) SD_ATTN_NH(T, 1);    \
@@ -1111,11 +1127,12 @@ extern "C" int sd_window_pool_attention(const float* q, int64_t ldq, const void*
   return SD_OK;
 }
 
-extern "C" int sd_rows_pool_attention(const float* q, int64_t ldq, const void* k_cache, const void* v_cache, float* pk_cache,
-                                      float* pv_cache, const int32_t* block_tables, int max_blocks, int page, int n_rows,
-                                      int H, int G, int dk, int dv, int window, int pool, float scale,
-                                      const float* head_bias, const int32_t* entries, int n_entries, float* out,
-                                      sd_stream_t stream) {
+namespace {
+// long_only: attention of the long portions (all portions' blocks are pooled)
+int rows_pool_attention(const float* q, int64_t ldq, const void* k_cache, const void* v_cache, float* pk_cache, float* pv_cache,
+                        const int32_t* block_tables, int max_blocks, int page, int n_rows, int H, int G, int dk, int dv,
+                        int window, int pool, float scale, const float* head_bias, const int32_t* entries, int n_entries,
+                        bool long_only, float* out, sd_stream_t stream) {
   SD_REQUIRE(q && k_cache && v_cache && pk_cache && pv_cache && block_tables && entries && out, SD_ERR_INVALID,
              "sd_rows_pool_attention: null argument");
   SD_REQUIRE(n_entries >= 1 && n_rows >= n_entries && H >= 1 && G >= 1 && window >= 1 && pool >= 1 && max_blocks >= 1 &&
@@ -1130,7 +1147,17 @@ extern "C" int sd_rows_pool_attention(const float* q, int64_t ldq, const void* k
       pslots, G, dk, dv, pool);
   SD_CHECK_LAUNCH("sd_rows_pool_attention (pool)");
   return sd_rows_pool_attention_(q, ldq, k_cache, v_cache, pk_cache, pv_cache, block_tables, max_blocks, n_rows, H, G, window,
-                                 pool, pslots, scale, head_bias, entries, n_entries, out, stream);
+                                 pool, pslots, scale, head_bias, entries, n_entries, long_only, out, stream);
+}
+}  // namespace
+
+extern "C" int sd_rows_pool_attention(const float* q, int64_t ldq, const void* k_cache, const void* v_cache, float* pk_cache,
+                                      float* pv_cache, const int32_t* block_tables, int max_blocks, int page, int n_rows,
+                                      int H, int G, int dk, int dv, int window, int pool, float scale,
+                                      const float* head_bias, const int32_t* entries, int n_entries, float* out,
+                                      sd_stream_t stream) {
+  return rows_pool_attention(q, ldq, k_cache, v_cache, pk_cache, pv_cache, block_tables, max_blocks, page, n_rows, H, G, dk,
+                             dv, window, pool, scale, head_bias, entries, n_entries, false, out, stream);
 }
 
 extern "C" int sd_gated_residual(float* x, const float* z1, const float* z2, int64_t ldz, const float* c1,
@@ -1644,15 +1671,15 @@ Portions portions(const sd_seq_batch& b) {
   return {shortest <= kLongPortion, longest > kLongPortion};
 }
 
-// Attention on the matrix cores for a pass with more than a few prompt rows (as for the chunked recurrences: of models
-// whose linear layers sum few and many rows in different orders anyway; a row's bits do not depend on the cut else).
+// Attention on the matrix cores for long portions (as for the chunked recurrences: of models whose linear layers sum few
+// and many rows in different orders anyway; portions of up to kLongPortion rows keep the kernel on the vector pipe, in the
+// same pass too).
 // 64 rows of one portion: 16 heads over 4 of 128 channels 14.8 -> 13.3 us from nothing, 362 -> 143 behind 4000 tokens;
-// 16 latent heads 63 -> 18 and 1305 -> 482; portions of 9 rows gain as much.  With a window of 1024 and pooled blocks (16
-// heads over 4): 21.7 -> 17.6 from nothing, 132 -> 65 behind 4000 tokens, 816 -> 78 for a prompt of 2048; with a window of
-// 128 no slower from nothing (16.9, 17.4) and 57 -> 48 behind 4000.
-constexpr int kPromptRows = 64;
+// 16 latent heads 63 -> 18 and 1305 -> 482.  With a window of 1024 and pooled blocks (16 heads over 4): 21.7 -> 17.6 from
+// nothing, 132 -> 65 behind 4000 tokens, 816 -> 78 for a prompt of 2048; with a window of 128 no slower from nothing (16.9,
+// 17.4) and 57 -> 48 behind 4000.
 bool rows_attention(const sd_seq_layer& l, const sd_seq_batch& b, int H, int G, int dk, int dv, bool latent) {
-  return l.w_in_tiled && sd_aligned16(l.k_cache) && (!l.v_cache || sd_aligned16(l.v_cache)) && b.n_rows - b.n_entries >= kPromptRows && l.window >= 1 &&
+  return l.w_in_tiled && sd_aligned16(l.k_cache) && (!l.v_cache || sd_aligned16(l.v_cache)) && portions(b).many && l.window >= 1 &&
          sd_rows_softmax_attention_fits_(H, G, dk, dv, b.page, latent);
 }
 
@@ -1696,14 +1723,15 @@ int postnorm_layer(const sd_seq_model& m, const sd_seq_layer& l, const sd_seq_ba
     if (dr > 0)
       SQ_TRY(sd_rope_copy_rows(pq, (int64_t)H * dh, dh, dk, qe, (int64_t)H * de, de, rk, b.row_pos, R, H, dr,
                                l.rot_dims, 1, l.inv_freq, l.rot_mag, stream));
-    if (rows_attention(l, b, H, 1, de, rk, true))
-      SQ_TRY(sd_rows_softmax_attention(qe, (int64_t)H * de, l.k_cache, nullptr, b.block_tables, b.max_blocks, b.page, R, H, 1,
-                                       de, rk, l.window, 0, l.score_scale, b.entries, b.n_entries, o, nullptr,
-                                       (int64_t)H * rk, stream));
-    else
-      SQ_TRY(sd_window_softmax_attention(qe, (int64_t)H * de, l.k_cache, nullptr, f32, b.row_pos, b.row_slot,
-                                       b.block_tables, b.max_blocks, b.page, R, H, 1, de, rk, l.window, 0,
-                                       l.score_scale, o, nullptr, base + w.attn, w.attn_bytes, stream));
+    const bool rows = rows_attention(l, b, H, 1, de, rk, true);
+    if (rows)
+      SQ_TRY(sd_rows_softmax_attention_(qe, (int64_t)H * de, l.k_cache, nullptr, b.block_tables, b.max_blocks, b.page, R, H,
+                                        1, de, rk, l.window, 0, l.score_scale, b.entries, b.n_entries, true, o, nullptr,
+                                        (int64_t)H * rk, stream));
+    if (!rows || portions(b).few)
+      SQ_TRY(sd_window_softmax_attention_(qe, (int64_t)H * de, l.k_cache, nullptr, f32, b.row_pos, b.row_slot,
+                                          b.block_tables, b.max_blocks, b.page, R, H, 1, de, rk, l.window, 0, l.score_scale,
+                                          b.entries, b.n_entries, rows, o, nullptr, base + w.attn, w.attn_bytes, stream));
     // a head's value expansion applied to its weighted latent
     SQ_TRY(sd_matmul_rows_batched(o, (int64_t)H * rk, rk, l.w_uv, f32, (int64_t)dv * rk, y, (int64_t)H * dv, dv,
                                   l.w_o_tiled ? yb : nullptr, R, dv, rk, H, stream));
@@ -1716,15 +1744,16 @@ int postnorm_layer(const sd_seq_model& m, const sd_seq_layer& l, const sd_seq_ba
     SQ_TRY(sd_qk_norm_append(proj + c.q, H * dk, l.q_norm_w, proj + c.k, G, dk, l.k_norm_w, proj + c.v, dv, ld, f32, eps,
                              l.k_cache, l.v_cache, b.row_pos, b.row_slot, b.block_tables, b.max_blocks, b.page, R,
                              stream));
-    if (ld % 4 == 0 && c.q % 4 == 0 && rows_attention(l, b, H, G, dk, dv, false))
-      SQ_TRY(sd_rows_softmax_attention(proj + c.q, ld, l.k_cache, l.v_cache, b.block_tables, b.max_blocks, b.page, R, H, G, dk,
-                                       dv, l.window, l.keep_first, l.score_scale, b.entries, b.n_entries, o,
-                                       l.w_o_tiled ? yb : nullptr, (int64_t)H * dv, stream));
-    else
-      SQ_TRY(sd_window_softmax_attention(proj + c.q, ld, l.k_cache, l.v_cache, f32, b.row_pos, b.row_slot,
-                                       b.block_tables, b.max_blocks, b.page, R, H, G, dk, dv, l.window, l.keep_first,
-                                       l.score_scale, o, l.w_o_tiled ? yb : nullptr, base + w.attn, w.attn_bytes,
-                                       stream));
+    const bool rows = ld % 4 == 0 && c.q % 4 == 0 && rows_attention(l, b, H, G, dk, dv, false);
+    if (rows)
+      SQ_TRY(sd_rows_softmax_attention_(proj + c.q, ld, l.k_cache, l.v_cache, b.block_tables, b.max_blocks, b.page, R, H, G,
+                                        dk, dv, l.window, l.keep_first, l.score_scale, b.entries, b.n_entries, true, o,
+                                        l.w_o_tiled ? yb : nullptr, (int64_t)H * dv, stream));
+    if (!rows || portions(b).few)
+      SQ_TRY(sd_window_softmax_attention_(proj + c.q, ld, l.k_cache, l.v_cache, f32, b.row_pos, b.row_slot,
+                                          b.block_tables, b.max_blocks, b.page, R, H, G, dk, dv, l.window, l.keep_first,
+                                          l.score_scale, b.entries, b.n_entries, rows, o, l.w_o_tiled ? yb : nullptr,
+                                          base + w.attn, w.attn_bytes, stream));
     SQ_TRY(seq_linear(l.w_o, l.w_o_tiled, f32, o, nullptr, (int64_t)H * dv, yb, (int64_t)H * dv, nullptr, mix, W, R, W,
                       H * dv, wide_ws, w.wide_bytes, stream));
     // state-space recurrence: convolution + silu over x, B, C; step sizes; scan; gate, group norm
@@ -2241,16 +2270,17 @@ extern "C" int sd_seq_model_forward(sd_seq_model* m, const sd_seq_batch* b, void
       SQ_TRY(sd_head_prep(proj + c.q, proj + c.k, proj + c.v, ld, b->row_pos, b->row_slot, R, H, G, dk, dv,
                           l.rot_dims, l.rot_layout, l.inv_freq, l.qk_unit_norm, d.norm_eps, l.q_scale, l.k_scale,
                           l.k_cache, l.v_cache, f32, b->block_tables, b->max_blocks, b->page, stream));
-      if (ld % 4 == 0 && c.q % 4 == 0 && sd_aligned16(l.pk_cache) && sd_aligned16(l.pv_cache) &&
-          rows_attention(l, *b, H, G, dk, dv, false))
-        SQ_TRY(sd_rows_pool_attention(proj + c.q, ld, l.k_cache, l.v_cache, l.pk_cache, l.pv_cache, b->block_tables,
-                                      b->max_blocks, b->page, R, H, G, dk, dv, l.window, l.pool, l.score_scale,
-                                      l.head_bias, b->entries, b->n_entries, o, stream));
-      else
-        SQ_TRY(sd_window_pool_attention(proj + c.q, ld, l.k_cache, l.v_cache, f32, l.pk_cache, l.pv_cache,
-                                      b->row_pos, b->row_slot, b->block_tables, b->max_blocks, b->page, R, H, G,
-                                      dk, dv, l.window, l.pool, l.score_scale, l.head_bias, o, base + w.attn,
-                                      w.attn_bytes, stream));
+      const bool rows = ld % 4 == 0 && c.q % 4 == 0 && sd_aligned16(l.pk_cache) && sd_aligned16(l.pv_cache) &&
+                        rows_attention(l, *b, H, G, dk, dv, false);
+      if (rows)
+        SQ_TRY(rows_pool_attention(proj + c.q, ld, l.k_cache, l.v_cache, l.pk_cache, l.pv_cache, b->block_tables,
+                                   b->max_blocks, b->page, R, H, G, dk, dv, l.window, l.pool, l.score_scale, l.head_bias,
+                                   b->entries, b->n_entries, true, o, stream));
+      if (!rows || portions(*b).few)
+        SQ_TRY(sd_window_pool_attention_(proj + c.q, ld, l.k_cache, l.v_cache, f32, l.pk_cache, l.pv_cache, b->row_pos,
+                                         b->row_slot, b->block_tables, b->max_blocks, b->page, R, H, G, dk, dv, l.window,
+                                         l.pool, l.score_scale, l.head_bias, b->entries, b->n_entries, rows, o,
+                                         base + w.attn, w.attn_bytes, stream));
       SQ_TRY(sd_head_post(o, proj + c.g, ld, nullptr, f32, 0, d.norm_eps, 1, y, y_b, R, H, dv, rnd, stream));
     } else {
       SQ_TRY(sd_head_prep(proj + c.q, proj + c.k, nullptr, ld, b->row_pos, b->row_slot, R, H, H, dk, dv,

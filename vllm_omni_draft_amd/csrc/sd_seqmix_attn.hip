@@ -36,7 +36,7 @@ struct RowsAttnArgs {
   bf16_t* out_b;
   int64_t ldo;
   float scale;
-  int max_blocks, n_entries, H, G, window, keep_first;
+  int max_blocks, n_entries, H, G, window, keep_first, above;   // above: portions of more rows than this
   // pooled keys and values of whole blocks of `pool` tokens behind the window (f32), `pslots` a page
   const float *pk, *pv, *head_bias;
   int pool, pslots;
@@ -99,7 +99,7 @@ __global__ __launch_bounds__(256, KS > 4 ? 1 : 2) void rows_attn_kernel(RowsAttn
   // the portion and the first token of this group of tokens; the last ones, which see most, first
   int e = 0, first = gridDim.x - 1 - blockIdx.x;
   for (; e < g.n_entries; ++e) {
-    const int n = (g.entries[4 * e + 2] + per - 1) / per;
+    const int rows = g.entries[4 * e + 2], n = rows > g.above ? (rows + per - 1) / per : 0;
     if (first < n) break;
     first -= n;
   }
@@ -507,13 +507,22 @@ extern "C" int sd_rows_softmax_attention(const float* q, int64_t ldq, const void
                                          const int32_t* block_tables, int max_blocks, int page, int n_rows, int H, int G,
                                          int dk, int dv, int window, int keep_first, float scale, const int32_t* entries,
                                          int n_entries, float* out, void* out_b, int64_t ldo, sd_stream_t stream) {
+  return sd_rows_softmax_attention_(q, ldq, k_cache, v_cache, block_tables, max_blocks, page, n_rows, H, G, dk, dv, window,
+                                    keep_first, scale, entries, n_entries, false, out, out_b, ldo, stream);
+}
+
+int sd_rows_softmax_attention_(const float* q, int64_t ldq, const void* k_cache, const void* v_cache,
+                               const int32_t* block_tables, int max_blocks, int page, int n_rows, int H, int G, int dk,
+                               int dv, int window, int keep_first, float scale, const int32_t* entries, int n_entries,
+                               bool long_only, float* out, void* out_b, int64_t ldo, sd_stream_t stream) {
   SD_REQUIRE(q && k_cache && block_tables && entries && (out || out_b) && max_blocks >= 1 && n_rows >= 1 && n_entries >= 1 &&
                  n_rows >= n_entries && H >= 1 && G >= 1 && window >= 1 && keep_first >= 0,
              SD_ERR_INVALID, "sd_rows_softmax_attention: bad argument");
   SD_REQUIRE(sd_rows_softmax_attention_fits_(H, G, dk, dv, page, !v_cache), SD_ERR_UNSUPPORTED,
              "sd_rows_softmax_attention: %d heads over %d of %d / %d channels, pages of %d", H, G, dk, dv, page);
   RowsAttnArgs g{q, ldq, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, entries, out, (bf16_t*)out_b, ldo,
-                 scale, max_blocks, n_entries, H, G, window, keep_first, nullptr, nullptr, nullptr, 1, 0};
+                 scale, max_blocks, n_entries, H, G, window, keep_first, long_only ? kLongPortion : 0, nullptr, nullptr, nullptr,
+                 1, 0};
   SD_REQUIRE(ldq % 4 == 0 && ldo % 4 == 0 && ldq >= (int64_t)H * dk && ldo >= (int64_t)H * dv && sd_aligned16(q) &&
                  sd_aligned16(k_cache) && (!v_cache || sd_aligned16(v_cache)) && (!out || sd_aligned16(out)) &&
                  (!out_b || (reinterpret_cast<uintptr_t>(out_b) & 7) == 0),
@@ -528,10 +537,10 @@ extern "C" int sd_rows_softmax_attention(const float* q, int64_t ldq, const void
 // Window and pooled blocks with sigmoid weights (the means of the rows' own blocks are in the cache already).
 int sd_rows_pool_attention_(const float* q, int64_t ldq, const void* k_cache, const void* v_cache, const float* pk, const float* pv,
                             const int32_t* block_tables, int max_blocks, int n_rows, int H, int G, int window, int pool, int pslots,
-                            float scale, const float* head_bias, const int32_t* entries, int n_entries, float* out,
-                            sd_stream_t stream) {
+                            float scale, const float* head_bias, const int32_t* entries, int n_entries, bool long_only,
+                            float* out, sd_stream_t stream) {
   RowsAttnArgs g{q, ldq, (const bf16_t*)k_cache, (const bf16_t*)v_cache, block_tables, entries, out, nullptr, (int64_t)H * 128,
-                 scale, max_blocks, n_entries, H, G, window, 0, pk, pv, head_bias, pool, pslots};
+                 scale, max_blocks, n_entries, H, G, window, 0, long_only ? kLongPortion : 0, pk, pv, head_bias, pool, pslots};
   SD_REQUIRE(ldq % 4 == 0 && sd_aligned16(q) && sd_aligned16(k_cache) && sd_aligned16(v_cache) && sd_aligned16(pk) &&
                  sd_aligned16(pv) && sd_aligned16(out),
              SD_ERR_INVALID, "sd_rows_pool_attention: rows must be 16-byte aligned");

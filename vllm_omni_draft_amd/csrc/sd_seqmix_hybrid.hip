@@ -239,7 +239,8 @@ __global__ __launch_bounds__(256) void window_softmax_attn_kernel(
     int keep_first, float scale, float* __restrict__ out, bf16_t* __restrict__ out_b, int n_hgroups, int n_splits,
     float* __restrict__ part_acc, float* __restrict__ part_ml, int chunk, float softcap,
     const float* __restrict__ sinks, int maps, const float* __restrict__ dist1, const float* __restrict__ dist2,
-    int64_t ldo, const float* __restrict__ gates, int64_t ldg) {
+    int64_t ldo, const float* __restrict__ gates, int64_t ldg, const int32_t* __restrict__ skip, int n_skip) {
+  if (skip && sd_in_long_portion(skip, n_skip, blockIdx.x)) return;   // (entries whose long portions have another kernel)
   extern __shared__ float lds[];
   constexpr int nthr = 256, nw = 4, PARTS = nthr / KT, KW = KT / 64;
   unsigned long long* vat = reinterpret_cast<unsigned long long*>(lds);  // [KT] cache row of the key
@@ -483,13 +484,14 @@ void launch_softmax_nc(dim3 grid, int kt, size_t lds, hipStream_t st, int nc, co
                        const int32_t* bt, int max_blocks, int page, int H, int G, int dk, int dv, int window,
                        int keep_first, float scale, float* out, bf16_t* out_b, int n_hgroups, int n_splits,
                        float* part_acc, float* part_ml, int chunk, float softcap, const float* sinks, int maps,
-                       const float* dist1, const float* dist2, int64_t ldo, const float* gates, int64_t ldg) {
+                       const float* dist1, const float* dist2, int64_t ldo, const float* gates, int64_t ldg,
+                       const int32_t* skip, int n_skip) {
 #define SD_GO2(NC, KT)                                                                                               \
   window_softmax_attn_kernel<T, NH, NC, KT><<<grid, 256, lds, st>>>(q, ldq, (const T*)kc, (const T*)vc, v_row, row_pos, \
                                                                     row_slot, bt, max_blocks, page, H, G, dk, dv,       \
                                                                     window, keep_first, scale, out, out_b, n_hgroups,   \
                                                                     n_splits, part_acc, part_ml, chunk, softcap, sinks, \
-                                                                    maps, dist1, dist2, ldo, gates, ldg)
+                                                                    maps, dist1, dist2, ldo, gates, ldg, skip, n_skip)
 #define SD_GO(NC)                                          \
   do {                                                     \
     if constexpr (NH <= 4) {                               \
@@ -2201,14 +2203,14 @@ extern "C" int sd_distance_softmax_attention(const float* q, int64_t ldq, const 
                                     scratch_bytes, stream);
 }
 
-extern "C" int sd_gated_softmax_attention(const float* q, int64_t ldq, const void* k_cache, const void* v_cache,
-                                          int cache_f32, const int32_t* row_pos, const int32_t* row_slot,
-                                          const int32_t* block_tables, int max_blocks, int page, int n_rows, int H,
-                                          int G, int maps, int dk, int dv, int window, int keep_first, int chunk,
-                                          float scale, float softcap, const float* sinks, const float* dist1,
-                                          const float* dist2, const float* gates, int64_t ldg, const int32_t* entries,
-                                          int n_entries, float* out, void* out_bf16, int64_t ldo, void* scratch,
-                                          size_t scratch_bytes, sd_stream_t stream) {
+namespace {
+// skip_long: without the rows of long portions
+int gated_attention(const float* q, int64_t ldq, const void* k_cache, const void* v_cache, int cache_f32,
+                    const int32_t* row_pos, const int32_t* row_slot, const int32_t* block_tables, int max_blocks, int page,
+                    int n_rows, int H, int G, int maps, int dk, int dv, int window, int keep_first, int chunk, float scale,
+                    float softcap, const float* sinks, const float* dist1, const float* dist2, const float* gates,
+                    int64_t ldg, const int32_t* entries, int n_entries, bool skip_long, float* out, void* out_bf16,
+                    int64_t ldo, void* scratch, size_t scratch_bytes, sd_stream_t stream) {
   SD_REQUIRE(q && k_cache && row_pos && row_slot && block_tables && (out || out_bf16) && !dist1 == !dist2, SD_ERR_INVALID,
              "sd_masked_softmax_attention: null argument");
   SD_REQUIRE(ldo >= (int64_t)H * maps * dv, SD_ERR_INVALID, "sd_masked_softmax_attention: output rows too short");
@@ -2220,7 +2222,7 @@ extern "C" int sd_gated_softmax_attention(const float* q, int64_t ldq, const voi
   SD_REQUIRE(dv >= 1 && dv <= 512 && (v_cache || dv <= dk), SD_ERR_UNSUPPORTED,
              "sd_masked_softmax_attention: value size %d outside 1..512 (or above the key row it is part of)", dv);
   hipStream_t st = (hipStream_t)stream;
-  if (entries && !cache_f32 && n_rows > kSplitRows && maps == 1 && chunk == 0 && v_cache) {
+  if (entries && !skip_long && !cache_f32 && n_rows > kSplitRows && maps == 1 && chunk == 0 && v_cache) {
     const int rc = sd_tiled_window_attention_(q, ldq, k_cache, v_cache, block_tables, max_blocks, page, n_rows,
                                               H, G, dk, dv, window, keep_first, scale, softcap, sinks, dist1, dist2, gates,
                                               ldg, entries, n_entries, out, out_bf16, ldo, stream);
@@ -2230,7 +2232,8 @@ extern "C" int sd_gated_softmax_attention(const float* q, int64_t ldq, const voi
   const int HM = H * maps;
   const size_t need = sd_multimap_softmax_attention_scratch_bytes(n_rows, H, maps, dv, window, keep_first, chunk,
                                                                   max_blocks * page);
-  const bool split = need > 0 && scratch && scratch_bytes >= need && sd_aligned16(scratch);
+  // (a pass with a long portion has more rows than are ever split)
+  const bool split = !skip_long && need > 0 && scratch && scratch_bytes >= need && sd_aligned16(scratch);
   const int n_splits = split ? (int)(need / ((size_t)n_rows * HM * (dv + 2) * sizeof(float))) : 1;
   const int kt = split ? kSplitKeys : 256;   // keys per tile
   // (a cut launch has many workgroups already: fewer heads each, so that a thread scores its key sooner)
@@ -2251,7 +2254,8 @@ extern "C" int sd_gated_softmax_attention(const float* q, int64_t ldq, const voi
 #define SD_NH(T, N)                                                                                                  \
   launch_softmax_nc<T, N>(grid, kt, lds, st, nc, q, ldq, k_cache, vc, v_row, row_pos, row_slot, block_tables,      \
                           max_blocks, page, H, G, dk, dv, window, keep_first, scale, out, (bf16_t*)out_bf16, n_hgroups, \
-                          n_splits, part_acc, part_ml, chunk, softcap, sinks, maps, dist1, dist2, ldo, gates, ldg)
+                          n_splits, part_acc, part_ml, chunk, softcap, sinks, maps, dist1, dist2, ldo, gates, ldg,        \
+                          skip_long ? entries : nullptr, n_entries)
 #define SD_T(T)                      \
   do {                               \
     if (NH == 1) SD_NH(T, 1);        \
@@ -2271,6 +2275,20 @@ extern "C" int sd_gated_softmax_attention(const float* q, int64_t ldq, const voi
   }
   return SD_OK;
 }
+}  // namespace
+
+extern "C" int sd_gated_softmax_attention(const float* q, int64_t ldq, const void* k_cache, const void* v_cache,
+                                          int cache_f32, const int32_t* row_pos, const int32_t* row_slot,
+                                          const int32_t* block_tables, int max_blocks, int page, int n_rows, int H,
+                                          int G, int maps, int dk, int dv, int window, int keep_first, int chunk,
+                                          float scale, float softcap, const float* sinks, const float* dist1,
+                                          const float* dist2, const float* gates, int64_t ldg, const int32_t* entries,
+                                          int n_entries, float* out, void* out_bf16, int64_t ldo, void* scratch,
+                                          size_t scratch_bytes, sd_stream_t stream) {
+  return gated_attention(q, ldq, k_cache, v_cache, cache_f32, row_pos, row_slot, block_tables, max_blocks, page, n_rows, H, G,
+                         maps, dk, dv, window, keep_first, chunk, scale, softcap, sinks, dist1, dist2, gates, ldg, entries,
+                         n_entries, false, out, out_bf16, ldo, scratch, scratch_bytes, stream);
+}
 
 extern "C" size_t sd_window_softmax_attention_scratch_bytes(int n_rows, int H, int dv, int window, int keep_first,
                                                              int max_ctx) {
@@ -2285,6 +2303,17 @@ extern "C" int sd_window_softmax_attention(const float* q, int64_t ldq, const vo
   return sd_masked_softmax_attention(q, ldq, k_cache, v_cache, cache_f32, row_pos, row_slot, block_tables, max_blocks,
                                      page, n_rows, H, G, dk, dv, window, keep_first, 0, scale, 0.f, nullptr, out,
                                      out_bf16, scratch, scratch_bytes, stream);
+}
+
+int sd_window_softmax_attention_(const float* q, int64_t ldq, const void* k_cache, const void* v_cache, int cache_f32,
+                                 const int32_t* row_pos, const int32_t* row_slot, const int32_t* block_tables,
+                                 int max_blocks, int page, int n_rows, int H, int G, int dk, int dv, int window,
+                                 int keep_first, float scale, const int32_t* entries, int n_entries, bool skip_long,
+                                 float* out, void* out_bf16, void* scratch, size_t scratch_bytes, sd_stream_t stream) {
+  return gated_attention(q, ldq, k_cache, v_cache, cache_f32, row_pos, row_slot, block_tables, max_blocks, page, n_rows, H, G,
+                         1, dk, dv, window, keep_first, 0, scale, 0.f, nullptr, nullptr, nullptr, nullptr, 0,
+                         skip_long ? entries : nullptr, n_entries, skip_long, out, out_bf16, (int64_t)H * dv, scratch,
+                         scratch_bytes, stream);
 }
 
 extern "C" int sd_causal_conv_rows(const float* x, int64_t ldx, const void* w, const void* b, int w_f32,

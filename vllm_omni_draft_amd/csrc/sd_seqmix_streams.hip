@@ -791,7 +791,7 @@ __global__ __launch_bounds__(kChunkThreads, DKP <= 128 ? 4 : 2) void decay_chunk
     if constexpr (MODE != kSums) {
       // A value that is no number stays out of the product with the inner sums, whose zeros would hand it to the tokens
       // before its own; the tokens behind it get it below.
-      auto odd = [](float x) { return !(fabsf(x) < INFINITY); };
+      auto odd = [](float x) -> int { return !(fabsf(x) < INFINITY); };
       const bool some = __any(odd(vv[0]) | odd(vv[1]) | odd(vv[2]) | odd(vv[3]));
       if (some) {
 #pragma unroll
@@ -816,7 +816,7 @@ __global__ __launch_bounds__(kChunkThreads, DKP <= 128 ? 4 : 2) void decay_chunk
           const float x = vs[from * LDV + c];
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            if (odd(x) & (4 * quad + i >= from)) o[i] = fmaf(as[(4 * quad + i) * kTokLd + from], x, o[i]);
+            if (odd(x) & (int)(4 * quad + i >= from)) o[i] = fmaf(as[(4 * quad + i) * kTokLd + from], x, o[i]);
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) vv[i] = vs[(4 * quad + i) * LDV + c];

@@ -75,3 +75,46 @@ def test_packed_prompts_have_the_bits_of_forward_passes(kw):
     assert torch.equal(one.k, two.k) and torch.equal(one.v, two.v)
     with pytest.raises(Exception):
         model.prompt(one, [(1, prompts[0], 0, True)], got)      # no pages for it
+
+
+def _model_and_prompts(lens, max_ctx=600):
+    from vllm_omni_draft_amd import config, weights
+    from vllm_omni_draft_amd.model_runner import DecoderModel
+    cfg = config.create_model_config(None, n_layers=2, hidden=256, n_heads=4, n_kv_heads=2, head_dim=64, ffn=512, vocab=512,
+                                     max_pos=max_ctx)
+    g = torch.Generator().manual_seed(5)
+    return (cfg, DecoderModel(weights.random_init(cfg, seed=3), max_ctx, wide=True),
+            [torch.randint(0, cfg.vocab, (n,), generator=g).tolist() for n in lens])
+
+
+def _cache(cfg, lens, max_ctx=600):
+    from vllm_omni_draft_amd.kv_cache import PagedKVCache
+    kv = PagedKVCache(cfg, PagedKVCache.pages_for(cfg, len(lens), max_ctx), len(lens), max_ctx)
+    for b, n in enumerate(lens):
+        kv.ensure_capacity(b, n)
+    return kv
+
+
+def test_prompts_on_two_streams_with_workspaces_of_their_own():
+    """Nothing of a prompt's size is allocated when it comes (the workspace is there since the model is), and two streams may
+    run prompts of one model at once, each in a workspace of its own."""
+    lens = [500, 460]
+    cfg, model, prompts = _model_and_prompts(lens)
+    kv = _cache(cfg, lens)
+    want = torch.empty(2, cfg.vocab, device="cuda")
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    model.prompt(kv, [(0, prompts[0], 0, True), (1, prompts[1], 0, True)], want)
+    assert torch.cuda.max_memory_allocated() - before < 1 << 17      # (tokens, rows and positions: 16 KiB)
+    kvs, got = [_cache(cfg, lens) for _ in range(2)], [torch.empty(1, cfg.vocab, device="cuda") for _ in range(2)]
+    spaces = [None, torch.empty_like(model.prompt_workspace)]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    for _ in range(4):
+        for i, st in enumerate(streams):
+            with torch.cuda.stream(st):
+                model.prompt(kvs[i], [(i, prompts[i], 0, True)], got[i], workspace=spaces[i])
+    torch.cuda.synchronize()
+    assert torch.equal(torch.cat(got), want)
+    with pytest.raises(Exception, match="workspace"):
+        model.prompt(kv, [(0, prompts[0], 0, True)], want, workspace=spaces[1][:64])

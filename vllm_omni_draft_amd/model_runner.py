@@ -52,7 +52,6 @@ class DecoderModel:
         # the rows of a forward pass, keep to forward() in chunks of prefill_rows.
         self.packs_prompts = (ops.on_gpu() and tp_group is None and bool(wide or wide_prefill)
                               and ops.prompt_attention_fits(max_ctx, split_tokens))
-        self._prompt_ws: Optional[torch.Tensor] = None
         if max_ctx > cfg.max_pos:
             raise ValueError(f"max_ctx {max_ctx} exceeds the model's max_pos {cfg.max_pos}")
         self.max_ctx = max_ctx
@@ -106,6 +105,9 @@ class DecoderModel:
         nbytes = lib.sd_model_workspace_bytes(self._handle, max(self.max_rows, self.prefill_rows),
                                               max_ctx, split_tokens)
         self.workspace = torch.empty(nbytes, dtype=torch.uint8, device=weights.embed.device)
+        # (reserved here, like the other: a prompt must not run out of memory once its pages are taken)
+        nbytes = lib.sd_model_prompt_workspace_bytes(self._handle, PROMPT_ROWS) if self.packs_prompts else 0
+        self.prompt_workspace = torch.empty(nbytes, dtype=torch.uint8, device=weights.embed.device)
         # fused_pairs: passes of <= 4 rows run each layer as attention + sd_chain_o_up +
         # sd_chain_down_qkv (three launches for five, same bits).  Opt-in: on MI355X the five
         # launches are faster (an in-launch exchange costs what a launch boundary costs).
@@ -208,14 +210,19 @@ class DecoderModel:
 
 
     def prompt(self, kv: PagedKVCache, runs, logits: Optional[torch.Tensor] = None,
-               input_embeds: Optional[torch.Tensor] = None, rope_pos: Optional[torch.Tensor] = None) -> None:
+               input_embeds: Optional[torch.Tensor] = None, rope_pos: Optional[torch.Tensor] = None,
+               workspace: Optional[torch.Tensor] = None) -> None:
         """Enqueues prompt tokens on the current stream: runs = [(cache slot, tokens, position of the first, whether
         the last one's logits are wanted)], their rows one behind the other in passes of at most PROMPT_ROWS.  The
         cache must hold pages for every position.  logits (f32 [wanted, head rows]) receives the wanted rows in the
-        order of the runs.  input_embeds [rows, hidden] bf16 and rope_pos [3, rows] int32 as for forward().  A row has
-        the bits that a forward() of the wide family gives it."""
+        order of the runs.  input_embeds [rows, hidden] bf16 and rope_pos [3, rows] int32 as for forward().  workspace:
+        another buffer of the size of self.prompt_workspace, for prompts that run concurrently on several streams.  A
+        row has the bits that a forward() of the wide family gives it."""
         if not self.packs_prompts:
             raise _lib.SdError("this model's prompts go through forward()")
+        ws = self.prompt_workspace if workspace is None else workspace
+        if ws.numel() < self.prompt_workspace.numel() or ws.dtype != torch.uint8:
+            raise _lib.SdError("workspace must be a uint8 tensor of at least self.prompt_workspace's size")
         runs = [(int(slot), np.asarray(toks, dtype=np.int32), int(pos), bool(want)) for slot, toks, pos, want in runs]
         total = sum(len(t) for _, t, _, _ in runs)
         wanted = sum(w for _, _, _, w in runs)
@@ -256,9 +263,6 @@ class DecoderModel:
             host = np.concatenate([np.asarray(items, np.int32).reshape(-1), *toks, *seq, *pos,
                                    np.asarray(out_rows, np.int32)])
             dev = torch.from_numpy(host).to(kv.block_tables.device)
-            need = int(_lib.load().sd_model_prompt_workspace_bytes(self._handle, rows))
-            if self._prompt_ws is None or self._prompt_ws.numel() < need:
-                self._prompt_ws = torch.empty(need, dtype=torch.uint8, device=dev.device)
             o, rp = 4 * len(items), None if rope_pos is None else rope_pos[:, done:done + rows].contiguous()
             kvd = _lib.KvCacheDesc(k_cache=kv.k.data_ptr(), v_cache=kv.v.data_ptr(),
                                    layer_stride_bytes=kv.layer_stride_bytes, block_tables=kv.block_tables.data_ptr(),
@@ -272,7 +276,7 @@ class DecoderModel:
                 wide_a8=int(self.fp8_activations), max_ctx=max(i[3] + i[1] for i in items),
                 split_tokens=self.split_tokens)
             _lib.check(_lib.load().sd_model_prompt(self._handle, C.byref(kvd), C.byref(args),
-                                                   self._prompt_ws.data_ptr(), self._prompt_ws.numel(), ops._stream()),
+                                                   ws.data_ptr(), ws.numel(), ops._stream()),
                        "sd_model_prompt")
             done += rows
             out_at += len(out_rows)

@@ -118,3 +118,18 @@ def test_prompts_on_two_streams_with_workspaces_of_their_own():
     assert torch.equal(torch.cat(got), want)
     with pytest.raises(Exception, match="workspace"):
         model.prompt(kv, [(0, prompts[0], 0, True)], want, workspace=spaces[1][:64])
+
+
+@pytest.mark.parametrize("where", ["cpu", "cuda"])
+def test_prompts_given_as_tensors(where):
+    """A prompt may be a tensor on any device, as well as a list of numbers: the same first token."""
+    from vllm_omni_draft_amd import config, weights
+    from vllm_omni_draft_amd.engine import EngineConfig, SpecEngine
+    cfg = config.create_model_config(None, n_layers=1, hidden=128, n_heads=2, n_kv_heads=1, head_dim=64, ffn=128, vocab=128, max_pos=256)
+    w = weights.random_init(cfg, seed=3)
+    prompts = [list(range(3, 60)), [5, 9, 11]]
+    tensors = [torch.tensor(p, device=where) for p in prompts]
+    first = lambda ps: SpecEngine(w, None, EngineConfig(k=0, max_seq_len=128, max_batch=2)).add_requests(ps)
+    want = first(prompts)
+    assert first(tensors) == want
+    assert SpecEngine(w, None, EngineConfig(k=0, max_seq_len=128)).add_request(0, tensors[0]) == want[0]

@@ -28,6 +28,15 @@ def _ptr(t):
     return t.data.data_ptr() if hasattr(t, "mode") else t.data_ptr()
 
 
+def _token_ids(toks) -> np.ndarray:
+    """Token ids as int32: of numbers, of a tensor or of tensors of one element, on any device."""
+    if isinstance(toks, torch.Tensor):
+        toks = toks.cpu()
+    elif len(toks) and isinstance(toks[0], torch.Tensor):
+        toks = [int(t) for t in toks]
+    return np.asarray(toks, dtype=np.int32)
+
+
 class DecoderModel:
     def __init__(self, weights: ModelWeights, max_ctx: int, split_tokens: int = 256,
                  tp_group=None, wide: bool = False, wide_prefill: bool = True,
@@ -223,7 +232,7 @@ class DecoderModel:
         ws = self.prompt_workspace if workspace is None else workspace
         if ws.numel() < self.prompt_workspace.numel() or ws.dtype != torch.uint8:
             raise _lib.SdError("workspace must be a uint8 tensor of at least self.prompt_workspace's size")
-        runs = [(int(slot), np.asarray(toks, dtype=np.int32), int(pos), bool(want)) for slot, toks, pos, want in runs]
+        runs = [(int(slot), _token_ids(toks), int(pos), bool(want)) for slot, toks, pos, want in runs]
         total = sum(len(t) for _, t, _, _ in runs)
         wanted = sum(w for _, _, _, w in runs)
         if any(len(t) < 1 or pos < 0 or pos + len(t) > self.max_ctx or not 0 <= slot < kv.block_tables.shape[0]

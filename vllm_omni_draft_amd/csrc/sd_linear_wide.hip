@@ -16,7 +16,8 @@
 // (sd_rows_linear_fits_ says which, and by how much it is faster).
 //
 // wide_gemm4_kernel (further down) serves the many-row passes of some matrices with another
-// chunk structure on four waves; same tiles, same sums, same bits.
+// chunk structure on four waves (fp8 weights; bf16 where sd_prompt.hip's kernel does not take the epilogue); same
+// tiles, same sums, same bits.
 //
 // Matrices with few tiles split K over several workgroups.  Partial sums go to a workspace
 // as f32 [split][row][tile row] and wide_epilogue_kernel adds the splits in index order and
@@ -825,13 +826,26 @@ int launch_gemm4_w(const WideArgs& a, int S, hipStream_t st) {
   return SD_OK;
 }
 
+// Whether bf16 weights come to the four-wave kernel with this epilogue: sd_rows_linear_fits_ takes every gated projection
+// and every f32 output of the matrices that it would be chosen for (one round of blocks at 33 rows and more; any number
+// of rounds above 192 rows).
+#if defined(SD_WIDE_EXP)
+template <int EPI>
+constexpr bool kBf16Four = true;
+#else
+template <int EPI>
+constexpr bool kBf16Four = EPI != SD_EPI_SILU_MUL && EPI != SD_EPI_F32;
+#endif
+
 template <int MT, int EPI, int TPW, int WAVES>
 int launch_gemm4(const WideArgs& a, int S, hipStream_t st) {
-#if defined(SD_WIDE_EXP) || defined(SD_WIDE_F32_ONLY)
+#if defined(SD_WIDE_EXP)
   return launch_gemm4_w<MT, EPI, TPW, false, WAVES>(a, S, st);
 #else
-  return a.epi.w_scale ? launch_gemm4_w<MT, EPI, TPW, true, WAVES>(a, S, st)
-                       : launch_gemm4_w<MT, EPI, TPW, false, WAVES>(a, S, st);
+  if (a.epi.w_scale) return launch_gemm4_w<MT, EPI, TPW, true, WAVES>(a, S, st);
+  if constexpr (kBf16Four<EPI>) return launch_gemm4_w<MT, EPI, TPW, false, WAVES>(a, S, st);
+  sd_set_error("sd_linear_wide: epilogue %d", EPI);   // (launch_gemm does not ask for it)
+  return SD_ERR_UNSUPPORTED;
 #endif
 }
 
@@ -848,13 +862,18 @@ int launch_gemm(const WideArgs& a, int S, hipStream_t st) {
 #endif
   // The four-wave kernel where it was measured faster (same bits either way): many rows,
   // 8-tile groups that cover the whole of K with the epilogue inside (the matrices of
-  // 1024..2047 tiles: a gated projection of 8192..16383 outputs, say), an even number of whole
+  // 1024..2047 tiles: a gated projection of 8192..16383 outputs in fp8, say), an even number of whole
   // chunks.  Split-K groups run a handful of chunks each and gain nothing; 16-tile groups
   // would need four tiles per wave and every register there is.
+#ifdef SD_WIDE_F32_ONLY
+  constexpr bool kHasFour = false;   // (no fp8 weights, and see kBf16Four)
+#else
   constexpr bool kHasFour = MT >= kFourWaveMT && EPI != EPI_PARTIAL && EPI != SD_EPI_RELU &&
                             EPI != SD_EPI_GELU_TANH;
+#endif
   if constexpr (kHasFour) {
-    bool four = !pair && S == 1 && a.K % (2 * kChunkCols) == 0;
+    const bool has = a.epi.w_scale || kBf16Four<EPI>;
+    bool four = has && !pair && S == 1 && a.K % (2 * kChunkCols) == 0;
 #ifdef SD_WIDE_HAS_SWITCH
     if (g_wide_four_waves >= 0) four = four && g_wide_four_waves != 0;
 #endif
@@ -862,7 +881,7 @@ int launch_gemm(const WideArgs& a, int S, hipStream_t st) {
     // 16-tile groups at 256 rows: the eight-wave kernel needs more registers than a wave of
     // eight has (it spills); the same tiles in 8-tile groups on four waves, in more rounds.
     if constexpr (MT == 16) {
-      bool split_pairs = pair && S == 1 && a.K % (2 * kChunkCols) == 0;
+      bool split_pairs = has && pair && S == 1 && a.K % (2 * kChunkCols) == 0;
 #ifdef SD_WIDE_HAS_SWITCH
       if (g_wide_four_waves >= 0) split_pairs = split_pairs && g_wide_four_waves != 0;
 #endif
@@ -1006,12 +1025,10 @@ int wide_common(const void* W, const void* x, int64_t ldx, int M, int K, int n_t
   e.NR = n_tiles * 16;
   a.epi = e;
   const int mt = (M + 15) / 16;
-#ifndef SD_WIDE_F32_ONLY
   if (!e.w_scale && sd_rows_linear_fits_(M, n_tiles, K, ldx, S, ksp, epi)) {  // (the same bits)
     const int rc = sd_rows_linear_(W, x, ldx, M, K, n_tiles, S, ksp, epi, e, (float*)workspace, st);
     return rc != SD_OK || S == 1 ? rc : epilogue_by_kind(e, epi, st);
   }
-#endif
   if (S == 1) return gemm_by_rows<true>(a, mt, epi, S, st);
   const int rc = gemm_by_rows<false>(a, mt, epi, S, st);
   if (rc != SD_OK) return rc;

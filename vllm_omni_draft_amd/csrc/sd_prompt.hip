@@ -6,11 +6,13 @@
 // S x rows x N floats written and read back) and left most of the matrix pipe idle (640 TFLOP/s on the split
 // matrices of an 8B model without their second launch, 880 on gate/up).  With hundreds of rows the op is bound
 // by the matrix pipe and by what feeds it.  Here both operands of a block pass through LDS by direct loads
-// (16 bytes a lane, no registers), 64 columns a stage, two stages; four waves, each with its own TN x TM tiles
+// (16 bytes a lane, no registers), 64 columns a stage, two to four stages; four waves, each with its own TN x TM tiles
 // of 16 x 16 in registers, so a fragment read from LDS feeds TM (or TN) MFMAs:
-//   8 x 8 tiles a wave (256 x 256 a block): 64 B of LDS reads a clock against 128, one wave a SIMD, every
+//   8 x 8 tiles a wave (256 x 256 a block), two stages: 64 B of LDS reads a clock against 128, one wave a SIMD, every
 //     accumulator register there is;
-//   4 x 4 (128 x 128): two blocks a CU, and room for a second set of sums.
+//   4 x 4 (128 x 128), two stages: two blocks a CU, and room for a second set of sums; four stages where there is at most
+//     one block a CU, whose loads nothing else covers;
+//   2, 4 or 5 x 2, 4, 6 or 8 (all rows of a pass of 33..256), three stages: what is left is the weights' way from memory.
 // The second set is for matrices whose K the narrower kernels split: a row's bits must not depend on how many
 // rows share its pass, so the sums of a split are chained in one accumulator, and the splits' sums are added in
 // index order from zero, as wide_epilogue_kernel adds them; in registers, without a second launch.

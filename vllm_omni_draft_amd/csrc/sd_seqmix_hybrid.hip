@@ -1316,11 +1316,11 @@ __device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// act[a, n] (bf16) = silu(s * gate) * (s * up); a wave owns 32 columns of gate and of up.  Xb (or
-// nullptr): the rows of X as bf16 already.
+// act[a, n] (bf16) = silu(s * gate) * (s * up); a wave owns 32 columns of gate and of up.  (Rows that are there as bf16
+// too take moe_rows_kernel but for buffers beyond its offsets.)
 template <int MT, int KC, bool GATED>
 __global__ __launch_bounds__(256) void moe_gate_up_mfma_kernel(
-    const float* __restrict__ X, const bf16_t* __restrict__ Xb, int64_t ldx, const int32_t* __restrict__ perm,
+    const float* __restrict__ X, int64_t ldx, const int32_t* __restrict__ perm,
     const int32_t* __restrict__ tiles, const int32_t* __restrict__ n_tiles, const float* __restrict__ sel_w,
     const bf16_t* __restrict__ Wgu, bf16_t* __restrict__ act, int top, int E, int F, int K, int scale_input, int act_kind,
     float limit) {
@@ -1347,25 +1347,15 @@ __global__ __launch_bounds__(256) void moe_gate_up_mfma_kernel(
   for (int kc0 = 0; kc0 < K; kc0 += KC) {
     const int kc = K - kc0 < KC ? K - kc0 : KC;
     __syncthreads();
-    if (Xb) {
-      for (int idx = tid; idx < 16 * m_tiles * (kc / 8); idx += 256) {
-        const int m = idx / (kc / 8), k8 = (idx % (kc / 8)) * 8;
-        const int a = arow[m];
-        bf16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
-        if (a >= 0) v = *reinterpret_cast<const bf16x8*>(Xb + (size_t)(a / top) * ldx + kc0 + k8);
-        *reinterpret_cast<bf16x8*>(xs + m * LD + k8) = v;
+    for (int idx = tid; idx < 16 * m_tiles * (kc / 4); idx += 256) {
+      const int m = idx / (kc / 4), k4 = (idx % (kc / 4)) * 4;
+      const int a = arow[m];
+      bf16x4 v = {0, 0, 0, 0};
+      if (a >= 0) {
+        const f32x4 xv = *reinterpret_cast<const f32x4*>(X + (size_t)(a / top) * ldx + kc0 + k4);
+        v = bf16x4{(bf16_t)xv[0], (bf16_t)xv[1], (bf16_t)xv[2], (bf16_t)xv[3]};
       }
-    } else {
-      for (int idx = tid; idx < 16 * m_tiles * (kc / 4); idx += 256) {
-        const int m = idx / (kc / 4), k4 = (idx % (kc / 4)) * 4;
-        const int a = arow[m];
-        bf16x4 v = {0, 0, 0, 0};
-        if (a >= 0) {
-          const f32x4 xv = *reinterpret_cast<const f32x4*>(X + (size_t)(a / top) * ldx + kc0 + k4);
-          v = bf16x4{(bf16_t)xv[0], (bf16_t)xv[1], (bf16_t)xv[2], (bf16_t)xv[3]};
-        }
-        *reinterpret_cast<bf16x4*>(xs + m * LD + k4) = v;
-      }
+      *reinterpret_cast<bf16x4*>(xs + m * LD + k4) = v;
     }
     __syncthreads();
 #pragma unroll(KC / 32 <= 4 ? KC / 32 : 4)
@@ -2547,12 +2537,11 @@ extern "C" int sd_moe_experts_clamped(const float* x, const void* x_bf16, int64_
     // (act holds n * F floats: its first half serves as the bf16 activations)
     bf16_t* act_b = (bf16_t*)act;
     const dim3 g1((F + 127) / 128, tiles_y), g2((W + 127) / 128, tiles_y);
-    const bf16_t* xb = (const bf16_t*)x_bf16;
     if (act_kind != 1)
-      moe_gate_up_mfma_kernel<2, 512, true><<<g1, 256, 0, st>>>(x, xb, ldx, perm, tiles, n_tiles, sel_weight,
+      moe_gate_up_mfma_kernel<2, 512, true><<<g1, 256, 0, st>>>(x, ldx, perm, tiles, n_tiles, sel_weight,
                                                                 (const bf16_t*)w_gate_up, act_b, top, E, F, W, scale_input, act_kind, limit);
     else
-      moe_gate_up_mfma_kernel<2, 512, false><<<g1, 256, 0, st>>>(x, xb, ldx, perm, tiles, n_tiles, sel_weight,
+      moe_gate_up_mfma_kernel<2, 512, false><<<g1, 256, 0, st>>>(x, ldx, perm, tiles, n_tiles, sel_weight,
                                                                  (const bf16_t*)w_gate_up, act_b, top, E, F, W, scale_input, act_kind, limit);
     SD_CHECK_LAUNCH("sd_moe_experts (gate, up)");
     moe_down_mfma_kernel<2, 512><<<g2, 256, 0, st>>>(act_b, perm, tiles, n_tiles, sel_weight, (const bf16_t*)w_down,

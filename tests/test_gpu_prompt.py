@@ -133,3 +133,69 @@ def test_prompts_given_as_tensors(where):
     want = first(prompts)
     assert first(tensors) == want
     assert SpecEngine(w, None, EngineConfig(k=0, max_seq_len=128)).add_request(0, tensors[0]) == want[0]
+
+
+@pytest.mark.parametrize("D,split,first", [(64, 128, 16400), (128, 128, 22400), (64, 256, 16384), (128, 256, 33000), (128, 256, 44900)])
+def test_prompt_attention_at_positions_beyond_its_page_table(D, split, first):
+    """Contexts of more pages than the kernel's table holds at a time (1024: it is filled again in the middle of a sweep and
+    at the second sweep's start), up to the longest that it takes, pages in any order: the bits of paged attention."""
+    from vllm_omni_draft_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(first + D)
+    Hq, n = 2, 70
+    pages = (first + n + 15) // 16
+    assert ops.prompt_attention_fits(first + n, split)
+    kc, vc = (torch.randn(pages, 1, 16 * D, generator=g, device="cuda").to(torch.bfloat16) for _ in range(2))
+    bt = torch.randperm(pages, generator=g, device="cuda").to(torch.int32).view(1, pages)
+    q = (torch.randn(n, Hq * D, generator=g, device="cuda") * 3).to(torch.bfloat16)
+    lens = torch.tensor([first], dtype=torch.int32, device="cuda")
+    ref = ops.paged_attention_blocked(q, kc, vc, bt, lens, 0, 1, n, 32, Hq, 1, D, D ** -0.5, max_ctx=pages * 16, split_tokens=split)
+    items = torch.tensor([[0, 64, 0, first], [64, n - 64, 0, first + 64]], dtype=torch.int32, device="cuda")
+    got = ops.prompt_attention(q, kc, vc, bt, items, Hq, 1, D, D ** -0.5, first + n, split)
+    assert torch.equal(got, ref.view(n, Hq * D))
+
+
+@pytest.mark.parametrize("mrope", [False, True])
+def test_prompts_of_several_passes(mrope):
+    """More rows than a pass takes (4096: a prompt is cut between two), wanted rows in every pass, embeddings and rotary
+    positions given for all rows: each prompt's logits and caches as by forward passes of its own."""
+    from vllm_omni_draft_amd import config, weights
+    from vllm_omni_draft_amd.engine import _KvView
+    from vllm_omni_draft_amd.model_runner import PROMPT_ROWS, DecoderModel
+    cfg = config.create_model_config(None, n_layers=1, hidden=128, n_heads=2, n_kv_heads=1, head_dim=64, ffn=128, vocab=128, max_pos=6000,
+                                     **({"mrope_section": (8, 12, 12)} if mrope else {}))
+    model = DecoderModel(weights.random_init(cfg, seed=3), 6000, wide=True)
+    lens = [PROMPT_ROWS - 300, 5, 700, 4100]
+    g = torch.Generator().manual_seed(5)
+    prompts = [torch.randint(0, cfg.vocab, (n,), generator=g).tolist() for n in lens]
+    total = sum(lens)
+    embeds = torch.randn(total, cfg.hidden, generator=g).to(torch.bfloat16).cuda() if mrope else None
+    pos = torch.randint(0, 5000, (3, total), generator=g).to(torch.int32).cuda() if mrope else None
+    one, two = _cache(cfg, lens, 6000), _cache(cfg, lens, 6000)
+    got = torch.empty(3, cfg.vocab, device="cuda")
+    want_of = [True, False, True, True]
+    model.prompt(one, [(b, p, 0, want_of[b]) for b, p in enumerate(prompts)], got, embeds, pos)
+    zero = torch.zeros(1, dtype=torch.int32, device="cuda")
+    at, wanted = 0, []
+    for b, n in enumerate(lens):
+        t = torch.tensor(prompts[b], dtype=torch.int32, device="cuda")
+        for c in range(0, n, 256):
+            m = min(256, n - c)
+            out = torch.empty(m, cfg.vocab, device="cuda")
+            kw = dict(input_embeds=embeds[at + c:at + c + m].contiguous(), rope_pos=pos[:, at + c:at + c + m].contiguous()) if mrope else {}
+            model.forward(_KvView(two, b), t, 0, c, zero, c, 1, m, out, wide=True, **kw)
+        if want_of[b]:
+            wanted.append(out[-1])
+        at += n
+    assert torch.equal(got, torch.stack(wanted)) and torch.equal(one.k, two.k) and torch.equal(one.v, two.v)
+
+
+def test_more_wanted_rows_than_a_pass_gives():
+    """300 prompts, the last row of each wanted (a pass gives 256 rows of logits)."""
+    lens = [1 + i % 3 for i in range(300)]
+    cfg, model, prompts = _model_and_prompts(lens, 64)
+    kv, got = _cache(cfg, lens, 64), torch.empty(300, 512, device="cuda")
+    model.prompt(kv, [(b, p, 0, True) for b, p in enumerate(prompts)], got)
+    few = torch.empty(300, 512, device="cuda")
+    for b in range(0, 300, 100):
+        model.prompt(kv, [(b + i, p, 0, True) for i, p in enumerate(prompts[b:b + 100])], few[b:b + 100])
+    assert torch.equal(got, few)

@@ -1674,10 +1674,10 @@ Portions portions(const sd_seq_batch& b) {
 // Attention on the matrix cores for long portions (as for the chunked recurrences: of models whose linear layers sum few
 // and many rows in different orders anyway; portions of up to kLongPortion rows keep the kernel on the vector pipe, in the
 // same pass too).
-// 64 rows of one portion: 16 heads over 4 of 128 channels 14.8 -> 13.3 us from nothing, 362 -> 143 behind 4000 tokens;
-// 16 latent heads 63 -> 18 and 1305 -> 482.  With a window of 1024 and pooled blocks (16 heads over 4): 21.7 -> 17.6 from
-// nothing, 132 -> 65 behind 4000 tokens, 816 -> 78 for a prompt of 2048; with a window of 128 no slower from nothing (16.9,
-// 17.4) and 57 -> 48 behind 4000.
+// 65 rows of one portion: 16 heads over 4 of 128 channels 14.8 -> 14.0 us from nothing, 362 -> 137 behind 4000 tokens;
+// 16 latent heads 63 -> 22 and 1305 -> 480.  With a window of 1024 and pooled blocks (16 heads over 4): 21.7 -> 17.1 from
+// nothing, 132 -> 73 behind 4000 tokens, 816 -> 87 for a prompt of 2048; with a window of 128 no slower from nothing (16.9,
+// 17.3) and 57 -> 51 behind 4000.
 bool rows_attention(const sd_seq_layer& l, const sd_seq_batch& b, int H, int G, int dk, int dv, bool latent) {
   return l.w_in_tiled && sd_aligned16(l.k_cache) && (!l.v_cache || sd_aligned16(l.v_cache)) && portions(b).many && l.window >= 1 &&
          sd_rows_softmax_attention_fits_(H, G, dk, dv, b.page, latent);

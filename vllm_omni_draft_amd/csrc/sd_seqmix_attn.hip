@@ -13,11 +13,11 @@
 // column, as they are the right operand of O^T = V^T P^T; V^T comes out of the row-major tile by the transposing LDS
 // read (a group of 16 lanes reads 4 keys x 16 channels, a lane receives 4 keys of one channel).
 // Bound by the matrix pipe and the exponentials between its parts (one wave a SIMD for latent rows, whose queries and
-// sums fill the registers): 1024 rows of 16 latent heads (576 / 512 channels) 972 -> 133 us, 1024 rows of 16 heads over 4
-// of 128 channels 344 -> 42 us.
-// 2048 rows of 16 heads over 4 with a window of 1024 and pooled blocks 789 -> 73 us.
+// sums fill the registers): 1024 rows of 16 latent heads (576 / 512 channels) 972 -> 135 us, 1024 rows of 16 heads over 4
+// of 128 channels 344 -> 40 us, 2048 rows of 16 heads over 4 with a window of 1024 and pooled blocks 816 -> 87 us.
 // A weight of 0 does not clear a value that is no number: in the stages that not all rows of a workgroup see whole, such
-// values become 0 as they arrive, and the rows that see them get them added (add_odd).
+// values become 0 as they arrive (clear_odd: 1-5 %, 10 % of 65 pooled rows behind 4000 tokens), and the rows that see them
+// get them added (add_odd).  Scores that are no numbers: see redo_query.
 #include <math.h>
 #include <type_traits>
 
@@ -46,6 +46,8 @@ typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(1))) const void global_void;
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+template <int N>
+using Number = std::integral_constant<int, N>;
 constexpr int kPage = 16, kKeys = 64, kRowsPerBlock = 64, kPooled = 32;
 
 // Two f32 values as three pairs of bf16 whose sums they are: 8 bits of the significand each, cut off (the differences
@@ -62,7 +64,7 @@ __device__ __forceinline__ void three_parts(float x, float y, unsigned& a, unsig
 }
 
 // e^x for x <= 0 (-inf: 0), to about one unit in the last place: the product with log2 e in two parts, no branch.
-// (The limits here and below let a NaN through, as fmaxf would not: one instruction either way.)
+// (The limit lets a NaN through, as fmaxf would not: one instruction either way.)
 __device__ __forceinline__ float exp_neg(float x) {
   x = __builtin_elementwise_maximum(x, -200.f);   // (e^-200 is 0 in f32)
   const float hi = x * 1.44269502f;
@@ -71,9 +73,9 @@ __device__ __forceinline__ float exp_neg(float x) {
   return fmaf(y, lo * 0.693147181f, y);
 }
 
-// 1 / (1 + e^-x), to about two units in the last place (below e^-87: 0 or next to it; +inf: 1)
+// 1 / (1 + e^-x) of a finite x, to about two units in the last place (below e^-87: 0 or next to it)
 __device__ __forceinline__ float sigmoid_of(float x) {
-  x = -__builtin_elementwise_minimum(__builtin_elementwise_maximum(x, -87.f), 87.f);
+  x = -fmaxf(x, -87.f);
   const float hi = x * 1.44269502f;
   const float lo = fmaf(x, 1.92596300e-8f, fmaf(x, 1.44269502f, -hi));
   const float y = __builtin_amdgcn_exp2f(hi);
@@ -196,7 +198,9 @@ __global__ __launch_bounds__(256, KS > 4 ? 1 : 2) void rows_attn_kernel(RowsAttn
   f32x4 o[VT];
 #pragma unroll
   for (int v = 0; v < VT; ++v) o[v] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m_run = -INFINITY, l_run = 0.f;                      // (a query's sum is spread over its four lanes)
+  // (a query's sum is spread over its four lanes; the largest score, pooled: the largest absolute value, is NaN once one
+  // was no number)
+  float m_run = POOLED ? 0.f : -INFINITY, l_run = 0.f;
   const int k_off = col * DK * 2;
   const int k_sw[2] = {(quad ^ (col & 7)) << 4, ((quad + 4) ^ (col & 7)) << 4};
   constexpr int kVRow = (LATENT ? DK : DV) * 2;
@@ -235,6 +239,7 @@ __global__ __launch_bounds__(256, KS > 4 ? 1 : 2) void rows_attn_kernel(RowsAttn
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const int r = 16 * u + 4 * qd + i;
+        m_run = __builtin_elementwise_maximum(m_run, fabsf(sc[u][i]));
         const float wt = sigmoid_of(sc[u][i] + bias);
         sc[u][i] = st * kPooled + r < my_blocks ? wt : 0.f;
       }
@@ -249,24 +254,6 @@ __global__ __launch_bounds__(256, KS > 4 ? 1 : 2) void rows_attn_kernel(RowsAttn
           o[v] = __builtin_amdgcn_mfma_f32_16x16x4f32(*reinterpret_cast<const float*>(at + (((4 * v + (cl >> 2)) ^ (r & 7)) << 4)),
                                                       sc[u][i], o[v], 0, 0, 0);
       }
-  };
-  // The scores again, term by term: a part of a query that is 0 makes a NaN of an infinite key, where the query's product
-  // with it is infinite and its weight a number.
-  auto plain_scores = [&](const char* s, f32x4 (&sc)[4]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) sc[u] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-    for (int c = 0; c < DK; ++c) {
-      const float x = qr[c] * g.scale;
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int r = 4 * quad + i;
-          const char* at = s + u * kKeyPage + r * DK * 2 + (c >> 6) * 128 + ((((c >> 3) & 7) ^ (r & 7)) << 4) + (c & 7) * 2;
-          sc[u][i] = fmaf(x, (float)*reinterpret_cast<const bf16_t*>(at), sc[u][i]);
-        }
-    }
   };
   auto attend = [&](const char* s, int st) __attribute__((always_inline)) {
     const int base = stage_base(st);
@@ -296,67 +283,41 @@ __global__ __launch_bounds__(256, KS > 4 ? 1 : 2) void rows_attn_kernel(RowsAttn
 #pragma unroll
         for (int u = 0; u < 4; ++u) sc[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], y[c], sc[u], 0, 0, 0);
     }
-    // The weights of a stage's scores in their place: the new maximum, the factor of what has been summed, the sum of the
-    // weights (a query's is spread over its four lanes; pooled: only whether it is a number matters)
-    auto weigh = [&](f32x4 (&x)[4], float& mx, float& corr) __attribute__((always_inline)) {
-      float sum = 0.f;
-      mx = m_run;
-      if constexpr (POOLED) {
+    if constexpr (POOLED) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+      for (int u = 0; u < 4; ++u)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int d = p - (base + 16 * u + 4 * quad + i);
-            const float wt = sigmoid_of(x[u][i] + bias);
-            x[u][i] = ((d >= 0) & (d < g.window)) ? wt : 0.f;
-            sum += x[u][i];
-          }
-      } else {
+        for (int i = 0; i < 4; ++i) {
+          const int d = p - (base + 16 * u + 4 * quad + i);
+          m_run = __builtin_elementwise_maximum(m_run, fabsf(sc[u][i]));
+          const float wt = sigmoid_of(sc[u][i] + bias);
+          sc[u][i] = ((d >= 0) & (d < g.window)) ? wt : 0.f;
+        }
+    } else {
+      float mx = m_run;
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+      for (int u = 0; u < 4; ++u)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const int j = base + 16 * u + 4 * quad + i, d = p - j;
-            // (bitwise: a chain of && would become branches)
-            const bool seen = (d >= 0) & ((d < g.window) | (j < g.keep_first)) & (j < key_end);
-            x[u][i] = seen ? x[u][i] : -INFINITY;
-            mx = fmaxf(mx, x[u][i]);
-          }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, SD_WAVE));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, SD_WAVE));
-        const float ref = mx == -INFINITY ? 0.f : mx;            // (no key seen yet)
-        corr = exp_neg(m_run - ref);   // (nothing summed yet: 0)
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            x[u][i] = exp_neg(x[u][i] - ref);
-            sum += x[u][i];
-          }
-      }
-      return sum;
-    };
-    float mx, corr = 1.f, sum = weigh(sc, mx, corr);
-    if constexpr (!LATENT) {   // (an infinite channel of a latent row is an infinite value too)
-      if (__any(sum != sum)) {   // of such queries only
-        f32x4 again[4];
-        float mx2, corr2 = 1.f;
-        plain_scores(s, again);
-        const float sum2 = weigh(again, mx2, corr2);
-        int redo = sum != sum;
-        redo |= __shfl_xor(redo, 16, SD_WAVE);
-        redo |= __shfl_xor(redo, 32, SD_WAVE);
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) sc[u][i] = redo ? again[u][i] : sc[u][i];
-        mx = redo ? mx2 : mx;
-        corr = redo ? corr2 : corr;
-        sum = redo ? sum2 : sum;
-      }
-    }
-    if constexpr (!POOLED) {
+        for (int i = 0; i < 4; ++i) {
+          const int j = base + 16 * u + 4 * quad + i, d = p - j;
+          // (bitwise: a chain of && would become branches)
+          const bool seen = (d >= 0) & ((d < g.window) | (j < g.keep_first)) & (j < key_end);
+          sc[u][i] = seen ? sc[u][i] : -INFINITY;
+          mx = __builtin_elementwise_maximum(mx, sc[u][i]);
+        }
+      mx = __builtin_elementwise_maximum(mx, __shfl_xor(mx, 16, SD_WAVE));
+      mx = __builtin_elementwise_maximum(mx, __shfl_xor(mx, 32, SD_WAVE));
+      const float ref = mx == -INFINITY ? 0.f : mx;            // (no key seen yet)
+      const float corr = exp_neg(m_run - ref);   // (nothing summed yet: 0)
       m_run = mx;
+      float sum = 0.f;
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          sc[u][i] = exp_neg(sc[u][i] - ref);
+          sum += sc[u][i];
+        }
       l_run = fmaf(l_run, corr, sum);
       if (__any(corr != 1.f)) {
 #pragma unroll
@@ -388,35 +349,42 @@ __global__ __launch_bounds__(256, KS > 4 ? 1 : 2) void rows_attn_kernel(RowsAttn
           for (int w = 0; w < 2; ++w) o[v + w] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[w], pw[u][c], o[v + w], 0, 0, 0);
       }
   };
-  // whether some row of the workgroup does not see all of stage st
+  // Whether some row of the workgroup does not see all of stage st: the last of the kept stages' pooled blocks, and the
+  // window's first and last stages
+  const int kept_mixed = POOLED ? blocks_of(pos0) / kPooled : kept_stages;
   auto mixed = [&](int st) {
-    if (st < kept_stages) return POOLED && (st + 1) * kPooled > blocks_of(pos0);
-    return stage_base(st) + kKeys - 1 > pos0 || stage_base(st) <= last - g.window;
+    if (st < kept_stages) return st >= kept_mixed;
+    const int base = stage_base(st);
+    return base + kKeys - 1 > pos0 || base <= last - g.window;
   };
-  // This wave's rows of a stage's values, once they are in LDS: what is no number becomes 0.  Returns the rows.
-  auto clear_odd = [&](char* rows, auto element, int row_bytes, int bytes) __attribute__((always_inline)) {
+  // This wave's rows of a stage's values (BYTES of them), once they are in LDS: what is no number becomes 0.  Returns the
+  // rows.
+  auto clear_odd = [&](char* rows, auto element, auto row_bytes, auto n_bytes) __attribute__((always_inline)) {
     constexpr bool kWide = sizeof(element) == 4;
-    unsigned found = 0;
-    for (int at = lane * 16; at < bytes; at += 64 * 16) {
-      const u32x4 d = *reinterpret_cast<const u32x4*>(rows + at);
-      unsigned bad[4], any = 0;   // the top bit of each element whose exponent is all ones
+    constexpr int kRow = decltype(row_bytes)::value, kBytes = decltype(n_bytes)::value;
+    // (the top bit of each element whose exponent is all ones)
+    auto bad = [](unsigned d) { return kWide ? ((d & 0x7f800000u) + 0x00800000u) & 0x80000000u : ((d & 0x7f807f80u) + 0x00800080u) & 0x80008000u; };
+    unsigned any = 0;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        bad[i] = kWide ? ((d[i] & 0x7f800000u) + 0x00800000u) & 0x80000000u : ((d[i] & 0x7f807f80u) + 0x00800080u) & 0x80008000u;
-        any |= bad[i];
-      }
-      if (any) {
-        u32x4 z = d;
+    for (int at = 0; at < kBytes; at += 64 * 16) {
+      const u32x4 d = *reinterpret_cast<const u32x4*>(rows + at + lane * 16);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) any |= bad(d[i]);
+    }
+    unsigned found = 0;
+    if (__any(any != 0)) {
+#pragma unroll 1
+      for (int at = lane * 16; at < kBytes; at += 64 * 16) {
+        u32x4 d = *reinterpret_cast<const u32x4*>(rows + at);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          if (bad[i] & 0x80000000u) z[i] &= kWide ? 0u : 0x0000ffffu;
-          if (bad[i] & 0x00008000u) z[i] &= 0xffff0000u;
+          const unsigned b = bad(d[i]);
+          found |= b ? 1u << at / kRow : 0u;
+          if (b & 0x80000000u) d[i] &= kWide ? 0u : 0x0000ffffu;
+          if (b & 0x00008000u) d[i] &= 0xffff0000u;
         }
-        *reinterpret_cast<u32x4*>(rows + at) = z;
-        found |= 1u << at / row_bytes;
+        *reinterpret_cast<u32x4*>(rows + at) = d;
       }
-    }
-    if (__any(found != 0)) {
 #pragma unroll
       for (int x = 1; x < 64; x <<= 1) found |= __shfl_xor(found, x, SD_WAVE);
     }
@@ -457,11 +425,16 @@ __global__ __launch_bounds__(256, KS > 4 ? 1 : 2) void rows_attn_kernel(RowsAttn
     if (left < kPage || some) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       char* rows = cur + (LATENT ? wave * kKeyPage : 4 * kKeyPage + wave * kValPage);
-      if (left < kPage)
+      if (left < kPage) {
         for (int at = max(left, 0) * kVRow + lane * 16; at < kPage * kVRow; at += 64 * 16) *reinterpret_cast<u32x4*>(rows + at) = u32x4{0, 0, 0, 0};
+        if (POOLED)   // (the keys too: their scores must be numbers)
+          for (int at = max(left, 0) * DK * 2 + lane * 16; at < kKeyPage; at += 64 * 16)
+            *reinterpret_cast<u32x4*>(cur + wave * kKeyPage + at) = u32x4{0, 0, 0, 0};
+      }
       if (some) {
-        const unsigned found = means ? clear_odd(cur + kPooled * 512 + wave * 4096, float(), 512, 4096)
-                                     : clear_odd(rows, bf16_t(), kVRow, kPage * kVRow);
+        unsigned found;
+        if (means) found = clear_odd(cur + kPooled * 512 + wave * 4096, float(), Number<512>{}, Number<4096>{});
+        else found = clear_odd(rows, bf16_t(), Number<kVRow>{}, Number<kPage * kVRow>{});
         if (lane == 0) odd[st & 1][wave] = found;
       }
     }
@@ -471,20 +444,93 @@ __global__ __launch_bounds__(256, KS > 4 ? 1 : 2) void rows_attn_kernel(RowsAttn
     else attend(cur, st);
     if (some && (odd[st & 1][0] | odd[st & 1][1] | odd[st & 1][2] | odd[st & 1][3])) add_odd(st, means);
   };
+  // Query m of the workgroup by a whole wave: a lane a key for the scores, two channels for the sums.
+  auto redo_query = [&](int m) __attribute__((always_inline)) {
+    const int t = m / qh, h = kvh * qh + m - t * qh, p = pos0 + t;
+    const float* q = g.q + (size_t)(row0 + first + t) * g.ldq + (size_t)h * DK;
+    const int t_first = max(p - g.window + 1, 0);
+    const int before = POOLED ? blocks_of(p) : min(g.keep_first, t_first), total = before + p - t_first + 1;
+    const float add = POOLED && g.head_bias ? g.head_bias[h] : 0.f;
+    // (row of the cache of key idx: pooled blocks or kept tokens first)
+    auto row_of = [&](int idx) {
+      if (POOLED && idx < before) {
+        const int lp = (idx * g.pool + g.pool - 1) / kPage;
+        return ((size_t)tbl[lp] * g.G + kvh) * g.pslots + idx - lp * kPage / g.pool;
+      }
+      const int j = idx < before ? idx : t_first + idx - before;
+      return ((size_t)tbl[j / kPage] * g.G + kvh) * kPage + j % kPage;
+    };
+    float top = -INFINITY, l = 0.f, y[2] = {0.f, 0.f};
+#pragma unroll 1
+    for (int base = 0; base < total; base += SD_WAVE) {
+      const int idx = min(base + lane, total - 1);
+      const size_t row = row_of(idx);
+      const bool block = POOLED && idx < before;
+      float score = 0.f;
+#pragma unroll 1
+      for (int c = 0; c < DK; ++c) score = fmaf(q[c], block ? g.pk[row * DK + c] : (float)g.kc[row * DK + c], score);
+      score *= g.scale;
+      float w;
+      if constexpr (POOLED) {
+        w = 1.f / (1.f + expf(-(score + add)));
+      } else {
+        float mx = base + lane < total ? score : -INFINITY;
+#pragma unroll
+        for (int x = 1; x < SD_WAVE; x <<= 1) mx = fmaxf(mx, __shfl_xor(mx, x, SD_WAVE));
+        mx = fmaxf(mx, top);
+        const float corr = top == -INFINITY ? 0.f : expf(top - mx);
+        top = mx;
+        w = expf(score - mx);
+        float sum = base + lane < total ? w : 0.f;
+#pragma unroll
+        for (int x = 1; x < SD_WAVE; x <<= 1) sum += __shfl_xor(sum, x, SD_WAVE);
+        l = l * corr + sum;
+        y[0] *= corr;
+        y[1] *= corr;
+      }
+#pragma unroll 1
+      for (int i = 0; i < min(SD_WAVE, total - base); ++i) {
+        const float wi = __shfl(w, i, SD_WAVE);
+        const size_t v = row_of(base + i) * DV + 2 * lane;
+        const bool of_block = POOLED && base + i < before;
+#pragma unroll
+        for (int x = 0; x < 2; ++x) y[x] = fmaf(wi, of_block ? g.pv[v + x] : (float)g.vc[v + x], y[x]);
+      }
+    }
+    static_assert(LATENT || (DK == 128 && DV == 128), "two channels a lane");
+    const size_t at = (size_t)(row0 + first + t) * g.ldo + (size_t)h * DV + 2 * lane;
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      const float r = POOLED ? y[x] : y[x] * (1.f / l);
+      if (g.out) g.out[at + x] = r;
+      if (g.out_b) g.out_b[at + x] = (bf16_t)r;
+    }
+  };
   load(s0, 0);
-  int st = 0;
-  for (; st + 1 < stages; st += 2) {
+#pragma unroll 1
+  for (int st = 0; st < stages; st += 2) {
     step(s0, s1, st);
-    step(s1, s0, st + 1);
+    if (st + 1 < stages) step(s1, s0, st + 1);
   }
-  if (st < stages) step(s0, s1, st);
+  // A part of a query that is 0 makes a NaN of an infinite key, where the query's product with it is infinite and its weight
+  // a number, and sigmoid_of wants finite scores: queries that met a score that is no number are done again, a key at a
+  // time as on the vector pipe.  (Not of latent rows, where an infinite channel is an infinite value too.)
+  bool done = !mine;
+  if constexpr (!LATENT) {
+    int odd_score = mine & (int)(POOLED ? !(m_run + fabsf(bias) < INFINITY) : m_run != m_run);
+    odd_score |= __shfl_xor(odd_score, 16, SD_WAVE);
+    odd_score |= __shfl_xor(odd_score, 32, SD_WAVE);
+    done |= odd_score;
+#pragma unroll 1
+    for (unsigned left = (unsigned)__ballot(odd_score) & 0xffffu; left; left &= left - 1) redo_query(16 * wave + __builtin_ctz(left));
+  }
   float inv = 1.f;
   if constexpr (!POOLED) {
     l_run += __shfl_xor(l_run, 16, SD_WAVE);
     l_run += __shfl_xor(l_run, 32, SD_WAVE);
     inv = 1.f / l_run;
   }
-  if (!mine) return;
+  if (done) return;
   const size_t at = (size_t)(row0 + first + t) * g.ldo + (size_t)h * DV + 4 * quad;
 #pragma unroll
   for (int v = 0; v < VT; ++v) {

@@ -305,6 +305,14 @@ int few_shape(const PromptArgs& a, hipStream_t st) {
   return tn == 4 ? launch_few<4, EPI>(a, 1, st) : launch_few<2, EPI>(a, 1, st);
 }
 
+// The block of a prompt pass, us of 256 x 256 (whole K only), 128 x 128 with four stages, with two:
+//   one block a CU at most (`small` <= 256): 6144 x 4096 at 512 rows 31.9 with four stages, 42.1 with two; 4096 x 14336 at
+//   1024 rows 103 against 145; above, two blocks a CU cover each other's loads: 2048 rows 206 against 192;
+//   whole K: 256 x 256 from 200 blocks on (14336 x 4096 gated: 272 rows 94, 101, 95; 1024 rows 195, 243, 231; 4096 rows 705,
+//   1010, 866; 18944 x 3584 gated, 1024 rows 262, 337, 289; 32000 x 2048, 512 rows 59, 83, 66).  Between the line at 128
+//   blocks and there both sides win: 18432 x 2048 at 512 rows (144 blocks) 52, 58, 54, at 272 rows 51, 37, 32; gated 8192 x
+//   2048 at 512 rows (128 blocks, 50, 41, 36); and where the second round is short (18944 x 3584, 272 rows, 296 blocks): 161,
+//   109, 107.
 template <int EPI>
 int prompt_shape(const PromptArgs& a, int S, hipStream_t st) {
   const long big = (long)((a.n_tiles + 15) / 16) * ((a.M + 255) / 256);

@@ -199,3 +199,30 @@ def test_more_wanted_rows_than_a_pass_gives():
     for b in range(0, 300, 100):
         model.prompt(kv, [(b + i, p, 0, True) for i, p in enumerate(prompts[b:b + 100])], few[b:b + 100])
     assert torch.equal(got, few)
+
+
+@pytest.mark.parametrize("pos,piece,final", [(3000, 200, False), (3000, 257, False), (3000, 40, True), (100, 40, True), (100, 1, True), (0, 256, False)])
+def test_pieces_of_a_prompt_go_where_they_are_quicker(pos, piece, final, monkeypatch):
+    """The next tokens of a prompt behind `pos` others: pieces that a forward pass holds go through one (and a last token
+    through one of its own) unless that last token's logits cost more than the piece's keys, larger ones through a prompt
+    pass; the first generated token is that of the whole prompt either way."""
+    from vllm_omni_draft_amd import config, weights
+    from vllm_omni_draft_amd.engine import EngineConfig, SpecEngine
+    from vllm_omni_draft_amd.model_runner import DecoderModel
+    cfg = config.create_model_config(None, n_layers=1, hidden=128, n_heads=2, n_kv_heads=1, head_dim=64, ffn=128, vocab=128, max_pos=6000)
+    w = weights.random_init(cfg, seed=3)
+    tail = 0 if final else 5
+    prompt = torch.randint(0, cfg.vocab, (pos + piece + tail,), generator=torch.Generator().manual_seed(1)).tolist()
+    want = SpecEngine(w, None, EngineConfig(k=0, max_seq_len=4096)).add_request(0, prompt)
+    eng = SpecEngine(w, None, EngineConfig(k=0, max_seq_len=4096))
+    h = eng.prefill_begin(prompt)
+    if pos:
+        assert eng.prefill_advance(h, pos) is None
+    calls = []
+    for name in ("prompt", "forward"):
+        real = getattr(DecoderModel, name)
+        monkeypatch.setattr(DecoderModel, name, lambda *a, _r=real, _n=name, **k: (calls.append(_n), _r(*a, **k))[1])
+    first = eng.prefill_advance(h, piece)
+    packed = piece > 256 or (final and piece > 1 and pos + piece <= 2048)
+    assert calls == (["prompt"] if packed else ["forward"] * (2 if final and piece > 1 else 1))
+    assert (first if final else eng.prefill_advance(h, tail)) == want

@@ -729,7 +729,7 @@ class SpecEngine:
     def _prefill_range(self, slot: int, prompt: Sequence[int], c_from: int, c_to: int, final: bool,
                        rope_positions=None, input_embeds=None, decoded_from: Optional[int] = None) -> None:
         """Passes over prompt tokens c_from..c_to-1 of the sequence in `slot` (both models: prompt passes,
-        or forward passes of prefill_rows tokens on the wide family where a model has none).  final: c_to
+        or forward passes of prefill_rows tokens on the wide family, as DecoderModel.packs says).  final: c_to
         is the prompt's end; its last token's logits (target) land in t_out[0].
         decoded_from: tokens from this position on were first computed by decode passes (the
         sequence is being rebuilt from its own output): a model whose decode passes run on the
@@ -745,10 +745,11 @@ class SpecEngine:
             logits = self.t_out if model is self.target else None
             embeds = input_embeds if model is self.target else None
             positions = rope_positions if model.cfg.mrope_section else None
-            c_done = c_from
-            if model.packs_prompts and c_from < min(c_to, narrow_from):
-                c_done = min(c_to, narrow_from)
-                want = final and c_done == n and model is self.target
+            c_done = min(c_to, narrow_from)
+            want = final and c_done == n and model is self.target
+            if not model.packs(c_done - c_from, c_done, want):
+                c_done = c_from
+            else:
                 model.prompt(kv, [(slot, prompt[c_from:c_done], c_from, want)], logits if want else None,
                              None if embeds is None else embeds[c_from:c_done].contiguous(),
                              None if positions is None else positions[:, c_from:c_done])

@@ -218,6 +218,16 @@ class DecoderModel:
         _lib.check(rc, "sd_model_forward")
 
 
+    def packs(self, rows: int, ctx: int, wanted: bool) -> bool:
+        """Whether `rows` consecutive tokens of one sequence, which then holds ctx, go through prompt() (and not
+        forward(), in chunks of prefill_rows and with a pass of its own for a last token whose logits are wanted;
+        the bits are the same).  A workgroup of prompt attention takes its rows through all keys, so a few rows behind
+        a long context leave most of the chip idle where forward() splits the keys: us for four layers of an 8B
+        model, 64 rows behind 0 / 1000 / 4000 / 38000 tokens 581 / 821 / 1518 / 9783 against 551 / 561 / 632 / 1793; 256
+        rows 857 / 1092 / 1804 / 10037 against 792 / 918 / 1254 / 5725; 512 rows even up to 16000.  The last token's pass
+        costs 436 to 473 more: worth it from about 2000 tokens on (1B: the same, 7B with 7 heads a group: 2300)."""
+        return self.packs_prompts and (rows > PREFILL_ROWS or (wanted and rows > 1 and ctx <= 2048))
+
     def prompt(self, kv: PagedKVCache, runs, logits: Optional[torch.Tensor] = None,
                input_embeds: Optional[torch.Tensor] = None, rope_pos: Optional[torch.Tensor] = None,
                workspace: Optional[torch.Tensor] = None) -> None:

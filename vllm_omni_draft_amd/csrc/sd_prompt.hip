@@ -325,11 +325,16 @@ int prompt_shape(const PromptArgs& a, int S, hipStream_t st) {
 }  // namespace
 
 bool sd_prompt_linear_fits_(int M, int n_tiles, int K, int64_t ldx) {
-  // 256 rows are one pass of the wide kernels.  Few blocks of a long K leave most CUs idle for a long time: 48 blocks
-  // of K 8192 59 us against 50 in two passes of the wide kernels (300 rows, 2048 outputs), 96 blocks of K 14336 as
-  // long as those, 48 blocks of K 2048 23 us against 36.
+  // 256 rows are one pass of the kernels for fewer.  A block takes a long K's time however few blocks there are, and two or
+  // three passes split it over the chip; us against those passes, weights from memory, 300 / 512 / 640 / 768 / 1024 rows:
+  // 4096 x 14336 107 / 135 / 136 / 136 / 138 against 69 / 87 / 122 / 133 / 173; 3584 x 18944 131 / 164 / 164 / 165 / 169
+  // against 78 / 98 / 135 / 146 / 193; 2048 x 8192 65 / 74 / 75 / 74 / 75 against 45 / 55 / 75 / 81 / 109.  A K of up to
+  // 4096: 4096 x 4096 39 / 45 / 46 / 45 / 47 against 52 / 59 / 69 / 75 / 100, 2048 x 2048 24 / 24 / 26 / 27 / 28 against 37
+  // / 46 / 61 / 68 / 90.  (Gated matrices whose blocks of 256 rows make a short second round lose too: 18944 x 3584 171 /
+  // 181 against 134 / 165 up to 512 rows, 8192 x 2048 54 / 57 against 40 / 50, 14336 x 4096 193 / 196 against 164 / 178 at
+  // 640 and 768.)
   const long blocks = (long)((n_tiles + 7) / 8) * ((M + 127) / 128);
-  return M > 256 && K % 64 == 0 && K >= 128 && (blocks > 64 || K <= 4096) && 512 * ldx < 0x7fffffff;
+  return M > 256 && K % 64 == 0 && K >= 128 && (K <= 4096 || (M > 768 && blocks > 64)) && 512 * ldx < 0x7fffffff;
 }
 
 // At most 256 rows: the products themselves (splits of K: the partial sums, for the caller's epilogue kernel).  Against

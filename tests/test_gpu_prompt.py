@@ -226,3 +226,24 @@ def test_pieces_of_a_prompt_go_where_they_are_quicker(pos, piece, final, monkeyp
     packed = piece > 256 or (final and piece > 1 and pos + piece <= 2048)
     assert calls == (["prompt"] if packed else ["forward"] * (2 if final and piece > 1 else 1))
     assert (first if final else eng.prefill_advance(h, tail)) == want
+
+
+@pytest.mark.parametrize("n", [257, 768, 769])
+def test_prompts_on_either_side_of_the_line_for_a_long_k(n):
+    """A matrix of more than 4096 columns goes through the kernels for 256 rows up to 768 rows, the last of them one row
+    here, and through the prompt kernel beyond: logits and caches as by forward passes."""
+    from vllm_omni_draft_amd import config, weights
+    from vllm_omni_draft_amd.engine import _KvView
+    from vllm_omni_draft_amd.model_runner import DecoderModel
+    cfg = config.create_model_config(None, n_layers=2, hidden=2048, n_heads=4, n_kv_heads=2, head_dim=64, ffn=4864, vocab=512, max_pos=800)
+    model = DecoderModel(weights.random_init(cfg, seed=3), 800, wide=True)
+    prompt = torch.randint(0, cfg.vocab, (n,), generator=torch.Generator().manual_seed(n)).tolist()
+    one, two = _cache(cfg, [n], 800), _cache(cfg, [n], 800)
+    got = torch.empty(1, cfg.vocab, device="cuda")
+    model.prompt(one, [(0, prompt, 0, True)], got)
+    zero, t = torch.zeros(1, dtype=torch.int32, device="cuda"), torch.tensor(prompt, dtype=torch.int32, device="cuda")
+    for c in range(0, n, 200):
+        m = min(200, n - c)
+        out = torch.empty(m, cfg.vocab, device="cuda")
+        model.forward(_KvView(two, 0), t, 0, c, zero, c, 1, m, out, wide=True)
+    assert torch.equal(got[0], out[-1]) and torch.equal(one.k, two.k) and torch.equal(one.v, two.v)

@@ -759,7 +759,7 @@ def test_chunked_recurrences_are_as_near_to_64_bits_as_the_scan(kind, H, Gq, dk,
 @pytest.mark.parametrize("n", [200, 40])
 def test_chunked_recurrences_of_values_that_are_no_numbers(kind, H, Gq, dk, dv, n):
     """Infinite and NaN values, keys and queries inside blocks of 16 tokens and chunks (and of a portion in one go, 40):
-    what the scan token by token leaves finite is finite and the same."""
+    what the scan token by token leaves finite is finite and the same; what it leaves infinite in the state is so too."""
     from vllm_omni_draft_amd import ops
     g = torch.Generator(device=DEV).manual_seed(H + n + dk)
     rn = lambda *shape: torch.randn(*shape, generator=g, device=DEV)
@@ -780,6 +780,7 @@ def test_chunked_recurrences_of_values_that_are_no_numbers(kind, H, Gq, dk, dv, 
             ok = torch.isfinite(want)
             assert torch.equal(torch.isfinite(got), ok)
             assert (got - want)[ok].abs().max() <= 2e-5 * want[ok].abs().max()
+        assert torch.equal(torch.isnan(S2), torch.isnan(S1))
         return a
     inf, nan = float("inf"), float("nan")
     for x, t, c, y in ((v, n - 3, 4, inf), (v, n - 20, 70 if H * dv > 140 else 1, nan), (q, 7, 3, nan), (v, 21, dv + 2, -inf), (k, n - 30, 5, nan)):

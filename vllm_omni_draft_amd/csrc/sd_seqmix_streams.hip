@@ -7,6 +7,7 @@
 // Arithmetic as in sd_seqmix.hip: activations are f32 buffers; streams, norms, decays and states are
 // f32 always; with bf16 weights the operands of matrix products are rounded to bf16 where they are
 // produced and the cache holds bf16.
+#include <float.h>
 #include <math.h>
 
 #include <mutex>
@@ -619,8 +620,10 @@ struct Product {
     lo = fmaf(lo, p.hi, fmaf(hi, p.lo, fmaf(hi, p.hi, -h)));
     hi = h;
   }
-  // x times it, plus y
-  __device__ __forceinline__ float of(float x, float y = 0.f) const { return fmaf(x, hi, fmaf(x, lo, y)); }
+  // x times it, plus y (an infinite x stays infinite: what is left of the rounding may be 0)
+  __device__ __forceinline__ float of(float x, float y = 0.f) const {
+    return fmaf(x, hi, fmaf(__builtin_amdgcn_fmed3f(x, -FLT_MAX, FLT_MAX), lo, y));
+  }
 };
 
 template <int DKP>

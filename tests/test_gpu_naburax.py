@@ -803,6 +803,30 @@ def test_decode_attention_from_lds_against_float64(H, G, dk, dv, maps, extras):
     assert off < 3e-6, off
 
 
+@pytest.mark.parametrize("H,G,dk,dv,maps", [(16, 1, 576, 512, 1), (7, 1, 576, 512, 1), (6, 2, 128, 128, 1), (4, 2, 256, 256, 1), (8, 2, 32, 256, 1),
+                                           (12, 2, 256, 40, 2)])
+def test_decode_attention_from_lds_sums_in_the_order_of_the_general_kernel(H, G, dk, dv, maps):
+    """The same bits as over an f32 cache of the same values, which the general kernel takes: parts of the channels and shares of
+    a tile's keys are added in one order in both.  Key rows of whole pieces of 32 channels are cut alike in either type; an
+    infinite key and one that is no number are among them."""
+    from vllm_omni_draft_amd import ops
+    g = torch.Generator().manual_seed(H + dk)
+    pos = [0, 2, 63, 64, 150, 199]
+    R, nb = len(pos), 13
+    kc = torch.randn(R * nb, G * maps, 16, dk, generator=g).to(torch.bfloat16)
+    vc = None if G == 1 else torch.randn(R * nb, G, 16, dv, generator=g).to(torch.bfloat16)
+    bt = torch.randperm(R * nb, generator=g).view(R, nb)
+    kc[bt[4, 3], 0, 5, 1], kc[bt[5, 8], 0, 0, 7] = float("inf"), float("nan")
+    q, sinks = torch.randn(R, H * maps * dk, generator=g), torch.randn(H * maps, generator=g)
+    for window, keep, chunk, cap, sk in ((100, 3, 0, 0.0, None), (0, 0, 160, 5.0, sinks)):
+        def run(cast):
+            k, v = cast(kc).cuda(), None if vc is None else cast(vc).cuda()
+            at = (dev(q), k, v, i32(pos), i32(list(range(R))), bt.int().cuda(), H, G)
+            rest = (dk, dv, dk ** -0.5, window, keep, chunk, cap, None if sk is None else dev(sk))
+            return (ops.multimap_softmax_attention(*at, maps, *rest) if maps > 1 else ops.masked_softmax_attention(*at, *rest)).cpu()
+        torch.testing.assert_close(run(lambda t: t), run(lambda t: t.float()), rtol=0, atol=0, equal_nan=True)
+
+
 def same_where_finite(got, want, tol=1e-5):
     """The same entries are finite in both, and those agree."""
     assert torch.equal(torch.isfinite(got), torch.isfinite(want))

@@ -431,18 +431,24 @@ __global__ __launch_bounds__(256) void window_softmax_attn_kernel(
   }
 }
 
-// The cut launch of a bf16 cache: the same workgroups and tiles of 64 keys, for decoding, where a launch is as long as one
-// workgroup's chain of dependent reads.  window_softmax_attn_kernel reads its keys a few pieces a lane at a time, then its
-// values in batches of rows, 2 bytes a lane (26 us for 4 rows of latent attention over 120 keys); here 1024 threads ask
-// for the tile's keys and values at once, 16 bytes each, and everything else is read from LDS: keys by 16 threads a key,
-// over consecutive parts of the channels whose sums are added in part order; values four columns a thread, every kp-th key
-// of the tile, whose sums are added in order of kp.  4 rows, 120
-// keys, us: 16 heads of 576 / 512 over one row a token 26.4 -> 13.2, 16 heads over 4 of 128 16.0 -> 9.5.
-constexpr int kFewThreads = 1024, kFewParts = kFewThreads / kSplitKeys, kFewHeads = 4;
+// The cut launch of a bf16 cache: the same workgroups, tiles of 64 keys and sums in the same order, so the same bits, for
+// decoding, where a launch is as long as one workgroup's chain of dependent reads.  window_softmax_attn_kernel reads its keys
+// a few pieces a lane at a time, then its values in batches of rows, 2 bytes a lane (26 us for 4 rows of latent attention over
+// 120 keys); here 1024 threads ask for the tile's keys and values at once, 16 bytes each, and everything else is read from
+// LDS.  A wave scores the tile's keys, a lane a key, for one part of the channels and one head; the parts' sums are added in
+// part order.  Values: four columns of a head a thread and one of four shares of the keys (every fourth), whose sums are
+// added in order.  4 rows, 120 keys, us: 16 heads of 576 / 512 over one row a token 26.4 -> 14.3, 16 heads over 4 of 128
+// 16.0 -> 9.4.  (Scores of two or four heads a wave, which unpack a key once for them: 14.6 and 16.4.)
+constexpr int kFewThreads = 1024, kFewParts = 4, kFewShares = 4, kFewHeads = 4;
 constexpr int kFewPad = 16;   // bytes behind a row of keys or values in LDS: rows start on different banks
-__host__ __device__ inline size_t few_lds(int dk, int dv, bool shared) {
-  return (size_t)kSplitKeys * (dk * 2 + kFewPad + (shared ? 0 : dv * 2 + kFewPad)) + sizeof(float) * kFewHeads * dk +
-         sizeof(float) * kFewHeads * kSplitKeys * (kFewParts + 1) + sizeof(unsigned long long) * 2 * kSplitKeys;
+// (values' sums, [share][head][dv]: over the keys, which are done with, where values lie elsewhere and there is room)
+__host__ __device__ inline bool few_sums_over_keys(int dk, int dv, int NH, bool shared) {
+  return !shared && (size_t)kSplitKeys * (dk * 2 + kFewPad) >= sizeof(float) * kFewShares * NH * dv;
+}
+__host__ __device__ inline size_t few_lds(int dk, int dv, int NH, bool shared) {
+  return (size_t)kSplitKeys * (dk * 2 + kFewPad + (shared ? 0 : dv * 2 + kFewPad)) + sizeof(unsigned long long) * 2 * kSplitKeys +
+         sizeof(float) * (NH * dk + kFewHeads * kSplitKeys * (kFewParts + 1)) +
+         (few_sums_over_keys(dk, dv, NH, shared) ? 0 : sizeof(float) * kFewShares * NH * dv);
 }
 __global__ __launch_bounds__(kFewThreads) void few_softmax_attn_kernel(
     const float* __restrict__ q, int64_t ldq, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
@@ -455,10 +461,11 @@ __global__ __launch_bounds__(kFewThreads) void few_softmax_attn_kernel(
   const int k_ld = dk * 2 + kFewPad, v_ld = shared ? k_ld : dv * 2 + kFewPad;
   char* ks = few_smem;                                                              // [64][k_ld]
   char* vs = shared ? ks : ks + kSplitKeys * k_ld;                                  // [64][v_ld]
-  float* ps = reinterpret_cast<float*>(ks + kSplitKeys * (k_ld + (shared ? 0 : v_ld)));   // [parts][4][64], then [kp][4][dv]
+  unsigned long long* at = reinterpret_cast<unsigned long long*>(ks + kSplitKeys * (k_ld + (shared ? 0 : v_ld)));   // [2][64] rows of the caches
+  float* ps = reinterpret_cast<float*>(at + 2 * kSplitKeys);                        // [parts][4][64]
   float* wt = ps + kFewParts * kFewHeads * kSplitKeys;                              // [4][64]
-  float* qs = wt + kFewHeads * kSplitKeys;                                          // [4][dk]
-  unsigned long long* at = reinterpret_cast<unsigned long long*>(qs + kFewHeads * dk);   // [2][64] rows of the caches
+  float* qs = wt + kFewHeads * kSplitKeys;                                          // [NH][dk]
+  float* sums = few_sums_over_keys(dk, dv, NH, shared) ? reinterpret_cast<float*>(ks) : qs + NH * dk;   // [shares][nh][dv]
   const int r = blockIdx.x, gk = blockIdx.y, g = gk / maps, mp = gk % maps, tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hgroup = blockIdx.z % n_hgroups, split = blockIdx.z / n_hgroups;
@@ -507,21 +514,19 @@ __global__ __launch_bounds__(kFewThreads) void few_softmax_attn_kernel(
     }
   }
   __syncthreads();
-  {   // scores: key `lane`, part `wave`
-    const int units = dk / 8, per = (units + kFewParts - 1) / kFewParts;
-    float s[kFewHeads] = {0.f, 0.f, 0.f, 0.f};
-    for (int u = wave * per; u < min((wave + 1) * per, units); ++u) {
-      float kf[8];
-      Piece<bf16_t>::unpack(*reinterpret_cast<const u32x4*>(ks + lane * k_ld + u * 16), kf);
+  {   // scores: key `lane`
+    const int hq = wave % kFewHeads, part = wave / kFewHeads, units = dk / 8, per = (units + kFewParts - 1) / kFewParts;
+    if (hq < nh) {
+      float sc = 0.f;
+#pragma unroll 2
+      for (int u = part * per; u < min((part + 1) * per, units); ++u) {
+        float kf[8];
+        Piece<bf16_t>::unpack(*reinterpret_cast<const u32x4*>(ks + lane * k_ld + u * 16), kf);
 #pragma unroll
-      for (int hq = 0; hq < kFewHeads; ++hq)
-        if (hq < nh) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) s[hq] = fmaf(qs[hq * dk + u * 8 + e], kf[e], s[hq]);
-        }
+        for (int e = 0; e < 8; ++e) sc = fmaf(qs[hq * dk + u * 8 + e], kf[e], sc);
+      }
+      ps[(part * kFewHeads + hq) * kSplitKeys + lane] = sc;
     }
-#pragma unroll
-    for (int hq = 0; hq < kFewHeads; ++hq) ps[(wave * kFewHeads + hq) * kSplitKeys + lane] = s[hq];
   }
   __syncthreads();
   if (wave < nh) {   // a wave a head
@@ -545,26 +550,25 @@ __global__ __launch_bounds__(kFewThreads) void few_softmax_attn_kernel(
   }
   __syncthreads();
   // values: thread = (share of the keys, head, four columns)
-  const int cols = dv / 4, kps = max(kFewThreads / (cols * kFewHeads), 1);
-  for (int t = tid; t < cols * kFewHeads * kps; t += kFewThreads) {
-    const int c = t % cols, hq = t / cols % kFewHeads, kp = t / (cols * kFewHeads);
+  const int cols = dv / 4;
+  for (int t = tid; t < cols * nh * kFewShares; t += kFewThreads) {
+    const int c = t % cols, hq = t / cols % nh, share = t / (cols * nh);
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-    if (hq < nh) {
-      for (int k = kp; k < n_here; k += kps) {
-        const bf16x4 v = *reinterpret_cast<const bf16x4*>(vs + k * v_ld + c * 8);
-        const float w = wt[hq * kSplitKeys + k];
+    for (int k = share; k < n_here; k += kFewShares) {
+      const bf16x4 v = *reinterpret_cast<const bf16x4*>(vs + k * v_ld + c * 8);
+      const float w = wt[hq * kSplitKeys + k];
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc[e] = fmaf(w, (float)v[e], acc[e]);
-      }
+      for (int e = 0; e < 4; ++e) acc[e] = fmaf(w, (float)v[e], acc[e]);
     }
-    *reinterpret_cast<f32x4*>(ps + ((size_t)kp * kFewHeads + hq) * dv + c * 4) = acc;
+    *reinterpret_cast<f32x4*>(sums + ((size_t)share * nh + hq) * dv + c * 4) = acc;
   }
   __syncthreads();
   for (int t = tid; t < nh * cols; t += kFewThreads) {
     const int c = t % cols, hq = t / cols;
-    f32x4 o = *reinterpret_cast<const f32x4*>(ps + hq * dv + c * 4);
-    for (int kp = 1; kp < kps; ++kp) {
-      const f32x4 v = *reinterpret_cast<const f32x4*>(ps + (kp * kFewHeads + hq) * dv + c * 4);
+    f32x4 o = *reinterpret_cast<const f32x4*>(sums + hq * dv + c * 4);
+#pragma unroll
+    for (int share = 1; share < kFewShares; ++share) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(sums + (share * nh + hq) * dv + c * 4);
 #pragma unroll
       for (int e = 0; e < 4; ++e) o[e] += v[e];
     }
@@ -2440,11 +2444,14 @@ int gated_attention(const float* q, int64_t ldq, const void* k_cache, const void
   float* part_acc = split ? (float*)scratch : nullptr;
   float* part_ml = split ? part_acc + (size_t)n_splits * n_rows * HM * dv : nullptr;
   dim3 grid(n_rows, G * maps, n_hgroups * n_splits);
-  // With a tile's work for 1024 threads: 4 heads of 128 + 128 columns a workgroup are quicker at every row count (1024 keys, us
-  // with the merge launch, 4 / 16 / 64 rows: 16.8 / 29.5 / 87 against 19.0 / 33.0 / 88), 4 of 576 + 512 too (22 / 56 / 199
-  // against 32 / 59 / 210), one head of 64 + 64 is not (17 / 43 / 143 against 19 / 31 / 95).
-  const size_t few_bytes = few_lds(dk, dv, !v_cache);
-  if (split && !cache_f32 && (long)NH * (dk + dv) >= 1024 && dk % 8 == 0 && dv % 8 == 0 && sd_aligned16(k_cache) && sd_aligned16(vc) && few_bytes <= 160 * 1024) {
+  // With a tile's work for 1024 threads, and room for a second workgroup on the CU unless the values are part of the keys.
+  // us with the merge launch, general kernel / this one, 1024 keys, 4 / 16 / 64 rows: 16 heads over 4 of 128 + 128 columns 18.5 /
+  // 14.7, 33.3 / 29.0, 88 / 82; 16 heads over one row a token of 576 with 512 values in it 32.3 / 23.9, 58.0 / 59.3, 211 / 212 (100
+  // keys of a cache for 1088: 30.3 / 20.4, 30.2 / 20.0, 80 / 54); 8 over 4 of 256 + 256 15.8 / 14.6, 30.4 / 29.2, 92 / 86.  But 4 over
+  // 4 of 512 + 512 (141 KB of LDS) 20.0 / 19.7, 38.8 / 47.7, 141 / 165, and one head of 64 + 64 a workgroup 19 / 17, 31 / 43, 95 / 143.
+  const size_t few_bytes = few_lds(dk, dv, NH, !v_cache);
+  if (split && !cache_f32 && (long)NH * (dk + dv) >= 1024 && dk % 8 == 0 && dv % 8 == 0 && sd_aligned16(k_cache) &&
+      sd_aligned16(vc) && few_bytes <= (v_cache ? 80 : 160) * 1024) {
     static std::once_flag once;
     static hipError_t err = hipSuccess;
     std::call_once(once, [] {

@@ -130,3 +130,37 @@ def test_a_steps_tokens_beyond_32_bits_are_refused():
     from vllm_omni_draft_amd.seq_engine import _ints
     with pytest.raises(RuntimeError):
         _ints([1, 2 ** 40])
+
+
+def test_single_tokens_beside_a_prompt_in_every_form_that_torch_takes():
+    """A request's one token and its wanted index may be elements of a device tensor, which numpy does not read; what does not fit
+    32 bits is refused as in a step of prompts alone."""
+    from types import SimpleNamespace
+    from vllm_omni_draft_amd.seq_engine import SeqEngine, _Seq, _ints
+
+    class Element:   # stands for an element of a device tensor
+        def __init__(self, v):
+            self.v = v
+
+        def __index__(self):
+            return self.v
+
+        def __lt__(self, other):
+            return self.v < other
+
+        def __ge__(self, other):
+            return self.v >= other
+
+        def __array__(self, *args, **kw):
+            raise TypeError("can't convert device type tensor to numpy")
+
+    got = []
+    eng = SimpleNamespace(cfg=SimpleNamespace(max_rows=64), _run_pass=lambda *a: got.append(a))
+    run = lambda token, want: SeqEngine._run_passes(eng, [(_Seq(2, 5, 9), [token], [want]), (_Seq(1), _ints([4, 6, 8]), _ints([2]))],
+                                                    [0, 0], [0, 1], None, None)
+    run(Element(7), Element(0))
+    host, R, E, dst, sizes = got[0][:5]
+    assert host.dtype == torch.int32 and (R, E, sizes, list(dst)) == (4, 2, (1, 3), [0, 1])
+    assert host.tolist() == [7, 4, 6, 8, 5, 0, 1, 2, 2, 1, 1, 1, 9, -1, 4, 6, 2, 0, 1, 5, 1, 1, 3, 0, 0, 3]
+    with pytest.raises(RuntimeError):
+        run(2 ** 40, 0)

@@ -187,6 +187,8 @@ class SeqEngine:
             toks, pos, slot, prev = batch[:4 * R].reshape(4, R)
             for e, (i, lo, hi, r0) in enumerate(parts):
                 s, t, w = plan[i]
+                if isinstance(t, list):   # (a single token; numpy does not take all that torch takes)
+                    t, w = _ints(t), _ints(w)
                 r1 = r0 + hi - lo
                 toks[r0:r1] = t[lo:hi]
                 pos[r0:r1] = np.arange(s.n + lo, s.n + hi)
@@ -195,7 +197,6 @@ class SeqEngine:
                 prev[r0 + 1:r1] = t[lo:hi - 1]
                 batch[4 * R + 4 * e:4 * R + 4 * e + 4] = s.slot, r0, hi - lo, s.n + lo
                 if len(w):
-                    w = np.asarray(w, np.int32)
                     here = np.arange(len(w)) if lo == 0 and hi == len(t) else np.nonzero((w >= lo) & (w < hi))[0]
                     rows.append(w[here] + np.int32(r0 - lo))
                     dst.append(here + out_at[i])

@@ -1,10 +1,30 @@
 """Helpers shared by the GPU tests (not collected by pytest)."""
+import ctypes as C
+import functools
+import subprocess
+
 import numpy as np
 import torch
 
 from oracle.attention import v_slot
 
 PAGE = 16
+
+
+@functools.lru_cache(maxsize=None)
+def _symbols():
+    from vllm_omni_draft_amd import _lib
+    out = subprocess.run(["nm", "-D", "--defined-only", _lib.load()._name], capture_output=True, text=True, check=True).stdout
+    return [line.split()[-1] for line in out.splitlines()]
+
+
+def internal(name, restype, *argtypes):
+    """A C++ function of the library that the header does not declare, by its name (no two have one name)."""
+    from vllm_omni_draft_amd import _lib
+    (symbol,) = [s for s in _symbols() if s.startswith(f"_Z{len(name)}{name}")]
+    f = getattr(C.CDLL(_lib.load()._name), symbol)
+    f.restype, f.argtypes = restype, list(argtypes)
+    return f
 
 
 def pack_cache(k, v, block_table, num_pages):

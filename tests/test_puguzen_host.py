@@ -164,3 +164,20 @@ def test_single_tokens_beside_a_prompt_in_every_form_that_torch_takes():
     assert host.tolist() == [7, 4, 6, 8, 5, 0, 1, 2, 2, 1, 1, 1, 9, -1, 4, 6, 2, 0, 1, 5, 1, 1, 3, 0, 0, 3]
     with pytest.raises(RuntimeError):
         run(2 ** 40, 0)
+
+
+def test_the_activation_joins_the_stacked_product_where_that_is_the_quicker_way():
+    """Either side of the rule at sizes that were measured both ways (width, columns before and behind the pair, feed-forward
+    width, rows); a matrix whose up tiles lie 2 GiB behind their gate tiles never."""
+    import ctypes as C
+    from tests.gpu_util import internal
+    fits = internal("sd_prompt_relu_pair_fits_", C.c_bool, C.c_int, C.c_int, C.c_int, C.c_int64, C.c_int, C.c_int)
+    way = lambda W, front, rest, F, M: fits(M, (front + 2 * F + rest) // 16, W, W, front // 16, F)
+    for M, pair in ((257, False), (300, False), (512, False), (1024, True), (2048, True)):
+        assert way(1024, 6144, 0, 4096, M) == pair, M
+    for M, pair in ((257, False), (512, False), (1500, True), (2048, True)):
+        assert way(2048, 10240, 64, 8192, M) == pair, M
+    for M in (257, 300, 777, 2048):
+        assert not way(2048, 10240, 0, 1024, M) and way(4096, 20480, 0, 16384, M)
+    assert not way(2048, 10240, 0, 8192, 256)
+    assert way(8192, 8192, 0, 122880, 2048) and not way(8192, 8192, 0, 131072, 2048)

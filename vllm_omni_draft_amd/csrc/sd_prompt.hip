@@ -404,10 +404,10 @@ constexpr Shape kWholeShapes[] = {
     {8, 8, 1, 16.2f, 0.f, {1.236f}},      {7, 8, 1, 8.7f, 0.f, {1.295f}},  {8, 6, 1, 12.3f, 0.f, {1.023f}},
     {4, 4, 2, 4.1f, 0.f, {.813f, .958f}}, {4, 4, 1, 5.8f, 0.f, {.477f}},   {4, 6, 1, 8.9f, 0.f, {.562f}}};
 
-float shape_us(const Shape& s, const PromptArgs& a, int S) {
-  const long blocks = (long)((a.n_tiles + 2 * s.tn - 1) / (2 * s.tn)) * ((a.M + 32 * s.tm - 1) / (32 * s.tm));
+float shape_us(const Shape& s, int M, int n_tiles, int K, int S) {
+  const long blocks = (long)((n_tiles + 2 * s.tn - 1) / (2 * s.tn)) * ((M + 32 * s.tm - 1) / (32 * s.tm));
   const long round = 256l * s.per_cu, full = blocks / round, rest = blocks - full * round;
-  const float fixed = s.fixed + s.split * S, stages = a.KS * .5f;
+  const float fixed = s.fixed + s.split * S, stages = K / 64;
   float us = full * (fixed + s.stage[s.per_cu - 1] * stages);
   if (rest) {
     // blocks a CU of the last round, which starts as the one before it ends here and there
@@ -417,19 +417,33 @@ float shape_us(const Shape& s, const PromptArgs& a, int S) {
   return us;
 }
 
+// pair: gate and up tiles in one block, an even number of tiles a wave
 template <int N>
-int best_shape(const Shape (&shapes)[N], const PromptArgs& a, int S, bool even) {
+const Shape& best_shape(const Shape (&shapes)[N], int M, int n_tiles, int K, int S, bool pair, float& us) {
   int best = 0;
-  for (int i = 1; i < N; ++i)
-    if ((!even || shapes[i].tn % 2 == 0) && shape_us(shapes[i], a, S) < shape_us(shapes[best], a, S)) best = i;
-  return best;
+  us = shape_us(shapes[0], M, n_tiles, K, S);
+  for (int i = 1; i < N; ++i) {
+    if (pair && shapes[i].tn % 2) continue;
+    const float t = shape_us(shapes[i], M, n_tiles, K, S);
+    if (t < us) us = t, best = i;
+  }
+  return shapes[best];
+}
+const Shape& best_shape(int M, int n_tiles, int K, int S, bool pair, float& us) {
+  return S == 1 ? best_shape(kWholeShapes, M, n_tiles, K, S, pair, us) : best_shape(kSplitShapes, M, n_tiles, K, S, pair, us);
+}
+
+int shape_number(int M, int n_tiles, int K, int S, bool pair) {
+  float us;
+  const Shape& s = best_shape(M, n_tiles, K, S, pair, us);
+  return s.tn * 100 + s.tm * 10 + s.per_cu;
 }
 
 template <int EPI>
 int prompt_shape(const PromptArgs& a, int S, hipStream_t st) {
   constexpr bool even = EPI == EPI_RELU_PAIR;
-  const Shape& s = S == 1 ? kWholeShapes[best_shape(kWholeShapes, a, S, even)] : kSplitShapes[best_shape(kSplitShapes, a, S, even)];
-  switch (s.tn * 100 + s.tm * 10 + s.per_cu) {
+  const int shape = shape_number(a.M, a.n_tiles, a.KS * 32, S, even);
+  switch (shape) {
     case 881: return launch_prompt<8, 8, 2, false, EPI, 2>(a, st);
     case 781:
       if constexpr (!even) return launch_prompt<7, 8, 2, false, EPI, 2>(a, st);
@@ -445,11 +459,19 @@ int prompt_shape(const PromptArgs& a, int S, hipStream_t st) {
     case 461: return launch_prompt<4, 6, 4, true, EPI>(a, st);
     case 481: return launch_prompt<4, 8, 3, true, EPI>(a, st);
   }
-  sd_set_error("sd_prompt_linear: no kernel of %d x %d tiles", s.tn, s.tm);
+  sd_set_error("sd_prompt_linear: no kernel of shape %d", shape);
   return SD_ERR_UNSUPPORTED;
 }
 
 }  // namespace
+
+// The block that a product of `n_tiles` of a matrix's `all_tiles` takes, tn * 100 + tm * 10 + blocks a CU, and 1000 where K
+// is split (tests ask whether their sizes reach every block).
+int sd_prompt_shape_(int M, int n_tiles, int all_tiles, int K, bool pair) {
+  int S, ksp, g;
+  plan_split(all_tiles, K, S, ksp, g);
+  return shape_number(M, n_tiles, K, S, pair) + (S > 1 ? 1000 : 0);
+}
 
 bool sd_prompt_linear_fits_(int M, int n_tiles, int K, int64_t ldx) {
   // 256 rows are one pass of the kernels for fewer.  A block takes a long K's time however few blocks there are, and two or
@@ -525,6 +547,29 @@ int sd_prompt_linear_(const void* W, const void* x, int64_t ldx, int M, int K, i
 // `gate_tile`): act = bf16(relu(gate) * up) from one launch, the other columns f32 into y from one or two.  Against all columns
 // in f32 and sd_relu_mul_rows (2048 rows of 2048 columns, 10240 or 14336 + 2 x 8192 outputs, us): 222 and 238 + 37 -> 108 + 90 and
 // 108 + 109, the f32 stores of gate and up and their reads gone.  The splits of K are those of the whole matrix: so are the sums' bits.
+//
+// Two launches more are longer than that where they leave CUs without a block: the modelled times decide (sd_relu_mul_rows: 3 us
+// and 4.5 TB/s), with a margin for what the model is off.  us of product and activation, all columns in f32 / this way: 10240 + 2 x
+// 8192 outputs of 2048 columns 257 rows 54 / 51, 512 68 / 70, 1024 125 / 104, 2048 250 / 201; with 64 columns behind the pair 54 / 65, 66 / 87,
+// 127 / 119, 247 / 214; 6144 + 2 x 4096 of 1024 columns 22 / 26, 29 / 32, 54 / 45, 100 / 81; 10240 + 2 x 1024 of 2048 30 / 33, 46 / 42, 77 / 71,
+// 122 / 125.  Of 90 such measurements the rule takes no slower way than all columns in f32, and is 1.6 % behind the better one.
+bool sd_prompt_relu_pair_fits_(int M, int n_tiles, int K, int64_t ldx, int gate_tile, int F) {
+  if (!sd_prompt_linear_fits_(M, n_tiles, K, ldx)) return false;
+  if ((int64_t)(F / 16 + 16) * K * 32 >= 0x7fffffff) return false;   // (an up tile's byte offset from its gate tile is an int)
+  int S, ksp, g;
+  plan_split(n_tiles, K, S, ksp, g);
+  const int rest = n_tiles - gate_tile - F / 8;
+  float whole, pair, us;
+  best_shape(M, n_tiles, K, S, false, whole);
+  best_shape(M, F / 8, K, S, true, pair);
+  for (const int tiles : {gate_tile, rest}) {
+    if (tiles <= 0) continue;
+    best_shape(M, tiles, K, S, false, us);
+    pair += us;
+  }
+  return 1.08f * pair < whole + 3.f + (float)M * F * (10 / 4.5e6f);
+}
+
 int sd_prompt_relu_pair_(const void* W, const void* x, int64_t ldx, int M, int K, int n_tiles, int gate_tile, int F, float* y,
                          int64_t ldy, void* act, sd_stream_t stream) {
   int S, ksp, g;

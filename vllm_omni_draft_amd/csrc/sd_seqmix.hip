@@ -2358,7 +2358,8 @@ extern "C" int sd_seq_model_forward(sd_seq_model* m, const sd_seq_batch* b, void
     // every matrix that reads h, in one product: q k v g | residual gates | ff gate, up | low-rank decay
     // (many rows: the feed-forward's activation comes out of the product itself)
     const bool act_done = l.w_in_tiled && l.ff > 0 && l.w_down_tiled && sd_aligned16(l.w_in_tiled) && sd_aligned16(hb) &&
-                          (c.gate | l.ff | c.total) % 16 == 0 && W % 8 == 0 && sd_prompt_linear_fits_(R, c.total / 16, W, W);
+                          (c.gate | l.ff | c.total) % 16 == 0 && W % 8 == 0 &&
+                          sd_prompt_relu_pair_fits_(R, c.total / 16, W, W, c.gate / 16, l.ff);
     if (act_done)
       SQ_TRY(sd_prompt_relu_pair_(l.w_in_tiled, hb, W, R, W, c.total / 16, c.gate / 16, l.ff, proj, ld, actb, stream));
     else

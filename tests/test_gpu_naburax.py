@@ -760,6 +760,28 @@ def test_moe_experts_in_tiles_of_192_rows_have_the_bits_of_few(act):
         assert torch.equal(a, ops.moe_experts(x, sel, sel_w, gu, dn, True, act)), full
 
 
+@pytest.mark.parametrize("act", ["silu", "relu2"])
+def test_moe_experts_in_tall_tiles_of_many_experts(act):
+    """The same where the rule takes tall tiles: 128 assignments an expert over 64 experts, columns and k that end inside a
+    tile of either product, groups of one to six tall tiles."""
+    import ctypes as C
+    from tests.gpu_util import internal
+    from vllm_omni_draft_amd import ops
+    E, F, W, n = 64, 552, 416, 4096
+    tall = internal("sd_moe_tall_", C.c_bool, *[C.c_int] * 5)
+    assert tall(2 * n, E, F, W, 0 if act == "silu" else 1)
+    g = torch.Generator(device="cuda").manual_seed(8)
+    x = torch.randn(n, W, generator=g, device="cuda")
+    gu = (torch.randn(E, (1 if act == "relu2" else 2) * F, W, generator=g, device="cuda") * 0.1).to(torch.bfloat16)
+    dn = (torch.randn(E, W, F, generator=g, device="cuda") * 0.1).to(torch.bfloat16)
+    sel_w = torch.rand(n, 2, generator=g, device="cuda")
+    for full in (1000, 193, 192, 17):   # assignments of expert 0; the last expert is never chosen
+        sel = torch.randint(1, E - 1, (n, 2), generator=g, device="cuda", dtype=torch.int32)
+        sel[:full, 0] = 0
+        a = ops.moe_experts(x, sel, sel_w, gu, dn, True, act, bf16_copy=True)
+        assert torch.equal(a, ops.moe_experts(x, sel, sel_w, gu, dn, True, act)), full
+
+
 @pytest.mark.parametrize("H,G,dk,dv,maps", [(16, 1, 576, 512, 1), (8, 1, 584, 8, 1), (6, 2, 128, 128, 1), (12, 2, 256, 40, 2)])
 @pytest.mark.parametrize("extras", [False, True])
 def test_decode_attention_from_lds_against_float64(H, G, dk, dv, maps, extras):

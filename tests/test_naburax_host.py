@@ -172,3 +172,13 @@ def test_routing_takes_the_largest_scores_and_scales_the_input():
     inside = W[f"e{e}.down"] @ (N.silu(W[f"e{e}.gate"] @ (s[t, e] * h[t])) * (W[f"e{e}.up"] @ (s[t, e] * h[t])))
     outside = s[t, e] * (W[f"e{e}.down"] @ (N.silu(W[f"e{e}.gate"] @ h[t]) * (W[f"e{e}.up"] @ h[t])))
     assert not torch.allclose(inside, outside, atol=1e-6)
+
+
+@pytest.mark.parametrize("E,F,W,rows,tall", [(16, 2048, 2048, 128, True), (16, 2048, 2048, 100, False), (8, 4096, 4096, 512, True), (16, 1024, 2048, 200, False),
+                                             (16, 1024, 2048, 256, True), (4, 4096, 1024, 200, False), (4, 4096, 1024, 1024, True),
+                                             (8, 1024, 1024, 384, False), (2, 8192, 2048, 256, False), (2, 2048, 1024, 1024, False)])
+def test_tall_expert_tiles_only_where_they_are_quicker(E, F, W, rows, tall):
+    """Either side of the rule at sizes that were measured both ways: rows an expert."""
+    import ctypes as C
+    from tests.gpu_util import internal
+    assert internal("sd_moe_tall_", C.c_bool, *[C.c_int] * 5)(rows * E, E, F, W, 0) == tall

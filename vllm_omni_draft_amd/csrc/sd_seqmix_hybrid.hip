@@ -2707,6 +2707,20 @@ extern "C" int sd_moe_experts(const float* x, const void* x_bf16, int64_t ldx, c
                                 W, scale_input, act_kind, 0.f, scratch, scratch_bytes, stream);
 }
 
+// Whether n assignments go in tiles of 192 rows of an expert instead of 64 (each tile reads the expert's weights again): where an
+// expert's rows would be two tiles of 64 and often three, and the tall tiles of either product are blocks for most of the chip;
+// not between one tall tile and one and a quarter, where many an expert has a second one that is nearly empty, unless
+// there are blocks for several rounds.  us of the call with tiles of 64 / 192, experts x F x W: 16 x 2048 x 2048 128 rows an expert 164 /
+// 153, 256 242 / 202, 512 406 / 330; 8 x 4096 x 4096 128 277 / 241, 512 702 / 534; 16 x 1024 x 2048 128 89 / 80, 200 101 / 106, 256 132 / 117; 64 x 512
+// x 1024 128 124 / 111, 180 161 / 172, 256 206 / 202; but 4 x 4096 x 1024 200 68 / 96, 512 118 / 124, 1024 214 / 182; 8 x 1024 x 1024 128 38 / 55,
+// 384 63 / 75, 512 83 / 81; 2 x 2048 x 1024 1024 63 / 82.  Of 190 such sizes the rule loses 3 % against tiles of 64 in one, and is .4 %
+// behind the better of the two.  Tiles of 128 lie between; three and four stages (a block a CU) are slower than two.
+bool sd_moe_tall_(int n, int E, int F, int W, int act_kind) {
+  const int rows_e = n / E, cols = act_kind != 1 ? kMoeCols / 2 : kMoeCols;
+  const long up = (long)((F + cols - 1) / cols) * n / kMoeTallBM, down = (long)((W + kMoeCols - 1) / kMoeCols) * n / kMoeTallBM;   // blocks
+  return rows_e >= 112 && up >= 160 && down >= 160 && up + down >= 360 && (rows_e <= 160 || rows_e >= 240 || up >= 600);
+}
+
 extern "C" int sd_moe_experts_clamped(const float* x, const void* x_bf16, int64_t ldx, const int32_t* sel_expert,
                                       const float* sel_weight, const void* w_gate_up, const void* w_down, int w_f32,
                                       float* out, int n_rows, int top, int E, int F, int W, int scale_input, int act_kind,
@@ -2736,12 +2750,7 @@ extern "C" int sd_moe_experts_clamped(const float* x, const void* x_bf16, int64_
   const int n = n_rows * top;
   const bool lds_rows = mfma && x_bf16 && n > kMoeDirect && sd_aligned16(out) && x_bytes < kOutside &&
                         act_bytes < kOutside && gu_bytes < kOutside && down_bytes < kOutside;
-  // Tiles of 192 rows where an expert's rows would be two tiles of 64 and often three (each reads its weights again), and
-  // there are blocks for the chip: us of the call with tiles of 64 / 192, 2 experts a row, 16 experts 2048 x 2048: 777 rows
-  // (97 an expert) 129 / 134, 1024 156 / 135, 2048 230 / 188; 8 experts 1024 x 1024: 1024 rows 57 / 64 (256 blocks), 2048
-  // 82 / 77 (384).  Tiles of 128 lie between the two; three and four stages (a block a CU) are slower than two from 1024 rows on.
-  const int rows_e = n / E, cols = act_kind != 1 ? kMoeCols / 2 : kMoeCols;
-  const bool tall = lds_rows && rows_e >= 112 && (long)((F + cols - 1) / cols) * E * ((rows_e + 191) / 192) >= 384;
+  const bool tall = lds_rows && sd_moe_tall_(n, E, F, W, act_kind);
   const int bm = tall ? kMoeTallBM : lds_rows ? kMoeLdsBM : kMoeBM;
   int tiles_y = n;
   if (n <= kMoeDirect) {   // a few assignments: each runs as a tile of its own, straight from the router's choice

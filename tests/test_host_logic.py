@@ -569,3 +569,15 @@ def test_a_refused_step_loses_no_tokens():
     assert eng.steps == 0 and eng.active == 1
     out = w.execute_model(ExecuteModelRequest([R("a"), P("b", [2, 2])]))
     assert out.sampled_token_ids == [[101], [200]] and eng.steps == 1
+
+
+@pytest.mark.parametrize("M,n_tiles,K,fp8,two", [(6, 384, 4096, True, False), (7, 384, 4096, True, True), (7, 384, 4096, False, True), (7, 1792, 4096, True, True),
+                                                 (7, 1792, 4096, False, False), (16, 1792, 4096, False, True), (16, 256, 4096, True, False),
+                                                 (3, 640, 8192, False, False), (7, 640, 8192, True, False), (7, 3584, 8192, False, True),
+                                                 (9, 2368, 3584, False, True), (8, 2368, 3584, False, False), (15, 8016, 2048, True, True)])
+def test_two_tiles_a_workgroup_only_where_rounds_of_pairs_are_shorter(M, n_tiles, K, fp8, two):
+    """Either side of the rule at sizes that were measured both ways: rows that leave room for one workgroup a CU, and rounds of
+    pairs over the chip against rounds of tiles."""
+    import ctypes as C
+    from tests.gpu_util import internal
+    assert internal("sd_linear_two_tiles_", C.c_bool, C.c_int, C.c_int, C.c_int, C.c_bool)(M, n_tiles, K, fp8) == two

@@ -21,6 +21,9 @@ void sd_set_error(const char* fmt, ...);
 // True if sd_norm_linear / sd_norm_qkv_rope can hold M normalised rows of K columns in LDS.
 bool sd_fused_norm_fits(int M, int K, bool layer_norm);
 
+// Whether the fused-RMS-norm linear kernel works on two tiles a workgroup (tile 2 i and 2 i + 1 of workgroup i).
+bool sd_linear_two_tiles_(int M, int n_tiles, int K, bool fp8);
+
 // Weight ranges that the idle compute units of an attention launch read ahead of the launches
 // that stream them (extra workgroups behind the attention grid): a matrix in 16-row tiles of
 // tile_bytes, its first n_units work units (tiles, or half tiles: the 128-byte halves of every

@@ -707,14 +707,27 @@ int launch_g(LinArgs& a, hipStream_t st) {
   return SD_OK;
 }
 
+}  // namespace
+
 // Rows whose norm is staged for one workgroup a CU only (7 or more of K 4096) leave half of the waves' places empty: two
-// tiles a workgroup then, where there are more tiles than CUs.  fp8 weights, us with one / two tiles a workgroup, 8 and 16
-// rows: gate and up of 14336 x 4096 27.2 / 24.3, 29.8 / 27.5; 6144 x 4096 11.4 / 10.7, 14.0 / 11.9.
+// tiles a workgroup then, unless that takes more of the chip's time.  A round of 256 pairs is as long as 1.6 rounds of tiles with
+// fp8 weights and 1.85 with bf16 ones, whose products take more of it; above eight rows, which eight waves stage in two
+// turns, one tile a workgroup is .4 rounds longer.  us, one / two tiles a workgroup, 8 and 16 rows: gate and up of 14336 x 4096 (7
+// rounds of tiles, 4 of pairs) fp8 27.0 / 24.6, 30.4 / 27.2, bf16 40.1 / 40.8, 44.1 / 43.3; 6144 x 4096 (2 and 1) fp8 10.9 / 9.6, 14.0 / 11.9,
+// bf16 14.1 / 13.0, 17.2 / 15.2; head of 128256 x 4096 (32 and 16) bf16 168 / 162, 176 / 168; gate and up of 18944 x 3584 (10 and 5) at 9
+// and 16 rows bf16 48.1 / 46.3, 49.0 / 48.0; 10240 x 8192 (3 and 2) at 3 and 7 rows fp8 21.8 / 22.6, 23.0 / 23.9, bf16 33.0 / 37.2, 34.8 / 38.4.
+bool sd_linear_two_tiles_(int M, int n_tiles, int K, bool fp8) {
+  const size_t lds = lin_lds_bytes(M, choose_kc(M, K, NORM_RMS), NORM_RMS);
+  if (lds * 2 <= 160 * 1024 || lds > 160 * 1024 || n_tiles <= 256) return false;
+  const long one = 20 * (long)((n_tiles + 255) / 256) + (M > kLinWaves ? 8 : 0), two = (n_tiles + 511) / 512;
+  return (fp8 ? 32 : 37) * two <= one;
+}
+
+namespace {
 template <int EPI, int NORM, bool HALF, bool W8>
 int launch_w(LinArgs& a, hipStream_t st) {
   if constexpr (NORM == NORM_RMS) {
-    const size_t lds = lin_lds_bytes(a.M, a.KC, NORM);
-    if (lds * 2 > 160 * 1024 && lds <= 160 * 1024 && a.n_tiles > 256) return launch_g<EPI, NORM, HALF, W8, 2>(a, st);
+    if (sd_linear_two_tiles_(a.M, a.n_tiles, a.K, W8)) return launch_g<EPI, NORM, HALF, W8, 2>(a, st);
   }
   // fp8 weights of a long K, a tile a CU: a segment's x is up to twice its weights, and one segment a wave in flight does
   // not cover its way from L2.  4096 x 14336, us with one / two segments in flight: 4 rows 12.9 / 12.9, 8 15.2 / 14.2,

@@ -581,3 +581,26 @@ def test_two_tiles_a_workgroup_only_where_rounds_of_pairs_are_shorter(M, n_tiles
     import ctypes as C
     from tests.gpu_util import internal
     assert internal("sd_linear_two_tiles_", C.c_bool, C.c_int, C.c_int, C.c_int, C.c_bool)(M, n_tiles, K, fp8) == two
+
+
+@pytest.mark.parametrize("M,N,K,fp8", [(6, 14336, 4096, 1), (16, 14336, 4096, 1), (8, 14336, 4096, 0), (16, 14336, 4096, 0), (16, 18952, 3584, 1)])
+def test_weights_are_read_ahead_into_the_l2_of_the_chiplet_that_reads_them(M, N, K, fp8):
+    """Gate and up behind a fused norm: tile t is read by workgroup t, or t / 2 where a workgroup takes two tiles, and
+    workgroups go round the eight chiplets; the read-ahead takes unit u to chiplet u % 8, and stays inside the matrix."""
+    import ctypes as C
+    from tests.gpu_util import internal
+
+    class Range(C.Structure):
+        _fields_ = [("base", C.c_void_p), ("tile_bytes", C.c_uint), ("n_units", C.c_uint), ("half", C.c_uint), ("consumer_grid", C.c_uint)]
+
+    two = internal("sd_linear_two_tiles_", C.c_bool, C.c_int, C.c_int, C.c_int, C.c_bool)
+    ahead = internal("sd_linear_pf_range", Range, C.c_void_p, *[C.c_int] * 7, C.c_size_t)
+    tiles, tile = N // 8, 16 * K * (1 if fp8 else 2)
+    group = 2 if two(M, tiles, K, bool(fp8)) else 1
+    grid = min(tiles // group, 256 if group == 2 else 512)
+    for cap in (1 << 40, 24 << 20, tile - 1):
+        r = ahead(1 << 20, M, N, K, 2, fp8, 1, 1, cap)   # (the gated epilogue)
+        assert (r.half, r.consumer_grid) == (0, grid) and r.n_units * r.tile_bytes <= min(cap, tiles * tile)
+        for t in range(r.n_units * r.tile_bytes // tile):
+            assert t * tile // r.tile_bytes % 8 == t // group % grid % 8, t
+    assert ahead(1 << 20, M, N, K, 2, fp8, 1, 1, 1 << 40).n_units == tiles // group

@@ -793,20 +793,22 @@ int launch_n(LinArgs& a, int epi, hipStream_t st) {
 
 }  // namespace
 
-// Mirrors launch_one / launch_w: which units the launch's workgroups ask for first.
-sd_pf_range sd_linear_pf_range(const void* W, int N, int K, int epi, int fp8, int fused_norm,
+// Mirrors launch_one / launch_w: which units the launch's workgroups ask for first.  Two tiles a workgroup: a pair is one unit (the
+// last tile of an odd number is left to its workgroup).
+sd_pf_range sd_linear_pf_range(const void* W, int M, int N, int K, int epi, int fp8, int fused_norm, int rms,
                                size_t max_bytes) {
   const bool paired = epi == SD_EPI_SILU_MUL || epi == EPI_QKV_ROPE;
   const int n_tiles = paired ? (N + 7) / 8 : (N + 15) / 16;
   const bool half = !paired && !fused_norm && n_tiles < 256;  // as launch_one decides
-  const unsigned tile_bytes = (unsigned)(16 * (size_t)K * (fp8 ? 1 : 2));
-  const unsigned n_units = half ? 2 * n_tiles : n_tiles;
-  const unsigned unit_bytes = half ? tile_bytes / 2 : tile_bytes;
+  const bool two = fused_norm && rms && sd_linear_two_tiles_(M, n_tiles, K, fp8);
+  const unsigned tile_bytes = (unsigned)(16 * (size_t)K * (fp8 ? 1 : 2)) * (two ? 2 : 1);
+  const unsigned n_units = half ? 2 * n_tiles : two ? n_tiles / 2 : n_tiles;
+  const unsigned unit_bytes = half ? tile_bytes / 2 : tile_bytes, grid = two ? 256 : 512;
   sd_pf_range r;
   r.base = W;
   r.tile_bytes = tile_bytes;
   r.half = half;
-  r.consumer_grid = n_units < 512 ? n_units : 512;
+  r.consumer_grid = n_units < grid ? n_units : grid;
   const size_t cap = max_bytes / unit_bytes;
   r.n_units = (unsigned)(cap < n_units ? cap : n_units);
   return r;

@@ -275,6 +275,24 @@ def test_fp8_two_segments_in_flight_are_the_bf16_kernel(M, K):
         assert torch.equal(ops.linear(Wt, x, None, r, epi), ops.linear(exact, x, None, r, epi)), epi
 
 
+@pytest.mark.parametrize("M", [1, 6, 7, 16])
+@pytest.mark.parametrize("K", [256, 768, 2048, 2304, 4864])
+def test_fp8_two_segments_in_flight_for_halved_and_whole_tiles(M, K):
+    """1 to 19 segments of K over eight waves: halved tiles (one, and 125 with a remainder), 313 and 512 whole ones, 513 (which
+    keep one segment in flight), and 448 gated ones, in every epilogue of the halved ones."""
+    ops = _ops()
+    gen = torch.Generator(device="cuda").manual_seed(M + K)
+    x = torch.randn(M, K, generator=gen, device="cuda").to(torch.bfloat16)
+    sizes = [(9, ops.EPI_F32), (1990, ops.EPI_STORE), (1990, ops.EPI_RESIDUAL), (1990, ops.EPI_RELU), (1990, ops.EPI_GELU_TANH), (5000, ops.EPI_RESIDUAL),
+             (8192, ops.EPI_STORE), (8193, ops.EPI_F32), (3584, ops.EPI_SILU_MUL)]
+    for N, epi in sizes:
+        rows = 2 * N if epi == ops.EPI_SILU_MUL else N
+        q, sc, exact = _fp8_pow2((torch.randn(rows, K, generator=gen, device="cuda") * K ** -0.5).to(torch.bfloat16))
+        Wt = ops.tile_weights(q, ops.TILE_GATED if epi == ops.EPI_SILU_MUL else ops.TILE_PLAIN, scale=sc)
+        r = torch.randn(M, N, generator=gen, device="cuda").to(torch.bfloat16) if epi == ops.EPI_RESIDUAL else None
+        assert torch.equal(ops.linear(Wt, x, None, r, epi), ops.linear(exact, x, None, r, epi)), (N, epi)
+
+
 def test_fp8_linear_general_scales_and_quantisation_error():
     """Arbitrary per-row scales: the f32 output is exactly (sum over the fp8 values) * scale,
     and the quantised layer stays within e4m3's relative step of the bf16 layer."""

@@ -103,7 +103,7 @@ __device__ unsigned long long sd_lin_stamps[16];
 // (the layer is bound by the weight stream, so the conversion is free and activations keep
 // bf16); the f32 scale of an output row multiplies its finished sum.
 // G: tiles a workgroup works on at a time, eight waves each; all of them read one staged x.
-// DEEP: two segments of a wave in flight while a third is used (fp8 weights and x from memory, a workgroup's one tile).
+// DEEP: two segments of a wave in flight while a third is used (fp8 weights and x from memory, a workgroup's one unit).
 template <int EPI, int NORM, bool HALF, bool W8, int G, bool DEEP>
 __global__ __launch_bounds__(kLinThreads * G) void linear_kernel(LinArgs a) {
   LSTAMP(0);
@@ -729,11 +729,15 @@ int launch_w(LinArgs& a, hipStream_t st) {
   if constexpr (NORM == NORM_RMS) {
     if (sd_linear_two_tiles_(a.M, a.n_tiles, a.K, W8)) return launch_g<EPI, NORM, HALF, W8, 2>(a, st);
   }
-  // fp8 weights of a long K, a tile a CU: a segment's x is up to twice its weights, and one segment a wave in flight does
-  // not cover its way from L2.  4096 x 14336, us with one / two segments in flight: 4 rows 12.9 / 12.9, 8 15.2 / 14.2,
-  // 16 20.4 / 18.3.
-  if constexpr (NORM == NORM_NONE && W8 && !HALF) {
-    if (a.n_tiles <= 256 && a.K % 256 == 0 && a.K >= 24 * 256) return launch_g<EPI, NORM, HALF, W8, 1, true>(a, st);
+  // fp8 weights, one unit a workgroup: one segment a wave in flight does not cover the weights' way from memory where a unit is
+  // half a tile, nor that of x from L2 where there are 7 and more rows (a segment's x is up to twice its weights).  us with one / two
+  // segments in flight, 1 / 8 / 16 rows; halved: 3584 x 18944 25.3 / 25.0, 30.0 / 30.0, 43.8 / 40.9; 2048 x 8192 8.2 / 7.5, 9.5 / 8.4, 11.8 /
+  // 10.9; 3072 x 3072 7.6 / 7.1, 8.8 / 8.1, 10.7 / 9.9; 896 x 4864 5.7 / 5.4, 6.7 / 6.2, 8.2 / 7.6; 1024 x 512 3.3 / 3.0, 3.8 / 2.9, 4.4 / 3.1.
+  // Whole, 8 / 16 rows: 4096 x 14336 16.6 / 15.7, 20.8 / 18.2; 4096 x 2048 4.7 / 4.8, 5.4 / 5.1; 5120 x 13824 25.6 / 24.5, 37.1 / 33.0; 8000 x 2560 9.4 /
+  // 8.2, 10.9 / 10.1; gated 3584 x 8192 18.8 / 17.7, 24.0 / 21.8, 1000 x 8192 9.3 / 8.9, 12.6 / 11.2.  Of fewer rows gated ones lose (3584 x 4096
+  // at 6 rows 9.8 / 10.4), and so does 4096 x 14336 at 4 (14.1 / 14.4).
+  if constexpr (NORM == NORM_NONE && W8) {
+    if (a.K % 256 == 0 && (HALF ? 2 : 1) * a.n_tiles <= 512 && (HALF || a.M > 6)) return launch_g<EPI, NORM, HALF, W8, 1, true>(a, st);
   }
   return launch_g<EPI, NORM, HALF, W8, 1>(a, st);
 }

@@ -362,6 +362,43 @@ def test_causal_conv_rows_in_portions(C, taps):
     assert rel(torch.cat(outs), want) < 1e-6
 
 
+@pytest.mark.parametrize("wdt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("C,H,taps", [(5, 3, 4), (256, 300, 1), (300, 8, 2), (1000, 32, 7), (513, 16, 8), (40, 4, 9)])
+def test_convolution_and_steps_of_decoded_tokens_in_one_launch(C, H, taps, wdt):
+    """A row an entry, contexts shorter and longer than the taps, beside others' rows in a stack with the step sizes' columns:
+    outputs, moved tails, step sizes and decays are the bits of the launches apart (nine taps still take those); no argument of
+    theirs may be missing."""
+    import ctypes as Ct
+    from tests.gpu_util import internal
+    from vllm_omni_draft_amd import ops
+    vp, i32_, i64_ = Ct.c_void_p, Ct.c_int, Ct.c_int64
+    f = internal("sd_conv_steps_", i32_, vp, i64_, vp, vp, i32_, vp, vp, vp, vp, i32_, vp, i64_, i32_, i32_, i32_, i32_, vp, vp, vp, vp, vp,
+                 i32_, vp)
+    g = torch.Generator().manual_seed(C + taps)
+    pos = [0, 1, taps - 1, taps, 50]
+    R, ld = len(pos), C + H + 3
+    stack = dev(torch.randn(R, ld, generator=g))
+    w, b, dt_bias, a_log = (dev(torch.randn(*s, generator=g).to(wdt)) for s in ((C, taps), (C,), (H,), (H,)))
+    tails = dev(torch.randn(R + 2, max(taps - 1, 1), C, generator=g))
+    slots, entries = i32([4, 0, 6, 2, 3]), i32([[s, r, 1, p] for r, (s, p) in enumerate(zip([4, 0, 6, 2, 3], pos))])
+    p = lambda t: None if t is None else t.data_ptr()
+    for bias in (b, None):
+        tail, out = tails.clone(), torch.empty(R, C, device=DEV)
+        step, decay = torch.empty(R, H, device=DEV), torch.empty(R, H, device=DEV)
+        args = [p(stack), ld, p(w), p(bias), int(wdt == torch.float32), p(tail), None, p(slots), p(entries), R, p(out), C, R, C, taps, 1,
+                p(stack) + 4 * C, p(dt_bias), p(a_log), p(step), p(decay), H, ops._stream()]
+        rows = i32(pos)
+        args[6] = p(rows)
+        assert f(*args) == 0
+        tail2 = tails.clone()
+        out2 = ops.causal_conv_rows(stack[:, :C].contiguous(), w, bias, tail2, i32(pos), slots, entries)
+        step2, decay2 = ops.ssd_steps(stack[:, C:C + H].contiguous(), dt_bias, a_log)
+        for got, want in ((out, out2), (tail, tail2), (step, step2), (decay, decay2)):
+            assert torch.equal(got, want)
+    for at in (0, 2, 5, 6, 7, 8, 10, 16, 17, 18, 19, 20):
+        assert f(*[None if i == at else v for i, v in enumerate(args)]) == -1, at
+
+
 def ssd_reference(x, B, C, dt, a_log, dt_bias, D, S):
     """x [T, H, P], B, C [T, G, N], dt [T, H]; S [H, N, P] changed in place."""
     T, H, P = x.shape

@@ -2563,6 +2563,10 @@ int sd_conv_steps_(const float* x, int64_t ldx, const void* w, const void* b, in
                                        taps, act, stream);
     return rc != SD_OK ? rc : sd_ssd_steps(dt, ldx, dt_bias, a_log, w_f32, step, decay, n_rows, H, stream);
   }
+  // (what either of them asks for)
+  SD_REQUIRE(x && w && conv_state && row_pos && row_slot && entries && out && out != x && n_rows >= 1 && C >= 1 && taps >= 1 &&
+                 ldx >= C && ldo >= C && dt && dt_bias && a_log && step && decay && H >= 1 && ldx >= H,
+             SD_ERR_INVALID, "sd_seq_model_forward (convolution, steps): bad argument");
   const dim3 grid(n_rows, (C + 255) / 256 + 1);
   if (w_f32)
     conv_steps_decode_kernel<float><<<grid, 256, 0, (hipStream_t)stream>>>(

@@ -182,3 +182,21 @@ def test_tall_expert_tiles_only_where_they_are_quicker(E, F, W, rows, tall):
     import ctypes as C
     from tests.gpu_util import internal
     assert internal("sd_moe_tall_", C.c_bool, *[C.c_int] * 5)(rows * E, E, F, W, 0) == tall
+
+
+@pytest.mark.parametrize("name", ["head_prep", "window_pool_attention", "rows_pool_attention", "cache_append", "window_softmax_attention",
+                                  "rows_softmax_attention", "masked_softmax_attention", "qk_head_norm_append", "latent_kv_prep",
+                                  "multimap_softmax_attention", "attn_prep", "distance_softmax_attention", "conv_attn_prep",
+                                  "gated_softmax_attention", "biased_qkv_prep", "latent_prep", "qk_norm_append"])
+def test_caches_of_other_pages_are_refused(name):
+    """The kernels take the page size from the caller's side of the binding: a cache laid out in other pages is refused before
+    anything else is looked at (no launch, no tensor on a device)."""
+    import inspect
+    from vllm_omni_draft_amd import _lib, ops
+    f = getattr(ops, name)
+    for cache in ("k_cache", "v_cache"):
+        if cache in inspect.signature(f).parameters:
+            args = {p: None for p in inspect.signature(f).parameters}
+            args[cache] = torch.zeros(3, 1, 64, 8)
+            with pytest.raises(_lib.SdError, match="pages of 16 tokens"):
+                f(**args)

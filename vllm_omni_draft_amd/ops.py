@@ -1082,6 +1082,13 @@ def _f32(t: torch.Tensor, name: str) -> None:
     _need(t, torch.float32, name)
 
 
+def _paged(*caches) -> None:
+    """Caches [pages, heads, PAGE, width]: of other pages, the kernels would look past the block table."""
+    for c in caches:
+        if c is not None and c.dim() == 4 and c.shape[2] != PAGE:
+            raise _lib.SdError(f"a cache of pages of {PAGE} tokens, got {tuple(c.shape)}")
+
+
 def _wkind(w: torch.Tensor, name: str) -> int:
     if w.dtype not in (torch.float32, torch.bfloat16) or not w.is_contiguous():
         raise _lib.SdError(f"{name}: a contiguous float32 or bfloat16 tensor")
@@ -1117,6 +1124,7 @@ def head_prep(q, k, row_pos, Hq, Hk, dk, *, rot_dims=0, rot_layout=0, inv_freq=N
               eps=1e-5, q_scale=1.0, k_scale=1.0, v=None, dv=0, k_cache=None, v_cache=None, row_slot=None,
               block_tables=None) -> None:
     """In place on q [rows, Hq*dk] and k [rows, Hk*dk] (each contiguous); see sd_head_prep."""
+    _paged(k_cache, v_cache)
     _f32(q, "q")
     _f32(k, "k")
     n = q.shape[0]
@@ -1175,6 +1183,7 @@ def window_pool_attention(q, k_cache, v_cache, pk_cache, pv_cache, row_pos, row_
                           dk, dv, window, pool, scale, head_bias=None, split=True) -> torch.Tensor:
     """q f32 [rows, H*dk] (prepared); caches as kv_cache.SeqCache lays them out; returns f32
     [rows, H*dv].  Also fills the pooled entries of blocks that these rows complete."""
+    _paged(k_cache, v_cache)
     _f32(q, "q")
     out = torch.empty(q.shape[0], H * dv, dtype=torch.float32, device=q.device)
     lib = _lib.load()
@@ -1193,6 +1202,7 @@ def rows_pool_attention(q, k_cache, v_cache, pk_cache, pv_cache, block_tables, e
                         window, pool, scale, head_bias=None) -> torch.Tensor:
     """window_pool_attention for a prompt's rows over a bf16 cache, on the matrix cores; entries int32 [n, 4] {slot, first
     row, rows, first position}."""
+    _paged(k_cache, v_cache)
     _f32(q, "q")
     _need(k_cache, torch.bfloat16, "k_cache")
     out = torch.empty(q.shape[0], H * dv, dtype=torch.float32, device=q.device)
@@ -1272,6 +1282,7 @@ def rope_rows(x, row_pos, heads, head_stride, offset, rot_dims, inv_freq, mag=1.
 
 
 def cache_append(k, v, k_cache, v_cache, row_pos, row_slot, block_tables, G, dk, dv) -> None:
+    _paged(k_cache, v_cache)
     _f32(k, "k")
     _lib.check(_lib.load().sd_cache_append(_p(k), k.shape[1], _p(v), v.shape[1] if v is not None else 0, _p(k_cache),
                                            _p(v_cache), int(k_cache.dtype == torch.float32), _p(row_pos),
@@ -1284,6 +1295,7 @@ def window_softmax_attention(q, k_cache, v_cache, row_pos, row_slot, block_table
     """q f32 [rows, H*dk]; caches [pages, G, PAGE, dk | dv]; v_cache None: values are the first dv
     channels of the key rows.  Returns f32 [rows, H*dv].  split=False: never cut a row's keys
     over workgroups (few rows are cut by default)."""
+    _paged(k_cache, v_cache)
     _f32(q, "q")
     out = torch.empty(q.shape[0], H * dv, dtype=torch.float32, device=q.device)
     lib = _lib.load()
@@ -1301,6 +1313,7 @@ def rows_softmax_attention(q, k_cache, v_cache, block_tables, entries, H, G, dk,
                            scale) -> torch.Tensor:
     """window_softmax_attention for a prompt's rows over a bf16 cache, on the matrix cores; entries int32 [n, 4] {slot,
     first row, rows, first position}."""
+    _paged(k_cache, v_cache)
     _f32(q, "q")
     _need(k_cache, torch.bfloat16, "k_cache")
     out = torch.empty(q.shape[0], H * dv, dtype=torch.float32, device=q.device)
@@ -1316,6 +1329,7 @@ def masked_softmax_attention(q, k_cache, v_cache, row_pos, row_slot, block_table
     """window_softmax_attention with the further masks of sd_masked_softmax_attention: window 0
     sees every earlier token, chunk > 0 only the keys of the row's own chunk; softcap > 0 caps the
     scores; sinks f32 [H]: a term without key or value in every head's denominator."""
+    _paged(k_cache, v_cache)
     _f32(q, "q")
     if sinks is not None:
         _f32(sinks, "sinks")
@@ -1338,6 +1352,7 @@ def qk_head_norm_append(q, q_norm_w, k, k_norm_w, v, H, G, dk, dv, eps, k_cache,
     """In place on q f32 [rows, H*dk] and k f32 [rows, G*dk] (every head normed by itself, one
     weight [dk] for the query heads and one for the key heads); appends k and v f32 [rows, G*dv] to
     the caches.  See sd_qk_head_norm_append."""
+    _paged(k_cache, v_cache)
     for t, nm in ((q, "q"), (k, "k"), (v, "v")):
         _f32(t, nm)
     buf = torch.cat([q, k, v], dim=1).contiguous()
@@ -1355,6 +1370,7 @@ def latent_kv_prep(kv, kv_norm_w, kv_rank, rot_dim, eps, rot_dims, inv_freq, k_c
                    block_tables, mag=1.0, layout=1) -> None:
     """latent_prep for queries that have no latent: in place on kv f32 [rows, kv_rank + rot_dim],
     which is appended to k_cache."""
+    _paged(k_cache)
     _f32(kv, "kv")
     _lib.check(_lib.load().sd_latent_prep(None, 0, None, None, 0, _p(kv), kv_rank, rot_dim, _p(kv_norm_w), kv.shape[1],
                                           _wkind(kv_norm_w, "kv_norm_w"), float(eps), rot_dims, layout, _p(inv_freq),
@@ -1429,6 +1445,7 @@ def multimap_softmax_attention(q, k_cache, v_cache, row_pos, row_slot, block_tab
     """masked_softmax_attention with `maps` score maps per head: q f32 [rows, H*maps*dk], k_cache
     [pages, G*maps, PAGE, dk], v_cache [pages, G, PAGE, dv]; returns every map's own output, f32
     [rows, H*maps*dv].  sinks f32 [H*maps]."""
+    _paged(k_cache, v_cache)
     _f32(q, "q")
     if sinks is not None:
         _f32(sinks, "sinks")
@@ -1452,6 +1469,7 @@ def attn_prep(q, k, v, dk, G, dv, row_pos, row_slot, block_tables, k_cache, v_ca
     [rows, G*dv] (or None: the values are the keys after their bias).  norm: "none", "full" (over
     the whole projection) or "head" (per unit, one weight [dk]).  Returns the prepared (q, k);
     keys and values are appended to the caches, whose dtype is the weights'."""
+    _paged(k_cache, v_cache)
     _f32(q, "q")
     parts = [q] + ([k] if k is not None else []) + ([v] if v is not None else [])
     buf = torch.cat(parts, dim=1).contiguous()
@@ -1526,6 +1544,7 @@ def distance_softmax_attention(q, k_cache, v_cache, row_pos, row_slot, block_tab
     scores lose dist1[h] * ln(1 + dist2[h] * distance); q f32 [rows, H*dk] -> f32 [rows, H*dv], or, with
     ldo > H*dv, a view of rows that far apart; bf16_only: bfloat16 instead.  entries int32 [n, 4] (or
     None): the rows' portions, with which many rows over bfloat16 caches run on the matrix cores."""
+    _paged(k_cache, v_cache)
     _f32(q, "q")
     window, ldo = int(window) or 0x7fffffff, int(ldo) or H * dv
     dt = torch.bfloat16 if bf16_only else torch.float32
@@ -1598,6 +1617,7 @@ def conv_attn_prep(proj, conv_w, conv_state, H, G, dk, dv, q_norm_w, k_norm_w, e
     """sd_conv_attn_prep on proj f32 [rows, channels] (q | k | v; q alone when k_cache is None), conv_w [taps, channels]: returns
     the prepared q f32 [rows, H*dk]; keys and values are appended, conv_state moves on.  act (or
     None): (z, coef, bias or None, out), an activation of the same rows computed in the launch."""
+    _paged(k_cache, v_cache)
     _f32(proj, "proj")
     q = torch.empty(proj.shape[0], H * dk, dtype=torch.float32, device=proj.device)
     part = _poly_norm_part(*act) if act is not None else None
@@ -1688,6 +1708,7 @@ def gated_softmax_attention(q, k_cache, v_cache, row_pos, row_slot, block_tables
     """masked_softmax_attention whose heads' outputs are multiplied by sigmoid(gates f32 [rows, H]).  entries
     int32 [n, 4]: the rows' portions; many rows over bfloat16 caches then run on the matrix cores.
     ldo: elements between output rows; bf16_only: the result in bfloat16 alone."""
+    _paged(k_cache, v_cache)
     _f32(q, "q")
     for t, nm in ((sinks, "sinks"), (gates, "gates")):
         if t is not None:
@@ -1811,6 +1832,7 @@ def biased_qkv_prep(q, k, v, biases, G, dk, dv, q_norm_w, k_norm_w, eps, k_cache
     None.  Returns the prepared q (in place where q, k, v are columns of one buffer); keys and values go to
     the caches.  step: the arguments of
     decay_step_rows up to norm_w (and q_scale), whose result is then returned too."""
+    _paged(k_cache, v_cache)
     p, ld, parts = _side_by_side(q, k, v)
     nq = q.shape[1]
     y, s = None, None
@@ -1982,6 +2004,7 @@ def latent_prep(q_latent, q_norm_w, kv, kv_norm_w, kv_rank, rot_dim, eps, rot_di
                 row_pos, row_slot, block_tables, layout=1) -> None:
     """In place on q_latent f32 [rows, q_rank] and kv f32 [rows, kv_rank + rot_dim]; appends the
     finished kv rows to k_cache [pages, 1, PAGE, kv_rank + rot_dim].  See sd_latent_prep."""
+    _paged(k_cache)
     _f32(q_latent, "q_latent")
     _f32(kv, "kv")
     n = kv.shape[0]
@@ -2000,6 +2023,7 @@ def qk_norm_append(q, q_norm_w, k, k_norm_w, v, G, dk, dv, eps, k_cache, v_cache
                    block_tables) -> None:
     """In place on q f32 [rows, n_q] and k f32 [rows, G*dk] (each normed over all its columns);
     appends k and v f32 [rows, G*dv] to the caches.  See sd_qk_norm_append."""
+    _paged(k_cache, v_cache)
     for t, nm in ((q, "q"), (k, "k"), (v, "v")):
         _f32(t, nm)
     buf = torch.cat([q, k, v], dim=1).contiguous()

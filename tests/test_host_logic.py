@@ -604,3 +604,14 @@ def test_weights_are_read_ahead_into_the_l2_of_the_chiplet_that_reads_them(M, N,
         for t in range(r.n_units * r.tile_bytes // tile):
             assert t * tile // r.tile_bytes % 8 == t // group % grid % 8, t
     assert ahead(1 << 20, M, N, K, 2, fp8, 1, 1, 1 << 40).n_units == tiles // group
+
+
+@pytest.mark.parametrize("M,N,K,chained", [(49, 64, 2048, False), (160, 64, 2048, False), (256, 64, 2048, True), (64, 384, 2048, False), (100, 384, 2048, True),
+                                           (49, 1024, 2048, False), (64, 1024, 2048, True), (48, 8192, 2048, False), (50, 8192, 2048, True),
+                                           (49, 64, 1024, False), (64, 64, 1024, True), (24, 384, 1024, False), (33, 384, 1024, True),
+                                           (24, 13312, 1024, True), (23, 13312, 1024, False), (64, 8192, 2112, False)])
+def test_splits_are_chained_in_a_block_only_where_that_is_quicker(M, N, K, chained):
+    """Either side of the rule at sizes that were measured both ways (eight splits of K)."""
+    import ctypes as C
+    from tests.gpu_util import internal
+    assert internal("sd_rows_chain_fits_", C.c_bool, C.c_int, C.c_int, C.c_int, C.c_int64, C.c_int)(M, N // 16, K, K, 8) == chained

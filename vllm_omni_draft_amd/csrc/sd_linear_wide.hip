@@ -1098,7 +1098,7 @@ int wide_common(const void* W, const void* x, int64_t ldx, int M, int K, int n_t
     *normed = true;
     return SD_OK;
   };
-  if (!e.w_scale && sd_rows_chain_fits_(M, K, ldx, S))  // (the same bits)
+  if (!e.w_scale && sd_rows_chain_fits_(M, n_tiles, K, ldx, S))  // (the same bits)
     return sd_prompt_linear_(W, x, ldx, M, K, n_tiles, epi, e, st);
   if (!e.w_scale && sd_rows_linear_fits_(M, n_tiles, K, ldx, S, ksp, epi)) {  // (the same bits)
     const int rc = sd_rows_linear_(W, x, ldx, M, K, n_tiles, S, ksp, epi, e, (float*)workspace, st);

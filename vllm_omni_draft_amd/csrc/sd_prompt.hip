@@ -491,8 +491,12 @@ bool sd_prompt_linear_fits_(int M, int n_tiles, int K, int64_t ldx) {
 // 2048 12.1 / 12.0 / 12.3 / 12.3 against 11.2 / 11.9 / 12.8 / 14.0, 7552 x 2048 13.9 / 14.0 / 14.2 / 14.3 against 12.3 / 12.7 /
 // 13.3 / 14.1 (64: 14.6, 15.4); 1024 x 1024 7.6 / 7.6 / 7.8 / 7.8 against 7.4 / 8.0 / 8.2 / 8.8, 13312 x 1024 9.5 / 9.4 / 9.6 / 9.7
 // against 11.3 / 11.5 / 12.4 / 13.6.
-bool sd_rows_chain_fits_(int M, int K, int64_t ldx, int S) {
-  return S > 1 && M >= (K <= 1024 ? 24 : 49) && K <= 2048 && K % 64 == 0 && K >= 128 && 512 * ldx < 0x7fffffff;
+// A narrow matrix leaves that block alone on the chip while the splits' workgroups share its K, so it takes more rows: 64 x 2048
+// 49 / 100 / 160 rows 11.7 / 11.8 / 11.9 against 9.3 / 10.5 / 11.4; 384 x 2048 49 / 64 12.0 / 12.0 against 10.9 / 11.7; 1024 x 2048 49 12.5 against
+// 12.0; 64 x 1024 24 / 49 7.2 / 7.6 against 6.5 / 7.2, 384 x 1024 24 7.6 against 7.4.
+bool sd_rows_chain_fits_(int M, int n_tiles, int K, int64_t ldx, int S) {
+  return S > 1 && M >= (K <= 1024 ? 24 + 128 / n_tiles : 49 + 512 / n_tiles) && K <= 2048 && K % 64 == 0 && K >= 128 &&
+         512 * ldx < 0x7fffffff;
 }
 
 // At most 256 rows: the products themselves (splits of K: the partial sums, for the caller's epilogue kernel).  Against

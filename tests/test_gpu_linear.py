@@ -747,13 +747,18 @@ def test_prompt_linear_has_the_bits_of_the_wide_kernels(M, N, K):
             assert torch.equal(got, few), (epi, b is not None)
 
 
-@pytest.mark.parametrize("M,N,K", [
-    (65, 130, 192), (513, 6000, 192), (65, 12000, 2048), (130, 12000, 2048), (513, 6000, 2048), (321, 12000, 192),
-    (800, 6000, 704), (321, 12000, 2048), (400, 12000, 4096),                                      # K in splits
-    (65, 130, 128), (65, 16400, 704), (130, 16400, 1024), (400, 16400, 128), (257, 30000, 704), (400, 30000, 1024)])
-def test_every_block_shape_has_the_bits_of_few_rows(M, N, K):
+@pytest.mark.parametrize("M,N,K,shape", [
+    (65, 130, 192, 1223), (513, 6000, 192, 1422), (65, 12000, 2048, 1241), (130, 12000, 2048, 1431), (513, 6000, 2048, 1441),
+    (321, 12000, 192, 1442), (800, 6000, 704, 1451), (321, 12000, 2048, 1461), (400, 12000, 4096, 1481),   # K in splits
+    (65, 130, 128, 442), (65, 16400, 704, 441), (130, 16400, 1024, 461), (400, 16400, 128, 781), (257, 30000, 704, 861),
+    (400, 30000, 1024, 881)])
+def test_every_block_shape_has_the_bits_of_few_rows(M, N, K, shape):
     """One size per block shape of the prompt kernels (the first whose modelled time makes it the choice), with a last block
     of rows and of outputs that is not full: every row has the bits that it has among 48."""
+    import ctypes as C
+    from tests.gpu_util import internal
+    tiles = -(-N // 16)
+    assert internal("sd_prompt_shape_", C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_bool)(M, tiles, tiles, K, False) == shape
     ops = _ops()
     gen = torch.Generator(device="cuda").manual_seed(M + N + K)
     x = torch.randn(M, K, generator=gen, device="cuda").to(torch.bfloat16)
@@ -762,6 +767,36 @@ def test_every_block_shape_has_the_bits_of_few_rows(M, N, K):
     for epi, r in ((ops.EPI_F32, None), (ops.EPI_RESIDUAL, res)):
         few = torch.cat([ops.linear_wide(W, x[i:i + 48], None, None if r is None else r[i:i + 48], epi) for i in range(0, M, 48)])
         assert torch.equal(ops.linear_prompt(W, x, None, r, epi), few), epi
+
+
+@pytest.mark.parametrize("M", [17, 64, 192, 256])
+@pytest.mark.parametrize("N,K,splits", [(3584, 18944, 9), (4112, 6400, 7), (8192, 4096, 4), (960, 4352, 17), (16, 2176, 17)])
+@pytest.mark.parametrize("fp8,bias", [(False, False), (False, True), (True, True)])
+def test_norm_with_the_launch_that_adds_the_splits(M, N, K, splits, fp8, bias):
+    """The residual epilogue of a split matrix with the RMS norm behind it in one launch: one to three batches of eight splits,
+    rows of one to two trips over the columns (and of 16 columns), fp8 scales and a bias; the bits of the two launches."""
+    import ctypes as C
+    from tests.gpu_util import internal
+    from vllm_omni_draft_amd import _lib
+    ops, lib = _ops(), _lib.load()
+    vp, i32 = C.c_void_p, C.c_int
+    f = internal("sd_linear_wide_norm_", i32, vp, vp, vp, C.c_int64, vp, vp, vp, i32, i32, i32, vp, C.c_size_t, vp, C.c_float, vp, vp)
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=gen, device="cuda").to(torch.bfloat16)
+    W = (torch.randn(N, K, generator=gen, device="cuda") * K ** -0.5).to(torch.bfloat16)
+    q, sc = ops.quantize_fp8(W) if fp8 else (W, None)
+    W = ops.tile_weights(q, ops.TILE_PLAIN, scale=sc)
+    res, g, b = (torch.randn(*s, generator=gen, device="cuda").to(torch.bfloat16) for s in ((M, N), (N,), (N,)))
+    b = b if bias else None
+    need = int(lib.sd_linear_wide_workspace_bytes(M, N, K, ops.EPI_RESIDUAL))
+    assert need == splits * M * N * 4
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    p = lambda t: None if t is None else t.data_ptr()
+    out, normed, want = res.clone(), torch.empty_like(res), torch.empty_like(res)
+    assert f(p(W.data), p(W.scale), p(x), K, p(b), p(out), p(out), M, N, K, p(ws), need, p(g), 1e-5, p(normed), ops._stream()) == 0
+    apart = ops.linear_wide(W, x, b, res, ops.EPI_RESIDUAL)
+    assert lib.sd_rmsnorm(p(apart), N, p(g), p(want), N, M, N, 1e-5, ops._stream()) == 0
+    assert torch.equal(out, apart) and torch.equal(normed, want)
 
 
 @pytest.mark.parametrize("M", [65, 128, 129, 256])

@@ -39,6 +39,30 @@ sd_pf_range sd_linear_pf_range(const void* W, int M, int N, int K, int epi, int 
 // Applies to the next attention launch of this host thread (then forgotten); n <= 2.
 void sd_attn_prefetch_next(const sd_pf_range* r, int n);
 
+// ---- what the kernels share whose operands come into LDS by direct loads (16 bytes a lane, no registers)
+typedef __attribute__((address_space(3))) void lds_void;
+constexpr unsigned kOutside = 0x80000000u;   // (buffers are smaller: reads of zero)
+// (less than 4 GiB)
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, size_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (unsigned)bytes, 0x00027000);
+}
+// Barrier of the workgroup behind this wave's LDS reads and all but the newest LEFT of its direct loads
+// (__syncthreads() would wait for every load in flight in some places and for none in others: it does not count
+// direct loads as LDS writes).
+template <int LEFT>
+__device__ __forceinline__ void meet() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LEFT) : "memory");
+}
+// Workgroups go round the 8 XCDs in launch order.  Each XCD takes a contiguous run of the work list, in which eight
+// row blocks of one weight block are next to each other: the 32 or 64 blocks that an XCD runs at once then read
+// about as many different weight blocks as row blocks, the least bytes for its L2 (all row blocks of a weight block
+// next to each other: 963 TFLOP/s at 4096 rows of 14336, where 2048 rows reached 1197).
+constexpr int kRowGroup = 8;
+__device__ __forceinline__ int xcd_order(int id, int n) {
+  const int q = n >> 3, r = n & 7, x = id & 7, i = id >> 3;
+  return x * q + min(x, r) + i;
+}
+
 // Layer-list models whose matrices are tiled: a portion of a pass with more rows than this runs on kernels for many
 // rows, which sum in another order than those for few.  A portion's own rows decide, so that what shares its pass does
 // not change its bits (linear layers, which have one rule for passes of up to 16 rows and one for others, aside).

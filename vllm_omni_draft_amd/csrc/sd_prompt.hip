@@ -45,31 +45,8 @@ struct PromptArgs {
   WideEpiArgs epi;
 };
 
-typedef __attribute__((address_space(3))) void lds_void;
 constexpr int EPI_PARTIAL = -1;  // the sums of one split of K, for wide_epilogue_kernel
 constexpr int EPI_RELU_PAIR = -2;  // bf16(relu(gate) * up) of two ranges of tiles of a stacked matrix
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, unsigned bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00027000);
-}
-
-// Workgroups go round the 8 XCDs in launch order.  Each XCD takes a contiguous run of the work list, in which eight
-// row blocks of one weight block are next to each other: the 32 or 64 blocks that an XCD runs at once then read
-// about as many different weight blocks as row blocks, the least bytes for its L2 (all row blocks of a weight block
-// next to each other: 963 TFLOP/s at 4096 rows of 14336, where 2048 rows reached 1197).
-constexpr int kRowGroup = 8;
-__device__ __forceinline__ int xcd_order(int id, int n) {
-  const int q = n >> 3, r = n & 7, x = id & 7, i = id >> 3;
-  return x * q + min(x, r) + i;
-}
-
-// Barrier of the workgroup behind this wave's LDS reads and all but the newest LEFT of its direct loads
-// (__syncthreads() would wait for every load in flight in some places and for none in others: it does not count
-// direct loads as LDS writes).
-template <int LEFT>
-__device__ __forceinline__ void meet() {
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LEFT) : "memory");
-}
 
 // Tile t of a block, from its first one
 template <bool PAIR, int TN>
@@ -473,7 +450,7 @@ int sd_prompt_shape_(int M, int n_tiles, int all_tiles, int K, bool pair) {
   return shape_number(M, n_tiles, K, S, pair) + (S > 1 ? 1000 : 0);
 }
 
-bool sd_prompt_linear_fits_(int M, int n_tiles, int K, int64_t ldx) {
+bool sd_prompt_linear_fits_(int M, int K, int64_t ldx) {
   // 256 rows are one pass of the kernels for fewer.  A block takes a long K's time however few blocks there are, and two or
   // three passes split it over the chip; us against those passes, weights from memory, 264 / 300 / 384 / 512 / 640 / 768
   // rows: 4096 x 14336 72 / 74 / 90 / 92 / 111 / 120 against 68 / 70 / 77 / 88 / 123 / 132; 3584 x 18944 89 / 92 / 112 / 113
@@ -558,7 +535,7 @@ int sd_prompt_linear_(const void* W, const void* x, int64_t ldx, int M, int K, i
 // 127 / 119, 247 / 214; 6144 + 2 x 4096 of 1024 columns 22 / 26, 29 / 32, 54 / 45, 100 / 81; 10240 + 2 x 1024 of 2048 30 / 33, 46 / 42, 77 / 71,
 // 122 / 125.  Of 90 such measurements the rule takes no slower way than all columns in f32, and is 1.6 % behind the better one.
 bool sd_prompt_relu_pair_fits_(int M, int n_tiles, int K, int64_t ldx, int gate_tile, int F) {
-  if (!sd_prompt_linear_fits_(M, n_tiles, K, ldx)) return false;
+  if (!sd_prompt_linear_fits_(M, K, ldx)) return false;
   if ((int64_t)(F / 16 + 16) * K * 32 >= 0x7fffffff) return false;   // (an up tile's byte offset from its gate tile is an int)
   int S, ksp, g;
   plan_split(n_tiles, K, S, ksp, g);

@@ -38,8 +38,6 @@ struct PromptAttnArgs {
   float scale_log2;
 };
 
-typedef __attribute__((address_space(3))) void lds_void;
-
 constexpr int kTable = 1024;       // page numbers kept in LDS at a time
 constexpr int kRows = SD_PROMPT_BLOCK_ROWS;
 

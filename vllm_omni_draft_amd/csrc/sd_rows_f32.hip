@@ -9,9 +9,9 @@
 // over the chip.
 //
 // A stage of a row is 128 bytes, 8 pieces of 4 k; piece c of row r lies at slot c ^ (r & 7), which spreads the fragment
-// reads over the banks; the source address carries the permutation.  A lane reads whole pieces and takes the two values
-// that its half of the wave multiplies (even or odd k).  Rows past the matrix and k past K are out of the buffers' bounds
-// and arrive as zeros.
+// reads over the banks; the source address carries the permutation.  Lane (r, q) of a product multiplies k = 4 c + q of row r
+// of either operand: one value of piece c.  Rows past the matrix and k past K are out of the buffers' bounds and arrive as
+// zeros.
 //
 // us, both operands through registers into two LDS buffers before / now: 777 rows of 13312 x 1024 251 / 188, 32000 x 1024
 // 528 / 413 (123 TFLOP/s), 1024 x 4096 gated 122 / 98, 1024 x 1024 33 / 22; 300 rows of 13312 x 1024 166 / 87, 33 rows 35 / 23;
@@ -28,25 +28,7 @@ struct F32Args {
   int M, N, K, n_blocks, m_blocks;
 };
 
-typedef __attribute__((address_space(3))) void lds_void;
-constexpr unsigned kOutside = 0x80000000u;   // (buffers are smaller: reads of zero)
 constexpr int kRow = 128;                    // bytes of a row and stage
-
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, size_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (unsigned)bytes, 0x00027000);
-}
-
-template <int LEFT>
-__device__ __forceinline__ void meet() {
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LEFT) : "memory");
-}
-
-// Each XCD takes a contiguous run of the blocks, in which eight row blocks of a weight block are next to each other.
-constexpr int kRowGroup = 8;
-__device__ __forceinline__ int xcd_order(int id, int n) {
-  const int q = n >> 3, r = n & 7, x = id & 7, i = id >> 3;
-  return x * q + min(x, r) + i;
-}
 
 constexpr int stage_bytes(int nt, int mt, bool gated) { return (64 * nt + 64 * mt * (gated ? 2 : 1)) * kRow; }
 // as many as leave room for two blocks a CU (128 x 64 gated: one)

@@ -312,9 +312,8 @@ extern "C" int sd_model_forward(sd_model* m, const sd_kv_cache* kv, const sd_for
                               Hq * D, proj_epi, wws, w.wide_ws_bytes, stream));
       }
       if (d.allreduce) SD_TRY(d.allreduce(h, (size_t)rows * H, d.allreduce_ctx, stream));
-      if (norms) {
-      } else if (llama) SD_TRY(sd_rmsnorm(h, H, l.mlp_norm_w, xn, H, rows, H, d.norm_eps, stream));
-      else SD_TRY(sd_layernorm(h, H, l.mlp_norm_w, l.mlp_norm_b, xn, H, rows, H, d.norm_eps, stream));
+      if (llama && !norms) SD_TRY(sd_rmsnorm(h, H, l.mlp_norm_w, xn, H, rows, H, d.norm_eps, stream));
+      if (!llama) SD_TRY(sd_layernorm(h, H, l.mlp_norm_w, l.mlp_norm_b, xn, H, rows, H, d.norm_eps, stream));
       if (a8) {
         SD_TRY(sd_row_scales_fp8(xn, H, rows, H, xsc, stream));
         SD_TRY(sd_linear_wide_a8(l.up_w, l.up_s, xsc, xn, H, l.up_b, nullptr, act, F, rows, F, H,
@@ -430,9 +429,8 @@ extern "C" int sd_model_forward(sd_model* m, const sd_kv_cache* kv, const sd_for
   }
   const int lm_vocab = d.lm_vocab > 0 ? d.lm_vocab : d.vocab;
   if (a->logits && wide) {
-    if (normed) {
-    } else if (llama) SD_TRY(sd_rmsnorm(h, H, d.final_norm_w, xn, H, rows, H, d.norm_eps, stream));
-    else SD_TRY(sd_layernorm(h, H, d.final_norm_w, d.final_norm_b, xn, H, rows, H, d.norm_eps, stream));
+    if (llama && !normed) SD_TRY(sd_rmsnorm(h, H, d.final_norm_w, xn, H, rows, H, d.norm_eps, stream));
+    if (!llama) SD_TRY(sd_layernorm(h, H, d.final_norm_w, d.final_norm_b, xn, H, rows, H, d.norm_eps, stream));
     if (a->wide_a8 && llama && d.lm_head_s && H % 128 == 0) {
       float* xsc = reinterpret_cast<float*>(base + w.x_scales);
       SD_TRY(sd_row_scales_fp8(xn, H, rows, H, xsc, stream));

@@ -830,11 +830,11 @@ __global__ __launch_bounds__(256) void matmul_skinny_kernel(
 }
 
 // The same product with bf16 weights for more rows, on the f32 matrix instruction (f32 weights: sd_rows_f32.hip):
-// v_mfma_f32_32x32x2_f32 is two fused multiply-adds in ascending k for every element, so the sums are matmul_rows_kernel's to the bit (tests compare them).  Four waves, NT x
-// MT tiles of 32 x 32 each; 32 columns of K a stage, through registers into two LDS buffers.  A row's 32 values lie
-// as 16 of even k, then 16 of odd k: the lanes of an instruction's first k read the former, those of its second the
-// latter, four instructions' worth in one 16-byte read.  Bound by the matrix pipe (64 FLOP a clock and SIMD): 777 x
-// 13312 x 1024 ran at 20 TFLOP/s on the vector pipe, whose inner loop read as many LDS words as it multiplied.
+// v_mfma_f32_32x32x2_f32 is two fused multiply-adds in ascending k for every element, so the sums are matmul_rows_kernel's to the
+// bit (tests compare them).  Four waves, NT x MT tiles of 32 x 32 each; 32 columns of K a stage, through registers into two LDS
+// buffers.  A row's 32 values lie as 16 of even k, then 16 of odd k: the lanes of an instruction's first k read the former,
+// those of its second the latter, four instructions' worth in one 16-byte read.  Bound by the matrix pipe (64 FLOP a clock and
+// SIMD).  (f32 weights, 777 x 13312 x 1024: 20 TFLOP/s on the vector pipe, whose inner loop read as many LDS words as it multiplied.)
 constexpr int kMmK = 32, kMmLd = kMmK + 4;
 template <int NT, int MT>
 __global__ __launch_bounds__(256, 2) void matmul_mfma_kernel(
@@ -1613,7 +1613,7 @@ int seq_linear(const void* w_rm, const void* w_tiled, int w_f32, const float* x,
   SD_REQUIRE(!bias, SD_ERR_INVALID, "seq_linear: a tiled matrix takes no f32 bias");
   if (M <= 16) return sd_linear(w_tiled, nullptr, x_b, ldxb, nullptr, nullptr, y, ldy, M, N, K, SD_EPI_F32, stream);
   if (sd_aligned16(w_tiled) && sd_aligned16(x_b) && ldxb % 8 == 0 && ldxb >= K &&
-      sd_prompt_linear_fits_(M, tiles_of(N, SD_EPI_F32), K, ldxb))
+      sd_prompt_linear_fits_(M, K, ldxb))
     return sd_linear_prompt(w_tiled, x_b, ldxb, nullptr, nullptr, y, ldy, M, N, K, SD_EPI_F32, stream);
   for (int r0 = 0; r0 < M; r0 += kWideRows) {
     const int mm = M - r0 < kWideRows ? M - r0 : kWideRows;

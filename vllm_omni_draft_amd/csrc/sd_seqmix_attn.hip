@@ -42,7 +42,6 @@ struct RowsAttnArgs {
   int pool, pslots;
 };
 
-typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(1))) const void global_void;
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;

@@ -1660,23 +1660,12 @@ struct MoeArgs {
   float limit;
 };
 
-typedef __attribute__((address_space(3))) void lds_void;
 constexpr int kMoeStep = 128, kMoeCols = 128;
 constexpr int moe_lds(int bm, int stages) { return (kMoeCols + bm) * kMoeStep * stages; }
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, unsigned bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00027000);
-}
 // 16 bytes a lane from byte `at` of a buffer to 1024 bytes of LDS, in order of the lanes
 __device__ __forceinline__ void load_lds(__amdgpu_buffer_rsrc_t b, char* lds, unsigned at) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(b, (lds_void*)lds, 16, at, 0, 0, 0);
 }
-constexpr unsigned kOutside = 0x80000000u;   // (buffers are smaller: reads of zero)
-
-template <int LEFT>
-__device__ __forceinline__ void meet() {
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LEFT) : "memory");
-}
-
 enum { kGated = 0, kSquare = 1, kDown = 2 };
 
 template <int BM, int S, int EPI>

@@ -867,7 +867,7 @@ def test_decode_attention_from_lds_against_float64(H, G, dk, dv, maps, extras):
 def test_decode_attention_from_lds_sums_in_the_order_of_the_general_kernel(H, G, dk, dv, maps):
     """The same bits as over an f32 cache of the same values, which the general kernel takes: parts of the channels and shares of
     a tile's keys are added in one order in both.  Key rows of whole pieces of 32 channels are cut alike in either type; an
-    infinite key and one that is no number are among them."""
+    infinite key and one that is no number are among them; scores that lose with distance, and gated heads."""
     from vllm_omni_draft_amd import ops
     g = torch.Generator().manual_seed(H + dk)
     pos = [0, 2, 63, 64, 150, 199]
@@ -883,6 +883,14 @@ def test_decode_attention_from_lds_sums_in_the_order_of_the_general_kernel(H, G,
             at = (dev(q), k, v, i32(pos), i32(list(range(R))), bt.int().cuda(), H, G)
             rest = (dk, dv, dk ** -0.5, window, keep, chunk, cap, None if sk is None else dev(sk))
             return (ops.multimap_softmax_attention(*at, maps, *rest) if maps > 1 else ops.masked_softmax_attention(*at, *rest)).cpu()
+        torch.testing.assert_close(run(lambda t: t), run(lambda t: t.float()), rtol=0, atol=0, equal_nan=True)
+    if maps > 1:
+        return
+    d1, d2, gates = (dev(torch.rand(*n, generator=g)) for n in ((H,), (H,), (R, H)))
+    for f, kw in ((ops.distance_softmax_attention, dict(dist1=d1, dist2=d2)), (ops.gated_softmax_attention, dict(gates=gates, sinks=dev(sinks)))):
+        def run(cast):
+            k, v = cast(kc).cuda(), None if vc is None else cast(vc).cuda()
+            return f(dev(q), k, v, i32(pos), i32(list(range(R))), bt.int().cuda(), H, G, dk, dv, dk ** -0.5, 120, softcap=4.0, **kw).cpu()
         torch.testing.assert_close(run(lambda t: t), run(lambda t: t.float()), rtol=0, atol=0, equal_nan=True)
 
 

@@ -757,9 +757,8 @@ def test_every_block_shape_has_the_bits_of_few_rows(M, N, K, shape):
     of rows and of outputs that is not full: every row has the bits that it has among 48."""
     import ctypes as C
     from tests.gpu_util import internal
-    tiles = -(-N // 16)
-    assert internal("sd_prompt_shape_", C.c_int, C.c_int, C.c_int, C.c_int, C.c_int, C.c_bool)(M, tiles, tiles, K, False) == shape
-    ops = _ops()
+    ops, tiles = _ops(), -(-N // 16)
+    assert internal("sd_prompt_shape_", C.c_int, *[C.c_int] * 5)(M, tiles, tiles, K, ops.EPI_F32) == shape
     gen = torch.Generator(device="cuda").manual_seed(M + N + K)
     x = torch.randn(M, K, generator=gen, device="cuda").to(torch.bfloat16)
     W = ops._tiled((torch.randn(N, K, generator=gen, device="cuda") * K ** -0.5).to(torch.bfloat16), ops.EPI_F32)

@@ -381,10 +381,15 @@ constexpr Shape kWholeShapes[] = {
     {8, 8, 1, 16.2f, 0.f, {1.236f}},      {7, 8, 1, 8.7f, 0.f, {1.295f}},  {8, 6, 1, 12.3f, 0.f, {1.023f}},
     {4, 4, 2, 4.1f, 0.f, {.813f, .958f}}, {4, 4, 1, 5.8f, 0.f, {.477f}},   {4, 6, 1, 8.9f, 0.f, {.562f}}};
 
-float shape_us(const Shape& s, int M, int n_tiles, int K, int S) {
+float shape_us(const Shape& s, int M, int n_tiles, int K, int S, int epi) {
   const long blocks = (long)((n_tiles + 2 * s.tn - 1) / (2 * s.tn)) * ((M + 32 * s.tm - 1) / (32 * s.tm));
   const long round = 256l * s.per_cu, full = blocks / round, rest = blocks - full * round;
-  const float fixed = s.fixed + s.split * S, stages = K / 64;
+  // The epilogue that rotates and writes pages moves 2 bytes at a time, and nothing covers that of a large block alone on its
+  // CU.  us of QKV products with it, as chosen without this term / with it: 6144 x 4096 at 4096 rows 248 (128 x 256) / 230 (128 x 128, two a CU),
+  // 4608 x 3584 at 1500 88.6 / 74.0, at 4096 221 / 211, 3072 x 2048 at 2946 82.7 / 79.3; of 40 such products (264..4096 rows) .5 % behind the
+  // best of the nine shapes.
+  const float rope = epi == EPI_QKV_ROPE && S > 1 && s.tn * s.tm > 16 ? .5f * (s.tn * s.tm - 16) : 0.f;
+  const float fixed = s.fixed + s.split * S + rope, stages = K / 64;
   float us = full * (fixed + s.stage[s.per_cu - 1] * stages);
   if (rest) {
     // blocks a CU of the last round, which starts as the one before it ends here and there
@@ -394,32 +399,32 @@ float shape_us(const Shape& s, int M, int n_tiles, int K, int S) {
   return us;
 }
 
-// pair: gate and up tiles in one block, an even number of tiles a wave
+// (EPI_RELU_PAIR: gate and up tiles in one block, an even number of tiles a wave)
 template <int N>
-const Shape& best_shape(const Shape (&shapes)[N], int M, int n_tiles, int K, int S, bool pair, float& us) {
+const Shape& best_shape(const Shape (&shapes)[N], int M, int n_tiles, int K, int S, int epi, float& us) {
   int best = 0;
-  us = shape_us(shapes[0], M, n_tiles, K, S);
+  us = shape_us(shapes[0], M, n_tiles, K, S, epi);
   for (int i = 1; i < N; ++i) {
-    if (pair && shapes[i].tn % 2) continue;
-    const float t = shape_us(shapes[i], M, n_tiles, K, S);
+    if (epi == EPI_RELU_PAIR && shapes[i].tn % 2) continue;
+    const float t = shape_us(shapes[i], M, n_tiles, K, S, epi);
     if (t < us) us = t, best = i;
   }
   return shapes[best];
 }
-const Shape& best_shape(int M, int n_tiles, int K, int S, bool pair, float& us) {
-  return S == 1 ? best_shape(kWholeShapes, M, n_tiles, K, S, pair, us) : best_shape(kSplitShapes, M, n_tiles, K, S, pair, us);
+const Shape& best_shape(int M, int n_tiles, int K, int S, int epi, float& us) {
+  return S == 1 ? best_shape(kWholeShapes, M, n_tiles, K, S, epi, us) : best_shape(kSplitShapes, M, n_tiles, K, S, epi, us);
 }
 
-int shape_number(int M, int n_tiles, int K, int S, bool pair) {
+int shape_number(int M, int n_tiles, int K, int S, int epi) {
   float us;
-  const Shape& s = best_shape(M, n_tiles, K, S, pair, us);
+  const Shape& s = best_shape(M, n_tiles, K, S, epi, us);
   return s.tn * 100 + s.tm * 10 + s.per_cu;
 }
 
 template <int EPI>
 int prompt_shape(const PromptArgs& a, int S, hipStream_t st) {
   constexpr bool even = EPI == EPI_RELU_PAIR;
-  const int shape = shape_number(a.M, a.n_tiles, a.KS * 32, S, even);
+  const int shape = shape_number(a.M, a.n_tiles, a.KS * 32, S, EPI);
   switch (shape) {
     case 881: return launch_prompt<8, 8, 2, false, EPI, 2>(a, st);
     case 781:
@@ -444,10 +449,10 @@ int prompt_shape(const PromptArgs& a, int S, hipStream_t st) {
 
 // The block that a product of `n_tiles` of a matrix's `all_tiles` takes, tn * 100 + tm * 10 + blocks a CU, and 1000 where K
 // is split (tests ask whether their sizes reach every block).
-int sd_prompt_shape_(int M, int n_tiles, int all_tiles, int K, bool pair) {
+int sd_prompt_shape_(int M, int n_tiles, int all_tiles, int K, int epi) {
   int S, ksp, g;
   plan_split(all_tiles, K, S, ksp, g);
-  return shape_number(M, n_tiles, K, S, pair) + (S > 1 ? 1000 : 0);
+  return shape_number(M, n_tiles, K, S, epi) + (S > 1 ? 1000 : 0);
 }
 
 bool sd_prompt_linear_fits_(int M, int K, int64_t ldx) {
@@ -541,11 +546,11 @@ bool sd_prompt_relu_pair_fits_(int M, int n_tiles, int K, int64_t ldx, int gate_
   plan_split(n_tiles, K, S, ksp, g);
   const int rest = n_tiles - gate_tile - F / 8;
   float whole, pair, us;
-  best_shape(M, n_tiles, K, S, false, whole);
-  best_shape(M, F / 8, K, S, true, pair);
+  best_shape(M, n_tiles, K, S, SD_EPI_F32, whole);
+  best_shape(M, F / 8, K, S, EPI_RELU_PAIR, pair);
   for (const int tiles : {gate_tile, rest}) {
     if (tiles <= 0) continue;
-    best_shape(M, tiles, K, S, false, us);
+    best_shape(M, tiles, K, S, SD_EPI_F32, us);
     pair += us;
   }
   return 1.08f * pair < whole + 3.f + (float)M * F * (10 / 4.5e6f);

@@ -241,7 +241,7 @@ int sd_prompt_linear_(const void* W, const void* x, int64_t ldx, int M, int K, i
 int sd_linear_wide_norm_(const void* W, const float* w_scale, const void* x, int64_t ldx, const void* bias, const void* residual,
                          void* out, int M, int N, int K, void* workspace, size_t workspace_bytes, const void* norm_w, float eps,
                          void* norm_out, sd_stream_t stream);  // (linear_wide's residual epilogue, and the rows' RMS norm)
-int sd_prompt_shape_(int M, int n_tiles, int all_tiles, int K, bool pair);
+int sd_prompt_shape_(int M, int n_tiles, int all_tiles, int K, int epi);
 bool sd_prompt_relu_pair_fits_(int M, int n_tiles, int K, int64_t ldx, int gate_tile, int F);
 int sd_prompt_relu_pair_(const void* W, const void* x, int64_t ldx, int M, int K, int n_tiles, int gate_tile, int F, float* y,
                          int64_t ldy, void* act, sd_stream_t stream);

@@ -160,6 +160,68 @@ __global__ void head_prep_kernel(float* __restrict__ q, float* __restrict__ k, c
                                  int dims, int layout, const double* __restrict__ inv_freq, int unit_norm,
                                  float eps, float q_scale, float k_scale, T* __restrict__ k_cache,
                                  T* __restrict__ v_cache, const int32_t* __restrict__ block_tables,
+                                 int max_blocks, int page) {
+  const int r = blockIdx.x, hh = blockIdx.y, lane = threadIdx.x;
+  const bool is_q = hh < Hq;
+  const int head = is_q ? hh : hh - Hq;
+  float* vec = (is_q ? q : k) + (size_t)r * ld + (size_t)head * dk;
+  const int pos = row_pos[r];
+  float ss = 0.f;
+  for (int i = lane; i < dims / 2; i += 64) {
+    const double a = (double)pos * inv_freq[i];
+    const float cs = (float)cos(a), sn = (float)sin(a);
+    const int iu = layout ? 2 * i : i, iv = layout ? 2 * i + 1 : i + dims / 2;
+    const float u = vec[iu], w = vec[iv];
+    const float ru = u * cs - w * sn, rw = w * cs + u * sn;
+    vec[iu] = ru;
+    vec[iv] = rw;
+    ss = fmaf(ru, ru, ss);
+    ss = fmaf(rw, rw, ss);
+  }
+  for (int c = dims + lane; c < dk; c += 64) ss = fmaf(vec[c], vec[c], ss);
+  float scale = is_q ? q_scale : k_scale;
+  if (unit_norm) {
+    ss = wave_sum(ss);
+    scale *= 1.f / sqrtf(ss / (float)dk + eps);
+  }
+  T* kc = nullptr;
+  T* vc = nullptr;
+  if (!is_q && k_cache) {
+    const int pg = block_tables[(size_t)row_slot[r] * max_blocks + pos / page];
+    const size_t at = ((size_t)pg * Hk + head) * page + pos % page;
+    kc = k_cache + at * dk;
+    vc = v_cache + at * dv;
+  }
+  for (int i = lane; i < dims / 2; i += 64) {
+    const int iu = layout ? 2 * i : i, iv = layout ? 2 * i + 1 : i + dims / 2;
+    const float ou = vec[iu] * scale, ov = vec[iv] * scale;
+    vec[iu] = ou;
+    vec[iv] = ov;
+    if (kc) {
+      st_f(kc + iu, ou);
+      st_f(kc + iv, ov);
+    }
+  }
+  for (int c = dims + lane; c < dk; c += 64) {
+    const float o = vec[c] * scale;
+    vec[c] = o;
+    if (kc) st_f(kc + c, o);
+  }
+  if (vc) {
+    const float* vr = v + (size_t)r * ld + (size_t)head * dv;
+    for (int c = lane; c < dv; c += 64) st_f(vc + c, vr[c]);
+  }
+}
+
+// The same for many rows: `heads` heads of a row a wave, one after the other, by the same sines and cosines (f64), whose forming
+// is most of a wave's work; heads whose pairs are a lane each stay in registers, four on their way at a time.
+template <typename T>
+__global__ void head_prep_rows_kernel(float* __restrict__ q, float* __restrict__ k, const float* __restrict__ v,
+                                 int64_t ld, const int32_t* __restrict__ row_pos,
+                                 const int32_t* __restrict__ row_slot, int Hq, int Hk, int dk, int dv,
+                                 int dims, int layout, const double* __restrict__ inv_freq, int unit_norm,
+                                 float eps, float q_scale, float k_scale, T* __restrict__ k_cache,
+                                 T* __restrict__ v_cache, const int32_t* __restrict__ block_tables,
                                  int max_blocks, int page, int heads) {
   const int r = blockIdx.x, lane = threadIdx.x;
   const int pos = row_pos[r];
@@ -1040,19 +1102,26 @@ extern "C" int sd_head_prep(float* q, float* k, const float* v, int64_t ld, cons
   SD_REQUIRE(!k_cache || (v_cache && v && row_slot && block_tables && page >= 1 && max_blocks >= 1),
              SD_ERR_INVALID, "sd_head_prep: a cache needs values, slots and block tables");
   hipStream_t st = (hipStream_t)stream;
-  // A wave turns up to eight heads of a row once there are waves for the chip, by the same sines and cosines (f64).
-  // 2048 rows of 32 / 20 heads of 128, us: a head a wave, each value read and written twice 31 / 28, now 19 / 24.
   if (rot_dims == 0 && !unit_norm && k_scale == 1.f && !k_cache) Hk = 0;   // (nothing to do to the keys)
-  const int heads = std::min(std::max(n_rows * (Hq + Hk) / 4096, 1), 8);
-  dim3 grid(n_rows, (Hq + Hk + heads - 1) / heads);
-  if (cache_f32)
-    head_prep_kernel<float><<<grid, 64, 0, st>>>(q, k, v, ld, row_pos, row_slot, Hq, Hk, dk, dv, rot_dims,
-                                                 rot_layout, inv_freq, unit_norm, eps, q_scale, k_scale,
-                                                 (float*)k_cache, (float*)v_cache, block_tables, max_blocks, page, heads);
-  else
-    head_prep_kernel<bf16_t><<<grid, 64, 0, st>>>(q, k, v, ld, row_pos, row_slot, Hq, Hk, dk, dv, rot_dims,
-                                                  rot_layout, inv_freq, unit_norm, eps, q_scale, k_scale,
-                                                  (bf16_t*)k_cache, (bf16_t*)v_cache, block_tables, max_blocks, page, heads);
+  // A wave turns up to eight heads of a row once there are waves for the chip.  us, a head a wave / this way, 17 / 256 / 512 / 2048 rows:
+  // 16 + 16 heads of 128, rotated 3.0 / 3.2, 6.5 / 6.2, 10.4 / 8.0, 32 / 20, not rotated 2.7 / 2.8, 4.9 / 5.1, 7.4 / 7.0, 25 / 18; 16 + 4 with keys
+  // appended 3.5 / 3.7, 5.6 / 6.7 (one head a wave), 8.3 / 7.9, 23 / 17.  Heads in memory (partly rotated, or more than 128
+  // channels) from sixteen a wave's share on: 8 + 2 of which 64 channels turn 17 rows 3.6 / 4.3, 1024 8.6 / 9.9; 16 + 16 of 256 1500 rows
+  // 40.5 / 42.2, 2048 53 / 49, 4096 102 / 87.
+  const int share = n_rows * (Hq + Hk) / 4096, heads = std::min(std::max(share, 1), 8);
+  const bool pairs = (rot_dims == dk && dk <= 128) || (rot_dims == 0 && dk == 128);
+  const bool many = share >= (!pairs ? 16 : rot_dims ? 2 : 3);
+  const dim3 grid(n_rows, many ? (Hq + Hk + heads - 1) / heads : Hq + Hk);
+  auto launch = [&](auto* kc, auto* vc) {
+    if (many)
+      head_prep_rows_kernel<<<grid, 64, 0, st>>>(q, k, v, ld, row_pos, row_slot, Hq, Hk, dk, dv, rot_dims, rot_layout, inv_freq, unit_norm,
+                                                 eps, q_scale, k_scale, kc, vc, block_tables, max_blocks, page, heads);
+    else
+      head_prep_kernel<<<grid, 64, 0, st>>>(q, k, v, ld, row_pos, row_slot, Hq, Hk, dk, dv, rot_dims, rot_layout, inv_freq, unit_norm, eps,
+                                            q_scale, k_scale, kc, vc, block_tables, max_blocks, page);
+  };
+  if (cache_f32) launch((float*)k_cache, (float*)v_cache);
+  else launch((bf16_t*)k_cache, (bf16_t*)v_cache);
   SD_CHECK_LAUNCH("sd_head_prep");
   return SD_OK;
 }

@@ -150,8 +150,11 @@ __global__ __launch_bounds__(256, blocks_per_cu(TN, TM, STAGES, SPLIT)) void pro
   constexpr int kReads = TN + TM, kMfma = TN * TM;
   constexpr int kOver = kMfma * 3 / 4 > kReads ? kMfma * 3 / 4 : kReads;
   // A stage's direct loads: the first kEarly behind the barrier that frees its place, the others behind the next
-  // stage's first products (two stages: no time for that)
-  constexpr int kEarly = STAGES >= 3 ? kPieces / 2 : kPieces;
+  // stage's first products (two stages: no time for that).  Splits of K of more than 128 rows ask for all of them at once: their
+  // blocks have few stages, and the rows' part of one is most of it.  us, spread / at once: 3584 x 18944 192 rows 47.3 / 44.9, 4096 x
+  // 14336 256 rows 47.0 / 45.4, 8192 x 8192 224 rows 51.0 / 46.5, 2048 x 8192 256 rows 29.6 / 28.4 (3584 x 3584 23.2 / 23.7); but 4096 x 4096
+  // 100 rows 18.0 / 18.4, 8192 x 8192 128 rows 37.9 / 38.9.
+  constexpr int kEarly = STAGES >= 3 && !(EPI == EPI_PARTIAL && TM >= 6) ? kPieces / 2 : kPieces;
   static_assert(kReads <= kMfma && kEarly <= kMfma && kPieces - kEarly <= kMfma, "at most one LDS read and one direct load an MFMA");
   // what is in flight and newer than the next stage at a step's barrier
   constexpr int kAheadLeft = AHEAD == 0 ? 0 : STAGES >= 3 ? STAGES - 2 : 1;

@@ -349,124 +349,6 @@ __global__ void sigmoid_power_kernel(const float* __restrict__ z, int64_t ldz, f
   }
 }
 
-// ------------------------------------------------------------------ decayed outer-product scan
-// S <- diag(d_t) S + k_t v_t^T,  o_t = S^T q_t, token by token, per (entry, head).  A thread owns
-// 16 consecutive key channels of one value column; the strips' partial dot products are added in
-// strip order.  d_t: a factor per key channel (PER_CHANNEL, [rows, H*dk]) or per head ([H]).
-constexpr int kStrip = 16;
-constexpr int kScanLoads = 8;    // q / k / decay elements a thread stages per chunk, at most
-constexpr int kScanLoadsV = 16;  // value elements
-constexpr int kScanChunk = 16;   // tokens per chunk, at most
-template <bool PER_CHANNEL>
-__global__ __launch_bounds__(256) void decay_scan_kernel(
-    const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v, int64_t ld,
-    const float* __restrict__ decay, float* __restrict__ state, const int32_t* __restrict__ entries,
-    float* __restrict__ out, int H, int dk, int dv, int CT, int NS, int CH, int max_rows) {
-  if (entries[4 * blockIdx.z + 2] > max_rows) return;
-  extern __shared__ float lds[];
-  const int dkp = NS * kStrip;
-  float* qs = lds;                  // [CH][dkp]
-  float* ks = qs + CH * dkp;        // [CH][dkp]
-  float* ds = ks + CH * dkp;        // [CH][dkp] (PER_CHANNEL only)
-  float* vs = ds + (PER_CHANNEL ? CH * dkp : 0);  // [CH][CT]
-  float* part = vs + CH * CT;       // [CH][NS][CT]
-  const int tid = threadIdx.x, nthr = CT * NS;
-  const int c = tid % CT, s = tid / CT;
-  const int h = blockIdx.y, e = blockIdx.z;
-  const int col = blockIdx.x * CT + c;
-  const int slot = entries[4 * e], row0 = entries[4 * e + 1], len = entries[4 * e + 2],
-            pos0 = entries[4 * e + 3];
-  float* st = state + ((size_t)slot * H + h) * dk * dv;
-  const int r0 = s * kStrip;
-  float S[kStrip];
-#pragma unroll
-  for (int r = 0; r < kStrip; ++r)
-    S[r] = (pos0 > 0 && r0 + r < dk && col < dv) ? st[(size_t)(r0 + r) * dv + col] : 0.f;
-  const float dh = PER_CHANNEL ? 0.f : decay[h];
-  // A chunk of CH tokens goes global -> registers -> LDS; the next chunk's loads are in flight
-  // while this one is computed.
-  float pq[kScanLoads], pk[kScanLoads], pd[kScanLoads], pv[kScanLoadsV];
-  auto fetch = [&](int t0) {
-    const int nt = len - t0 < CH ? len - t0 : CH;
-#pragma unroll
-    for (int i = 0; i < kScanLoads; ++i) {
-      const int idx = tid + i * nthr;
-      const int t = idx / dkp, ch = idx % dkp;
-      const bool in = idx < nt * dkp && ch < dk;
-      // (every load is issued, on an address clamped into the chunk: a guarded load would become
-      // a branch whose join waits for the loads in flight)
-      const int tc = t < nt ? t : nt - 1, cc = ch < dk ? ch : dk - 1;
-      const size_t at = (size_t)(row0 + t0 + tc) * ld + (size_t)h * dk + cc;
-      const float lq = q[at], lk = k[at];
-      pq[i] = in ? lq : 0.f;
-      pk[i] = in ? lk : 0.f;
-      if (PER_CHANNEL) {
-        const float ldc = decay[(size_t)(row0 + t0 + tc) * ((size_t)H * dk) + (size_t)h * dk + cc];
-        pd[i] = in ? ldc : 0.f;
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < kScanLoadsV; ++i) {
-      const int idx = tid + i * nthr;
-      const int t = idx / CT, vcol = blockIdx.x * CT + idx % CT;
-      const bool in = idx < nt * CT && vcol < dv;
-      const int tc = t < nt ? t : nt - 1, vc2 = vcol < dv ? vcol : dv - 1;
-      const float lv = v[(size_t)(row0 + t0 + tc) * ld + (size_t)h * dv + vc2];
-      pv[i] = in ? lv : 0.f;
-    }
-  };
-  fetch(0);
-  for (int t0 = 0; t0 < len; t0 += CH) {
-    const int nt = len - t0 < CH ? len - t0 : CH;
-#pragma unroll
-    for (int i = 0; i < kScanLoads; ++i) {
-      const int idx = tid + i * nthr;
-      if (idx < CH * dkp) {
-        qs[idx] = pq[i];
-        ks[idx] = pk[i];
-        if (PER_CHANNEL) ds[idx] = pd[i];
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < kScanLoadsV; ++i) {
-      const int idx = tid + i * nthr;
-      if (idx < CH * CT) vs[idx] = pv[i];
-    }
-    __syncthreads();
-    if (t0 + CH < len) fetch(t0 + CH);
-    for (int t = 0; t < nt; ++t) {
-      const float vv = vs[t * CT + c];
-      const float* qt = qs + t * dkp + r0;
-      const float* kt = ks + t * dkp + r0;
-      const float* dt = ds + t * dkp + r0;
-      float acc = 0.f;
-#pragma unroll
-      for (int r = 0; r < kStrip; ++r) {
-        const float d = PER_CHANNEL ? dt[r] : dh;
-        S[r] = fmaf(d, S[r], kt[r] * vv);
-        acc = fmaf(S[r], qt[r], acc);
-      }
-      part[(t * NS + s) * CT + c] = acc;
-    }
-    __syncthreads();
-    for (int idx = tid; idx < nt * CT; idx += nthr) {
-      const int t = idx / CT, cc = idx % CT;
-      const int ocol = blockIdx.x * CT + cc;
-      if (ocol >= dv) continue;
-      float o = part[(t * NS) * CT + cc];
-      for (int ss = 1; ss < NS; ++ss) o += part[(t * NS + ss) * CT + cc];
-      out[(size_t)(row0 + t0 + t) * ((size_t)H * dv) + (size_t)h * dv + ocol] = o;
-    }
-    // (the next chunk's LDS stores touch qs / ks / ds / vs only; `part` is rewritten after the
-    // barrier that follows them)
-  }
-  if (col < dv) {
-#pragma unroll
-    for (int r = 0; r < kStrip; ++r)
-      if (r0 + r < dk) st[(size_t)(r0 + r) * dv + col] = S[r];
-  }
-}
-
 // y[r, h*dv + c] = o * (unit_norm ? rstd(o over the head) : 1) * (norm_w ? norm_w[c] : 1) * gate(g)
 // gate: 0 = silu, 1 = sigmoid.  One wave per (row, head).
 template <typename T>
@@ -1132,41 +1014,6 @@ extern "C" int sd_sigmoid_power(const float* z, int64_t ldz, float tau, float* o
   sigmoid_power_kernel<<<dim3(n_rows, (n_cols + kColsPerBlock - 1) / kColsPerBlock), 256, 0, (hipStream_t)stream>>>(
       z, ldz, 1.f / tau, out, n_cols);
   SD_CHECK_LAUNCH("sd_sigmoid_power");
-  return SD_OK;
-}
-
-extern "C" int sd_decay_scan(const float* q, const float* k, const float* v, int64_t ld, const float* decay,
-                             int per_channel, float* state, const int32_t* entries, int n_entries,
-                             float* out, int H, int dk, int dv, sd_stream_t stream) {
-  return sd_decay_scan_(q, k, v, ld, decay, per_channel, state, entries, n_entries, INT_MAX, out, H, dk, dv, stream);
-}
-
-int sd_decay_scan_(const float* q, const float* k, const float* v, int64_t ld, const float* decay, int per_channel,
-                   float* state, const int32_t* entries, int n_entries, int max_rows, float* out, int H, int dk, int dv,
-                   sd_stream_t stream) {
-  SD_REQUIRE(q && k && v && decay && state && entries && out && n_entries >= 1 && H >= 1 && dv >= 1,
-             SD_ERR_INVALID, "sd_decay_scan: bad argument");
-  SD_REQUIRE(dk >= 1 && dk <= 256, SD_ERR_UNSUPPORTED, "sd_decay_scan: key size %d outside 1..256", dk);
-  const int NS = (dk + kStrip - 1) / kStrip;
-  hipStream_t st = (hipStream_t)stream;
-  int CT = 256 / NS;
-  if (CT > dv) CT = dv;
-  if (CT > 64) CT = 64;
-  const int tiles = (dv + CT - 1) / CT;
-  const int dkp = NS * kStrip;
-  int CH = kScanLoads * (CT * NS) / dkp;   // a chunk's q / k elements fit kScanLoads per thread
-  if (CH > kScanChunk) CH = kScanChunk;
-  SD_REQUIRE(CH >= 1 && CH * CT <= kScanLoadsV * CT * NS, SD_ERR_UNSUPPORTED,
-             "sd_decay_scan: key size %d with value size %d leaves no chunk", dk, dv);
-  const size_t lds = sizeof(float) * ((size_t)(per_channel ? 3 : 2) * CH * dkp + (size_t)CH * CT + (size_t)CH * NS * CT);
-  dim3 grid(tiles, H, n_entries);
-  if (per_channel)
-    decay_scan_kernel<true><<<grid, CT * NS, lds, st>>>(q, k, v, ld, decay, state, entries, out, H, dk, dv, CT, NS, CH,
-                                                        max_rows);
-  else
-    decay_scan_kernel<false><<<grid, CT * NS, lds, st>>>(q, k, v, ld, decay, state, entries, out, H, dk, dv, CT, NS, CH,
-                                                         max_rows);
-  SD_CHECK_LAUNCH("sd_decay_scan");
   return SD_OK;
 }
 

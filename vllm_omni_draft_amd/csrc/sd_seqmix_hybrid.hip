@@ -1019,124 +1019,6 @@ __global__ __launch_bounds__(256) void conv_steps_decode_kernel(
     if (s < taps) st[(size_t)(s - 1) * C] = in[s];
 }
 
-// ------------------------------------------------------------------ scan with a decay per (row, head)
-constexpr int kStrip = 16;
-constexpr int kScanLoads = 8;
-constexpr int kScanLoadsV = 16;
-constexpr int kScanChunk = 16;
-// S <- d_t S + (a_t k_t) v_t^T, o_t = S^T q_t + skip v_t.  A thread owns 16 consecutive key channels
-// of one value column; strips' partial dot products are added in strip order (the skip term rides
-// on strip 0).  Chunks of tokens go global -> registers -> LDS with the next chunk's loads in flight.
-template <typename T>
-__global__ __launch_bounds__(256) void decay_scan_rows_kernel(
-    const float* __restrict__ q, const float* __restrict__ k, int64_t ldqk, const float* __restrict__ v, int64_t ldv,
-    const float* __restrict__ decay, const float* __restrict__ k_scale, const T* __restrict__ skip,
-    float* __restrict__ state, const int32_t* __restrict__ entries,
-    float* __restrict__ out, int H, int hpg, int dk, int dv, int CT, int NS, int CH, int max_rows) {
-  if (entries[4 * blockIdx.z + 2] > max_rows) return;
-  extern __shared__ float lds[];
-  const int dkp = NS * kStrip;
-  float* qs = lds;                  // [CH][dkp]
-  float* ks = qs + CH * dkp;        // [CH][dkp]
-  float* vs = ks + CH * dkp;        // [CH][CT]
-  float* dsc = vs + CH * CT;        // [CH] decay
-  float* asc = dsc + CH;            // [CH] key scale
-  float* part = asc + CH;           // [CH][NS][CT]
-  const int tid = threadIdx.x, nthr = CT * NS;
-  const int c = tid % CT, s = tid / CT;
-  const int h = blockIdx.y, e = blockIdx.z;
-  const int gq = h / hpg;
-  const int col = blockIdx.x * CT + c;
-  const int slot = entries[4 * e], row0 = entries[4 * e + 1], len = entries[4 * e + 2], pos0 = entries[4 * e + 3];
-  float* st = state + ((size_t)slot * H + h) * dk * dv;
-  const int r0 = s * kStrip;
-  float S[kStrip];
-#pragma unroll
-  for (int r = 0; r < kStrip; ++r)
-    S[r] = (pos0 > 0 && r0 + r < dk && col < dv) ? st[(size_t)(r0 + r) * dv + col] : 0.f;
-  const float skip_h = skip ? ld_f(skip + h) : 0.f;
-  float pq[kScanLoads], pk[kScanLoads], pv[kScanLoadsV], pd = 0.f, pa = 1.f;
-  auto fetch = [&](int t0) {
-    const int nt = len - t0 < CH ? len - t0 : CH;
-#pragma unroll
-    for (int i = 0; i < kScanLoads; ++i) {
-      const int idx = tid + i * nthr;
-      const int t = idx / dkp, ch = idx % dkp;
-      const bool in = idx < nt * dkp && ch < dk;
-      const int tc = t < nt ? t : nt - 1, cc = ch < dk ? ch : dk - 1;
-      const size_t at = (size_t)(row0 + t0 + tc) * ldqk + (size_t)gq * dk + cc;
-      const float lq = q[at], lk = k[at];
-      pq[i] = in ? lq : 0.f;
-      pk[i] = in ? lk : 0.f;
-    }
-#pragma unroll
-    for (int i = 0; i < kScanLoadsV; ++i) {
-      const int idx = tid + i * nthr;
-      const int t = idx / CT, vcol = blockIdx.x * CT + idx % CT;
-      const bool in = idx < nt * CT && vcol < dv;
-      const int tc = t < nt ? t : nt - 1, vc2 = vcol < dv ? vcol : dv - 1;
-      const float lv = v[(size_t)(row0 + t0 + tc) * ldv + (size_t)h * dv + vc2];
-      pv[i] = in ? lv : 0.f;
-    }
-    {
-      const int tc = tid < nt ? tid : nt - 1;
-      pd = decay[(size_t)(row0 + t0 + tc) * H + h];
-      pa = k_scale ? k_scale[(size_t)(row0 + t0 + tc) * H + h] : 1.f;
-    }
-  };
-  fetch(0);
-  for (int t0 = 0; t0 < len; t0 += CH) {
-    const int nt = len - t0 < CH ? len - t0 : CH;
-#pragma unroll
-    for (int i = 0; i < kScanLoads; ++i) {
-      const int idx = tid + i * nthr;
-      if (idx < CH * dkp) {
-        qs[idx] = pq[i];
-        ks[idx] = pk[i];
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < kScanLoadsV; ++i) {
-      const int idx = tid + i * nthr;
-      if (idx < CH * CT) vs[idx] = pv[i];
-    }
-    if (tid < CH) {
-      dsc[tid] = pd;
-      asc[tid] = pa;
-    }
-    __syncthreads();
-    if (t0 + CH < len) fetch(t0 + CH);
-    for (int t = 0; t < nt; ++t) {
-      const float vv = vs[t * CT + c];
-      const float d = dsc[t], av = asc[t] * vv;
-      const float* qt = qs + t * dkp + r0;
-      const float* kt = ks + t * dkp + r0;
-      float acc = 0.f;
-#pragma unroll
-      for (int r = 0; r < kStrip; ++r) {
-        S[r] = fmaf(d, S[r], kt[r] * av);
-        acc = fmaf(S[r], qt[r], acc);
-      }
-      if (s == 0) acc = fmaf(skip_h, vv, acc);
-      part[(t * NS + s) * CT + c] = acc;
-    }
-    __syncthreads();
-    for (int idx = tid; idx < nt * CT; idx += nthr) {
-      const int t = idx / CT, cc = idx % CT;
-      const int ocol = blockIdx.x * CT + cc;
-      if (ocol >= dv) continue;
-      float o = part[(t * NS) * CT + cc];
-      for (int ss = 1; ss < NS; ++ss) o += part[(t * NS + ss) * CT + cc];
-      out[(size_t)(row0 + t0 + t) * ((size_t)H * dv) + (size_t)h * dv + ocol] = o;
-    }
-  }
-  if (col < dv) {
-#pragma unroll
-    for (int r = 0; r < kStrip; ++r)
-      if (r0 + r < dk) st[(size_t)(r0 + r) * dv + col] = S[r];
-  }
-}
-
 // ------------------------------------------------------------------ routed experts
 // One wave per row: scores, then `top` rounds of a wave-wide arg-max (lowest index among equals).
 __global__ void moe_route_kernel(const float* __restrict__ logits, int64_t ld, int32_t* __restrict__ sel_e,
@@ -2580,46 +2462,6 @@ extern "C" int sd_ssd_steps(const float* dt, int64_t ld, const void* dt_bias, co
   else
     ssd_steps_kernel<bf16_t><<<(n + 255) / 256, 256, 0, st>>>(dt, ld, (const bf16_t*)dt_bias, (const bf16_t*)a_log, step, decay, n, H);
   SD_CHECK_LAUNCH("sd_ssd_steps");
-  return SD_OK;
-}
-
-extern "C" int sd_decay_scan_rows(const float* q, const float* k, int64_t ldqk, const float* v, int64_t ldv,
-                                  const float* decay, const float* k_scale, const void* skip, int w_f32, float* state,
-                                  const int32_t* entries, int n_entries, float* out, int H, int Gq, int dk, int dv,
-                                  sd_stream_t stream) {
-  return sd_decay_scan_rows_(q, k, ldqk, v, ldv, decay, k_scale, skip, w_f32, state, entries, n_entries, INT_MAX, out, H,
-                             Gq, dk, dv, stream);
-}
-
-int sd_decay_scan_rows_(const float* q, const float* k, int64_t ldqk, const float* v, int64_t ldv, const float* decay,
-                        const float* k_scale, const void* skip, int w_f32, float* state, const int32_t* entries,
-                        int n_entries, int max_rows, float* out, int H, int Gq, int dk, int dv, sd_stream_t stream) {
-  SD_REQUIRE(q && k && v && decay && state && entries && out && n_entries >= 1 && H >= 1 && Gq >= 1 && H % Gq == 0 &&
-                 dv >= 1,
-             SD_ERR_INVALID, "sd_decay_scan_rows: bad argument");
-  SD_REQUIRE(dk >= 1 && dk <= 256, SD_ERR_UNSUPPORTED, "sd_decay_scan_rows: key size %d outside 1..256", dk);
-  SD_REQUIRE(H <= 4096, SD_ERR_UNSUPPORTED, "sd_decay_scan_rows: more than 4096 heads");
-  const int NS = (dk + kStrip - 1) / kStrip;
-  hipStream_t st = (hipStream_t)stream;
-  int CT = 256 / NS;
-  if (CT > dv) CT = dv;
-  if (CT > 64) CT = 64;
-  const int tiles = (dv + CT - 1) / CT;
-  const int dkp = NS * kStrip;
-  int CH = kScanLoads * (CT * NS) / dkp;
-  if (CH > kScanChunk) CH = kScanChunk;
-  SD_REQUIRE(CH >= 1 && CH * CT <= kScanLoadsV * CT * NS, SD_ERR_UNSUPPORTED,
-             "sd_decay_scan_rows: key size %d with value size %d leaves no chunk", dk, dv);
-  const size_t lds = sizeof(float) * ((size_t)2 * CH * dkp + (size_t)CH * CT + 2 * (size_t)CH + (size_t)CH * NS * CT);
-  dim3 grid(tiles, H, n_entries);
-  const int hpg = H / Gq;
-  if (w_f32)
-    decay_scan_rows_kernel<float><<<grid, CT * NS, lds, st>>>(q, k, ldqk, v, ldv, decay, k_scale, (const float*)skip,
-                                                              state, entries, out, H, hpg, dk, dv, CT, NS, CH, max_rows);
-  else
-    decay_scan_rows_kernel<bf16_t><<<grid, CT * NS, lds, st>>>(q, k, ldqk, v, ldv, decay, k_scale, (const bf16_t*)skip,
-                                                               state, entries, out, H, hpg, dk, dv, CT, NS, CH, max_rows);
-  SD_CHECK_LAUNCH("sd_decay_scan_rows");
   return SD_OK;
 }
 

@@ -176,6 +176,23 @@ int sd_rejection_sample_split(const float* target_probs, const int64_t* bonus_id
                               int64_t* counters, int B, int k, int V,
                               void* scratch, sd_stream_t stream);
 
+/* The split forms in one launch each: the slices of a row tell each other what they hold through `state`
+ * (sd_sampling_state_bytes(state_rows) bytes, 8-byte aligned, zero before its first use, then kept by these
+ * three functions; of one stream at a time, like scratch).  sd_softmax_rows_once: temperatures as
+ * sd_softmax_rows_seq, or NULL and one temperature.  spins: how often a workgroup looks for another slice's
+ * numbers before it computes them itself; negative: the default.  Rows beyond state_rows, results over their
+ * own logits and slices too long for registers take the split forms, with `scratch`.              */
+size_t sd_sampling_state_bytes(int state_rows);
+int sd_softmax_rows_once(const float* logits, int64_t ld, const float* temperatures, int rows_per_seq,
+                         float temperature, float* probs, int64_t ld_probs, int R, int V, void* scratch,
+                         void* state, int state_rows, int spins, sd_stream_t stream);
+int sd_sample_rows_once(const float* probs, int64_t ld, const float* uniforms, int64_t* ids, int R, int V,
+                        void* scratch, void* state, int state_rows, int spins, sd_stream_t stream);
+int sd_rejection_sample_once(const float* target_probs, const int64_t* bonus_ids, const float* draft_probs,
+                             const int64_t* draft_ids, const float* u_accept, const float* u_recover,
+                             const int32_t* proposal_lens, int64_t* out_ids, int64_t* counters, int B, int k,
+                             int V, void* scratch, void* state, int state_rows, int spins, sd_stream_t stream);
+
 /* out[i] = uniform in [0, 1) (24 bits) from a counter-based hash of (seed,
  * *counter, i); then *counter += 1.  Lets a captured step draw fresh uniforms
  * on every replay without host work.  (The acceptance entry points take their

@@ -475,3 +475,58 @@ def test_token_logprobs_without_top_entries():
     want = torch.log_softmax(x, dim=-1)[torch.arange(4), toks.long()]
     assert ids.shape == (4, 1) and ids[:, 0].cpu().tolist() == toks.tolist()
     torch.testing.assert_close(lps[:, 0].cpu(), want, rtol=0, atol=2e-5)
+
+
+@pytest.mark.parametrize("V", [4, 252, 32000, 50272, 152064, 400000])
+@pytest.mark.parametrize("R", [1, 7, 32, 33, 90])
+def test_slices_of_a_row_in_one_launch(V, R):
+    """Softmax, draws and the rejection step in one launch against two, over 64 and 32 slices a row and every number of entries
+    a thread holds (400000: two launches where slices are too long): the same draws and the same probabilities but for rounding; again and again on one state, with workgroups that wait for nothing, and for results over their logits."""
+    from vllm_omni_draft_amd import _lib, ops
+    lib = _lib.load()
+    k, B = 4, max(R // 5, 1)
+    g = torch.Generator(device="cuda").manual_seed(V + R)
+    x = torch.randn(R, V, generator=g, device="cuda") * 3
+    x[R // 2, V // 3:] = float("-inf")
+    temps = torch.rand(R, generator=g, device="cuda") + 0.3
+    temps[R - 1] = 0.0
+    u = torch.rand(R, generator=g, device="cuda")
+    plain = torch.empty_like(ops.sampling_scratch(R))
+    want = ops.softmax_rows(x, temps, scratch=plain)
+    ids = ops.sample_rows(want, u, scratch=plain)
+    t, d = (torch.softmax(torch.randn(B, n, V, generator=g, device="cuda"), -1) for n in (k + 1, k))
+    d_ids = torch.randint(0, V, (B, k), generator=g, device="cuda")
+    args = (t, torch.arange(B, device="cuda"), d, d_ids, torch.rand(B, k, generator=g, device="cuda") * 1.5,
+            torch.rand(B, k + 1, generator=g, device="cuda"))
+    out = ops.rejection_sample(*args, scratch=plain)
+    sc = ops.sampling_scratch(R)
+    # Scores of up to 128 less two different maxima: half of 2^-17 off each; below 2^-126 an exponential (want) or a slice's factor (got) and
+    # their product are rounded to multiples of 2^-149: 1.5 and 1 of these off.
+    off = lambda p: ((p - want).abs() / (2.0 ** -16 * want + 2.5 * 2.0 ** -149)).max().item()
+    for _ in range(3):
+        got = ops.softmax_rows(x, temps, scratch=sc)
+        assert torch.equal(got[R - 1], want[R - 1]) and off(got) <= 1
+        assert torch.equal(ops.sample_rows(want, u, scratch=sc), ids)
+        assert torch.equal(ops.rejection_sample(*args, scratch=sc), out)
+    state = (sc.sd_state.data_ptr(), sc.sd_state_rows)
+    late, late_ids, over = torch.empty_like(x), torch.empty_like(ids), x.clone()
+    for dst, src in ((late, x), (over, over)):
+        _lib.check(lib.sd_softmax_rows_once(src.data_ptr(), V, temps.data_ptr(), 1, 1.0, dst.data_ptr(), V, R, V, sc.data_ptr(), *state, 0,
+                                            ops._stream()), "sd_softmax_rows_once")
+    assert torch.equal(late, got) and off(over) <= 1
+    _lib.check(lib.sd_sample_rows_once(want.data_ptr(), V, u.data_ptr(), late_ids.data_ptr(), R, V, sc.data_ptr(), *state, 0,
+                                       ops._stream()), "sd_sample_rows_once")
+    assert torch.equal(late_ids, ids)
+    with torch.cuda.stream(torch.cuda.Stream()):      # replayed, with eager work between
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            ops.softmax_rows(x, temps, out=late, scratch=sc)
+            ops.sample_rows(late, u, out=late_ids, scratch=sc)
+        for i in range(4):
+            late.zero_()
+            late_ids.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(late, got) and torch.equal(late_ids, ops.sample_rows(got, u, scratch=plain)), i
+            assert torch.equal(ops.sample_rows(want, u, scratch=sc), ids)

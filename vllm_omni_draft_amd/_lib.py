@@ -241,6 +241,10 @@ SIGNATURES = {
     "sd_softmax_rows_split": (i32, [vp, i64, C.c_float, vp, i64, i32, i32, vp, vp]),
     "sd_sample_rows_split": (i32, [vp, i64, vp, vp, i32, i32, vp, vp]),
     "sd_rejection_sample_split": (i32, [vp, vp, vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, vp, vp]),
+    "sd_sampling_state_bytes": (C.c_size_t, [i32]),
+    "sd_softmax_rows_once": (i32, [vp, i64, vp, i32, C.c_float, vp, i64, i32, i32, vp, vp, i32, i32, vp]),
+    "sd_sample_rows_once": (i32, [vp, i64, vp, vp, i32, i32, vp, vp, i32, i32, vp]),
+    "sd_rejection_sample_once": (i32, [vp, vp, vp, vp, vp, vp, vp, vp, vp, i32, i32, i32, vp, vp, i32, i32, vp]),
     "sd_ipc_buffer_bytes": (C.c_size_t, [C.c_size_t]),
     "sd_ipc_buffer_create": (i32, [C.c_size_t, C.POINTER(vp), vp]),
     "sd_ipc_buffer_open": (i32, [vp, C.POINTER(vp)]),

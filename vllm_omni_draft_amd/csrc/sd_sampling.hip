@@ -924,22 +924,23 @@ __global__ __launch_bounds__(kPartThreads) void softmax_finish_kernel(
   }
 }
 
-// First rejected position of sequence b (or L when every proposal is accepted).
+// First rejected position of sequence b (or L when every proposal is accepted): a lane a proposal, L <= 63.
 __device__ __forceinline__ int first_reject(const float* __restrict__ pb, const float* __restrict__ qb,
                                             const int64_t* __restrict__ draft_ids,
                                             const float* __restrict__ u_accept, int b, int k, int L,
                                             int V) {
-  int j = L;
-  for (int i = L - 1; i >= 0; --i) {
+  const int i = threadIdx.x & 63;
+  bool ok = true;
+  if (i < L) {
     const int64_t x = draft_ids[(size_t)b * k + i];
-    bool ok = false;
+    ok = false;
     if (x >= 0 && x < V) {
       const float uq = __fmul_rn(u_accept[(size_t)b * k + i], qb[(size_t)i * V + x]);
       ok = uq < pb[(size_t)i * V + x];
     }
-    if (!ok) j = i;
   }
-  return j;
+  const unsigned long long bad = __ballot(!ok);
+  return bad ? __ffsll(bad) - 1 : L;
 }
 
 struct ResidualRows {  // which rows the residual max(p - q, 0) of "row r" is taken from
@@ -973,18 +974,16 @@ __device__ __forceinline__ bool residual_rows(const ResidualRows& a, int r, int 
   return !(j == L && L == a.k);  // all accepted: the bonus token, no residual draw
 }
 
-__global__ __launch_bounds__(kPartThreads) void residual_mass_kernel(ResidualRows a, RowScratch sc,
-                                                                    int V) {
+// Mass of slice `part` of a residual row and its last index with mass, for thread 0.  Whole block.
+__device__ __forceinline__ void slice_mass(const float* __restrict__ p, const float* __restrict__ q, int part, int V,
+                                           double& total, int& last_pos) {
   __shared__ double s_d[kPartThreads / 64];
   __shared__ int s_i[kPartThreads / 64];
-  const int part = blockIdx.x, r = blockIdx.y, tid = threadIdx.x;
-  const float *p, *q;
-  int j, L;
-  if (!residual_rows(a, r, V, p, q, j, L)) return;
+  const int tid = threadIdx.x;
   int lo, hi;
   part_range(part, V, lo, hi);
   double local = 0.0;
-  int last_pos = -1;
+  last_pos = -1;
   for (int i = lo + tid * 4; i < hi; i += kPartThreads * 4) {
     const float4 pv = *reinterpret_cast<const float4*>(p + i);
     float4 qv = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -997,22 +996,34 @@ __global__ __launch_bounds__(kPartThreads) void residual_mass_kernel(ResidualRow
       if (e[jj] > 0.f) last_pos = i + jj;
     }
   }
-  const double total = part_block_sum(local, s_d);
+  total = part_block_sum(local, s_d);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) last_pos = max(last_pos, __shfl_xor(last_pos, o, 64));
   if ((tid & 63) == 0) s_i[tid >> 6] = last_pos;
   __syncthreads();
-  if (tid == 0) {
+  if (tid == 0)
     for (int w = 1; w < kPartThreads / 64; ++w) last_pos = max(last_pos, s_i[w]);
+}
+
+__global__ __launch_bounds__(kPartThreads) void residual_mass_kernel(ResidualRows a, RowScratch sc,
+                                                                    int V) {
+  const int part = blockIdx.x, r = blockIdx.y;
+  const float *p, *q;
+  int j, L;
+  if (!residual_rows(a, r, V, p, q, j, L)) return;
+  double total;
+  int last_pos;
+  slice_mass(p, q, part, V, total, last_pos);
+  if (threadIdx.x == 0) {
     sc.mass[(size_t)r * kRowParts + part] = total;
     sc.last[(size_t)r * kRowParts + part] = last_pos;
   }
 }
 
-// Inverse-CDF pick for row r from the slice masses: the slice whose running sum first exceeds
+// Inverse-CDF pick from the slices' masses [kRowParts] and last indexes: the slice whose running sum first exceeds
 // u * total, then a scan inside it (same rule as block_sample_residual).  Whole block.
 __device__ int pick_from_parts(const float* __restrict__ p, const float* __restrict__ q, int V,
-                               float u, const RowScratch& sc, int r) {
+                               float u, const double* mass, const int32_t* last) {
   __shared__ double s_prefix[kRowParts + 1];
   __shared__ double s_w[kPartThreads / 64];
   __shared__ int s_found, s_part;
@@ -1023,7 +1034,7 @@ __device__ int pick_from_parts(const float* __restrict__ p, const float* __restr
   // all: 64 reads, two walks; 13.0 and 10.6 us for 8 rows of 128256 in the two launches that pick, now 7.4 and 5.1)
   static_assert(kRowParts == 64, "a slice a lane");
   if (wave == 0) {
-    const double m = sc.mass[(size_t)r * kRowParts + lane];
+    const double m = mass[lane];
     double c = 0.0, before = 0.0;
 #pragma unroll
     for (int pp = 0; pp < kRowParts; ++pp) {
@@ -1111,7 +1122,7 @@ __device__ int pick_from_parts(const float* __restrict__ p, const float* __restr
   const int found = s_found;
   if (found != 0x7fffffff) return found;
   int last_pos = -1;  // rounding left no index: the last one with mass
-  for (int pp = 0; pp < kRowParts; ++pp) last_pos = max(last_pos, sc.last[(size_t)r * kRowParts + pp]);
+  for (int pp = 0; pp < kRowParts; ++pp) last_pos = max(last_pos, last[pp]);
   return max(last_pos, 0);
 }
 
@@ -1119,22 +1130,15 @@ __global__ __launch_bounds__(kPartThreads) void sample_finish_kernel(
     ResidualRows a, RowScratch sc, const float* __restrict__ uniforms, int64_t* __restrict__ ids,
     int V) {
   const int r = blockIdx.x;
-  const int idx = pick_from_parts(a.p + (size_t)r * a.ld_p, nullptr, V, uniforms[r], sc, r);
+  const int idx = pick_from_parts(a.p + (size_t)r * a.ld_p, nullptr, V, uniforms[r], sc.mass + (size_t)r * kRowParts,
+                                  sc.last + (size_t)r * kRowParts);
   if (threadIdx.x == 0) ids[r] = idx;
 }
 
-__global__ __launch_bounds__(kPartThreads) void rejection_finish_kernel(
-    ResidualRows a, RowScratch sc, const int64_t* __restrict__ bonus_ids,
-    const float* __restrict__ u_recover, int64_t* __restrict__ out_ids,
-    unsigned long long* __restrict__ counters, int V) {
-  const int b = blockIdx.x, tid = threadIdx.x, k = a.k;
-  const float *p, *q;
-  int j, L;
-  int64_t tok;
-  if (residual_rows(a, b, V, p, q, j, L))
-    tok = pick_from_parts(p, q, V, u_recover[(size_t)b * (k + 1) + j], sc, b);
-  else
-    tok = bonus_ids[b];
+// The emitted tokens of sequence b from its first rejected position j of L and the token there
+__device__ __forceinline__ void emit_tokens(const ResidualRows& a, int b, int j, int L, int64_t tok, int64_t* __restrict__ out_ids,
+                                            unsigned long long* __restrict__ counters) {
+  const int tid = threadIdx.x, k = a.k;
   if (tid <= k) {
     int64_t v = -1;
     if (tid < j) v = a.draft_ids[(size_t)b * k + tid];
@@ -1146,6 +1150,249 @@ __global__ __launch_bounds__(kPartThreads) void rejection_finish_kernel(
     atomicAdd(&counters[1], (unsigned long long)(j + 1));
     atomicAdd(&counters[2], (unsigned long long)L);
   }
+}
+
+__global__ __launch_bounds__(kPartThreads) void rejection_finish_kernel(
+    ResidualRows a, RowScratch sc, const int64_t* __restrict__ bonus_ids,
+    const float* __restrict__ u_recover, int64_t* __restrict__ out_ids,
+    unsigned long long* __restrict__ counters, int V) {
+  const int b = blockIdx.x;
+  const float *p, *q;
+  int j, L;
+  int64_t tok;
+  if (residual_rows(a, b, V, p, q, j, L))
+    tok = pick_from_parts(p, q, V, u_recover[(size_t)b * (a.k + 1) + j], sc.mass + (size_t)b * kRowParts,
+                          sc.last + (size_t)b * kRowParts);
+  else
+    tok = bonus_ids[b];
+  emit_tokens(a, b, j, L, tok, out_ids, counters);
+}
+
+// ---- the split forms in one launch each.
+// What the slices of a row tell each other goes through words of {value, number}, written and read whole at the scope of the
+// device.  A slice's words are written once a launch, by its own workgroup, which counts their number up from what it finds there; so
+// the slices of a row have the same number between launches, and a word of another slice is there once its number is the
+// reader's own next one, whatever else is under way.  (A counter a row that all raise: 64 atomic operations on one address, 6 us.)
+// None is ever cleared.  State per row, zero before the first launch on it, used by one launch at a time:
+//   softmax: words [64][2] and [32][2] {maximum, sum};   draws: words [64][3] {mass low, mass high, last index}.
+// Workgroups start in the order of their rows, so the ones a row waits for are running or next; one that has waited for long
+// (`spins` looks) computes the missing slices itself instead, so every wait ends.
+// us in two launches / in one, 128256 entries: softmax of 48 rows 9.4 + 15.1 / 15.1, of 40 8.4 + 13.2 / 13.5; 8 sequences, k = 5: draw 4.7 + 4.8 /
+// 7.7, rejection 4.7 + 9.5 / 8.6; and a launch less each (between 1.5 and 4).
+struct OnceState {
+  unsigned long long* soft64;  // [rows][64][2]
+  unsigned long long* soft32;  // [rows][32][2]
+  unsigned long long* draw;    // [rows][64][3]
+};
+constexpr int kOnceWords = 64 * 2 + 32 * 2 + 64 * 3;   // of a row
+inline size_t once_state_bytes(int rows) { return (size_t)rows * kOnceWords * sizeof(unsigned long long); }
+inline OnceState once_state(void* base, int rows) {
+  OnceState s;
+  s.soft64 = reinterpret_cast<unsigned long long*>(base);
+  s.soft32 = s.soft64 + (size_t)rows * 64 * 2;
+  s.draw = s.soft32 + (size_t)rows * 32 * 2;
+  return s;
+}
+constexpr int kOnceSpins = 1 << 14;
+constexpr int kOnceRows = 32;   // rows of 64 workgroups of four waves that the chip holds at once
+// The number of a slice's words in this launch
+__device__ __forceinline__ unsigned next_number(const unsigned long long* word) {
+  return (unsigned)(__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 32) + 1;
+}
+__device__ __forceinline__ void tell(unsigned long long* word, unsigned value, unsigned number) {
+  __hip_atomic_store(word, (unsigned long long)number << 32 | value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// The N words of this lane's slice (lanes below `parts`), of one wave; returns the slices that did not come.
+template <int N>
+__device__ __forceinline__ unsigned long long hear(const unsigned long long* words, int parts, unsigned number, int spins,
+                                                   unsigned (&value)[N]) {
+  const int lane = threadIdx.x & 63;
+  for (int look = 0;; ++look) {
+    bool here = true;
+    if (lane < parts)
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        const unsigned long long w = __hip_atomic_load(words + lane * N + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        here = here && (unsigned)(w >> 32) == number;
+        value[i] = (unsigned)w;
+      }
+    const unsigned long long missing = __ballot(!here);
+    if (!missing || look >= spins) return missing;
+    __builtin_amdgcn_s_sleep(1);
+  }
+}
+
+// A slice's entries (those past its end: the last one again)
+template <int PARTS>
+__device__ __forceinline__ void once_range(int part, int V, int& lo, int& hi) {
+  const int chunk = ((V + PARTS - 1) / PARTS + 3) & ~3;
+  lo = min(part * chunk, V);
+  hi = min(lo + chunk, V);
+}
+// Maximum of a slice and the sum of its exponentials over that from what its threads hold: entry(u) is the thread's u-th, of `n` in
+// the slice; keep(u, e) takes the exponential.  greedy: the maximum alone.  Whole block.
+template <int UNROLL, class F, class K>
+__device__ __forceinline__ void slice_stats(F entry, K keep, int entries, int n, float inv_t, bool greedy, float& mx, float& total) {
+  __shared__ float s_f[kPartThreads / 64];
+  __shared__ double s_d[kPartThreads / 64];
+  const int tid = threadIdx.x;
+  mx = -INFINITY;
+  if (n > 0)
+#pragma unroll UNROLL
+    for (int u = 0; u < entries; ++u) mx = fmaxf(mx, entry(u) * inv_t);
+  mx = wave_max(mx);
+  __syncthreads();
+  if ((tid & 63) == 0) s_f[tid >> 6] = mx;
+  __syncthreads();
+  mx = s_f[0];
+  for (int w = 1; w < kPartThreads / 64; ++w) mx = fmaxf(mx, s_f[w]);
+  double sum = 0.0;
+  if (!greedy) {
+#pragma unroll UNROLL
+    for (int u = 0; u < entries; ++u) {
+      const float e = mx != -INFINITY ? expf(entry(u) * inv_t - mx) : 0.f;
+      if (tid + u * kPartThreads < n) sum += (double)e;
+      keep(u, e);
+    }
+  }
+  total = (float)part_block_sum(sum, s_d);
+}
+
+// Rows in PARTS slices of at most E * kPartThreads entries, which stay in registers from the first reading to the results, their
+// exponentials over the slice's maximum instead of them from its sum on (a slice's factor comes from 64 bits, so a result has no more
+// roundings than one exponential over the row's maximum).  Half the slices where 64 a row would be more workgroups than the
+// chip holds at once.
+template <int PARTS, int E>
+__global__ __launch_bounds__(kPartThreads, E <= 16 ? 6 : 4) void softmax_once_kernel(
+    const float* __restrict__ logits, int64_t ld, RowTemps tm, OnceState state, float* __restrict__ probs, int64_t ld_probs, int V,
+    int spins) {
+  __shared__ float s_max[PARTS], s_sum[PARTS], s_factor;
+  __shared__ unsigned long long s_missing;
+  const int part = blockIdx.x, r = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+  unsigned long long* words = (PARTS == 64 ? state.soft64 : state.soft32) + (size_t)r * PARTS * 2;
+  const unsigned number = tid < 64 ? next_number(words + 2 * part) : 0;   // (the wave that writes them)
+  bool greedy;
+  const float inv_t = row_inv_t(tm, r, greedy);   // greedy rows: slice maxima of the raw logits
+  const float* row = logits + (size_t)r * ld;
+  float* out = probs + (size_t)r * ld_probs;
+  int lo, hi;
+  once_range<PARTS>(part, V, lo, hi);
+  float v[E];
+#pragma unroll
+  for (int u = 0; u < E; ++u) v[u] = row[min(lo + tid + u * kPartThreads, hi - 1)];
+  float mx, sum;
+  slice_stats<E>([&](int u) { return v[u]; }, [&](int u, float e) { v[u] = e; }, E, hi - lo, inv_t, greedy, mx, sum);
+  if (tid == 0) {
+    tell(words + 2 * part, __float_as_uint(mx), number);
+    tell(words + 2 * part + 1, __float_as_uint(sum), number);
+  }
+  if (tid < 64) {
+    unsigned value[2];
+    const unsigned long long missing = hear(words, PARTS, number, spins, value);
+    if (lane < PARTS) {
+      s_max[lane] = __uint_as_float(value[0]);
+      s_sum[lane] = __uint_as_float(value[1]);
+    }
+    if (lane == 0) s_missing = missing;
+  }
+  __syncthreads();
+  for (unsigned long long missing = s_missing; missing; missing &= missing - 1) {
+    const int p = __ffsll(missing) - 1;
+    int from, end;
+    once_range<PARTS>(p, V, from, end);
+    slice_stats<1>([&](int u) { return row[min(from + tid + u * kPartThreads, end - 1)]; }, [](int, float) {}, E, end - from, inv_t,
+                   greedy, mx, sum);
+    if (tid == 0) {
+      s_max[p] = mx;
+      s_sum[p] = sum;
+    }
+    __syncthreads();
+  }
+  if (greedy) {   // all mass on the first maximum: the lowest slice that holds it, lowest index
+    __shared__ int s_first[kPartThreads / 64];
+    const float pm = lane < PARTS ? fmaxf(s_max[lane], -INFINITY) : -INFINITY;
+    mx = wave_max(pm);
+    const int first_part = __ffsll((unsigned long long)__ballot(lane < PARTS && pm == mx)) - 1;
+    int mine = INT_MAX;
+    if (part == first_part)
+#pragma unroll
+      for (int u = 0; u < E; ++u)
+        if (lo + tid + u * kPartThreads < hi && v[u] == mx) mine = min(mine, lo + tid + u * kPartThreads);
+    for (int o = 32; o > 0; o >>= 1) mine = min(mine, __shfl_xor(mine, o, 64));
+    if (lane == 0) s_first[tid >> 6] = mine;
+    __syncthreads();
+    int best = s_first[0];
+    for (int w = 1; w < kPartThreads / 64; ++w) best = min(best, s_first[w]);
+    for (int i = lo + tid; i < hi; i += kPartThreads) out[i] = i == best ? 1.f : 0.f;
+    return;
+  }
+  if (tid < 64) {   // the row's sum, a lane a slice, in order of the slices
+    const float pm = lane < PARTS ? fmaxf(s_max[lane], -INFINITY) : -INFINITY;
+    const float row_max = wave_max(pm);
+    const double over = exp((double)pm - (double)row_max);
+    const double term = pm != -INFINITY ? (double)s_sum[lane] * over : 0.0;
+    double total = 0.0;
+#pragma unroll
+    for (int p = 0; p < PARTS; ++p) total += lane_of(term, p);
+    if (lane == part) s_factor = (float)(over / total);
+  }
+  __syncthreads();
+  const float factor = s_factor;
+#pragma unroll
+  for (int u = 0; u < E; ++u)
+    if (lo + tid + u * kPartThreads < hi) out[lo + tid + u * kPartThreads] = v[u] * factor;
+}
+
+// A draw from every row's residual, and with bonus_ids the tokens that a sequence emits.  The last slice's workgroup draws.
+__global__ __launch_bounds__(kPartThreads) void draw_once_kernel(
+    ResidualRows a, OnceState state, const float* __restrict__ uniforms, const int64_t* __restrict__ bonus_ids,
+    int64_t* __restrict__ ids, unsigned long long* __restrict__ counters, int V, int spins) {
+  __shared__ double s_mass[kRowParts];
+  __shared__ int32_t s_last[kRowParts];
+  __shared__ unsigned long long s_missing;
+  const int part = blockIdx.x, r = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+  unsigned long long* words = state.draw + (size_t)r * kRowParts * 3;
+  const unsigned number = tid < 64 ? next_number(words + 3 * part) : 0;   // (the wave that writes them)
+  const float *p, *q;
+  int j, L;
+  const bool draws = residual_rows(a, r, V, p, q, j, L);
+  double total;
+  int last_pos;
+  if (draws) {
+    slice_mass(p, q, part, V, total, last_pos);
+    if (tid == 0) {
+      const unsigned long long m = __builtin_bit_cast(unsigned long long, total);
+      tell(words + 3 * part, (unsigned)m, number);
+      tell(words + 3 * part + 1, (unsigned)(m >> 32), number);
+      tell(words + 3 * part + 2, (unsigned)last_pos, number);
+    }
+  }
+  if (part != kRowParts - 1) return;
+  int64_t tok;
+  if (draws) {
+    if (tid < 64) {
+      unsigned value[3] = {0, 0, 0};
+      const unsigned long long missing = hear(words, kRowParts, number, spins, value);
+      s_mass[lane] = __builtin_bit_cast(double, (unsigned long long)value[1] << 32 | value[0]);
+      s_last[lane] = (int)value[2];
+      if (lane == 0) s_missing = missing;
+    }
+    __syncthreads();
+    for (unsigned long long missing = s_missing; missing; missing &= missing - 1) {
+      const int m = __ffsll(missing) - 1;
+      slice_mass(p, q, m, V, total, last_pos);
+      if (tid == 0) {
+        s_mass[m] = total;
+        s_last[m] = last_pos;
+      }
+      __syncthreads();
+    }
+    tok = pick_from_parts(p, q, V, uniforms[bonus_ids ? (size_t)r * (a.k + 1) + j : (size_t)r], s_mass, s_last);
+  } else {
+    tok = bonus_ids[r];
+  }
+  if (bonus_ids) emit_tokens(a, r, j, L, tok, ids, counters);
+  else if (tid == 0) ids[r] = tok;
 }
 
 // u[i] = 24-bit uniform in [0, 1) from (seed, *counter, i); one workgroup, which then advances
@@ -1771,6 +2018,81 @@ extern "C" int sd_rejection_sample_split(const float* target_probs, const int64_
                      a, sc, bonus_ids, u_recover, out_ids,
                      reinterpret_cast<unsigned long long*>(counters), V);
   SD_CHECK_LAUNCH("sd_rejection_sample_split");
+  return SD_OK;
+}
+
+extern "C" size_t sd_sampling_state_bytes(int rows) { return rows > 0 ? once_state_bytes(rows) : 0; }
+
+extern "C" int sd_softmax_rows_once(const float* logits, int64_t ld, const float* temperatures, int rows_per_seq,
+                                    float temperature, float* probs, int64_t ld_probs, int R, int V, void* scratch,
+                                    void* state, int state_rows, int spins, sd_stream_t stream) {
+  SD_REQUIRE(R >= 0 && V >= 1 && ld >= V && ld_probs >= V && logits && probs && scratch && state && rows_per_seq >= 1 &&
+                 (temperatures || temperature > 0.f) && (reinterpret_cast<uintptr_t>(state) & 7) == 0,
+             SD_ERR_INVALID, "sd_softmax_rows_once: bad arguments (R=%d V=%d rows_per_seq=%d)", R, V, rows_per_seq);
+  if (R == 0) return SD_OK;
+  const int parts = R <= kOnceRows ? 64 : 32, chunk = ((V + parts - 1) / parts + 3) & ~3;
+  const float *in_end = logits + (size_t)(R - 1) * ld + V, *out_end = probs + (size_t)(R - 1) * ld_probs + V;
+  const bool apart = in_end <= probs || out_end <= logits;   // (a late workgroup reads its row again)
+  if (R > state_rows || !apart || chunk > 24 * kPartThreads)
+    return temperatures ? sd_softmax_rows_seq(logits, ld, temperatures, rows_per_seq, probs, ld_probs, R, V, scratch, stream)
+                        : sd_softmax_rows_split(logits, ld, temperature, probs, ld_probs, R, V, scratch, stream);
+  const RowTemps tm{temperatures, rows_per_seq, temperatures ? 1.f : 1.0f / temperature};
+  const OnceState st = once_state(state, state_rows);
+  const int n = spins < 0 ? kOnceSpins : spins;
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(parts, R), dim3(kPartThreads), 0, (hipStream_t)stream, logits, ld, tm, st, probs, ld_probs, V, n);
+  };
+  if (parts == 64) {
+    if (chunk <= 8 * kPartThreads) go(softmax_once_kernel<64, 8>);
+    else if (chunk <= 12 * kPartThreads) go(softmax_once_kernel<64, 12>);
+    else go(softmax_once_kernel<64, 24>);
+  } else {
+    if (chunk <= 8 * kPartThreads) go(softmax_once_kernel<32, 8>);
+    else if (chunk <= 16 * kPartThreads) go(softmax_once_kernel<32, 16>);
+    else go(softmax_once_kernel<32, 24>);
+  }
+  SD_CHECK_LAUNCH("sd_softmax_rows_once");
+  return SD_OK;
+}
+
+extern "C" int sd_sample_rows_once(const float* probs, int64_t ld, const float* uniforms, int64_t* ids, int R, int V,
+                                   void* scratch, void* state, int state_rows, int spins, sd_stream_t stream) {
+  SD_REQUIRE(state && (reinterpret_cast<uintptr_t>(state) & 7) == 0, SD_ERR_INVALID, "sd_sample_rows_once: no state");
+  if (R > state_rows) return sd_sample_rows_split(probs, ld, uniforms, ids, R, V, scratch, stream);
+  SD_REQUIRE(R >= 0 && V >= 4 && ld >= V && probs && uniforms && ids, SD_ERR_INVALID,
+             "sd_sample_rows_once: bad arguments (R=%d V=%d)", R, V);
+  SD_REQUIRE(V % 4 == 0 && ld % 4 == 0 && sd_aligned16(probs), SD_ERR_UNSUPPORTED,
+             "sd_sample_rows_once: V and ld must be multiples of 4, rows 16-byte aligned");
+  if (R == 0) return SD_OK;
+  const ResidualRows a{probs, ld, nullptr, nullptr, nullptr, nullptr, 0};
+  hipLaunchKernelGGL(draw_once_kernel, dim3(kRowParts, R), dim3(kPartThreads), 0, (hipStream_t)stream, a,
+                     once_state(state, state_rows), uniforms, (const int64_t*)nullptr, ids, (unsigned long long*)nullptr, V,
+                     spins < 0 ? kOnceSpins : spins);
+  SD_CHECK_LAUNCH("sd_sample_rows_once");
+  return SD_OK;
+}
+
+extern "C" int sd_rejection_sample_once(const float* target_probs, const int64_t* bonus_ids, const float* draft_probs,
+                                        const int64_t* draft_ids, const float* u_accept, const float* u_recover,
+                                        const int32_t* proposal_lens, int64_t* out_ids, int64_t* counters, int B, int k, int V,
+                                        void* scratch, void* state, int state_rows, int spins, sd_stream_t stream) {
+  SD_REQUIRE(state && (reinterpret_cast<uintptr_t>(state) & 7) == 0, SD_ERR_INVALID, "sd_rejection_sample_once: no state");
+  if (B > state_rows)
+    return sd_rejection_sample_split(target_probs, bonus_ids, draft_probs, draft_ids, u_accept, u_recover, proposal_lens, out_ids,
+                                     counters, B, k, V, scratch, stream);
+  SD_REQUIRE(B >= 0 && k >= 1 && k <= 63 && V >= 4, SD_ERR_INVALID,
+             "sd_rejection_sample_once: need B>=0, 1<=k<=63, V>=4 (B=%d k=%d V=%d)", B, k, V);
+  SD_REQUIRE(V % 4 == 0, SD_ERR_UNSUPPORTED, "sd_rejection_sample_once: V %% 4 != 0 (V=%d)", V);
+  SD_REQUIRE(target_probs && bonus_ids && draft_probs && draft_ids && u_accept && u_recover && out_ids, SD_ERR_INVALID,
+             "sd_rejection_sample_once: null pointer");
+  SD_REQUIRE(sd_aligned16(target_probs) && sd_aligned16(draft_probs), SD_ERR_INVALID,
+             "sd_rejection_sample_once: probability rows must be 16-byte aligned");
+  if (B == 0) return SD_OK;
+  const ResidualRows a{target_probs, 0, draft_probs, draft_ids, u_accept, proposal_lens, k};
+  hipLaunchKernelGGL(draw_once_kernel, dim3(kRowParts, B), dim3(kPartThreads), 0, (hipStream_t)stream, a,
+                     once_state(state, state_rows), u_recover, bonus_ids, out_ids, reinterpret_cast<unsigned long long*>(counters), V,
+                     spins < 0 ? kOnceSpins : spins);
+  SD_CHECK_LAUNCH("sd_rejection_sample_once");
   return SD_OK;
 }
 

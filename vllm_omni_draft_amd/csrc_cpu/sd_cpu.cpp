@@ -636,6 +636,23 @@ extern "C" int sd_sample_rows_split(const float* p, int64_t ld, const float* u, 
   return sd_sample_rows(p, ld, u, ids, R, V, s);
 }
 
+extern "C" size_t sd_sampling_state_bytes(int rows) { return rows > 0 ? 64 : 0; }
+extern "C" int sd_softmax_rows_once(const float* l, int64_t ld, const float* temps, int rows_per_seq, float t, float* p, int64_t ldp,
+                                    int R, int V, void* scratch, void*, int, int, sd_stream_t s) {
+  return temps ? sd_softmax_rows_seq(l, ld, temps, rows_per_seq, p, ldp, R, V, scratch, s) : sd_softmax_rows(l, ld, t, p, ldp, R, V, s);
+}
+extern "C" int sd_sample_rows_once(const float* p, int64_t ld, const float* u, int64_t* ids, int R, int V, void*, void*, int, int,
+                                   sd_stream_t s) {
+  return sd_sample_rows(p, ld, u, ids, R, V, s);
+}
+extern "C" int sd_rejection_sample_once(const float* target_probs, const int64_t* bonus_ids, const float* draft_probs,
+                                        const int64_t* draft_ids, const float* u_accept, const float* u_recover,
+                                        const int32_t* proposal_lens, int64_t* out_ids, int64_t* counters, int B, int k, int V,
+                                        void*, void*, int, int, sd_stream_t s) {
+  return sd_rejection_sample(target_probs, bonus_ids, draft_probs, draft_ids, u_accept, u_recover, proposal_lens, out_ids,
+                             counters, B, k, V, s);
+}
+
 namespace {
 inline float uniform24(unsigned long long seed, unsigned long long c, unsigned long long i) {
   unsigned long long z = seed ^ (c * 0x9e3779b97f4a7c15ull) ^ (i << 32 | (unsigned)i);

@@ -51,9 +51,21 @@ def device_info():
 # ---------------------------------------------------------------- acceptance
 def sampling_scratch(rows: int, device="cuda") -> torch.Tensor:
     """Scratch for the split (many-workgroups-per-row) forms of softmax_rows, sample_rows and
-    rejection_sample over up to `rows` rows / sequences."""
-    return torch.empty(max(int(_lib.load().sd_sampling_scratch_bytes(rows)), 16),
-                       dtype=torch.uint8, device=device)
+    rejection_sample over up to `rows` rows / sequences.  It carries the state with which these run in one launch each
+    (another buffer of sd_sampling_scratch_bytes(rows) bytes does too, in two launches); one stream at a time uses it."""
+    lib = _lib.load()
+    scratch = torch.empty(max(int(lib.sd_sampling_scratch_bytes(rows)), 16), dtype=torch.uint8, device=device)
+    if scratch.is_cuda and rows > 0:
+        scratch.sd_state = torch.zeros(int(lib.sd_sampling_state_bytes(rows)), dtype=torch.uint8, device=device)
+        scratch.sd_state_rows = rows
+        torch.cuda.current_stream(scratch.device).synchronize()   # (zero for whatever stream uses it)
+    return scratch
+
+
+def _once(scratch, rows):
+    """(state, its rows) of a scratch buffer that carries them, or None."""
+    state = getattr(scratch, "sd_state", None)
+    return None if state is None or rows > scratch.sd_state_rows else (_p(state), scratch.sd_state_rows)
 
 
 def _scratch_ok(scratch, rows, what):
@@ -84,6 +96,12 @@ def rejection_sample(target_probs, bonus_ids, draft_probs, draft_ids, u_accept, 
     if out is None:
         out = torch.empty(B, k + 1, dtype=torch.int64, device=target_probs.device)
     if scratch is not None:
+        once = _once(scratch, B)
+        if once:
+            _lib.check(_lib.load().sd_rejection_sample_once(
+                _p(target_probs), _p(bonus), _p(draft_probs), _p(draft_ids), _p(u_accept), _p(u_recover), _p(proposal_lens),
+                _p(out), _p(counters), B, k, V, _p(scratch), *once, -1, _stream()), "sd_rejection_sample_once")
+            return out
         _scratch_ok(scratch, B, "rejection_sample")
         _lib.check(_lib.load().sd_rejection_sample_split(
             _p(target_probs), _p(bonus), _p(draft_probs), _p(draft_ids), _p(u_accept),
@@ -168,12 +186,24 @@ def softmax_rows(logits: torch.Tensor, temperature=1.0, out=None, *, row_offset=
         if rows_per_seq < 1 or temperature.numel() * rows_per_seq < R:
             raise _lib.SdError("softmax_rows: fewer temperatures than sequences")
         if scratch is not None:
+            once = _once(scratch, R)
+            if once:
+                _lib.check(_lib.load().sd_softmax_rows_once(
+                    logits.data_ptr() + row_offset * V * 4, V * row_step, _p(temperature), rows_per_seq, 1.0, dst, out_ld or V, R, V,
+                    _p(scratch), *once, -1, _stream()), "sd_softmax_rows_once")
+                return out
             _scratch_ok(scratch, R, "softmax_rows")
         _lib.check(_lib.load().sd_softmax_rows_seq(
             logits.data_ptr() + row_offset * V * 4, V * row_step, _p(temperature), rows_per_seq, dst,
             out_ld or V, R, V, _p(scratch), _stream()), "sd_softmax_rows_seq")
         return out
     if scratch is not None:
+        once = _once(scratch, R)
+        if once:
+            _lib.check(_lib.load().sd_softmax_rows_once(
+                logits.data_ptr() + row_offset * V * 4, V * row_step, None, 1, float(temperature), dst, out_ld or V, R, V,
+                _p(scratch), *once, -1, _stream()), "sd_softmax_rows_once")
+            return out
         _scratch_ok(scratch, R, "softmax_rows")
         _lib.check(_lib.load().sd_softmax_rows_split(
             logits.data_ptr() + row_offset * V * 4, V * row_step, float(temperature), dst,
@@ -253,6 +283,12 @@ def sample_rows(probs: torch.Tensor, uniforms: torch.Tensor, out=None, *, row_of
     if out is None:
         out = torch.empty(R, dtype=torch.int64, device=probs.device)
     if scratch is not None:
+        once = _once(scratch, R)
+        if once:
+            _lib.check(_lib.load().sd_sample_rows_once(
+                probs.data_ptr() + row_offset * V * 4, V * row_step, _p(uniforms), _p(out), R, V, _p(scratch), *once, -1, _stream()),
+                "sd_sample_rows_once")
+            return out
         _scratch_ok(scratch, R, "sample_rows")
         _lib.check(_lib.load().sd_sample_rows_split(
             probs.data_ptr() + row_offset * V * 4, V * row_step, _p(uniforms), _p(out), R, V,

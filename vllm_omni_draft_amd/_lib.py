@@ -14,6 +14,7 @@ _LIB_NAME = "libsd_amd.so"
 # library has not been built (a first run in a fresh checkout); it exports a subset of the ABI.
 _SEQ_LIB_NAME = "libsd_seq.so"
 _lib: Optional[C.CDLL] = None
+_backend: Optional[str] = None   # of the library that is loaded (asking the environment for every call: 0.5 us a time)
 _partial = False
 
 c_i32p = C.POINTER(C.c_int32)
@@ -382,6 +383,8 @@ def backend() -> str:
     the same ABI for hosts without a GPU), chosen for the whole process by SD_AMD_BACKEND before
     the first call.  The choice is explicit: a missing GPU library is an error, never a reason
     to load the other one."""
+    if _backend is not None:
+        return _backend
     b = os.environ.get("SD_AMD_BACKEND", "gpu").lower()
     if b not in ("gpu", "cpu"):
         raise SdError(f"SD_AMD_BACKEND must be 'gpu' or 'cpu', not {b!r}")
@@ -410,7 +413,7 @@ def load() -> C.CDLL:
     if not os.path.exists(path):
         raise SdError(f"{path} is missing: build it with `make` (hipcc --offload-arch=gfx950; "
                       "g++ for the CPU build); nothing falls back to another library or to PyTorch")
-    global _partial
+    global _partial, _backend
     lib = C.CDLL(path)
     _partial = os.path.basename(path) == _SEQ_LIB_NAME
     for name, (res, args) in SIGNATURES.items():
@@ -419,7 +422,7 @@ def load() -> C.CDLL:
         fn = getattr(lib, name)  # AttributeError if a declared symbol is not exported
         fn.restype = res
         fn.argtypes = args
-    _lib = lib
+    _lib, _backend = lib, backend()
     return lib
 
 

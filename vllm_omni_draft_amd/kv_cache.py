@@ -250,10 +250,10 @@ class SeqCache:
         if need - len(tbl) > self.allocator.num_free:
             raise OutOfPages("KV cache is out of pages")
         first_new = len(tbl)
-        while len(tbl) < need:
-            tbl.append(self.allocator.alloc())
-        self.block_tables[slot, first_new:need].copy_(torch.tensor(tbl[first_new:], dtype=torch.int32),
-                                                      non_blocking=False)
+        tbl += [self.allocator.alloc() for _ in range(need - first_new)]
+        # (from pinned memory, in order on the caller's stream: the host does not wait)
+        new = torch.tensor(tbl[first_new:], dtype=torch.int32, pin_memory=self.block_tables.is_cuda)
+        self.block_tables[slot, first_new:need].copy_(new, non_blocking=True)
 
     def release(self, slot: int) -> None:
         self.allocator.free(self._host_tables[slot])

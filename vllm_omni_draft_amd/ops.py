@@ -20,7 +20,7 @@ def on_gpu() -> bool:
 
 
 def _stream():
-    return torch.cuda.current_stream().cuda_stream if on_gpu() else None
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()) if on_gpu() else None
 
 
 def _p(t: Optional[torch.Tensor]) -> Optional[int]:
@@ -28,10 +28,11 @@ def _p(t: Optional[torch.Tensor]) -> Optional[int]:
 
 
 def _need(t: torch.Tensor, dtype: torch.dtype, name: str) -> None:
-    if on_gpu() and not t.is_cuda:
+    gpu = on_gpu()
+    if gpu and not t.is_cuda:
         raise _lib.SdError(f"{name}: tensor must live on the GPU (got {t.device}); "
                            "the GPU library has no CPU path")
-    if not on_gpu() and t.is_cuda:
+    if not gpu and t.is_cuda:
         raise _lib.SdError(f"{name}: this process runs the CPU build of the library "
                            f"(SD_AMD_BACKEND=cpu) and takes host tensors, got {t.device}")
     if t.dtype != dtype:

@@ -118,7 +118,8 @@ class SeqEngine:
             seen.add(rid)
             if len(toks) < 1:
                 raise ValueError(f"request {rid}: an entry needs at least one token")
-            if len(want) and (min(want) < 0 or max(want) >= len(toks)):
+            ends = (want[0], want[-1]) if isinstance(want, range) and len(want) else want
+            if len(want) and (min(ends) < 0 or max(ends) >= len(toks)):
                 raise ValueError(f"request {rid}: wanted index outside its tokens")
             if rid not in self.seqs:
                 self.add(rid)
@@ -146,7 +147,7 @@ class SeqEngine:
         for i, (_, _, w) in enumerate(plan):
             out_at[i] = acc
             acc += len(w)
-        torch.cuda.current_stream(self.device).synchronize()   # the caller's work on its own stream
+        torch.cuda.current_stream(self.device).synchronize()   # the caller's work on its own stream, page tables
         with torch.cuda.stream(self.stream):
             self._run_passes(plan, done, out_at, logits, trace)
         self.stream.synchronize()
@@ -168,7 +169,8 @@ class SeqEngine:
             if not parts:
                 return
             E = len(parts)
-            # tokens, positions, slots, tokens before them, entries, wanted rows: one array, one copy to the GPU
+            # tokens, positions, slots, tokens before them, entries, wanted rows: one array in pinned memory (which torch gives
+            # back once its copy is done), one copy to the GPU
             rows, dst = [], []
             if R == E:   # single tokens: lists are quicker
                 at = [(*plan[i], lo) for i, lo, _, _ in parts]
@@ -180,15 +182,24 @@ class SeqEngine:
                             dst.append(out_at[i] + j)
                 host = torch.tensor([int(t[lo]) for _, t, _, lo in at] + [s.n + lo for s, _, _, lo in at] +
                                     [s.slot for s, _, _, _ in at] + [int(t[lo - 1]) if lo else s.last for s, t, _, lo in at] +
-                                    ents + rows, dtype=torch.int32)
+                                    ents + rows, dtype=torch.int32, pin_memory=True)
                 self._run_pass(host, R, E, dst, (1, 1), logits, trace)
                 continue
-            batch = np.empty(4 * R + 4 * E, np.int32)
+            wants = []
+            for i, lo, hi, r0 in parts:
+                w = plan[i][2]
+                w = _ints(w) if isinstance(w, list) else w
+                here = np.arange(len(w)) if lo == 0 and hi == len(plan[i][1]) else np.nonzero((w >= lo) & (w < hi))[0]
+                wants.append(w[here] + np.int32(r0 - lo))
+                dst.append(here + out_at[i])
+            host = torch.empty(4 * R + 4 * E + sum(len(w) for w in wants), dtype=torch.int32, pin_memory=True)
+            batch = host.numpy()
+            np.concatenate(wants, out=batch[4 * R + 4 * E:])
             toks, pos, slot, prev = batch[:4 * R].reshape(4, R)
             for e, (i, lo, hi, r0) in enumerate(parts):
-                s, t, w = plan[i]
+                s, t, _ = plan[i]
                 if isinstance(t, list):   # (a single token; numpy does not take all that torch takes)
-                    t, w = _ints(t), _ints(w)
+                    t = _ints(t)
                 r1 = r0 + hi - lo
                 toks[r0:r1] = t[lo:hi]
                 pos[r0:r1] = np.arange(s.n + lo, s.n + hi)
@@ -196,13 +207,8 @@ class SeqEngine:
                 prev[r0] = t[lo - 1] if lo > 0 else s.last
                 prev[r0 + 1:r1] = t[lo:hi - 1]
                 batch[4 * R + 4 * e:4 * R + 4 * e + 4] = s.slot, r0, hi - lo, s.n + lo
-                if len(w):
-                    here = np.arange(len(w)) if lo == 0 and hi == len(t) else np.nonzero((w >= lo) & (w < hi))[0]
-                    rows.append(w[here] + np.int32(r0 - lo))
-                    dst.append(here + out_at[i])
             sizes = [hi - lo for _, lo, hi, _ in parts]
-            self._run_pass(torch.from_numpy(np.concatenate([batch] + rows)), R, E,
-                           np.concatenate(dst) if dst else dst, (min(sizes), max(sizes)), logits, trace)
+            self._run_pass(host, R, E, np.concatenate(dst), (min(sizes), max(sizes)), logits, trace)
 
     def _drop_graphs(self) -> None:
         lib = _lib.load()
@@ -244,7 +250,7 @@ class SeqEngine:
                 rc = lib.sd_graph_end(stream, C.byref(handle))
             _lib.check(rc, "sd_graph_end")
             g["graph"], g["workspace"] = handle, self.model.workspace.data_ptr()
-        dev.copy_(host)
+        dev.copy_(host, non_blocking=True)
         _lib.check(lib.sd_graph_launch(g["graph"], ops._stream()), "sd_graph_launch")
         if O and self._in_row(out_dst):
             logits[out_dst[0]:out_dst[0] + O].copy_(g["logits"][:O])
@@ -263,7 +269,7 @@ class SeqEngine:
         if self.cfg.use_graph and trace is None and R == E and R <= self.cfg.graph_max_rows:
             if self._run_graph_pass(host, R, E, O, out_dst, logits):
                 return
-        dev = host.to(self.device)
+        dev = host.to(self.device, non_blocking=True)
         a = dev[0:R]
         b = dev[R:2 * R]
         c = dev[2 * R:3 * R]

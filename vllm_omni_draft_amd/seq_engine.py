@@ -171,6 +171,7 @@ class SeqEngine:
             E = len(parts)
             # tokens, positions, slots, tokens before them, entries, wanted rows: one array in pinned memory (which torch gives
             # back once its copy is done), one copy to the GPU
+            pinned = logits is not None and logits.is_cuda
             rows, dst = [], []
             if R == E:   # single tokens: lists are quicker
                 at = [(*plan[i], lo) for i, lo, _, _ in parts]
@@ -182,7 +183,7 @@ class SeqEngine:
                             dst.append(out_at[i] + j)
                 host = torch.tensor([int(t[lo]) for _, t, _, lo in at] + [s.n + lo for s, _, _, lo in at] +
                                     [s.slot for s, _, _, _ in at] + [int(t[lo - 1]) if lo else s.last for s, t, _, lo in at] +
-                                    ents + rows, dtype=torch.int32, pin_memory=True)
+                                    ents + rows, dtype=torch.int32, pin_memory=pinned)
                 self._run_pass(host, R, E, dst, (1, 1), logits, trace)
                 continue
             wants = []
@@ -192,7 +193,7 @@ class SeqEngine:
                 here = np.arange(len(w)) if lo == 0 and hi == len(plan[i][1]) else np.nonzero((w >= lo) & (w < hi))[0]
                 wants.append(w[here] + np.int32(r0 - lo))
                 dst.append(here + out_at[i])
-            host = torch.empty(4 * R + 4 * E + sum(len(w) for w in wants), dtype=torch.int32, pin_memory=True)
+            host = torch.empty(4 * R + 4 * E + sum(len(w) for w in wants), dtype=torch.int32, pin_memory=pinned)
             batch = host.numpy()
             np.concatenate(wants, out=batch[4 * R + 4 * E:])
             toks, pos, slot, prev = batch[:4 * R].reshape(4, R)

@@ -77,6 +77,40 @@ def test_packed_prompts_have_the_bits_of_forward_passes(kw):
         model.prompt(one, [(1, prompts[0], 0, True)], got)      # no pages for it
 
 
+@pytest.mark.parametrize("kw", [{}, {"qkv_bias": True, "n_kv_heads": 1, "n_heads": 7}, {"hidden": 512, "n_heads": 8, "head_dim": 128}])
+@pytest.mark.parametrize("lens", [[301, 2, 67], [3, 290, 17, 1], [258]])
+def test_keys_and_values_of_prompts_that_start_anywhere(kw, lens):
+    """Prompts whose rows start at every remainder of four (values go to their pages four tokens at a time where a page allows it), in
+    one pass: the caches of the same prompts in passes of at most 100 rows of one, bit for bit, and nothing else of the pages."""
+    from vllm_omni_draft_amd import config, weights
+    from vllm_omni_draft_amd.engine import _KvView
+    from vllm_omni_draft_amd.kv_cache import PagedKVCache
+    from vllm_omni_draft_amd.model_runner import DecoderModel
+    cfg = config.create_model_config(None, **{**dict(n_layers=1, hidden=256, n_heads=4, n_kv_heads=2, head_dim=64, ffn=512, vocab=512,
+                                                     max_pos=1024), **kw})
+    model = DecoderModel(weights.random_init(cfg, seed=4), 600, wide=True)
+    g = torch.Generator().manual_seed(sum(lens))
+    prompts = [torch.randint(0, cfg.vocab, (n,), generator=g).tolist() for n in lens]
+    caches = []
+    for whole in (True, False):
+        kv = PagedKVCache(cfg, PagedKVCache.pages_for(cfg, len(lens), 600), len(lens), 600)
+        kv.k.fill_(7.0)
+        kv.v.fill_(7.0)
+        for b, n in enumerate(lens):
+            kv.ensure_capacity(b, n)
+        if whole:
+            model.prompt(kv, [(b, p, 0, True) for b, p in enumerate(prompts)], torch.empty(len(lens), cfg.vocab, device="cuda"))
+        else:
+            zero = torch.zeros(1, dtype=torch.int32, device="cuda")
+            for b, p in enumerate(prompts):
+                t = torch.tensor(p, dtype=torch.int32, device="cuda")
+                for c in range(0, len(p), 100):
+                    n = min(100, len(p) - c)
+                    model.forward(_KvView(kv, b), t, 0, c, zero, c, 1, n, torch.empty(n, cfg.vocab, device="cuda"), wide=True)
+        caches.append(kv)
+    assert torch.equal(caches[0].k, caches[1].k) and torch.equal(caches[0].v, caches[1].v)
+
+
 def _model_and_prompts(lens, max_ctx=600):
     from vllm_omni_draft_amd import config, weights
     from vllm_omni_draft_amd.model_runner import DecoderModel

@@ -56,6 +56,45 @@ __device__ __forceinline__ int tile_at(int t, int up_tiles) {
   return t / TN * (TN / 2) + (i < TN / 2 ? i : i - TN / 2 + up_tiles);
 }
 
+// Sixteen token rows (from m0) of a wave's TN tiles of values, from their image in LDS: four tokens of a channel a lane.  Tokens at
+// positions 4 p .. 4 p + 3 of a page are four neighbours of its channel's row; the four lanes of a channel's sixteen
+// tokens and the sixteen channels of a tile are next to each other.  Others (a prompt that starts at a row or a position that is
+// no multiple of four, the last rows) go one by one.
+template <int TN, int LD>
+__device__ __forceinline__ void emit_values(const WideEpiArgs& a, const float* img, const int* pos, int page_at, int m0, int tile0,
+                                            int n_tiles, int lane) {
+  const WideRope& rp = a.rope;
+  const int D = rp.D, tiles_per_head = D / 16;
+  const bool aligned = (reinterpret_cast<uintptr_t>(rp.vc) & 7) == 0;
+#pragma unroll 1
+  for (int n = lane; n < 4 * 16 * TN; n += 64) {
+    const int r = (n & 3) * 4, col = n >> 2, tile = tile0 + (col >> 4), row = col & 15;
+    if (tile >= n_tiles) break;
+    const int head = tile / tiles_per_head, i = (tile - head * tiles_per_head) * 8 + (row & 7) + (row & 8 ? D / 2 : 0);
+    int p[4];
+    bf16x4 v;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      p[k] = pos[r + k];
+      float y = img[(r + k) * LD + col];
+      if (p[k] >= 0 && a.x_scale) y *= a.x_scale[m0 + r + k];
+      if (a.w_scale) y *= a.w_scale[head * D + i];
+      if (a.bias) y += (float)a.bias[head * D + i];
+      v[k] = (bf16_t)y;
+    }
+    const int page = pos[page_at + r];
+    auto at = [&](int pg) { return rp.vc + (((size_t)pg * rp.Hkv + (head - rp.Hq - rp.Hkv)) * D + i) * 16; };
+    if (aligned && (p[0] & 3) == 0 && p[0] >= 0 && p[1] == p[0] + 1 && p[2] == p[0] + 2 && p[3] == p[0] + 3 &&
+        pos[page_at + r + 3] == page) {
+      *reinterpret_cast<bf16x4*>(at(page) + sd_v_slot(p[0] & 15)) = v;
+    } else {
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        if (p[k] >= 0) at(pos[page_at + r + k])[sd_v_slot(p[k] & 15)] = v[k];
+    }
+  }
+}
+
 // Blocks a CU has room for: LDS, and the registers of two sets of accumulators.
 constexpr int blocks_per_cu(int tn, int tm, int stages, bool split) {
   const int lds = 160 / (4 * (tn + tm) * stages), regs = !split || tn * tm > 16 ? 1 : tn * tm <= 4 ? 3 : 2;
@@ -294,6 +333,27 @@ __global__ __launch_bounds__(256, blocks_per_cu(TN, TM, STAGES, SPLIT)) void pro
   float* img = reinterpret_cast<float*>(wave < 2 ? s0 : s1) + (wave & 1) * 16 * kLd;
   const int u = lane % kUnits, ui = PAIRED ? u >> 1 : u >> 2, r0 = PAIRED ? (u & 1) * 4 : (u & 3) * 4;
   const int tile = tile0 + wn * (PAIR ? TN / 2 : TN) + ui;
+  // EPI_QKV_ROPE: positions and pages of the wave's rows, asked for once (a row outside the pass: position -1), and whether the
+  // wave's tiles are values (the last heads): these are written four tokens at a time, a page row of a channel holding its tokens
+  // side by side.
+  constexpr bool QKV = EPI == EPI_QKV_ROPE;
+  int* place = reinterpret_cast<int*>(reinterpret_cast<float*>(wave < 2 ? s0 : s1) + 2 * 16 * kLd) + (wave & 1) * 2 * TM * 16;
+  static_assert(!QKV || (2 * 16 * kLd + 4 * TM * 16) * 4 <= kABytes + kBBytes, "images and places of two waves in a stage");
+  bool values = false;
+  if constexpr (QKV) {
+    const WideRope& rp = a.epi.rope;
+#pragma unroll
+    for (int r = 0; r < TM * 16; r += 64) {
+      const int m = row0 + wm * TM * 16 + r + lane, b = qkv_sequence(rp, min(m, a.M - 1));
+      if (r + lane < TM * 16) {
+        const int pos = m < a.M ? qkv_position(rp, m, b) : -1;
+        place[r + lane] = pos;
+        place[TM * 16 + r + lane] = pos >= 0 ? qkv_page(rp, b, pos) : 0;
+      }
+    }
+    values = (tile0 + wn * TN) / (rp.D / 16) >= rp.Hq + rp.Hkv;
+    asm volatile("" ::: "memory");  // (other lanes read them)
+  }
 #pragma unroll
   for (int j = 0; j < TM; ++j) {
 #pragma unroll
@@ -305,6 +365,12 @@ __global__ __launch_bounds__(256, blocks_per_cu(TN, TM, STAGES, SPLIT)) void pro
       *reinterpret_cast<f32x4*>(img + xc * kLd + i * 16 + 4 * xq) = y;
     }
     asm volatile("" ::: "memory");  // (other lanes read them: the stores of a lane without a unit stay here)
+    if constexpr (QKV) {
+      if (values) {
+        emit_values<TN, kLd>(a.epi, img, place + j * 16, TM * 16, row0 + (wm * TM + j) * 16, tile0 + wn * TN, a.n_tiles, lane);
+        continue;
+      }
+    }
 #pragma unroll 1
     for (int r = lane < 64 / kUnits * kUnits ? lane / kUnits : 16; r < 16; r += 64 / kUnits) {
       const int m = row0 + (wm * TM + j) * 16 + r;
@@ -318,7 +384,10 @@ __global__ __launch_bounds__(256, blocks_per_cu(TN, TM, STAGES, SPLIT)) void pro
               bf16x4{(bf16_t)lo[0], (bf16_t)lo[1], (bf16_t)lo[2], (bf16_t)lo[3]};
         else if constexpr (EPI == EPI_PARTIAL)
           *reinterpret_cast<f32x4*>(a.part + ((size_t)split * a.M + m) * a.n_tiles * 16 + tile * 16 + r0) = lo;
-        else emit_unit<EPI>(a.epi, m, tile, r0, lo, hi);
+        else if constexpr (QKV) {
+          const int pos = place[j * 16 + r];
+          if (pos >= 0) emit_qkv(a.epi, m, tile, r0, lo, hi, qkv_sequence(a.epi.rope, m), pos, place[TM * 16 + j * 16 + r]);
+        } else emit_unit<EPI>(a.epi, m, tile, r0, lo, hi);
       }
     }
   }
@@ -387,10 +456,10 @@ constexpr Shape kWholeShapes[] = {
 float shape_us(const Shape& s, int M, int n_tiles, int K, int S, int epi) {
   const long blocks = (long)((n_tiles + 2 * s.tn - 1) / (2 * s.tn)) * ((M + 32 * s.tm - 1) / (32 * s.tm));
   const long round = 256l * s.per_cu, full = blocks / round, rest = blocks - full * round;
-  // The epilogue that rotates and writes pages moves 2 bytes at a time, and nothing covers that of a large block alone on its
-  // CU.  us of QKV products with it, as chosen without this term / with it: 6144 x 4096 at 4096 rows 248 (128 x 256) / 230 (128 x 128, two a CU),
-  // 4608 x 3584 at 1500 88.6 / 74.0, at 4096 221 / 211, 3072 x 2048 at 2946 82.7 / 79.3; of 40 such products (264..4096 rows) .5 % behind the
-  // best of the nine shapes.
+  // The epilogue that rotates and writes pages is longer than a plain one, and nothing covers that of a large block alone on its CU.
+  // us of QKV products with it, as chosen without this term / with it: 6144 x 4096 at 2500 rows 152 (128 x 256) / 140 (128 x 128, two a CU), at
+  // 4000 226 / 206, 4608 x 3584 at 1500 81.8 / 69.7, 3072 x 2048 at 4000 87.9 / 79.4, 2946 rows 74.2 / 70.4; with .15 or .3 for .5 a tile
+  // between the two.
   const float rope = epi == EPI_QKV_ROPE && S > 1 && s.tn * s.tm > 16 ? .5f * (s.tn * s.tm - 16) : 0.f;
   const float fixed = s.fixed + s.split * S + rope, stages = K / 64;
   float us = full * (fixed + s.stage[s.per_cu - 1] * stages);

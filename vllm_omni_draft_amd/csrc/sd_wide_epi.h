@@ -68,6 +68,102 @@ struct WideEpiArgs {
   WideRope rope;
 };
 
+// Where row m of a QKV product goes: its position, and the page that holds it.
+__device__ __forceinline__ int qkv_sequence(const WideRope& rp, int m) { return rp.q_len == 1 ? m : m / rp.q_len; }
+__device__ __forceinline__ int qkv_position(const WideRope& rp, int m, int b) {
+  return rp.seq_lens[b] + rp.pos_offset + m - b * rp.q_len;
+}
+__device__ __forceinline__ int qkv_page(const WideRope& rp, int b, int pos) {
+  return rp.block_tables[(size_t)(rp.row_seq ? rp.row_seq[b] : b) * rp.max_blocks + (pos >> 4)];
+}
+
+// Four units (i0 .. i0 + 3 and their partners half a head on) of a rotated row: a lane's four queries, and its four keys, lie next
+// to each other in memory, so they are one store of 8 bytes where the buffers' starts allow it (2 bytes at a time, 6144 x 4096 at
+// 1024 rows 82.1 us, 4096 229; now 76.3 and 206; 4608 x 3584 at 2946 rows of 8 prompts 138 and 130).
+__device__ __forceinline__ void emit_qkv(const WideEpiArgs& a, int m, int tile, int r0, f32x4 lo, f32x4 hi, int b, int pos,
+                                         int page) {
+  const WideRope& rp = a.rope;
+  const int D = rp.D, half = D / 2, tiles_per_head = D / 16;
+  const int head = tile / tiles_per_head;
+  const int i0 = (tile - head * tiles_per_head) * 8 + r0;
+  const int slot = pos & 15;
+  if (a.w_scale) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      lo[j] *= a.w_scale[head * D + i0 + j];
+      hi[j] *= a.w_scale[head * D + i0 + j + half];
+    }
+  }
+  if (a.bias) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      lo[j] += (float)a.bias[head * D + i0 + j];
+      hi[j] += (float)a.bias[head * D + i0 + j + half];
+    }
+  }
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    lo[j] = round_bf16(lo[j]);
+    hi[j] = round_bf16(hi[j]);
+  }
+  if (head < rp.Hq + rp.Hkv && rp.cs) {
+    f32x4 c, sn;
+    if (!rp.mp.pos && (reinterpret_cast<uintptr_t>(rp.cs) & 15) == 0) {   // (one position for all of a row)
+      const float* cs = rp.cs + (size_t)min(max(sd_rope_position(rp.mp, pos, b, m, 0), 0), rp.max_pos - 1) * D + i0;
+      c = *reinterpret_cast<const f32x4*>(cs);
+      sn = *reinterpret_cast<const f32x4*>(cs + half);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int r_pos = max(sd_rope_position(rp.mp, pos, b, m, i0 + j), 0);
+        const float* cs = rp.cs + (size_t)min(r_pos, rp.max_pos - 1) * D;
+        c[j] = cs[i0 + j];
+        sn[j] = cs[half + i0 + j];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float nl = lo[j] * c[j] - hi[j] * sn[j], nh = hi[j] * c[j] + lo[j] * sn[j];
+      lo[j] = nl;
+      hi[j] = nh;
+    }
+  }
+  bf16x4 l, h;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    l[j] = (bf16_t)lo[j];
+    h[j] = (bf16_t)hi[j];
+  }
+  auto four = [&](bf16_t* to, const bf16x4& v, bool aligned) __attribute__((always_inline)) {
+    if (aligned) {
+      *reinterpret_cast<bf16x4*>(to) = v;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) to[j] = v[j];
+    }
+  };
+  if (head < rp.Hq) {
+    bf16_t* q = reinterpret_cast<bf16_t*>(a.out) + (size_t)m * a.ldo + (size_t)head * D + i0;
+    const bool aligned = (a.ldo & 3) == 0 && (reinterpret_cast<uintptr_t>(a.out) & 7) == 0;
+    four(q, l, aligned);
+    four(q + half, h, aligned);
+  } else if (head < rp.Hq + rp.Hkv) {
+    bf16_t* kp = rp.kc + ((size_t)page * rp.Hkv + (head - rp.Hq)) * D * 16;
+    const bool aligned = (reinterpret_cast<uintptr_t>(rp.kc) & 7) == 0;
+    const int i2 = i0 + half;
+    four(kp + ((i0 >> 3) * 16 + slot) * 8 + (i0 & 7), l, aligned);
+    four(kp + ((i2 >> 3) * 16 + slot) * 8 + (i2 & 7), h, aligned);
+  } else {
+    bf16_t* vp = rp.vc + ((size_t)page * rp.Hkv + (head - rp.Hq - rp.Hkv)) * D * 16;
+    const int sl = sd_v_slot(slot);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      vp[(i0 + j) * 16 + sl] = l[j];
+      vp[(i0 + j + half) * 16 + sl] = h[j];
+    }
+  }
+}
+
 // The epilogue of 4 consecutive tile rows r0..r0+3 of tile `tile` for token row m: lo holds
 // their sums; in the paired modes hi holds the sums of rows r0+8..r0+11 (the up rows of a
 // gated tile, the rotation partners of a rotary tile) and r0 is 0 or 4.
@@ -84,52 +180,9 @@ __device__ __forceinline__ void emit_unit(const WideEpiArgs& a, int m, int tile,
   }
   if (EPI == EPI_QKV_ROPE) {
     const WideRope& rp = a.rope;
-    const int D = rp.D, half = D / 2, tiles_per_head = D / 16;
-    const int head = tile / tiles_per_head;
-    const int i0 = (tile % tiles_per_head) * 8 + r0;
-    const int b = m / rp.q_len, t = m - b * rp.q_len;
-    const int pos = rp.seq_lens[b] + rp.pos_offset + t;
+    const int b = qkv_sequence(rp, m), pos = qkv_position(rp, m, b);
     if (pos < 0) return;
-    const int page = head >= rp.Hq ? rp.block_tables[(size_t)(rp.row_seq ? rp.row_seq[b] : b) * rp.max_blocks + (pos >> 4)] : 0;
-    const int slot = pos & 15;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int i = i0 + j;
-      float l = lo[j], h = hi[j];
-      if (a.w_scale) {
-        l *= a.w_scale[head * D + i];
-        h *= a.w_scale[head * D + i + half];
-      }
-      if (a.bias) {
-        l += (float)a.bias[head * D + i];
-        h += (float)a.bias[head * D + i + half];
-      }
-      l = round_bf16(l);
-      h = round_bf16(h);
-      if (head < rp.Hq + rp.Hkv && rp.cs) {
-        const int r_pos = max(sd_rope_position(rp.mp, pos, b, m, i), 0);
-        const float* cs = rp.cs + (size_t)min(r_pos, rp.max_pos - 1) * D;
-        const float c = cs[i], sn = cs[half + i];
-        const float nl = l * c - h * sn, nh = h * c + l * sn;
-        l = nl;
-        h = nh;
-      }
-      if (head < rp.Hq) {
-        bf16_t* q = reinterpret_cast<bf16_t*>(a.out) + (size_t)m * a.ldo + (size_t)head * D;
-        q[i] = (bf16_t)l;
-        q[i + half] = (bf16_t)h;
-      } else if (head < rp.Hq + rp.Hkv) {
-        bf16_t* kp = rp.kc + ((size_t)page * rp.Hkv + (head - rp.Hq)) * D * 16;
-        const int i2 = i + half;
-        kp[((i >> 3) * 16 + slot) * 8 + (i & 7)] = (bf16_t)l;
-        kp[((i2 >> 3) * 16 + slot) * 8 + (i2 & 7)] = (bf16_t)h;
-      } else {
-        bf16_t* vp = rp.vc + ((size_t)page * rp.Hkv + (head - rp.Hq - rp.Hkv)) * D * 16;
-        const int sl = sd_v_slot(slot);
-        vp[i * 16 + sl] = (bf16_t)l;
-        vp[(i + half) * 16 + sl] = (bf16_t)h;
-      }
-    }
+    emit_qkv(a, m, tile, r0, lo, hi, b, pos, tile / (rp.D / 16) >= rp.Hq ? qkv_page(rp, b, pos) : 0);
   } else if (EPI == SD_EPI_SILU_MUL) {
     const int n0 = tile * 8 + r0;
     if (n0 + 3 < a.N && ((a.ldo | a.N) & 3) == 0) {  // four outputs in one store

@@ -637,6 +637,21 @@ def test_a_step_larger_than_a_pass():
     assert rel(out[:4], wa[[0, 15, 16, 44]]) < 3e-6 and rel(out[4], wb[20]) < 3e-6
 
 
+@pytest.mark.parametrize("shape", sorted(SHAPES))
+def test_norm_and_router_in_one_launch_have_the_bits_of_two(shape):
+    """More than 256 rows (the norm, then the router) against pieces of 1, 64, 255 and 256 rows (one launch)."""
+    cfg = SHAPES[shape]
+    st, eng = build(cfg, torch.float32)
+    toks = prompt(cfg, 577)
+    want = eng.step([("a", toks, range(577))])
+    eng.finish("a")
+    at, got = 0, []
+    for n in (1, 64, 1, 255, 256):
+        got.append(eng.step([("b", toks[at:at + n], range(n))]))
+        at += n
+    assert at == 577 and torch.equal(torch.cat(got), want)
+
+
 def test_a_far_token_through_the_recurrence_and_a_kept_first_token():
     """The recurrence's decay made (almost) one, so that a token 150 positions back still carries
     weight; and a kept first token whose key every later query finds."""

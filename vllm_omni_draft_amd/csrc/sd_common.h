@@ -111,6 +111,11 @@ int sd_conv_steps_(const float* x, int64_t ldx, const void* w, const void* b, in
                    int taps, int act, const float* dt, const void* dt_bias, const void* a_log, float* step, float* decay, int H,
                    sd_stream_t stream);
 
+// sd_postnorm_residual (one row of a each), and the router's product and choice (sd_moe_route_rows, sigmoid scores) on its result
+int sd_postnorm_route_(float* x, const float* a, float sa, const float* b, float sb, const void* norm_w, int w_f32, float eps,
+                       void* x_bf16, const void* w_router, float* logits, int32_t* sel_expert, float* sel_weight, int n_rows, int E,
+                       int W, int top, sd_stream_t stream);
+
 // sd_window_softmax_attention and sd_window_pool_attention without the rows of long portions (skip_long; the pooled
 // blocks are in the cache already then), whose attention is sd_rows_softmax_attention's and sd_rows_pool_attention's:
 // here with the long portions alone (long_only; all portions' blocks are pooled).

@@ -1747,7 +1747,6 @@ int postnorm_layer(const sd_seq_model& m, const sd_seq_layer& l, const sd_seq_ba
                                   l.w_o_tiled ? yb : nullptr, R, dv, rk, H, stream));
     SQ_TRY(seq_linear(l.w_o, l.w_o_tiled, f32, y, nullptr, (int64_t)H * dv, yb, (int64_t)H * dv, nullptr, mix, W, R, W,
                       H * dv, wide_ws, w.wide_bytes, stream));
-    SQ_TRY(sd_postnorm_residual(x, mix, 1, 1.f, nullptr, 0.f, l.norm_w, f32, eps, hb, R, W, stream));
   } else {
     const int G = l.kv_heads;
     // attention: q and k normed over the whole projection, no rotation
@@ -1790,15 +1789,20 @@ int postnorm_layer(const sd_seq_model& m, const sd_seq_layer& l, const sd_seq_ba
                             inner, R, inner, l.s_norm_groups, rnd, stream));
     SQ_TRY(seq_linear(l.w_o2, l.w_o2_tiled, f32, y, nullptr, inner, yb, inner, nullptr, mix2, W, R, W, inner, wide_ws,
                       w.wide_bytes, stream));
-    SQ_TRY(sd_postnorm_residual(x, mix, 1, l.left_scale, mix2, l.right_scale, l.norm_w, f32, eps, hb, R, W, stream));
   }
-  if (l.n_experts > 0) {
+  // the mixer's result: of the parallel mixer its two sides, weighted
+  const bool two = l.kind != SD_MIX_LATENT;
+  const float sa = two ? l.left_scale : 1.f, sb = two ? l.right_scale : 0.f;
+  const float* side = two ? mix2 : nullptr;
+  if (l.n_experts <= 0) {
+    SQ_TRY(sd_postnorm_residual(x, mix, 1, sa, side, sb, l.norm_w, f32, eps, hb, R, W, stream));
+  } else {
     float* rlog = (float*)(base + w.rlog);
     int32_t* sel_e = (int32_t*)(base + w.sel_e);
     float* sel_w = (float*)(base + w.sel_w);
     float* dn = (float*)(base + w.dn);
     const int E = l.n_experts;
-    SQ_TRY(sd_moe_route_rows(x, W, l.w_router, f32, rlog, sel_e, sel_w, R, E, W, l.top, 0, 0, stream));
+    SQ_TRY(sd_postnorm_route_(x, mix, sa, side, sb, l.norm_w, f32, eps, hb, l.w_router, rlog, sel_e, sel_w, R, E, W, l.top, stream));
     SQ_TRY(sd_moe_experts(x, hb, W, sel_e, sel_w, l.w_gate_up, l.w_down_e, f32, dn, R, l.top, E, l.expert_ff, W, 1, 0,
                           base + w.moe, w.moe_bytes, stream));
     SQ_TRY(sd_postnorm_residual(x, dn, l.top, 1.f, nullptr, 0.f, l.norm2_w, f32, eps, hb, R, W, stream));

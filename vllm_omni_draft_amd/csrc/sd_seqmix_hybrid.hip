@@ -1019,6 +1019,89 @@ __global__ __launch_bounds__(256) void conv_steps_decode_kernel(
     if (s < taps) st[(size_t)(s - 1) * C] = in[s];
 }
 
+// ------------------------------------------------------------------ residual update, norm on the output
+// x += rms_norm(sa * (the sum of the row's n_a rows of a) + sb * b) * w, x_b (or nullptr) the same as bf16.
+template <typename T>
+struct PostNorm {
+  float* x;
+  const float* a;
+  int n_a;
+  float sa;
+  const float* b;
+  float sb;
+  const T* w;
+  float eps;
+  bf16_t* x_b;
+  int W;
+};
+// Row r, by the first 256 threads of a workgroup; the others meet them at the barrier.  keep(c, v): the updated row's channel c.  Reads in
+// batches as in rmsnorm_parts_kernel (4 rows of 2048 columns, two parts: 9.8 us a column at a time, 4.8).
+template <typename T, class F>
+__device__ __forceinline__ void postnorm_row(const PostNorm<T>& p, int r, F keep) {
+  __shared__ float red[4];
+  const int tid = threadIdx.x, W = p.W;
+  float* __restrict__ x = p.x + (size_t)r * W;
+  const float* __restrict__ b = p.b;
+  const T* __restrict__ w_norm = p.w;
+  float t[kRowBatch], xv[kRowBatch], wv[kRowBatch];
+  // columns c, c + 256, ..., the last one again for those past the row
+  auto load = [&](int c) __attribute__((always_inline)) {
+    const float* __restrict__ ar = p.a + (size_t)r * p.n_a * W;
+    float bv[kRowBatch];
+#pragma unroll
+    for (int u = 0; u < kRowBatch; ++u) t[u] = ar[min(c + 256 * u, W - 1)];
+#pragma unroll
+    for (int u = 0; u < kRowBatch; ++u) {
+      const int cc = min(c + 256 * u, W - 1);
+      xv[u] = x[cc];
+      wv[u] = ld_f(w_norm + cc);
+      bv[u] = b ? b[(size_t)r * W + cc] : 0.f;
+    }
+    for (int j = 1; j < p.n_a; ++j) {
+      float v[kRowBatch];
+#pragma unroll
+      for (int u = 0; u < kRowBatch; ++u) v[u] = ar[(size_t)j * W + min(c + 256 * u, W - 1)];
+#pragma unroll
+      for (int u = 0; u < kRowBatch; ++u) t[u] += v[u];
+    }
+#pragma unroll
+    for (int u = 0; u < kRowBatch; ++u) {
+      t[u] *= p.sa;
+      if (b) t[u] += p.sb * bv[u];
+    }
+  };
+  float ss = 0.f;
+  if (tid < 256)
+    for (int c = tid; c < W; c += 256 * kRowBatch) {
+      load(c);
+#pragma unroll
+      for (int u = 0; u < kRowBatch; ++u)
+        if (c + 256 * u < W) ss = fmaf(t[u], t[u], ss);
+    }
+  ss = wave_sum(ss);
+  if (tid < 256 && (tid & 63) == 0) red[tid >> 6] = ss;
+  __syncthreads();
+  if (tid >= 256) return;
+  ss = red[0];
+  for (int w = 1; w < 4; ++w) ss += red[w];
+  const float rstd = 1.f / sqrtf(ss / (float)W + p.eps);
+  for (int c = tid; c < W; c += 256 * kRowBatch) {
+    if (W > 256 * kRowBatch) load(c);   // (a narrower row is still here)
+#pragma unroll
+    for (int u = 0; u < kRowBatch; ++u)
+      if (c + 256 * u < W) {
+        const float xn = xv[u] + t[u] * rstd * wv[u];
+        x[c + 256 * u] = xn;
+        if (p.x_b) p.x_b[(size_t)r * W + c + 256 * u] = (bf16_t)xn;
+        keep(c + 256 * u, xn);
+      }
+  }
+}
+template <typename T>
+__global__ __launch_bounds__(256) void postnorm_residual_kernel(PostNorm<T> p) {
+  postnorm_row(p, blockIdx.x, [](int, float) {});
+}
+
 // ------------------------------------------------------------------ routed experts
 // One wave per row: scores, then `top` rounds of a wave-wide arg-max (lowest index among equals).
 __global__ void moe_route_kernel(const float* __restrict__ logits, int64_t ld, int32_t* __restrict__ sel_e,
@@ -1078,7 +1161,9 @@ __global__ void moe_route_kernel(const float* __restrict__ logits, int64_t ld, i
 // (lanes stride over the row's channels, then a butterfly sum: an order that no other row
 // changes), then the first wave chooses as moe_route_kernel does; with a correction [E] the choice is
 // made by score + correction, the weight is the score.
-template <typename T>
+// POST: the residual update that the row comes out of first (postnorm_row), the row then from LDS; a wave asks for its first expert's
+// weights before that.
+template <typename T, bool POST>
 __global__ __launch_bounds__(1024) void moe_route_rows_kernel(const float* __restrict__ x, int64_t ldx,
                                                              const T* __restrict__ w, float* __restrict__ logits,
                                                              int32_t* __restrict__ sel_e, float* __restrict__ sel_w,
@@ -1087,16 +1172,39 @@ __global__ __launch_bounds__(1024) void moe_route_rows_kernel(const float* __res
                                                              const T* __restrict__ w_gate, int n_gate,
                                                              float* __restrict__ gate_out,
                                                              const float* __restrict__ bias,
-                                                             const float* __restrict__ correction) {
-  extern __shared__ float sc[];   // [E]
+                                                             const float* __restrict__ correction, PostNorm<T> post) {
+  extern __shared__ float sc[];   // [E] (POST: and the row [K])
   const int r = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nw = blockDim.x >> 6;
-  const float* xr = x + (size_t)r * ldx;
+  const float* xr = POST ? sc + E : x + (size_t)r * ldx;
   constexpr int kU = 8;   // loads of a lane in flight
+  constexpr int kFirst = POST ? 4 : 1;   // batches of the first expert's weights asked for ahead
+  T ahead[kFirst][kU];
+  if constexpr (POST) {
+    const T* wr = wave < E ? w + (size_t)wave * K : w;
+#pragma unroll
+    for (int i = 0; i < kFirst; ++i)
+#pragma unroll
+      for (int u = 0; u < kU; ++u) ahead[i][u] = wr[min((i * kU + u) * 64 + lane, K - 1)];
+    postnorm_row(post, r, [&](int c, float v) { sc[E + c] = v; });
+    __syncthreads();
+  }
   // (rows E .. E + n_gate - 1 are further products of the same input: gates computed as the router is)
   for (int e = wave; e < E + n_gate; e += nw) {
     const T* wr = e < E ? w + (size_t)e * K : w_gate + (size_t)(e - E) * K;
     float acc = 0.f;
-    for (int k0 = 0; k0 < K; k0 += 64 * kU) {
+    int from = 0;
+    if constexpr (POST)
+      if (e == wave && e < E) {
+#pragma unroll
+        for (int i = 0; i < kFirst; ++i)
+#pragma unroll
+          for (int u = 0; u < kU; ++u) {
+            const int k = (i * kU + u) * 64 + lane;
+            if (k < K) acc = fmaf(maybe_round(xr[k], round), (float)ahead[i][u], acc);
+          }
+        from = kFirst * kU * 64;
+      }
+    for (int k0 = from; k0 < K; k0 += 64 * kU) {
       float xv[kU], wv[kU];
 #pragma unroll
       for (int u = 0; u < kU; ++u) {   // unguarded, on an index clamped into the row
@@ -1799,63 +1907,7 @@ MoeScratch moe_plan(int n_rows, int top, int E, int F) {
   return s;
 }
 
-// ------------------------------------------------------------------ residual update, norm on the output
-// One workgroup a row; reads in batches as in rmsnorm_parts_kernel (4 rows of 2048 columns, two parts: 9.8 us a
-// column at a time, 4.8).
-template <typename T>
-__global__ __launch_bounds__(256) void postnorm_residual_kernel(float* __restrict__ x, const float* __restrict__ a, int n_a, float sa,
-                                                                const float* __restrict__ b, float sb, const T* __restrict__ w,
-                                                                float eps, bf16_t* __restrict__ x_b, int W) {
-  __shared__ float red[4];
-  const int r = blockIdx.x, tid = threadIdx.x;
-  float t[kRowBatch], xv[kRowBatch], wv[kRowBatch];
-  // columns c, c + 256, ..., the last one again for those past the row
-  auto load = [&](int c) __attribute__((always_inline)) {
-    const float* ar = a + (size_t)r * n_a * W;
-    float bv[kRowBatch];
-#pragma unroll
-    for (int u = 0; u < kRowBatch; ++u) t[u] = ar[min(c + 256 * u, W - 1)];
-#pragma unroll
-    for (int u = 0; u < kRowBatch; ++u) {
-      const int cc = min(c + 256 * u, W - 1);
-      xv[u] = x[(size_t)r * W + cc];
-      wv[u] = ld_f(w + cc);
-      bv[u] = b ? b[(size_t)r * W + cc] : 0.f;
-    }
-    for (int j = 1; j < n_a; ++j) {
-      float v[kRowBatch];
-#pragma unroll
-      for (int u = 0; u < kRowBatch; ++u) v[u] = ar[(size_t)j * W + min(c + 256 * u, W - 1)];
-#pragma unroll
-      for (int u = 0; u < kRowBatch; ++u) t[u] += v[u];
-    }
-#pragma unroll
-    for (int u = 0; u < kRowBatch; ++u) {
-      t[u] *= sa;
-      if (b) t[u] += sb * bv[u];
-    }
-  };
-  float ss = 0.f;
-  for (int c = tid; c < W; c += 256 * kRowBatch) {
-    load(c);
-#pragma unroll
-    for (int u = 0; u < kRowBatch; ++u)
-      if (c + 256 * u < W) ss = fmaf(t[u], t[u], ss);
-  }
-  ss = block_sum(ss, red);
-  const float rstd = 1.f / sqrtf(ss / (float)W + eps);
-  for (int c = tid; c < W; c += 256 * kRowBatch) {
-    if (W > 256 * kRowBatch) load(c);   // (a narrower row is still here)
-#pragma unroll
-    for (int u = 0; u < kRowBatch; ++u)
-      if (c + 256 * u < W) {
-        const float xn = xv[u] + t[u] * rstd * wv[u];
-        x[(size_t)r * W + c + 256 * u] = xn;
-        if (x_b) x_b[(size_t)r * W + c + 256 * u] = (bf16_t)xn;
-      }
-  }
-}
-
+// ------------------------------------------------------------------ a layer normed around its sublayers
 // A layer normed before and after its sublayers, per row, in one launch:
 //   t = the sum of the row's n_a rows of a (+ sigmoid(b_gate[r]) * b[r]);  x += rms_norm(t) * w_post
 // (a == nullptr: no update); x_copy (or nullptr) receives the row as it is then; x += add (a
@@ -2508,13 +2560,13 @@ extern "C" int sd_moe_route_rows_corrected(const float* x, int64_t ldx, const vo
   hipStream_t st = (hipStream_t)stream;
   const int nthr = 64 * (E >= 16 ? 16 : (E >= 8 ? 8 : 4));   // a wave per expert, up to 16 at a time
   if (w_f32)
-    moe_route_rows_kernel<float><<<n_rows, nthr, sizeof(float) * E, st>>>(
+    moe_route_rows_kernel<float, false><<<n_rows, nthr, sizeof(float) * E, st>>>(
         x, ldx, (const float*)w_router, logits, sel_expert, sel_weight, E, K, top, score_kind, renorm, 0, renorm_eps,
-        weight_scale, (const float*)w_gate, n_gate, gate_out, router_bias, correction);
+        weight_scale, (const float*)w_gate, n_gate, gate_out, router_bias, correction, PostNorm<float>{});
   else
-    moe_route_rows_kernel<bf16_t><<<n_rows, nthr, sizeof(float) * E, st>>>(
+    moe_route_rows_kernel<bf16_t, false><<<n_rows, nthr, sizeof(float) * E, st>>>(
         x, ldx, (const bf16_t*)w_router, logits, sel_expert, sel_weight, E, K, top, score_kind, renorm, 1, renorm_eps,
-        weight_scale, (const bf16_t*)w_gate, n_gate, gate_out, router_bias, correction);
+        weight_scale, (const bf16_t*)w_gate, n_gate, gate_out, router_bias, correction, PostNorm<bf16_t>{});
   SD_CHECK_LAUNCH("sd_moe_route_rows");
   return SD_OK;
 }
@@ -2665,10 +2717,37 @@ extern "C" int sd_postnorm_residual(float* x, const float* a, int n_a, float sa,
   SD_REQUIRE(x && a && w && n_a >= 1 && n_rows >= 1 && W >= 1, SD_ERR_INVALID, "sd_postnorm_residual: bad argument");
   hipStream_t st = (hipStream_t)stream;
   if (w_f32)
-    postnorm_residual_kernel<float><<<n_rows, 256, 0, st>>>(x, a, n_a, sa, b, sb, (const float*)w, eps, (bf16_t*)x_bf16, W);
+    postnorm_residual_kernel<<<n_rows, 256, 0, st>>>(PostNorm<float>{x, a, n_a, sa, b, sb, (const float*)w, eps, (bf16_t*)x_bf16, W});
   else
-    postnorm_residual_kernel<bf16_t><<<n_rows, 256, 0, st>>>(x, a, n_a, sa, b, sb, (const bf16_t*)w, eps, (bf16_t*)x_bf16, W);
+    postnorm_residual_kernel<<<n_rows, 256, 0, st>>>(PostNorm<bf16_t>{x, a, n_a, sa, b, sb, (const bf16_t*)w, eps, (bf16_t*)x_bf16, W});
   SD_CHECK_LAUNCH("sd_postnorm_residual");
+  return SD_OK;
+}
+
+// One launch while a workgroup a CU holds all rows: it has 1024 threads, of which the norm uses 256.  us in two launches / in one, 16 experts, 2048
+// columns: 4 rows 16.8 / 9.8, 64 12.5 / 9.6, 200 13.0 / 10.2, 400 15.8 / 18.5, 1000 26.0 / 34.6; 8 experts, 1024 columns: 4 rows 14.2 / 8.0, 64
+// 16.6 / 8.6, 200 10.3 / 8.4, 400 10.3 / 14.7.
+constexpr int kPostRouteRows = 256;
+int sd_postnorm_route_(float* x, const float* a, float sa, const float* b, float sb, const void* norm_w, int w_f32, float eps, void* x_bf16,
+                       const void* w_router, float* logits, int32_t* sel_expert, float* sel_weight, int n_rows, int E, int W, int top,
+                       sd_stream_t stream) {
+  const size_t lds = sizeof(float) * ((size_t)E + W);
+  if (n_rows > kPostRouteRows || lds > 32 * 1024) {
+    const int rc = sd_postnorm_residual(x, a, 1, sa, b, sb, norm_w, w_f32, eps, x_bf16, n_rows, W, stream);
+    return rc != SD_OK ? rc : sd_moe_route_rows(x, W, w_router, w_f32, logits, sel_expert, sel_weight, n_rows, E, W, top, 0, 0, stream);
+  }
+  SD_REQUIRE(x && a && norm_w && w_router && sel_expert && sel_weight && n_rows >= 1 && E >= 1 && W >= 1 && top >= 1 && top <= E,
+             SD_ERR_INVALID, "sd_postnorm_route: bad argument");
+  hipStream_t st = (hipStream_t)stream;
+  auto go = [&](auto* nw, auto* rw) {
+    using T = std::remove_const_t<std::remove_pointer_t<decltype(nw)>>;
+    moe_route_rows_kernel<T, true><<<n_rows, 1024, lds, st>>>(x, W, rw, logits, sel_expert, sel_weight, E, W, top, 0, 0, !w_f32, 0.f, 1.f,
+                                                               (const T*)nullptr, 0, nullptr, nullptr, nullptr,
+                                                               PostNorm<T>{x, a, 1, sa, b, sb, nw, eps, (bf16_t*)x_bf16, W});
+  };
+  if (w_f32) go((const float*)norm_w, (const float*)w_router);
+  else go((const bf16_t*)norm_w, (const bf16_t*)w_router);
+  SD_CHECK_LAUNCH("sd_postnorm_route");
   return SD_OK;
 }
 

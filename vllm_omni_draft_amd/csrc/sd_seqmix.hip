@@ -15,6 +15,8 @@
 #include <algorithm>
 #include <vector>
 
+#include <type_traits>
+
 #include "sd_common.h"
 #include "sd_wide_epi.h"
 
@@ -511,10 +513,16 @@ __device__ __forceinline__ void score_key(const KT* __restrict__ kr, const float
   }
 }
 
+// STAGED (f32 rows of 16, 32, 64 or 128 channels, passes of many rows): 64 keys at a time come through LDS, whole rows a load, and a
+// lane takes a key's product with one head, whose query it reads by scalar loads: the same sums.  (A thread a key reads its row 16 bytes
+// at a time, 64 rows apart in a wave; with all rows' workgroups on a CU the first-level cache holds none of their lines until the
+// next piece, and L2 is read eight times over: 777 rows of 8 heads over 2 of 128 channels 131 us, 107
+// staged; 300 rows 43 / 31, 777 of 64 channels and a window of 256 60 / 40; before, the values' addresses in vector registers too, 151, 49 and 69.)
 // NH: query heads per workgroup (of one kv head), NC: value columns per lane (vdim <= 64 * NC).
 // n_splits > 1: workgroup (.., .., z) takes the keys of tile z / n_hgroups only and writes its sum
 // to out + split * split_stride (sum_splits_kernel adds the splits in order).
-template <typename T, int NH, int NC>
+constexpr int kStagedKeys = 64, kStagedPad = 4;
+template <typename T, int NH, int NC, bool STAGED>
 __global__ __launch_bounds__(256) void window_pool_attn_kernel(
     const float* __restrict__ q, int64_t ldq, const T* __restrict__ k_cache, const T* __restrict__ v_cache,
     const float* __restrict__ pk_cache, const float* __restrict__ pv_cache,
@@ -525,10 +533,11 @@ __global__ __launch_bounds__(256) void window_pool_attn_kernel(
     int n_skip) {
   if (skip && sd_in_long_portion(skip, n_skip, blockIdx.x)) return;   // (entries whose long portions have another kernel)
   extern __shared__ float lds[];
-  unsigned long long* vat = reinterpret_cast<unsigned long long*>(lds);  // [kAttnTile] cache row of the value
-  float* wt = reinterpret_cast<float*>(vat + kAttnTile);                 // [NH][kAttnTile]
+  unsigned long long* vat = reinterpret_cast<unsigned long long*>(lds);  // [kAttnTile] address of the value row (STAGED: first, the key row's)
+  float* wt = reinterpret_cast<float*>(vat + kAttnTile);                 // [kAttnTile][NH]
   float* qs = wt + NH * kAttnTile;                                       // [nh][dk]
   float* red = qs + NH * dk;                                             // [4][nh][dv]
+  float* staged = red;                                                   // [64][dk + 4]  (STAGED: before the sums)
   const int r = blockIdx.x, g = blockIdx.y, tid = threadIdx.x;
   const int hgroup = blockIdx.z % n_hgroups, split = blockIdx.z / n_hgroups;
   const int qh = H / G;
@@ -536,7 +545,8 @@ __global__ __launch_bounds__(256) void window_pool_attn_kernel(
   const int nh = qh - hgroup * NH < NH ? qh - hgroup * NH : NH;
   const int i = row_pos[r];
   const int32_t* tbl = block_tables + (size_t)row_slot[r] * max_blocks;
-  for (int c = tid; c < nh * dk; c += 256) qs[c] = q[(size_t)r * ldq + (size_t)h0 * dk + c];
+  if (!STAGED)
+    for (int c = tid; c < nh * dk; c += 256) qs[c] = q[(size_t)r * ldq + (size_t)h0 * dk + c];
   const int t_first = i - window + 1 > 0 ? i - window + 1 : 0;
   const int n_blocks = i - window + 1 >= 0 ? (i - window + 1) / pool : 0;
   const int total = n_blocks + (i - t_first + 1);
@@ -547,7 +557,7 @@ __global__ __launch_bounds__(256) void window_pool_attn_kernel(
   float bias[NH];
 #pragma unroll
   for (int hq = 0; hq < NH; ++hq) bias[hq] = (head_bias && hq < nh) ? head_bias[h0 + hq] : 0.f;
-  const int wave = tid >> 6, lane = tid & 63;
+  const int wave = tid >> 6, lane = tid & 63, uwave = __builtin_amdgcn_readfirstlane(wave);
   float acc[NH][NC];
 #pragma unroll
   for (int hq = 0; hq < NH; ++hq)
@@ -556,7 +566,58 @@ __global__ __launch_bounds__(256) void window_pool_attn_kernel(
   __syncthreads();
   for (int base = key_lo; base < key_hi; base += kAttnTile) {
     const int idx = base + tid;
-    if (idx < key_hi) {
+    if constexpr (STAGED) {
+      const int n_here = min(key_hi - base, kAttnTile);
+      size_t at = 0;
+      if (idx < key_hi) {
+        if (idx < n_blocks) {
+          const int lp = (idx * pool + pool - 1) / page;
+          at = ((size_t)tbl[lp] * G + g) * pslots + pooled_slot(idx, lp, page, pool);
+          vat[tid] = reinterpret_cast<uintptr_t>(pk_cache + at * dk);
+        } else {
+          const int j = t_first + (idx - n_blocks);
+          at = ((size_t)tbl[j / page] * G + g) * page + j % page;
+          vat[tid] = reinterpret_cast<uintptr_t>(k_cache + at * dk);
+        }
+      }
+      __syncthreads();
+      const int pieces = dk >> 2, per = 256 / pieces, row = tid / pieces, c = (tid - row * pieces) * 4;   // (a power of two)
+      const int n_loads = kStagedKeys / per, ld = dk + kStagedPad;
+      f32x4 raw[8];
+      auto fetch = [&](int sub) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          if (u >= n_loads) break;
+          const int kk = min(sub + row + u * per, n_here - 1);
+          raw[u] = *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(vat[kk]) + c);
+        }
+      };
+      fetch(0);
+      for (int sub = 0; sub < n_here; sub += kStagedKeys) {
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          if (u >= n_loads) break;
+          *reinterpret_cast<f32x4*>(staged + (row + u * per) * ld + c) = raw[u];
+        }
+        __syncthreads();
+        if (sub + kStagedKeys < n_here) fetch(sub + kStagedKeys);
+        for (int hq = uwave; hq < nh; hq += 4) {
+          const float* qh_row = q + (size_t)r * ldq + (size_t)(h0 + hq) * dk;
+          const float* kr = staged + lane * ld;
+          float s = 0.f;
+#pragma unroll 4
+          for (int cc = 0; cc < dk; cc += 4) {
+            const f32x4 kf = *reinterpret_cast<const f32x4*>(kr + cc);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s = fmaf(qh_row[cc + e], kf[e], s);
+          }
+          if (sub + lane < n_here) wt[(sub + lane) * NH + hq] = sigmoid_f(s * scale + (head_bias ? head_bias[h0 + hq] : 0.f));
+        }
+      }
+      // (the last keys were asked for behind the barrier before the one that every wave has passed: nobody reads their addresses any more)
+      if (idx < key_hi) vat[tid] = idx < n_blocks ? reinterpret_cast<uintptr_t>(pv_cache + at * dv) : reinterpret_cast<uintptr_t>(v_cache + at * dv);
+    } else if (idx < key_hi) {
       float s[NH];
 #pragma unroll
       for (int hq = 0; hq < NH; ++hq) s[hq] = 0.f;
@@ -564,16 +625,16 @@ __global__ __launch_bounds__(256) void window_pool_attn_kernel(
         const int last = idx * pool + pool - 1, lp = last / page;
         const size_t at = ((size_t)tbl[lp] * G + g) * pslots + pooled_slot(idx, lp, page, pool);
         score_key<float, NH>(pk_cache + at * dk, qs, dk, nh, vec_p, s);
-        vat[tid] = at;
+        vat[tid] = reinterpret_cast<uintptr_t>(pv_cache + at * dv);
       } else {
         const int j = t_first + (idx - n_blocks);
         const size_t at = ((size_t)tbl[j / page] * G + g) * page + j % page;
         score_key<T, NH>(k_cache + at * dk, qs, dk, nh, vec_t, s);
-        vat[tid] = at;
+        vat[tid] = reinterpret_cast<uintptr_t>(v_cache + at * dv);
       }
 #pragma unroll
       for (int hq = 0; hq < NH; ++hq)
-        if (hq < nh) wt[hq * kAttnTile + tid] = sigmoid_f(s[hq] * scale + bias[hq]);
+        if (hq < nh) wt[tid * NH + hq] = sigmoid_f(s[hq] * scale + bias[hq]);
     }
     __syncthreads();
     const int n_here = key_hi - base < kAttnTile ? key_hi - base : kAttnTile;
@@ -582,35 +643,39 @@ __global__ __launch_bounds__(256) void window_pool_attn_kernel(
     // unguarded loads on clamped addresses.
     const int nb_here = n_blocks - base < 0 ? 0 : (n_blocks - base < n_here ? n_blocks - base : n_here);
     constexpr int kBatch = NC <= 2 ? 2 * kAttnBatch : kAttnBatch;
-    auto sweep = [&](int lo, int hi, auto load_row) {
-      for (int kk0 = lo + wave; kk0 < hi; kk0 += 4 * kBatch) {
+    // (a key is the wave's: its row's address goes to scalar registers, and a lane's columns are an offset that stays)
+    auto sweep = [&](int lo, int hi, auto* type) __attribute__((always_inline)) {
+      using V = std::remove_pointer_t<decltype(type)>;
+      for (int kk0 = lo + uwave; kk0 < hi; kk0 += 4 * kBatch) {
         float vf[kBatch][NC];
 #pragma unroll
         for (int u = 0; u < kBatch; ++u) {
-          const int kk = kk0 + 4 * u < hi ? kk0 + 4 * u : hi - 1;
-          const size_t at = vat[kk];
+          const unsigned long long at = vat[kk0 + 4 * u < hi ? kk0 + 4 * u : hi - 1];
+          const V* row = reinterpret_cast<const V*>((unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(at >> 32)) << 32 |
+                                                    (unsigned)__builtin_amdgcn_readfirstlane((unsigned)at));
 #pragma unroll
-          for (int m = 0; m < NC; ++m) vf[u][m] = load_row(at, lane + 64 * m < dv ? lane + 64 * m : dv - 1);
+          for (int m = 0; m < NC; ++m) vf[u][m] = ld_f(row + (lane + 64 * m < dv ? lane + 64 * m : dv - 1));
         }
 #pragma unroll
         for (int u = 0; u < kBatch; ++u) {
           const int kk = kk0 + 4 * u;
           if (kk < hi) {
+            float w[NH];
+#pragma unroll
+            for (int hq = 0; hq < NH; ++hq) w[hq] = wt[kk * NH + hq];
 #pragma unroll
             for (int hq = 0; hq < NH; ++hq) {
               if (hq < nh) {
-                const float w = wt[hq * kAttnTile + kk];
 #pragma unroll
-                for (int m = 0; m < NC; ++m)
-                  if (lane + 64 * m < dv) acc[hq][m] = fmaf(w, vf[u][m], acc[hq][m]);
+                for (int m = 0; m < NC; ++m) acc[hq][m] = fmaf(w[hq], vf[u][m], acc[hq][m]);   // (columns past the row: not stored)
               }
             }
           }
         }
       }
     };
-    sweep(0, nb_here, [&](size_t at, int col) { return pv_cache[at * dv + col]; });
-    sweep(nb_here, n_here, [&](size_t at, int col) { return ld_f(v_cache + at * dv + col); });
+    sweep(0, nb_here, (float*)nullptr);
+    sweep(nb_here, n_here, (T*)nullptr);
     __syncthreads();
   }
 #pragma unroll
@@ -637,14 +702,14 @@ __global__ void sum_splits_kernel(const float* __restrict__ part, size_t split_s
   out[i] = sum;
 }
 
-template <typename T, int NH>
+template <typename T, int NH, bool STAGED = false>
 void launch_attn_nc(dim3 grid, size_t lds, hipStream_t st, int nc, const float* q, int64_t ldq, const void* kc,
                     const void* vc, const float* pk, const float* pv, const int32_t* row_pos,
                     const int32_t* row_slot, const int32_t* bt, int max_blocks, int page, int pslots, int H, int G,
                     int dk, int dv, int window, int pool, float scale, const float* head_bias, float* out,
                     int n_hgroups, int n_splits, size_t split_stride, const int32_t* skip, int n_skip) {
 #define SD_ATTN_GO(NC)                                                                                           \
-  window_pool_attn_kernel<T, NH, NC><<<grid, 256, lds, st>>>(q, ldq, (const T*)kc, (const T*)vc, pk, pv, row_pos, \
+  window_pool_attn_kernel<T, NH, NC, STAGED><<<grid, 256, lds, st>>>(q, ldq, (const T*)kc, (const T*)vc, pk, pv, row_pos, \
                                                              row_slot, bt, max_blocks, page, pslots, H, G, dk, dv, \
                                                              window, pool, scale, head_bias, out, n_hgroups,       \
                                                              n_splits, split_stride, skip, n_skip)
@@ -1115,7 +1180,15 @@ int sd_window_pool_attention_(const float* q, int64_t ldq, const void* k_cache, 
     else if (NH == 4) SD_ATTN_NH(T, 4); \
     else SD_ATTN_NH(T, 8);            \
   } while (0)
-  if (cache_f32) SD_ATTN_T(float);
+  // (the staged keys lie where the waves' sums come after them; more than a wave's heads, and rows that are not aligned, the other way)
+  const size_t staged = lds + sizeof(float) * (std::max((size_t)kStagedKeys * (dk + kStagedPad), (size_t)4 * nh * dv) - (size_t)4 * nh * dv);
+  const bool many = cache_f32 && !split && n_rows > kAttnSplitRows && NH == 4 && dk >= 16 && dk <= 128 && (dk & (dk - 1)) == 0 &&
+                    staged <= 64 * 1024 && sd_aligned16(k_cache) && sd_aligned16(pk_cache);
+  if (many)
+    launch_attn_nc<float, 4, true>(ga, staged, st, nc, q, ldq, k_cache, v_cache, pk_cache, pv_cache, row_pos, row_slot, block_tables,
+                                   max_blocks, page, pslots, H, G, dk, dv, window, pool, scale, head_bias, dst, n_hgroups, n_splits,
+                                   split_stride, skip_long ? entries : nullptr, n_entries);
+  else if (cache_f32) SD_ATTN_T(float);
   else SD_ATTN_T(bf16_t);
 #undef SD_ATTN_T
 #undef SD_ATTN_NH

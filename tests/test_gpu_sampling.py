@@ -500,7 +500,7 @@ def test_slices_of_a_row_in_one_launch(V, R):
             torch.rand(B, k + 1, generator=g, device="cuda"))
     out = ops.rejection_sample(*args, scratch=plain)
     sc = ops.sampling_scratch(R)
-    # Scores of up to 128 less two different maxima: half of 2^-17 off each; below 2^-126 an exponential (want) or a slice's factor (got) and
+    # Scores of up to 128, rounded or not, less two different maxima: half of 2^-17 off each; below 2^-126 an exponential (want) or a slice's factor (got) and
     # their product are rounded to multiples of 2^-149: 1.5 and 1 of these off.
     off = lambda p: ((p - want).abs() / (2.0 ** -16 * want + 2.5 * 2.0 ** -149)).max().item()
     for _ in range(3):

@@ -1250,7 +1250,8 @@ __device__ __forceinline__ void slice_stats(F entry, K keep, int entries, int n,
   if (!greedy) {
 #pragma unroll UNROLL
     for (int u = 0; u < entries; ++u) {
-      const float e = mx != -INFINITY ? expf(entry(u) * inv_t - mx) : 0.f;
+      // (the product unrounded: the two-launch form's rounding of it is most of its error)
+      const float e = mx != -INFINITY ? expf(fmaf(entry(u), inv_t, -mx)) : 0.f;
       if (tid + u * kPartThreads < n) sum += (double)e;
       keep(u, e);
     }

@@ -530,3 +530,25 @@ def test_slices_of_a_row_in_one_launch(V, R):
             torch.cuda.synchronize()
             assert torch.equal(late, got) and torch.equal(late_ids, ops.sample_rows(got, u, scratch=plain)), i
             assert torch.equal(ops.sample_rows(want, u, scratch=sc), ids)
+
+
+@pytest.mark.parametrize("V", [252, 50272, 128256, 152064, 200000, 400000])
+def test_a_rows_probabilities_do_not_depend_on_what_shares_its_call(V):
+    """The bits of 90 rows in calls of 1, 8, 32, 33 and 60 of them, at the front and at the end, in one launch, in two and over their
+    logits (a seeded request samples the same tokens whatever else is in the batch)."""
+    from vllm_omni_draft_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(V)
+    x = torch.randn(90, V, generator=g, device="cuda") * 3
+    temps = torch.rand(90, generator=g, device="cuda") + 0.3
+    temps[4] = 0.0
+    sc = ops.sampling_scratch(90)
+    plain = torch.empty_like(sc)
+    whole, half = ops.softmax_rows(x, temps, scratch=sc), ops.softmax_rows(x, 0.5, scratch=sc)
+    for n in (1, 8, 32, 33, 60, 90):
+        for at in (0, 90 - n):
+            rows, t = x[at:at + n], temps[at:at + n]
+            for s in (sc, plain):
+                assert torch.equal(ops.softmax_rows(rows, t, scratch=s), whole[at:at + n]), (n, at, s is sc)
+                assert torch.equal(ops.softmax_rows(rows, 0.5, scratch=s), half[at:at + n]), (n, at, s is sc)
+            over = rows.clone()
+            assert torch.equal(ops.softmax_rows(over, t, out=over, scratch=sc), whole[at:at + n]), (n, at)

@@ -839,6 +839,19 @@ __device__ __forceinline__ void part_load(const float* row, int i, int hi, float
   for (int u = 0; u < kPartBatch; ++u) v[u] = row[min(i + u * kPartThreads, hi - 1)];
 }
 
+// What every form of the softmax over slices computes, so that a row has the same bits in each of them and whatever shares its call:
+// an entry's exponential over its slice's maximum (the product unrounded: rounding it is most of an error), times the slice's factor.
+__device__ __forceinline__ float slice_exp(float x, float inv_t, float mx) {
+  return mx != -INFINITY ? expf(fmaf(x, inv_t, -mx)) : 0.f;
+}
+// Factor of every lane's slice from the slices' maxima and sums, a lane a slice, in 64 bits.
+__device__ __forceinline__ float slice_factor(float pm, float ps) {
+  static_assert(kRowParts == 64, "a slice a lane");
+  pm = fmaxf(pm, -INFINITY);
+  const double over = exp((double)pm - (double)wave_max(pm));
+  return (float)(over / wave_sum(pm != -INFINITY ? (double)ps * over : 0.0));
+}
+
 __global__ __launch_bounds__(kPartThreads) void softmax_partial_kernel(
     const float* __restrict__ logits, int64_t ld, RowTemps tm, RowScratch sc, int V) {
   __shared__ float s_f[kPartThreads / 64];
@@ -866,7 +879,7 @@ __global__ __launch_bounds__(kPartThreads) void softmax_partial_kernel(
       if (hi - lo > kPartBatch * kPartThreads) part_load(row, i, hi, v);   // (a shorter slice is still here)
 #pragma unroll
       for (int u = 0; u < kPartBatch; ++u)
-        if (i + u * kPartThreads < hi) sum += (double)expf(v[u] * inv_t - mx);
+        if (i + u * kPartThreads < hi) sum += (double)slice_exp(v[u], inv_t, mx);
     }
   const double total = part_block_sum(sum, s_d);
   if (tid == 0) {
@@ -881,8 +894,7 @@ __global__ __launch_bounds__(kPartThreads) void softmax_finish_kernel(
   const int part = blockIdx.x, r = blockIdx.y, tid = threadIdx.x;
   bool greedy;
   const float inv_t = row_inv_t(tm, r, greedy);
-  // every wave folds the row's slice statistics the same way, a lane a slice, the sum in order of the slices
-  static_assert(kRowParts == 64, "a slice a lane");
+  // every wave folds the row's slice statistics the same way, a lane a slice
   const int lane = tid & 63;
   const float pm = fmaxf(sc.pmax[(size_t)r * kRowParts + lane], -INFINITY);
   const float ps = sc.psum[(size_t)r * kRowParts + lane];
@@ -906,11 +918,7 @@ __global__ __launch_bounds__(kPartThreads) void softmax_finish_kernel(
     for (int i = lo + tid; i < hi; i += kPartThreads) out[i] = i == best ? 1.f : 0.f;
     return;
   }
-  const double term = pm != -INFINITY ? (double)ps * (double)expf(pm - mx) : 0.0;
-  double total = 0.0;
-#pragma unroll
-  for (int p = 0; p < kRowParts; ++p) total += lane_of(term, p);
-  const float inv = (float)(1.0 / total);
+  const float factor = __shfl(slice_factor(pm, ps), part, 64), own = __shfl(pm, part, 64);
   int lo, hi;
   part_range(part, V, lo, hi);
   const float* row = logits + (size_t)r * ld;
@@ -920,7 +928,7 @@ __global__ __launch_bounds__(kPartThreads) void softmax_finish_kernel(
     part_load(row, i, hi, v);
 #pragma unroll
     for (int u = 0; u < kPartBatch; ++u)
-      if (i + u * kPartThreads < hi) out[i + u * kPartThreads] = expf(v[u] * inv_t - mx) * inv;
+      if (i + u * kPartThreads < hi) out[i + u * kPartThreads] = slice_exp(v[u], inv_t, own) * factor;
   }
 }
 
@@ -1174,27 +1182,23 @@ __global__ __launch_bounds__(kPartThreads) void rejection_finish_kernel(
 // the slices of a row have the same number between launches, and a word of another slice is there once its number is the
 // reader's own next one, whatever else is under way.  (A counter a row that all raise: 64 atomic operations on one address, 6 us.)
 // None is ever cleared.  State per row, zero before the first launch on it, used by one launch at a time:
-//   softmax: words [64][2] and [32][2] {maximum, sum};   draws: words [64][3] {mass low, mass high, last index}.
+//   softmax: words [64][2] {maximum, sum};   draws: words [64][3] {mass low, mass high, last index}.
 // Workgroups start in the order of their rows, so the ones a row waits for are running or next; one that has waited for long
 // (`spins` looks) computes the missing slices itself instead, so every wait ends.
-// us in two launches / in one, 128256 entries: softmax of 48 rows 9.4 + 15.1 / 15.1, of 40 8.4 + 13.2 / 13.5; 8 sequences, k = 5: draw 4.7 + 4.8 /
-// 7.7, rejection 4.7 + 9.5 / 8.6; and a launch less each (between 1.5 and 4).
+// us of the 8 sequences' draw and rejection (k = 5, 128256 entries) in two launches / in one: 4.7 + 4.8 / 7.7, 4.7 + 9.5 / 8.6.
 struct OnceState {
-  unsigned long long* soft64;  // [rows][64][2]
-  unsigned long long* soft32;  // [rows][32][2]
-  unsigned long long* draw;    // [rows][64][3]
+  unsigned long long* soft;  // [rows][64][2]
+  unsigned long long* draw;  // [rows][64][3]
 };
-constexpr int kOnceWords = 64 * 2 + 32 * 2 + 64 * 3;   // of a row
+constexpr int kOnceWords = kRowParts * (2 + 3);   // of a row
 inline size_t once_state_bytes(int rows) { return (size_t)rows * kOnceWords * sizeof(unsigned long long); }
 inline OnceState once_state(void* base, int rows) {
   OnceState s;
-  s.soft64 = reinterpret_cast<unsigned long long*>(base);
-  s.soft32 = s.soft64 + (size_t)rows * 64 * 2;
-  s.draw = s.soft32 + (size_t)rows * 32 * 2;
+  s.soft = reinterpret_cast<unsigned long long*>(base);
+  s.draw = s.soft + (size_t)rows * kRowParts * 2;
   return s;
 }
 constexpr int kOnceSpins = 1 << 14;
-constexpr int kOnceRows = 32;   // rows of 64 workgroups of four waves that the chip holds at once
 // The number of a slice's words in this launch
 __device__ __forceinline__ unsigned next_number(const unsigned long long* word) {
   return (unsigned)(__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 32) + 1;
@@ -1202,146 +1206,169 @@ __device__ __forceinline__ unsigned next_number(const unsigned long long* word) 
 __device__ __forceinline__ void tell(unsigned long long* word, unsigned value, unsigned number) {
   __hip_atomic_store(word, (unsigned long long)number << 32 | value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-// The N words of this lane's slice (lanes below `parts`), of one wave; returns the slices that did not come.
+// The N words of this lane's slice, of one wave; returns the slices that did not come.
 template <int N>
-__device__ __forceinline__ unsigned long long hear(const unsigned long long* words, int parts, unsigned number, int spins,
-                                                   unsigned (&value)[N]) {
+__device__ __forceinline__ unsigned long long hear(const unsigned long long* words, unsigned number, int spins, unsigned (&value)[N]) {
   const int lane = threadIdx.x & 63;
   for (int look = 0;; ++look) {
     bool here = true;
-    if (lane < parts)
 #pragma unroll
-      for (int i = 0; i < N; ++i) {
-        const unsigned long long w = __hip_atomic_load(words + lane * N + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        here = here && (unsigned)(w >> 32) == number;
-        value[i] = (unsigned)w;
-      }
+    for (int i = 0; i < N; ++i) {
+      const unsigned long long w = __hip_atomic_load(words + lane * N + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      here = here && (unsigned)(w >> 32) == number;
+      value[i] = (unsigned)w;
+    }
     const unsigned long long missing = __ballot(!here);
     if (!missing || look >= spins) return missing;
     __builtin_amdgcn_s_sleep(1);
   }
 }
 
-// A slice's entries (those past its end: the last one again)
-template <int PARTS>
-__device__ __forceinline__ void once_range(int part, int V, int& lo, int& hi) {
-  const int chunk = ((V + PARTS - 1) / PARTS + 3) & ~3;
-  lo = min(part * chunk, V);
-  hi = min(lo + chunk, V);
+// wave_sum / wave_max of N = 1 or 2 values a lane, the first one's for lane 0, the second one's for lane 32: with two, a half of the wave
+// folds each from the first step on (the same pairs, so the same bits).
+template <int N, class T, class Op>
+__device__ __forceinline__ T wave_fold(const T (&v)[N], Op op) {
+  const int lane = threadIdx.x & 63;
+  T x = v[0];
+  if constexpr (N == 1) x = op(x, __shfl_xor(x, 32, 64));
+  else x = op(lane < 32 ? v[0] : v[1], __shfl_xor(lane < 32 ? v[1] : v[0], 32, 64));
+#pragma unroll
+  for (int o = 16; o > 0; o >>= 1) x = op(x, __shfl_xor(x, o, 64));
+  return x;
 }
-// Maximum of a slice and the sum of its exponentials over that from what its threads hold: entry(u) is the thread's u-th, of `n` in
-// the slice; keep(u, e) takes the exponential.  greedy: the maximum alone.  Whole block.
-template <int UNROLL, class F, class K>
-__device__ __forceinline__ void slice_stats(F entry, K keep, int entries, int n, float inv_t, bool greedy, float& mx, float& total) {
-  __shared__ float s_f[kPartThreads / 64];
-  __shared__ double s_d[kPartThreads / 64];
-  const int tid = threadIdx.x;
-  mx = -INFINITY;
-  if (n > 0)
+// Maxima of N slices and the sums of their exponentials over them from what the threads hold: entry(s, u) is the thread's u-th, of n[s]
+// in slice s; keep(s, u, e) takes the exponential.  greedy: the maxima alone.  Whole block.
+template <int N, int UNROLL, class F, class K>
+__device__ __forceinline__ void slice_stats(F entry, K keep, int entries, const int (&n)[N], float inv_t, bool greedy, float (&mx)[N],
+                                            float (&total)[N]) {
+  constexpr int kWaves = kPartThreads / 64;
+  __shared__ float s_f[N][kWaves];
+  __shared__ double s_d[N][kWaves];
+  const int tid = threadIdx.x, wave = tid >> 6, half = (tid & 63) >> 5;
+  const bool writes = (tid & 31) == 0 && half < N;   // (a lane a slice)
+#pragma unroll
+  for (int s = 0; s < N; ++s) {
+    mx[s] = -INFINITY;
+    if (n[s] > 0)
 #pragma unroll UNROLL
-    for (int u = 0; u < entries; ++u) mx = fmaxf(mx, entry(u) * inv_t);
-  mx = wave_max(mx);
+      for (int u = 0; u < entries; ++u) mx[s] = fmaxf(mx[s], entry(s, u) * inv_t);
+  }
+  const float wave_mx = wave_fold<N>(mx, [](float a, float b) { return fmaxf(a, b); });
   __syncthreads();
-  if ((tid & 63) == 0) s_f[tid >> 6] = mx;
+  if (writes) s_f[half][wave] = wave_mx;
   __syncthreads();
-  mx = s_f[0];
-  for (int w = 1; w < kPartThreads / 64; ++w) mx = fmaxf(mx, s_f[w]);
-  double sum = 0.0;
-  if (!greedy) {
+  double sum[N];
+#pragma unroll
+  for (int s = 0; s < N; ++s) {
+    mx[s] = s_f[s][0];
+    for (int w = 1; w < kWaves; ++w) mx[s] = fmaxf(mx[s], s_f[s][w]);
+    sum[s] = 0.0;
+    if (!greedy) {
 #pragma unroll UNROLL
-    for (int u = 0; u < entries; ++u) {
-      // (the product unrounded: the two-launch form's rounding of it is most of its error)
-      const float e = mx != -INFINITY ? expf(fmaf(entry(u), inv_t, -mx)) : 0.f;
-      if (tid + u * kPartThreads < n) sum += (double)e;
-      keep(u, e);
+      for (int u = 0; u < entries; ++u) {
+        const float e = slice_exp(entry(s, u), inv_t, mx[s]);
+        if (tid + u * kPartThreads < n[s]) sum[s] += (double)e;
+        keep(s, u, e);
+      }
     }
   }
-  total = (float)part_block_sum(sum, s_d);
+  const double wave_total = wave_fold<N>(sum, [](double a, double b) { return a + b; });
+  if (writes) s_d[half][wave] = wave_total;
+  __syncthreads();
+#pragma unroll
+  for (int s = 0; s < N; ++s) {
+    double t = 0.0;
+    for (int w = 0; w < kWaves; ++w) t += s_d[s][w];
+    total[s] = (float)t;
+  }
 }
 
-// Rows in PARTS slices of at most E * kPartThreads entries, which stay in registers from the first reading to the results, their
+// A workgroup has SLICES slices of at most E * kPartThreads entries, which stay in registers from the first reading to the results, their
 // exponentials over the slice's maximum instead of them from its sum on (a slice's factor comes from 64 bits, so a result has no more
-// roundings than one exponential over the row's maximum).  Half the slices where 64 a row would be more workgroups than the
-// chip holds at once.
-template <int PARTS, int E>
-__global__ __launch_bounds__(kPartThreads, E <= 16 ? 6 : 4) void softmax_once_kernel(
+// roundings than one exponential over the row's maximum).
+template <int SLICES, int E>
+__global__ __launch_bounds__(kPartThreads, SLICES * E <= 16 ? 6 : 4) void softmax_once_kernel(
     const float* __restrict__ logits, int64_t ld, RowTemps tm, OnceState state, float* __restrict__ probs, int64_t ld_probs, int V,
     int spins) {
-  __shared__ float s_max[PARTS], s_sum[PARTS], s_factor;
+  __shared__ float s_max[kRowParts], s_sum[kRowParts], s_factor[SLICES];
   __shared__ unsigned long long s_missing;
-  const int part = blockIdx.x, r = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
-  unsigned long long* words = (PARTS == 64 ? state.soft64 : state.soft32) + (size_t)r * PARTS * 2;
-  const unsigned number = tid < 64 ? next_number(words + 2 * part) : 0;   // (the wave that writes them)
+  const int part0 = blockIdx.x * SLICES, r = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+  unsigned long long* words = state.soft + (size_t)r * kRowParts * 2;
+  const unsigned number = tid < 64 ? next_number(words + 2 * part0) : 0;   // (the wave that writes them)
   bool greedy;
   const float inv_t = row_inv_t(tm, r, greedy);   // greedy rows: slice maxima of the raw logits
   const float* row = logits + (size_t)r * ld;
   float* out = probs + (size_t)r * ld_probs;
-  int lo, hi;
-  once_range<PARTS>(part, V, lo, hi);
-  float v[E];
+  int lo[SLICES], hi[SLICES], n[SLICES];
+  float v[SLICES][E];
 #pragma unroll
-  for (int u = 0; u < E; ++u) v[u] = row[min(lo + tid + u * kPartThreads, hi - 1)];
-  float mx, sum;
-  slice_stats<E>([&](int u) { return v[u]; }, [&](int u, float e) { v[u] = e; }, E, hi - lo, inv_t, greedy, mx, sum);
-  if (tid == 0) {
-    tell(words + 2 * part, __float_as_uint(mx), number);
-    tell(words + 2 * part + 1, __float_as_uint(sum), number);
+  for (int s = 0; s < SLICES; ++s) {
+    part_range(part0 + s, V, lo[s], hi[s]);
+    n[s] = hi[s] - lo[s];
+#pragma unroll
+    for (int u = 0; u < E; ++u) v[s][u] = row[min(lo[s] + tid + u * kPartThreads, hi[s] - 1)];   // (past the end: the last one again)
   }
+  float mx[SLICES], sum[SLICES];
+  slice_stats<SLICES, E>([&](int s, int u) { return v[s][u]; }, [&](int s, int u, float e) { v[s][u] = e; }, E, n, inv_t, greedy, mx, sum);
+  if (tid == 0)
+#pragma unroll
+    for (int s = 0; s < SLICES; ++s) {
+      tell(words + 2 * (part0 + s), __float_as_uint(mx[s]), number);
+      tell(words + 2 * (part0 + s) + 1, __float_as_uint(sum[s]), number);
+    }
   if (tid < 64) {
     unsigned value[2];
-    const unsigned long long missing = hear(words, PARTS, number, spins, value);
-    if (lane < PARTS) {
-      s_max[lane] = __uint_as_float(value[0]);
-      s_sum[lane] = __uint_as_float(value[1]);
-    }
+    const unsigned long long missing = hear(words, number, spins, value);
+    s_max[lane] = __uint_as_float(value[0]);
+    s_sum[lane] = __uint_as_float(value[1]);
     if (lane == 0) s_missing = missing;
   }
   __syncthreads();
   for (unsigned long long missing = s_missing; missing; missing &= missing - 1) {
     const int p = __ffsll(missing) - 1;
     int from, end;
-    once_range<PARTS>(p, V, from, end);
-    slice_stats<1>([&](int u) { return row[min(from + tid + u * kPartThreads, end - 1)]; }, [](int, float) {}, E, end - from, inv_t,
-                   greedy, mx, sum);
+    part_range(p, V, from, end);
+    const int late_n[1] = {end - from};
+    float late_mx[1], late_sum[1];
+    slice_stats<1, 1>([&](int, int u) { return row[min(from + tid + u * kPartThreads, end - 1)]; }, [](int, int, float) {}, E, late_n,
+                      inv_t, greedy, late_mx, late_sum);
     if (tid == 0) {
-      s_max[p] = mx;
-      s_sum[p] = sum;
+      s_max[p] = late_mx[0];
+      s_sum[p] = late_sum[0];
     }
     __syncthreads();
   }
   if (greedy) {   // all mass on the first maximum: the lowest slice that holds it, lowest index
     __shared__ int s_first[kPartThreads / 64];
-    const float pm = lane < PARTS ? fmaxf(s_max[lane], -INFINITY) : -INFINITY;
-    mx = wave_max(pm);
-    const int first_part = __ffsll((unsigned long long)__ballot(lane < PARTS && pm == mx)) - 1;
+    const float pm = fmaxf(s_max[lane], -INFINITY), row_max = wave_max(pm);
+    const int first_part = __ffsll((unsigned long long)__ballot(pm == row_max)) - 1;
     int mine = INT_MAX;
-    if (part == first_part)
 #pragma unroll
-      for (int u = 0; u < E; ++u)
-        if (lo + tid + u * kPartThreads < hi && v[u] == mx) mine = min(mine, lo + tid + u * kPartThreads);
+    for (int s = 0; s < SLICES; ++s)
+      if (part0 + s == first_part)
+#pragma unroll
+        for (int u = 0; u < E; ++u)
+          if (lo[s] + tid + u * kPartThreads < hi[s] && v[s][u] == row_max) mine = min(mine, lo[s] + tid + u * kPartThreads);
     for (int o = 32; o > 0; o >>= 1) mine = min(mine, __shfl_xor(mine, o, 64));
     if (lane == 0) s_first[tid >> 6] = mine;
     __syncthreads();
     int best = s_first[0];
     for (int w = 1; w < kPartThreads / 64; ++w) best = min(best, s_first[w]);
-    for (int i = lo + tid; i < hi; i += kPartThreads) out[i] = i == best ? 1.f : 0.f;
+    for (int i = lo[0] + tid; i < hi[SLICES - 1]; i += kPartThreads) out[i] = i == best ? 1.f : 0.f;
     return;
   }
-  if (tid < 64) {   // the row's sum, a lane a slice, in order of the slices
-    const float pm = lane < PARTS ? fmaxf(s_max[lane], -INFINITY) : -INFINITY;
-    const float row_max = wave_max(pm);
-    const double over = exp((double)pm - (double)row_max);
-    const double term = pm != -INFINITY ? (double)s_sum[lane] * over : 0.0;
-    double total = 0.0;
-#pragma unroll
-    for (int p = 0; p < PARTS; ++p) total += lane_of(term, p);
-    if (lane == part) s_factor = (float)(over / total);
+  if (tid < 64) {
+    const float factor = slice_factor(s_max[lane], s_sum[lane]);
+    if (lane >= part0 && lane < part0 + SLICES) s_factor[lane - part0] = factor;
   }
   __syncthreads();
-  const float factor = s_factor;
 #pragma unroll
-  for (int u = 0; u < E; ++u)
-    if (lo + tid + u * kPartThreads < hi) out[lo + tid + u * kPartThreads] = v[u] * factor;
+  for (int s = 0; s < SLICES; ++s) {
+    const float factor = s_factor[s];
+#pragma unroll
+    for (int u = 0; u < E; ++u)
+      if (lo[s] + tid + u * kPartThreads < hi[s]) out[lo[s] + tid + u * kPartThreads] = v[s][u] * factor;
+  }
 }
 
 // A draw from every row's residual, and with bonus_ids the tokens that a sequence emits.  The last slice's workgroup draws.
@@ -1373,7 +1400,7 @@ __global__ __launch_bounds__(kPartThreads) void draw_once_kernel(
   if (draws) {
     if (tid < 64) {
       unsigned value[3] = {0, 0, 0};
-      const unsigned long long missing = hear(words, kRowParts, number, spins, value);
+      const unsigned long long missing = hear(words, number, spins, value);
       s_mass[lane] = __builtin_bit_cast(double, (unsigned long long)value[1] << 32 | value[0]);
       s_last[lane] = (int)value[2];
       if (lane == 0) s_missing = missing;
@@ -2024,6 +2051,14 @@ extern "C" int sd_rejection_sample_split(const float* target_probs, const int64_
 
 extern "C" size_t sd_sampling_state_bytes(int rows) { return rows > 0 ? once_state_bytes(rows) : 0; }
 
+// How many slices a workgroup has, and whether there is one launch (the bits are the same).  Workgroups that wait for their row hold places, so
+// more than 8 rows go in workgroups of two slices, and long slices (more than 12 entries a thread) of more than 20 rows in two launches.
+// us in two launches / one slice a workgroup / two: of 128256 entries 8 rows 8.3 / 7.9 / 8.0, 16 10.7 / 10.4 / 9.0, 33 16.1 / 18.7 / 12.4, 48 20.3 / 21.8 /
+// 15.2, 192 61.7 / 76.5 / 52; of 32000 8 rows 7.5 / 7.0 / 6.7, 48 16.5 / 17.8 / 11.1, 192 48 / 56 / 31; of 152064 8 rows 9.9 / 8.3 / 8.5, 16 13.0 / 10.8 /
+// 10.2, 48 27.9 / 24.1 / 21.9, 256 115 / 126 / 94; of 200000 (long slices) 16 rows 13.7 / 12.8 / 13.8, 24 17.5 / 19.1 / 17.0, 33 23.6 / 23.7 / 26.3, 192 100 /
+// 121 / 105.
+constexpr int kOnceRows = 8, kOnceLong = 12 * kPartThreads, kOnceLongRows = 20;
+
 extern "C" int sd_softmax_rows_once(const float* logits, int64_t ld, const float* temperatures, int rows_per_seq,
                                     float temperature, float* probs, int64_t ld_probs, int R, int V, void* scratch,
                                     void* state, int state_rows, int spins, sd_stream_t stream) {
@@ -2031,26 +2066,28 @@ extern "C" int sd_softmax_rows_once(const float* logits, int64_t ld, const float
                  (temperatures || temperature > 0.f) && (reinterpret_cast<uintptr_t>(state) & 7) == 0,
              SD_ERR_INVALID, "sd_softmax_rows_once: bad arguments (R=%d V=%d rows_per_seq=%d)", R, V, rows_per_seq);
   if (R == 0) return SD_OK;
-  const int parts = R <= kOnceRows ? 64 : 32, chunk = ((V + parts - 1) / parts + 3) & ~3;
+  const int chunk = ((V + kRowParts - 1) / kRowParts + 3) & ~3;
+  const int slices = chunk > kOnceLong || R <= kOnceRows ? 1 : 2;
   const float *in_end = logits + (size_t)(R - 1) * ld + V, *out_end = probs + (size_t)(R - 1) * ld_probs + V;
   const bool apart = in_end <= probs || out_end <= logits;   // (a late workgroup reads its row again)
-  if (R > state_rows || !apart || chunk > 24 * kPartThreads)
+  if (R > state_rows || !apart || chunk > 24 * kPartThreads || (chunk > kOnceLong && R > kOnceLongRows))
     return temperatures ? sd_softmax_rows_seq(logits, ld, temperatures, rows_per_seq, probs, ld_probs, R, V, scratch, stream)
                         : sd_softmax_rows_split(logits, ld, temperature, probs, ld_probs, R, V, scratch, stream);
   const RowTemps tm{temperatures, rows_per_seq, temperatures ? 1.f : 1.0f / temperature};
   const OnceState st = once_state(state, state_rows);
   const int n = spins < 0 ? kOnceSpins : spins;
   auto go = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, dim3(parts, R), dim3(kPartThreads), 0, (hipStream_t)stream, logits, ld, tm, st, probs, ld_probs, V, n);
+    hipLaunchKernelGGL(kernel, dim3(kRowParts / slices, R), dim3(kPartThreads), 0, (hipStream_t)stream, logits, ld, tm, st, probs, ld_probs, V, n);
   };
-  if (parts == 64) {
-    if (chunk <= 8 * kPartThreads) go(softmax_once_kernel<64, 8>);
-    else if (chunk <= 12 * kPartThreads) go(softmax_once_kernel<64, 12>);
-    else go(softmax_once_kernel<64, 24>);
+  if (slices == 1) {
+    if (chunk <= 4 * kPartThreads) go(softmax_once_kernel<1, 4>);
+    else if (chunk <= 8 * kPartThreads) go(softmax_once_kernel<1, 8>);
+    else if (chunk <= 12 * kPartThreads) go(softmax_once_kernel<1, 12>);
+    else go(softmax_once_kernel<1, 24>);
   } else {
-    if (chunk <= 8 * kPartThreads) go(softmax_once_kernel<32, 8>);
-    else if (chunk <= 16 * kPartThreads) go(softmax_once_kernel<32, 16>);
-    else go(softmax_once_kernel<32, 24>);
+    if (chunk <= 4 * kPartThreads) go(softmax_once_kernel<2, 4>);
+    else if (chunk <= 8 * kPartThreads) go(softmax_once_kernel<2, 8>);
+    else go(softmax_once_kernel<2, 12>);
   }
   SD_CHECK_LAUNCH("sd_softmax_rows_once");
   return SD_OK;

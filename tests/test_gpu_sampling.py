@@ -552,3 +552,42 @@ def test_a_rows_probabilities_do_not_depend_on_what_shares_its_call(V):
                 assert torch.equal(ops.softmax_rows(rows, 0.5, scratch=s), half[at:at + n]), (n, at, s is sc)
             over = rows.clone()
             assert torch.equal(ops.softmax_rows(over, t, out=over, scratch=sc), whole[at:at + n]), (n, at)
+
+
+@pytest.mark.parametrize("V", [4, 252, 32000, 152064])
+def test_softmax_of_rows_with_infinities_and_nan(V):
+    """NaN over whole slices of a row (which stay NaN; the rest of the row is what it is without them), a single NaN, all of a row -inf or
+    NaN, +inf (all of the row NaN): one launch and two, and what each entry is."""
+    from vllm_omni_draft_amd import ops
+    nan, inf = float("nan"), float("inf")
+    g = torch.Generator(device="cuda").manual_seed(V)
+    x = torch.randn(20, V, generator=g, device="cuda")
+    chunk = (-(-V // 64) + 3) // 4 * 4                      # entries a slice
+    x[0, -(-V // 2) // chunk * chunk:] = nan                # whole slices (V = 4: all of the row)
+    x[1, :chunk] = nan
+    x[2, :chunk] = -inf
+    x[2, 1] = nan
+    x[3] = nan
+    x[4] = -inf
+    x[5, V // 2] = nan
+    x[6, V // 2] = inf
+    x[7, : V // 2] = -inf
+    sc = ops.sampling_scratch(20)
+    plain = torch.empty_like(sc)
+    for temp in (torch.full((20,), 0.8, device="cuda"), 0.8):
+        for n in (8, 20):
+            t = temp if isinstance(temp, float) else temp[:n]
+            got = ops.softmax_rows(x[:n], t, scratch=sc)
+            want = ops.softmax_rows(x[:n], t, scratch=plain)
+            assert torch.equal(got.nan_to_num(nan=-1.0), want.nan_to_num(nan=-1.0))
+            ref = x[:n].double() / 0.8
+            for r in range(n):
+                bad = torch.isnan(ref[r])
+                whole = bad | (ref[r] == -inf)
+                slices = torch.nn.functional.pad(whole, (0, -V % chunk), value=True).view(-1, chunk).all(1).repeat_interleave(chunk)[:V]
+                if (bad & ~slices).any() or (ref[r] == inf).any() or slices.all():
+                    assert torch.isnan(got[r]).all(), r
+                else:
+                    assert torch.equal(torch.isnan(got[r]), bad), r
+                    p = torch.softmax(torch.where(bad, -inf, ref[r]), -1)
+                    torch.testing.assert_close(got[r][~bad].double(), p[~bad], rtol=2.0 ** -16, atol=2.0 ** -140)

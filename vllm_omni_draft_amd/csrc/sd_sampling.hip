@@ -841,8 +841,12 @@ __device__ __forceinline__ void part_load(const float* row, int i, int hi, float
 
 // What every form of the softmax over slices computes, so that a row has the same bits in each of them and whatever shares its call:
 // an entry's exponential over its slice's maximum (the product unrounded: rounding it is most of an error), times the slice's factor.
+// A slice whose maximum is -inf holds nothing but -inf, whose exponential is 0, and NaN, which stays (and counts in no sum, so the
+// rest of the row is what it would be without).
 __device__ __forceinline__ float slice_exp(float x, float inv_t, float mx) {
-  return mx != -INFINITY ? expf(fmaf(x, inv_t, -mx)) : 0.f;
+  if (mx != -INFINITY) return expf(fmaf(x, inv_t, -mx));
+  const float y = x * inv_t;
+  return y == -INFINITY ? 0.f : y;
 }
 // Factor of every lane's slice from the slices' maxima and sums, a lane a slice, in 64 bits.
 __device__ __forceinline__ float slice_factor(float pm, float ps) {
@@ -1267,7 +1271,7 @@ __device__ __forceinline__ void slice_stats(F entry, K keep, int entries, const 
 #pragma unroll UNROLL
       for (int u = 0; u < entries; ++u) {
         const float e = slice_exp(entry(s, u), inv_t, mx[s]);
-        if (tid + u * kPartThreads < n[s]) sum[s] += (double)e;
+        if (tid + u * kPartThreads < n[s] && mx[s] != -INFINITY) sum[s] += (double)e;
         keep(s, u, e);
       }
     }

@@ -1182,30 +1182,43 @@ __global__ __launch_bounds__(kPartThreads) void rejection_finish_kernel(
 
 // ---- the split forms in one launch each.
 // What the slices of a row tell each other goes through words of {value, number}, written and read whole at the scope of the
-// device.  A slice's words are written once a launch, by its own workgroup, which counts their number up from what it finds there; so
-// the slices of a row have the same number between launches, and a word of another slice is there once its number is the
-// reader's own next one, whatever else is under way.  (A counter a row that all raise: 64 atomic operations on one address, 6 us.)
-// None is ever cleared.  State per row, zero before the first launch on it, used by one launch at a time:
-//   softmax: words [64][2] {maximum, sum};   draws: words [64][3] {mass low, mass high, last index}.
+// device, and the number says which launch wrote them.  A row has a counter that each of its 64 slices raises by one in every launch,
+// after it has read it, so all of them read the same multiple of 64 and something, whatever else is under way, and the number is the multiple
+// and one: another one in every launch, and nothing is ever cleared.  Two launches at a time on one state, which it is not made
+// for, are wrong while they last; the next one starts from the multiple that both left.  Nobody waits for the counter (64 atomic operations
+// on one address, 6 us where all of them were waited for).
+// State per row, zero before the first launch on it, used by one launch at a time:
+//   softmax: words [64][2] {maximum, sum};   draws: words [64][3] {mass low, mass high, last index};   behind all words, a row's two counters.
 // Workgroups start in the order of their rows, so the ones a row waits for are running or next; one that has waited for long
 // (`spins` looks) computes the missing slices itself instead, so every wait ends.
 // us of the 8 sequences' draw and rejection (k = 5, 128256 entries) in two launches / in one: 4.7 + 4.8 / 7.7, 4.7 + 9.5 / 8.6.
 struct OnceState {
   unsigned long long* soft;  // [rows][64][2]
   unsigned long long* draw;  // [rows][64][3]
+  unsigned long long* count; // [rows][2 lines]: softmax, draws
 };
+constexpr int kOnceCount = 16;   // (a counter has a line of its own)
 constexpr int kOnceWords = kRowParts * (2 + 3);   // of a row
-inline size_t once_state_bytes(int rows) { return (size_t)rows * kOnceWords * sizeof(unsigned long long); }
+inline size_t once_state_bytes(int rows) {
+  return (size_t)rows * (kOnceWords + 2 * kOnceCount) * sizeof(unsigned long long);
+}
 inline OnceState once_state(void* base, int rows) {
   OnceState s;
   s.soft = reinterpret_cast<unsigned long long*>(base);
   s.draw = s.soft + (size_t)rows * kRowParts * 2;
+  s.count = s.draw + (size_t)rows * kRowParts * 3;
   return s;
 }
 constexpr int kOnceSpins = 1 << 14;
-// The number of a slice's words in this launch
-__device__ __forceinline__ unsigned next_number(const unsigned long long* word) {
-  return (unsigned)(__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 32) + 1;
+// The number of a row's words in this launch, for the first wave, which writes and reads them: there behind the next barrier, and then
+// the last wave counts the workgroup's slices (not the first one, whose next loads would wait for that).
+__device__ __forceinline__ unsigned this_number(const unsigned long long* count) {
+  return threadIdx.x < 64 ? (unsigned)(__hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) / kRowParts) + 1 : 0;
+}
+__device__ __forceinline__ void have(unsigned number) { asm volatile("" ::"v"(number) : "memory"); }
+__device__ __forceinline__ void count_slices(unsigned long long* count, int slices) {
+  if (threadIdx.x == kPartThreads - 1)
+    __hip_atomic_fetch_add(count, (unsigned long long)slices, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ void tell(unsigned long long* word, unsigned value, unsigned number) {
   __hip_atomic_store(word, (unsigned long long)number << 32 | value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1298,7 +1311,8 @@ __global__ __launch_bounds__(kPartThreads, SLICES * E <= 16 ? 6 : 4) void softma
   __shared__ unsigned long long s_missing;
   const int part0 = blockIdx.x * SLICES, r = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
   unsigned long long* words = state.soft + (size_t)r * kRowParts * 2;
-  const unsigned number = tid < 64 ? next_number(words + 2 * part0) : 0;   // (the wave that writes them)
+  unsigned long long* count = state.count + (size_t)r * 2 * kOnceCount;
+  const unsigned number = this_number(count);
   bool greedy;
   const float inv_t = row_inv_t(tm, r, greedy);   // greedy rows: slice maxima of the raw logits
   const float* row = logits + (size_t)r * ld;
@@ -1313,13 +1327,13 @@ __global__ __launch_bounds__(kPartThreads, SLICES * E <= 16 ? 6 : 4) void softma
     for (int u = 0; u < E; ++u) v[s][u] = row[min(lo[s] + tid + u * kPartThreads, hi[s] - 1)];   // (past the end: the last one again)
   }
   float mx[SLICES], sum[SLICES];
+  have(number);
   slice_stats<SLICES, E>([&](int s, int u) { return v[s][u]; }, [&](int s, int u, float e) { v[s][u] = e; }, E, n, inv_t, greedy, mx, sum);
-  if (tid == 0)
-#pragma unroll
-    for (int s = 0; s < SLICES; ++s) {
-      tell(words + 2 * (part0 + s), __float_as_uint(mx[s]), number);
-      tell(words + 2 * (part0 + s) + 1, __float_as_uint(sum[s]), number);
-    }
+  count_slices(count, SLICES);
+  if (tid < 2 * SLICES) {
+    const float m = tid < 2 ? mx[0] : mx[SLICES - 1], t = tid < 2 ? sum[0] : sum[SLICES - 1];
+    tell(words + 2 * part0 + tid, __float_as_uint(tid & 1 ? t : m), number);
+  }
   if (tid < 64) {
     unsigned value[2];
     const unsigned long long missing = hear(words, number, spins, value);
@@ -1384,7 +1398,8 @@ __global__ __launch_bounds__(kPartThreads) void draw_once_kernel(
   __shared__ unsigned long long s_missing;
   const int part = blockIdx.x, r = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
   unsigned long long* words = state.draw + (size_t)r * kRowParts * 3;
-  const unsigned number = tid < 64 ? next_number(words + 3 * part) : 0;   // (the wave that writes them)
+  unsigned long long* count = state.count + ((size_t)r * 2 + 1) * kOnceCount;
+  const unsigned number = this_number(count);
   const float *p, *q;
   int j, L;
   const bool draws = residual_rows(a, r, V, p, q, j, L);
@@ -1392,13 +1407,13 @@ __global__ __launch_bounds__(kPartThreads) void draw_once_kernel(
   int last_pos;
   if (draws) {
     slice_mass(p, q, part, V, total, last_pos);
-    if (tid == 0) {
-      const unsigned long long m = __builtin_bit_cast(unsigned long long, total);
-      tell(words + 3 * part, (unsigned)m, number);
-      tell(words + 3 * part + 1, (unsigned)(m >> 32), number);
-      tell(words + 3 * part + 2, (unsigned)last_pos, number);
-    }
+    const int last_at = __builtin_amdgcn_readfirstlane(last_pos);
+    const unsigned long long m = __builtin_bit_cast(unsigned long long, total);
+    if (tid < 3) tell(words + 3 * part + tid, tid == 0 ? (unsigned)m : tid == 1 ? (unsigned)(m >> 32) : (unsigned)last_at, number);
   }
+  have(number);
+  __syncthreads();
+  count_slices(count, 1);   // (also where nothing is drawn: every slice, every launch)
   if (part != kRowParts - 1) return;
   int64_t tok;
   if (draws) {
@@ -2057,10 +2072,10 @@ extern "C" size_t sd_sampling_state_bytes(int rows) { return rows > 0 ? once_sta
 
 // How many slices a workgroup has, and whether there is one launch (the bits are the same).  Workgroups that wait for their row hold places, so
 // more than 8 rows go in workgroups of two slices, and long slices (more than 12 entries a thread) of more than 20 rows in two launches.
-// us in two launches / one slice a workgroup / two: of 128256 entries 8 rows 8.3 / 7.9 / 8.0, 16 10.7 / 10.4 / 9.0, 33 16.1 / 18.7 / 12.4, 48 20.3 / 21.8 /
-// 15.2, 192 61.7 / 76.5 / 52; of 32000 8 rows 7.5 / 7.0 / 6.7, 48 16.5 / 17.8 / 11.1, 192 48 / 56 / 31; of 152064 8 rows 9.9 / 8.3 / 8.5, 16 13.0 / 10.8 /
-// 10.2, 48 27.9 / 24.1 / 21.9, 256 115 / 126 / 94; of 200000 (long slices) 16 rows 13.7 / 12.8 / 13.8, 24 17.5 / 19.1 / 17.0, 33 23.6 / 23.7 / 26.3, 192 100 /
-// 121 / 105.
+// us in two launches / one slice a workgroup / two: of 128256 entries 8 rows 8.4 / 7.9 / 8.0, 16 10.3 / 9.9 / 9.0, 33 15.6 / 18.4 / 12.0, 48 19.5 / 21.0 /
+// 14.6, 192 57 / 71 / 47; of 32000 4 rows 6.9 / 6.1 / 6.5, 8 7.5 / 7.1 / 6.5, 48 14.3 / 17.9 / 9.9, 192 39 / 56 / 28; of 152064 8 rows 9.6 / 8.5 / 8.7, 16
+// 12.1 / 10.9 / 10.0, 48 24.7 / 23.1 / 20.9, 256 100 / 121 / 86; of 200000 (long slices) in two launches / one of one slice a workgroup: 16 rows 13.1 / 12.6,
+// 24 16.6 / 19.9, 48 28.5 / 32.0, 192 90 / 120.
 constexpr int kOnceRows = 8, kOnceLong = 12 * kPartThreads, kOnceLongRows = 20;
 
 extern "C" int sd_softmax_rows_once(const float* logits, int64_t ld, const float* temperatures, int rows_per_seq,

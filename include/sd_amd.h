@@ -181,9 +181,9 @@ int sd_rejection_sample_split(const float* target_probs, const int64_t* bonus_id
  * three functions; of one stream at a time, like scratch: calls that overlap may give wrong results, the ones
  * after them do not).  sd_softmax_rows_once: temperatures as sd_softmax_rows_seq, or NULL and one temperature.
  * spins: how often a workgroup looks for another slice's numbers before it computes them itself; negative: the
- * default.  Rows beyond state_rows, results over their own logits and long slices (many rows of them, or too
- * long for registers) take the split forms, with `scratch`.  A row's bits are those of the split forms, and do
- * not depend on R.                                                                                     */
+ * default.  Rows beyond state_rows, draws of many rows, results over their own logits and long slices (many rows
+ * of them, or too long for registers) take the split forms, with `scratch`.  A row's bits are those of the split
+ * forms, and do not depend on R.                                                                        */
 size_t sd_sampling_state_bytes(int state_rows);
 int sd_softmax_rows_once(const float* logits, int64_t ld, const float* temperatures, int rows_per_seq,
                          float temperature, float* probs, int64_t ld_probs, int R, int V, void* scratch,

@@ -616,3 +616,24 @@ def test_a_sampling_buffer_after_calls_that_overlapped():
     for i in (2, 3, 0, 1):
         assert torch.equal(ops.softmax_rows(x[i], 0.9, scratch=sc), want[i]), i
         assert torch.equal(ops.sample_rows(want[i][:16], u[:16], scratch=sc), ids[i]), i
+
+
+def test_a_sampling_buffer_made_under_capture():
+    """A buffer made while its stream is captured takes the launches that need no state, with the same bits, replay after replay."""
+    from vllm_omni_draft_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(9)
+    x, u = torch.randn(6, 32000, generator=g, device="cuda"), torch.rand(6, generator=g, device="cuda")
+    sc = ops.sampling_scratch(6)
+    want = ops.softmax_rows(x, 0.9, scratch=sc)
+    ids = ops.sample_rows(want, u, scratch=sc)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        own = ops.sampling_scratch(6)
+        got = ops.softmax_rows(x, 0.9, scratch=own)
+        got_ids = ops.sample_rows(got, u, scratch=own)
+    for _ in range(3):
+        got.zero_()
+        graph.replay()
+        assert torch.equal(got, want) and torch.equal(got_ids, ids)
+        assert torch.equal(ops.softmax_rows(x, 0.9, scratch=sc), want)

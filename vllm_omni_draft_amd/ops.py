@@ -53,10 +53,11 @@ def device_info():
 def sampling_scratch(rows: int, device="cuda") -> torch.Tensor:
     """Scratch for the split (many-workgroups-per-row) forms of softmax_rows, sample_rows and
     rejection_sample over up to `rows` rows / sequences.  It carries the state with which these run in one launch each
-    (another buffer of sd_sampling_scratch_bytes(rows) bytes does too, in two launches); one stream at a time uses it."""
+    (another buffer of sd_sampling_scratch_bytes(rows) bytes does too, in two launches, as does one made while the stream is
+    being captured, where nothing can be zeroed before its use); one stream at a time uses it."""
     lib = _lib.load()
     scratch = torch.empty(max(int(lib.sd_sampling_scratch_bytes(rows)), 16), dtype=torch.uint8, device=device)
-    if scratch.is_cuda and rows > 0:
+    if scratch.is_cuda and rows > 0 and not torch.cuda.is_current_stream_capturing():
         scratch.sd_state = torch.zeros(int(lib.sd_sampling_state_bytes(rows)), dtype=torch.uint8, device=device)
         scratch.sd_state_rows = rows
         torch.cuda.current_stream(scratch.device).synchronize()   # (zero for whatever stream uses it)

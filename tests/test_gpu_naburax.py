@@ -637,6 +637,29 @@ def test_a_step_larger_than_a_pass():
     assert rel(out[:4], wa[[0, 15, 16, 44]]) < 3e-6 and rel(out[4], wb[20]) < 3e-6
 
 
+def test_page_tables_are_there_for_any_stream_after_a_refused_step():
+    """A step refused at its second entry, under a stream that is busy: the first entry's pages are in the table for a step under another
+    stream; and so are those that SeqCache.ensure_capacity took."""
+    from vllm_omni_draft_amd.kv_cache import OutOfPages
+    cfg = SHAPES[sorted(SHAPES)[0]]
+    toks = prompt(cfg, 200)
+    want = build(cfg)[1].step([("a", toks, range(200))])
+    _, eng = build(cfg)
+    eng.step([("pad", prompt(cfg, 40, 9), [])])        # (the pages of "a" are not the table's zeros)
+    busy = torch.cuda.Stream()
+    with torch.cuda.stream(busy):
+        torch.cuda._sleep(50_000_000)
+        with pytest.raises(OutOfPages):
+            eng.step([("a", toks, range(200)), ("b", [1] * 5000, [])])
+    assert busy.query()
+    assert torch.equal(eng.step([("a", toks, range(200))]), want)
+    slot = eng.seqs["a"].slot
+    with torch.cuda.stream(busy):
+        torch.cuda._sleep(50_000_000)
+        eng.cache.ensure_capacity(slot, 500)
+    assert eng.cache.block_tables[slot, :32].tolist() == eng.cache.pages_of(slot)
+
+
 @pytest.mark.parametrize("shape", sorted(SHAPES))
 def test_norm_and_router_in_one_launch_have_the_bits_of_two(shape):
     """More than 256 rows (the norm, then the router) against pieces of 1, 64, 255 and 256 rows (one launch)."""

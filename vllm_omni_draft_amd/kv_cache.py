@@ -237,8 +237,9 @@ class SeqCache:
     def pages_of(self, slot: int) -> List[int]:
         return self._host_tables[slot]
 
-    def ensure_capacity(self, slot: int, n_tokens: int) -> None:
-        """Slot `slot` owns pages for positions 0..n_tokens-1 afterwards (window layers only)."""
+    def ensure_capacity(self, slot: int, n_tokens: int, wait: bool = True) -> None:
+        """Slot `slot` owns pages for positions 0..n_tokens-1 afterwards (window layers only), and the device's table says so for
+        whatever stream reads it next; with wait=False once the caller's current stream has come that far."""
         if not self.has_pages:
             return
         need = (n_tokens + PAGE - 1) // PAGE
@@ -251,9 +252,10 @@ class SeqCache:
             raise OutOfPages("KV cache is out of pages")
         first_new = len(tbl)
         tbl += [self.allocator.alloc() for _ in range(need - first_new)]
-        # (from pinned memory, in order on the caller's stream: the host does not wait)
         new = torch.tensor(tbl[first_new:], dtype=torch.int32, pin_memory=self.block_tables.is_cuda)
         self.block_tables[slot, first_new:need].copy_(new, non_blocking=True)
+        if wait and self.block_tables.is_cuda:
+            torch.cuda.current_stream(self.block_tables.device).synchronize()
 
     def release(self, slot: int) -> None:
         self.allocator.free(self._host_tables[slot])

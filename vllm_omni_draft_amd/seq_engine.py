@@ -110,6 +110,36 @@ class SeqEngine:
         the device, in the order of the entries and of their indices (and, with layer_out, the
         residual after every layer run, [layer runs, rows, width]; a layer that runs several times
         over counts each time)."""
+        try:
+            plan = self._plan(entries)
+            n_want = sum(len(w) for _, _, w in plan)
+            V = self.model_cfg.vocab
+            logits = torch.empty(n_want, V, dtype=torch.float32, device=self.device)
+            total = sum(len(t) for _, t, _ in plan)
+            if layer_out and total > self.cfg.max_rows:
+                raise ValueError("layer_out needs a step of at most max_rows rows")
+            trace = (torch.empty(self.model_cfg.n_runs, total, self.model_cfg.width, dtype=torch.float32,
+                                 device=self.device) if layer_out else None)
+            # cut the step into passes of at most max_rows rows (an entry may span passes)
+            done = [0] * len(plan)
+            out_at = [0] * len(plan)
+            acc = 0
+            for i, (_, _, w) in enumerate(plan):
+                out_at[i] = acc
+                acc += len(w)
+        finally:   # (also of a step that is refused: the page tables of the entries before)
+            torch.cuda.current_stream(self.device).synchronize()   # the caller's work on its own stream, page tables
+        with torch.cuda.stream(self.stream):
+            self._run_passes(plan, done, out_at, logits, trace)
+        self.stream.synchronize()
+        for s, t, _ in plan:
+            s.n += len(t)
+            s.last = int(t[-1])
+        return (logits, trace) if layer_out else logits
+
+    def _plan(self, entries):
+        """(sequence, tokens, wanted indices) of every entry, with pages for its tokens, which the current stream still has to
+        write into the page tables."""
         plan = []
         seen = set()
         for rid, toks, want in entries:
@@ -126,35 +156,13 @@ class SeqEngine:
             s = self.seqs[rid]
             if s.n + len(toks) > self.max_seq_len:
                 raise OutOfPages(f"request {rid}: {s.n + len(toks)} tokens exceed max_seq_len {self.max_seq_len}")
-            self.cache.ensure_capacity(s.slot, s.n + len(toks))
+            self.cache.ensure_capacity(s.slot, s.n + len(toks), wait=False)
             if len(toks) == 1:
                 plan.append((s, list(toks), list(want)))
             else:
                 plan.append((s, _ints(toks), np.arange(want.start, want.stop, want.step, dtype=np.int32)
                              if isinstance(want, range) else _ints(want)))
-        n_want = sum(len(w) for _, _, w in plan)
-        V = self.model_cfg.vocab
-        logits = torch.empty(n_want, V, dtype=torch.float32, device=self.device)
-        total = sum(len(t) for _, t, _ in plan)
-        if layer_out and total > self.cfg.max_rows:
-            raise ValueError("layer_out needs a step of at most max_rows rows")
-        trace = (torch.empty(self.model_cfg.n_runs, total, self.model_cfg.width, dtype=torch.float32,
-                             device=self.device) if layer_out else None)
-        # cut the step into passes of at most max_rows rows (an entry may span passes)
-        done = [0] * len(plan)
-        out_at = [0] * len(plan)
-        acc = 0
-        for i, (_, _, w) in enumerate(plan):
-            out_at[i] = acc
-            acc += len(w)
-        torch.cuda.current_stream(self.device).synchronize()   # the caller's work on its own stream, page tables
-        with torch.cuda.stream(self.stream):
-            self._run_passes(plan, done, out_at, logits, trace)
-        self.stream.synchronize()
-        for s, t, _ in plan:
-            s.n += len(t)
-            s.last = int(t[-1])
-        return (logits, trace) if layer_out else logits
+        return plan
 
     def _run_passes(self, plan, done, out_at, logits, trace) -> None:
         while True:

@@ -56,13 +56,13 @@ __device__ __forceinline__ int tile_at(int t, int up_tiles) {
   return t / TN * (TN / 2) + (i < TN / 2 ? i : i - TN / 2 + up_tiles);
 }
 
-// Sixteen token rows (from m0) of a wave's TN tiles of values, from their image in LDS: four tokens of a channel a lane.  Tokens at
+// Sixteen token rows of a wave's TN tiles of values, from their image in LDS: four tokens of a channel a lane.  Tokens at
 // positions 4 p .. 4 p + 3 of a page are four neighbours of its channel's row; the four lanes of a channel's sixteen
 // tokens and the sixteen channels of a tile are next to each other.  Others (a prompt that starts at a row or a position that is
 // no multiple of four, the last rows) go one by one.
 template <int TN, int LD>
-__device__ __forceinline__ void emit_values(const WideEpiArgs& a, const float* img, const int* pos, int page_at, int m0, int tile0,
-                                            int n_tiles, int lane) {
+__device__ __forceinline__ void emit_values(const WideEpiArgs& a, const float* img, const int* pos, int page_at, int tile0, int n_tiles,
+                                            int lane) {
   const WideRope& rp = a.rope;
   const int D = rp.D, tiles_per_head = D / 16;
   const bool aligned = (reinterpret_cast<uintptr_t>(rp.vc) & 7) == 0;
@@ -77,8 +77,6 @@ __device__ __forceinline__ void emit_values(const WideEpiArgs& a, const float* i
     for (int k = 0; k < 4; ++k) {
       p[k] = pos[r + k];
       float y = img[(r + k) * LD + col];
-      if (p[k] >= 0 && a.x_scale) y *= a.x_scale[m0 + r + k];
-      if (a.w_scale) y *= a.w_scale[head * D + i];
       if (a.bias) y += (float)a.bias[head * D + i];
       v[k] = (bf16_t)y;
     }
@@ -367,7 +365,7 @@ __global__ __launch_bounds__(256, blocks_per_cu(TN, TM, STAGES, SPLIT)) void pro
     asm volatile("" ::: "memory");  // (other lanes read them: the stores of a lane without a unit stay here)
     if constexpr (QKV) {
       if (values) {
-        emit_values<TN, kLd>(a.epi, img, place + j * 16, TM * 16, row0 + (wm * TM + j) * 16, tile0 + wn * TN, a.n_tiles, lane);
+        emit_values<TN, kLd>(a.epi, img, place + j * 16, TM * 16, tile0 + wn * TN, a.n_tiles, lane);
         continue;
       }
     }
@@ -571,15 +569,17 @@ bool sd_rows_linear_fits_(int M, int n_tiles, int K, int64_t ldx, int S, int ks_
 
 int sd_rows_linear_(const void* W, const void* x, int64_t ldx, int M, int K, int n_tiles, int S, int ks_per_split, int epi,
                     const WideEpiArgs& epi_args, float* part, sd_stream_t stream) {
+  SD_REQUIRE(!epi_args.w_scale && !epi_args.x_scale, SD_ERR_UNSUPPORTED, "sd_rows_linear: fp8 weights or activations");
   PromptArgs a{(const bf16_t*)W, (const bf16_t*)x, ldx, M, K / 32, n_tiles, ks_per_split, 0, 0, part, 0, epi_args};
   hipStream_t st = (hipStream_t)stream;
   if (S > 1) return launch_few<4, EPI_PARTIAL>(a, S, st);
   return epi == SD_EPI_F32 ? few_shape<SD_EPI_F32>(a, st) : few_shape<SD_EPI_SILU_MUL>(a, st);
 }
 
-// epi: an SD_EPI_* number or EPI_QKV_ROPE, with what that epilogue reads in `e`.
+// epi: an SD_EPI_* number or EPI_QKV_ROPE, with what that epilogue reads in `e` (no fp8 scales: the epilogues of this file know none).
 int sd_prompt_linear_(const void* W, const void* x, int64_t ldx, int M, int K, int n_tiles, int epi,
                       const WideEpiArgs& epi_args, sd_stream_t stream) {
+  SD_REQUIRE(!epi_args.w_scale && !epi_args.x_scale, SD_ERR_UNSUPPORTED, "sd_prompt_linear: fp8 weights or activations");
   int S, ksp, g;
   WideEpiArgs e = epi_args;
   e.M = M;

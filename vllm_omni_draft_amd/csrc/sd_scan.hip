@@ -12,7 +12,10 @@
 //   - 64 workgroups of 8 heads of 128 x 128 instead of 32, a wave a SIMD.
 // us, before (256 threads of a strip a lane, 32 columns a workgroup) / now: 777 rows of 8 heads of 128 x 128, a decay per channel 404 / 92,
 // per head 284 / 80, per row 312 / 95; 400 rows of 32 heads of 128 x 64 per row 165 / 53; 64 portions of 60 rows of 16 heads per channel
-// 357 / 228, per head 286 / 199; one row of each of 4 requests, 32 heads of 128 x 64, 7.7 / 5.2.  The products alone are 31 us of the 92.
+// 357 / 228, per head 286 / 199; one row of each of 4 requests, 32 heads of 128 x 64, 7.7 / 5.2; 16 heads of 64 x 64 per row,
+// 16 portions of 24 rows 16.1 / 9.8, 300 rows 123 / 35; of 32 x 128 per channel 21.7 / 10.9, 166 / 39; of 16 x 16 per head 19.2 / 5.7, 182 / 29.  The products alone are 31 us of the 92.
+#include <type_traits>
+
 #include "sd_common.h"
 
 namespace {
@@ -65,19 +68,21 @@ __device__ __forceinline__ float behind(float x) {
 // the next one), while the one behind that is on its way, and add the strips' sums of the chunk before.  (Every wave doing
 // all of that: 158 us instead of 92, per channel as above.)  A group of 16 lanes has its own ring, so a token's place is an
 // immediate offset, and rings lie 16 (8) banks apart.
-template <int CH>
+template <int CH, int COLS>
 struct Lds {
   static constexpr int kq = (3 * CH + 1) * kStrip;   // floats of a group's ring: [token][8 of k, 8 of q]
   static constexpr int d = (3 * CH + 1) * kHalf;     // [token][8]
-  static constexpr int part = (2 * CH + 1) * kCols;  // a strip's sums: [token][16]
-  static constexpr int v = (3 * CH + 1) * kCols;     // [token][16]  (a token behind the ring's last one is read and not used)
+  static constexpr int part = (2 * CH + 1) * COLS;   // a strip's sums: [token][COLS]
+  static constexpr int v = (3 * CH + 1) * COLS;      // [token][COLS]  (a token behind the ring's last one is read and not used)
   static constexpr int row = (3 * CH + 1) * 2;       // per row: [token][decay, keys' scale]
 };
 
-template <int DECAY, int CH>
+// COLS: columns of a workgroup; 32: two groups of sixteen columns of the one strip that sixteen key channels or fewer are.
+template <int DECAY, int CH, int COLS>
 __global__ __launch_bounds__(1024) void decay_scan_kernel(ScanArgs a) {
-  using L = Lds<CH>;
-  const int nthr = blockDim.x / 2, strips = nthr / 32, lane = threadIdx.x & 63;   // (an even number of strips: a wave has two)
+  using L = Lds<CH, COLS>;
+  const int nthr = blockDim.x / 2, lane = threadIdx.x & 63;
+  const int strips = COLS > kCols ? 1 : nthr / 32;   // (else an even number of strips: a wave has two)
   const bool carries = (int)threadIdx.x >= nthr;
   const int tid = carries ? threadIdx.x - nthr : threadIdx.x, wave = tid >> 6;
   const int work = xcd_order(blockIdx.x, gridDim.x);
@@ -100,32 +105,33 @@ __global__ __launch_bounds__(1024) void decay_scan_kernel(ScanArgs a) {
     const float* d_src = a.decay + (DECAY == kPerChannel ? (size_t)row0 * a.H * dk + (size_t)h * dk + min(dr, dk - 1)
                                                          : (size_t)row0 * a.H + h);
     const int64_t d_step = DECAY == kPerChannel ? (int64_t)a.H * dk : a.H;
-    const float* v_src = a.v + (size_t)row0 * a.ldv + (size_t)h * dv + min(tile * kCols + tid % kCols, dv - 1);
+    const float* v_src = a.v + (size_t)row0 * a.ldv + (size_t)h * dv + min(tile * COLS + tid % COLS, dv - 1);
     float* kq_to = kq + (tid >> 4) * L::kq + (tid & 15);
     float* d_to = ds + (dr >> 3) * L::d + (dr & 7) + d_late * kHalf;
-    constexpr int kV = CH * kCols / 64;  // (of a wave alone)
-    const int v_loads = (CH * kCols + nthr - 1) / nthr;
+    constexpr int kV = CH * COLS / 64;  // (of a wave alone)
+    const int v_loads = (CH * COLS + nthr - 1) / nthr;
     float pkq[CH], pd[CH / 2], pv[kV], pa = 1.f;
     // (every load is issued, on an address clamped into the portion: a guarded load would become a branch whose join waits
     // for the loads in flight)
-    auto fetch = [&](int t0) __attribute__((always_inline)) {
-      const bool whole = t0 + CH <= len;
+    auto fetch = [&](int t0, auto tokens) __attribute__((always_inline)) {
+      constexpr int N = decltype(tokens)::value;
+      const bool whole = N == CH && t0 + N <= len;
       const float* p = kq_src + t0 * a.ldqk;
       if (whole) {
 #pragma unroll
-        for (int i = 0; i < CH; ++i, p += a.ldqk) pkq[i] = *p;
+        for (int i = 0; i < N; ++i, p += a.ldqk) pkq[i] = *p;
       } else {
 #pragma unroll
-        for (int i = 0; i < CH; ++i) pkq[i] = kq_src[min(t0 + i, len - 1) * a.ldqk];
+        for (int i = 0; i < N; ++i) pkq[i] = kq_src[min(t0 + i, len - 1) * a.ldqk];
       }
       if (DECAY == kPerChannel) {
         p = d_src + (t0 + d_late) * d_step;
         if (whole) {
 #pragma unroll
-          for (int i = 0; i < CH / 2; ++i, p += 2 * d_step) pd[i] = *p;
+          for (int i = 0; i < N / 2; ++i, p += 2 * d_step) pd[i] = *p;
         } else {
 #pragma unroll
-          for (int i = 0; i < CH / 2; ++i) pd[i] = d_src[min(t0 + 2 * i + d_late, len - 1) * d_step];
+          for (int i = 0; i < N / 2; ++i) pd[i] = d_src[min(t0 + 2 * i + d_late, len - 1) * d_step];
         }
       }
       if (DECAY == kPerRow) {
@@ -134,17 +140,19 @@ __global__ __launch_bounds__(1024) void decay_scan_kernel(ScanArgs a) {
         if (a.k_scale) pa = a.k_scale[(size_t)row0 * a.H + h + at];
       }
 #pragma unroll
-      for (int i = 0; i < kV; ++i) {
+      for (int i = 0; i < (kV * N + CH - 1) / CH; ++i) {
         if (i >= v_loads) break;
-        pv[i] = v_src[min(t0 + (tid + i * nthr) / kCols, len - 1) * a.ldv];
+        pv[i] = v_src[min(t0 + (tid + i * nthr) / COLS, len - 1) * a.ldv];
       }
     };
     auto put = [&](int at) __attribute__((always_inline)) {   // (in tokens)
 #pragma unroll
-      for (int i = 0; i < CH; ++i) kq_to[(at + i) * kStrip] = kr < dk ? pkq[i] : 0.f;
+      for (int i = 0; i < CH; ++i)
+        if (COLS == kCols || kr < kStrip) kq_to[(at + i) * kStrip] = kr < dk ? pkq[i] : 0.f;
       if (DECAY == kPerChannel) {
 #pragma unroll
-        for (int i = 0; i < CH / 2; ++i) d_to[(at + 2 * i) * kHalf] = dr < dk ? pd[i] : 0.f;
+        for (int i = 0; i < CH / 2; ++i)
+          if (COLS == kCols || dr < kStrip) d_to[(at + 2 * i) * kHalf] = dr < dk ? pd[i] : 0.f;
       }
       if (DECAY == kPerRow && tid < CH) {
         ds[(at + tid) * 2] = pd[0];
@@ -154,14 +162,14 @@ __global__ __launch_bounds__(1024) void decay_scan_kernel(ScanArgs a) {
       for (int i = 0; i < kV; ++i) {
         if (i >= v_loads) break;
         const int idx = tid + i * nthr;
-        if (idx < CH * kCols) vs[at * kCols + idx] = tile * kCols + idx % kCols < dv ? pv[i] : 0.f;
+        if (idx < CH * COLS) vs[at * COLS + idx] = tile * COLS + idx % COLS < dv ? pv[i] : 0.f;
       }
     };
     // The strips' sums of tokens lo .. hi - 1
     auto emit = [&](int lo, int hi) __attribute__((always_inline)) {
-      for (int idx = tid; idx < (hi - lo) * kCols; idx += nthr) {
-        const int t = lo + idx / kCols, cc = idx % kCols;
-        const float* p = part + (t & (2 * CH - 1)) * kCols + cc;
+      for (int idx = tid; idx < (hi - lo) * COLS; idx += nthr) {
+        const int t = lo + idx / COLS, cc = idx % COLS;
+        const float* p = part + (t & (2 * CH - 1)) * COLS + cc;
         float o = p[0];
         for (int i = 1; i < a.strips; i += 7) {
           float x[7];
@@ -170,17 +178,22 @@ __global__ __launch_bounds__(1024) void decay_scan_kernel(ScanArgs a) {
 #pragma unroll
           for (int j = 0; j < 7; ++j) o = i + j < a.strips ? o + x[j] : o;
         }
-        if (tile * kCols + cc < dv) a.out[(size_t)(row0 + t) * ((size_t)a.H * dv) + (size_t)h * dv + tile * kCols + cc] = o;
+        if (tile * COLS + cc < dv) a.out[(size_t)(row0 + t) * ((size_t)a.H * dv) + (size_t)h * dv + tile * COLS + cc] = o;
       }
     };
-    fetch(0);
+    // (nobody uses a token behind the last one: a portion of half a chunk asks for no more where a token has three values of a channel, and
+    // a portion of one chunk does not ask for a second one.  16 heads of 128 x 256 per channel, 256 portions of one row 440 / 338, 300 of three 552 /
+    // 429; per head 351 / 270 and 458 / 343.  The half for all decays, or the tokens one by one: up to 20 % slower.)
+    using Chunk = std::integral_constant<int, CH>;
+    if (DECAY == kPerChannel && CH == 8 && len <= CH / 2) fetch(0, std::integral_constant<int, CH / 2>());
+    else fetch(0, Chunk());
     put(0);
-    fetch(CH);
+    if (len > CH) fetch(CH, Chunk());
     for (int ch = 0; ch < n_chunks; ++ch) {
       __syncthreads();
       ring = ring == 2 * CH ? 0 : ring + CH;
       if (ch + 1 < n_chunks) put(ring);
-      if (ch + 2 < n_chunks) fetch((ch + 2) * CH);
+      if (ch + 2 < n_chunks) fetch((ch + 2) * CH, Chunk());
       if (ch > 0) emit(max((ch - 1) * CH - 1, 0), ch * CH - 1);
     }
     __syncthreads();
@@ -188,8 +201,8 @@ __global__ __launch_bounds__(1024) void decay_scan_kernel(ScanArgs a) {
     return;
   }
 
-  const int upper = lane >> 5, s = wave * 2 + ((lane >> 4) & 1), c = lane & 15;
-  const int col = tile * kCols + c, r0 = s * kStrip + upper * kHalf;
+  const int upper = lane >> 5, s = COLS > kCols ? 0 : wave * 2 + ((lane >> 4) & 1), c = lane % COLS;   // (an upper lane: that of lane - 32)
+  const int col = tile * COLS + c, r0 = s * kStrip + upper * kHalf;
   float* st = a.state + ((size_t)slot * a.H + h) * dk * dv;
   float S[kHalf];
 #pragma unroll
@@ -197,7 +210,7 @@ __global__ __launch_bounds__(1024) void decay_scan_kernel(ScanArgs a) {
   const float dh = DECAY == kPerHead ? a.decay[h] : 0.f;
   const float skip_h = DECAY == kPerRow && a.skip
                            ? a.w_f32 ? ((const float*)a.skip)[h] : (float)((const bf16_t*)a.skip)[h] : 0.f;
-  const float* kq_mine = kq + (s * 2 + upper) * L::kq + c;
+  const float* kq_mine = kq + (s * 2 + upper) * L::kq + (lane & 15);
   const float* d_mine = DECAY == kPerChannel ? ds + (s * 2 + upper) * L::d + (c & 7) : ds;
   const float* v_mine = vs + c;
   struct Token {
@@ -208,7 +221,7 @@ __global__ __launch_bounds__(1024) void decay_scan_kernel(ScanArgs a) {
     x.kq = kq_mine[at * kStrip + i * kStrip];
     x.d = DECAY == kPerChannel ? d_mine[at * kHalf + i * kHalf] : DECAY == kPerRow ? d_mine[at * 2 + i * 2] : dh;
     x.a = DECAY == kPerRow ? d_mine[at * 2 + i * 2 + 1] : 1.f;
-    x.v = v_mine[at * kCols + i * kCols];
+    x.v = v_mine[at * COLS + i * COLS];
     return x;
   };
   float sum = 0.f;                       // of the token this lane has just seen
@@ -224,8 +237,8 @@ __global__ __launch_bounds__(1024) void decay_scan_kernel(ScanArgs a) {
     __syncthreads();
     const int t0 = ch * CH, at = ring + 1 - upper;   // of the step behind t0
     Token x = read(upper ? (ring == 0 ? 3 * CH : ring) - 1 : ring, 0);
-    float* kept = part_mine + (ch & 1) * CH * kCols - kCols;   // places of tokens t0 - 1 and t0
-    float* before = ch & 1 ? kept : part_mine + (2 * CH - 1) * kCols;
+    float* kept = part_mine + (ch & 1) * CH * COLS - COLS;   // places of tokens t0 - 1 and t0
+    float* before = ch & 1 ? kept : part_mine + (2 * CH - 1) * COLS;
     if (ch > 0 && t0 + CH <= len) {
 #pragma unroll
       for (int i = 0; i < CH; ++i) {
@@ -233,7 +246,7 @@ __global__ __launch_bounds__(1024) void decay_scan_kernel(ScanArgs a) {
         __builtin_amdgcn_sched_barrier(0);               // (a token ahead of its use: left to itself the compiler reads it right there)
         sum = behind(sum);
         products(x);
-        keep(i == 0 ? before : kept + i * kCols, x);
+        keep(i == 0 ? before : kept + i * COLS, x);
         x = y;
       }
     } else {
@@ -242,7 +255,7 @@ __global__ __launch_bounds__(1024) void decay_scan_kernel(ScanArgs a) {
         sum = behind(sum);
         // the first token's step is the lower lanes' alone, the one behind the last token's the upper lanes'
         if (t0 + i == 0 ? !upper : t0 + i < len || upper) products(x);
-        if (t0 + i > 0) keep(i == 0 ? before : kept + i * kCols, x);
+        if (t0 + i > 0) keep(i == 0 ? before : kept + i * COLS, x);
         x = y;
       }
     }
@@ -256,26 +269,36 @@ __global__ __launch_bounds__(1024) void decay_scan_kernel(ScanArgs a) {
   }
 }
 
-template <int DECAY, int CH>
+template <int DECAY, int CH, int COLS>
 void launch_scan(const ScanArgs& a, int grid, int nthr, hipStream_t st) {
-  using L = Lds<CH>;
-  const int strips = nthr / 32, d = DECAY == kPerChannel ? 2 * strips * L::d : DECAY == kPerRow ? L::row : 0;
+  using L = Lds<CH, COLS>;
+  const int strips = COLS > kCols ? 1 : nthr / 32, d = DECAY == kPerChannel ? 2 * strips * L::d : DECAY == kPerRow ? L::row : 0;
   // (64 floats and a ring's length behind the last strip's sums: the lower lanes' places)
   const size_t lds = sizeof(float) * (2 * strips * L::kq + d + L::v + (strips + 1) * L::part + 64);
-  decay_scan_kernel<DECAY, CH><<<grid, 2 * nthr, lds, st>>>(a);
+  decay_scan_kernel<DECAY, CH, COLS><<<grid, 2 * nthr, lds, st>>>(a);
 }
 
+// Workgroups of 16 columns from which keys of one strip take 32: a wave's second strip would be nothing but padding, and the chip has more to do than
+// it holds at once.  16 heads of 16 x 128 in workgroups of 64 columns and no carrying waves / of 16 / of 32: 256 portions of one row per channel 27.6 / 46 /
+// 25.5, per row 28.8 / 36 / 20.5, per head 26.0 / 36 / 21.7; 64 of 24 tokens per channel 25.5 / 30.1 / 20.1; below it 16 / 32: one of 300 tokens per channel 34 /
+// 42, 16 of 60 of 16 x 64 11.6 / 12.3.
+constexpr int kManyGroups = 4096;
 template <int DECAY>
 int scan(ScanArgs a, int n_entries, const char* name, hipStream_t st) {
   SD_REQUIRE(a.dk >= 1 && a.dk <= 256, SD_ERR_UNSUPPORTED, "%s: key size %d outside 1..256", name, a.dk);
-  a.tiles = (a.dv + kCols - 1) / kCols;
   a.strips = (a.dk + kStrip - 1) / kStrip;
+  const int nthr = (a.strips + 1) / 2 * 64;
+  const bool wide = a.strips == 1 && (int64_t)((a.dv + kCols - 1) / kCols) * a.H * n_entries >= kManyGroups;
+  const int cols = wide ? 2 * kCols : kCols;
+  a.tiles = (a.dv + cols - 1) / cols;
   const int64_t grid = (int64_t)a.tiles * a.H * n_entries;
   SD_REQUIRE(grid < INT_MAX, SD_ERR_UNSUPPORTED, "%s: more than 2^31 workgroups", name);
-  const int nthr = (a.strips + 1) / 2 * 64;
-  // (chunks of four tokens beyond 128 channels: at most 52 KB of LDS either way, three workgroups a CU)
-  if (nthr <= 256) launch_scan<DECAY, 8>(a, (int)grid, nthr, st);
-  else launch_scan<DECAY, 4>(a, (int)grid, nthr, st);
+  // Chunks of eight tokens are at most 52 KB of LDS up to 128 channels, chunks of four beyond; three workgroups a CU up to 160 channels, two of
+  // twelve waves or more from there on.  us in chunks of four / eight, 16 heads of 128 x 128 per channel: 300 tokens 47.9 / 34.4, 8 portions of 100 41.2 / 36.8, 32 of one
+  // row 19.1 / 23.9; of 256 x 128: 73.8 / 50.5, 76.1 / 76.8, 36.5 / 59.4.
+  if (wide) launch_scan<DECAY, 8, 2 * kCols>(a, (int)grid, nthr, st);
+  else if (nthr <= 256) launch_scan<DECAY, 8, kCols>(a, (int)grid, nthr, st);
+  else launch_scan<DECAY, 4, kCols>(a, (int)grid, nthr, st);
   SD_CHECK_LAUNCH(name);
   return SD_OK;
 }

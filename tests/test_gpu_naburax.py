@@ -512,6 +512,40 @@ def test_postnorm_residual():
     assert rel(xd, x.double() + N.rms_norm(y, w.double(), 1e-5)) < 1e-6
 
 
+@pytest.mark.parametrize("W", [255, 257, 512, 513, 1024, 1025, 2047, 2048, 2049, 4100])
+@pytest.mark.parametrize("wdt", [torch.float32, torch.bfloat16])
+def test_rows_of_more_columns_than_a_thread_holds(W, wdt):
+    """Residual update, embedding and the norms of both preparations at the edges of one, two, four and eight columns a thread (256 a
+    workgroup), and beyond, where a second batch of columns is read and the norms read them twice; a float32 sum of 4100 products in strands
+    of 17 is within 1e-6 of a float64 one."""
+    from vllm_omni_draft_amd import ops
+    g = torch.Generator().manual_seed(W)
+    rn = lambda *shape: torch.randn(*shape, generator=g)
+    n, rnd = 3, wdt == torch.bfloat16
+    x, a, b, w = rn(n, W), rn(2 * n, W), rn(n, W), rn(W).to(wdt)
+    xd = dev(x)
+    ops.postnorm_residual(xd, dev(a), dev(w), 1e-5, n_a=2, sa=0.6, b=dev(b), sb=0.5)
+    y = 0.6 * a.double().view(n, 2, W).sum(1) + 0.5 * b.double()
+    assert rel(xd, x.double() + N.rms_norm(y, w.double(), 1e-5)) < 1e-6
+    table, bg, toks = rn(20, W).to(wdt), rn(8, W).to(wdt), [3, 19, 0]
+    e, e_b = ops.embed_hashed(i32(toks), dev(table), 2.5, i32([-1] + toks[:-1]), dev(bg), 31, 7, bf16_copy=True)
+    rows = [7] + [(p * 31 + t * 7) % 7 for p, t in zip(toks, toks[1:])]
+    assert rel(e, table.double()[toks] * 2.5 + bg.double()[rows]) < 1e-6 and torch.equal(e_b, e.to(torch.bfloat16))
+    pos, slot, bt = i32([14, 15, 16]), i32([0] * n), i32([[1, 0]])
+    kv, dr = rn(n, W + 8), 8
+    f = torch.zeros(dr // 2, dtype=torch.float64)       # (no rotation)
+    kvd, xq, cache = dev(kv), dev(x), torch.zeros(2, 1, PAGE, W + dr, dtype=wdt, device=DEV)
+    ops.latent_prep(xq, dev(w), kvd, dev(w), W, dr, 1e-5, dr, dev(f), 1.0, cache, pos, slot, bt)
+    assert torch.equal(xq, ops.rmsnorm_parts(dev(x), dev(w), 1e-5, round_bf16=rnd))
+    assert torch.equal(kvd[:, :W], ops.rmsnorm_parts(dev(kv[:, :W]), dev(w), 1e-5, round_bf16=rnd))
+    assert torch.equal(kvd[:, W:].cpu(), kv[:, W:]) and torch.equal(cache[[1, 1, 0], 0, [14, 15, 0]], kvd.to(wdt))
+    q, k, v = dev(x), dev(b), dev(a[:n])
+    kc, vc = (torch.zeros(2, 1, PAGE, W, dtype=wdt, device=DEV) for _ in range(2))
+    ops.qk_norm_append(q, dev(w), k, dev(w), v, 1, W, W, 1e-5, kc, vc, pos, slot, bt)
+    assert rel(q, N.rms_norm(x.double(), w.double(), 1e-5)) < 1e-6 and rel(k, N.rms_norm(b.double(), w.double(), 1e-5)) < 1e-6
+    assert torch.equal(kc[[1, 1, 0], 0, [14, 15, 0]], k.to(wdt)) and torch.equal(vc[[1, 1, 0], 0, [14, 15, 0]], v.to(wdt))
+
+
 # ------------------------------------------------------------------ whole models
 @pytest.mark.parametrize("shape", list(SHAPES))
 def test_prompt_logits_match_the_plain_model(shape):

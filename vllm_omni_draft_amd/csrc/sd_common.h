@@ -4,6 +4,9 @@
 #include <limits.h>
 #include <stdint.h>
 #include <stdio.h>
+
+#include <type_traits>
+
 #include "../../include/sd_amd.h"
 
 typedef __bf16 bf16_t;
@@ -61,6 +64,19 @@ constexpr int kRowGroup = 8;
 __device__ __forceinline__ int xcd_order(int id, int n) {
   const int q = n >> 3, r = n & 7, x = id & 7, i = id >> 3;
   return x * q + min(x, r) + i;
+}
+
+// Columns of a row that each of 256 threads asks for before it uses one (256 apart; the last one again for those past the row): body(U).
+// A few rows are a chain of reads, each a round trip, so as many as eight; but no more than a narrow row has: of many rows each read counts, and
+// those past the end cost as much as others.  us a column at a time / always eight / now: row norm of 4 rows of 2048 columns 4.5 / 3.3 / 3.4, 4096 of
+// 256 5.9 / 7.5 / 5.2, 4096 of 2048 19.0 / 16.1 / 15.1; queries and keys normed and appended, 4096 of 256 9.4 / 11.6 / 8.6, 1024 of 1024 5.5 / 6.3 / 5.1, of
+// 2560 (two batches, the second mostly past the end) 7.9 / 9.3 / 8.7; embedding 4096 of 256 5.0 / 5.7 / 5.0.
+template <class F>
+__device__ __forceinline__ void by_columns(int n, F body) {
+  if (n <= 256) body(std::integral_constant<int, 1>());
+  else if (n <= 512) body(std::integral_constant<int, 2>());
+  else if (n <= 1024) body(std::integral_constant<int, 4>());
+  else body(std::integral_constant<int, 8>());
 }
 
 // Layer-list models whose matrices are tiled: a portion of a pass with more rows than this runs on kernels for many

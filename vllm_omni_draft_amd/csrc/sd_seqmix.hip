@@ -59,9 +59,6 @@ __global__ void embed_rows_kernel(const int32_t* __restrict__ tokens, const T* _
 }
 
 // out[i] = x[rows ? rows[i] : i] / sqrt(mean(x^2) + eps) * (offset + w); out_b: the same as bf16
-// A thread asks for eight columns of every operand before it uses one and keeps them for the second pass (4 rows of 2048 columns a
-// column at a time 7.9 us, now 4.8).
-constexpr int kRowBatch = 8;
 template <typename T>
 __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const float* __restrict__ x, const int32_t* __restrict__ rows,
                                     const T* __restrict__ w, float offset, float eps,
@@ -69,33 +66,36 @@ __global__ __launch_bounds__(256) void rmsnorm_rows_kernel(const float* __restri
   __shared__ float red[4];
   const int i = blockIdx.x;
   const float* xr = x + (size_t)(rows ? rows[i] : i) * W;
-  float xv[kRowBatch], wv[kRowBatch];
-  auto load = [&](int c) __attribute__((always_inline)) {   // (the last column again for those past the row)
+  by_columns(W, [&](auto batch) __attribute__((always_inline)) {
+    constexpr int U = decltype(batch)::value;
+    float xv[U], wv[U];
+    auto load = [&](int c) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < kRowBatch; ++u) {
-      xv[u] = xr[min(c + 256 * u, W - 1)];
-      wv[u] = ld_f(w + min(c + 256 * u, W - 1));
-    }
-  };
-  float ss = 0.f;
-  for (int c = threadIdx.x; c < W; c += 256 * kRowBatch) {
-    load(c);
-#pragma unroll
-    for (int u = 0; u < kRowBatch; ++u)
-      if (c + 256 * u < W) ss = fmaf(xv[u], xv[u], ss);
-  }
-  ss = block_sum(ss, red);
-  const float rstd = 1.f / sqrtf(ss / (float)W + eps);
-  for (int c = threadIdx.x; c < W; c += 256 * kRowBatch) {
-    if (W > 256 * kRowBatch) load(c);   // (a narrower row is still here)
-#pragma unroll
-    for (int u = 0; u < kRowBatch; ++u)
-      if (c + 256 * u < W) {
-        const float v = maybe_round(xv[u] * rstd * (offset + wv[u]), round);
-        out[(size_t)i * W + c + 256 * u] = v;
-        if (out_b) out_b[(size_t)i * W + c + 256 * u] = (bf16_t)v;
+      for (int u = 0; u < U; ++u) {
+        xv[u] = xr[min(c + 256 * u, W - 1)];
+        wv[u] = ld_f(w + min(c + 256 * u, W - 1));
       }
-  }
+    };
+    float ss = 0.f;
+    for (int c = threadIdx.x; c < W; c += 256 * U) {
+      load(c);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (c + 256 * u < W) ss = fmaf(xv[u], xv[u], ss);
+    }
+    ss = block_sum(ss, red);
+    const float rstd = 1.f / sqrtf(ss / (float)W + eps);
+    for (int c = threadIdx.x; c < W; c += 256 * U) {
+      if (W > 256 * U) load(c);   // (a narrower row is still here)
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (c + 256 * u < W) {
+          const float v = maybe_round(xv[u] * rstd * (offset + wv[u]), round);
+          out[(size_t)i * W + c + 256 * u] = v;
+          if (out_b) out_b[(size_t)i * W + c + 256 * u] = (bf16_t)v;
+        }
+    }
+  });
 }
 
 // Y[M, N] = X[M, K] W[N, K]^T + bias.  X is f32 (rounded to bf16 values on load when `round`;

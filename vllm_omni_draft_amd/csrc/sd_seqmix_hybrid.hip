@@ -39,12 +39,10 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
   return s;
 }
 
-// A few rows are a chain of reads, each a round trip, so a thread asks for kRowBatch columns of every operand (256 apart, the last
-// one again for those past the row) before it uses one.
+// Columns of a norm over parts or a residual update that a thread asks for before it uses one (as by_columns for wide rows).
 constexpr int kRowBatch = 8;
 
 // ------------------------------------------------------------------ embedding
-// (4 rows of 2048 columns a column at a time 10.4 us, now 4.0)
 template <typename T>
 __global__ __launch_bounds__(256) void embed_hashed_kernel(const int32_t* __restrict__ tokens, const int32_t* __restrict__ prev,
                                     const T* __restrict__ table, const T* __restrict__ bigram, float scale,
@@ -62,23 +60,26 @@ __global__ __launch_bounds__(256) void embed_hashed_kernel(const int32_t* __rest
   }
   const T* tr = table + (size_t)tok * W;
   const T* br = brow >= 0 ? bigram + (size_t)brow * W : tr;
-  for (int c = threadIdx.x; c < W; c += 256 * kRowBatch) {
-    T t[kRowBatch], b[kRowBatch];
+  by_columns(W, [&](auto batch) __attribute__((always_inline)) {
+    constexpr int U = decltype(batch)::value;
+    for (int c = threadIdx.x; c < W; c += 256 * U) {
+      T t[U], b[U];
 #pragma unroll
-    for (int u = 0; u < kRowBatch; ++u) {
-      t[u] = tr[min(c + 256 * u, W - 1)];
-      b[u] = br[min(c + 256 * u, W - 1)];
-    }
+      for (int u = 0; u < U; ++u) {
+        t[u] = tr[min(c + 256 * u, W - 1)];
+        b[u] = br[min(c + 256 * u, W - 1)];
+      }
 #pragma unroll
-    for (int u = 0; u < kRowBatch; ++u) {
-      float v = ld_f(&t[u]) * scale;
-      if (brow >= 0) v += ld_f(&b[u]);
-      if (c + 256 * u < W) {
-        x[(size_t)r * W + c + 256 * u] = v;
-        if (x_b) x_b[(size_t)r * W + c + 256 * u] = (bf16_t)v;
+      for (int u = 0; u < U; ++u) {
+        float v = ld_f(&t[u]) * scale;
+        if (brow >= 0) v += ld_f(&b[u]);
+        if (c + 256 * u < W) {
+          x[(size_t)r * W + c + 256 * u] = v;
+          if (x_b) x_b[(size_t)r * W + c + 256 * u] = (bf16_t)v;
+        }
       }
     }
-  }
+  });
 }
 
 // ------------------------------------------------------------------ norm over parts of a row
@@ -672,38 +673,40 @@ void launch_softmax_nc(dim3 grid, int kt, size_t lds, hipStream_t st, int nc, co
 
 // ------------------------------------------------------------------ fused preparation of attention inputs
 // Row norm over n columns in place (times w, rounded to bf16 values when round), by a whole
-// workgroup of 256 threads: the sums of rmsnorm_parts_kernel with one part, the same bits.  (4 rows of 2048 queries and keys appended: a column
-// at a time 7.6 us, kRowBatch at a time 5.5.)
+// workgroup of 256 threads: the sums of rmsnorm_parts_kernel with one part, the same bits.
 template <typename T>
 __device__ __forceinline__ void norm_in_place(float* __restrict__ v, const T* __restrict__ w, int n, float eps,
                                               int round, bf16_t* __restrict__ copy, float* red) {
-  float x[kRowBatch], wv[kRowBatch];
-  auto load = [&](int c) __attribute__((always_inline)) {
+  by_columns(n, [&](auto batch) __attribute__((always_inline)) {
+    constexpr int U = decltype(batch)::value;
+    float x[U], wv[U];
+    auto load = [&](int c) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < kRowBatch; ++u) {
-      x[u] = v[min(c + 256 * u, n - 1)];
-      wv[u] = ld_f(w + min(c + 256 * u, n - 1));
-    }
-  };
-  float ss = 0.f;
-  for (int c = threadIdx.x; c < n; c += 256 * kRowBatch) {
-    load(c);
-#pragma unroll
-    for (int u = 0; u < kRowBatch; ++u)
-      if (c + 256 * u < n) ss = fmaf(x[u], x[u], ss);
-  }
-  ss = block_sum(ss, red);
-  const float rstd = 1.f / sqrtf(ss / (float)n + eps);
-  for (int c = threadIdx.x; c < n; c += 256 * kRowBatch) {
-    if (n > 256 * kRowBatch) load(c);   // (a narrower row is still here)
-#pragma unroll
-    for (int u = 0; u < kRowBatch; ++u)
-      if (c + 256 * u < n) {
-        const float o = maybe_round(x[u] * rstd * wv[u], round);
-        v[c + 256 * u] = o;
-        if (copy) copy[c + 256 * u] = (bf16_t)o;
+      for (int u = 0; u < U; ++u) {
+        x[u] = v[min(c + 256 * u, n - 1)];
+        wv[u] = ld_f(w + min(c + 256 * u, n - 1));
       }
-  }
+    };
+    float ss = 0.f;
+    for (int c = threadIdx.x; c < n; c += 256 * U) {
+      load(c);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (c + 256 * u < n) ss = fmaf(x[u], x[u], ss);
+    }
+    ss = block_sum(ss, red);
+    const float rstd = 1.f / sqrtf(ss / (float)n + eps);
+    for (int c = threadIdx.x; c < n; c += 256 * U) {
+      if (n > 256 * U) load(c);   // (a narrower row is still here)
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (c + 256 * u < n) {
+          const float o = maybe_round(x[u] * rstd * wv[u], round);
+          v[c + 256 * u] = o;
+          if (copy) copy[c + 256 * u] = (bf16_t)o;
+        }
+    }
+  });
 }
 
 // Latent attention, per row.  Workgroup (r, 0): the query latent normed in place (+ bf16 copy).

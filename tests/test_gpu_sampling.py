@@ -28,6 +28,18 @@ def test_library_loads_on_gpu():
     assert cus > 0 and "gfx" in name
 
 
+@pytest.mark.parametrize("raw", [True, False])
+def test_launches_go_to_the_current_stream(raw, monkeypatch):
+    """With and without torch's way to a stream's handle that is not public."""
+    ops = _ops()
+    if not raw:
+        monkeypatch.setattr(ops, "_raw_stream", None)
+    assert ops._stream() == torch.cuda.current_stream().cuda_stream
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        assert ops._stream() == side.cuda_stream
+
+
 def _scratch(ops, split, rows):
     """None (one workgroup per row) or scratch for the split forms."""
     return ops.sampling_scratch(rows) if split else None

@@ -19,8 +19,16 @@ def on_gpu() -> bool:
     return _lib.backend() == "gpu"
 
 
+# The current stream's handle without an object around it, where this torch has that (0.35 us a call; the public way 2.8)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream():
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()) if on_gpu() else None
+    if not on_gpu():
+        return None
+    if _raw_stream is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(torch.cuda.current_device())
 
 
 def _p(t: Optional[torch.Tensor]) -> Optional[int]:

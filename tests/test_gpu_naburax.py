@@ -709,6 +709,20 @@ def test_norm_and_router_in_one_launch_have_the_bits_of_two(shape):
     assert at == 577 and torch.equal(torch.cat(got), want)
 
 
+@pytest.mark.parametrize("width,n", [(2047, 17), (2048, 16), (2049, 33), (2112, 5), (4100, 17)])
+@pytest.mark.parametrize("wdt", [torch.float32, torch.bfloat16])
+def test_norm_and_router_of_wide_rows_in_one_launch_have_the_bits_of_two(width, n, wdt):
+    """Rows of one load ahead and of more (2048 columns), a wave's second and third expert, weights of both types: twelve prompts of 24
+    tokens in one pass (288 rows: two launches) against six at a time (144 rows: one)."""
+    cfg = model_cfg([latent(mlp=experts(n, 3, 8)), parallel(mlp=experts(n, 2, 8))], width=width)
+    _, eng = build(cfg, wdt, max_seqs=12)
+    step = lambda ids: eng.step([(f"r{i}", prompt(cfg, 24, i), range(24)) for i in ids])
+    want = step(range(12))
+    for i in range(12):
+        eng.finish(f"r{i}")
+    assert torch.equal(torch.cat([step(range(6)), step(range(6, 12))]), want)
+
+
 def test_a_far_token_through_the_recurrence_and_a_kept_first_token():
     """The recurrence's decay made (almost) one, so that a token 150 positions back still carries
     weight; and a kept first token whose key every later query finds."""

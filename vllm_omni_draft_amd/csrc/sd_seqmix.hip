@@ -537,8 +537,9 @@ __device__ __forceinline__ void score_key(const KT* __restrict__ kr, const float
 // STAGED (f32 rows of 16, 32, 64 or 128 channels, passes of many rows): 64 keys at a time come through LDS, whole rows a load, and a
 // lane takes a key's product with one head, whose query it reads by scalar loads: the same sums.  (A thread a key reads its row 16 bytes
 // at a time, 64 rows apart in a wave; with all rows' workgroups on a CU the first-level cache holds none of their lines until the
-// next piece, and L2 is read eight times over: 777 rows of 8 heads over 2 of 128 channels 131 us, 107
-// staged; 300 rows 43 / 31, 777 of 64 channels and a window of 256 60 / 40; before, the values' addresses in vector registers too, 151, 49 and 69.)
+// next piece, and L2 is read eight times over: 777 rows of 8 heads over 2 of 128 channels 131 us, 107 staged; 300 rows 43 / 31, 777 of
+// 64 channels and a window of 256 60 / 40; before, the values' addresses in vector registers too, 151, 49 and 69.  65 rows before / now: 128
+// channels, window 4 and blocks of 2 28.7 / 12.8, window 1024 22.0 / 15.0; 16 channels 13.7 / 10.8 and 13.6 / 11.7.)
 // NH: query heads per workgroup (of one kv head), NC: value columns per lane (vdim <= 64 * NC).
 // n_splits > 1: workgroup (.., .., z) takes the keys of tile z / n_hgroups only and writes its sum
 // to out + split * split_stride (sum_splits_kernel adds the splits in order).

@@ -768,6 +768,32 @@ def test_every_block_shape_has_the_bits_of_few_rows(M, N, K, shape):
         assert torch.equal(ops.linear_prompt(W, x, None, r, epi), few), epi
 
 
+@pytest.mark.parametrize("M,N,K", [(273, 128, 192), (273, 132, 192), (130, 16400, 1024), (275, 30016, 704), (257, 16416, 1024)])
+def test_outputs_stored_from_registers_have_the_bits_of_few_rows(M, N, K):
+    """Blocks of tiles that are all there store from registers, others (the last tiles of a matrix that is no multiple of a block
+    or of 16) through LDS: every epilogue, with and without a bias, last rows that fill no tile, and f32 and bf16 outputs in
+    rows that are longer than the outputs."""
+    ops = _ops()
+    from vllm_omni_draft_amd import _lib
+    gen = torch.Generator(device="cuda").manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=gen, device="cuda").to(torch.bfloat16)
+    W = (torch.randn(2 * N, K, generator=gen, device="cuda") * K ** -0.5).to(torch.bfloat16)
+    bias = torch.randn(2 * N, generator=gen, device="cuda").to(torch.bfloat16)
+    p = lambda t: None if t is None else t.data_ptr()
+    for epi in range(6):
+        gated = epi == ops.EPI_SILU_MUL
+        Wt = ops._tiled(W if gated else W[:N].contiguous(), epi)
+        dtype = torch.float32 if epi == ops.EPI_F32 else torch.bfloat16
+        for b, ld in ((None, N), (bias if gated else bias[:N].contiguous(), N + 12), (None, N + 2)):
+            res = torch.randn(M, ld, generator=gen, device="cuda").to(torch.bfloat16) if epi == ops.EPI_RESIDUAL else None
+            out = torch.full((M, ld), 7.0, dtype=dtype, device="cuda")
+            _lib.check(_lib.load().sd_linear_prompt(p(Wt.data), p(x), K, p(b), p(res), p(out), ld, M, N, K, epi, ops._stream()), "prompt")
+            few = torch.cat([ops.linear_wide(Wt, x[i:i + 48], b, None if res is None else res[i:i + 48, :N].contiguous(), epi)
+                             for i in range(0, M, 48)])
+            assert torch.equal(out[:, :N], few), (epi, b is not None, ld)
+            assert (out[:, N:] == 7.0).all()
+
+
 @pytest.mark.parametrize("M", [17, 64, 192, 256])
 @pytest.mark.parametrize("N,K,splits", [(3584, 18944, 9), (4112, 6400, 7), (8192, 4096, 4), (960, 4352, 17), (16, 2176, 17)])
 @pytest.mark.parametrize("fp8,bias", [(False, False), (False, True), (True, True)])

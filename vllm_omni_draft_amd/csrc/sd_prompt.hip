@@ -56,39 +56,279 @@ __device__ __forceinline__ int tile_at(int t, int up_tiles) {
   return t / TN * (TN / 2) + (i < TN / 2 ? i : i - TN / 2 + up_tiles);
 }
 
-// Sixteen token rows of a wave's TN tiles of values, from their image in LDS: four tokens of a channel a lane.  Tokens at
-// positions 4 p .. 4 p + 3 of a page are four neighbours of its channel's row; the four lanes of a channel's sixteen
-// tokens and the sixteen channels of a tile are next to each other.  Others (a prompt that starts at a row or a position that is
-// no multiple of four, the last rows) go one by one.
-template <int TN, int LD>
-__device__ __forceinline__ void emit_values(const WideEpiArgs& a, const float* img, const int* pos, int page_at, int tile0, int n_tiles,
-                                            int lane) {
-  const WideRope& rp = a.rope;
-  const int D = rp.D, tiles_per_head = D / 16;
-  const bool aligned = (reinterpret_cast<uintptr_t>(rp.vc) & 7) == 0;
-#pragma unroll 1
-  for (int n = lane; n < 4 * 16 * TN; n += 64) {
-    const int r = (n & 3) * 4, col = n >> 2, tile = tile0 + (col >> 4), row = col & 15;
-    if (tile >= n_tiles) break;
-    const int head = tile / tiles_per_head, i = (tile - head * tiles_per_head) * 8 + (row & 7) + (row & 8 ? D / 2 : 0);
-    int p[4];
-    bf16x4 v;
+// acc[i][j][reg] = (tile row 4 * xq + reg of tile i, token 16 j + xc), lane = 16 xq + xc: a lane holds four neighbouring outputs of a
+// token.  Gated and rotary tiles hold the partners of rows 0..7 in rows 8..15, half a wave on: of two tiles the wave's halves
+// change places, and each lane has both sums of four outputs of one of the two.
+// A wave is alone on its SIMD here, and nothing hides what its epilogue waits for: through LDS, four tokens at a time, each trip a
+// read, a residual's read, a chain of arithmetic and a store, 4096 x 4096 outputs of 4096 columns took 144 us, now 131 (with the residuals of
+// sixteen tokens at a time 145: all of a wave's are asked for at once); 2946 x 3584 of 18944 363, now 348; 14336 gated outputs of 4096 columns,
+// 1024 rows 194.5, now 191; 6144 x 4096 with rotation and pages, 1024 rows 74.0, now 66.
+// The four lanes of a token and tile store 32 bytes (bf16), sixteen tokens at once; the L2 joins them.  f32 outputs, 64 bytes, go out as
+// whole lines instead, eight tokens of two tiles at once (half lines: 2.5 % of a layer-list model's pass slower).
+struct TileSums {
+  f32x4 lo, hi;
+};
+__device__ __forceinline__ TileSums split_halves(const f32x4& even, const f32x4& odd) {
+  TileSums s;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      p[k] = pos[r + k];
-      float y = img[(r + k) * LD + col];
-      if (a.bias) y += (float)a.bias[head * D + i];
-      v[k] = (bf16_t)y;
+  for (int e = 0; e < 4; ++e) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(even[e]), __float_as_uint(odd[e]), false, false);
+    s.lo[e] = __uint_as_float(r[0]);
+    s.hi[e] = __uint_as_float(r[1]);
+  }
+  return s;
+}
+
+// Of two tiles' sums of tokens 0..7 (even) and 8..15 (odd lanes of eight): lanes 8..15 of a row of sixteen give the first tile to the lanes eight below
+// and take the second.  Then x0 holds tile (xc >> 3) of token xc & 7, x1 that of token 8 + (xc & 7).
+__device__ __forceinline__ void trade_tiles(f32x4& x0, f32x4& x1, bool late) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const float got = __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(late ? x0[e] : x1[e]), 0x128 /* row_ror:8 */, 0xf, 0xf, true));
+    const float a = x0[e], b = x1[e];
+    x0[e] = late ? got : a;
+    x1[e] = late ? b : got;
+  }
+}
+
+// A wave with more sums than there are vector registers beside them: the sums of a tile of tokens leave the accumulator registers when it is
+// their turn (left alone the compiler brings all of them out first, and spills 24 to 240 registers a lane).
+template <int TN, int TM>
+__device__ __forceinline__ void in_turn(f32x4 (&acc)[TN][TM], int j) {
+  if constexpr (TN * TM > 32) {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < TN; ++i) asm volatile("" : "+a"(acc[i][j]));
+  }
+}
+
+// Whether the outputs of all of a wave's tiles exist and a token's four neighbours are one store (`tiles` from `tile0`, `cols` outputs each)
+__device__ __forceinline__ bool whole_tiles(const WideEpiArgs& a, int tile0, int tiles, int n_tiles, int cols) {
+  return tile0 + tiles <= n_tiles && (tile0 + tiles) * cols <= a.N && ((a.ldo | a.N) & 3) == 0;
+}
+
+template <int EPI, int TN, int TM>
+__device__ __forceinline__ void emit_tiles(const PromptArgs& p, f32x4 (&acc)[TN][TM], int tile0, int row0, int split, int lane) {
+  const WideEpiArgs& a = p.epi;
+  const int xc = lane & 15, xq = lane >> 4;
+  if constexpr (EPI == SD_EPI_SILU_MUL) {
+    bf16_t* out = reinterpret_cast<bf16_t*>(a.out) + (size_t)(row0 + xc) * a.ldo + (tile0 + (xq >> 1)) * 8 + (xq & 1) * 4;
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+      const bool here = row0 + 16 * j + xc < p.M;
+      in_turn(acc, j);
+#pragma unroll
+      for (int i = 0; i < TN; i += 2) {
+        const TileSums s = split_halves(acc[i][j], acc[i + 1 < TN ? i + 1 : i][j]);
+        const bf16x4 r = gated_of(s.lo, s.hi);
+        if (here && (i + 1 < TN || xq < 2)) *reinterpret_cast<bf16x4*>(out + (size_t)16 * j * a.ldo + i * 8) = r;
+      }
     }
-    const int page = pos[page_at + r];
-    auto at = [&](int pg) { return rp.vc + (((size_t)pg * rp.Hkv + (head - rp.Hq - rp.Hkv)) * D + i) * 16; };
-    if (aligned && (p[0] & 3) == 0 && p[0] >= 0 && p[1] == p[0] + 1 && p[2] == p[0] + 2 && p[3] == p[0] + 3 &&
-        pos[page_at + r + 3] == page) {
-      *reinterpret_cast<bf16x4*>(at(page) + sd_v_slot(p[0] & 15)) = v;
-    } else {
+  } else if constexpr (EPI == EPI_RELU_PAIR) {
+    bf16_t* out = reinterpret_cast<bf16_t*>(a.out) + (size_t)(row0 + xc) * a.ldo + tile0 * 16 + xq * 4;
 #pragma unroll
-      for (int k = 0; k < 4; ++k)
-        if (p[k] >= 0) at(pos[page_at + r + k])[sd_v_slot(p[k] & 15)] = v[k];
+    for (int j = 0; j < TM; ++j)
+      if (row0 + 16 * j + xc < p.M) {
+#pragma unroll
+        for (int i = 0; i < TN / 2; ++i) {
+          bf16x4 r;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) r[e] = (bf16_t)(fmaxf(acc[i][j][e], 0.f) * acc[i + TN / 2][j][e]);
+          *reinterpret_cast<bf16x4*>(out + (size_t)16 * j * a.ldo + i * 16) = r;
+        }
+      }
+  } else if constexpr (EPI == EPI_PARTIAL || EPI == SD_EPI_F32) {
+    const int64_t ld = EPI == EPI_PARTIAL ? p.n_tiles * 16 : a.ldo;
+    float* out = (EPI == EPI_PARTIAL ? p.part + (size_t)split * p.M * ld : reinterpret_cast<float*>(a.out)) + tile0 * 16 + xq * 4;
+    const bool late = xc & 8;
+    f32x4 bias[TN];
+    if (EPI == SD_EPI_F32 && a.bias) {
+#pragma unroll
+      for (int i = 0; i < TN; ++i) {
+        const bf16x4 b = *reinterpret_cast<const bf16x4*>(a.bias + (tile0 + i) * 16 + xq * 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) bias[i][e] = (float)b[e];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+      in_turn(acc, j);
+      const int m = row0 + 16 * j;
+#pragma unroll
+      for (int i = 0; i < TN; i += 2) {
+        f32x4 y[2] = {acc[i][j], acc[i + 1 < TN ? i + 1 : i][j]};
+        if (EPI == SD_EPI_F32 && a.bias)
+#pragma unroll
+          for (int n = 0; n < 2; ++n) y[n] += bias[i + n < TN ? i + n : i];
+        if (i + 1 < TN) {
+          trade_tiles(y[0], y[1], late);
+          float* to = out + (size_t)(m + (xc & 7)) * ld + (i + late) * 16;
+          if (m + (xc & 7) < p.M) *reinterpret_cast<f32x4*>(to) = y[0];
+          if (m + 8 + (xc & 7) < p.M) *reinterpret_cast<f32x4*>(to + 8 * ld) = y[1];
+        } else if (m + xc < p.M) {
+          *reinterpret_cast<f32x4*>(out + (size_t)(m + xc) * ld + i * 16) = y[0];
+        }
+      }
+    }
+  } else {
+    const size_t at = (size_t)(row0 + xc) * a.ldo + tile0 * 16 + xq * 4;
+    bf16_t* out = reinterpret_cast<bf16_t*>(a.out) + at;
+    const bf16_t* residual = a.residual + at;
+    // residuals of kBatch tiles of tokens at once, before the first store, which may change them for all the compiler knows
+    constexpr int kBatch = EPI == SD_EPI_RESIDUAL && TN * TM > 32 ? 32 / TN : TM;
+    bf16x4 bias[TN];
+    if (a.bias) {
+#pragma unroll
+      for (int i = 0; i < TN; ++i) bias[i] = *reinterpret_cast<const bf16x4*>(a.bias + (tile0 + i) * 16 + xq * 4);
+    }
+#pragma unroll
+    for (int j0 = 0; j0 < TM; j0 += kBatch) {
+      bf16x4 res[kBatch][TN];
+      if (EPI == SD_EPI_RESIDUAL) {
+#pragma unroll
+        for (int j = j0; j < TM && j < j0 + kBatch; ++j)
+          if (row0 + 16 * j + xc < p.M) {
+#pragma unroll
+            for (int i = 0; i < TN; ++i) res[j - j0][i] = *reinterpret_cast<const bf16x4*>(residual + (size_t)16 * j * a.ldo + i * 16);
+          }
+      }
+#pragma unroll
+      for (int j = j0; j < TM && j < j0 + kBatch; ++j) {
+        in_turn(acc, j);
+        if (row0 + 16 * j + xc < p.M) {
+#pragma unroll
+          for (int i = 0; i < TN; ++i) {
+            f32x4 y = acc[i][j];
+            if (a.bias) {
+#pragma unroll
+              for (int e = 0; e < 4; ++e) y[e] += (float)bias[i][e];
+            }
+            *reinterpret_cast<bf16x4*>(out + (size_t)16 * j * a.ldo + i * 16) = four_of<EPI>(y, res[j - j0][i]);
+          }
+        }
+        }
+    }
+  }
+}
+
+// Whether a wave's tiles of a QKV product can be stored from registers: pairs of tiles in one head, one position for all of a row, and
+// starts that four neighbours in one store allow.
+__device__ __forceinline__ bool whole_heads(const WideEpiArgs& a, int tile0, int tiles, int n_tiles) {
+  const WideRope& rp = a.rope;
+  const uintptr_t at = reinterpret_cast<uintptr_t>(a.out) | reinterpret_cast<uintptr_t>(rp.kc) | reinterpret_cast<uintptr_t>(rp.vc);
+  return tile0 + tiles <= n_tiles && rp.D % 32 == 0 && (tile0 & 1) == 0 && rp.cs && !rp.mp.pos && (a.ldo & 3) == 0 && (at & 7) == 0 &&
+         (reinterpret_cast<uintptr_t>(rp.cs) & 15) == 0;
+}
+
+// The four tokens of a quad's lanes and four channels, turned: lane b of the quad has channel b's four tokens.
+__device__ __forceinline__ bf16x4 turn_quad(const bf16x4& v, int lane) {
+  typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+  const u32x2 d = __builtin_bit_cast(u32x2, v);
+  unsigned t[2];
+#pragma unroll
+  for (int e = 0; e < 2; ++e) {   // (channel 2 e + (lane & 1) of this lane's token and its neighbour's)
+    const unsigned other = __builtin_amdgcn_mov_dpp(d[e], 0xB1, 0xf, 0xf, true);
+    const bool odd = lane & 1;
+    t[e] = __builtin_amdgcn_perm(odd ? d[e] : other, odd ? other : d[e], odd ? 0x07060302u : 0x05040100u);
+  }
+  const bool late = lane & 2;
+  const unsigned other = __builtin_amdgcn_mov_dpp(late ? t[0] : t[1], 0x4E, 0xf, 0xf, true);
+  const u32x2 r = {late ? other : t[0], late ? t[1] : other};
+  return __builtin_bit_cast(bf16x4, r);
+}
+
+// A wave's tiles of a QKV product: queries and keys rotated, keys and values into their pages.  A key's eight channels of a
+// page are 16 bytes, next to the next token's; a page row of a value's channel holds its tokens side by side, so four tokens of
+// a channel go in one store where they lie at neighbouring positions from a multiple of four on (others one by one).
+template <int TN, int TM>
+__device__ __forceinline__ void emit_heads(const PromptArgs& p, f32x4 (&acc)[TN][TM], int tile0, int row0, int lane) {
+  const WideEpiArgs& a = p.epi;
+  const WideRope& rp = a.rope;
+  const int xc = lane & 15, xq = lane >> 4, D = rp.D, half = D / 2, tph = D / 16;
+  int pos[TM], page[TM], turn[TM];   // position (-1: no such row), page, row of the cosines
+#pragma unroll
+  for (int j = 0; j < TM; ++j) {
+    const int m = row0 + 16 * j + xc, b = qkv_sequence(rp, min(m, p.M - 1));
+    pos[j] = m < p.M ? qkv_position(rp, m, b) : -1;
+    turn[j] = min(max(sd_rope_position(rp.mp, pos[j], b, m, 0), 0), rp.max_pos - 1);
+  }
+  if ((tile0 + TN - 1) / tph >= rp.Hq) {
+#pragma unroll
+    for (int j = 0; j < TM; ++j) page[j] = pos[j] >= 0 ? qkv_page(rp, qkv_sequence(rp, row0 + 16 * j + xc), pos[j]) : 0;
+  }
+#pragma unroll
+  for (int i = 0; i < TN; i += 2) {
+    if constexpr (TN * TM > 32) {   // (as in_turn)
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < TM; ++j) {
+        asm volatile("" : "+a"(acc[i][j]));
+        asm volatile("" : "+a"(acc[i + 1][j]));
+      }
+    }
+    const int head = (tile0 + i) / tph, in_head = (tile0 + i - head * tph) * 8;
+    if (head >= rp.Hq + rp.Hkv) {
+      bf16_t* vp = rp.vc + (size_t)(head - rp.Hq - rp.Hkv) * D * 16;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const int i0 = in_head + 8 * e + (xq & 1) * 4 + (xq >> 1) * half;   // channel of acc[..][0]
+        f32x4 bias = {0.f, 0.f, 0.f, 0.f};
+        if (a.bias)
+#pragma unroll
+          for (int c = 0; c < 4; ++c) bias[c] = (float)a.bias[head * D + i0 + c];
+#pragma unroll
+        for (int j = 0; j < TM; ++j) {
+          bf16x4 v;
+#pragma unroll
+          for (int c = 0; c < 4; ++c) v[c] = (bf16_t)(a.bias ? acc[i + e][j][c] + bias[c] : acc[i + e][j][c]);
+          const int p0 = __builtin_amdgcn_mov_dpp(pos[j], 0, 0xf, 0xf, true), g0 = __builtin_amdgcn_mov_dpp(page[j], 0, 0xf, 0xf, true);
+          const unsigned long long ok = __ballot(pos[j] >= 0 && (p0 & 3) == 0 && pos[j] == p0 + (lane & 3) && page[j] == g0);
+          const bf16x4 t = turn_quad(v, lane);
+          bf16_t* to = vp + (size_t)page[j] * rp.Hkv * D * 16;
+          if ((ok >> (lane & 60) & 15) == 15) {
+            *reinterpret_cast<bf16x4*>(to + (i0 + (lane & 3)) * 16 + sd_v_slot(p0 & 15)) = t;
+          } else if (pos[j] >= 0) {
+#pragma unroll
+            for (int c = 0; c < 4; ++c) to[(i0 + c) * 16 + sd_v_slot(pos[j] & 15)] = v[c];
+          }
+        }
+      }
+      continue;
+    }
+    const int i0 = in_head + (xq >> 1) * 8 + (xq & 1) * 4;   // channel of the even halves' first sum
+    f32x4 b_lo = {0.f, 0.f, 0.f, 0.f}, b_hi = b_lo;
+    if (a.bias)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        b_lo[c] = (float)a.bias[head * D + i0 + c];
+        b_hi[c] = (float)a.bias[head * D + i0 + half + c];
+      }
+    f32x4 cs[TM], sn[TM];
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+      cs[j] = *reinterpret_cast<const f32x4*>(rp.cs + (size_t)turn[j] * D + i0);
+      sn[j] = *reinterpret_cast<const f32x4*>(rp.cs + (size_t)turn[j] * D + i0 + half);
+    }
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+      const TileSums s = split_halves(acc[i][j], acc[i + 1][j]);
+      bf16x4 l, h;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const float lo = round_bf16(a.bias ? s.lo[c] + b_lo[c] : s.lo[c]), hi = round_bf16(a.bias ? s.hi[c] + b_hi[c] : s.hi[c]);
+        l[c] = (bf16_t)(lo * cs[j][c] - hi * sn[j][c]);
+        h[c] = (bf16_t)(hi * cs[j][c] + lo * sn[j][c]);
+      }
+      if (pos[j] < 0) {
+      } else if (head < rp.Hq) {
+        bf16_t* q = reinterpret_cast<bf16_t*>(a.out) + (size_t)(row0 + 16 * j + xc) * a.ldo + head * D + i0;
+        *reinterpret_cast<bf16x4*>(q) = l;
+        *reinterpret_cast<bf16x4*>(q + half) = h;
+      } else {
+        bf16_t* k = rp.kc + ((size_t)page[j] * rp.Hkv + (head - rp.Hq)) * D * 16 + (pos[j] & 15) * 8 + (i0 & 7);
+        *reinterpret_cast<bf16x4*>(k + (i0 >> 3) * 128) = l;
+        *reinterpret_cast<bf16x4*>(k + ((i0 + half) >> 3) * 128) = h;
+      }
     }
   }
 }
@@ -322,36 +562,29 @@ __global__ __launch_bounds__(256, blocks_per_cu(TN, TM, STAGES, SPLIT)) void pro
 #pragma unroll
       for (int j = 0; j < TM; ++j) acc[i][j] = tot[i][j] + acc[i][j];
   }
-  // acc[i][j][reg] = (tile row 4 * xq + reg of tile i, token 16 j + xc).  Through LDS, 16 token rows at a time
-  // and each wave for itself, so that the lanes of a store hold neighbouring outputs of a row (and the epilogue
-  // is there once per token tile, not once per pair of tiles).
+  if constexpr (EPI != EPI_QKV_ROPE) {
+    constexpr int kTiles = PAIR ? TN / 2 : TN, kCols = EPI == SD_EPI_SILU_MUL ? 8 : 16;
+    const int first = tile0 + wn * kTiles, tiles = PAIR ? a.n_tiles / 2 : a.n_tiles;
+    if (EPI == EPI_PARTIAL ? first + kTiles <= tiles : whole_tiles(a.epi, first, kTiles, tiles, kCols) && !(EPI == SD_EPI_SILU_MUL && a.epi.bias)) {
+      emit_tiles<EPI, TN, TM>(a, acc, first, row0 + wm * TM * 16, split, lane);
+      return;
+    }
+  }
+  constexpr bool QKV = EPI == EPI_QKV_ROPE;
+  if constexpr (QKV && TN % 2 == 0) {
+    if (whole_heads(a.epi, tile0 + wn * TN, TN, a.n_tiles)) {
+      emit_heads<TN, TM>(a, acc, tile0 + wn * TN, row0 + wm * TM * 16, lane);
+      return;
+    }
+  }
+  // Other outputs through LDS, 16 token rows at a time and each wave for itself, so that the lanes of a store hold
+  // neighbouring outputs of a row (and the epilogue is there once per token tile, not once per pair of tiles).
   constexpr bool PAIRED = EPI == SD_EPI_SILU_MUL || EPI == EPI_QKV_ROPE;
   constexpr int kLd = TN * 16 + 4;                        // floats; 16 rows start on different banks
   constexpr int kUnits = PAIRED || PAIR ? TN * 2 : TN * 4;  // of a row; 64 lanes take 64 / kUnits rows at once
   float* img = reinterpret_cast<float*>(wave < 2 ? s0 : s1) + (wave & 1) * 16 * kLd;
   const int u = lane % kUnits, ui = PAIRED ? u >> 1 : u >> 2, r0 = PAIRED ? (u & 1) * 4 : (u & 3) * 4;
   const int tile = tile0 + wn * (PAIR ? TN / 2 : TN) + ui;
-  // EPI_QKV_ROPE: positions and pages of the wave's rows, asked for once (a row outside the pass: position -1), and whether the
-  // wave's tiles are values (the last heads): these are written four tokens at a time, a page row of a channel holding its tokens
-  // side by side.
-  constexpr bool QKV = EPI == EPI_QKV_ROPE;
-  int* place = reinterpret_cast<int*>(reinterpret_cast<float*>(wave < 2 ? s0 : s1) + 2 * 16 * kLd) + (wave & 1) * 2 * TM * 16;
-  static_assert(!QKV || (2 * 16 * kLd + 4 * TM * 16) * 4 <= kABytes + kBBytes, "images and places of two waves in a stage");
-  bool values = false;
-  if constexpr (QKV) {
-    const WideRope& rp = a.epi.rope;
-#pragma unroll
-    for (int r = 0; r < TM * 16; r += 64) {
-      const int m = row0 + wm * TM * 16 + r + lane, b = qkv_sequence(rp, min(m, a.M - 1));
-      if (r + lane < TM * 16) {
-        const int pos = m < a.M ? qkv_position(rp, m, b) : -1;
-        place[r + lane] = pos;
-        place[TM * 16 + r + lane] = pos >= 0 ? qkv_page(rp, b, pos) : 0;
-      }
-    }
-    values = (tile0 + wn * TN) / (rp.D / 16) >= rp.Hq + rp.Hkv;
-    asm volatile("" ::: "memory");  // (other lanes read them)
-  }
 #pragma unroll
   for (int j = 0; j < TM; ++j) {
 #pragma unroll
@@ -363,12 +596,6 @@ __global__ __launch_bounds__(256, blocks_per_cu(TN, TM, STAGES, SPLIT)) void pro
       *reinterpret_cast<f32x4*>(img + xc * kLd + i * 16 + 4 * xq) = y;
     }
     asm volatile("" ::: "memory");  // (other lanes read them: the stores of a lane without a unit stay here)
-    if constexpr (QKV) {
-      if (values) {
-        emit_values<TN, kLd>(a.epi, img, place + j * 16, TM * 16, tile0 + wn * TN, a.n_tiles, lane);
-        continue;
-      }
-    }
 #pragma unroll 1
     for (int r = lane < 64 / kUnits * kUnits ? lane / kUnits : 16; r < 16; r += 64 / kUnits) {
       const int m = row0 + (wm * TM + j) * 16 + r;
@@ -382,10 +609,7 @@ __global__ __launch_bounds__(256, blocks_per_cu(TN, TM, STAGES, SPLIT)) void pro
               bf16x4{(bf16_t)lo[0], (bf16_t)lo[1], (bf16_t)lo[2], (bf16_t)lo[3]};
         else if constexpr (EPI == EPI_PARTIAL)
           *reinterpret_cast<f32x4*>(a.part + ((size_t)split * a.M + m) * a.n_tiles * 16 + tile * 16 + r0) = lo;
-        else if constexpr (QKV) {
-          const int pos = place[j * 16 + r];
-          if (pos >= 0) emit_qkv(a.epi, m, tile, r0, lo, hi, qkv_sequence(a.epi.rope, m), pos, place[TM * 16 + j * 16 + r]);
-        } else emit_unit<EPI>(a.epi, m, tile, r0, lo, hi);
+        else emit_unit<EPI>(a.epi, m, tile, r0, lo, hi);
       }
     }
   }

@@ -79,7 +79,7 @@ __device__ __forceinline__ int qkv_page(const WideRope& rp, int b, int pos) {
 
 // Four units (i0 .. i0 + 3 and their partners half a head on) of a rotated row: a lane's four queries, and its four keys, lie next
 // to each other in memory, so they are one store of 8 bytes where the buffers' starts allow it (2 bytes at a time, 6144 x 4096 at
-// 1024 rows 82.1 us, 4096 229; now 76.3 and 206; 4608 x 3584 at 2946 rows of 8 prompts 138 and 130).
+// 1024 rows 82.1 us, 4096 229; 8 bytes 76.3 and 206; 4608 x 3584 at 2946 rows of 8 prompts 138 and 130).
 __device__ __forceinline__ void emit_qkv(const WideEpiArgs& a, int m, int tile, int r0, f32x4 lo, f32x4 hi, int b, int pos,
                                          int page) {
   const WideRope& rp = a.rope;
@@ -164,6 +164,26 @@ __device__ __forceinline__ void emit_qkv(const WideEpiArgs& a, int m, int tile, 
   }
 }
 
+// Four neighbouring outputs of their sums (and residuals), and of their gate and up sums.
+template <int EPI>
+__device__ __forceinline__ bf16x4 four_of(const f32x4& y, const bf16x4& res) {
+  bf16x4 r;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    if (EPI == SD_EPI_STORE) r[j] = (bf16_t)y[j];
+    else if (EPI == SD_EPI_RESIDUAL) r[j] = (bf16_t)(round_bf16(y[j]) + (float)res[j]);
+    else if (EPI == SD_EPI_RELU) r[j] = (bf16_t)fmaxf(round_bf16(y[j]), 0.f);
+    else r[j] = (bf16_t)gelu_tanh_w(round_bf16(y[j]));
+  }
+  return r;
+}
+__device__ __forceinline__ bf16x4 gated_of(const f32x4& g, const f32x4& up) {
+  bf16x4 r;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) r[j] = (bf16_t)(round_bf16(silu_w(round_bf16(g[j]))) * round_bf16(up[j]));
+  return r;
+}
+
 // The epilogue of 4 consecutive tile rows r0..r0+3 of tile `tile` for token row m: lo holds
 // their sums; in the paired modes hi holds the sums of rows r0+8..r0+11 (the up rows of a
 // gated tile, the rotation partners of a rotary tile) and r0 is 0 or 4.
@@ -203,11 +223,7 @@ __device__ __forceinline__ void emit_unit(const WideEpiArgs& a, int m, int tile,
           up[j] += (float)a.bias[a.N + n0 + j];
         }
       }
-      bf16x4 r;
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        r[j] = (bf16_t)(round_bf16(silu_w(round_bf16(g[j]))) * round_bf16(up[j]));
-      *reinterpret_cast<bf16x4*>(reinterpret_cast<bf16_t*>(a.out) + (size_t)m * a.ldo + n0) = r;
+      *reinterpret_cast<bf16x4*>(reinterpret_cast<bf16_t*>(a.out) + (size_t)m * a.ldo + n0) = gated_of(g, up);
       return;
     }
 #pragma unroll
@@ -245,17 +261,9 @@ __device__ __forceinline__ void emit_unit(const WideEpiArgs& a, int m, int tile,
         *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(a.out) + o) = y;
         return;
       }
-      bf16x4 r;
       bf16x4 res = {0, 0, 0, 0};
       if (EPI == SD_EPI_RESIDUAL) res = *reinterpret_cast<const bf16x4*>(a.residual + o);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if (EPI == SD_EPI_STORE) r[j] = (bf16_t)y[j];
-        else if (EPI == SD_EPI_RESIDUAL) r[j] = (bf16_t)(round_bf16(y[j]) + (float)res[j]);
-        else if (EPI == SD_EPI_RELU) r[j] = (bf16_t)fmaxf(round_bf16(y[j]), 0.f);
-        else r[j] = (bf16_t)gelu_tanh_w(round_bf16(y[j]));
-      }
-      *reinterpret_cast<bf16x4*>(reinterpret_cast<bf16_t*>(a.out) + o) = r;
+      *reinterpret_cast<bf16x4*>(reinterpret_cast<bf16_t*>(a.out) + o) = four_of<EPI>(y, res);
       return;
     }
 #pragma unroll

@@ -222,6 +222,16 @@ __device__ __forceinline__ float wave_max(float v) {
   return v;
 }
 
+// Maximum and sum over a pair of lanes half a wave apart.
+__device__ __forceinline__ float halves_max(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float halves_sum(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
 // Rotary position of frequency index i (0 <= i < D/2) of token row m of sequence b whose
 // cache position is cache_pos: the cache position itself, or the multimodal one.
 struct RopePos {

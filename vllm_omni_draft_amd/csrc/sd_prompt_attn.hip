@@ -15,8 +15,13 @@
 // added in order, then the splits, against the maximum over all splits.  A row thus has the bits that a decode pass
 // gives it, and the bits do not depend on how a prompt is cut.  The weights of chains and splits need the maxima of
 // everything first: a first sweep computes the scores for the maxima alone (a third of the matrix work), which costs
-// less than keeping the splits' sums.  A stage is one chain of a split (tiles c and c + 4 of eight), so that only one
-// chain's sums, a quarter of the channels at a time, are live beside the split's and the row's.
+// less than keeping the splits' sums.  It needs keys only and no order, so its stages are 128 keys, half the barriers of the second
+// sweep's, in which a stage is one chain of a split (tiles c and c + 4 of eight), so that only one chain's sums, a quarter of the
+// channels at a time, are live beside the split's and the row's.
+// What bounds it: products and vector work of a wave follow each other (two waves a SIMD: 55 % and 36 % of the time at 4096 tokens).  us, stages of
+// one chain in both sweeps and exchanges through LDS / now, 32 heads over 8: 4096 tokens of size 128 302 / 278, 1024 64 / 60, of
+// size 64 38 / 35; 8 prompts of 64..1000, 28 over 4, 72 / 67.  Four stages in flight where a block is alone on its CU, both tiles' products before
+// their weights, and raised wave priority around products were no faster.
 #include <mutex>
 #include <type_traits>
 
@@ -49,8 +54,9 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(PromptAttnArgs a) {
   constexpr int kLoads = kPage / 1024;          // direct loads of a page
   constexpr int kPages = 2 * TPC;               // pages of a stage: a wave brings one (of K and of V)
   constexpr int kSplit = 128 * TPC, kSplitPages = kSplit / 16;
-  __shared__ __attribute__((aligned(1024))) char s0[2 * kPages * kPage];
-  __shared__ __attribute__((aligned(1024))) char s1[2 * kPages * kPage];
+  static_assert(2 * kPages <= 8, "a stage of either sweep");
+  __shared__ __attribute__((aligned(1024))) char s0[8 * kPage];
+  __shared__ __attribute__((aligned(1024))) char s1[8 * kPage];
   __shared__ int32_t table[kTable];
   extern __shared__ float split_max[];          // [splits][kRows]
 
@@ -65,7 +71,9 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(PromptAttnArgs a) {
   const int m_rows = n_tok * G;
   const int kv_len = pos0 + n_tok;
   const int last_page = (kv_len - 1) >> 4;
-  const int n_st = (kv_len + kSplit - 1) / kSplit * 4;   // stages of a sweep
+  const int n_st = (kv_len + kSplit - 1) / kSplit * 4;   // stages of the second sweep
+  constexpr int kWide = 128 / 32;                        // tiles of a stage of the first sweep
+  const int n_max = (kv_len + 255) / 256 * 2;            // its stages, an even number: half a split or a whole one
 
   // this lane's query row, its keys, and how far the wave's rows see
   const int m = wave * 32 + r;
@@ -93,26 +101,28 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(PromptAttnArgs a) {
     for (int e = tid; e < kTable; e += 256) table[e] = bt[min(min(first + e, last_page), a.max_blocks - 1)];
   };
   auto first_page = [&](int st) { return (st >> 2) * kSplitPages; };
-  // stage st of a sweep: chain st & 3 of split st >> 2; wave w brings page w & 1 of tile chain + 4 (w >> 1): K, and in
-  // the second sweep V behind the K pages
-  auto load = [&](char* s, int st, bool values) __attribute__((always_inline)) {
-    if (wave >= kPages) return;
-    const int page = min(first_page(st) + 2 * ((st & 3) + 4 * (wave >> 1)) + (wave & 1), last_page);
-    const int blk = __builtin_amdgcn_readfirstlane(table[max(page - table0, 0)]);
+  auto bring = [&](char* to, const bf16_t* pool, int page) __attribute__((always_inline)) {
+    const int blk = __builtin_amdgcn_readfirstlane(table[max(min(page, last_page) - table0, 0)]);
     const size_t at = ((size_t)blk * a.Hkv + kvh) * (size_t)(D * 16);
-    const auto kr = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(a.kc + at), 0, kPage, 0x00027000);
+    const auto from = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(pool + at), 0, kPage, 0x00027000);
 #pragma unroll
     for (int i = 0; i < kLoads; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(kr, (lds_void*)(s + wave * kPage + i * 1024), 16, lane * 16 + i * 1024,
-                                               0, 0, 0);
-    if (!values) return;
-    const auto vr = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(a.vc + at), 0, kPage, 0x00027000);
-#pragma unroll
-    for (int i = 0; i < kLoads; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(vr, (lds_void*)(s + (kPages + wave) * kPage + i * 1024), 16,
-                                               lane * 16 + i * 1024, 0, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (lds_void*)(to + i * 1024), 16, lane * 16 + i * 1024, 0, 0, 0);
   };
-  // scores of tile u of the stage (key0: its first key), times the scale, what a row does not see at -inf; their maximum
+  // first sweep: stage st holds the K pages of 128 keys, two a wave
+  auto load_keys = [&](char* s, int st) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) bring(s + (wave * 2 + i) * kPage, a.kc, st * 8 + wave * 2 + i);
+  };
+  // second sweep: stage st is chain st & 3 of split st >> 2; wave w brings page w & 1 of tile chain + 4 (w >> 1): K, and V behind
+  // the K pages
+  auto load = [&](char* s, int st) __attribute__((always_inline)) {
+    if (wave >= kPages) return;
+    const int page = first_page(st) + 2 * ((st & 3) + 4 * (wave >> 1)) + (wave & 1);
+    bring(s + wave * kPage, a.kc, page);
+    bring(s + (kPages + wave) * kPage, a.vc, page);
+  };
+  // scores of tile u of a stage's K pages (key0: its first key), what a row does not see at -inf
   auto scores = [&](const char* s, int u, int key0, f32x16& sc) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) sc[i] = 0.f;
@@ -122,26 +132,30 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(PromptAttnArgs a) {
     for (int ks = 0; ks < KS; ++ks)
       sc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(kp + ks * 512), qf[ks], sc, 0, 0, 0);
     if (key0 + 32 > wave_first) {  // some row does not see all of the tile
+      const int left = see - key0 - 4 * h;
 #pragma unroll
       for (int i = 0; i < 16; ++i)
-        if (key0 + (i & 3) + 8 * (i >> 2) + 4 * h >= see) sc[i] = -INFINITY;
+        if ((i & 3) + 8 * (i >> 2) >= left) sc[i] = -INFINITY;
     }
+  };
+  auto max_of = [&](const f32x16& sc) __attribute__((always_inline)) {
     float top = sc[0];
 #pragma unroll
     for (int i = 1; i < 16; ++i) top = fmaxf(top, sc[i]);
-    top *= a.scale_log2;  // (positive: rounding keeps the order, the maximum is that of the scaled scores)
-    return fmaxf(top, __shfl_xor(top, 32, 64));
+    return top;
   };
   auto key_of = [&](int st, int u) { return (st >> 2) * kSplit + ((st & 3) + 4 * u) * 32; };
   auto find_max = [&](const char* s, int st) __attribute__((always_inline)) {
-#pragma unroll
-    for (int u = 0; u < TPC; ++u)
-      if (key_of(st, u) < wave_last) {
+#pragma unroll 2   // (all four: 288 us for 278, registers in scratch)
+    for (int u = 0; u < kWide; ++u)
+      if (st * 128 + u * 32 < wave_last) {
         f32x16 sc;
-        top_split = fmaxf(top_split, scores(s, u, key_of(st, u), sc));
+        scores(s, u, st * 128 + u * 32, sc);
+        top_split = fmaxf(top_split, max_of(sc));
       }
-    if ((st & 3) == 3) {
-      if (h == 0) split_max[(st >> 2) * kRows + m] = top_split;
+    if (TPC == 1 ? st * 128 < kv_len : st & 1) {   // (the split's last stage)
+      top_split = halves_max(top_split * a.scale_log2);  // (positive: rounding keeps the order, the maximum is that of the scaled scores)
+      if (h == 0) split_max[st / TPC * kRows + m] = top_split;
       top_row = fmaxf(top_row, top_split);
       top_split = -INFINITY;
     }
@@ -162,7 +176,8 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(PromptAttnArgs a) {
           continue;
         }
         f32x16 sc;
-        const float top_new = fmaxf(top, scores(s, u, key0, sc));
+        scores(s, u, key0, sc);
+        const float top_new = fmaxf(top, halves_max(max_of(sc) * a.scale_log2));
         const float use = top_new == -INFINITY ? 0.f : top_new;
         alpha = __builtin_amdgcn_exp2f(top - use);
         top = top_new;
@@ -175,7 +190,7 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(PromptAttnArgs a) {
         }
         l = l * alpha + sum;
       }
-      l += __shfl_xor(l, 32, 64);
+      l = halves_sum(l);
       const float w = top_all == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(top - top_all);
       l_split += w * l;
       const bool rescale = TPC > 1 && __any(alpha != 1.f);  // (a factor of exactly 1 in every lane changes nothing)
@@ -213,31 +228,34 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(PromptAttnArgs a) {
         }
     }
   };
-  // stage x of the two sweeps is in `cur` once this wave's loads have landed and every wave is here; then nobody
-  // reads `nxt` any more
+  // stage x (the first sweep's, then the second's) is in `cur` once this wave's loads have landed and every wave is here; then
+  // nobody reads `nxt` any more
   auto step = [&](char* cur, char* nxt, int x, auto sweep) __attribute__((always_inline)) {
+    constexpr bool kFirst = decltype(sweep)::value == 0;
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     const int y = x + 1;
-    if (y < 2 * n_st) {  // (uniform)
-      const int st = y < n_st ? y : y - n_st;
-      if (first_page(st) < table0 || first_page(st) + kSplitPages > table0 + kTable) {
-        fill_table(first_page(st));
+    if (y < n_max + n_st) {  // (uniform)
+      const bool keys = kFirst && y < n_max;
+      const int first = keys ? y * 8 : first_page(y - n_max), pages = keys ? 8 : kSplitPages;
+      if (first < table0 || first + pages > table0 + kTable) {
+        fill_table(first);
         __syncthreads();
       }
-      load(nxt, st, y >= n_st);
+      if (keys) load_keys(nxt, y);
+      else load(nxt, y - n_max);
     }
-    if constexpr (decltype(sweep)::value == 0) find_max(cur, x);
-    else attend(cur, x - n_st);
+    if constexpr (kFirst) find_max(cur, x);
+    else attend(cur, x - n_max);
   };
   fill_table(0);
   __syncthreads();
-  load(s0, 0, false);
+  load_keys(s0, 0);
   // (an even number of stages in each sweep)
-  for (int x = 0; x < n_st; x += 2) {
+  for (int x = 0; x < n_max; x += 2) {
     step(s0, s1, x, std::integral_constant<int, 0>{});
     step(s1, s0, x + 1, std::integral_constant<int, 0>{});
   }
-  for (int x = n_st; x < 2 * n_st; x += 2) {
+  for (int x = n_max; x < n_max + n_st; x += 2) {
     step(s0, s1, x, std::integral_constant<int, 1>{});
     step(s1, s0, x + 1, std::integral_constant<int, 1>{});
   }

@@ -846,6 +846,31 @@ def test_rows_softmax_attention_against_float64(H, G, dk, dv, window, keep):
     assert off < 3e-6, off
 
 
+@pytest.mark.parametrize("F,W", [(8, 8), (40, 504), (2040, 512), (24, 2048), (2056, 2064), (13 * 8, 4104)])
+@pytest.mark.parametrize("act", ["silu", "relu2"])
+def test_moe_experts_of_a_few_assignments(F, W, act):
+    """Rows and matrices of less than 512 columns, at the edges of the 2048 whose weights and values are asked for ahead, and of more; column
+    counts that leave waves without work; an index of no expert among the chosen (its row is left as it was)."""
+    from vllm_omni_draft_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(F * W)
+    n, E, top, mats = 5, 3, 2, 1 if act == "relu2" else 2
+    x = torch.randn(n, W, generator=g, device="cuda")
+    gu = (torch.randn(E, mats * F, W, generator=g, device="cuda") * W ** -0.5).to(torch.bfloat16)
+    dn = (torch.randn(E, W, F, generator=g, device="cuda") * F ** -0.5).to(torch.bfloat16)
+    sel = torch.tensor([[0, 1], [2, 0], [1, 2], [2, 1], [0, E]], dtype=torch.int32, device="cuda")
+    w = torch.rand(n, top, generator=g, device="cuda") + 0.5
+    out = ops.moe_experts(x, sel, w, gu, dn, True, act)
+    for r in range(n):
+        for t in range(top):
+            e = int(sel[r, t])
+            if e >= E:
+                continue
+            h = (gu[e].double() @ x[r].to(torch.bfloat16).double()) * w[r, t].double()
+            a = torch.relu(h) ** 2 if mats == 1 else torch.nn.functional.silu(h[:F]) * h[F:]
+            # (an activation beside a rounding edge of bf16 may round the other way: 2^-8 of it at most)
+            assert rel(out[r, t], dn[e].double() @ a.to(torch.bfloat16).double()) < 2 ** -8, (r, t)
+
+
 @pytest.mark.parametrize("E,F,W,n", [(4, 96, 160, 100), (3, 64, 128, 63), (2, 160, 96, 300), (5, 320, 64, 200)])
 @pytest.mark.parametrize("act,scale_input", [("silu", True), ("silu", False), ("relu2", False)])
 def test_moe_experts_of_many_rows_have_the_bits_of_few(E, F, W, n, act, scale_input):

@@ -13,9 +13,9 @@
 // of either operand: one value of piece c.  Rows past the matrix and k past K are out of the buffers' bounds and arrive as
 // zeros.
 //
-// us, both operands through registers into two LDS buffers before / now: 777 rows of 13312 x 1024 251 / 188, 32000 x 1024
-// 528 / 413 (123 TFLOP/s), 1024 x 4096 gated 122 / 98, 1024 x 1024 33 / 22; 300 rows of 13312 x 1024 166 / 87, 33 rows 35 / 23;
-// 2048 rows of 4096 x 4096 615 / 490 (140 TFLOP/s).
+// us, both operands through registers into two LDS buffers / this way with four waves a block / with eight: 777 rows of 13312 x 1024 251 / 182 /
+// 180, 32000 x 1024 528 / 412 / 406 (125 TFLOP/s), 1024 x 4096 gated 122 / 89 / 81, 1024 x 1024 33 / 21.7 / 20.3; 300 rows of 13312 x
+// 1024 166 / 86 / 83, 4096 x 4096 - / 133 / 128; 2048 rows of 4096 x 4096 615 / 489 / 485 (142 TFLOP/s), gated 1024 x 4096 - / 157 / 142.
 #include "sd_common.h"
 
 namespace {
@@ -34,10 +34,13 @@ constexpr int stage_bytes(int nt, int mt, bool gated) { return (64 * nt + 64 * m
 // as many as leave room for two blocks a CU (128 x 64 gated: one)
 constexpr int stages_of(int nt, int mt, bool gated) { return stage_bytes(nt, mt, gated) * 8 <= 160 * 1024 ? 4 : 3; }
 
+// Eight waves, a quarter of the rows and half the columns each: two on a SIMD where a block is alone on its CU, so that one multiplies
+// while the other reads its fragments or waits for the barrier (four waves before: see the figures above).
+constexpr int kWaves = 8;
 template <int NT, int MT, bool GATED>
-__global__ __launch_bounds__(256, NT > 1 && GATED ? 1 : 2) void rows_f32_kernel(F32Args a) {
+__global__ __launch_bounds__(64 * kWaves, NT > 1 && GATED ? 1 : 2) void rows_f32_kernel(F32Args a) {
   constexpr int BN = 64 * NT, BM = 64 * MT, S = stages_of(NT, MT, GATED), kStage = stage_bytes(NT, MT, GATED);
-  constexpr int kWLoads = BN / 32, kXLoads = BM / 32, kLoads = kWLoads + kXLoads * (GATED ? 2 : 1);   // of a wave and stage
+  constexpr int kWLoads = BN / (8 * kWaves), kXLoads = BM / (8 * kWaves), kLoads = kWLoads + kXLoads * (GATED ? 2 : 1);   // of a wave and stage
   __shared__ __attribute__((aligned(1024))) char s0[kStage];
   __shared__ __attribute__((aligned(1024))) char s1[kStage];
   __shared__ __attribute__((aligned(1024))) char s2[kStage];
@@ -85,7 +88,7 @@ __global__ __launch_bounds__(256, NT > 1 && GATED ? 1 : 2) void rows_f32_kernel(
       put(i < kWLoads ? wr : i < kWLoads + kXLoads ? xr : gr, s + at * 1024, in && row != kOutside ? row + k : kOutside);
     }
   };
-  constexpr int TN = 2 * NT, TM = 2 * MT;   // tiles of 16 x 16 of a wave
+  constexpr int TN = 2 * NT, TM = 8 * MT / kWaves;   // tiles of 16 x 16 of a wave
   f32x4 acc[TN][TM];
 #pragma unroll
   for (int i = 0; i < TN; ++i)
@@ -203,8 +206,8 @@ int launch(F32Args a, int batch, hipStream_t st) {
   a.n_blocks = (a.N + 64 * NT - 1) / (64 * NT);
   a.m_blocks = (a.M + 64 * MT - 1) / (64 * MT);
   const dim3 grid(a.n_blocks * a.m_blocks, 1, batch);
-  if (a.x2) rows_f32_kernel<NT, MT, true><<<grid, 256, 0, st>>>(a);
-  else rows_f32_kernel<NT, MT, false><<<grid, 256, 0, st>>>(a);
+  if (a.x2) rows_f32_kernel<NT, MT, true><<<grid, 64 * kWaves, 0, st>>>(a);
+  else rows_f32_kernel<NT, MT, false><<<grid, 64 * kWaves, 0, st>>>(a);
   SD_CHECK_LAUNCH("sd_matmul_rows");
   return SD_OK;
 }
@@ -216,10 +219,9 @@ int sd_rows_f32_(const float* x, const float* x2, int64_t ldx, const float* w, c
                  int N, int K, int batch, int64_t bx, int64_t bw, int64_t by, bf16_t* yb, hipStream_t st) {
   const F32Args a{x, x2, w, bias, y, yb, ldx, ldy, bx, bw, by, M, N, K, 0, 0};
   // Blocks go over the CUs in rounds, and a round of 128 x 64 costs 1.85 of 64 x 64 (a 64 x 64 block alone on its CU .60 us a
-  // stage of 32 columns, one of two or more .53; 128 x 64: 1.05 and .98).  us of 64 x 64 / 128 x 64: 13312 x 1024 at 300 rows
-  // 95 / 106, 777 188 / 191, 2048 426 / 411; 32000 x 1024 at 777 rows 421 / 410; 4096 x 4096 at 777 262 / 245, 1024 x 4096
-  // 79 / 136.  128 x 128, 192 x 128 and 256 x 128 are slower than the better of the two everywhere (13312 x 1024 at 2048 rows 481,
-  // 503, 528).
+  // stage of 32 columns, one of two or more .53; 128 x 64: 1.05 and .98).  us of 64 x 64 / 128 x 64: 13312 x 1024 at 2048 rows 422 / 407;
+  // 32000 x 1024 at 777 421 / 406; 4096 x 4096 at 777 248 / 242, 300 125 / 128; 1024 x 4096 gated at 2048 153 / 142, 777 81 / 136.
+  // 128 x 128, 192 x 128 and 256 x 128 (of four waves) are slower than the better of the two everywhere (13312 x 1024 at 2048 rows 481, 503, 528).
   const long n1 = ((long)((N + 63) / 64) * ((M + 63) / 64) * batch + 255) / 256;
   const long n2 = ((long)((N + 127) / 128) * ((M + 63) / 64) * batch + 255) / 256;
   const float us1 = n1 == 1 ? .60f : .53f * n1, us2 = n2 == 1 ? 1.05f : .98f * n2;

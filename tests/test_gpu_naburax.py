@@ -871,6 +871,24 @@ def test_moe_experts_of_a_few_assignments(F, W, act):
             assert rel(out[r, t], dn[e].double() @ a.to(torch.bfloat16).double()) < 2 ** -8, (r, t)
 
 
+@pytest.mark.parametrize("E,n", [(1, 9), (3, 512), (3, 513), (1024, 700), (1025, 700), (2050, 1300)])
+def test_assignments_grouped_by_expert(E, n):
+    """One expert, groups at the edges of the 1024 assignments that a trip takes and of the 1024 experts counted at a time, experts that
+    nobody chose, and indices of no expert (their rows are left): rows grouped with others against eight rows at a time, whose
+    assignments are not grouped."""
+    from vllm_omni_draft_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(E + n)
+    F = W = 16
+    x = torch.randn(n, W, generator=g, device="cuda")
+    gu, dn = (torch.randn(E, r, W, generator=g, device="cuda") for r in (2 * F, W))
+    sel = torch.randint(0, E + 1, (n, 2), generator=g, device="cuda").to(torch.int32)
+    sel[n // 2:, 0] = E - 1
+    w = torch.rand(n, 2, generator=g, device="cuda")
+    out = ops.moe_experts(x, sel, w, gu, dn)
+    few = torch.cat([ops.moe_experts(x[i:i + 8], sel[i:i + 8], w[i:i + 8], gu, dn) for i in range(0, n, 8)])
+    assert torch.equal(out[sel < E], few[sel < E])
+
+
 @pytest.mark.parametrize("E,F,W,n", [(4, 96, 160, 100), (3, 64, 128, 63), (2, 160, 96, 300), (5, 320, 64, 200)])
 @pytest.mark.parametrize("act,scale_input", [("silu", True), ("silu", False), ("relu2", False)])
 def test_moe_experts_of_many_rows_have_the_bits_of_few(E, F, W, n, act, scale_input):

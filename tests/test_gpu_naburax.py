@@ -889,6 +889,23 @@ def test_assignments_grouped_by_expert(E, n):
     assert torch.equal(out[sel < E], few[sel < E])
 
 
+@pytest.mark.parametrize("n,E,K", [(769, 5, 70), (770, 16, 2048), (771, 24, 513), (772, 2048, 64), (770, 2049, 64)])
+@pytest.mark.parametrize("wdt", [torch.float32, torch.bfloat16])
+def test_router_of_four_rows_a_workgroup_has_the_bits_of_one(n, E, K, wdt):
+    """Row counts that leave one to four rows to the last workgroup, fewer and more experts than waves, the most and one more than that
+    share a workgroup's LDS; gates, a bias, a correction, both scores: against the same rows 250 at a time, one a workgroup."""
+    from vllm_omni_draft_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(n + E)
+    x = torch.randn(n, K, generator=g, device="cuda")
+    w, wg = (torch.randn(r, K, generator=g, device="cuda").to(wdt) for r in (E, 3))
+    c = torch.randn(E, generator=g, device="cuda")
+    calls = [lambda t: ops.moe_route_rows_gated(t, w, 2, "softmax", True, 1e-3, 1.5, wg), lambda t: ops.moe_route_rows_biased(t, w, c, 3),
+             lambda t: ops.moe_route_rows_corrected(t, w, c, 2, "sigmoid")]
+    for f in calls:
+        for got, few in zip(f(x), zip(*[f(x[i:i + 250]) for i in range(0, n, 250)])):
+            assert torch.equal(got, torch.cat(few))
+
+
 @pytest.mark.parametrize("E,F,W,n", [(4, 96, 160, 100), (3, 64, 128, 63), (2, 160, 96, 300), (5, 320, 64, 200)])
 @pytest.mark.parametrize("act,scale_input", [("silu", True), ("silu", False), ("relu2", False)])
 def test_moe_experts_of_many_rows_have_the_bits_of_few(E, F, W, n, act, scale_input):

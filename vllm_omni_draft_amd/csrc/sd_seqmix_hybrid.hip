@@ -1198,9 +1198,10 @@ __global__ void moe_route_kernel(const float* __restrict__ logits, int64_t ld, i
 // (lanes stride over the row's channels, then a butterfly sum: an order that no other row
 // changes), then the first wave chooses as moe_route_kernel does; with a correction [E] the choice is
 // made by score + correction, the weight is the score.
+// ROWS: rows of a workgroup, whose waves read an expert's weights once for all of them and then choose a row each.
 // POST: the residual update that the row comes out of first (postnorm_row), the row then from LDS; a wave asks for its first expert's
 // weights before that.
-template <typename T, bool POST>
+template <typename T, bool POST, int ROWS = 1>
 __global__ __launch_bounds__(1024) void moe_route_rows_kernel(const float* __restrict__ x, int64_t ldx,
                                                              const T* __restrict__ w, float* __restrict__ logits,
                                                              int32_t* __restrict__ sel_e, float* __restrict__ sel_w,
@@ -1209,10 +1210,14 @@ __global__ __launch_bounds__(1024) void moe_route_rows_kernel(const float* __res
                                                              const T* __restrict__ w_gate, int n_gate,
                                                              float* __restrict__ gate_out,
                                                              const float* __restrict__ bias,
-                                                             const float* __restrict__ correction, PostNorm<T> post) {
-  extern __shared__ float sc[];   // [E] (POST: and the row [K])
-  const int r = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nw = blockDim.x >> 6;
-  const float* xr = POST ? sc + E : x + (size_t)r * ldx;
+                                                             const float* __restrict__ correction, PostNorm<T> post,
+                                                             int n_rows) {
+  extern __shared__ float scores[];   // [ROWS][E] (POST: and the row [K])
+  static_assert(!POST || ROWS == 1, "one row in LDS");
+  const int r0 = blockIdx.x * ROWS, wave = threadIdx.x >> 6, lane = threadIdx.x & 63, nw = blockDim.x >> 6;
+  const float* xr[ROWS];
+#pragma unroll
+  for (int j = 0; j < ROWS; ++j) xr[j] = POST ? scores + E : x + (size_t)min(r0 + j, n_rows - 1) * ldx;
   constexpr int kU = 8;   // loads of a lane in flight
   constexpr int kFirst = POST ? 4 : 1;   // batches of the first expert's weights asked for ahead
   T ahead[kFirst][kU];
@@ -1222,13 +1227,15 @@ __global__ __launch_bounds__(1024) void moe_route_rows_kernel(const float* __res
     for (int i = 0; i < kFirst; ++i)
 #pragma unroll
       for (int u = 0; u < kU; ++u) ahead[i][u] = wr[min((i * kU + u) * 64 + lane, K - 1)];
-    postnorm_row(post, r, [&](int c, float v) { sc[E + c] = v; });
+    postnorm_row(post, r0, [&](int c, float v) { scores[E + c] = v; });
     __syncthreads();
   }
   // (rows E .. E + n_gate - 1 are further products of the same input: gates computed as the router is)
   for (int e = wave; e < E + n_gate; e += nw) {
     const T* wr = e < E ? w + (size_t)e * K : w_gate + (size_t)(e - E) * K;
-    float acc = 0.f;
+    float acc[ROWS];
+#pragma unroll
+    for (int j = 0; j < ROWS; ++j) acc[j] = 0.f;
     int from = 0;
     if constexpr (POST)
       if (e == wave && e < E) {
@@ -1237,35 +1244,43 @@ __global__ __launch_bounds__(1024) void moe_route_rows_kernel(const float* __res
 #pragma unroll
           for (int u = 0; u < kU; ++u) {
             const int k = (i * kU + u) * 64 + lane;
-            if (k < K) acc = fmaf(maybe_round(xr[k], round), (float)ahead[i][u], acc);
+            if (k < K) acc[0] = fmaf(maybe_round(xr[0][k], round), (float)ahead[i][u], acc[0]);
           }
         from = kFirst * kU * 64;
       }
     for (int k0 = from; k0 < K; k0 += 64 * kU) {
-      float xv[kU], wv[kU];
+      float xv[ROWS][kU], wv[kU];
 #pragma unroll
       for (int u = 0; u < kU; ++u) {   // unguarded, on an index clamped into the row
         const int k = k0 + 64 * u + lane < K ? k0 + 64 * u + lane : K - 1;
-        xv[u] = xr[k];
+#pragma unroll
+        for (int j = 0; j < ROWS; ++j) xv[j][u] = xr[j][k];
         wv[u] = ld_f(wr + k);
       }
 #pragma unroll
       for (int u = 0; u < kU; ++u)
-        if (k0 + 64 * u + lane < K) acc = fmaf(maybe_round(xv[u], round), wv[u], acc);
+        if (k0 + 64 * u + lane < K)
+#pragma unroll
+          for (int j = 0; j < ROWS; ++j) acc[j] = fmaf(maybe_round(xv[j][u], round), wv[u], acc[j]);
     }
-    acc = wave_sum(acc);
-    if (lane == 0) {
-      if (e < E) {
-        if (bias) acc += bias[e];
-        sc[e] = acc;
-        if (logits) logits[(size_t)r * E + e] = acc;
-      } else {
-        gate_out[(size_t)r * n_gate + e - E] = acc;
+#pragma unroll
+    for (int j = 0; j < ROWS; ++j) {
+      float z = wave_sum(acc[j]);
+      if (lane == 0 && r0 + j < n_rows) {
+        if (e < E) {
+          if (bias) z += bias[e];
+          scores[j * E + e] = z;
+          if (logits) logits[(size_t)(r0 + j) * E + e] = z;
+        } else {
+          gate_out[(size_t)(r0 + j) * n_gate + e - E] = z;
+        }
       }
     }
   }
   __syncthreads();
-  if (wave != 0) return;
+  const int r = r0 + wave;   // a wave a row from here on
+  if (wave >= ROWS || r >= n_rows) return;
+  float* sc = scores + wave * E;
   if (score_kind == 0) {
     for (int e = lane; e < E; e += 64) sc[e] = sigmoid_f(sc[e]);
   } else {
@@ -2624,14 +2639,21 @@ extern "C" int sd_moe_route_rows_corrected(const float* x, int64_t ldx, const vo
   SD_REQUIRE(E <= 8192, SD_ERR_UNSUPPORTED, "sd_moe_route_rows: more than 8192 experts");
   hipStream_t st = (hipStream_t)stream;
   const int nthr = 64 * (E >= 16 ? 16 : (E >= 8 ? 8 : 4));   // a wave per expert, up to 16 at a time
-  if (w_f32)
-    moe_route_rows_kernel<float, false><<<n_rows, nthr, sizeof(float) * E, st>>>(
-        x, ldx, (const float*)w_router, logits, sel_expert, sel_weight, E, K, top, score_kind, renorm, 0, renorm_eps,
-        weight_scale, (const float*)w_gate, n_gate, gate_out, router_bias, correction, PostNorm<float>{});
-  else
-    moe_route_rows_kernel<bf16_t, false><<<n_rows, nthr, sizeof(float) * E, st>>>(
-        x, ldx, (const bf16_t*)w_router, logits, sel_expert, sel_weight, E, K, top, score_kind, renorm, 1, renorm_eps,
-        weight_scale, (const bf16_t*)w_gate, n_gate, gate_out, router_bias, correction, PostNorm<bf16_t>{});
+  auto go = [&](auto* w, auto rows) {
+    using T = std::remove_const_t<std::remove_pointer_t<decltype(w)>>;
+    constexpr int ROWS = decltype(rows)::value;
+    moe_route_rows_kernel<T, false, ROWS><<<(n_rows + ROWS - 1) / ROWS, nthr, sizeof(float) * ROWS * E, st>>>(
+        x, ldx, w, logits, sel_expert, sel_weight, E, K, top, score_kind, renorm, !w_f32, renorm_eps, weight_scale, (const T*)w_gate, n_gate,
+        gate_out, router_bias, correction, PostNorm<T>{}, n_rows);
+  };
+  // Four rows a workgroup once one row each is more than a round of them (two a CU, with 16 waves each).  us, one / four: 16 experts, 2048 columns
+  // 512 rows 10.6 / 12.2, 700 13.8 / 12.2, 1024 17.1 / 12.6, 2048 29.2 / 21.5; 64 experts 512 29.9 / 35.5, 1024 49.6 / 36.0, 2048 92.9 / 68.2; 8
+  // experts, 1024 columns 700 6.7 / 7.0, 1024 7.8 / 7.1, 2048 11.2 / 8.8.
+  const bool four = n_rows > 768 && E <= 2048;
+  if (w_f32 && four) go((const float*)w_router, std::integral_constant<int, 4>{});
+  else if (w_f32) go((const float*)w_router, std::integral_constant<int, 1>{});
+  else if (four) go((const bf16_t*)w_router, std::integral_constant<int, 4>{});
+  else go((const bf16_t*)w_router, std::integral_constant<int, 1>{});
   SD_CHECK_LAUNCH("sd_moe_route_rows");
   return SD_OK;
 }
@@ -2805,7 +2827,7 @@ int sd_postnorm_route_(float* x, const float* a, float sa, const float* b, float
     using T = std::remove_const_t<std::remove_pointer_t<decltype(nw)>>;
     moe_route_rows_kernel<T, true><<<n_rows, 1024, lds, st>>>(x, W, rw, logits, sel_expert, sel_weight, E, W, top, 0, 0, !w_f32, 0.f, 1.f,
                                                                (const T*)nullptr, 0, nullptr, nullptr, nullptr,
-                                                               PostNorm<T>{x, a, 1, sa, b, sb, nw, eps, (bf16_t*)x_bf16, W});
+                                                               PostNorm<T>{x, a, 1, sa, b, sb, nw, eps, (bf16_t*)x_bf16, W}, n_rows);
   };
   if (w_f32) go((const float*)norm_w, (const float*)w_router);
   else go((const bf16_t*)norm_w, (const bf16_t*)w_router);

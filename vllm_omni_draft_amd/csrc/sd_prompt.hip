@@ -658,7 +658,8 @@ int few_shape(const PromptArgs& a, hipStream_t st) {
 // The block of a prompt pass: the shape whose time by this model is the least.  The blocks go over the chip in rounds of 256 x
 // per_cu; a round takes `fixed` us (launch, first loads, epilogue), `split` us a split of K (its sums join the others')
 // and `stage` us a stage of 64 columns, which depends on how many blocks share a CU.  Fitted to 342 measured passes
-// (N 512..18944, K 512..18944, 272..4096 rows, weights from memory; 6-9 % off at the root of the mean square): the shapes it takes
+// (N 512..18944, K 512..18944, 272..4096 rows, weights from memory, epilogues through LDS, which took 2 to 8 us a block longer than those from
+// registers; 6-9 % off at the root of the mean square): the shapes it takes
 // are 1 % slower than the best of all there, 24 % faster than one block shape of 128 x 128 (whole K: 8 %).  Both sides
 // where it matters most, us, chosen shape against 128 x 128: 1024 x 2048 at 1024 rows 12.6 (64 x 64) and 25.6; 4096 x 4096
 // at 512 rows 29.3 (64 x 128) and 42.1; 6144 x 4096 at 1024 rows 63.3 (128 x 256) and 70.4; 3584 x 18944 at 2946 rows 354

@@ -906,6 +906,30 @@ def test_router_of_four_rows_a_workgroup_has_the_bits_of_one(n, E, K, wdt):
             assert torch.equal(got, torch.cat(few))
 
 
+@pytest.mark.parametrize("lens,C", [([1, 2, 3, 5, 100, 4, 13], 300), ([127, 1], 257), ([126, 3], 64), ([1] * 130, 40)])
+@pytest.mark.parametrize("wdt,bias", [(torch.float32, True), (torch.bfloat16, False)])
+def test_four_rows_a_thread_of_a_convolution_have_the_bits_of_one(lens, C, wdt, bias):
+    """128 rows and more (four taps): portions that begin and end inside a thread's four rows, shorter than the taps, alone in it, with the
+    inputs kept before them and without, and a last thread of one to four rows; against every portion by itself, outputs and kept inputs."""
+    from vllm_omni_draft_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(sum(lens) + C)
+    n, E = sum(lens), len(lens)
+    x, w = torch.randn(n, C, generator=g, device="cuda"), torch.randn(C, 4, generator=g, device="cuda").to(wdt)
+    b = torch.randn(C, generator=g, device="cuda").to(wdt) if bias else None
+    start = [(0, 7, 1, 2)[e % 4] for e in range(E)]
+    kept = torch.randn(E, 3, C, generator=g, device="cuda")
+    pos = [start[e] + i for e in range(E) for i in range(lens[e])]
+    slot = [e for e in range(E) for _ in range(lens[e])]
+    rows = [sum(lens[:e]) for e in range(E)]
+    one, all_ = kept.clone(), kept.clone()
+    got = ops.causal_conv_rows(x, w, b, all_, i32(pos), i32(slot), i32([[e, rows[e], lens[e], start[e]] for e in range(E)]))
+    for e in range(E):
+        s = slice(rows[e], rows[e] + lens[e])
+        alone = ops.causal_conv_rows(x[s].contiguous(), w, b, one, i32(pos[s]), i32(slot[s]), i32([[e, 0, lens[e], start[e]]]))
+        assert torch.equal(got[s], alone), e
+    assert torch.equal(all_, one)
+
+
 @pytest.mark.parametrize("E,F,W,n", [(4, 96, 160, 100), (3, 64, 128, 63), (2, 160, 96, 300), (5, 320, 64, 200)])
 @pytest.mark.parametrize("act,scale_input", [("silu", True), ("silu", False), ("relu2", False)])
 def test_moe_experts_of_many_rows_have_the_bits_of_few(E, F, W, n, act, scale_input):

@@ -107,8 +107,10 @@ __device__ __forceinline__ bool whole_tiles(const WideEpiArgs& a, int tile0, int
   return tile0 + tiles <= n_tiles && (tile0 + tiles) * cols <= a.N && ((a.ldo | a.N) & 3) == 0;
 }
 
+// EPI_RELU_PAIR: the tiles that exist, of n_tiles in all (their widths are whole tiles: there is no other epilogue for this one).  Other epilogues: all of
+// the wave's tiles exist.
 template <int EPI, int TN, int TM>
-__device__ __forceinline__ void emit_tiles(const PromptArgs& p, f32x4 (&acc)[TN][TM], int tile0, int row0, int lane) {
+__device__ __forceinline__ void emit_tiles(const PromptArgs& p, f32x4 (&acc)[TN][TM], int tile0, int n_tiles, int row0, int lane) {
   const WideEpiArgs& a = p.epi;
   const int xc = lane & 15, xq = lane >> 4;
   if constexpr (EPI == SD_EPI_SILU_MUL) {
@@ -127,16 +129,19 @@ __device__ __forceinline__ void emit_tiles(const PromptArgs& p, f32x4 (&acc)[TN]
   } else if constexpr (EPI == EPI_RELU_PAIR) {
     bf16_t* out = reinterpret_cast<bf16_t*>(a.out) + (size_t)(row0 + xc) * a.ldo + tile0 * 16 + xq * 4;
 #pragma unroll
-    for (int j = 0; j < TM; ++j)
+    for (int j = 0; j < TM; ++j) {
+      in_turn(acc, j);
       if (row0 + 16 * j + xc < p.M) {
 #pragma unroll
         for (int i = 0; i < TN / 2; ++i) {
+          if (tile0 + i >= n_tiles) break;
           bf16x4 r;
 #pragma unroll
           for (int e = 0; e < 4; ++e) r[e] = (bf16_t)(fmaxf(acc[i][j][e], 0.f) * acc[i + TN / 2][j][e]);
           *reinterpret_cast<bf16x4*>(out + (size_t)16 * j * a.ldo + i * 16) = r;
         }
       }
+    }
   } else if constexpr (EPI == SD_EPI_F32) {
     const int64_t ld = a.ldo;
     float* out = reinterpret_cast<float*>(a.out) + tile0 * 16 + xq * 4;
@@ -240,94 +245,100 @@ __device__ __forceinline__ bf16x4 turn_quad(const bf16x4& v, int lane) {
 // A wave's tiles of a QKV product: queries and keys rotated, keys and values into their pages.  A key's eight channels of a
 // page are 16 bytes, next to the next token's; a page row of a value's channel holds its tokens side by side, so four tokens of
 // a channel go in one store where they lie at neighbouring positions from a multiple of four on (others one by one).
+// 8 x 8 tiles go four of tokens at a time (all eight's cosines and sines beside the accumulators: 19 registers a lane were spilled).
 template <int TN, int TM>
 __device__ __forceinline__ void emit_heads(const PromptArgs& p, f32x4 (&acc)[TN][TM], int tile0, int row0, int lane) {
   const WideEpiArgs& a = p.epi;
   const WideRope& rp = a.rope;
   const int xc = lane & 15, xq = lane >> 4, D = rp.D, half = D / 2, tph = D / 16;
-  int pos[TM], page[TM], turn[TM];   // position (-1: no such row), page, row of the cosines
+  constexpr int kBatch = TN * TM > 32 && TM % 4 == 0 ? 4 : TM;
 #pragma unroll
-  for (int j = 0; j < TM; ++j) {
-    const int m = row0 + 16 * j + xc, b = qkv_sequence(rp, min(m, p.M - 1));
-    pos[j] = m < p.M ? qkv_position(rp, m, b) : -1;
-    turn[j] = min(max(sd_rope_position(rp.mp, pos[j], b, m, 0), 0), rp.max_pos - 1);
-  }
-  if ((tile0 + TN - 1) / tph >= rp.Hq) {
+  for (int j0 = 0; j0 < TM; j0 += kBatch) {
+    int pos[kBatch], page[kBatch], turn[kBatch];   // position (-1: no such row), page, row of the cosines
 #pragma unroll
-    for (int j = 0; j < TM; ++j) page[j] = pos[j] >= 0 ? qkv_page(rp, qkv_sequence(rp, row0 + 16 * j + xc), pos[j]) : 0;
-  }
-#pragma unroll
-  for (int i = 0; i < TN; i += 2) {
-    if constexpr (TN * TM > 32) {   // (as in_turn)
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int j = 0; j < TM; ++j) {
-        asm volatile("" : "+a"(acc[i][j]));
-        asm volatile("" : "+a"(acc[i + 1][j]));
-      }
+    for (int j = 0; j < kBatch; ++j) {
+      const int m = row0 + 16 * (j0 + j) + xc, b = qkv_sequence(rp, min(m, p.M - 1));
+      pos[j] = m < p.M ? qkv_position(rp, m, b) : -1;
+      turn[j] = min(max(sd_rope_position(rp.mp, pos[j], b, m, 0), 0), rp.max_pos - 1);
     }
-    const int head = (tile0 + i) / tph, in_head = (tile0 + i - head * tph) * 8;
-    if (head >= rp.Hq + rp.Hkv) {
-      bf16_t* vp = rp.vc + (size_t)(head - rp.Hq - rp.Hkv) * D * 16;
+    if ((tile0 + TN - 1) / tph >= rp.Hq) {
 #pragma unroll
-      for (int e = 0; e < 2; ++e) {
-        const int i0 = in_head + 8 * e + (xq & 1) * 4 + (xq >> 1) * half;   // channel of acc[..][0]
-        f32x4 bias = {0.f, 0.f, 0.f, 0.f};
-        if (a.bias)
+      for (int j = 0; j < kBatch; ++j) page[j] = pos[j] >= 0 ? qkv_page(rp, qkv_sequence(rp, row0 + 16 * (j0 + j) + xc), pos[j]) : 0;
+    }
 #pragma unroll
-          for (int c = 0; c < 4; ++c) bias[c] = (float)a.bias[head * D + i0 + c];
+    for (int i = 0; i < TN; i += 2) {
+      if constexpr (TN * TM > 32) {   // (as in_turn)
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int j = 0; j < TM; ++j) {
-          bf16x4 v;
-#pragma unroll
-          for (int c = 0; c < 4; ++c) v[c] = (bf16_t)(a.bias ? acc[i + e][j][c] + bias[c] : acc[i + e][j][c]);
-          const int p0 = __builtin_amdgcn_mov_dpp(pos[j], 0, 0xf, 0xf, true), g0 = __builtin_amdgcn_mov_dpp(page[j], 0, 0xf, 0xf, true);
-          const unsigned long long ok = __ballot(pos[j] >= 0 && (p0 & 3) == 0 && pos[j] == p0 + (lane & 3) && page[j] == g0);
-          const bf16x4 t = turn_quad(v, lane);
-          bf16_t* to = vp + (size_t)page[j] * rp.Hkv * D * 16;
-          if ((ok >> (lane & 60) & 15) == 15) {
-            *reinterpret_cast<bf16x4*>(to + (i0 + (lane & 3)) * 16 + sd_v_slot(p0 & 15)) = t;
-          } else if (pos[j] >= 0) {
-#pragma unroll
-            for (int c = 0; c < 4; ++c) to[(i0 + c) * 16 + sd_v_slot(pos[j] & 15)] = v[c];
-          }
+        for (int j = j0; j < j0 + kBatch; ++j) {
+          asm volatile("" : "+a"(acc[i][j]));
+          asm volatile("" : "+a"(acc[i + 1][j]));
         }
       }
-      continue;
-    }
-    const int i0 = in_head + (xq >> 1) * 8 + (xq & 1) * 4;   // channel of the even halves' first sum
-    f32x4 b_lo = {0.f, 0.f, 0.f, 0.f}, b_hi = b_lo;
-    if (a.bias)
+      const int head = (tile0 + i) / tph, in_head = (tile0 + i - head * tph) * 8;
+      if (head >= rp.Hq + rp.Hkv) {
+        bf16_t* vp = rp.vc + (size_t)(head - rp.Hq - rp.Hkv) * D * 16;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        b_lo[c] = (float)a.bias[head * D + i0 + c];
-        b_hi[c] = (float)a.bias[head * D + i0 + half + c];
+        for (int e = 0; e < 2; ++e) {
+          const int i0 = in_head + 8 * e + (xq & 1) * 4 + (xq >> 1) * half;   // channel of acc[..][0]
+          f32x4 bias = {0.f, 0.f, 0.f, 0.f};
+          if (a.bias)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) bias[c] = (float)a.bias[head * D + i0 + c];
+#pragma unroll
+          for (int j = 0; j < kBatch; ++j) {
+            const f32x4& y = acc[i + e][j0 + j];
+            bf16x4 v;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) v[c] = (bf16_t)(a.bias ? y[c] + bias[c] : y[c]);
+            const int p0 = __builtin_amdgcn_mov_dpp(pos[j], 0, 0xf, 0xf, true), g0 = __builtin_amdgcn_mov_dpp(page[j], 0, 0xf, 0xf, true);
+            const unsigned long long ok = __ballot(pos[j] >= 0 && (p0 & 3) == 0 && pos[j] == p0 + (lane & 3) && page[j] == g0);
+            const bf16x4 t = turn_quad(v, lane);
+            bf16_t* to = vp + (size_t)page[j] * rp.Hkv * D * 16;
+            if ((ok >> (lane & 60) & 15) == 15) {
+              *reinterpret_cast<bf16x4*>(to + (i0 + (lane & 3)) * 16 + sd_v_slot(p0 & 15)) = t;
+            } else if (pos[j] >= 0) {
+#pragma unroll
+              for (int c = 0; c < 4; ++c) to[(i0 + c) * 16 + sd_v_slot(pos[j] & 15)] = v[c];
+            }
+          }
+        }
+        continue;
       }
-    f32x4 cs[TM], sn[TM];
+      const int i0 = in_head + (xq >> 1) * 8 + (xq & 1) * 4;   // channel of the even halves' first sum
+      f32x4 b_lo = {0.f, 0.f, 0.f, 0.f}, b_hi = b_lo;
+      if (a.bias)
 #pragma unroll
-    for (int j = 0; j < TM; ++j) {
-      cs[j] = *reinterpret_cast<const f32x4*>(rp.cs + (size_t)turn[j] * D + i0);
-      sn[j] = *reinterpret_cast<const f32x4*>(rp.cs + (size_t)turn[j] * D + i0 + half);
-    }
+        for (int c = 0; c < 4; ++c) {
+          b_lo[c] = (float)a.bias[head * D + i0 + c];
+          b_hi[c] = (float)a.bias[head * D + i0 + half + c];
+        }
+      f32x4 cs[kBatch], sn[kBatch];
 #pragma unroll
-    for (int j = 0; j < TM; ++j) {
-      const TileSums s = split_halves(acc[i][j], acc[i + 1][j]);
-      bf16x4 l, h;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const float lo = round_bf16(a.bias ? s.lo[c] + b_lo[c] : s.lo[c]), hi = round_bf16(a.bias ? s.hi[c] + b_hi[c] : s.hi[c]);
-        l[c] = (bf16_t)(lo * cs[j][c] - hi * sn[j][c]);
-        h[c] = (bf16_t)(hi * cs[j][c] + lo * sn[j][c]);
+      for (int j = 0; j < kBatch; ++j) {
+        cs[j] = *reinterpret_cast<const f32x4*>(rp.cs + (size_t)turn[j] * D + i0);
+        sn[j] = *reinterpret_cast<const f32x4*>(rp.cs + (size_t)turn[j] * D + i0 + half);
       }
-      if (pos[j] < 0) {
-      } else if (head < rp.Hq) {
-        bf16_t* q = reinterpret_cast<bf16_t*>(a.out) + (size_t)(row0 + 16 * j + xc) * a.ldo + head * D + i0;
-        *reinterpret_cast<bf16x4*>(q) = l;
-        *reinterpret_cast<bf16x4*>(q + half) = h;
-      } else {
-        bf16_t* k = rp.kc + ((size_t)page[j] * rp.Hkv + (head - rp.Hq)) * D * 16 + (pos[j] & 15) * 8 + (i0 & 7);
-        *reinterpret_cast<bf16x4*>(k + (i0 >> 3) * 128) = l;
-        *reinterpret_cast<bf16x4*>(k + ((i0 + half) >> 3) * 128) = h;
+#pragma unroll
+      for (int j = 0; j < kBatch; ++j) {
+        const TileSums s = split_halves(acc[i][j0 + j], acc[i + 1][j0 + j]);
+        bf16x4 l, h;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const float lo = round_bf16(a.bias ? s.lo[c] + b_lo[c] : s.lo[c]), hi = round_bf16(a.bias ? s.hi[c] + b_hi[c] : s.hi[c]);
+          l[c] = (bf16_t)(lo * cs[j][c] - hi * sn[j][c]);
+          h[c] = (bf16_t)(hi * cs[j][c] + lo * sn[j][c]);
+        }
+        if (pos[j] < 0) {
+        } else if (head < rp.Hq) {
+          bf16_t* q = reinterpret_cast<bf16_t*>(a.out) + (size_t)(row0 + 16 * (j0 + j) + xc) * a.ldo + head * D + i0;
+          *reinterpret_cast<bf16x4*>(q) = l;
+          *reinterpret_cast<bf16x4*>(q + half) = h;
+        } else {
+          bf16_t* k = rp.kc + ((size_t)page[j] * rp.Hkv + (head - rp.Hq)) * D * 16 + (pos[j] & 15) * 8 + (i0 & 7);
+          *reinterpret_cast<bf16x4*>(k + (i0 >> 3) * 128) = l;
+          *reinterpret_cast<bf16x4*>(k + ((i0 + half) >> 3) * 128) = h;
+        }
       }
     }
   }
@@ -562,11 +573,13 @@ __global__ __launch_bounds__(256, blocks_per_cu(TN, TM, STAGES, SPLIT)) void pro
 #pragma unroll
       for (int j = 0; j < TM; ++j) acc[i][j] = tot[i][j] + acc[i][j];
   }
-  if constexpr (EPI != EPI_QKV_ROPE && EPI != EPI_PARTIAL) {
-    constexpr int kTiles = PAIR ? TN / 2 : TN, kCols = EPI == SD_EPI_SILU_MUL ? 8 : 16;
-    const int first = tile0 + wn * kTiles, tiles = PAIR ? a.n_tiles / 2 : a.n_tiles;
-    if (whole_tiles(a.epi, first, kTiles, tiles, kCols) && !(EPI == SD_EPI_SILU_MUL && a.epi.bias)) {
-      emit_tiles<EPI, TN, TM>(a, acc, first, row0 + wm * TM * 16, lane);
+  if constexpr (PAIR) {
+    emit_tiles<EPI, TN, TM>(a, acc, tile0 + wn * (TN / 2), a.n_tiles / 2, row0 + wm * TM * 16, lane);
+    return;
+  } else if constexpr (EPI != EPI_QKV_ROPE && EPI != EPI_PARTIAL) {
+    const int first = tile0 + wn * TN;
+    if (whole_tiles(a.epi, first, TN, a.n_tiles, EPI == SD_EPI_SILU_MUL ? 8 : 16) && !(EPI == SD_EPI_SILU_MUL && a.epi.bias)) {
+      emit_tiles<EPI, TN, TM>(a, acc, first, a.n_tiles, row0 + wm * TM * 16, lane);
       return;
     }
   }
@@ -582,20 +595,14 @@ __global__ __launch_bounds__(256, blocks_per_cu(TN, TM, STAGES, SPLIT)) void pro
   // neighbouring outputs of a row (and the epilogue is there once per token tile, not once per pair of tiles).
   constexpr bool PAIRED = EPI == SD_EPI_SILU_MUL || EPI == EPI_QKV_ROPE;
   constexpr int kLd = TN * 16 + 4;                        // floats; 16 rows start on different banks
-  constexpr int kUnits = PAIRED || PAIR ? TN * 2 : TN * 4;  // of a row; 64 lanes take 64 / kUnits rows at once
+  constexpr int kUnits = PAIRED ? TN * 2 : TN * 4;        // of a row; 64 lanes take 64 / kUnits rows at once
   float* img = reinterpret_cast<float*>(wave < 2 ? s0 : s1) + (wave & 1) * 16 * kLd;
   const int u = lane % kUnits, ui = PAIRED ? u >> 1 : u >> 2, r0 = PAIRED ? (u & 1) * 4 : (u & 3) * 4;
-  const int tile = tile0 + wn * (PAIR ? TN / 2 : TN) + ui;
+  const int tile = tile0 + wn * TN + ui;
 #pragma unroll
   for (int j = 0; j < TM; ++j) {
 #pragma unroll
-    for (int i = 0; i < (PAIR ? TN / 2 : TN); ++i) {
-      f32x4 y = acc[i][j];
-      if constexpr (PAIR)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) y[e] = fmaxf(y[e], 0.f) * acc[i + TN / 2][j][e];
-      *reinterpret_cast<f32x4*>(img + xc * kLd + i * 16 + 4 * xq) = y;
-    }
+    for (int i = 0; i < TN; ++i) *reinterpret_cast<f32x4*>(img + xc * kLd + i * 16 + 4 * xq) = acc[i][j];
     asm volatile("" ::: "memory");  // (other lanes read them: the stores of a lane without a unit stay here)
 #pragma unroll 1
     for (int r = lane < 64 / kUnits * kUnits ? lane / kUnits : 16; r < 16; r += 64 / kUnits) {
@@ -604,11 +611,8 @@ __global__ __launch_bounds__(256, blocks_per_cu(TN, TM, STAGES, SPLIT)) void pro
       const f32x4 lo = *reinterpret_cast<const f32x4*>(src);
       f32x4 hi = zero;
       if (PAIRED) hi = *reinterpret_cast<const f32x4*>(src + 8);
-      if (tile < (PAIR ? a.n_tiles / 2 : a.n_tiles) && m < a.M) {
-        if constexpr (PAIR)
-          *reinterpret_cast<bf16x4*>((bf16_t*)a.epi.out + (size_t)m * a.epi.ldo + tile * 16 + r0) =
-              bf16x4{(bf16_t)lo[0], (bf16_t)lo[1], (bf16_t)lo[2], (bf16_t)lo[3]};
-        else if constexpr (EPI == EPI_PARTIAL)
+      if (tile < a.n_tiles && m < a.M) {
+        if constexpr (EPI == EPI_PARTIAL)
           *reinterpret_cast<f32x4*>(a.part + ((size_t)split * a.M + m) * a.n_tiles * 16 + tile * 16 + r0) = lo;
         else emit_unit<EPI>(a.epi, m, tile, r0, lo, hi);
       }

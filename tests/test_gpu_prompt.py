@@ -1,5 +1,7 @@
 """Prompt passes: packed rows of several prompts through sd_model_prompt and its attention, against the passes of
 sd_model_forward, whose bits they must have."""
+import ctypes as C
+
 import pytest
 import torch
 
@@ -281,3 +283,113 @@ def test_prompts_on_either_side_of_the_line_for_a_long_k(n):
         out = torch.empty(m, cfg.vocab, device="cuda")
         model.forward(_KvView(two, 0), t, 0, c, zero, c, 1, m, out, wide=True)
     assert torch.equal(got[0], out[-1]) and torch.equal(one.k, two.k) and torch.equal(one.v, two.v)
+
+
+class _RopePos(C.Structure):
+    _fields_ = [("pos", C.c_void_p), ("delta", C.c_void_p), ("s_t", C.c_int), ("s_th", C.c_int), ("rows", C.c_int)]
+
+
+class _Rope(C.Structure):
+    _fields_ = [("cs", C.c_void_p), ("max_pos", C.c_int), ("kc", C.c_void_p), ("vc", C.c_void_p), ("block_tables", C.c_void_p),
+                ("max_blocks", C.c_int), ("seq_lens", C.c_void_p), *[(n, C.c_int) for n in ("pos_offset", "q_len", "Hq", "Hkv", "D")],
+                ("mp", _RopePos), ("row_seq", C.c_void_p)]
+
+
+class _Epilogue(C.Structure):
+    """WideEpiArgs of sd_wide_epi.h."""
+    _fields_ = [("part", C.c_void_p), *[(n, C.c_int) for n in ("S", "M", "NR", "N")], ("w_scale", C.c_void_p), ("x_scale", C.c_void_p),
+                ("bias", C.c_void_p), ("residual", C.c_void_p), ("out", C.c_void_p), ("ldo", C.c_int64), ("rope", _Rope)]
+
+
+# block -> rows, query heads, key heads, head size, columns: the smallest of a search over sizes for which the modelled times choose it
+QKV_SHAPES = {442: (257, 1, 1, 64, 128), 461: (901, 128, 2, 128, 1024), 861: (389, 128, 2, 128, 1024),
+              881: (645, 320, 5, 64, 1024), 1223: (257, 1, 1, 64, 192), 1241: (777, 10, 5, 64, 2048), 1422: (777, 26, 2, 128, 192),
+              1431: (2053, 4, 2, 128, 2048), 1441: (1541, 14, 2, 128, 2048), 1442: (1541, 40, 1, 64, 192), 1451: (901, 75, 3, 64, 1024),
+              1461: (2053, 10, 5, 128, 2048), 1481: (3073, 8, 4, 128, 8192)}
+
+
+@pytest.mark.parametrize("shape", sorted(QKV_SHAPES))
+@pytest.mark.parametrize("turn", ["rotary", "unaligned", "none", "sections", "odd sections"])
+def test_queries_keys_and_values_of_every_block_shape(shape, turn):
+    """The QKV product of a prompt pass in every block that the modelled times can choose, rotated by the cache's positions (the table
+    off 16 bytes too), by three positions a row (sections of channels that begin at multiples of four, and that do not) or not at all,
+    with and without a bias: queries and caches as passes of 48 rows leave them, bit for bit.  Sequences start at every remainder of four,
+    rows of no position (-1) are left out, and the last block of rows is not full."""
+    from tests.gpu_util import internal
+    from vllm_omni_draft_amd import ops
+    M, Hq, Hkv, D, K = QKV_SHAPES[shape]
+    N = (Hq + 2 * Hkv) * D
+    assert internal("sd_prompt_shape_", C.c_int, *[C.c_int] * 5)(M, N // 16, N // 16, K, 100) == shape and M % 32
+    product = internal("sd_prompt_linear_", C.c_int, C.c_void_p, C.c_void_p, C.c_int64, *[C.c_int] * 4, C.POINTER(_Epilogue), C.c_void_p)
+    g = torch.Generator(device="cuda").manual_seed(shape)
+    W = ops.tile_weights((torch.randn(N, K, generator=g, device="cuda") * K ** -0.5).to(torch.bfloat16), ops.TILE_ROTARY, head_dim=D)
+    x = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+    lens, starts = [M - 103, 66, 1, 34, 2], [5, 0, 31, 2, 15]
+    pos = torch.cat([torch.arange(s, s + n) for s, n in zip(starts, lens)]).to(torch.int32)
+    pos[-3:-1] = -1
+    seq = torch.repeat_interleave(torch.arange(5), torch.tensor(lens)).to(torch.int32)
+    pages = (M + 40 + 15) // 16
+    tables = torch.randperm(5 * pages, generator=torch.Generator().manual_seed(shape)).to(torch.int32).view(5, pages).cuda()
+    pos, seq = pos.cuda(), seq.cuda()
+    table = torch.randn(M * D + 1, generator=g, device="cuda")
+    cs = None if turn == "none" else (table[1:] if turn == "unaligned" else table[:-1]).view(M, D)
+    section = {"sections": (D // 8, D * 3 // 16), "odd sections": (D // 8 + 1, D * 3 // 16 - 2)}.get(turn)
+    rope_pos = torch.randint(0, M + 50, (3, M), generator=g, device="cuda", dtype=torch.int32) if section else None
+    for bias in (None, torch.randn(N, generator=g, device="cuda").to(torch.bfloat16)):
+        p = lambda t: None if t is None else t.data_ptr()
+        new = lambda *s: torch.full(s, 7.0, dtype=torch.bfloat16, device="cuda")
+        q, kc, vc = new(M, Hq * D), new(5 * pages, Hkv, 16 * D), new(5 * pages, Hkv, 16 * D)
+        mp = _RopePos(p(rope_pos), None, *((section[0], sum(section)) if section else (0, 0)), M)
+        e = _Epilogue(None, 1, M, N, N, None, None, p(bias), None, p(q), Hq * D,
+                      _Rope(p(cs), M, p(kc), p(vc), p(tables), pages, p(pos), 0, 1, Hq, Hkv, D, mp, p(seq)))
+        assert product(W.data.data_ptr(), x.data_ptr(), K, M, K, N // 16, 100, C.byref(e), ops._stream()) == 0
+        few, k2, v2 = new(M, Hq * D), new(5 * pages, Hkv, 16 * D), new(5 * pages, Hkv, 16 * D)
+        for i in range(0, M, 48):
+            n = min(48, M - i)
+            few[i:i + n] = ops.qkv_rope_wide(W, x[i:i + n], bias, cs, k2, v2, tables[seq[i:i + n].long()].contiguous(), pos[i:i + n].contiguous(), 0, n, 1,
+                                             Hq, Hkv, D, rope_pos=None if section is None else rope_pos[:, i:i + n].contiguous(),
+                                             mrope_section=section)
+        live = pos >= 0
+        assert torch.equal(q[live], few[live]) and bool((q[~live] == 7.0).all())
+        assert torch.equal(kc, k2) and torch.equal(vc, v2)
+
+
+@pytest.mark.parametrize("turn", ["none", "sections"])
+def test_other_rotations_take_no_longer_than_the_plain_one(turn):
+    """The QKV product of a model without a rotary table, and of one with three positions a row, at a size whose epilogue weighs (2946 rows, 12 heads of
+    64, 768 columns): through LDS with positions looked up for every output they took 1.12 to 1.16 and 1.3 times the plain rotation's time, from
+    registers .91 and 1.01.  The best of ten replays in turn."""
+    from tests.gpu_util import internal
+    from vllm_omni_draft_amd import ops
+    M, H, D, K = 2946, 12, 64, 768
+    N, pages = 3 * H * D, (M + 15) // 16
+    product = internal("sd_prompt_linear_", C.c_int, C.c_void_p, C.c_void_p, C.c_int64, *[C.c_int] * 4, C.POINTER(_Epilogue), C.c_void_p)
+    W = ops.tile_weights((torch.randn(N, K, device="cuda") * K ** -0.5).to(torch.bfloat16), ops.TILE_ROTARY, head_dim=D)
+    x = torch.randn(M, K, device="cuda").to(torch.bfloat16)
+    q, kc, vc = (torch.empty(s, dtype=torch.bfloat16, device="cuda") for s in ((M, H * D), (pages, H, 16 * D), (pages, H, 16 * D)))
+    pos, tables = (torch.arange(n, dtype=torch.int32, device="cuda") for n in (M, pages))
+    cs = torch.randn(M, D, device="cuda")
+    seq, three = torch.zeros_like(pos), pos.repeat(3, 1).contiguous()
+    graphs = []
+    for kind in ("rotary", turn):
+        mp = _RopePos(three.data_ptr() if kind == "sections" else None, None, 8, 20, M)
+        e = _Epilogue(None, 1, M, N, N, None, None, None, None, q.data_ptr(), H * D,
+                      _Rope(None if kind == "none" else cs.data_ptr(), M, kc.data_ptr(), vc.data_ptr(), tables.data_ptr(), pages, pos.data_ptr(), 0, 1,
+                            H, H, D, mp, seq.data_ptr()))
+        go = lambda: product(W.data.data_ptr(), x.data_ptr(), K, M, K, N // 16, 100, C.byref(e), ops._stream())
+        assert go() == 0
+        torch.cuda.synchronize()
+        graphs.append(torch.cuda.CUDAGraph())
+        with torch.cuda.graph(graphs[-1]):
+            for _ in range(40):
+                assert go() == 0
+    best = [1e9, 1e9]
+    for _ in range(10):
+        for i, graph in enumerate(graphs):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            graph.replay()
+            b.record()
+            b.synchronize()
+            best[i] = min(best[i], a.elapsed_time(b))
+    assert best[1] < 1.1 * best[0], best

@@ -1230,7 +1230,7 @@ int sd_linear_rows_(const void* W, const float* w_scale, float* x_scales, const 
                     int n_tiles, int epi, const WideEpiArgs& all, void* workspace, size_t ws_bytes, sd_stream_t stream) {
   hipStream_t st = (hipStream_t)stream;
   const bool aligned = sd_aligned16(W) && sd_aligned16(x) && ldx % 8 == 0 && ldx >= K;
-  if (!w_scale && aligned && sd_prompt_linear_fits_(M, K, ldx))
+  if (!w_scale && aligned && sd_prompt_linear_fits_(M, K, ldx) && (epi != EPI_QKV_ROPE || sd_prompt_heads_fit_(all)))
     return sd_prompt_linear_(W, x, ldx, M, K, n_tiles, epi, all, stream);
   const size_t out_el = epi == SD_EPI_F32 ? 4 : 2;
   for (int r0 = 0; r0 < M; r0 += 256) {

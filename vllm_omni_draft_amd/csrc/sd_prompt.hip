@@ -216,15 +216,6 @@ __device__ __forceinline__ void emit_tiles(const PromptArgs& p, f32x4 (&acc)[TN]
   }
 }
 
-// Whether a wave's tiles of a QKV product can be stored from registers: pairs of tiles in one head, one position for all of a row, and
-// starts that four neighbours in one store allow.
-__device__ __forceinline__ bool whole_heads(const WideEpiArgs& a, int tile0, int tiles, int n_tiles) {
-  const WideRope& rp = a.rope;
-  const uintptr_t at = reinterpret_cast<uintptr_t>(a.out) | reinterpret_cast<uintptr_t>(rp.kc) | reinterpret_cast<uintptr_t>(rp.vc);
-  return tile0 + tiles <= n_tiles && rp.D % 32 == 0 && (tile0 & 1) == 0 && rp.cs && !rp.mp.pos && (a.ldo & 3) == 0 && (at & 7) == 0 &&
-         (reinterpret_cast<uintptr_t>(rp.cs) & 15) == 0;
-}
-
 // The four tokens of a quad's lanes and four channels, turned: lane b of the quad has channel b's four tokens.
 __device__ __forceinline__ bf16x4 turn_quad(const bf16x4& v, int lane) {
   typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
@@ -242,96 +233,137 @@ __device__ __forceinline__ bf16x4 turn_quad(const bf16x4& v, int lane) {
   return __builtin_bit_cast(bf16x4, r);
 }
 
-// A wave's tiles of a QKV product: queries and keys rotated, keys and values into their pages.  A key's eight channels of a
-// page are 16 bytes, next to the next token's; a page row of a value's channel holds its tokens side by side, so four tokens of
+// One position for four neighbouring channels of a row (sections of them begin at multiples of four), four cosines in one load
+__device__ __forceinline__ bool one_position_of_four(const WideRope& rp) {
+  return (reinterpret_cast<uintptr_t>(rp.cs) & 15) == 0 && (!rp.mp.pos || ((rp.mp.s_t | rp.mp.s_th) & 3) == 0);
+}
+
+// A wave's tiles of a QKV product (those of n_tiles that exist): queries and keys rotated, keys and values into their pages.  A key's eight
+// channels of a page are 16 bytes, next to the next token's; a page row of a value's channel holds its tokens side by side, so four tokens of
 // a channel go in one store where they lie at neighbouring positions from a multiple of four on (others one by one).
-// 8 x 8 tiles go four of tokens at a time (all eight's cosines and sines beside the accumulators: 19 registers a lane were spilled).
-template <int TN, int TM>
+// Two tiles of a head at a time: an even number of tiles a wave.
+// kBatch tiles of tokens from J0 on: 8 x 8 tiles go four at a time (all eight's cosines and sines beside the accumulators: 19 registers a
+// lane were spilled).
+constexpr int heads_batch(int tn, int tm) { return tn * tm > 32 && tm % 4 == 0 ? 4 : tm; }
+// PLAIN: all of the wave's tiles exist and one position turns four neighbouring channels, by cosines in one load (with the tests for the others
+// inside, 18432 x 2048 at 4096 rows 325 us for 307).
+template <int TN, int TM, bool PLAIN, int J0 = 0>
 __device__ __forceinline__ void emit_heads(const PromptArgs& p, f32x4 (&acc)[TN][TM], int tile0, int row0, int lane) {
   const WideEpiArgs& a = p.epi;
   const WideRope& rp = a.rope;
   const int xc = lane & 15, xq = lane >> 4, D = rp.D, half = D / 2, tph = D / 16;
-  constexpr int kBatch = TN * TM > 32 && TM % 4 == 0 ? 4 : TM;
+  static_assert(TN % 2 == 0, "two tiles of a head at a time");
+  constexpr int kBatch = heads_batch(TN, TM);
+  const bool fours = PLAIN || one_position_of_four(rp);
+  auto turn_of = [&](int at) { return min(max(at, 0), rp.max_pos - 1); };
+  int pos[kBatch], page[kBatch], turn[kBatch];   // position (-1: no such row), page, row of the cosines (without positions of their own)
+  auto row_of = [&](int j) { return min(row0 + 16 * (J0 + j) + xc, p.M - 1); };
 #pragma unroll
-  for (int j0 = 0; j0 < TM; j0 += kBatch) {
-    int pos[kBatch], page[kBatch], turn[kBatch];   // position (-1: no such row), page, row of the cosines
+  for (int j = 0; j < kBatch; ++j) {
+    const int m = row_of(j), b = qkv_sequence(rp, m);
+    pos[j] = row0 + 16 * (J0 + j) + xc < p.M ? qkv_position(rp, m, b) : -1;
+    turn[j] = !PLAIN && rp.mp.pos ? 0 : turn_of(sd_rope_position(rp.mp, pos[j], b, m, 0));
+  }
+  if ((tile0 + TN - 1) / tph >= rp.Hq) {
 #pragma unroll
-    for (int j = 0; j < kBatch; ++j) {
-      const int m = row0 + 16 * (j0 + j) + xc, b = qkv_sequence(rp, min(m, p.M - 1));
-      pos[j] = m < p.M ? qkv_position(rp, m, b) : -1;
-      turn[j] = min(max(sd_rope_position(rp.mp, pos[j], b, m, 0), 0), rp.max_pos - 1);
-    }
-    if ((tile0 + TN - 1) / tph >= rp.Hq) {
+    for (int j = 0; j < kBatch; ++j) page[j] = pos[j] >= 0 ? qkv_page(rp, qkv_sequence(rp, row_of(j)), pos[j]) : 0;
+  }
 #pragma unroll
-      for (int j = 0; j < kBatch; ++j) page[j] = pos[j] >= 0 ? qkv_page(rp, qkv_sequence(rp, row0 + 16 * (j0 + j) + xc), pos[j]) : 0;
-    }
+  for (int i = 0; i < TN; i += 2) {
+    if (!PLAIN && tile0 + i >= p.n_tiles) break;
+    if constexpr (TN * TM > 32) {   // (as in_turn)
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < TN; i += 2) {
-      if constexpr (TN * TM > 32) {   // (as in_turn)
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int j = j0; j < j0 + kBatch; ++j) {
-          asm volatile("" : "+a"(acc[i][j]));
-          asm volatile("" : "+a"(acc[i + 1][j]));
-        }
+      for (int j = J0; j < J0 + kBatch; ++j) {
+        asm volatile("" : "+a"(acc[i][j]));
+        asm volatile("" : "+a"(acc[i + 1][j]));
       }
-      const int head = (tile0 + i) / tph, in_head = (tile0 + i - head * tph) * 8;
-      if (head >= rp.Hq + rp.Hkv) {
-        bf16_t* vp = rp.vc + (size_t)(head - rp.Hq - rp.Hkv) * D * 16;
+    }
+    const int head = (tile0 + i) / tph, in_head = (tile0 + i - head * tph) * 8;
+    if (head >= rp.Hq + rp.Hkv) {
+      bf16_t* vp = rp.vc + (size_t)(head - rp.Hq - rp.Hkv) * D * 16;
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          const int i0 = in_head + 8 * e + (xq & 1) * 4 + (xq >> 1) * half;   // channel of acc[..][0]
-          f32x4 bias = {0.f, 0.f, 0.f, 0.f};
-          if (a.bias)
+      for (int e = 0; e < 2; ++e) {
+        const int i0 = in_head + 8 * e + (xq & 1) * 4 + (xq >> 1) * half;   // channel of acc[..][0]
+        f32x4 bias = {0.f, 0.f, 0.f, 0.f};
+        if (a.bias)
 #pragma unroll
-            for (int c = 0; c < 4; ++c) bias[c] = (float)a.bias[head * D + i0 + c];
+          for (int c = 0; c < 4; ++c) bias[c] = (float)a.bias[head * D + i0 + c];
 #pragma unroll
-          for (int j = 0; j < kBatch; ++j) {
-            const f32x4& y = acc[i + e][j0 + j];
-            bf16x4 v;
+        for (int j = 0; j < kBatch; ++j) {
+          const f32x4& y = acc[i + e][J0 + j];
+          bf16x4 v;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) v[c] = (bf16_t)(a.bias ? y[c] + bias[c] : y[c]);
-            const int p0 = __builtin_amdgcn_mov_dpp(pos[j], 0, 0xf, 0xf, true), g0 = __builtin_amdgcn_mov_dpp(page[j], 0, 0xf, 0xf, true);
-            const unsigned long long ok = __ballot(pos[j] >= 0 && (p0 & 3) == 0 && pos[j] == p0 + (lane & 3) && page[j] == g0);
-            const bf16x4 t = turn_quad(v, lane);
-            bf16_t* to = vp + (size_t)page[j] * rp.Hkv * D * 16;
-            if ((ok >> (lane & 60) & 15) == 15) {
-              *reinterpret_cast<bf16x4*>(to + (i0 + (lane & 3)) * 16 + sd_v_slot(p0 & 15)) = t;
-            } else if (pos[j] >= 0) {
+          for (int c = 0; c < 4; ++c) v[c] = (bf16_t)(a.bias ? y[c] + bias[c] : y[c]);
+          const int p0 = __builtin_amdgcn_mov_dpp(pos[j], 0, 0xf, 0xf, true), g0 = __builtin_amdgcn_mov_dpp(page[j], 0, 0xf, 0xf, true);
+          const unsigned long long ok = __ballot(pos[j] >= 0 && (p0 & 3) == 0 && pos[j] == p0 + (lane & 3) && page[j] == g0);
+          const bf16x4 t = turn_quad(v, lane);
+          bf16_t* to = vp + (size_t)page[j] * rp.Hkv * D * 16;
+          if ((ok >> (lane & 60) & 15) == 15) {
+            *reinterpret_cast<bf16x4*>(to + (i0 + (lane & 3)) * 16 + sd_v_slot(p0 & 15)) = t;
+          } else if (pos[j] >= 0) {
 #pragma unroll
-              for (int c = 0; c < 4; ++c) to[(i0 + c) * 16 + sd_v_slot(pos[j] & 15)] = v[c];
-            }
+            for (int c = 0; c < 4; ++c) to[(i0 + c) * 16 + sd_v_slot(pos[j] & 15)] = v[c];
           }
         }
-        continue;
       }
-      const int i0 = in_head + (xq >> 1) * 8 + (xq & 1) * 4;   // channel of the even halves' first sum
-      f32x4 b_lo = {0.f, 0.f, 0.f, 0.f}, b_hi = b_lo;
-      if (a.bias)
+      continue;
+    }
+    const int i0 = in_head + (xq >> 1) * 8 + (xq & 1) * 4;   // channel of the even halves' first sum
+    f32x4 b_lo = {0.f, 0.f, 0.f, 0.f}, b_hi = b_lo;
+    if (a.bias)
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          b_lo[c] = (float)a.bias[head * D + i0 + c];
-          b_hi[c] = (float)a.bias[head * D + i0 + half + c];
-        }
+      for (int c = 0; c < 4; ++c) {
+        b_lo[c] = (float)a.bias[head * D + i0 + c];
+        b_hi[c] = (float)a.bias[head * D + i0 + half + c];
+      }
+    auto put = [&](auto rotated) __attribute__((always_inline)) {
+      constexpr bool kRotated = decltype(rotated)::value;
       f32x4 cs[kBatch], sn[kBatch];
+      if constexpr (kRotated) {
+        int at[kBatch];
+        if (!PLAIN && rp.mp.pos) {
 #pragma unroll
-      for (int j = 0; j < kBatch; ++j) {
-        cs[j] = *reinterpret_cast<const f32x4*>(rp.cs + (size_t)turn[j] * D + i0);
-        sn[j] = *reinterpret_cast<const f32x4*>(rp.cs + (size_t)turn[j] * D + i0 + half);
+          for (int j = 0; j < kBatch; ++j) at[j] = turn_of(sd_rope_position(rp.mp, 0, 0, row_of(j), i0));
+        } else {
+#pragma unroll
+          for (int j = 0; j < kBatch; ++j) at[j] = turn[j];
+        }
+        if (fours) {
+#pragma unroll
+          for (int j = 0; j < kBatch; ++j) {
+            cs[j] = *reinterpret_cast<const f32x4*>(rp.cs + (size_t)at[j] * D + i0);
+            sn[j] = *reinterpret_cast<const f32x4*>(rp.cs + (size_t)at[j] * D + i0 + half);
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < kBatch; ++j)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+              const int to = rp.mp.pos && c ? turn_of(sd_rope_position(rp.mp, 0, 0, row_of(j), i0 + c)) : at[j];
+              cs[j][c] = rp.cs[(size_t)to * D + i0 + c];
+              sn[j][c] = rp.cs[(size_t)to * D + i0 + half + c];
+            }
+        }
       }
 #pragma unroll
       for (int j = 0; j < kBatch; ++j) {
-        const TileSums s = split_halves(acc[i][j0 + j], acc[i + 1][j0 + j]);
+        const TileSums s = split_halves(acc[i][J0 + j], acc[i + 1][J0 + j]);
         bf16x4 l, h;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
           const float lo = round_bf16(a.bias ? s.lo[c] + b_lo[c] : s.lo[c]), hi = round_bf16(a.bias ? s.hi[c] + b_hi[c] : s.hi[c]);
-          l[c] = (bf16_t)(lo * cs[j][c] - hi * sn[j][c]);
-          h[c] = (bf16_t)(hi * cs[j][c] + lo * sn[j][c]);
+          if constexpr (kRotated) {
+            l[c] = (bf16_t)(lo * cs[j][c] - hi * sn[j][c]);
+            h[c] = (bf16_t)(hi * cs[j][c] + lo * sn[j][c]);
+          } else {
+            l[c] = (bf16_t)lo;
+            h[c] = (bf16_t)hi;
+          }
         }
         if (pos[j] < 0) {
         } else if (head < rp.Hq) {
-          bf16_t* q = reinterpret_cast<bf16_t*>(a.out) + (size_t)(row0 + 16 * (j0 + j) + xc) * a.ldo + head * D + i0;
+          bf16_t* q = reinterpret_cast<bf16_t*>(a.out) + (size_t)(row0 + 16 * (J0 + j) + xc) * a.ldo + head * D + i0;
           *reinterpret_cast<bf16x4*>(q) = l;
           *reinterpret_cast<bf16x4*>(q + half) = h;
         } else {
@@ -340,8 +372,12 @@ __device__ __forceinline__ void emit_heads(const PromptArgs& p, f32x4 (&acc)[TN]
           *reinterpret_cast<bf16x4*>(k + ((i0 + half) >> 3) * 128) = h;
         }
       }
-    }
+    };
+    if constexpr (PLAIN) put(std::true_type{});
+    else if (rp.cs) put(std::true_type{});
+    else put(std::false_type{});
   }
+  if constexpr (J0 + kBatch < TM) emit_heads<TN, TM, PLAIN, J0 + kBatch>(p, acc, tile0, row0, lane);
 }
 
 // Blocks a CU has room for: LDS, and the registers of two sets of accumulators.
@@ -576,24 +612,23 @@ __global__ __launch_bounds__(256, blocks_per_cu(TN, TM, STAGES, SPLIT)) void pro
   if constexpr (PAIR) {
     emit_tiles<EPI, TN, TM>(a, acc, tile0 + wn * (TN / 2), a.n_tiles / 2, row0 + wm * TM * 16, lane);
     return;
-  } else if constexpr (EPI != EPI_QKV_ROPE && EPI != EPI_PARTIAL) {
+  } else if constexpr (EPI == EPI_QKV_ROPE) {
+    const int first = tile0 + wn * TN;
+    if (a.epi.rope.cs && !a.epi.rope.mp.pos && one_position_of_four(a.epi.rope) && first + TN <= a.n_tiles)
+      emit_heads<TN, TM, true>(a, acc, first, row0 + wm * TM * 16, lane);
+    else emit_heads<TN, TM, false>(a, acc, first, row0 + wm * TM * 16, lane);
+    return;
+  } else if constexpr (EPI != EPI_PARTIAL) {
     const int first = tile0 + wn * TN;
     if (whole_tiles(a.epi, first, TN, a.n_tiles, EPI == SD_EPI_SILU_MUL ? 8 : 16) && !(EPI == SD_EPI_SILU_MUL && a.epi.bias)) {
       emit_tiles<EPI, TN, TM>(a, acc, first, a.n_tiles, row0 + wm * TM * 16, lane);
       return;
     }
   }
-  constexpr bool QKV = EPI == EPI_QKV_ROPE;
-  if constexpr (QKV && TN % 2 == 0) {
-    if (whole_heads(a.epi, tile0 + wn * TN, TN, a.n_tiles)) {
-      emit_heads<TN, TM>(a, acc, tile0 + wn * TN, row0 + wm * TM * 16, lane);
-      return;
-    }
-  }
   // Other outputs, and the partial sums of splits (3584 x 3584 at 107 / 192 / 256 rows 15.9 / 19.8 / 23.2 us with their epilogue's launch, from
   // registers 16.3 / 20.6 / 23.9), through LDS, 16 token rows at a time and each wave for itself, so that the lanes of a store hold
   // neighbouring outputs of a row (and the epilogue is there once per token tile, not once per pair of tiles).
-  constexpr bool PAIRED = EPI == SD_EPI_SILU_MUL || EPI == EPI_QKV_ROPE;
+  constexpr bool PAIRED = EPI == SD_EPI_SILU_MUL;
   constexpr int kLd = TN * 16 + 4;                        // floats; 16 rows start on different banks
   constexpr int kUnits = PAIRED ? TN * 2 : TN * 4;        // of a row; 64 lanes take 64 / kUnits rows at once
   float* img = reinterpret_cast<float*>(wave < 2 ? s0 : s1) + (wave & 1) * 16 * kLd;
@@ -699,13 +734,15 @@ float shape_us(const Shape& s, int M, int n_tiles, int K, int S, int epi) {
   return us;
 }
 
-// (EPI_RELU_PAIR: gate and up tiles in one block, an even number of tiles a wave)
+// Shapes with an odd number of tiles a wave are not for the epilogues that take two at a time: gate and up (EPI_RELU_PAIR), and a head's
+// (18432 x 2048 with rotation at 700 / 2000 rows: 224 x 256 blocks through LDS 79 / 216 us, what is chosen without them 66 / 194).
+constexpr bool even_tiles(int epi) { return epi == EPI_RELU_PAIR || epi == EPI_QKV_ROPE; }
 template <int N>
 const Shape& best_shape(const Shape (&shapes)[N], int M, int n_tiles, int K, int S, int epi, float& us) {
   int best = 0;
   us = shape_us(shapes[0], M, n_tiles, K, S, epi);
   for (int i = 1; i < N; ++i) {
-    if (epi == EPI_RELU_PAIR && shapes[i].tn % 2) continue;
+    if (even_tiles(epi) && shapes[i].tn % 2) continue;
     const float t = shape_us(shapes[i], M, n_tiles, K, S, epi);
     if (t < us) us = t, best = i;
   }
@@ -723,7 +760,7 @@ int shape_number(int M, int n_tiles, int K, int S, int epi) {
 
 template <int EPI>
 int prompt_shape(const PromptArgs& a, int S, hipStream_t st) {
-  constexpr bool even = EPI == EPI_RELU_PAIR;
+  constexpr bool even = even_tiles(EPI);
   const int shape = shape_number(a.M, a.n_tiles, a.KS * 32, S, EPI);
   switch (shape) {
     case 881: return launch_prompt<8, 8, 2, false, EPI, 2>(a, st);
@@ -753,6 +790,12 @@ int sd_prompt_shape_(int M, int n_tiles, int all_tiles, int K, int epi) {
   int S, ksp, g;
   plan_split(all_tiles, K, S, ksp, g);
   return shape_number(M, n_tiles, K, S, epi) + (S > 1 ? 1000 : 0);
+}
+
+// What the QKV epilogue of this file takes: two tiles of a head at a time, four neighbours in a store.
+bool sd_prompt_heads_fit_(const WideEpiArgs& e) {
+  const uintptr_t at = reinterpret_cast<uintptr_t>(e.out) | reinterpret_cast<uintptr_t>(e.rope.kc) | reinterpret_cast<uintptr_t>(e.rope.vc);
+  return e.rope.D % 32 == 0 && (e.ldo & 3) == 0 && (at & 7) == 0;
 }
 
 bool sd_prompt_linear_fits_(int M, int K, int64_t ldx) {
@@ -810,6 +853,8 @@ int sd_rows_linear_(const void* W, const void* x, int64_t ldx, int M, int K, int
 int sd_prompt_linear_(const void* W, const void* x, int64_t ldx, int M, int K, int n_tiles, int epi,
                       const WideEpiArgs& epi_args, sd_stream_t stream) {
   SD_REQUIRE(!epi_args.w_scale && !epi_args.x_scale, SD_ERR_UNSUPPORTED, "sd_prompt_linear: fp8 weights or activations");
+  SD_REQUIRE(epi != EPI_QKV_ROPE || sd_prompt_heads_fit_(epi_args), SD_ERR_UNSUPPORTED, "sd_prompt_linear: heads of %d, or unaligned outputs",
+             epi_args.rope.D);
   int S, ksp, g;
   WideEpiArgs e = epi_args;
   e.M = M;

@@ -297,6 +297,7 @@ int sd_rows_linear_(const void* W, const void* x, int64_t ldx, int M, int K, int
                     const sd_wide::WideEpiArgs& epi_args, float* part, sd_stream_t stream);
 bool sd_rows_chain_fits_(int M, int n_tiles, int K, int64_t ldx, int S);  // (sd_prompt_linear_ takes these rows)
 bool sd_prompt_linear_fits_(int M, int K, int64_t ldx);
+bool sd_prompt_heads_fit_(const WideEpiArgs& e);  // (and EPI_QKV_ROPE's outputs)
 int sd_prompt_linear_(const void* W, const void* x, int64_t ldx, int M, int K, int n_tiles, int epi,
                       const WideEpiArgs& e, sd_stream_t stream);
 int sd_linear_wide_norm_(const void* W, const float* w_scale, const void* x, int64_t ldx, const void* bias, const void* residual,

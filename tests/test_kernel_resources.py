@@ -45,3 +45,12 @@ def test_no_product_of_a_prompt_keeps_registers_in_scratch():
     products = _named("18prompt_gemm_kernel")
     assert len(products) > 80
     assert {n: k[".vgpr_spill_count"] for n, k in products.items() if k[".vgpr_spill_count"] or k[".private_segment_fixed_size"]} == {}
+
+
+def test_two_workgroups_of_prompt_attention_share_a_cu():
+    """A workgroup's LDS is its two stages, its page table and, given at launch, 512 bytes a split for the splits' maxima: in splits of 128 keys
+    (template argument 1) two have room beside each other up to 11264 keys."""
+    split_maxima = 11264 // 128 * 512
+    for size in (64, 128):
+        (kernel,) = _named(f"18prompt_attn_kernelILi{size}ELi1E").values()
+        assert 2 * (kernel[".group_segment_fixed_size"] + split_maxima) <= 160 * 1024, size

@@ -15,12 +15,13 @@
 // added in order, then the splits, against the maximum over all splits.  A row thus has the bits that a decode pass
 // gives it, and the bits do not depend on how a prompt is cut.  The weights of chains and splits need the maxima of
 // everything first: a first sweep computes the scores for the maxima alone (a third of the matrix work), which costs
-// less than keeping the splits' sums.  It needs keys only and no order, so its stages are 128 keys, half the barriers of the second
-// sweep's, in which a stage is one chain of a split (tiles c and c + 4 of eight), so that only one chain's sums, a quarter of the
+// less than keeping the splits' sums.  It needs keys only and no order, so its stages are 128 keys (64: see kKeys), half the barriers of the
+// second sweep's, in which a stage is one chain of a split (tiles c and c + 4 of eight), so that only one chain's sums, a quarter of the
 // channels at a time, are live beside the split's and the row's.
 // What bounds it: products and vector work of a wave follow each other (two waves a SIMD: 55 % and 36 % of the time at 4096 tokens).  us, stages of
-// one chain in both sweeps and exchanges through LDS / now, 32 heads over 8: 4096 tokens of size 128 302 / 278, 1024 64 / 60, of
-// size 64 38 / 35; 8 prompts of 64..1000, 28 over 4, 72 / 67.  Four stages in flight where a block is alone on its CU, both tiles' products before
+// one chain in both sweeps and exchanges through LDS / now, the call by itself in a graph, 32 heads over 8 in splits of 256: 4096 tokens of
+// size 128 288 / 271, 1024 59.2 / 54.3, of size 64 36.0 / 33.5; 8 prompts of 64..1000, 28 over 4, 64.8 / 59.5 (between a model's other launches, with
+// cold keys and on slower cards, 4096 tokens take up to 350).  Four stages in flight where a block is alone on its CU, both tiles' products before
 // their weights, and raised wave priority around products were no faster.
 #include <mutex>
 #include <type_traits>
@@ -54,9 +55,12 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(PromptAttnArgs a) {
   constexpr int kLoads = kPage / 1024;          // direct loads of a page
   constexpr int kPages = 2 * TPC;               // pages of a stage: a wave brings one (of K and of V)
   constexpr int kSplit = 128 * TPC, kSplitPages = kSplit / 16;
-  static_assert(2 * kPages <= 8, "a stage of either sweep");
-  __shared__ __attribute__((aligned(1024))) char s0[8 * kPage];
-  __shared__ __attribute__((aligned(1024))) char s1[8 * kPage];
+  // Keys of a stage of the first sweep: 128, but 64 where 128 of K alone are more than the second sweep's K and V and cost the room of a second
+  // workgroup on the CU (size 128 in splits of 128: 4096 tokens 284 us, with 128 keys a stage 408; of size 64 1024 tokens 37.6, with 128 36.9).
+  constexpr int kKeyPages = D == 64 ? 8 : 2 * kPages, kKeys = 16 * kKeyPages;
+  static_assert(kKeyPages >= 2 * kPages && kKeyPages % 4 == 0 && (kKeys == kSplit || 2 * kKeys == kSplit), "a stage of either sweep; a split's stages");
+  __shared__ __attribute__((aligned(1024))) char s0[kKeyPages * kPage];
+  __shared__ __attribute__((aligned(1024))) char s1[kKeyPages * kPage];
   __shared__ int32_t table[kTable];
   extern __shared__ float split_max[];          // [splits][kRows]
 
@@ -72,8 +76,7 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(PromptAttnArgs a) {
   const int kv_len = pos0 + n_tok;
   const int last_page = (kv_len - 1) >> 4;
   const int n_st = (kv_len + kSplit - 1) / kSplit * 4;   // stages of the second sweep
-  constexpr int kWide = 128 / 32;                        // tiles of a stage of the first sweep
-  const int n_max = (kv_len + 255) / 256 * 2;            // its stages, an even number: half a split or a whole one
+  const int n_max = (kv_len + 2 * kKeys - 1) / (2 * kKeys) * 2;   // and of the first, an even number: half a split or a whole one each
 
   // this lane's query row, its keys, and how far the wave's rows see
   const int m = wave * 32 + r;
@@ -109,10 +112,13 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(PromptAttnArgs a) {
     for (int i = 0; i < kLoads; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (lds_void*)(to + i * 1024), 16, lane * 16 + i * 1024, 0, 0, 0);
   };
-  // first sweep: stage st holds the K pages of 128 keys, two a wave
+  // first sweep: stage st holds K pages alone, a quarter of them a wave
   auto load_keys = [&](char* s, int st) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) bring(s + (wave * 2 + i) * kPage, a.kc, st * 8 + wave * 2 + i);
+    for (int i = 0; i < kKeyPages / 4; ++i) {
+      const int page = wave * (kKeyPages / 4) + i;
+      bring(s + page * kPage, a.kc, st * kKeyPages + page);
+    }
   };
   // second sweep: stage st is chain st & 3 of split st >> 2; wave w brings page w & 1 of tile chain + 4 (w >> 1): K, and V behind
   // the K pages
@@ -147,15 +153,15 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(PromptAttnArgs a) {
   auto key_of = [&](int st, int u) { return (st >> 2) * kSplit + ((st & 3) + 4 * u) * 32; };
   auto find_max = [&](const char* s, int st) __attribute__((always_inline)) {
 #pragma unroll 2   // (all four: 288 us for 278, registers in scratch)
-    for (int u = 0; u < kWide; ++u)
-      if (st * 128 + u * 32 < wave_last) {
+    for (int u = 0; u < kKeys / 32; ++u)
+      if (st * kKeys + u * 32 < wave_last) {
         f32x16 sc;
-        scores(s, u, st * 128 + u * 32, sc);
+        scores(s, u, st * kKeys + u * 32, sc);
         top_split = fmaxf(top_split, max_of(sc));
       }
-    if (TPC == 1 ? st * 128 < kv_len : st & 1) {   // (the split's last stage)
+    if (kKeys == kSplit ? st * kKeys < kv_len : st & 1) {   // (the split's last stage)
       top_split = halves_max(top_split * a.scale_log2);  // (positive: rounding keeps the order, the maximum is that of the scaled scores)
-      if (h == 0) split_max[st / TPC * kRows + m] = top_split;
+      if (h == 0) split_max[st * kKeys / kSplit * kRows + m] = top_split;
       top_row = fmaxf(top_row, top_split);
       top_split = -INFINITY;
     }
@@ -236,7 +242,7 @@ __global__ __launch_bounds__(256, 2) void prompt_attn_kernel(PromptAttnArgs a) {
     const int y = x + 1;
     if (y < n_max + n_st) {  // (uniform)
       const bool keys = kFirst && y < n_max;
-      const int first = keys ? y * 8 : first_page(y - n_max), pages = keys ? 8 : kSplitPages;
+      const int first = keys ? y * kKeyPages : first_page(y - n_max), pages = keys ? kKeyPages : kSplitPages;
       if (first < table0 || first + pages > table0 + kTable) {
         fill_table(first);
         __syncthreads();

@@ -626,3 +626,13 @@ def test_block_of_a_product_that_rotates_and_writes_pages(N, K, M, plain, rotary
     from tests.gpu_util import internal
     shape = internal("sd_prompt_shape_", C.c_int, *[C.c_int] * 5)
     assert (shape(M, N // 16, N // 16, K, 4), shape(M, N // 16, N // 16, K, 100)) == (plain, rotary)
+
+
+@pytest.mark.parametrize("N,M,gated,wide", [(32000, 33, False, False), (32000, 777, False, True), (13312, 1024, False, False), (13312, 2048, False, True),
+                                            (13312, 1024, True, False), (13312, 2048, True, True), (4096, 300, True, True), (4096, 512, False, False),
+                                            (1024, 777, True, False), (1024, 1500, True, True), (8192, 200, False, False), (64, 33, False, False)])
+def test_block_of_f32_row_products(N, M, gated, wide):
+    """Sizes that were measured with blocks of 64 x 64 and of 128 x 64."""
+    import ctypes as C
+    from tests.gpu_util import internal
+    assert internal("sd_rows_f32_wide_", C.c_bool, C.c_int, C.c_int, C.c_int, C.c_bool)(M, N, 1, gated) == wide

@@ -214,16 +214,23 @@ int launch(F32Args a, int batch, hipStream_t st) {
 
 }  // namespace
 
+// Whether blocks of 128 x 64 are quicker than 64 x 64 ones.  Blocks go over the CUs in rounds; us a stage of 32 columns and round, of a first
+// round alone / of further ones (medians of 308 sizes, 64..32000 x 512..4096, 33..2048 rows, with eight waves a block): 64 x 64 .60 / .53, gated .71 / .62;
+// 128 x 64 1.08 / 1.00, gated (one a CU) 1.18 / 1.17.  The rule's choice is .005 % slower than the better of the two on average, 0.7 % at most
+// (6144 x 2048 at 130 rows).  us of 64 x 64 / 128 x 64: 13312 x 1024 at 2048 rows 422 / 407, 1024 216 / 223; 32000 x 1024 at 777 421 / 406, 33 38.8 / 41.9;
+// 4096 x 1024 at 512 37.0 / 37.7; 4096 x 4096 at 300 127.8 / 127.7, gated 153 / 140; 1024 x 4096 gated at 1500 150 / 139, 777 81 / 136.
+// 128 x 128, 192 x 128 and 256 x 128 (of four waves) are slower than the better of the two everywhere (13312 x 1024 at 2048 rows 481, 503, 528).
+bool sd_rows_f32_wide_(int M, int N, int batch, bool gated) {
+  const long n1 = ((long)((N + 63) / 64) * ((M + 63) / 64) * batch + 255) / 256;
+  const long n2 = ((long)((N + 127) / 128) * ((M + 63) / 64) * batch + 255) / 256;
+  const float us1 = n1 == 1 ? (gated ? .71f : .60f) : (gated ? .62f : .53f) * n1;
+  const float us2 = n2 == 1 ? (gated ? 1.18f : 1.08f) : (gated ? 1.17f : 1.00f) * n2;
+  return us2 < us1;
+}
+
 // 16-byte aligned rows (K, ldx and the batch strides multiples of four)
 int sd_rows_f32_(const float* x, const float* x2, int64_t ldx, const float* w, const float* bias, float* y, int64_t ldy, int M,
                  int N, int K, int batch, int64_t bx, int64_t bw, int64_t by, bf16_t* yb, hipStream_t st) {
   const F32Args a{x, x2, w, bias, y, yb, ldx, ldy, bx, bw, by, M, N, K, 0, 0};
-  // Blocks go over the CUs in rounds, and a round of 128 x 64 costs 1.85 of 64 x 64 (a 64 x 64 block alone on its CU .60 us a
-  // stage of 32 columns, one of two or more .53; 128 x 64: 1.05 and .98).  us of 64 x 64 / 128 x 64: 13312 x 1024 at 2048 rows 422 / 407;
-  // 32000 x 1024 at 777 421 / 406; 4096 x 4096 at 777 248 / 242, 300 125 / 128; 1024 x 4096 gated at 2048 153 / 142, 777 81 / 136.
-  // 128 x 128, 192 x 128 and 256 x 128 (of four waves) are slower than the better of the two everywhere (13312 x 1024 at 2048 rows 481, 503, 528).
-  const long n1 = ((long)((N + 63) / 64) * ((M + 63) / 64) * batch + 255) / 256;
-  const long n2 = ((long)((N + 127) / 128) * ((M + 63) / 64) * batch + 255) / 256;
-  const float us1 = n1 == 1 ? .60f : .53f * n1, us2 = n2 == 1 ? 1.05f : .98f * n2;
-  return us1 <= us2 ? launch<1, 1>(a, batch, st) : launch<2, 1>(a, batch, st);
+  return sd_rows_f32_wide_(M, N, batch, x2) ? launch<2, 1>(a, batch, st) : launch<1, 1>(a, batch, st);
 }

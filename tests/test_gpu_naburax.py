@@ -889,7 +889,8 @@ def test_assignments_grouped_by_expert(E, n):
     assert torch.equal(out[sel < E], few[sel < E])
 
 
-@pytest.mark.parametrize("n,E,K", [(769, 5, 70), (770, 16, 2048), (771, 24, 513), (772, 2048, 64), (770, 2049, 64)])
+@pytest.mark.parametrize("n,E,K", [(769, 5, 70), (770, 16, 2048), (771, 24, 513), (772, 2048, 64), (770, 2049, 64), (1537, 5, 70), (513, 17, 130),
+                                   (771, 9, 2048)])
 @pytest.mark.parametrize("wdt", [torch.float32, torch.bfloat16])
 def test_router_of_four_rows_a_workgroup_has_the_bits_of_one(n, E, K, wdt):
     """Row counts that leave one to four rows to the last workgroup, fewer and more experts than waves, the most and one more than that

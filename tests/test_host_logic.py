@@ -636,3 +636,14 @@ def test_block_of_f32_row_products(N, M, gated, wide):
     import ctypes as C
     from tests.gpu_util import internal
     assert internal("sd_rows_f32_wide_", C.c_bool, C.c_int, C.c_int, C.c_int, C.c_bool)(M, N, 1, gated) == wide
+
+
+@pytest.mark.parametrize("E,one,four", [(256, [256, 512, 1100, 1280], [560, 700, 768, 1024, 1536, 2048, 4096]), (16, [256, 512, 1100], [560, 700, 1024, 1536, 2048]),
+                                        (8, [512, 768, 1100, 1280], [900, 1024, 1536, 2048, 4096]), (4, [768, 1024, 1280, 1536], [1800, 2048, 4096]),
+                                        (2049, [1024, 4096], [])])
+def test_rows_of_a_routers_workgroup(E, one, four):
+    """Row counts that were measured with one row a workgroup and with four (more than 2048 experts: one, whose scores fit)."""
+    import ctypes as C
+    from tests.gpu_util import internal
+    rule = internal("sd_route_four_rows_", C.c_bool, C.c_int, C.c_int)
+    assert not any(rule(n, E) for n in one) and all(rule(n, E) for n in four)

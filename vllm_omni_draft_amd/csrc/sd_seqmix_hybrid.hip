@@ -2678,6 +2678,18 @@ extern "C" int sd_moe_route_rows_biased(const float* x, int64_t ldx, const void*
                                      gate_out, stream);
 }
 
+// Whether a router's workgroup takes four rows, which read the experts' weights once, or one.  With one the time grows with every 256 rows (a
+// workgroup more on each CU), with four with every 1024, about three times as much where 16 waves share the experts; with 8 or 4 waves by
+// less, from a longer start.  us, one / four, 2048 columns: 256 experts 512 rows 105 / 127, 700 142 / 127, 1024 179 / 128, 1100 219 / 247, 1536 262 / 248,
+// 2048 340 / 251; 64 experts 512 29.1 / 35.5, 700 38.8 / 35.6, 1100 59.3 / 66.8, 2048 90.6 / 67.8; 16 experts 512 11.0 / 12.7, 700 14.7 / 12.8, 1100
+// 20.6 / 21.2, 1536 23.8 / 21.3; 8 experts 700 9.5 / 9.9, 1024 11.1 / 10.0, 1100 12.3 / 12.8, 1536 13.9 / 12.9; 4 experts 1024 8.1 / 9.0, 1536 9.9 / 10.1, 1800
+// 11.5 / 10.3, 4096 18.3 / 14.0.  Of 240 such sizes the rule takes the slower one in three (by 1 to 6 %).
+bool sd_route_four_rows_(int n_rows, int E) {
+  const int one = (n_rows + 255) / 256, four = (n_rows + 1023) / 1024;
+  if (E > 2048) return false;   // (their scores: 32 KB of LDS)
+  return E >= 16 ? one >= 3 * four : E >= 8 ? one > 2 * four + 1 : one > 6;
+}
+
 extern "C" int sd_moe_route_rows_corrected(const float* x, int64_t ldx, const void* w_router, const float* router_bias,
                                            const float* correction, int w_f32, float* logits, int32_t* sel_expert,
                                            float* sel_weight, int n_rows, int E, int K, int top, int score_kind,
@@ -2698,10 +2710,7 @@ extern "C" int sd_moe_route_rows_corrected(const float* x, int64_t ldx, const vo
         x, ldx, w, logits, sel_expert, sel_weight, E, K, top, score_kind, renorm, !w_f32, renorm_eps, weight_scale, (const T*)w_gate, n_gate,
         gate_out, router_bias, correction, PostNorm<T>{}, n_rows);
   };
-  // Four rows a workgroup once one row each is more than a round of them (two a CU, with 16 waves each).  us, one / four: 16 experts, 2048 columns
-  // 512 rows 10.6 / 12.2, 700 13.8 / 12.2, 1024 17.1 / 12.6, 2048 29.2 / 21.5; 64 experts 512 29.9 / 35.5, 1024 49.6 / 36.0, 2048 92.9 / 68.2; 8
-  // experts, 1024 columns 700 6.7 / 7.0, 1024 7.8 / 7.1, 2048 11.2 / 8.8.
-  const bool four = n_rows > 768 && E <= 2048;
+  const bool four = sd_route_four_rows_(n_rows, E);
   if (w_f32 && four) go((const float*)w_router, std::integral_constant<int, 4>{});
   else if (w_f32) go((const float*)w_router, std::integral_constant<int, 1>{});
   else if (four) go((const bf16_t*)w_router, std::integral_constant<int, 4>{});

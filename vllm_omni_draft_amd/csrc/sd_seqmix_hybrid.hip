@@ -1402,6 +1402,7 @@ constexpr int kMoeDirect = 16;  // at most this many assignments: each is its ow
 // experts up to its own for itself: a launch for the counts and one workgroup of 256 an expert took 4.7 + 5.9 us at 2048
 // assignments of 16 experts, and the gap between them; this one 4.9.
 constexpr int kGroupThreads = 1024, kGroupCounts = 1024;   // (experts counted at a time)
+static_assert(kGroupThreads == kGroupCounts, "a thread clears and adds up one expert's count");
 __global__ __launch_bounds__(kGroupThreads) void moe_group_kernel(const int32_t* __restrict__ sel_e, int n, int E, int32_t* __restrict__ perm,
                                                                   int32_t* __restrict__ tiles, int32_t* __restrict__ n_tiles, int bm) {
   constexpr int kWaves = kGroupThreads / 64;

@@ -696,14 +696,13 @@ int few_shape(const PromptArgs& a, hipStream_t st) {
 
 // The block of a prompt pass: the shape whose time by this model is the least.  The blocks go over the chip in rounds of 256 x
 // per_cu; a round takes `fixed` us (launch, first loads, epilogue), `split` us a split of K (its sums join the others')
-// and `stage` us a stage of 64 columns, which depends on how many blocks share a CU.  Fitted to 342 measured passes
-// (N 512..18944, K 512..18944, 272..4096 rows, weights from memory, epilogues through LDS, which took 2 to 8 us a block longer than those from
-// registers; 6-9 % off at the root of the mean square): the shapes it takes
-// are 1 % slower than the best of all there, 24 % faster than one block shape of 128 x 128 (whole K: 8 %).  Both sides
-// where it matters most, us, chosen shape against 128 x 128: 1024 x 2048 at 1024 rows 12.6 (64 x 64) and 25.6; 4096 x 4096
-// at 512 rows 29.3 (64 x 128) and 42.1; 6144 x 4096 at 1024 rows 63.3 (128 x 256) and 70.4; 3584 x 18944 at 2946 rows 354
-// (128 x 192) and 480; whole K, 14336 x 4096 gated: 1024 rows 188 (224 x 256) and 200 (256 x 256), 300 rows 86
-// (256 x 192) and 99.
+// and `stage` us a stage of 64 columns, which depends on how many blocks share a CU.  Fitted to 342 passes with epilogues through LDS, which took 2 to
+// 8 us a block longer than those from registers; with these, over 672 passes (N 512..32000, K 768..18944, 272..4096 rows, weights from memory),
+// the shapes it takes are .7 % (368 of split K), .6 % (128 QKV products), .4 % (96 gated, whole K) and 1.4 % (80 plain, whole K) slower than the
+// best of all, where constants fitted to these times are .7, 1.5, .2 and .5 %.  128 x 128 throughout, two a CU, is 43, 29, 24 and 15 %
+// slower than the shapes chosen.  us, chosen shape against 128 x 128: 1024 x 2048 at 1024 rows 13.3 (64 x 64) and 26.7; 4096 x 4096 at 512 rows 28.1
+// (64 x 128) and 55.3; 6144 x 4096 with rotation at 1024 rows 63.6 (128 x 256) and 72.5; 3584 x 18944 at 2946 rows 345 (128 x 192) and 467; whole K,
+// 14336 x 4096 gated: 1024 rows 181 (224 x 256) and 264, 300 rows 82 (256 x 192) and 117.
 struct Shape {
   int tn, tm, per_cu;
   float fixed, split, stage[3];
@@ -720,10 +719,10 @@ float shape_us(const Shape& s, int M, int n_tiles, int K, int S, int epi) {
   const long blocks = (long)((n_tiles + 2 * s.tn - 1) / (2 * s.tn)) * ((M + 32 * s.tm - 1) / (32 * s.tm));
   const long round = 256l * s.per_cu, full = blocks / round, rest = blocks - full * round;
   // The epilogue that rotates and writes pages is longer than a plain one, and nothing covers that of a large block alone on its CU.
-  // us of QKV products with it, as chosen without this term / with it: 6144 x 4096 at 2500 rows 152 (128 x 256) / 140 (128 x 128, two a CU), at
-  // 4000 226 / 206, 4608 x 3584 at 1500 81.8 / 69.7, 3072 x 2048 at 4000 87.9 / 79.4, 2946 rows 74.2 / 70.4; with .15 or .3 for .5 a tile
-  // between the two.
-  const float rope = epi == EPI_QKV_ROPE && S > 1 && s.tn * s.tm > 16 ? .5f * (s.tn * s.tm - 16) : 0.f;
+  // Of 128 QKV products (1152 x 896 to 10240 x 8192, 272..4096 rows) the shapes with .25 a tile are .6 % slower than the best of all, with 0 .7 %, with
+  // .5 (which the epilogue through LDS took) 1.0 %; any from .16 to .37 chooses the same.  us with .5 (128 x 128, two a CU) / with .25 (128 x 256):
+  // 6144 x 4096 at 1024 rows 72.5 / 63.6, 2500 130 / 125, 4096 201 / 190; 10240 x 8192 at 1300 240 / 206.
+  const float rope = epi == EPI_QKV_ROPE && S > 1 && s.tn * s.tm > 16 ? .25f * (s.tn * s.tm - 16) : 0.f;
   const float fixed = s.fixed + s.split * S + rope, stages = K / 64;
   float us = full * (fixed + s.stage[s.per_cu - 1] * stages);
   if (rest) {

@@ -62,7 +62,7 @@ __device__ __forceinline__ int tile_at(int t, int up_tiles) {
 // A wave is alone on its SIMD here, and nothing hides what its epilogue waits for: through LDS, four tokens at a time, each trip a
 // read, a residual's read, a chain of arithmetic and a store, 4096 x 4096 outputs of 4096 columns took 144 us, now 131 (with the residuals of
 // sixteen tokens at a time 145: all of a wave's are asked for at once); 2946 x 3584 of 18944 363, now 348; 14336 gated outputs of 4096 columns,
-// 1024 rows 194.5, now 191; 6144 x 4096 with rotation and pages, 1024 rows 74.0, now 66.
+// 1024 rows 194.5, now 191; 6144 x 4096 with rotation and pages, 1024 rows 74.5, now 63.6 (128 x 256 blocks; 128 x 128 70.9).
 // The four lanes of a token and tile store 32 bytes (bf16), sixteen tokens at once; the L2 joins them.  f32 outputs, 64 bytes, go out as
 // whole lines instead, eight tokens of two tiles at once (half lines: 2.5 % of a layer-list model's pass slower).
 struct TileSums {
@@ -241,7 +241,8 @@ __device__ __forceinline__ bool one_position_of_four(const WideRope& rp) {
 // A wave's tiles of a QKV product (those of n_tiles that exist): queries and keys rotated, keys and values into their pages.  A key's eight
 // channels of a page are 16 bytes, next to the next token's; a page row of a value's channel holds its tokens side by side, so four tokens of
 // a channel go in one store where they lie at neighbouring positions from a multiple of four on (others one by one).
-// Two tiles of a head at a time: an even number of tiles a wave.
+// Two tiles of a head at a time: an even number of tiles a wave.  us of products whose rows have three positions or none, through LDS with a row's place
+// looked up for every four outputs / this way: 4608 x 3584, three, 1024 rows 50.6 / 42.9, 2946 122 / 107; 2304 x 768, none, 2946 rows 25.0 / 19.7.
 // kBatch tiles of tokens from J0 on: 8 x 8 tiles go four at a time (all eight's cosines and sines beside the accumulators: 19 registers a
 // lane were spilled).
 constexpr int heads_batch(int tn, int tm) { return tn * tm > 32 && tm % 4 == 0 ? 4 : tm; }

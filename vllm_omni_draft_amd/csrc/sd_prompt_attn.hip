@@ -20,8 +20,8 @@
 // channels at a time, are live beside the split's and the row's.
 // What bounds it: products and vector work of a wave follow each other (two waves a SIMD: 55 % and 36 % of the time at 4096 tokens).  us, stages of
 // one chain in both sweeps and exchanges through LDS / now, the call by itself in a graph, 32 heads over 8 in splits of 256: 4096 tokens of
-// size 128 288 / 271, 1024 59.2 / 54.3, of size 64 36.0 / 33.5; 8 prompts of 64..1000, 28 over 4, 64.8 / 59.5 (between a model's other launches, with
-// cold keys and on slower cards, 4096 tokens take up to 350).  Four stages in flight where a block is alone on its CU, both tiles' products before
+// size 128 288 / 271, 1024 59.2 / 54.3, of size 64 36.0 / 33.5; 8 prompts of 64..1000, 28 over 4, 64.8 / 59.5 (in an 8B
+// model's prompt, with cold keys, 4096 tokens take 338 / 319).  Size 128 in splits of 256 keeps 22 registers a lane in scratch at two blocks a CU.  Four stages in flight where a block is alone on its CU, both tiles' products before
 // their weights, and raised wave priority around products were no faster.
 #include <mutex>
 #include <type_traits>
